@@ -37,6 +37,7 @@ extern "C" {
 #define SLA_F32 0
 #define SLA_BF16 1
 #define SLA_F16 2
+#define SLA_MASK_GIVEN (-1) /* in_dtype of sla_module_fwd: q, k, v are in `dtype` and lut already holds the selection */
 
 /* feature maps of the linear branch (reference core.py:43-57) */
 #define SLA_FMAP_ELU 0
@@ -54,6 +55,8 @@ extern "C" {
 #define SLA_WS_LINEAR_STATES 7 /* not an operation: the leading bytes of the SLA_WS_LINEAR_FWD workspace that hold the
                                   finished per-head states (see sla_linear_bwd, SLA_BWD_STATES_READY) */
 #define SLA_WS_LINEAR_COMPLEMENT_BWD 8
+#define SLA_WS_MODULE_FWD 9    /* dtype: that of the inputs */
+#define SLA_WS_LINEAR_BWD_STATES_APART 10 /* linear_workspace of sla_module_bwd_states */
 
 /* flags of sla_linear_bwd */
 #define SLA_BWD_ACCUMULATE 1   /* dq, dk, dv already hold the sparse branch's gradients: add to them */
@@ -212,6 +215,32 @@ int sla_module_bwd(const void* q, const void* k, const void* v, const int64_t* q
                    float* d_bias, int dtype, int fmap, int B, int H, int L, int D, int BLKQ, int BLKK, int topk,
                    float qk_scale, int flags, void* sparse_workspace, int64_t sparse_workspace_bytes, void* linear_workspace,
                    int64_t linear_workspace_bytes, void* stream, void* side_stream);
+
+/* sla_module_bwd with the forward's finished states (what sla_module_fwd left in `states`) read where they lie.
+ * linear_workspace: SLA_WS_LINEAR_BWD_STATES_APART bytes. */
+int sla_module_bwd_states(const void* q, const void* k, const void* v, const int64_t* qkv_strides, const void* o_s,
+                          const void* d_out, const int64_t* do_strides, const float* lse, const int8_t* sparse_map,
+                          const void* lut, int lut_elem_bytes, const float* weight, const float* bias, const void* states,
+                          void* dq, void* dk, void* dv, float* d_weight, float* d_bias, int dtype, int fmap, int B, int H,
+                          int L, int D, int BLKQ, int BLKK, int topk, float qk_scale, void* sparse_workspace,
+                          int64_t sparse_workspace_bytes, void* linear_workspace, int64_t linear_workspace_bytes,
+                          void* stream, void* side_stream);
+
+/* Forward of the whole module in one call: the kernels of sla_block_map_fwd, sla_linear_state_fwd and
+ * sla_sparse_attn_linear_fwd, bit-identical results.  q, k, v in `dtype` (in_dtype == dtype; qkv_strides may then name
+ * row-contiguous views, out_strides the output's), or contiguous fp32 (in_dtype == SLA_F32): the mask is then built
+ * from them as they are, and `cast` (3 * B*H*L*D 16-bit elements) receives the copies in `dtype` the rest works on.
+ * With in_dtype == SLA_MASK_GIVEN the caller has filled lut (a mask built from tensors of a third dtype, say).
+ * states (SLA_WS_LINEAR_STATES bytes) receives the finished per-head states, which sla_module_bwd_states reads.
+ * o_s and sparse_map may be NULL when no backward will need them.  side_stream (optional, same device, default
+ * priority): for large inputs the state build runs on it beside the mask builder; `stream` waits for it before the call returns.
+ * Workspace: SLA_WS_MODULE_FWD with dtype = in_dtype.
+ * Replaces SparseLinearAttention.forward, sparse_linear_attention/core.py:69-105. */
+int sla_module_fwd(const void* q, const void* k, const void* v, const int64_t* qkv_strides, int in_dtype, void* cast,
+                   const float* weight, const float* bias, void* out, const int64_t* out_strides, void* o_s, float* lse,
+                   int8_t* sparse_map, void* lut, int lut_elem_bytes, void* states, int dtype, int fmap, int B, int H,
+                   int L, int D, int BLKQ, int BLKK, int topk, float qk_scale, void* workspace, int64_t workspace_bytes,
+                   void* stream, void* side_stream);
 
 /* Linear branch in "complement" mode (opt-in): query block i attends linearly only to the key
  * blocks (of 64 rows) that its look-up row did NOT select; projection, bias and residual as in

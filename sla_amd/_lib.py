@@ -6,6 +6,7 @@ the import of any operator raises, there is no eager fallback.
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 
 import torch
@@ -15,9 +16,11 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.environ.get("SLA_HIP_LIB") or os.path.join(_HERE, "lib", "libsla_hip.so")
 
 SLA_F32, SLA_BF16, SLA_F16 = 0, 1, 2
+SLA_MASK_GIVEN = -1
+_DTYPE_CODES = {torch.float32: SLA_F32, torch.bfloat16: SLA_BF16, torch.float16: SLA_F16}
 FMAP = {"elu": 0, "relu": 1, "softmax": 2}
 (WS_BLOCK_MAP, WS_SPARSE_BWD, WS_LINEAR_FWD, WS_LINEAR_BWD, WS_SAGE_QUANT, WS_LINEAR_COMPLEMENT, WS_SAGE_PREPARE,
- WS_LINEAR_STATES, WS_LINEAR_COMPLEMENT_BWD) = range(9)
+ WS_LINEAR_STATES, WS_LINEAR_COMPLEMENT_BWD, WS_MODULE_FWD, WS_LINEAR_BWD_STATES_APART) = range(11)
 BWD_ACCUMULATE, BWD_STATES_READY = 1, 2
 
 ERR_BAD_ARG, ERR_UNSUPPORTED, ERR_LAUNCH, ERR_WORKSPACE = -1, -2, -3, -4
@@ -59,6 +62,10 @@ SIGNATURES = {
     "sla_linear_bwd": (_I, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P, _I64, _P]),
     "sla_module_bwd": (_I, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I,
                             _I, _I, _F, _I, _P, _I64, _P, _I64, _P, _P]),
+    "sla_module_bwd_states": (_I, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I,
+                                   _I, _I, _I, _I, _F, _P, _I64, _P, _I64, _P, _P]),
+    "sla_module_fwd": (_I, [_P, _P, _P, _P, _I, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _F,
+                            _P, _I64, _P, _P]),
     "sage_quant_qk": (_I, [_P, _P, _I, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _I64, _P]),
     "sage_prepare": (_I, [_P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P, _P, _I, _P, _P, _P, _P, _P, _P, _F, _P, _I64, _P]),
     "sage_quant_v": (_I, [_P, _I, _I, _I, _I, _I, _P, _P, _F, _P, _I64, _P]),
@@ -110,17 +117,17 @@ def check(rc: int) -> None:
 
 
 def dtype_code(dt: torch.dtype) -> int:
-    if dt == torch.float32:
-        return SLA_F32
-    if dt == torch.bfloat16:
-        return SLA_BF16
-    if dt == torch.float16:
-        return SLA_F16
-    raise TypeError(f"unsupported dtype {dt}")
+    code = _DTYPE_CODES.get(dt)
+    if code is None:
+        raise TypeError(f"unsupported dtype {dt}")
+    return code
 
 
 def stream_ptr(device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """hipStream_t of the current stream (the raw query: building a torch.cuda.Stream object for it costs several
+    microseconds, which the short calls notice)."""
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 def require_gpu(*tensors) -> None:
@@ -172,8 +179,13 @@ def empty_like_rows(t):
     return out.permute(inv)
 
 
-def workspace(op: int, dtype: int, B, H, L, D, BLKQ, BLKK, topk, device) -> torch.Tensor:
+@functools.lru_cache(maxsize=1024)
+def workspace_bytes(op: int, dtype: int, B, H, L, D, BLKQ, BLKK, topk) -> int:
     n = load().sla_workspace_bytes(op, dtype, B, H, L, D, BLKQ, BLKK, topk)
     if n < 0:
         check(int(n))
-    return torch.empty(max(int(n), 256), dtype=torch.uint8, device=device)
+    return max(int(n), 256)
+
+
+def workspace(op: int, dtype: int, B, H, L, D, BLKQ, BLKK, topk, device) -> torch.Tensor:
+    return torch.empty(workspace_bytes(op, dtype, B, H, L, D, BLKQ, BLKK, topk), dtype=torch.uint8, device=device)

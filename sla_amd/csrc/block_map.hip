@@ -11,7 +11,7 @@
 //                ascending order; group sums added in ascending order; one IEEE division by L;
 //   score      : acc = acc + (a_d * b_d), d ascending, no fused multiply-add.
 // Selection is by (score descending, index ascending); -0.0 == +0.0.
-#include "common.h"
+#include "fwd_steps.h"
 
 #include <mutex>
 
@@ -472,8 +472,8 @@ __global__ __launch_bounds__(256) void topk_kernel(const typename IO::raw* __res
   // bins); lane l then owns the four highest undecided digits 255 - 4l .. 252 - 4l, a prefix sum over the lanes
   // gives the number of keys above them, and the one lane whose digits straddle the wanted rank names the digit.
   if (T <= 0) {              // nothing to select (a ratio that rounds to no block at all): an all-zero map row, no table row
-    int8_t* zrow = sparse_map + row * N;
-    for (int i = lane; i < N; i += 64) zrow[i] = 0;
+    if (sparse_map)
+      for (int i = lane; i < N; i += 64) sparse_map[row * N + i] = 0;
     return;
   }
   uint32_t thr = 0;          // digits decided so far
@@ -552,7 +552,7 @@ __global__ __launch_bounds__(256) void topk_kernel(const typename IO::raw* __res
     const bool sel = gt || (eq && eq_rank < need_eq);
     const unsigned long long bsel = __ballot(sel);
     const int pos = run_sel + __popcll(bsel & lt_mask);
-    if (in) mrow[i] = sel ? 1 : 0;
+    if (in && sparse_map) mrow[i] = sel ? 1 : 0;
     if (sel && pos < T) {              // (pos < T always holds; the test keeps a wrong count from ever leaving the row)
       if (lut64)
         reinterpret_cast<long long*>(lut)[row * T + pos] = i;
@@ -709,26 +709,10 @@ void launch_map_from_pooled(int dtype, const void* pq, const void* pk, void* sco
   }
 }
 
-}  // namespace sla
-
-using namespace sla;
-
-extern "C" int sla_mean_pool(const void* x, void* out, int dtype, int BH, int L, int D, int BLK, void* stream) {
-  int rc = validate_pool(dtype, BH, L, D, BLK);
-  if (rc) return rc;
-  SLA_REQUIRE(x && out, SLA_ERR_BAD_ARG, "null pointer");
-  SLA_REQUIRE(((uintptr_t)x | (uintptr_t)out) % 16 == 0, SLA_ERR_BAD_ARG, "pointers must be 16-byte aligned");
-  hipStream_t st = (hipStream_t)stream;
-  const RowLayout lay = contiguous_layout(BH, L, D);
-  if (dtype == SLA_F32) launch_pool<IoF32, 1>(x, lay, nullptr, out, BH, L, D, BLK, st);
-  else if (dtype == SLA_BF16) launch_pool<IoBf16, 1>(x, lay, nullptr, out, BH, L, D, BLK, st);
-  else launch_pool<IoF16, 1>(x, lay, nullptr, out, BH, L, D, BLK, st);
-  return check_launch("mean_pool");
-}
-
-static int block_map_entry(const void* q, const void* k, const int64_t* strides, int dtype, int B, int H, int L, int D,
-                           int BLKQ, int BLKK, int topk, void* workspace, int64_t workspace_bytes, int8_t* sparse_map,
-                           void* lut, int lut_elem_bytes, void* stream) {
+// (want_map = false: the caller needs the look-up table only, sparse_map may be null)
+int block_map_entry(const void* q, const void* k, const int64_t* strides, int dtype, int B, int H, int L, int D, int BLKQ,
+                    int BLKK, int topk, void* workspace, int64_t workspace_bytes, int8_t* sparse_map, bool want_map, void* lut,
+                    int lut_elem_bytes, void* stream) {
   SLA_REQUIRE(B > 0 && H > 0, SLA_ERR_BAD_ARG, "non-positive batch/head count (B=%d H=%d)", B, H);
   const int64_t BH64 = (int64_t)B * H;
   SLA_REQUIRE(BH64 <= 65535, SLA_ERR_UNSUPPORTED, "B*H=%lld exceeds 65535", (long long)BH64);
@@ -745,7 +729,7 @@ static int block_map_entry(const void* q, const void* k, const int64_t* strides,
   SLA_REQUIRE((int64_t)BH * M < (1ll << 31), SLA_ERR_UNSUPPORTED, "too many query-block rows");
   SLA_REQUIRE(lut_elem_bytes == 4 || lut_elem_bytes == 8, SLA_ERR_BAD_ARG, "lut_elem_bytes must be 4 or 8, got %d",
               lut_elem_bytes);
-  SLA_REQUIRE(q && k && workspace && sparse_map && (lut || topk == 0), SLA_ERR_BAD_ARG, "null pointer");
+  SLA_REQUIRE(q && k && workspace && (sparse_map || !want_map) && (lut || topk == 0), SLA_ERR_BAD_ARG, "null pointer");
   SLA_REQUIRE(((uintptr_t)q | (uintptr_t)k | (uintptr_t)workspace | (uintptr_t)lut) % 16 == 0, SLA_ERR_BAD_ARG,
               "pointers must be 16-byte aligned");
   const int64_t need = block_map_workspace_bytes(dtype, BH, L, D, BLKQ, BLKK);
@@ -764,10 +748,27 @@ static int block_map_entry(const void* q, const void* k, const int64_t* strides,
   return block_map_impl<IoF16>(q, k, lay, dtype, BH, L, D, BLKQ, BLKK, topk, ws, sparse_map, lut, lut64, st);
 }
 
+}  // namespace sla
+
+using namespace sla;
+
+extern "C" int sla_mean_pool(const void* x, void* out, int dtype, int BH, int L, int D, int BLK, void* stream) {
+  int rc = validate_pool(dtype, BH, L, D, BLK);
+  if (rc) return rc;
+  SLA_REQUIRE(x && out, SLA_ERR_BAD_ARG, "null pointer");
+  SLA_REQUIRE(((uintptr_t)x | (uintptr_t)out) % 16 == 0, SLA_ERR_BAD_ARG, "pointers must be 16-byte aligned");
+  hipStream_t st = (hipStream_t)stream;
+  const RowLayout lay = contiguous_layout(BH, L, D);
+  if (dtype == SLA_F32) launch_pool<IoF32, 1>(x, lay, nullptr, out, BH, L, D, BLK, st);
+  else if (dtype == SLA_BF16) launch_pool<IoBf16, 1>(x, lay, nullptr, out, BH, L, D, BLK, st);
+  else launch_pool<IoF16, 1>(x, lay, nullptr, out, BH, L, D, BLK, st);
+  return check_launch("mean_pool");
+}
+
 extern "C" int sla_block_map_fwd(const void* q, const void* k, int dtype, int B, int H, int L, int D, int BLKQ, int BLKK,
                                  int topk, void* workspace, int64_t workspace_bytes, int8_t* sparse_map, void* lut,
                                  int lut_elem_bytes, void* stream) {
-  return block_map_entry(q, k, nullptr, dtype, B, H, L, D, BLKQ, BLKK, topk, workspace, workspace_bytes, sparse_map, lut,
+  return block_map_entry(q, k, nullptr, dtype, B, H, L, D, BLKQ, BLKK, topk, workspace, workspace_bytes, sparse_map, true, lut,
                          lut_elem_bytes, stream);
 }
 
@@ -819,7 +820,7 @@ extern "C" int sla_block_map_fwd_static(const void* q, const void* k, int dtype,
   // every part of the scratch is written by one kernel of the sequence before a later one reads it: nothing
   // has to be cleared between calls
   return block_map_entry(q, k, nullptr, dtype, B, H, L, D, BLKQ, BLKK, topk, ws, (int64_t)SLA_STATIC_SCRATCH_BYTES,
-                         sparse_map, lut, lut_elem_bytes, stream);
+                         sparse_map, true, lut, lut_elem_bytes, stream);
 }
 
 extern "C" int sla_block_map_fwd_strided(const void* q, const void* k, const int64_t* qk_strides, int dtype, int B, int H,
@@ -827,6 +828,6 @@ extern "C" int sla_block_map_fwd_strided(const void* q, const void* k, const int
                                          int64_t workspace_bytes, int8_t* sparse_map, void* lut, int lut_elem_bytes,
                                          void* stream) {
   SLA_REQUIRE(qk_strides, SLA_ERR_BAD_ARG, "null strides");
-  return block_map_entry(q, k, qk_strides, dtype, B, H, L, D, BLKQ, BLKK, topk, workspace, workspace_bytes, sparse_map, lut,
+  return block_map_entry(q, k, qk_strides, dtype, B, H, L, D, BLKQ, BLKK, topk, workspace, workspace_bytes, sparse_map, true, lut,
                          lut_elem_bytes, stream);
 }

@@ -24,6 +24,10 @@ constexpr int LB_ALL = 15;
 int linear_bwd_steps(const void* q, const void* k, const void* v, const int64_t* qkv_strides, const float* weight,
                      const float* bias, const void* d_out, const int64_t* do_strides, void* dq, void* dk, void* dv,
                      float* d_weight, float* d_bias, int dtype, int fmap, int B, int H, int L, int D, int flags,
-                     void* workspace, int64_t workspace_bytes, void* stream, int steps);
+                     const void* states, void* workspace, int64_t workspace_bytes, void* stream, int steps);
+// (states: the forward's finished states where they lie, or null: they are built, or with SLA_BWD_STATES_READY found, at the
+//  start of the workspace.  With states given the workspace needs linear_bwd_states_apart_bytes() only.)
+int64_t linear_bwd_states_apart_bytes(int BH, int L, int D);
+int64_t sparse_bwd_workspace_bytes(int BH, int L, int D, int BLKQ, int BLKK, int topk);
 
 }  // namespace sla

@@ -1,5 +1,5 @@
 // Library-wide pieces of the C ABI: version, error text, workspace sizes.
-#include "common.h"
+#include "side_events.h"
 
 namespace sla {
 
@@ -18,6 +18,32 @@ int check_launch(const char* what) {
     set_error("%s: launch failed: %s", what, hipGetErrorString(e));
     return SLA_ERR_LAUNCH;
   }
+  return SLA_OK;
+}
+
+std::mutex& side_events_mutex() {
+  static std::mutex mu;
+  return mu;
+}
+
+int side_events_for_current_device(SideEvents** out) {
+  static SideEvents per_device[64];
+  int dev = 0;
+  SLA_REQUIRE(hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < 64, SLA_ERR_LAUNCH, "no current device");
+  SideEvents& e = per_device[dev];
+  if (!e.fork) {
+    // all four or none: the set is published only when every event exists
+    hipEvent_t made[4] = {nullptr, nullptr, nullptr, nullptr};
+    for (int i = 0; i < 4; ++i) {
+      if (hipEventCreateWithFlags(&made[i], hipEventDisableTiming) != hipSuccess) {
+        for (int j = 0; j < i; ++j) (void)hipEventDestroy(made[j]);
+        set_error("hipEventCreate failed");
+        return SLA_ERR_LAUNCH;
+      }
+    }
+    e = SideEvents{made[0], made[1], made[2], made[3]};
+  }
+  *out = &e;
   return SLA_OK;
 }
 
@@ -57,6 +83,8 @@ int64_t sage_prepare_workspace_bytes(int BH, int L, int D);
 int64_t linear_states_bytes(int BH, int L, int D);
 int64_t linear_complement_workspace_bytes(int BH, int L, int D);
 int64_t linear_complement_bwd_workspace_bytes(int BH, int L, int D, int BLKQ);
+int64_t linear_bwd_states_apart_bytes(int BH, int L, int D);
+int64_t module_fwd_workspace_bytes(int in_dtype, int BH, int L, int D, int BLKQ, int BLKK);
 
 }  // namespace sla
 
@@ -93,6 +121,12 @@ extern "C" int64_t sla_workspace_bytes(int op, int dtype, int B, int H, int L, i
     case SLA_WS_LINEAR_COMPLEMENT_BWD:
       SLA_REQUIRE(BLKQ == 64 || BLKQ == 128, SLA_ERR_UNSUPPORTED, "BLKQ=%d (64 or 128)", BLKQ);
       return linear_complement_bwd_workspace_bytes(BH, L, D, BLKQ);
+    case SLA_WS_LINEAR_BWD_STATES_APART:
+      return linear_bwd_states_apart_bytes(BH, L, D);
+    case SLA_WS_MODULE_FWD:
+      SLA_REQUIRE(BLKQ > 0 && BLKK > 0, SLA_ERR_BAD_ARG, "non-positive block size");
+      SLA_REQUIRE(dtype == SLA_F32 || dtype == SLA_BF16 || dtype == SLA_F16, SLA_ERR_BAD_ARG, "unknown dtype %d", dtype);
+      return module_fwd_workspace_bytes(dtype, BH, L, D, BLKQ, BLKK);
     default:
       set_error("unknown workspace op %d", op);
       return SLA_ERR_BAD_ARG;

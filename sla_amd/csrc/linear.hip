@@ -17,6 +17,7 @@
 //                   per-query divisor is a per-lane scalar; the tile is scaled, biased, parked in LDS
 //                   and written (plus the residual) with whole-row 16-byte accesses.
 #include "linear_state.h"
+#include "fwd_steps.h"
 #include "sage_steps.h"
 
 namespace sla {
@@ -110,15 +111,31 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // ---- host side ----------------------------------------------------------------------------
 int64_t linear_fwd_workspace_bytes(int BH, int L, int D) { return (int64_t)lin_ws(BH, L, D).total; }
 int64_t linear_states_bytes(int BH, int L, int D) { return (int64_t)lin_ws(BH, L, D).states_end; }
+int64_t linear_parts_bytes(int BH, int L, int D) {
+  const LinWs w = lin_ws(BH, L, D);
+  return (int64_t)(w.total - w.states_end);
+}
 
 template <typename Tag, int D>
 static int linear_state_impl(const void* k, const void* v, const RowLayout& lay, const float* weight, int fmap, int BH, int L,
-                             char* ws, hipStream_t st) {
+                             char* ws, char* parts, hipStream_t st) {
   const LinWs w = lin_ws(BH, L, D);
-  launch_state_build<Tag, D>(k, v, lay, weight, fmap, BH, L, ws, w, st, false);
+  launch_state_build<Tag, D>(k, v, lay, weight, fmap, BH, L, ws, parts, w, st, false);
   hipLaunchKernelGGL((linear_fold_kernel<Tag>), dim3(D / (1024 / D), BH), dim3(256), 0, st,
                      (const uint16_t*)(ws + w.kvt), weight, (uint16_t*)(ws + w.kvwt), (uint16_t*)(ws + w.wt), D);
   return check_launch("linear_state_fwd");
+}
+
+int linear_state_run(const void* k, const void* v, const RowLayout& lay, const float* weight, int dtype, int fmap, int BH, int L,
+                     int D, char* states, char* parts, hipStream_t st) {
+#define SLA_LIN_CASE(TAG, DD) return linear_state_impl<TAG, DD>(k, v, lay, weight, fmap, BH, L, states, parts, st)
+  if (dtype == SLA_BF16) {
+    if (D == 128) SLA_LIN_CASE(bf16_tag, 128);
+    SLA_LIN_CASE(bf16_tag, 64);
+  }
+  if (D == 128) SLA_LIN_CASE(f16_tag, 128);
+  SLA_LIN_CASE(f16_tag, 64);
+#undef SLA_LIN_CASE
 }
 
 // The same with v quantised to FP8 on the way: the state kernel, which streams v anyway, leaves the column maxima of
@@ -197,14 +214,7 @@ static int linear_state_entry(const void* k, const void* v, const int64_t* strid
   if (rc) return rc;
   hipStream_t st = (hipStream_t)stream;
   char* ws = (char*)workspace;
-#define SLA_LIN_CASE(TAG, DD) return linear_state_impl<TAG, DD>(k, v, lay, weight, fmap, BH, L, ws, st)
-  if (dtype == SLA_BF16) {
-    if (D == 128) SLA_LIN_CASE(bf16_tag, 128);
-    SLA_LIN_CASE(bf16_tag, 64);
-  }
-  if (D == 128) SLA_LIN_CASE(f16_tag, 128);
-  SLA_LIN_CASE(f16_tag, 64);
-#undef SLA_LIN_CASE
+  return linear_state_run(k, v, lay, weight, dtype, fmap, BH, L, D, ws, ws + linear_states_bytes(BH, L, D), st);
 }
 
 extern "C" int sla_linear_state_fwd(const void* k, const void* v, const float* weight, int dtype, int fmap, int B, int H,

@@ -587,16 +587,19 @@ struct LinBwdWs {
   LinSplit ss;   // slices of the stream kernel (one workgroup per compute unit, 128 rows per step): never more than st's
   size_t dn, y, dden, ds_part, dw_part, dz_part, db_part, ds, dst, dz, dw_head, db_head, total;
 };
-static LinBwdWs lin_bwd_ws(int BH, int L, int D) {
+// (own_states = false: the forward's states lie elsewhere, the workspace holds none.  Head dim 128 never takes the path with
+//  row-wise temporaries.)
+static LinBwdWs lin_bwd_ws(int BH, int L, int D, bool own_states) {
   LinBwdWs w;
   w.fwd = lin_ws(BH, L, D);
   w.st = lin_split(BH, L, 512);
   w.ss = lin_split(BH, L, 256, LBS_TR);
   const int64_t np = (int64_t)BH * w.st.nsplit;
-  size_t off = w.fwd.total;
-  w.dn = off;      off += align_up((int64_t)BH * L * D * 2, 256);
-  w.y = off;       off += align_up((int64_t)BH * L * D * 2, 256);
-  w.dden = off;    off += align_up((int64_t)BH * L * 4, 256);
+  size_t off = own_states ? w.fwd.total : 0;
+  const int64_t rows = D == 128 ? 0 : (int64_t)BH * L;
+  w.dn = off;      off += align_up(rows * D * 2, 256);
+  w.y = off;       off += align_up(rows * D * 2, 256);
+  w.dden = off;    off += align_up(rows * 4, 256);
   w.ds_part = off; off += align_up(np * D * D * 4, 256);
   // (the stream path keeps M of every head there in both orientations: two matrices per head at least)
   w.dw_part = off; off += align_up((np > 2 * BH ? np : 2 * (int64_t)BH) * D * D * 4, 256);
@@ -610,23 +613,25 @@ static LinBwdWs lin_bwd_ws(int BH, int L, int D) {
   w.total = off;
   return w;
 }
-int64_t linear_bwd_workspace_bytes(int BH, int L, int D) { return (int64_t)lin_bwd_ws(BH, L, D).total; }
+int64_t linear_bwd_workspace_bytes(int BH, int L, int D) { return (int64_t)lin_bwd_ws(BH, L, D, true).total; }
+int64_t linear_bwd_states_apart_bytes(int BH, int L, int D) { return (int64_t)lin_bwd_ws(BH, L, D, false).total; }
 
 template <typename Tag, int D>
 static int linear_bwd_impl(const void* q, const void* k, const void* v, const float* weight, const void* d_out, void* dq,
                            void* dk, void* dv, const RowLayout& lin, const RowLayout& ldo, float* d_weight, float* d_bias,
-                           int fmap, int BH, int L, int flags, char* ws, hipStream_t st, int steps) {
+                           int fmap, int BH, int L, int flags, const char* states, char* ws, hipStream_t st, int steps) {
   if (steps == 0) return SLA_OK;        // (arguments checked, nothing asked for)
-  const LinBwdWs w = lin_bwd_ws(BH, L, D);
+  const LinBwdWs w = lin_bwd_ws(BH, L, D, !states);
   const int accumulate = flags & SLA_BWD_ACCUMULATE;
-  if ((steps & LB_STATES) && !(flags & SLA_BWD_STATES_READY)) {
+  if ((steps & LB_STATES) && !states && !(flags & SLA_BWD_STATES_READY)) {
     // everything the forward's state build leaves: transposed state, z, and (fold) the folded state + 16-bit weight
-    launch_state_build<Tag, D>(k, v, lin, weight, fmap, BH, L, ws, w.fwd, st, false);
+    launch_state_build<Tag, D>(k, v, lin, weight, fmap, BH, L, ws, ws + w.fwd.states_end, w.fwd, st, false);
     hipLaunchKernelGGL((linear_fold_kernel<Tag>), dim3(D / (1024 / D), BH), dim3(256), 0, st,
                        (const uint16_t*)(ws + w.fwd.kvt), weight, (uint16_t*)(ws + w.fwd.kvwt), (uint16_t*)(ws + w.fwd.wt), D);
   }
-  uint16_t* kvt = (uint16_t*)(ws + w.fwd.kvt);
-  uint16_t* z = (uint16_t*)(ws + w.fwd.z);
+  if (!states) states = ws;
+  const uint16_t* kvt = (const uint16_t*)(states + w.fwd.kvt);
+  const uint16_t* z = (const uint16_t*)(states + w.fwd.z);
   constexpr int NW_ROWS = 4, NW_KV = 8;   // one workgroup per compute unit either way (LDS)
   const int tiles_kv = balanced_tiles(cdiv(L, 32 * NW_KV), BH, 1);
   // (the stream kernel addresses a head's rows through 32-bit buffer offsets)
@@ -642,7 +647,7 @@ static int linear_bwd_impl(const void* q, const void* k, const void* v, const fl
     if (steps & LB_QUERY) {
 #define SLA_LBS_LAUNCH(FM)                                                                                                  \
   hipLaunchKernelGGL((linear_bwd_stream_kernel<Tag, FM>), dim3(w.ss.nsplit, BH), dim3(512), 0, st, (const uint16_t*)q,        \
-                     (const uint16_t*)d_out, (const uint16_t*)(ws + w.fwd.kvwt), z, (uint16_t*)dq, lin, ldo, m_part,          \
+                     (const uint16_t*)d_out, (const uint16_t*)(states + w.fwd.kvwt), z, (uint16_t*)dq, lin, ldo, m_part,          \
                      (float*)(ws + w.dz_part), (float*)(ws + w.db_part), L, w.ss.rows_per_split, accumulate)
     if (fmap == SLA_FMAP_ELU) SLA_LBS_LAUNCH(SLA_FMAP_ELU);
     else if (fmap == SLA_FMAP_RELU) SLA_LBS_LAUNCH(SLA_FMAP_RELU);
@@ -664,7 +669,7 @@ static int linear_bwd_impl(const void* q, const void* k, const void* v, const fl
   const int tiles_rows = balanced_tiles(cdiv(L, 32 * NW_ROWS), BH, 1);
   if (steps & LB_QUERY) {
   hipLaunchKernelGGL((linear_bwd_rows_kernel<Tag, D, NW_ROWS>), dim3(cdiv(L, 32 * NW_ROWS * tiles_rows), BH), dim3(64 * NW_ROWS), 0, st, (const uint16_t*)q,
-                     (const uint16_t*)d_out, kvt, (const uint16_t*)(ws + w.fwd.kvp), z, (const uint16_t*)(ws + w.fwd.wt), (uint16_t*)dq, lin, ldo, dn, y,
+                     (const uint16_t*)d_out, kvt, (const uint16_t*)(states + w.fwd.kvp), z, (const uint16_t*)(states + w.fwd.wt), (uint16_t*)dq, lin, ldo, dn, y,
                      dden, L, fmap, tiles_rows, accumulate);
   hipLaunchKernelGGL((linear_bwd_states_kernel<Tag, D>), dim3(w.st.nsplit, BH), dim3(256), 0, st, (const uint16_t*)q, dn,
                      (const uint16_t*)d_out, y, dden, lin, ldo, (float*)(ws + w.ds_part), (float*)(ws + w.dw_part),
@@ -759,7 +764,7 @@ void launch_weight_grads(int dtype, int D, const void* q, const void* dn, const 
 int linear_bwd_steps(const void* q, const void* k, const void* v, const int64_t* qkv_strides, const float* weight,
                      const float* bias, const void* d_out, const int64_t* do_strides, void* dq, void* dk, void* dv,
                      float* d_weight, float* d_bias, int dtype, int fmap, int B, int H, int L, int D, int flags,
-                     void* workspace, int64_t workspace_bytes, void* stream, int steps) {
+                     const void* states, void* workspace, int64_t workspace_bytes, void* stream, int steps) {
   int rc = validate_linear(dtype, fmap, B, H, L, D);
   if (rc) return rc;
   SLA_REQUIRE((flags & ~(SLA_BWD_ACCUMULATE | SLA_BWD_STATES_READY)) == 0, SLA_ERR_BAD_ARG, "unknown flag bits in %d", flags);
@@ -767,10 +772,10 @@ int linear_bwd_steps(const void* q, const void* k, const void* v, const int64_t*
   SLA_REQUIRE(q && k && v && weight && d_out && dq && dk && dv && d_weight && d_bias && workspace, SLA_ERR_BAD_ARG,
               "null pointer");
   SLA_REQUIRE(((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)d_out | (uintptr_t)dq | (uintptr_t)dk | (uintptr_t)dv |
-               (uintptr_t)weight | (uintptr_t)workspace) % 16 == 0,
+               (uintptr_t)weight | (uintptr_t)states | (uintptr_t)workspace) % 16 == 0,
               SLA_ERR_BAD_ARG, "pointers must be 16-byte aligned");
   const int BH = B * H;
-  const int64_t need = linear_bwd_workspace_bytes(BH, L, D);
+  const int64_t need = (int64_t)lin_bwd_ws(BH, L, D, !states).total;
   SLA_REQUIRE(workspace_bytes >= need, SLA_ERR_WORKSPACE, "workspace of %lld bytes, need %lld", (long long)workspace_bytes,
               (long long)need);
   RowLayout lin, ldo;
@@ -781,7 +786,7 @@ int linear_bwd_steps(const void* q, const void* k, const void* v, const int64_t*
   hipStream_t st = (hipStream_t)stream;
   char* ws = (char*)workspace;
 #define SLA_LINB_CASE(TAG, DD) \
-  return linear_bwd_impl<TAG, DD>(q, k, v, weight, d_out, dq, dk, dv, lin, ldo, d_weight, d_bias, fmap, BH, L, flags, ws, st, \
+  return linear_bwd_impl<TAG, DD>(q, k, v, weight, d_out, dq, dk, dv, lin, ldo, d_weight, d_bias, fmap, BH, L, flags, (const char*)states, ws, st, \
                                   steps)
   if (dtype == SLA_BF16) {
     if (D == 128) SLA_LINB_CASE(bf16_tag, 128);
@@ -801,7 +806,7 @@ extern "C" int sla_linear_bwd(const void* q, const void* k, const void* v, const
                               int fmap, int B, int H, int L, int D, int flags, void* workspace,
                               int64_t workspace_bytes, void* stream) {
   return linear_bwd_steps(q, k, v, nullptr, weight, bias, d_out, nullptr, dq, dk, dv, d_weight, d_bias, dtype, fmap, B, H, L,
-                          D, flags, workspace, workspace_bytes, stream, LB_ALL);
+                          D, flags, nullptr, workspace, workspace_bytes, stream, LB_ALL);
 }
 
 extern "C" int sla_linear_bwd_strided(const void* q, const void* k, const void* v, const int64_t* qkv_strides,
@@ -811,5 +816,5 @@ extern "C" int sla_linear_bwd_strided(const void* q, const void* k, const void* 
                                       void* stream) {
   SLA_REQUIRE(qkv_strides && do_strides, SLA_ERR_BAD_ARG, "null strides");
   return linear_bwd_steps(q, k, v, qkv_strides, weight, bias, d_out, do_strides, dq, dk, dv, d_weight, d_bias, dtype, fmap, B,
-                          H, L, D, flags, workspace, workspace_bytes, stream, LB_ALL);
+                          H, L, D, flags, nullptr, workspace, workspace_bytes, stream, LB_ALL);
 }

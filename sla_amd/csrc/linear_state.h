@@ -326,11 +326,13 @@ static inline LinWs lin_ws(int BH, int L, int D) {
 
 
 // Streams K and V once and leaves KVT, KVP, z (16 bit) and the 16-bit transposed weight in the workspace.
+// (ws: where the states go; parts: where the slices' partial sums go, the offsets of `w` past states_end)
 template <typename Tag, int D>
 static inline void launch_state_build(const void* k, const void* v, const RowLayout& lay, const float* weight, int fmap,
-                                      int BH, int L, char* ws, const LinWs& w, hipStream_t st, bool copy_weight = true) {
-  float* kv_part = (float*)(ws + w.kv_part);
-  float* z_part = (float*)(ws + w.z_part);
+                                      int BH, int L, char* ws, char* parts, const LinWs& w, hipStream_t st,
+                                      bool copy_weight = true) {
+  float* kv_part = (float*)(parts + (w.kv_part - w.states_end));
+  float* z_part = (float*)(parts + (w.z_part - w.states_end));
   uint16_t* kvt = (uint16_t*)(ws + w.kvt);
   uint16_t* z = (uint16_t*)(ws + w.z);
   hipLaunchKernelGGL((linear_state_partial_kernel<Tag, D>), dim3(w.nsplit, BH), dim3(256), 0, st, (const uint16_t*)k,

@@ -13,6 +13,7 @@
 // softmax, its V during PV.  Register use is held to 256 so two waves share a SIMD and one
 // wave's softmax (vector ALU) overlaps the other's MFMAs (three waves at head dim 64, where the registers allow it:
 // 6 % faster there).
+#include "fwd_steps.h"
 #include "linear_state.h"
 
 namespace sla {
@@ -491,6 +492,16 @@ int validate_attn_shape(int dtype, int B, int H, int L, int D, int BLKQ, int BLK
   return SLA_OK;
 }
 
+int attn_linear_run(const void* q, const void* k, const void* v, const RowLayout& lin, const void* lut, int lut_elem_bytes,
+                    const char* states, const float* bias, void* o_s, void* out, const RowLayout& lout, float* lse, int dtype,
+                    int fmap, int BH, int L, int D, int BLKQ, int topk, float qk_scale, hipStream_t st) {
+  const LinWs w = lin_ws(BH, L, D);
+  const FusedLinear fl{(const uint16_t*)(states + w.kvwt), (const uint16_t*)(states + w.z), bias, fmap, (uint16_t*)o_s};
+  if (dtype == SLA_BF16)
+    return launch_fwd<bf16_tag>(q, k, v, lut, lut_elem_bytes == 8, out, lse, lin, lout, BH, L, D, BLKQ, topk, qk_scale, &fl, st);
+  return launch_fwd<f16_tag>(q, k, v, lut, lut_elem_bytes == 8, out, lse, lin, lout, BH, L, D, BLKQ, topk, qk_scale, &fl, st);
+}
+
 }  // namespace sla
 
 using namespace sla;
@@ -529,18 +540,13 @@ static int attn_linear_entry(const void* q, const void* k, const void* v, const 
   const LinWs w = lin_ws(BH, L, D);
   SLA_REQUIRE(linear_workspace_bytes >= (int64_t)w.total, SLA_ERR_WORKSPACE, "workspace of %lld bytes, need %lld",
               (long long)linear_workspace_bytes, (long long)w.total);
-  const char* ws = (const char*)linear_workspace;
-  FusedLinear fl{(const uint16_t*)(ws + w.kvwt), (const uint16_t*)(ws + w.z), bias, fmap, (uint16_t*)o_s};
   RowLayout lin, lout;
   rc = make_layout(qkv_strides, B, H, L, D, 2, &lin);
   if (rc) return rc;
   rc = make_layout(out_strides, B, H, L, D, 2, &lout);
   if (rc) return rc;
-  hipStream_t st = (hipStream_t)stream;
-  if (dtype == SLA_BF16)
-    return launch_fwd<bf16_tag>(q, k, v, lut, lut_elem_bytes == 8, out, lse, lin, lout, BH, L, D, BLKQ, topk, qk_scale, &fl,
-                                st);
-  return launch_fwd<f16_tag>(q, k, v, lut, lut_elem_bytes == 8, out, lse, lin, lout, BH, L, D, BLKQ, topk, qk_scale, &fl, st);
+  return attn_linear_run(q, k, v, lin, lut, lut_elem_bytes, (const char*)linear_workspace, bias, o_s, out, lout, lse, dtype, fmap,
+                         BH, L, D, BLKQ, topk, qk_scale, (hipStream_t)stream);
 }
 
 extern "C" int sla_sparse_attn_linear_fwd(const void* q, const void* k, const void* v, const void* lut, int lut_elem_bytes,

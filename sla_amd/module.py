@@ -2,13 +2,15 @@
 module (``sparse_linear_attention/core.py:24-105``), running on the HIP kernels."""
 from __future__ import annotations
 
+import functools
+
 import torch
 import torch.nn as nn
 
 from . import _lib
-from .block_map import get_block_map
-from .linear import linear_complement_bwd, linear_complement_fwd, linear_state_fwd, linear_state_quant_v_fwd, saved_states
-from .sparse_attn import sparse_attn_bwd, sparse_attn_fwd, sparse_attn_linear_fwd
+from .block_map import get_block_map, topk_count
+from .linear import linear_complement_bwd, linear_complement_fwd, linear_state_fwd, linear_state_quant_v_fwd
+from .sparse_attn import sparse_attn_bwd, sparse_attn_fwd
 
 FEATURE_MAPS = ("elu", "relu", "softmax")
 
@@ -51,15 +53,97 @@ def module_bwd(q, k, v, o_s, d_out, lse, sparse_map, lut, topk, BLKQ, BLKK, qk_s
     return dq, dk, dv, dw, db
 
 
-def _backward_side_stream(dev):
-    """The stream the short kernels of the backward go to: the one the forward's state build uses (default priority,
-    one per device); none while a graph is being captured (the work then stays on the capturing stream)."""
+def _side_stream(dev):
+    """Handle of the stream that takes what may run beside the main one (default priority, one per device; the library uses it
+    where that pays); none while a graph is being captured (the work then stays on the capturing stream)."""
     if torch.cuda.is_current_stream_capturing():
         return None
-    side = _StateBuild._side.get(dev.index)
-    if side is None:
-        side = _StateBuild._side[dev.index] = torch.cuda.Stream(device=dev)
-    return side
+    handle = _side_handles.get(dev.index)
+    if handle is None:
+        side = _StateBuild._side[dev.index] = _StateBuild._side.get(dev.index) or torch.cuda.Stream(device=dev)
+        handle = _side_handles[dev.index] = side.cuda_stream
+    return handle
+
+
+_side_handles = {}
+
+
+@functools.lru_cache(maxsize=1024)
+def _plan(in_dt, dt, B, H, L, D, BLKQ, BLKK, T, keep):
+    """Sizes of one forward: ``(workspace bytes, bytes to keep, offsets)``.  What a backward needs of the forward lies in one
+    allocation (states, look-up table, log-sum-exp, and with ``keep`` map, attention output, the 16-bit copies of
+    fp32 inputs); without a backward the same parts are scratch behind the workspace."""
+    M, N = -(-L // BLKQ), -(-L // BLKK)
+    elems = B * H * L * D
+    parts = {"states": _lib.workspace_bytes(_lib.WS_LINEAR_STATES, dt, B, H, L, D, 64, 64, 0),
+             "lut": B * H * M * T * 4, "lse": B * H * L * 4}
+    if keep:
+        parts["map"] = B * H * M * N
+        parts["o_s"] = elems * 2
+    if in_dt == _lib.SLA_F32:
+        parts["cast"] = 3 * elems * 2
+    ws = -(-_lib.workspace_bytes(_lib.WS_MODULE_FWD, in_dt if in_dt >= 0 else dt, B, H, L, D, BLKQ, BLKK, T) // 256) * 256
+    off, at = {}, 0 if keep else ws
+    for name, n in parts.items():
+        off[name] = at
+        at += -(-n // 256) * 256
+    return ws, at, off
+
+
+def _module_fwd(q, k, v, weight, bias, topk_ratio, BLKQ, BLKK, fmap, dtype, keep, mask=None):
+    """The whole forward as one library call (``sla_module_fwd``).  q, k, v: ``dtype`` (contiguous, or row-contiguous views
+    sharing their strides) or contiguous fp32; ``mask``: a ``(sparse_map, lut)`` built elsewhere.  Returns
+    ``(out in dtype, kept allocation or None, real topk)``."""
+    B, H, L, D = q.shape
+    dev = q.device
+    dt, in_dt = _lib.dtype_code(dtype), _lib.dtype_code(q.dtype)
+    T = topk_count(-(-L // BLKK), topk_ratio)
+    if mask is not None:
+        in_dt = _lib.SLA_MASK_GIVEN
+    ws_bytes, total, off = _plan(in_dt, dt, B, H, L, D, BLKQ, BLKK, T, keep)
+    ws = torch.empty(ws_bytes if keep else total, dtype=torch.uint8, device=dev)
+    saved = torch.empty(total, dtype=torch.uint8, device=dev) if keep else None
+    base = (saved if keep else ws).data_ptr()
+    if mask is not None:
+        sparse_map, lut = mask
+        (saved if keep else ws)[off["lut"]:off["lut"] + lut.numel() * 4].view(torch.int32).copy_(lut.view(-1))
+        if keep:
+            saved[off["map"]:off["map"] + sparse_map.numel()].view(torch.int8).copy_(sparse_map.view(-1))
+    if q.is_contiguous() and k.is_contiguous() and v.is_contiguous():
+        s_in = s_out = None
+        out = torch.empty((B, H, L, D), dtype=dtype, device=dev)
+    else:
+        assert _lib.row_strided(q, k, v), "q, k, v must be contiguous or share row-contiguous strides"
+        out = _lib.empty_like_rows(q)
+        s_in, s_out = _lib.strides_arg(q), _lib.strides_arg(out)
+    rc = _lib.load().sla_module_fwd(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), s_in, in_dt, base + off["cast"] if in_dt == _lib.SLA_F32 else None,
+        weight.data_ptr(), bias.data_ptr(), out.data_ptr(), s_out, base + off["o_s"] if keep else None, base + off["lse"],
+        base + off["map"] if keep else None, base + off["lut"], 4, base + off["states"], dt, _lib.FMAP[fmap], B, H, L, D, BLKQ,
+        BLKK, T, D ** -0.5, ws.data_ptr(), ws_bytes, _lib.stream_ptr(dev), _side_stream(dev))
+    _lib.check(rc)
+    return out, saved, T
+
+
+def _module_bwd_saved(saved, off, q_ptr, k_ptr, v_ptr, s_qkv, d_out, s_do, weight, bias, grads, shape, dtype, T, BLKQ, BLKK, fmap):
+    """Backward from what :func:`_module_fwd` kept; writes ``grads`` (three pointers, laid out like q, k, v) and returns
+    ``(d_weight, d_bias)``."""
+    B, H, L, D = shape
+    dev = saved.device
+    dt = _lib.dtype_code(dtype)
+    n_s = _lib.workspace_bytes(_lib.WS_SPARSE_BWD, dt, B, H, L, D, BLKQ, BLKK, T)
+    n_l = _lib.workspace_bytes(_lib.WS_LINEAR_BWD_STATES_APART, dt, B, H, L, D, 64, 64, 0)
+    n_s = -(-n_s // 256) * 256
+    ws = torch.empty(n_s + n_l, dtype=torch.uint8, device=dev)
+    dwb = torch.empty(D * D + D, dtype=torch.float32, device=dev)
+    base, w0 = saved.data_ptr(), ws.data_ptr()
+    rc = _lib.load().sla_module_bwd_states(
+        q_ptr, k_ptr, v_ptr, s_qkv, base + off["o_s"], d_out.data_ptr(), s_do, base + off["lse"], base + off["map"],
+        base + off["lut"], 4, weight.data_ptr(), bias.data_ptr(), base + off["states"], *grads, dwb.data_ptr(),
+        dwb.data_ptr() + D * D * 4, dt, _lib.FMAP[fmap], B, H, L, D, BLKQ, BLKK, T, D ** -0.5, w0, n_s, w0 + n_s, n_l,
+        _lib.stream_ptr(dev), _side_stream(dev))
+    _lib.check(rc)
+    return dwb[:D * D].view(D, D), dwb[D * D:]
 
 
 class _sla_core(torch.autograd.Function):
@@ -70,34 +154,34 @@ class _sla_core(torch.autograd.Function):
     """
 
     @staticmethod
-    def forward(ctx, q, k, v, weight, bias, sparse_map, lut, topk, BLKQ, BLKK, fmap, state, needs_grad=True):
-        # (row-contiguous views are accepted on the inference path only: the backward kernels take (B, H, L, D))
-        assert (q.is_contiguous() and k.is_contiguous() and v.is_contiguous()) or not needs_grad
-        assert sparse_map.is_contiguous() and lut.is_contiguous()
-        assert BLKQ == 64 or BLKQ == 128
-        assert BLKK == 64
-        qk_scale = q.shape[-1] ** -0.5
-        bias = bias.contiguous()
-        # one kernel: attention over the selected blocks, then the linear branch of the same rows from the
-        # per-head state, projection and sum in its epilogue; o_s is only written when a backward will need it
-        state_ws = state.join()
-        out, o_s, lse = sparse_attn_linear_fwd(q, k, v, lut, topk, BLKQ, BLKK, qk_scale, state_ws, bias, fmap,
-                                               want_o_s=needs_grad)
-        if not needs_grad:
-            return out
-        # the finished states (a few D x D matrices per head) are kept for the backward, the partial sums are not
-        ctx.save_for_backward(q, k, v, weight, bias, sparse_map, lut, lse, o_s, saved_states(state_ws, q))
-        ctx.cfg = (topk, BLKQ, BLKK, fmap, qk_scale)
+    def forward(ctx, q, k, v, weight, bias, topk_ratio, BLKQ, BLKK, fmap, dtype, mask):
+        assert q.is_contiguous() and k.is_contiguous() and v.is_contiguous()
+        out, saved, T = _module_fwd(q, k, v, weight, bias, topk_ratio, BLKQ, BLKK, fmap, dtype, True, mask)
+        if q.dtype == dtype:
+            ctx.save_for_backward(weight, bias, saved, q, k, v)
+        else:                                   # (the backward works on the 16-bit copies among what is kept)
+            ctx.save_for_backward(weight, bias, saved)
+            out = out.to(q.dtype)
+        in_dt = _lib.dtype_code(q.dtype) if mask is None else _lib.SLA_MASK_GIVEN
+        ctx.cfg = (tuple(q.shape), in_dt, T, BLKQ, BLKK, fmap, dtype, q.dtype)
         return out
 
     @staticmethod
     def backward(ctx, d_out):
-        q, k, v, weight, bias, sparse_map, lut, lse, o_s, states = ctx.saved_tensors
-        topk, BLKQ, BLKK, fmap, qk_scale = ctx.cfg
-        d_out = d_out.contiguous()
-        dq, dk, dv, dw, db = module_bwd(q, k, v, o_s, d_out, lse, sparse_map, lut, topk, BLKQ, BLKK, qk_scale, weight, bias,
-                                        fmap, states=states, side_stream=_backward_side_stream(q.device))
-        return dq, dk, dv, dw, db, None, None, None, None, None, None, None, None
+        weight, bias, saved, *qkv = ctx.saved_tensors
+        shape, in_dt, T, BLKQ, BLKK, fmap, dtype, in_dtype = ctx.cfg
+        off = _plan(in_dt, _lib.dtype_code(dtype), *shape, BLKQ, BLKK, T, True)[2]
+        d_out = d_out.contiguous().to(dtype)
+        g = torch.empty((3, *shape), dtype=dtype, device=d_out.device)
+        step = g.stride(0) * g.element_size()
+        g0 = g.data_ptr()
+        if qkv:
+            ptrs = [t.data_ptr() for t in qkv]
+        else:
+            ptrs = [saved.data_ptr() + off["cast"] + i * step for i in range(3)]
+        dw, db = _module_bwd_saved(saved, off, *ptrs, None, d_out, None, weight, bias, (g0, g0 + step, g0 + 2 * step), shape,
+                                   dtype, T, BLKQ, BLKK, fmap)
+        return (*g.to(in_dtype).unbind(0), dw, db, None, None, None, None, None, None)
 
 
 class _sla_complement(torch.autograd.Function):
@@ -142,32 +226,26 @@ class _sla_packed(torch.autograd.Function):
     def forward(ctx, qkv, weight, bias, topk_ratio, BLKQ, BLKK, fmap):
         assert qkv.dim() == 5 and qkv.shape[2] == 3 and qkv.is_contiguous()
         q, k, v = (qkv[:, :, i].permute(0, 2, 1, 3) for i in range(3))          # (B, H, L, D) views
-        weight = weight.contiguous()
-        bias = bias.contiguous()
-        state_ws = _StateBuild(k, v, weight, fmap)
-        sparse_map, lut, topk = get_block_map(q, k, topk_ratio=topk_ratio, BLKQ=BLKQ, BLKK=BLKK)
-        needs_grad = any(ctx.needs_input_grad[:3])
-        qk_scale = q.shape[-1] ** -0.5
-        out, o_s, lse = sparse_attn_linear_fwd(q, k, v, lut, topk, BLKQ, BLKK, qk_scale, state_ws.join(), bias, fmap,
-                                               want_o_s=needs_grad)
-        if needs_grad:
-            ctx.save_for_backward(qkv, weight, bias, sparse_map, lut, lse, o_s, saved_states(state_ws.ws, q))
-            ctx.cfg = (topk, BLKQ, BLKK, fmap, qk_scale)
-        ctx.density = topk / sparse_map.shape[-1]
+        out, saved, T = _module_fwd(q, k, v, weight, bias, topk_ratio, BLKQ, BLKK, fmap, qkv.dtype, True)
+        ctx.save_for_backward(qkv, weight, bias, saved)
+        ctx.cfg = (tuple(q.shape), T, BLKQ, BLKK, fmap)
         return out.permute(0, 2, 1, 3)                                            # (B, L, H, D), contiguous
 
     @staticmethod
     def backward(ctx, d_out):
-        qkv, weight, bias, sparse_map, lut, lse, o_s, states = ctx.saved_tensors
-        topk, BLKQ, BLKK, fmap, qk_scale = ctx.cfg
-        q, k, v = (qkv[:, :, i].permute(0, 2, 1, 3) for i in range(3))
+        qkv, weight, bias, saved = ctx.saved_tensors
+        shape, T, BLKQ, BLKK, fmap = ctx.cfg
+        q = qkv[:, :, 0].permute(0, 2, 1, 3)
         d_out = d_out.permute(0, 2, 1, 3)                                         # (B, H, L, D) view
         if not _lib.row_strided(d_out):
             d_out = d_out.contiguous()
         d_qkv = torch.empty_like(qkv)
-        grads = tuple(d_qkv[:, :, i].permute(0, 2, 1, 3) for i in range(3))
-        _, _, _, dw, db = module_bwd(q, k, v, o_s, d_out, lse, sparse_map, lut, topk, BLKQ, BLKK, qk_scale, weight, bias,
-                                     fmap, states=states, grads=grads, side_stream=_backward_side_stream(qkv.device))
+        dt = _lib.dtype_code(qkv.dtype)
+        off = _plan(dt, dt, *shape, BLKQ, BLKK, T, True)[2]
+        step = shape[1] * shape[3] * qkv.element_size()                           # from a token's q to its k, to its v
+        p, g = qkv.data_ptr(), d_qkv.data_ptr()
+        dw, db = _module_bwd_saved(saved, off, p, p + step, p + 2 * step, _lib.strides_arg(q), d_out, _lib.strides_arg(d_out),
+                                   weight, bias, (g, g + step, g + 2 * step), shape, qkv.dtype, T, BLKQ, BLKK, fmap)
         return d_qkv, dw, db, None, None, None, None
 
 
@@ -284,24 +362,23 @@ class SparseLinearAttention(nn.Module):
             k = k.contiguous()
             v = v.contiguous()
 
-        qc = q.to(self.dtype)
-        kc = k.to(self.dtype)
-        vc = v.to(self.dtype)
         if self.linear_mode == "complement":
-            return self._forward_complement(q, k, qc, kc, vc, dtype, return_sparsity)
+            return self._forward_complement(q, k, q.to(self.dtype), k.to(self.dtype), v.to(self.dtype), dtype, return_sparsity)
         weight = self.proj_l.weight.contiguous()
-        with torch.no_grad():
-            state = _StateBuild(kc, vc, weight, self.feature_map)
-
-        # the mask is built from the inputs in their own dtype (reference core.py:83)
-        sparse_map, lut, real_topk = get_block_map(q, k, topk_ratio=self.topk, BLKQ=self.BLKQ, BLKK=self.BLKK)
-
-        o = _sla_core.apply(qc, kc, vc, weight, self.proj_l.bias, sparse_map, lut, real_topk, self.BLKQ,
-                            self.BLKK, self.feature_map, state, needs_grad)
-        o = o.to(dtype)
-
+        bias = self.proj_l.bias.contiguous()
+        mask = None
+        if not (q.dtype == k.dtype == v.dtype and (dtype == self.dtype or dtype == torch.float32)):
+            # the mask is built from the inputs in their own dtype (reference core.py:83), the rest works on copies
+            with torch.no_grad():
+                mask = get_block_map(q, k, topk_ratio=self.topk, BLKQ=self.BLKQ, BLKK=self.BLKK)[:2]
+            q, k, v = q.to(self.dtype), k.to(self.dtype), v.to(self.dtype)
+        args = (q, k, v, weight, bias, self.topk, self.BLKQ, self.BLKK, self.feature_map, self.dtype)
+        o = _sla_core.apply(*args, mask) if needs_grad else _module_fwd(*args, False, mask)[0]
+        if o.dtype != dtype:
+            o = o.to(dtype)
         if return_sparsity:
-            return o, real_topk / sparse_map.shape[-1]
+            N = -(-q.shape[2] // self.BLKK)
+            return o, topk_count(N, self.topk) / N
         return o
 
     def forward_packed(self, qkv, return_sparsity=False):
@@ -320,8 +397,13 @@ class SparseLinearAttention(nn.Module):
             o = res[0] if return_sparsity else res
             o = o.permute(0, 2, 1, 3)
             return (o, res[1]) if return_sparsity else o
-        o = _sla_packed.apply(qkv.contiguous(), self.proj_l.weight, self.proj_l.bias, self.topk, self.BLKQ, self.BLKK,
-                              self.feature_map)
+        args = (qkv.contiguous(), self.proj_l.weight.contiguous(), self.proj_l.bias.contiguous(), self.topk, self.BLKQ, self.BLKK,
+                self.feature_map)
+        if torch.is_grad_enabled() and any(t.requires_grad for t in args[:3]):
+            o = _sla_packed.apply(*args)
+        else:
+            q, k, v = (args[0][:, :, i].permute(0, 2, 1, 3) for i in range(3))
+            o = _module_fwd(q, k, v, *args[1:], self.dtype, False)[0].permute(0, 2, 1, 3)
         if return_sparsity:
             N = (qkv.shape[1] + self.BLKK - 1) // self.BLKK
             return o, min(N, int(self.topk * N)) / N

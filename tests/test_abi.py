@@ -121,6 +121,16 @@ def test_other_entry_points_validate():
     assert mb(ws_l=8) == _lib.ERR_WORKSPACE
     assert mb(w=None) == _lib.ERR_BAD_ARG
     assert mb(fmap=5) == _lib.ERR_BAD_ARG
+    # the one-call forward
+    mf = lambda **kw: lib.sla_module_fwd(  # noqa: E731
+        FAKE, FAKE, FAKE, kw.get("qs"), kw.get("in_dtype", 1), kw.get("cast"), kw.get("w", FAKE), FAKE, FAKE, None, None, FAKE,
+        None, FAKE, 4, kw.get("states", FAKE), 1, kw.get("fmap", 0), 1, 1, 128, 128, kw.get("BLKQ", 64), 64, kw.get("topk", 1),
+        0.1, FAKE, kw.get("ws", 1 << 30), None, None)
+    assert mf(in_dtype=2) == _lib.ERR_BAD_ARG and "in_dtype" in _lib.last_error()
+    assert mf(in_dtype=0) == _lib.ERR_BAD_ARG and mf(states=None) == _lib.ERR_BAD_ARG and mf(w=None) == _lib.ERR_BAD_ARG
+    assert mf(in_dtype=0, cast=FAKE, qs=(ctypes.c_int64 * 3)(16384, 16384, 128)) == _lib.ERR_BAD_ARG
+    assert mf(ws=8) == _lib.ERR_WORKSPACE and mf(BLKQ=32) == _lib.ERR_UNSUPPORTED
+    assert mf(topk=3) == _lib.ERR_BAD_ARG and mf(fmap=5) == _lib.ERR_BAD_ARG
     assert lib.sage_quant_qk(FAKE, FAKE, 1, 1, 1, 128, 128, 64, 64, FAKE, FAKE, FAKE, FAKE, FAKE, 1 << 30, None) == _lib.ERR_UNSUPPORTED
     assert "BLKQ=128" in _lib.last_error()
     assert lib.sage_quant_v(FAKE, 1, 1, 1, 128, 32, FAKE, FAKE, 448.0, FAKE, 1 << 30, None) == _lib.ERR_UNSUPPORTED

@@ -1,0 +1,44 @@
+"""sla_module_fwd / sla_module_bwd_states (what SparseLinearAttention runs) against the single-step entry points they string
+together: the same bits, below and above the size from which a second stream is used (16 MiB per tensor)."""
+import pytest
+import torch
+
+from sla_amd import SparseLinearAttention, get_block_map
+from sla_amd.inputs import make_proj
+from sla_amd.linear import linear_bwd, linear_state_fwd
+from sla_amd.sparse_attn import sparse_attn_bwd, sparse_attn_linear_fwd
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("H,L,D,BLKQ,in_dtype,half", [
+    (3, 2100, 128, 64, torch.bfloat16, False), (2, 1000, 64, 128, torch.float32, False), (2, 777, 128, 64, torch.float32, True),
+    (2, 640, 64, 64, torch.float16, False),          # a mask from half precision, bf16 compute
+    (12, 6001, 128, 64, torch.bfloat16, False), (24, 6001, 64, 64, torch.float32, True)])
+def test_one_call_equals_the_steps(dev, H, L, D, BLKQ, in_dtype, half):
+    ratio, fmap, dtype = 0.1, "elu" if not half else "softmax", torch.float16 if half else torch.bfloat16
+    g = torch.Generator().manual_seed(L + D)
+    q, k, v, do = (torch.randn(1, H, L, D, generator=g).to(in_dtype).to(dev) for _ in range(4))
+    w, b = (t.to(dev) for t in make_proj(D))
+    mod = SparseLinearAttention(D, ratio, fmap, BLKQ, 64, use_bf16=not half).to(dev)
+    with torch.no_grad():
+        mod.proj_l.weight.copy_(w)
+        mod.proj_l.bias.copy_(b)
+    # the steps, on one stream
+    sparse_map, lut, T = get_block_map(q, k, ratio, BLKQ, 64)
+    qc, kc, vc, dc = (t.to(dtype) for t in (q, k, v, do))
+    state = linear_state_fwd(kc, vc, w, fmap)
+    out, o_s, lse = sparse_attn_linear_fwd(qc, kc, vc, lut, T, BLKQ, 64, D ** -0.5, state, b, fmap, want_o_s=True)
+    ref = sparse_attn_bwd(qc, kc, vc, o_s, dc, lse, sparse_map, lut, T, BLKQ, 64, D ** -0.5)
+    _, _, _, dw, db = linear_bwd(qc, kc, vc, w, b, dc, fmap, accumulate_into=ref)
+    for _ in range(2):                               # (twice: the events between the streams are used again)
+        qg, kg, vg = (t.clone().requires_grad_(True) for t in (q, k, v))
+        mod.zero_grad()
+        o = mod(qg, kg, vg)
+        o.backward(do)
+        assert o.dtype == in_dtype and torch.equal(o.detach(), out.to(in_dtype))
+        with torch.no_grad():
+            assert torch.equal(mod(q, k, v), out.to(in_dtype))
+        for name, t, r in zip(("dq", "dk", "dv"), (qg, kg, vg), ref):
+            assert torch.equal(t.grad, r.to(in_dtype)), name
+        assert torch.equal(mod.proj_l.weight.grad, dw) and torch.equal(mod.proj_l.bias.grad, db)
