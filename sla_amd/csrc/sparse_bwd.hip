@@ -738,8 +738,11 @@ static int bwd_impl(const void* q, const void* k, const void* v, const void* o, 
   const int total_q64 = BH * Mblk64;
   const bool stream_dkdv = D == 128 && (BLKQ == 64 || BLKQ == 128) && (uint64_t)lin.sl * 2u * (uint64_t)L < (1ull << 31) &&
                            (uint64_t)ldo.sl * 2u * (uint64_t)L < (1ull << 31);
-  // (enough query blocks for a wave on every SIMD; the stream kernel keeps a look-up row as 16-bit key block indices)
-  const bool stream_dq = stream_dkdv && topk <= DQ_STREAM_MAX_T && total_q64 >= 1024 && Mblk64 <= 65535;
+  // (The stream kernel keeps a look-up row as 16-bit key block indices.  One wave of it walks a block that the general
+  // kernel gives two waves, and it forms delta itself: with 64-row blocks it is ahead from a wave for every third SIMD on
+  // (whole backward, 324 blocks 62.6 / 65.8 us, 512 blocks 87.2 / 91.8; 260 blocks 54.6 / 53.4); with 128-row blocks, to which
+  // the general kernel gives four waves sharing their tiles, only when every SIMD has one (390 blocks 94.6 / 93.0).)
+  const bool stream_dq = stream_dkdv && topk <= DQ_STREAM_MAX_T && total_q64 >= (wide ? 1024 : 320) && Mblk64 <= 65535;
   // delta = rowsum(dO * O): the dQ kernel of the common shape forms it for its own rows, the general one reads it
   if ((steps & SB_DQ) && !stream_dq)
     hipLaunchKernelGGL((bwd_delta_kernel<Tag, D>), dim3((unsigned)((rows + RPB - 1) / RPB)), dim3(256), 0, st,

@@ -434,13 +434,15 @@ static int launch_fwd(const void* q, const void* k, const void* v, const void* l
   const float c = qk_scale * 1.4426950408889634f;
   // The common shape (head dim 128, 64-row query blocks) has a kernel of its own, which shares key blocks between
   // neighbouring query blocks; it addresses a head with 32-bit byte offsets and indexes key blocks with 12 bits.
-  // (Two query blocks per workgroup halve the number of workgroups: a launch too small to give every compute unit
-  // its two workgroups keeps one query block per workgroup.)
+  // (Two query blocks per workgroup halve the number of workgroups, but a lone workgroup of it still outruns two of the
+  // other kernel on a compute unit.  Measured with iid rows, this kernel against the other, in us with the epilogue:
+  // 260 pairs, 12 key blocks per row 25.4 / 32.1; 192 pairs, 76 key blocks 93 / 135; 162 pairs, 6 key blocks 17.8 / 21.6.
+  // At half a workgroup per compute unit the two meet (132 pairs, 6 key blocks 17.6 / 16.9; 65 pairs, 12: 23.8 / 23.7).)
   // 128-row query blocks go the same way: the two halves of a block are a pair whose rows of the table are one row.
   const int Mblk64 = cdiv(L, 64);
   const int total_p = BH * ((Mblk64 + 1) / 2);
   if (D == 128 && (BLKQ == 64 || BLKQ == 128) && topk <= PAIR_MAX_T && Mblk64 <= 4096 &&
-      (uint64_t)lin.sl * 2u * (uint64_t)L < (1ull << 31) && total_p >= 512) {
+      (uint64_t)lin.sl * 2u * (uint64_t)L < (1ull << 31) && total_p >= PAIR_MIN_PAIRS) {
     const int grid_p = xcd_grid(total_p);
     const int one_row = BLKQ == 128;
     if (fl)

@@ -31,6 +31,7 @@
 namespace sla {
 
 constexpr int PAIR_MAX_T = 1024;      // look-up rows longer than this, or more than 4096 key blocks, take sparse_fwd_kernel
+constexpr int PAIR_MIN_PAIRS = 144;   // as do launches of fewer pairs (measured at its use)
 
 template <typename Tag, bool FUSED>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void sparse_fwd_pair_kernel(
