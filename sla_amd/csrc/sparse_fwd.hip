@@ -432,28 +432,30 @@ static int launch_fwd(const void* q, const void* k, const void* v, const void* l
   const int total = (int)total64;
   const int grid = xcd_grid(total);
   const float c = qk_scale * 1.4426950408889634f;
-  // The common shape (head dim 128, 64-row query blocks) has a kernel of its own, which shares key blocks between
-  // neighbouring query blocks; it addresses a head with 32-bit byte offsets and indexes key blocks with 12 bits.
+  // The common shapes have a kernel of their own, which shares key blocks between neighbouring query blocks; it addresses
+  // a head with 32-bit byte offsets and indexes key blocks with 12 bits.
   // (Two query blocks per workgroup halve the number of workgroups, but a lone workgroup of it still outruns two of the
   // other kernel on a compute unit.  Measured with iid rows, this kernel against the other, in us with the epilogue:
   // 260 pairs, 12 key blocks per row 25.4 / 32.1; 192 pairs, 76 key blocks 93 / 135; 162 pairs, 6 key blocks 17.8 / 21.6.
-  // At half a workgroup per compute unit the two meet (132 pairs, 6 key blocks 17.6 / 16.9; 65 pairs, 12: 23.8 / 23.7).)
+  // At half a workgroup per compute unit the two meet (132 pairs, 6 key blocks 17.6 / 16.9; 65 pairs, 12: 23.8 / 23.7); so
+  // they do at head dim 64 (162 pairs, 12 key blocks 18.1 / 20.9; 130 pairs, 12: 18.2 / 16.9).)
   // 128-row query blocks go the same way: the two halves of a block are a pair whose rows of the table are one row.
   const int Mblk64 = cdiv(L, 64);
   const int total_p = BH * ((Mblk64 + 1) / 2);
-  if (D == 128 && (BLKQ == 64 || BLKQ == 128) && topk <= PAIR_MAX_T && Mblk64 <= 4096 &&
+  if ((BLKQ == 64 || BLKQ == 128) && topk <= PAIR_MAX_T && Mblk64 <= 4096 &&
       (uint64_t)lin.sl * 2u * (uint64_t)L < (1ull << 31) && total_p >= PAIR_MIN_PAIRS) {
     const int grid_p = xcd_grid(total_p);
     const int one_row = BLKQ == 128;
-    if (fl)
-      hipLaunchKernelGGL((sparse_fwd_pair_kernel<Tag, true>), dim3(grid_p), dim3(256), 0, st, (const uint16_t*)q,
-                         (const uint16_t*)k, (const uint16_t*)v, lut, lut64, (uint16_t*)o, lse, lin, lout, L, Mblk64, topk, c,
-                         total_p, fl->kvwt, fl->zst, fl->bias, fl->fmap, fl->o_s, one_row);
-    else
-      hipLaunchKernelGGL((sparse_fwd_pair_kernel<Tag, false>), dim3(grid_p), dim3(256), 0, st, (const uint16_t*)q,
-                         (const uint16_t*)k, (const uint16_t*)v, lut, lut64, (uint16_t*)o, lse, lin, lout, L, Mblk64, topk, c,
-                         total_p, (const uint16_t*)nullptr, (const uint16_t*)nullptr, (const float*)nullptr, 0,
-                         (uint16_t*)nullptr, one_row);
+#define SLA_PAIR_LAUNCH(DD, FUSED)                                                                                          \
+  hipLaunchKernelGGL((sparse_fwd_pair_kernel<Tag, DD, FUSED>), dim3(grid_p), dim3(256), 0, st, (const uint16_t*)q,           \
+                     (const uint16_t*)k, (const uint16_t*)v, lut, lut64, (uint16_t*)o, lse, lin, lout, L, Mblk64, topk, c,   \
+                     total_p, fl ? fl->kvwt : nullptr, fl ? fl->zst : nullptr, fl ? fl->bias : nullptr, fl ? fl->fmap : 0,   \
+                     fl ? fl->o_s : nullptr, one_row)
+    if (D == 128 && fl) SLA_PAIR_LAUNCH(128, true);
+    else if (D == 128) SLA_PAIR_LAUNCH(128, false);
+    else if (fl) SLA_PAIR_LAUNCH(64, true);
+    else SLA_PAIR_LAUNCH(64, false);
+#undef SLA_PAIR_LAUNCH
     return check_launch("sparse_attn_fwd");
   }
 #define SLA_FWD_CASE(DD, BQ)                                                                                          \

@@ -1,6 +1,6 @@
-// Block-sparse FlashAttention forward for 64-row query blocks at head dim 128: two adjacent query blocks per
-// workgroup, two wavefronts per query block (32 query rows each), two workgroups per compute unit, so that every SIMD
-// holds two waves of different workgroups.
+// Block-sparse FlashAttention forward: two adjacent 64-row query blocks per workgroup, two wavefronts per query block (32
+// query rows each), two workgroups per compute unit at head dim 128 and three at head dim 64, so that every SIMD holds
+// two (three) waves of different workgroups.
 //
 // Stands in for _attn_fwd of the reference (sparse_linear_attention/kernel.py:21-82) like sparse_fwd_kernel,
 // whose arithmetic it shares (S^T = K Q^T, thresholded reference maximum, P^T as B operand of O^T = V^T P^T).
@@ -25,6 +25,11 @@
 // m * (qk_scale * log2 e), with the reference maximum's part in one register per lane.  (Scaling Q instead, once, and
 // rounding it to 16 bit again would spare that instruction and shift the log-sum-exp by up to 0.02: too much for the
 // backward pass, which forms its probabilities from it.)
+// Head dim 64 (figures of a unit there in brackets below) has half the products per score and is bound by the vector ALU: 72
+// instructions and 8 products per wave and unit, vector ALU active in 66 % of a SIMD's cycles, matrix pipe in 48 %, at a
+// clock the power limit holds near 1.7 GHz.  Against one query block per workgroup with tiles through registers and
+// three barriers per key block (sparse_fwd_kernel): B1 H40 L32760, 51 key blocks per row 1391 -> 1160 us (944 TFLOP/s), B1 H12
+// L32760, 25: 217 -> 183 us, B2 H16 L7813, 12: 75.9 -> 70.3 us (128-row blocks 72.5 -> 67.0).
 #pragma once
 #include "linear_state.h"
 
@@ -33,16 +38,19 @@ namespace sla {
 constexpr int PAIR_MAX_T = 1024;      // look-up rows longer than this, or more than 4096 key blocks, take sparse_fwd_kernel
 constexpr int PAIR_MIN_PAIRS = 144;   // as do launches of fewer pairs (measured at its use)
 
-template <typename Tag, bool FUSED>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void sparse_fwd_pair_kernel(
+template <typename Tag, int D, bool FUSED>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 3 : 2, D == 64 ? 3 : 2))) void sparse_fwd_pair_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v, const void* __restrict__ lut,
     int lut64, uint16_t* __restrict__ o, float* __restrict__ lse, const RowLayout lin, const RowLayout lout, int L, int Mblk,
     int topk, float scale_log2e, int total, const uint16_t* __restrict__ kvwt, const uint16_t* __restrict__ zst,
     const float* __restrict__ bias, int fmap, uint16_t* __restrict__ o_s, int one_row) {
   using E = Elem<Tag>;
-  constexpr int D = 128, DC = D / 16, DT = D / 32;
+  constexpr int DC = D / 16, DT = D / 32;
   constexpr int ROWB = D * 2;                         // bytes per row in LDS (unpadded)
-  constexpr int SLOT = 32 * ROWB;                     // one half-tile: 8 KB
+  constexpr int SLOT = 32 * ROWB;                     // one half-tile: 8 KB (4 KB at head dim 64)
+  constexpr int LPR = D / 8;                          // lanes (16-byte pieces) per row of a request
+  constexpr int RPI = 64 / LPR;                       // rows one request instruction moves: 4 (8)
+  constexpr int NJ = 8 / RPI;                         // instructions per eight rows: 2 (1)
   constexpr int SSTR = TileRows<D>::SSTR;
   constexpr float PLIM = 1024.0f;   // a lane's 16 probabilities of a unit may sum to this before the reference moves
 
@@ -205,15 +213,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   // as much, its memory address, and its lane part makes up the difference to four rows.  The row the wave's first
   // request starts at is part of the buffer descriptor, formed with scalar instructions (its range ends with the
   // head's last row, so rows past L still lie outside it), not of the vector offset.
+  // (At head dim 64 two rows share the 256 bytes of LDS that all banks span: one instruction covers eight rows, the swizzles
+  //  are row / 2 for K and 4 (row / 2 % 2) + (row / 4) % 2 for V.)
+  auto swz_k = [](int row) __attribute__((always_inline)) { return D == 128 ? row & 15 : (row >> 1) & 7; };
+  auto swz_v = [](int row) __attribute__((always_inline)) {
+    return D == 128 ? ((row & 3) << 2) | ((row >> 2) & 1) : (((row >> 1) & 1) << 2) | ((row >> 2) & 1);
+  };
   const int nunits = 2 * topk;
-  const int lrow = lane >> 4, lslot = lane & 15;
+  const int lrow = lane / LPR, lslot = lane & (LPR - 1);
   const uint32_t smem_addr = (uint32_t)(size_t)smem;      // LDS address of the rings
   const uint32_t row_bytes = pitch * 2;                   // bytes between rows in memory (at least 256)
-  uint32_t koff[2], voff[2];          // lane part of the byte offset of instruction j
+  uint32_t koff[NJ], voff[NJ];        // lane part of the byte offset of instruction j
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    koff[j] = (uint32_t)(4 * j + lrow) * row_bytes + ((lslot ^ ((8 * qt + 4 * j + lrow) & 15)) * 16) - 1024u * j;
-    voff[j] = (uint32_t)(4 * j + lrow) * row_bytes + ((lslot ^ ((lrow << 2) | j)) * 16) - 1024u * j;
+  for (int j = 0; j < NJ; ++j) {
+    koff[j] = (uint32_t)(RPI * j + lrow) * row_bytes + ((lslot ^ swz_k(8 * qt + RPI * j + lrow)) * 16) - 1024u * j;
+    voff[j] = (uint32_t)(RPI * j + lrow) * row_bytes + ((lslot ^ swz_v(RPI * j + lrow)) * 16) - 1024u * j;
   }
   // What the requests of a step need, by kind of step: the byte offset of the first row this wave fetches and the LDS
   // address (inside a generation's slot pair) of its first instruction.
@@ -251,10 +265,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   //  probabilities are 0.  The s_nop is the wait state the hardware wants between a scalar write of M0 and a memory ->
   //  LDS load that reads it.)
 #define SLA_PAIR_FETCH2(RSRC, LANEOFF, DST, RING)                                                                      \
-  asm volatile("s_add_u32 m0, %0, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %3, 0 offen lds\n\t"                                  \
-               "buffer_load_dwordx4 %2, %3, 0 offen offset:1024 lds" ::"s"(DST), "v"((LANEOFF)[0]), "v"((LANEOFF)[1]),   \
-               "s"(RSRC), "n"(RING)                                                                                    \
-               : "memory", "scc")
+  do {                                                                                                                 \
+    if constexpr (D == 128)                                                                                            \
+      asm volatile("s_add_u32 m0, %0, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %3, 0 offen lds\n\t"                  \
+                   "buffer_load_dwordx4 %2, %3, 0 offen offset:1024 lds" ::"s"(DST), "v"((LANEOFF)[0]),                 \
+                   "v"((LANEOFF)[NJ - 1]), "s"(RSRC), "n"(RING)                                                         \
+                   : "memory", "scc");                                                                                 \
+    else                                                                                                               \
+      asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(DST),           \
+                   "v"((LANEOFF)[0]), "s"(RSRC), "n"(RING)                                                              \
+                   : "memory", "scc");                                                                                 \
+  } while (0)
   // all requests of this wave for one half-tile (HALFOFF: byte offset of the half inside the tile)
 #define SLA_PAIR_FETCH_HALF(HEAD, LANEOFF, STEP, HALFOFF, RING)                                                        \
   do {                                                                                                                 \
@@ -262,17 +283,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     SLA_PAIR_FETCH2(rs_, LANEOFF, (STEP).dst, RING);                                                                   \
     if ((STEP).own) {                                                                                                  \
       const u32x4_t rs2_ = rows_from(HEAD, (STEP).rb + (HALFOFF) + sixteen_rows);                       \
-      SLA_PAIR_FETCH2(rs2_, LANEOFF, (STEP).dst, (RING) + 4096);                                                       \
+      SLA_PAIR_FETCH2(rs2_, LANEOFF, (STEP).dst, (RING) + SLOT / 2);                                                   \
     }                                                                                                                  \
   } while (0)
   // fragment addressing (bytes from the start of the rings; the slot of the current kind of step is added when the
   // kind changes)
   int kfo[DC];                      // K fragment c of this lane: row r, piece 2c + g
 #pragma unroll
-  for (int c = 0; c < DC; ++c) kfo[c] = r * ROWB + (((2 * c + g) ^ (r & 15)) * 16);
+  for (int c = 0; c < DC; ++c) kfo[c] = r * ROWB + (((2 * c + g) ^ swz_k(r)) * 16);
   const int tr_row = (lane & 15) >> 2;
   const int v_row = 4 * g + tr_row;                  // + 16 * group (+ 8 for the second read)
-  const int v_swz = ((v_row & 3) << 2) | ((v_row >> 2) & 1);      // (the same for row + 8)
+  const int v_swz = swz_v(v_row);                    // (the same for row + 8)
   int vfo[DT];                      // V^T fragment dt: 8 bytes at element 4 * (lane % 4) of the 16-column strip 2 dt + (lane / 16) % 2
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt) {
@@ -300,6 +321,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   };
 
   // ---- pieces of the arithmetic ----
+  // Score products.  Head dim 128: written as instructions, Q in the accumulation registers (see mfma_scores).  At head dim 64
+  // everything fits the 168 vector registers of three waves per SIMD, and the compiler's own products keep to them.
+  auto score_first = [&](f32x16_t& d, const i16x8_t& a, const i16x8_t& b) __attribute__((always_inline)) {
+    if constexpr (D == 128) {
+      mfma_scores_first<Tag>(d, a, b);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) d[i] = 0.f;
+      d = E::mfma32(a, b, d);
+    }
+  };
+  auto score_next = [&](f32x16_t& d, const i16x8_t& a, const i16x8_t& b) __attribute__((always_inline)) {
+    if constexpr (D == 128) mfma_scores<Tag>(d, a, b);
+    else d = E::mfma32(a, b, d);
+  };
   auto row_max = [&](const f32x16_t& sv) __attribute__((always_inline)) {
     float mx = sv[0];
 #pragma unroll
@@ -324,6 +360,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     // The output accumulators live in the accumulation registers and, on the common path, are only ever touched by
     // MFMAs.  They are scaled in place through one temporary, so that the register allocator has no reason to
     // move the whole accumulator through the vector registers around the loop.
+    if constexpr (D == 64) {
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) oacc[dt][i] *= f;
+      return;
+    }
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");     // (the last products into these registers have landed)
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
@@ -352,7 +395,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   // Q is only ever an MFMA operand and is parked in the accumulation registers: the vector registers are left for the
   // score tiles, the fragments and the softmax arithmetic
 #pragma unroll
-  for (int c = 0; c < DC; ++c) asm volatile("" : "+a"(qf[c]));
+  for (int c = 0; c < DC; ++c)
+    if constexpr (D == 128) asm volatile("" : "+a"(qf[c]));
+    else asm volatile("" : "+v"(qf[c]));      // (the wait for the rows belongs here, not among the requests of the loop)
   if (nunits > 0) {
     cur = step_of(__builtin_amdgcn_readfirstlane(step_lookup(0)));
     nxt = step_of(__builtin_amdgcn_readfirstlane(step_lookup(1)));
@@ -365,8 +410,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     read_k(0, kf);
 #pragma unroll
     for (int c = 0; c < DC; ++c) {
-      if (c == 0) mfma_scores_first<Tag>(s_a, kf[c], qf[c]);
-      else mfma_scores<Tag>(s_a, kf[c], qf[c]);
+      if (c == 0) score_first(s_a, kf[c], qf[c]);
+      else score_next(s_a, kf[c], qf[c]);
     }
     read_k(1, kf);
     point_v(cur.own);
@@ -394,6 +439,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   // Unit u is half HALF of step `cur`; u+1 belongs to `cur` (HALF 0) or `nxt` (HALF 1), u+2 to `nxt`, u+3 to `nxt`
   // (HALF 0) or `nn` (HALF 1); u-1 to the step before `cur` (HALF 0) or to `cur` (HALF 1).
   // (A score product's result is first looked at by the vector ALU eight products after the end of its chain.)
+  constexpr int NS = 2 * DC;        // products (slots) per unit: 16 (8)
+  constexpr int EPS = 16 / NS;      // scores per slot: 1 (2)
+  static_assert(2 * DT == DC, "as many V fragments as K fragments");
   int step_index = 0;
   auto softmax_unit = [&](const f32x16_t& sv, i32x4_t (&pb)[2]) __attribute__((always_inline)) -> float {     // (rare path) all eight pairs of a unit
     float psum = 0.f;
@@ -406,8 +454,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
     return psum;
   };
-  auto read_vf = [&](int gen, int f) __attribute__((always_inline)) {         // fragment f = 4 * group + dt of the V half-tile in `gen`
-    const int gi = f >> 2, dt = f & 3;
+  auto read_vf = [&](int gen, int f) __attribute__((always_inline)) {         // fragment f = DT * group + dt of the V half-tile in `gen`
+    const int gi = f / DT, dt = f % DT;
     const uint8_t* p0 = smem + gen * 2 * SLOT + 16 * gi * ROWB + vfo[dt];
     vf[gi][dt] = concat4(lds_read_tr16(reinterpret_cast<const uint16_t*>(p0)),
                          lds_read_tr16(reinterpret_cast<const uint16_t*>(p0 + 8 * ROWB)));
@@ -434,59 +482,60 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     float t_arg = __builtin_fmaf(s_cur[0], scale_log2e, nmc);      // the exponent's argument is formed a slot ahead of its
     __builtin_amdgcn_sched_barrier(0);                             // exponential, the sum a slot behind it
 #pragma unroll
-    for (int sl = 0; sl < 16; ++sl) {
-      if (sl < 8) {
-        if (sl == 0) mfma_scores_first<Tag>(s_nxt, kf[sl], qf[sl]);
-        else mfma_scores<Tag>(s_nxt, kf[sl], qf[sl]);
+    for (int sl = 0; sl < NS; ++sl) {
+      if (sl < DC) {
+        if (sl == 0) score_first(s_nxt, kf[sl], qf[sl]);
+        else score_next(s_nxt, kf[sl], qf[sl]);
       } else {
-        const int c2 = (sl - 8) >> 2, dt = (sl - 8) & 3;
+        const int c2 = (sl - DC) / DT, dt = (sl - DC) % DT;
         oacc[dt] = E::mfma32(vf[c2][dt], __builtin_bit_cast(i16x8_t, pb_prev[c2]), oacc[dt]);
       }
-      {                                    // one score of unit u: exponential, sum; every second slot packs a pair
+#pragma unroll
+      for (int x = sl * EPS; x < (sl + 1) * EPS; ++x) {      // scores of unit u: exponential, sum; every second one packs a pair
         float e = fast_exp2(t_arg);
         asm volatile("" : "+v"(e));        // (stays in its slot: nothing moves this work towards its first use)
-        if (sl < 15) t_arg = __builtin_fmaf(s_cur[sl + 1], scale_log2e, nmc);
-        if (sl > 0) ps += e_prev;
-        if (sl & 1) {
+        if (x < 15) t_arg = __builtin_fmaf(s_cur[x + 1], scale_log2e, nmc);
+        if (x > 0) ps += e_prev;
+        if (x & 1) {
           uint32_t pw = E::pack2(e_prev, e);
           asm volatile("" : "+v"(pw), "+v"(ps));
-          pb_cur[sl >> 3][(sl >> 1) & 3] = (int)pw;
+          pb_cur[x >> 3][(x >> 1) & 3] = (int)pw;
         }
-        if (sl == 15) ps += e;
+        if (x == 15) ps += e;
         e_prev = e;
       }
       if (sl == 0) {
-        // The requests of the previous iteration have had fourteen slots to land.  After the barrier: V_{u-1} and
+        // The requests of the previous iteration have had all but two of its slots to land.  After the barrier: V_{u-1} and
         // K_{u+2} are visible, and everyone has fetched its fragments of V_{u-2} and K_{u+1}, whose places this
         // iteration's requests overwrite.
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
       }
-      // memory -> LDS: V_u in slot 1, K_{u+3} in slot 5, the further rows of own steps in slot 3 (one branch for both)
+      // memory -> LDS: V_u in slot 1, K_{u+3} in slot 5 (3), the further rows of own steps in slot 3 (2; one branch for both)
       if (sl == 1) {
         const u32x4_t rs = rows_from(v_head, cur.rb + (HALF ? half_bytes : 0u));
         if (gen) SLA_PAIR_FETCH2(rs, voff, cur.dst, 6 * SLOT);
         else SLA_PAIR_FETCH2(rs, voff, cur.dst, 4 * SLOT);
-      } else if (sl == 5) {
+      } else if (sl == (D == 128 ? 5 : 3)) {
         const u32x4_t rs = rows_from(k_head, ks.rb + (HALF ? 0u : half_bytes));
         if (gen) SLA_PAIR_FETCH2(rs, koff, ks.dst, 0 * SLOT);
         else SLA_PAIR_FETCH2(rs, koff, ks.dst, 2 * SLOT);
-      } else if (sl == 3 && __builtin_expect(cur.own | ks.own, 0)) {
+      } else if (sl == (D == 128 ? 3 : 2) && __builtin_expect(cur.own | ks.own, 0)) {
         if (cur.own) {
           const u32x4_t rs = rows_from(v_head, cur.rb + (HALF ? half_bytes : 0u) + sixteen_rows);
-          if (gen) SLA_PAIR_FETCH2(rs, voff, cur.dst, 6 * SLOT + 4096);
-          else SLA_PAIR_FETCH2(rs, voff, cur.dst, 4 * SLOT + 4096);
+          if (gen) SLA_PAIR_FETCH2(rs, voff, cur.dst, 6 * SLOT + SLOT / 2);
+          else SLA_PAIR_FETCH2(rs, voff, cur.dst, 4 * SLOT + SLOT / 2);
         }
         if (ks.own) {
           const u32x4_t rs = rows_from(k_head, ks.rb + (HALF ? 0u : half_bytes) + sixteen_rows);
-          if (gen) SLA_PAIR_FETCH2(rs, koff, ks.dst, 0 * SLOT + 4096);
-          else SLA_PAIR_FETCH2(rs, koff, ks.dst, 2 * SLOT + 4096);
+          if (gen) SLA_PAIR_FETCH2(rs, koff, ks.dst, 0 * SLOT + SLOT / 2);
+          else SLA_PAIR_FETCH2(rs, koff, ks.dst, 2 * SLOT + SLOT / 2);
         }
       }
-      // LDS reads: V_{u-1} fragments in slots 1..8 (used from slot 8 on), K_{u+2} fragments in slots 8..15 (used from
-      // slot 0 of the next iteration on)
-      if (sl >= 1 && sl <= 8) read_vf(gen ^ 1, sl - 1);
-      if (sl >= 8) kf[sl - 8] = *reinterpret_cast<const i16x8_t*>(smem + gen * 2 * SLOT + kfo[sl - 8]);
+      // LDS reads: V_{u-1} fragments in slots 1..DC (used from slot DC on), K_{u+2} fragments in slots DC..2 DC-1 (used
+      // from slot 0 of the next iteration on)
+      if (sl >= 1 && sl <= DC) read_vf(gen ^ 1, sl - 1);
+      if (sl >= DC) kf[sl - DC] = *reinterpret_cast<const i16x8_t*>(smem + gen * 2 * SLOT + kfo[sl - DC]);
       __builtin_amdgcn_sched_barrier(0);
     }
     // rare path (one branch): the probabilities came out too large: move the reference to this unit's maximum and form
@@ -516,7 +565,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   //  a register, or spilled, across the loop)
   int lane_e = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
   asm volatile("" : "+v"(lane_e));
-  const int g_e = lane_e >> 5, r_e = lane_e & 31, lrow_e = lane_e >> 4, lslot_e = lane_e & 15;
+  const int g_e = lane_e >> 5, r_e = lane_e & 31, lrow_e = lane_e / LPR, lslot_e = lane_e & (LPR - 1);
   if (FUSED) {
     // Fused linear branch: the per-head state KVW^T (D x D, 16 bit) goes into the K ring, which nobody reads any more,
     // the way K half-tiles do (rows of 256 bytes, swizzled pieces, each wave requests a quarter), while the last
@@ -527,19 +576,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                       (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32)), (uint32_t)(D * D * 2),
                       0x00020000u};
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int row = 32 * w + 4 * i + lrow_e;                 // (lane part: row 4 (i % 4) + lrow of sixteen, swizzled piece)
-      const uint32_t soff = (uint32_t)(row * ROWB + ((lslot_e ^ ((4 * i + lrow_e) & 15)) * 16));
-      const uint32_t ldst = smem_addr + (uint32_t)((32 * w + 4 * i) * ROWB);
+    for (int i = 0; i < D / 4 / RPI; ++i) {
+      const int row = (D / 4) * w + RPI * i + lrow_e;          // (lane part: row RPI i + lrow of sixteen, swizzled piece)
+      const uint32_t soff = (uint32_t)(row * ROWB + ((lslot_e ^ swz_k(RPI * i + lrow_e)) * 16));
+      const uint32_t ldst = smem_addr + (uint32_t)(((D / 4) * w + RPI * i) * ROWB);
       asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(ldst), "v"(soff), "s"(sth) : "memory");
     }
   }
   if (nunits > 0) {
 #pragma unroll
-    for (int f = 0; f < 8; ++f) read_vf(1, f);
+    for (int f = 0; f < DC; ++f) read_vf(1, f);
 #pragma unroll
-    for (int sl = 0; sl < 8; ++sl) {
-      const int c2 = sl >> 2, dt = sl & 3;
+    for (int sl = 0; sl < DC; ++sl) {
+      const int c2 = sl / DT, dt = sl % DT;
       oacc[dt] = E::mfma32(vf[c2][dt], __builtin_bit_cast(i16x8_t, pb_b[c2]), oacc[dt]);
     }
   }
@@ -582,7 +631,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     // the accumulation registers the loop read them from: left to itself the compiler keeps a second copy of them
     // across the loop for this use.)
 #pragma unroll
-    for (int c = 0; c < DC; ++c) asm volatile("" : "+a"(qf[c]));
+    for (int c = 0; c < DC; ++c)
+      if constexpr (D == 128) asm volatile("" : "+a"(qf[c]));
     const uint16_t* z_h = zst + (size_t)bh * D;
     i16x8_t fq[DC], zreg[DC];
 #pragma unroll
@@ -598,7 +648,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       i16x8_t a[DC];
 #pragma unroll
       for (int c = 0; c < DC; ++c)
-        a[c] = *reinterpret_cast<const i16x8_t*>(smem + (32 * et + r_e) * ROWB + (((2 * c + g_e) ^ (r_e & 15)) * 16));
+        a[c] = *reinterpret_cast<const i16x8_t*>(smem + (32 * et + r_e) * ROWB + (((2 * c + g_e) ^ swz_k(r_e)) * 16));
       f32x16_t acc;
 #pragma unroll
       for (int i = 0; i < 16; ++i) acc[i] = 0.f;
