@@ -21,6 +21,7 @@ constexpr int LB_QUERY = 2;   // dq and the sums over the rows (needs LB_STATES)
 constexpr int LB_REDUCE = 4;  // dS, dz, d_weight, d_bias from those sums (short kernels)
 constexpr int LB_KEYS = 8;    // dk, dv (needs LB_REDUCE)
 constexpr int LB_ALL = 15;
+constexpr int LB_BESIDE = 16; // with LB_REDUCE: the launches run beside dK / dV and have to fit into what it leaves free
 int linear_bwd_steps(const void* q, const void* k, const void* v, const int64_t* qkv_strides, const float* weight,
                      const float* bias, const void* d_out, const int64_t* do_strides, void* dq, void* dk, void* dv,
                      float* d_weight, float* d_bias, int dtype, int fmap, int B, int H, int L, int D, int flags,

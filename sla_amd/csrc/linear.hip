@@ -10,9 +10,9 @@
 //   state_partial : streams K and V once; each workgroup owns a slice of L and forms its
 //                   share of phi(K)^T V on the MFMA (both operands read transposed from LDS)
 //                   and of sum phi(K) on the vector ALU; fp32 partials to the workspace.
-//   state_reduce  : adds the partials in ascending slice order, rounds to 16 bit, stores the
-//                   state TRANSPOSED (KVT[d2][d1]) so the next kernel reads MFMA rows directly.
-//   fold          : KVW = KV W^T per head (16 bit), so numerator and projection are one product.
+//   state_finish  : adds the partials in ascending slice order, rounds to 16 bit, stores the
+//                   state TRANSPOSED (KVT[d2][d1]) so the next kernel reads MFMA rows directly, and forms
+//                   KVW = KV W^T per head (16 bit), so that numerator and projection are one product.
 //   out           : one wavefront per 32 queries.  OUT^T = KVW^T phi(Q)^T is formed transposed so the
 //                   per-query divisor is a per-lane scalar; the tile is scaled, biased, parked in LDS
 //                   and written (plus the residual) with whole-row 16-byte accesses.
@@ -120,9 +120,7 @@ template <typename Tag, int D>
 static int linear_state_impl(const void* k, const void* v, const RowLayout& lay, const float* weight, int fmap, int BH, int L,
                              char* ws, char* parts, hipStream_t st) {
   const LinWs w = lin_ws(BH, L, D);
-  launch_state_build<Tag, D>(k, v, lay, weight, fmap, BH, L, ws, parts, w, st, false);
-  hipLaunchKernelGGL((linear_fold_kernel<Tag>), dim3(D / (1024 / D), BH), dim3(256), 0, st,
-                     (const uint16_t*)(ws + w.kvt), weight, (uint16_t*)(ws + w.kvwt), (uint16_t*)(ws + w.wt), D);
+  launch_state_build<Tag, D>(k, v, lay, weight, fmap, BH, L, ws, parts, w, st);
   return check_launch("linear_state_fwd");
 }
 
@@ -151,11 +149,7 @@ static int linear_state_quant_v_impl(const void* k, const void* v, const RowLayo
   int rc = quant_v_from_partial_amax(v, lay, dtype, BH, L, D, (const float*)(ws + w.vmax_part), w.nsplit, v_fp8, v_scale,
                                      v_range, st);
   if (rc) return rc;
-  hipLaunchKernelGGL((linear_state_reduce_kernel<Tag>), dim3(cdiv(D * D, 256), BH), dim3(256), 0, st,
-                     (const float*)(ws + w.kv_part), (const float*)(ws + w.z_part), (uint16_t*)(ws + w.kvt),
-                     (uint16_t*)(ws + w.kvp), (uint16_t*)(ws + w.z), w.nsplit, D * D, D);
-  hipLaunchKernelGGL((linear_fold_kernel<Tag>), dim3(D / (1024 / D), BH), dim3(256), 0, st,
-                     (const uint16_t*)(ws + w.kvt), weight, (uint16_t*)(ws + w.kvwt), (uint16_t*)(ws + w.wt), D);
+  launch_state_finish<Tag, D>(weight, BH, ws, ws + w.states_end, w, st);
   return check_launch("linear_state_quant_v_fwd");
 }
 

@@ -601,8 +601,7 @@ static LinBwdWs lin_bwd_ws(int BH, int L, int D, bool own_states) {
   w.y = off;       off += align_up(rows * D * 2, 256);
   w.dden = off;    off += align_up(rows * 4, 256);
   w.ds_part = off; off += align_up(np * D * D * 4, 256);
-  // (the stream path keeps M of every head there in both orientations: two matrices per head at least)
-  w.dw_part = off; off += align_up((np > 2 * BH ? np : 2 * (int64_t)BH) * D * D * 4, 256);
+  w.dw_part = off; off += align_up(D == 128 ? 0 : np * D * D * 4, 256);
   w.dz_part = off; off += align_up(np * D * 4, 256);
   w.db_part = off; off += align_up(np * D * 4, 256);
   w.ds = off;      off += align_up((int64_t)BH * D * D * 2, 256);
@@ -625,9 +624,7 @@ static int linear_bwd_impl(const void* q, const void* k, const void* v, const fl
   const int accumulate = flags & SLA_BWD_ACCUMULATE;
   if ((steps & LB_STATES) && !states && !(flags & SLA_BWD_STATES_READY)) {
     // everything the forward's state build leaves: transposed state, z, and (fold) the folded state + 16-bit weight
-    launch_state_build<Tag, D>(k, v, lin, weight, fmap, BH, L, ws, ws + w.fwd.states_end, w.fwd, st, false);
-    hipLaunchKernelGGL((linear_fold_kernel<Tag>), dim3(D / (1024 / D), BH), dim3(256), 0, st,
-                       (const uint16_t*)(ws + w.fwd.kvt), weight, (uint16_t*)(ws + w.fwd.kvwt), (uint16_t*)(ws + w.fwd.wt), D);
+    launch_state_build<Tag, D>(k, v, lin, weight, fmap, BH, L, ws, ws + w.fwd.states_end, w.fwd, st);
   }
   if (!states) states = ws;
   const uint16_t* kvt = (const uint16_t*)(states + w.fwd.kvt);
@@ -639,11 +636,8 @@ static int linear_bwd_impl(const void* q, const void* k, const void* v, const fl
   bool streamed = false;
   if constexpr (D == 128) streamed = fits32(lin) && fits32(ldo);
   if constexpr (D == 128) if (streamed) {
-    // q and G once: dq, and the partial sums M^T, dz, db of every slice (the slices' partials and the per-head M^T
-    // take the places of the two-matrix partials of the general path: ds_part, dw_part)
+    // q and G once: dq, and the partial sums M^T, dz, db of every slice (M^T's take the place of the general path's ds_part)
     float* m_part = (float*)(ws + w.ds_part);
-    float* mt_head = (float*)(ws + w.dw_part);
-    float* m_head = mt_head + (size_t)BH * D * D;
     if (steps & LB_QUERY) {
 #define SLA_LBS_LAUNCH(FM)                                                                                                  \
   hipLaunchKernelGGL((linear_bwd_stream_kernel<Tag, FM>), dim3(w.ss.nsplit, BH), dim3(512), 0, st, (const uint16_t*)q,        \
@@ -655,11 +649,14 @@ static int linear_bwd_impl(const void* q, const void* k, const void* v, const fl
 #undef SLA_LBS_LAUNCH
     }
     if (steps & LB_REDUCE) {
-    hipLaunchKernelGGL(linear_bwd_sum_kernel, dim3(cdiv(D * D, 256), BH), dim3(256), 0, st, (const float*)m_part,
-                       (const float*)(ws + w.dz_part), (const float*)(ws + w.db_part), mt_head, m_head, (float*)(ws + w.dz),
-                       (float*)(ws + w.db_head), w.ss.nsplit, D);
-    hipLaunchKernelGGL((linear_bwd_products_kernel<Tag>), dim3(D * D / 256, BH, 2), dim3(256), 0, st, (const float*)mt_head,
-                       (const float*)m_head, weight, kvt, (uint16_t*)(ws + w.ds), (uint16_t*)(ws + w.dst), (float*)(ws + w.dw_head), D);
+#define SLA_LBF_LAUNCH(HALVES)                                                                                               \
+  hipLaunchKernelGGL((linear_bwd_finish_kernel<Tag, D, HALVES>), dim3(xcd_grid((int64_t)BH * (D / 8))), dim3(256 * HALVES), 0, \
+                     st, (const float*)m_part, (const float*)(ws + w.dz_part), (const float*)(ws + w.db_part), weight, kvt,   \
+                     (uint16_t*)(ws + w.ds), (uint16_t*)(ws + w.dst), (float*)(ws + w.dz), (float*)(ws + w.dw_head),           \
+                     (float*)(ws + w.db_head), w.ss.nsplit, BH * (D / 8))
+    if (steps & LB_BESIDE) SLA_LBF_LAUNCH(1);
+    else SLA_LBF_LAUNCH(2);
+#undef SLA_LBF_LAUNCH
     }
   }
   if (!streamed) {

@@ -14,8 +14,8 @@
 //              (16x16x32 products, the row spread over 4 lanes), leaves a/den and dq in LDS; then the workgroup adds the
 //              tile's (a/den)^T G to M (32x32x16 products, both operands read transposed from LDS), dz and db on the
 //              vector ALU, and writes the dq rows whole.
-//   reduce   : fixed-order sums of the slices' partials -> M^T (fp32), dz, db per head
-//   products : dS = M W (16 bit, both orientations) and this head's dW = M^T S (fp32)
+//   finish   : fixed-order sums of the slices' partials -> M^T (fp32), dz, db per head, and from them
+//              dS = M W (16 bit, both orientations) and this head's dW = M^T S (fp32)
 #pragma once
 #include "linear_state.h"
 
@@ -585,85 +585,120 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   }
 }
 
-// Sums of the slices' partials in ascending slice order: M per head (fp32, both orientations), dz, db per head.
-// grid (cdiv(D*D, 256), BH).
-__global__ __launch_bounds__(256) void linear_bwd_sum_kernel(const float* __restrict__ m_part, const float* __restrict__ dz_part,
-                                                             const float* __restrict__ db_part, float* __restrict__ mt_head,
-                                                             float* __restrict__ m_head, float* __restrict__ dz,
-                                                             float* __restrict__ db_head, int nsplit, int D) {
-  const int DD = D * D;
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  const int bh = blockIdx.y;
-  if (i < DD) {
-    const float* p = m_part + (size_t)bh * nsplit * DD + i;
-    float s = 0.f;
-#pragma unroll 8
-    for (int sp = 0; sp < nsplit; ++sp) s += p[(size_t)sp * DD];
-    mt_head[(size_t)bh * DD + i] = s;                               // M^T [e][d1]
-    m_head[(size_t)bh * DD + (size_t)(i % D) * D + i / D] = s;      // M   [d1][e]
-  }
-  if (i < D) {
-    const float* p = dz_part + (size_t)bh * nsplit * D + i;
-    const float* pb = db_part + (size_t)bh * nsplit * D + i;
-    float s = 0.f, sb = 0.f;
-    for (int sp = 0; sp < nsplit; ++sp) {
-      s += p[(size_t)sp * D];
-      sb += pb[(size_t)sp * D];
-    }
-    dz[(size_t)bh * D + i] = s;
-    db_head[(size_t)bh * D + i] = sb;
-  }
-}
-
-// Per head, from M (fp32, both orientations):
+// From the slices' partials of a head (fp32, [e][d1]), added in ascending slice order to M^T, dz, db:
 //   dS[d1][d2]    = sum_e  M^T[e][d1] * round16(W[e][d2])    -> ds [d1][d2] and dst [d2][d1], 16 bit
 //   dW^T[d2][e]   = sum_d1 M[d1][e] * S[d1][d2]              -> dw_head [d2][e], fp32  (S^T = kvt[d2][d1], 16 bit)
-// grid (D*D/256, BH, 2): z = 0 forms dS, z = 1 forms dW.  Ascending order of the summed index; a workgroup's threads
-// share the first factor and read the second side by side.
-template <typename Tag>
-__global__ __launch_bounds__(256) void linear_bwd_products_kernel(const float* __restrict__ mt_head,
-                                                                  const float* __restrict__ m_head,
-                                                                  const float* __restrict__ weight,
-                                                                  const uint16_t* __restrict__ kvt, uint16_t* __restrict__ ds,
-                                                                  uint16_t* __restrict__ dst, float* __restrict__ dw_head,
-                                                                  int D) {
+// M stays in fp32 and meets the other factor on the fp32 matrix product (16x16x4).  One workgroup per head, sixteen indices
+// and kind (neighbouring workgroups on one XCD):
+//   kind 0: sums the columns d1 = i0 .. + 15 of every row e and forms 16 rows of dS;
+//   kind 1: sums the rows e = i0 .. + 15 and forms 16 columns of dW^T.
+// Either way it holds all its products need of M after one hand-over through LDS; the partials are read twice, from the
+// caches.  The slices are summed in two halves, whose sums are then added:
+//   HALVES 2: 512 threads, the halves side by side, eight slices' loads in flight: for a launch that has the chip to itself;
+//   HALVES 1: 256 threads, one half after the other, at most 72 registers per lane: what the dK/dV kernel of head dim 128
+//             leaves free beside its two workgroups on a compute unit (with more the launch would only get its turn when
+//             dK/dV is done).  The same bits.
+// Against a kernel for the sums and one for the products (on the vector ALU, M through memory in both orientations): 9.3
+// against 12.8 + 10.5 us (B2 H4 L4096), beside dK/dV 18 against 14 + 37 us (B1 H12 L9360) and 25 against 19 + 46 (L32760).
+template <typename Tag, int D, int HALVES>
+__global__ __launch_bounds__(256 * HALVES) __attribute__((amdgpu_waves_per_eu(HALVES == 2 ? 4 : 7))) void linear_bwd_finish_kernel(
+    const float* __restrict__ m_part, const float* __restrict__ dz_part, const float* __restrict__ db_part,
+    const float* __restrict__ weight, const uint16_t* __restrict__ kvt, uint16_t* __restrict__ ds, uint16_t* __restrict__ dst,
+    float* __restrict__ dz, float* __restrict__ dw_head, float* __restrict__ db_head, int nsplit, int total) {
   using E = Elem<Tag>;
-  const int DD = D * D;
-  const int bh = blockIdx.y;
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= DD) return;
-  if (blockIdx.z == 0) {
-    const int d1 = i / D, d2 = i % D;
-    const float* m = mt_head + (size_t)bh * DD + d1;
-    const float* w = weight + d2;
-    float acc = 0.f;
-    for (int e0 = 0; e0 < D; e0 += 16) {       // (16 pairs of loads in flight, then their products in order)
-      float a[16], b[16];
+  constexpr int DD = D * D;
+  constexpr int NR = D / 64;               // f32x4 sums per thread
+  constexpr int KQ = D / 4;                // products per tile: four summed indices each
+  constexpr int EP = D + 1;                // row pitch of the strip of rows
+  constexpr int NT = HALVES == 2 ? 1 : NR; // 16-wide tiles per wave
+  constexpr int BATCH = HALVES == 2 ? 8 : 4;
+  __shared__ __attribute__((aligned(16))) float s_half[HALVES == 2 ? NR * 256 * 4 : 4];
+  __shared__ __attribute__((aligned(16))) float sm[16 * EP];
+  const int logical = xcd_remap(blockIdx.x, gridDim.x, total);
+  if (logical < 0) return;
+  const int bh = logical / (D / 8), rest = logical % (D / 8), kind = rest / (D / 16), i0 = 16 * (rest % (D / 16));
+  const int tid = threadIdx.x & 255, half = threadIdx.x >> 8, lane = tid & 63, wave = threadIdx.x >> 6;
+  const int l = lane & 15, h = lane >> 4;
+  const int n0 = (nsplit + 1) >> 1;
+  const float* mp = m_part + (size_t)bh * nsplit * DD;
+  const int er = kind == 0 ? tid >> 2 : tid >> 4, dc = kind == 0 ? 4 * (tid & 3) : 4 * (tid & 15);
+  mp += kind == 0 ? (size_t)er * D + i0 + dc : (size_t)(i0 + er) * D + dc;
+  const size_t vec = kind == 0 ? (size_t)64 * D : 64;
+  f32x4_t acc[NR], acc2[NR];
 #pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        a[j] = m[(size_t)(e0 + j) * D];
-        b[j] = w[(size_t)(e0 + j) * D];
-      }
+  for (int i = 0; i < NR; ++i) {
+    acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    acc2[i] = acc[i];
+  }
+  if (HALVES == 2) {
+    sum_slices<NR, BATCH>(mp + (half ? (size_t)n0 * DD : 0), half ? nsplit - n0 : n0, DD, vec, acc);
+    if (half)
 #pragma unroll
-      for (int j = 0; j < 16; ++j) acc = __builtin_fmaf(a[j], round16<Tag>(b[j]), acc);
-    }
-    const uint16_t hv = E::from_float(acc);
-    ds[(size_t)bh * DD + i] = hv;
-    dst[(size_t)bh * DD + (size_t)d2 * D + d1] = hv;
+      for (int i = 0; i < NR; ++i) *reinterpret_cast<f32x4_t*>(s_half + (i * 256 + tid) * 4) = acc[i];
   } else {
-    const int d2 = i / D, e = i % D;
-    const uint16_t* s = kvt + (size_t)bh * DD + (size_t)d2 * D;
-    const float* m = m_head + (size_t)bh * DD + e;
-    float acc = 0.f;
-    for (int d0 = 0; d0 < D; d0 += 16) {
-      float a[16];
-      const i16x8_t s0 = *reinterpret_cast<const i16x8_t*>(s + d0), s1 = *reinterpret_cast<const i16x8_t*>(s + d0 + 8);
+    sum_slices<NR, BATCH>(mp, n0, DD, vec, acc);
+    sum_slices<NR, BATCH>(mp + (size_t)n0 * DD, nsplit - n0, DD, vec, acc2);
+  }
+  if (kind == 0 && half == HALVES - 1 && tid < 32) {
+    const float* q = (tid < 16 ? dz_part : db_part) + (size_t)bh * nsplit * D + i0 + (tid & 15);
+    float sum = 0.f;
+#pragma unroll 8
+    for (int sp = 0; sp < nsplit; ++sp) sum += q[(size_t)sp * D];
+    (tid < 16 ? dz : db_head)[(size_t)bh * D + i0 + (tid & 15)] = sum;
+  }
+  if (HALVES == 2) __syncthreads();
+  if (!half)
 #pragma unroll
-      for (int j = 0; j < 16; ++j) a[j] = m[(size_t)(d0 + j) * D];
+    for (int i = 0; i < NR; ++i) {
+      if (HALVES == 2) acc2[i] = *reinterpret_cast<const f32x4_t*>(s_half + (i * 256 + tid) * 4);
+      acc[i] += acc2[i];
+      if (kind == 0) {
+        *reinterpret_cast<f32x4_t*>(sm + (er + 64 * i) * 16 + dc) = acc[i];                    // [e][d1]
+      } else {
 #pragma unroll
-      for (int j = 0; j < 16; ++j) acc = __builtin_fmaf(a[j], E::to_float((uint16_t)(j < 8 ? s0[j] : s1[j - 8])), acc);
+        for (int j = 0; j < 4; ++j) sm[er * EP + dc + 64 * i + j] = acc[i][j];                 // [e][d1]
+      }
     }
-    dw_head[(size_t)bh * DD + i] = acc;      // [d][e] with d = d2: the layout linear_bwd_reduce_heads_kernel adds up
+  __syncthreads();
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    const int tile = NT * wave + t;
+    if (tile >= D / 16) break;
+    f32x4_t o = {0.f, 0.f, 0.f, 0.f};
+    if (kind == 0) {
+      // row d1 = l of M, column d2 = 16 tile + l of W; summed index e = 4 kk + h
+      const int d2 = 16 * tile + l;
+#pragma unroll
+      for (int k0 = 0; k0 < KQ; k0 += 16) {
+        float wb[16];
+#pragma unroll
+        for (int x = 0; x < 16; ++x) wb[x] = weight[(size_t)(4 * (k0 + x) + h) * D + d2];
+#pragma unroll
+        for (int x = 0; x < 16; ++x)
+          o = __builtin_amdgcn_mfma_f32_16x16x4f32(sm[(4 * (k0 + x) + h) * 16 + l], round16<Tag>(wb[x]), o, 0, 0, 0);
+      }
+      // rows d1 = 4 h + i, column d2
+      i32x2_t w;
+      w[0] = (int)E::pack2(o[0], o[1]);
+      w[1] = (int)E::pack2(o[2], o[3]);
+      *reinterpret_cast<i32x2_t*>(dst + (size_t)bh * DD + (size_t)d2 * D + i0 + 4 * h) = w;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        ds[(size_t)bh * DD + (size_t)(i0 + 4 * h + i) * D + d2] = (uint16_t)((uint32_t)w[i >> 1] >> (16 * (i & 1)));
+    } else {
+      // row d2 = 16 tile + l of S^T, column e = l of M; summed index d1 = KQ h + kk (adjacent per lane)
+      const uint16_t* st = kvt + (size_t)bh * DD + (size_t)(16 * tile + l) * D + KQ * h;
+#pragma unroll
+      for (int c = 0; c < KQ / 8; ++c) {
+        const i16x8_t sf = *reinterpret_cast<const i16x8_t*>(st + 8 * c);
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          o = __builtin_amdgcn_mfma_f32_16x16x4f32(E::to_float((uint16_t)sf[j]), sm[l * EP + KQ * h + 8 * c + j], o, 0, 0, 0);
+      }
+      // rows d2 = 16 tile + 4 h + i, column e: the layout linear_bwd_reduce_heads_kernel adds up
+#pragma unroll
+      for (int i = 0; i < 4; ++i) dw_head[(size_t)bh * DD + (size_t)(16 * tile + 4 * h + i) * D + i0 + l] = o[i];
+    }
   }
 }
 

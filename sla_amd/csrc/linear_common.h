@@ -169,10 +169,10 @@ struct LinSplit {
 };
 // Slices of the sequence for the kernels that reduce over L: as many (head, slice) workgroups as fit the chip at
 // once (`slots` = 256 compute units x workgroups per unit), never more, so there is no second, part-filled round.
-// Slices are multiples of `gran` rows (the rows a kernel takes per step).
-static inline LinSplit lin_split(int BH, int L, int slots = 768, int gran = 64) {
+// Slices are multiples of `gran` rows (the rows a kernel takes per step) and at least `min_rows` long.
+static inline LinSplit lin_split(int BH, int L, int slots = 768, int gran = 64, int min_rows = 0) {
   int nsplit = slots / BH;
-  const int max_split = cdiv(L, gran);
+  const int max_split = cdiv(L, min_rows > gran ? min_rows : gran);
   if (nsplit > max_split) nsplit = max_split;
   if (nsplit < 1) nsplit = 1;
   LinSplit s;

@@ -199,40 +199,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
   }
 }
 
-// ---- kernel 2: reduce partials, round to 16 bit -------------------------------------------
 // Position of column d2 inside a row whose columns are re-ordered to the accumulator slot order of the
 // 32x32 MFMA: slot j of 16-column chunk c, lane group gg  <->  d2 = 16c + 8*(j/4) + 4gg + j%4.
 static __device__ __host__ __forceinline__ int slot_order_pos(int d2) {
   const int c = d2 >> 4, w16 = d2 & 15;
   const int gg = (w16 >> 2) & 1, j = ((w16 >> 3) << 2) | (w16 & 3);
   return 16 * c + 8 * gg + j;
-}
-
-// kvt[bh][d2][d1] (transposed state) and kvp[bh][d1][slot order of d2] (for the backward's S dn^T product)
-template <typename Tag>
-__global__ void linear_state_reduce_kernel(const float* __restrict__ kv_part, const float* __restrict__ z_part,
-                                           uint16_t* __restrict__ kvt, uint16_t* __restrict__ kvp, uint16_t* __restrict__ z,
-                                           int nsplit, int DD, int D) {
-  using E = Elem<Tag>;
-  const int bh = blockIdx.y;
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < DD) {
-    const float* p = kv_part + (size_t)bh * nsplit * DD + i;
-    float s = 0.f;
-#pragma unroll 8
-    for (int sp = 0; sp < nsplit; ++sp) s += p[(size_t)sp * DD];
-    const uint16_t h = E::from_float(s);
-    kvt[(size_t)bh * DD + i] = h;
-    const int d2 = i / D, d1 = i % D;
-    kvp[(size_t)bh * DD + d1 * D + slot_order_pos(d2)] = h;
-  }
-  if (i < D) {
-    const float* p = z_part + (size_t)bh * nsplit * D + i;
-    float s = 0.f;
-#pragma unroll 8
-    for (int sp = 0; sp < nsplit; ++sp) s += p[(size_t)sp * D];
-    z[(size_t)bh * D + i] = E::from_float(s);
-  }
 }
 
 // 16-bit transposed copy of the projection weight: wt[d][e] (A operand of dY^T = W^T G^T).
@@ -247,51 +219,140 @@ __global__ void linear_prep_weight_kernel(const float* __restrict__ weight, uint
   wt[d * D + e] = h;
 }
 
-// ---- kernel 3 (forward, and a backward that has to rebuild the states): fold the projection into the state -------------------------------------------------
-// kvwt[bh][e][d1] = round16( sum_d2 round16(W[e][d2]) * KVT[d2][d1] ), fp32 accumulation in ascending d2.
+// ---- kernel 2 (forward, and a backward that has to rebuild the states): finish the states ----------------------------
+// From the slices' partial states of a head: their sums in ascending slice order, rounded to 16 bit (kvt, the transposed
+// state; kvp, its transpose in slot order, which only the head-dim-64 backward reads; z), and with the projection folded in
+//   kvwt[bh][e][d1] = round16( sum_d2 round16(W[e][d2]) * KVT[d2][d1] ), fp32 accumulation:
 // (phi(Q) KV / den) W^T = (phi(Q) (KV W^T)) / den, so the output kernel needs one product per query tile.
-// grid (D / (1024 / D), BH), 256 threads: a workgroup forms 1024 / D rows e for all d1, thread = (row e, four adjacent d1).
-// It sits between the state kernels and the attention kernel with nothing to overlap it, and its arithmetic is nothing:
-// the head's state and the workgroup's rows of W come into LDS with every load in flight at once, the sums then run
-// out of LDS.
-// The workgroups of head 0 also leave the 16-bit transposed weight wt[d][e] that a backward reads (what
-// linear_prep_weight_kernel writes), which saves the forward one launch in its chain of small kernels.
-template <typename Tag>
-__global__ __launch_bounds__(256) void linear_fold_kernel(const uint16_t* __restrict__ kvt, const float* __restrict__ weight,
-                                                          uint16_t* __restrict__ kvwt, uint16_t* __restrict__ wt, int D) {
+// One workgroup of 512 threads per head and 16 columns d1 (neighbouring workgroups on one XCD, so that the two halves of a
+// 128-byte line meet in its L2): the two halves of the workgroup sum one half of the slices each, over every row d2, and meet
+// in LDS; holding all a row of kvwt needs of the state, the workgroup then multiplies by W on the matrix cores.  Bound by
+// latency: the loads of eight slices and the workgroup's rows of W are in flight at once.  The workgroups of head 0 also
+// leave the 16-bit transposed weight wt[d][e] that a backward reads.
+// Against a summing and a folding kernel (the latter on the vector ALU), B1 H12 L9360 D128: 16.3 against 10.1 + 8.5 us and one
+// launch less; state build of 40 heads x 32760 x 128: 159 against 172 us, of 16 heads x 6001 x 64: 17.5 against 20.9.
+template <int NV, int BATCH = 8>
+static __device__ __forceinline__ void sum_slices(const float* __restrict__ p, int n, size_t slice_stride, size_t vec_stride,
+                                                  f32x4_t (&acc)[NV]) {
+  // acc[i] += the 16 bytes at p + i vec_stride of n slices, in ascending order, BATCH slices' loads in flight
+  int sp = 0;
+  for (; sp + BATCH <= n; sp += BATCH) {
+    f32x4_t b[BATCH][NV];
+#pragma unroll
+    for (int x = 0; x < BATCH; ++x)
+#pragma unroll
+      for (int i = 0; i < NV; ++i) b[x][i] = *reinterpret_cast<const f32x4_t*>(p + (size_t)(sp + x) * slice_stride + i * vec_stride);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int x = 0; x < BATCH; ++x)
+#pragma unroll
+      for (int i = 0; i < NV; ++i) acc[i] += b[x][i];
+  }
+  if (sp < n) {                      // the rest: the last slice again where there is none, not added
+    f32x4_t b[BATCH][NV];
+#pragma unroll
+    for (int x = 0; x < BATCH; ++x)
+#pragma unroll
+      for (int i = 0; i < NV; ++i)
+        b[x][i] = *reinterpret_cast<const f32x4_t*>(p + (size_t)min(sp + x, n - 1) * slice_stride + i * vec_stride);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int x = 0; x < BATCH; ++x)
+      if (sp + x < n) {
+#pragma unroll
+        for (int i = 0; i < NV; ++i) acc[i] += b[x][i];
+      }
+  }
+}
+
+template <typename Tag, int D>
+__global__ __launch_bounds__(512) void linear_state_finish_kernel(const float* __restrict__ kv_part,
+                                                                  const float* __restrict__ z_part,
+                                                                  const float* __restrict__ weight, uint16_t* __restrict__ kvt,
+                                                                  uint16_t* __restrict__ kvp, uint16_t* __restrict__ kvwt,
+                                                                  uint16_t* __restrict__ z, uint16_t* __restrict__ wt, int nsplit,
+                                                                  int total) {
   using E = Elem<Tag>;
-  __shared__ __attribute__((aligned(16))) uint16_t s_kv[128 * 128];      // [d2][d1]
-  __shared__ float s_w[16 * 128];                                          // [row][d2], rounded to 16 bit
-  const int bh = blockIdx.y, tid = threadIdx.x;
-  const int groups = D >> 2;                       // threads per row e
-  const int rows = 256 / groups;                   // rows e per workgroup (8 at D 128, 16 at D 64)
-  const int e0 = blockIdx.x * rows;
-  const uint16_t* src = kvt + (size_t)bh * D * D;
-  for (int i = tid; i < D * D / 8; i += 256)
-    reinterpret_cast<i16x8_t*>(s_kv)[i] = reinterpret_cast<const i16x8_t*>(src)[i];
-  for (int i = tid; i < rows * D; i += 256) {
-    const float wv = weight[(size_t)e0 * D + i];
-    s_w[i] = round16<Tag>(wv);
-    if (bh == 0) {
-      const int e = e0 + i / D, d = i % D;
-      wt[d * D + e] = E::from_float(wv);
+  constexpr int DD = D * D;
+  constexpr int STR = D + 8;               // row pitch of the strip in LDS
+  constexpr int NR = D / 64;               // rows d2 per thread
+  __shared__ __attribute__((aligned(16))) float s_half[NR * 256 * 4];     // sums of the upper half of the slices
+  __shared__ __attribute__((aligned(16))) uint16_t s_kv[16 * STR];        // [d1][d2]
+  const int logical = xcd_remap(blockIdx.x, gridDim.x, total);
+  if (logical < 0) return;
+  const int bh = logical / (D / 16), d1_0 = 16 * (logical % (D / 16));
+  const int tid = threadIdx.x & 255, half = threadIdx.x >> 8, lane = tid & 63, wave = threadIdx.x >> 6;
+  const int l = lane & 15, h = lane >> 4;
+  const int tile = wave < D / 16 ? wave : 0;         // 16 rows e per wave (head dim 64: four of the eight waves)
+
+  // B operand of (KV W^T)^T = KV^T-strip x W^T: column e = 16 tile + l, rows d2 = 32 c + 8 h ..
+  f32x4_t wraw[D / 32][2];
+#pragma unroll
+  for (int c = 0; c < D / 32; ++c)
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+      wraw[c][x] = *reinterpret_cast<const f32x4_t*>(weight + (size_t)(16 * tile + l) * D + 32 * c + 8 * h + 4 * x);
+
+  const int dr = tid >> 2, dc = 4 * (tid & 3);      // rows dr (+ 64), columns d1_0 + dc .. + 3
+  f32x4_t acc[NR];
+#pragma unroll
+  for (int i = 0; i < NR; ++i) acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  const int n0 = (nsplit + 1) >> 1, first = half ? n0 : 0, n = half ? nsplit - n0 : n0;
+  sum_slices<NR>(kv_part + ((size_t)bh * nsplit + first) * DD + (size_t)dr * D + d1_0 + dc, n, DD, (size_t)64 * D, acc);
+  if (half) {
+#pragma unroll
+    for (int i = 0; i < NR; ++i) *reinterpret_cast<f32x4_t*>(s_half + (i * 256 + tid) * 4) = acc[i];
+    if (tid < 16) {
+      const float* pz = z_part + (size_t)bh * nsplit * D + d1_0 + tid;
+      float sum = 0.f;
+#pragma unroll 8
+      for (int sp = 0; sp < nsplit; ++sp) sum += pz[(size_t)sp * D];
+      z[(size_t)bh * D + d1_0 + tid] = E::from_float(sum);
+    }
+    if (bh == 0)
+      for (int i = tid; i < 16 * D; i += 256) {
+        const int d = d1_0 + i / D, e = i % D;
+        wt[d * D + e] = E::from_float(weight[(size_t)e * D + d]);
+      }
+  }
+  __syncthreads();
+  if (!half) {
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+      const int d2 = dr + 64 * i;
+      acc[i] += *reinterpret_cast<const f32x4_t*>(s_half + (i * 256 + tid) * 4);
+      i32x2_t w;
+      w[0] = (int)E::pack2(acc[i][0], acc[i][1]);
+      w[1] = (int)E::pack2(acc[i][2], acc[i][3]);
+      *reinterpret_cast<i32x2_t*>(kvt + (size_t)bh * DD + (size_t)d2 * D + d1_0 + dc) = w;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) s_kv[(dc + j) * STR + d2] = (uint16_t)((uint32_t)w[j >> 1] >> (16 * (j & 1)));
     }
   }
   __syncthreads();
-  const int el = tid / groups, d1 = (tid % groups) * 4;
-  float acc[4] = {0.f, 0.f, 0.f, 0.f};
-  const float* w = s_w + el * D;
-#pragma unroll 8
-  for (int d2 = 0; d2 < D; ++d2) {
-    const i16x4_t kv4 = *reinterpret_cast<const i16x4_t*>(&s_kv[d2 * D + d1]);
-    const float wv = w[d2];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[j] += wv * E::to_float((uint16_t)kv4[j]);
+  if constexpr (D == 64) {
+    // slots 8 piece .. of a row hold d2 = 16 c + 4 gg .. + 3 and 8 further on (piece = 2 c + gg)
+    if (half && tid < 16 * (D / 8)) {
+      const int row = tid / (D / 8), piece = tid % (D / 8);
+      const uint16_t* src = s_kv + row * STR + 16 * (piece >> 1) + 4 * (piece & 1);
+      const i16x8_t v8 = concat4(*reinterpret_cast<const i16x4_t*>(src), *reinterpret_cast<const i16x4_t*>(src + 8));
+      *reinterpret_cast<i16x8_t*>(kvp + (size_t)bh * DD + (size_t)(d1_0 + row) * D + 8 * piece) = v8;
+    }
   }
-  i32x2_t out;
-  out[0] = (int)E::pack2(acc[0], acc[1]);
-  out[1] = (int)E::pack2(acc[2], acc[3]);
-  *reinterpret_cast<i32x2_t*>(kvwt + (size_t)bh * D * D + (size_t)(e0 + el) * D + d1) = out;
+  if (wave >= D / 16) return;
+  f32x4_t o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int c = 0; c < D / 32; ++c) {
+    i32x4_t w;
+#pragma unroll
+    for (int x = 0; x < 4; ++x) w[x] = (int)E::pack2(wraw[c][x >> 1][2 * (x & 1)], wraw[c][x >> 1][2 * (x & 1) + 1]);
+    o = E::mfma16(*reinterpret_cast<const i16x8_t*>(s_kv + l * STR + 32 * c + 8 * h), __builtin_bit_cast(i16x8_t, w), o);
+  }
+  // rows d1 = 4 h + i, column e
+  i32x2_t w;
+  w[0] = (int)E::pack2(o[0], o[1]);
+  w[1] = (int)E::pack2(o[2], o[3]);
+  *reinterpret_cast<i32x2_t*>(kvwt + (size_t)bh * DD + (size_t)(16 * tile + l) * D + d1_0 + 4 * h) = w;
 }
 
 // ---- workspace layout of the state build -----------------------------------------------------
@@ -306,8 +367,11 @@ static inline LinWs lin_ws(int BH, int L, int D) {
   LinWs w;
   // Two workgroups per compute unit: the state kernel shares the memory system with the mask builder's passes on the
   // other stream, and more, shorter slices (three per unit fit) only add partial states to write and to add up again
-  // (module forward at B1 H12 L32760: 0.510 against 0.519 ms).
-  const LinSplit sp = lin_split(BH, L, 512);
+  // (module forward at B1 H12 L32760: 0.510 against 0.519 ms).  Short sequences: at most sixteen slices, or slices of 256
+  // rows; more only lengthen the chain that adds them up (state build of 8 heads x 4096 rows x 128: 64 slices 34.6 us, 16
+  // slices 23.8; 4 heads x 7813 x 64: 123 slices 23.5, 31 slices 15.3; with 1024 rows 16 slices of 64 rows 14.7, 4 of 256 19.4).
+  const int min_rows = L >= 4096 ? 256 : cdiv(L, 16);
+  const LinSplit sp = lin_split(BH, L, 512, 64, min_rows);
   w.nsplit = sp.nsplit;
   w.rows_per_split = sp.rows_per_split;
   size_t off = 0;
@@ -325,24 +389,23 @@ static inline LinWs lin_ws(int BH, int L, int D) {
 }
 
 
-// Streams K and V once and leaves KVT, KVP, z (16 bit) and the 16-bit transposed weight in the workspace.
-// (ws: where the states go; parts: where the slices' partial sums go, the offsets of `w` past states_end)
+// (ws: where the states go; parts: where the slices' partial sums lie, the offsets of `w` past states_end)
+template <typename Tag, int D>
+static inline void launch_state_finish(const float* weight, int BH, char* ws, char* parts, const LinWs& w, hipStream_t st) {
+  hipLaunchKernelGGL((linear_state_finish_kernel<Tag, D>), dim3(xcd_grid((int64_t)BH * (D / 16))), dim3(512), 0, st,
+                     (const float*)(parts + (w.kv_part - w.states_end)), (const float*)(parts + (w.z_part - w.states_end)), weight,
+                     (uint16_t*)(ws + w.kvt), (uint16_t*)(ws + w.kvp), (uint16_t*)(ws + w.kvwt), (uint16_t*)(ws + w.z),
+                     (uint16_t*)(ws + w.wt), w.nsplit, BH * (D / 16));
+}
+
+// Streams K and V once and leaves the finished states and the 16-bit transposed weight.
 template <typename Tag, int D>
 static inline void launch_state_build(const void* k, const void* v, const RowLayout& lay, const float* weight, int fmap,
-                                      int BH, int L, char* ws, char* parts, const LinWs& w, hipStream_t st,
-                                      bool copy_weight = true) {
-  float* kv_part = (float*)(parts + (w.kv_part - w.states_end));
-  float* z_part = (float*)(parts + (w.z_part - w.states_end));
-  uint16_t* kvt = (uint16_t*)(ws + w.kvt);
-  uint16_t* z = (uint16_t*)(ws + w.z);
+                                      int BH, int L, char* ws, char* parts, const LinWs& w, hipStream_t st) {
   hipLaunchKernelGGL((linear_state_partial_kernel<Tag, D>), dim3(w.nsplit, BH), dim3(256), 0, st, (const uint16_t*)k,
-                     (const uint16_t*)v, lay, kv_part, z_part, L, w.rows_per_split, fmap);
-  hipLaunchKernelGGL((linear_state_reduce_kernel<Tag>), dim3(cdiv(D * D, 256), BH), dim3(256), 0, st, kv_part, z_part, kvt,
-                     (uint16_t*)(ws + w.kvp), z, w.nsplit, D * D, D);
-  // (copy_weight = false: the caller's next kernel writes the 16-bit transposed weight on the side)
-  if (copy_weight)
-    hipLaunchKernelGGL((linear_prep_weight_kernel<Tag>), dim3(cdiv(D * D, 256)), dim3(256), 0, st, weight,
-                       (uint16_t*)(ws + w.wt), D);
+                     (const uint16_t*)v, lay, (void*)(parts + (w.kv_part - w.states_end)),
+                     (float*)(parts + (w.z_part - w.states_end)), L, w.rows_per_split, fmap);
+  launch_state_finish<Tag, D>(weight, BH, ws, parts, w, st);
 }
 
 }  // namespace sla

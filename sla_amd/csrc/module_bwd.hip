@@ -59,7 +59,7 @@ static int module_bwd_run(const void* q, const void* k, const void* v, const int
     SLA_HIP_OK(hipEventRecord(ev->second, st));
     // side: the small products of the linear branch.  main: dK/dV, then the key side of the linear branch
     SLA_HIP_OK(hipStreamWaitEvent(side, ev->second, 0));
-    if ((r = linear(side, LB_REDUCE))) return r;
+    if ((r = linear(side, LB_REDUCE | LB_BESIDE))) return r;
     SLA_HIP_OK(hipEventRecord(ev->third, side));
     SLA_HIP_OK(hipStreamWaitEvent(st, ev->first, 0));
     if ((r = sparse(st, SB_DKDV))) return r;
