@@ -1,0 +1,20 @@
+// Where the mask builder's score kernels want the block means (block_map.hip; the quantisers of sage.hip write them too).
+#pragma once
+#include "common.h"
+
+namespace sla {
+
+// 16-bit dtypes, head dim 64 or 128: the means are written in the order the matrix products of the scores read them; other
+// dtypes and head dims take rows.
+static inline int score_takes_tiled(int dtype, int D) { return dtype != SLA_F32 && (D == 64 || D == 128); }
+
+// Operand order: tiles of 32 blocks; per tile and 16 columns a fragment of 64 lanes x 8 elements, lane (r, h) = (block % 32,
+// column % 2), element j = columns 16 c + 2 j + h: what lane r + 32 h feeds the 32x32x2 product chain, two columns a step.
+static __host__ __device__ __forceinline__ size_t tiled_head(int bh, int nblk, int D) {
+  return (size_t)bh * (size_t)((nblk + 31) & ~31) * (size_t)D;
+}
+static __host__ __device__ __forceinline__ size_t tiled_pos(int blk, int d, int D) {
+  return ((size_t)((blk >> 5) * (D >> 4) + (d >> 4)) * 64 + 32 * (d & 1) + (blk & 31)) * 8 + ((d & 15) >> 1);
+}
+
+}  // namespace sla

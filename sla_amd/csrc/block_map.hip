@@ -11,6 +11,7 @@
 //                ascending order; group sums added in ascending order; one IEEE division by L;
 //   score      : acc = acc + (a_d * b_d), d ascending, no fused multiply-add.
 // Selection is by (score descending, index ascending); -0.0 == +0.0.
+#include "block_map.h"
 #include "fwd_steps.h"
 
 #include <mutex>
@@ -54,10 +55,11 @@ struct alignas(16) Vec16 {
 // MODE 1: block mean in the input dtype        -> out     (BH, nblk, D)
 // MODE 2: block mean of round(x - colmean)     -> out     (BH, nblk, D)
 // One thread owns VEC adjacent columns of one block and walks its rows in order.
+// tiled: the means go out in operand order (16-bit dtypes; tiled_pos) instead of as rows.
 template <typename IO, int MODE>
 static __device__ __forceinline__ void pool_body(const typename IO::raw* __restrict__ x, const RowLayout lay,
                                                  const typename IO::raw* __restrict__ colmean, void* __restrict__ out, int L,
-                                                 int D, int BLK, int nblk, int bx, int bh) {
+                                                 int D, int BLK, int nblk, int tiled, int bx, int bh) {
   constexpr int VEC = IO::VEC;
   const int tpr = D / VEC;
   const int bpw = 256 / tpr;
@@ -113,6 +115,19 @@ static __device__ __forceinline__ void pool_body(const typename IO::raw* __restr
     Vec16<IO> r;
 #pragma unroll
     for (int e = 0; e < VEC; ++e) r.e[e] = IO::st(acc[e] / cnt);
+    if constexpr (VEC == 8) {
+      if (tiled) {             // four even and four odd columns, adjacent in their places
+        uint16_t* t = reinterpret_cast<uint16_t*>(out) + tiled_head(bh, nblk, D);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          i16x4_t w;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) w[j] = (short)r.e[2 * j + h];
+          *reinterpret_cast<i16x4_t*>(t + tiled_pos(blk, c + h, D)) = w;
+        }
+        return;
+      }
+    }
     *reinterpret_cast<Vec16<IO>*>(reinterpret_cast<typename IO::raw*>(out) + o) = r;
   }
 }
@@ -120,8 +135,8 @@ static __device__ __forceinline__ void pool_body(const typename IO::raw* __restr
 template <typename IO, int MODE>
 __global__ __launch_bounds__(256) void pool_kernel(const typename IO::raw* __restrict__ x, const RowLayout lay,
                                                    const typename IO::raw* __restrict__ colmean,
-                                                   void* __restrict__ out, int L, int D, int BLK, int nblk) {
-  pool_body<IO, MODE>(x, lay, colmean, out, L, D, BLK, nblk, blockIdx.x, blockIdx.y);
+                                                   void* __restrict__ out, int L, int D, int BLK, int nblk, int tiled) {
+  pool_body<IO, MODE>(x, lay, colmean, out, L, D, BLK, nblk, tiled, blockIdx.x, blockIdx.y);
 }
 
 // The two independent first passes of the mask builder in one launch (neither fills the memory system alone):
@@ -132,11 +147,11 @@ template <typename IO>
 __global__ __launch_bounds__(256) void pool_pair_kernel(const typename IO::raw* __restrict__ k, float* __restrict__ chunk_sums,
                                                         int nchunk, const typename IO::raw* __restrict__ q,
                                                         const RowLayout lay, typename IO::raw* __restrict__ pq, int BLKQ,
-                                                        int nblkq, int L, int D) {
+                                                        int nblkq, int L, int D, int tiled) {
   if (blockIdx.z == 1)
-    pool_body<IO, 0>(k, lay, nullptr, chunk_sums, L, D, KMEAN_CHUNK, nchunk, blockIdx.x, blockIdx.y);
+    pool_body<IO, 0>(k, lay, nullptr, chunk_sums, L, D, KMEAN_CHUNK, nchunk, 0, blockIdx.x, blockIdx.y);
   else
-    pool_body<IO, 1>(q, lay, nullptr, pq, L, D, BLKQ, nblkq, blockIdx.x, blockIdx.y);
+    pool_body<IO, 1>(q, lay, nullptr, pq, L, D, BLKQ, nblkq, tiled, blockIdx.x, blockIdx.y);
 }
 
 // Column mean of K, levels 2 and 3 of the fixed summation order:
@@ -185,10 +200,16 @@ __global__ __launch_bounds__(256) void colmean_fused_kernel(const float* __restr
   for (int g = tid / COLMEAN_SLAB; g < ngroup; g += 256 / COLMEAN_SLAB) {
     const int c0 = g * KMEAN_GROUP;
     const int n = min(KMEAN_GROUP, nchunk - c0);
+    // (a group's loads all in flight, then added in order: mask builder of 16 heads x 6001 x 64 25.3 -> 23.2 us, of 40 x 75600 x 128 656 -> 652)
     const float* p = chunk_sums + ((size_t)bh * nchunk + c0) * D + d;
+    float x[KMEAN_GROUP];
+#pragma unroll
+    for (int i = 0; i < KMEAN_GROUP; ++i) x[i] = p[(size_t)min(i, n - 1) * D];
+    __builtin_amdgcn_sched_barrier(0);
     float acc = 0.f;
-#pragma unroll 8
-    for (int i = 0; i < n; ++i) acc = acc + p[(size_t)i * D];
+#pragma unroll
+    for (int i = 0; i < KMEAN_GROUP; ++i)
+      if (i < n) acc = acc + x[i];
     gs[g * COLMEAN_SLAB + c] = acc;
   }
   __syncthreads();
@@ -294,81 +315,64 @@ __global__ __launch_bounds__(256) void score_kernel(const typename IO::raw* __re
 // d = 0, 2, 4, ... therefore is the d-ascending chain of fp32 fused multiply-adds of score_kernel, bit for bit (the
 // product of two 16-bit values is exact in fp32, so fused or not makes no difference; values whose products fall
 // into the fp32 subnormal range aside), at twice the rate of the vector ALU.
-// 64 x 64NW scores per workgroup, one wave per 32 x 32NW part (NW independent accumulation chains).  The 64 pooled rows of either operand go through LDS
-// (coalesced 16-byte loads; rows padded by 16 bytes, so that the row-per-lane reads are free of bank conflicts);
-// lanes l and l + 32 read the same rows and feed the even and the odd d.  The rounded scores go back through LDS
-// and leave in 256-byte runs.
-template <typename IO, int D, int NW>
+// The operands arrive in the order the products read them (tiled_pos, written by the pooling kernels): a fragment is one
+// coalesced load, straight into registers.
+template <typename IO, int D>
+struct ScoreFrags {
+  static constexpr int NC = D / 16;              // fragments (16 d of 32 blocks) per tile
+  i32x4_t w[NC];
+  __device__ __forceinline__ void load(const typename IO::raw* p, int bh, int nblk, int tile, int lane) {
+    const i16x8_t* t = reinterpret_cast<const i16x8_t*>(p + tiled_head(bh, nblk, D)) + (size_t)tile * (NC * 64) + lane;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) w[c] = __builtin_bit_cast(i32x4_t, t[c * 64]);
+  }
+  __device__ __forceinline__ float at(int c, int j) const {      // column 16 c + 2 j + lane / 32 of the lane's block
+    return IO::ld((typename IO::raw)((uint32_t)w[c][j >> 1] >> (16 * (j & 1))));
+  }
+};
+template <typename IO, int D>
+static __device__ __forceinline__ f32x16_t score_tile(const ScoreFrags<IO, D>& a, const ScoreFrags<IO, D>& b) {
+  __builtin_amdgcn_sched_barrier(0);             // (every load of both tiles first)
+  f32x16_t acc;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+#pragma unroll
+  for (int c = 0; c < D / 16; ++c)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.at(c, j), b.at(c, j), acc, 0, 0, 0);
+  return acc;                                    // register i of lane (r, h): query block 8 (i / 4) + i % 4 + 4 h, key block r
+}
+
+// 64 x 64 scores per workgroup, one wave per 32 x 32 part; the rounded scores go through LDS and leave in 128-byte runs.
+// Bound by the fp32 matrix rate (40 heads x 1182 x 1182: 91 us at the nominal rate); with both operand tiles through LDS
+// 158 us, now 140.
+template <typename IO, int D>
 __global__ __launch_bounds__(256) void score_mfma_kernel(const typename IO::raw* __restrict__ pq,
                                                          const typename IO::raw* __restrict__ pk,
                                                          typename IO::raw* __restrict__ score, int M, int N) {
-  static_assert(sizeof(typename IO::raw) == 2 && D % 32 == 0, "16-bit dtypes, 256 threads fetch whole rows");
-  constexpr int NC = D / 8;              // 16-byte pieces per row
-  constexpr int RS = D * 2 + 16;         // bytes between rows in LDS
-  constexpr int OS = 64 * NW * 2 + 4;         // bytes between rows of the staged scores
-  constexpr int TN = 64 * NW;            // scores per row of the workgroup's tile
-  __shared__ __attribute__((aligned(16))) uint8_t sm[(64 + TN) * RS];
-  static_assert(64 * OS <= (64 + TN) * RS, "the staged scores reuse the operand tiles");
+  constexpr int OS = 64 + 2;             // staged scores between rows
+  __shared__ __attribute__((aligned(16))) typename IO::raw sm[64 * OS];
   const int bh = blockIdx.z, tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
   const int r = lane & 31, h = lane >> 5;
-  const int m0 = blockIdx.y * 64, n0 = blockIdx.x * (64 * NW);
-  const __amdgpu_buffer_rsrc_t qh = make_rsrc(pq + (size_t)bh * M * D, (uint32_t)M * D * 2);    // rows past the end read as zero
-  const __amdgpu_buffer_rsrc_t kh = make_rsrc(pk + (size_t)bh * N * D, (uint32_t)N * D * 2);
-#pragma unroll
-  for (int i = 0; i < 64 * NC / 256; ++i) {
-    const int p = tid + 256 * i, row = p / NC, pc = p % NC;
-    const i16x8_t a = buf_load_b128(qh, ((uint32_t)(m0 + row) * D + 8 * pc) * 2);
-    i16x8_t b[NW];
-#pragma unroll
-    for (int t = 0; t < NW; ++t) b[t] = buf_load_b128(kh, ((uint32_t)(n0 + 64 * t + row) * D + 8 * pc) * 2);
-    *reinterpret_cast<i16x8_t*>(sm + row * RS + pc * 16) = a;
-#pragma unroll
-    for (int t = 0; t < NW; ++t) *reinterpret_cast<i16x8_t*>(sm + (64 + 64 * t + row) * RS + pc * 16) = b[t];
-  }
-  __syncthreads();
+  const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
   const int wm = wave >> 1, wn = wave & 1;
-  const uint8_t* arow = sm + (wm * 32 + r) * RS;
-  const uint8_t* brow = sm + (64 + wn * 32 * NW + r) * RS;      // this wave's NW tiles of 32 columns lie side by side
-  f32x16_t acc[NW];
+  if (m0 + 32 * wm < M && n0 + 32 * wn < N) {
+    ScoreFrags<IO, D> a, b;
+    a.load(pq, bh, M, (m0 >> 5) + wm, lane);
+    b.load(pk, bh, N, (n0 >> 5) + wn, lane);
+    const f32x16_t acc = score_tile<IO, D>(a, b);
 #pragma unroll
-  for (int t = 0; t < NW; ++t)
-#pragma unroll
-    for (int i = 0; i < 16; ++i) acc[t][i] = 0.f;
-  const int sh = 16 * h;
-#pragma unroll
-  for (int c = 0; c < NC; ++c) {
-    const i32x4_t aw = *reinterpret_cast<const i32x4_t*>(arow + c * 16);
-    i32x4_t bw[NW];
-#pragma unroll
-    for (int t = 0; t < NW; ++t) bw[t] = *reinterpret_cast<const i32x4_t*>(brow + 32 * t * RS + c * 16);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const float av = IO::ld((typename IO::raw)((uint32_t)aw[j] >> sh));
-#pragma unroll
-      for (int t = 0; t < NW; ++t) {
-        const float bv = IO::ld((typename IO::raw)((uint32_t)bw[t][j] >> sh));
-        acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(av, bv, acc[t], 0, 0, 0);
-      }
-    }
+    for (int i = 0; i < 16; ++i) sm[(wm * 32 + 8 * (i >> 2) + (i & 3) + 4 * h) * OS + wn * 32 + r] = IO::st(acc[i]);
   }
-  __syncthreads();                       // every wave has read its operands: the tiles make room for the scores
-#pragma unroll
-  for (int t = 0; t < NW; ++t)
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int m = wm * 32 + 8 * (i >> 2) + (i & 3) + 4 * h;
-      *reinterpret_cast<typename IO::raw*>(sm + m * OS + (wn * 32 * NW + 32 * t + r) * 2) = IO::st(acc[t][i]);
-    }
   __syncthreads();
   typename IO::raw* out = score + (size_t)bh * M * N;
-  constexpr int TPR = 32 * NW;           // threads per row of staged scores, two scores each
-  const int orow = tid / TPR, ocol = (tid % TPR) * 2;
+  const int orow = tid >> 5, ocol = (tid & 31) * 2;      // two scores per thread and pass
 #pragma unroll
-  for (int pass = 0; pass < 64 * TPR / 256; ++pass) {
-    const int ml = pass * (256 / TPR) + orow, m = m0 + ml, n = n0 + ocol;
+  for (int pass = 0; pass < 8; ++pass) {
+    const int ml = pass * 8 + orow, m = m0 + ml, n = n0 + ocol;
     if (m >= M || n >= N) continue;
-    const uint32_t two = *reinterpret_cast<const uint32_t*>(sm + ml * OS + ocol * 2);
+    const uint32_t two = *reinterpret_cast<const uint32_t*>(&sm[ml * OS + ocol]);
     typename IO::raw* dst = out + (size_t)m * N + n;
     if (!(N & 1) && n + 1 < N) {
       *reinterpret_cast<uint32_t*>(dst) = two;          // (N even: every pair starts 4-byte aligned)
@@ -380,18 +384,13 @@ __global__ __launch_bounds__(256) void score_mfma_kernel(const typename IO::raw*
 }
 
 template <typename IO>
-static void launch_score(const typename IO::raw* pq, const typename IO::raw* pk, typename IO::raw* score, int BH, int M, int N,
-                         int D, hipStream_t st) {
+static void launch_score(const typename IO::raw* pq, const typename IO::raw* pk, int tiled, typename IO::raw* score, int BH, int M,
+                         int N, int D, hipStream_t st) {
   const dim3 grid(cdiv(N, 64), cdiv(M, 64), BH);
   if constexpr (sizeof(typename IO::raw) == 2) {
-    const bool fits = (int64_t)M * D * 2 < (1ll << 32) && (int64_t)N * D * 2 < (1ll << 32);
-    // (NW = 2, two column tiles per wave, is no faster: 159 against 153 us for 40 heads of 1182 x 1182 scores)
-    if (D == 128 && fits) {
-      hipLaunchKernelGGL((score_mfma_kernel<IO, 128, 1>), grid, dim3(256), 0, st, pq, pk, score, M, N);
-      return;
-    }
-    if (D == 64 && fits) {
-      hipLaunchKernelGGL((score_mfma_kernel<IO, 64, 1>), grid, dim3(256), 0, st, pq, pk, score, M, N);
+    if (tiled) {
+      if (D == 128) hipLaunchKernelGGL((score_mfma_kernel<IO, 128>), grid, dim3(256), 0, st, pq, pk, score, M, N);
+      else hipLaunchKernelGGL((score_mfma_kernel<IO, 64>), grid, dim3(256), 0, st, pq, pk, score, M, N);
       return;
     }
   }
@@ -432,143 +431,370 @@ static __device__ __forceinline__ int wave_inclusive_sum(int x, int lane) {
   return x;
 }
 
+static __device__ __forceinline__ int lanes_before(unsigned long long b) {       // set bits of b below this lane
+  return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(b >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)b, 0u));
+}
+
+// Writes the selection of a row whose keys lie in EPL registers per lane (key e of lane l: index 64 e + l): everything above
+// `thr` and the first `need_eq` keys equal to it, in ascending index order, into the look-up row and the int8 map row (null:
+// not wanted).
+template <int EPL>
+static __device__ __forceinline__ void emit_row(const uint32_t (&keys)[EPL], uint32_t thr, int need_eq, int8_t* mrow, void* lut,
+                                                int lut64, size_t lut_row, int N, int T, int lane) {
+  int run_eq = 0, run_sel = 0;
+#pragma unroll
+  for (int e = 0; e < EPL; ++e) {
+    if (e * 64 >= N) break;
+    const int i = e * 64 + lane;
+    const bool in = i < N;
+    const bool gt = in && keys[e] > thr;
+    const bool eq = in && keys[e] == thr;
+    const unsigned long long beq = __ballot(eq);
+    const int eq_rank = run_eq + lanes_before(beq);
+    const bool sel = gt || (eq && eq_rank < need_eq);
+    const unsigned long long bsel = __ballot(sel);
+    const int pos = run_sel + lanes_before(bsel);
+    if (in && mrow) mrow[i] = sel ? 1 : 0;
+    if (sel && pos < T) {              // (pos < T always holds; the test keeps a wrong count from ever leaving the row)
+      if (lut64)
+        reinterpret_cast<long long*>(lut)[lut_row + pos] = i;
+      else
+        reinterpret_cast<int*>(lut)[lut_row + pos] = i;
+    }
+    run_eq += __popcll(beq);
+    run_sel += __popcll(bsel);
+    __builtin_amdgcn_sched_barrier(0);      // (not every ballot first: a pair of scalar registers each)
+  }
+}
+
+// The T-th largest of W keys per lane, for R rows at once, built bit by bit from the top (a bit stays when at least T keys are
+// at or above the value it gives; counts through the wave's ballots).  The rows' chains hide each other's latency.
+// Missing keys are 0.
+template <int R, int W, int LOW_BIT>
+static __device__ __forceinline__ void kth_largest(const uint32_t (&kx)[R][W], int T, uint32_t (&thr)[R]) {
+#pragma unroll
+  for (int x = 0; x < R; ++x) thr[x] = 0;
+  for (int b = 31; b >= LOW_BIT; --b) {
+    int cnt[R];
+#pragma unroll
+    for (int x = 0; x < R; ++x) {
+      cnt[x] = 0;
+#pragma unroll
+      for (int e = 0; e < W; ++e) cnt[x] += __popcll(__ballot(kx[x][e] >= (thr[x] | (1u << b))));
+    }
+#pragma unroll
+    for (int x = 0; x < R; ++x)
+      if (cnt[x] >= T) thr[x] |= 1u << b;
+  }
+}
+template <int W>
+static __device__ __forceinline__ int count_above(const uint32_t (&k)[W], uint32_t thr) {
+  int n = 0;
+#pragma unroll
+  for (int e = 0; e < W; ++e) n += __popcll(__ballot(k[e] > thr));
+  return n;
+}
+
+constexpr int SELECT_CAND = 128;       // candidates a short list holds
+
+// Selection for R rows (wave-wide; row x's keys: kx[x][e] of lane l is index 64 e + l, 0 past the end of the row).
+// The instructions of a threshold search grow with the keys per lane, so it runs twice on few of them where T allows: first on
+// S group maxima per lane, whose T-th largest value is at most the row's; the keys not below it, usually little more than
+// T, go into a short list in LDS in index order, and the exact search and the emission run on that.  (S 64 T-th maxima:
+// T <= 32 with one group, T <= 80 with two leave about 1.2 T .. 1.6 T candidates of distinct random scores.)  Longer rows of
+// selected blocks, and lists that overflow because many scores are equal, search all keys.
+// Kernel of 12 heads x 512 rows x 512, T = 25: 13.8 -> 11.2 us; of 40 x 1182 x 1182, T = 59: 129 -> 89 us.
+// `list`: SELECT_CAND keys, then SELECT_CAND indices, then the map row; private to the wave.
+template <int EPL, int LOW_BIT, int R>
+static __device__ __forceinline__ void select_rows(const uint32_t (&kx)[R][EPL], uint32_t* list, int8_t* sparse_map, void* lut,
+                                                   int lut64, size_t row0, int rows, int N, int T, int lane) {
+  uint32_t thr[R];
+  bool short_list = EPL > 2 && T <= 80;
+  if constexpr (EPL > 2) {
+    if (short_list) {
+      if (T <= 32) {
+        uint32_t mx[R][1];
+#pragma unroll
+        for (int x = 0; x < R; ++x) {
+          mx[x][0] = kx[x][0];
+#pragma unroll
+          for (int e = 1; e < EPL; ++e) mx[x][0] = max(mx[x][0], kx[x][e]);
+        }
+        kth_largest<R, 1, LOW_BIT>(mx, T, thr);
+      } else {
+        uint32_t mx[R][2];
+#pragma unroll
+        for (int x = 0; x < R; ++x)
+#pragma unroll
+          for (int s = 0; s < 2; ++s) {
+            mx[x][s] = kx[x][s];
+#pragma unroll
+            for (int e = 2 + s; e < EPL; e += 2) mx[x][s] = max(mx[x][s], kx[x][e]);
+          }
+        kth_largest<R, 2, LOW_BIT>(mx, T, thr);
+      }
+    }
+  }
+  if (!short_list) kth_largest<R, EPL, LOW_BIT>(kx, T, thr);
+#pragma unroll
+  for (int x = 0; x < R; ++x) {
+    if (x >= rows) break;
+    const size_t row = row0 + x;
+    int8_t* const mrow = sparse_map ? sparse_map + row * N : nullptr;
+    if constexpr (EPL > 2) {
+      if (short_list) {
+        const uint32_t lb = thr[x];
+        uint32_t* const li = list + SELECT_CAND;
+        int n = 0;
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) {
+          const bool in = kx[x][e] >= lb && 64 * e + lane < N;
+          const unsigned long long b = __ballot(in);
+          const int pos = n + lanes_before(b);
+          if (in && pos < SELECT_CAND) {
+            list[pos] = kx[x][e];
+            li[pos] = (uint32_t)(64 * e + lane);
+          }
+          n += __popcll(b);
+        }
+        if (n <= SELECT_CAND) {
+          int8_t* const lm = reinterpret_cast<int8_t*>(list + 2 * SELECT_CAND);
+          if (mrow)
+#pragma unroll
+            for (int e = 0; e < EPL / 4; ++e) reinterpret_cast<uint32_t*>(lm)[64 * e + lane] = 0u;
+          wave_lds_fence();
+          uint32_t ck[1][2], idx[2];
+#pragma unroll
+          for (int w = 0; w < 2; ++w) {
+            const bool in = 64 * w + lane < n;
+            ck[0][w] = in ? list[64 * w + lane] : 0u;
+            idx[w] = in ? li[64 * w + lane] : 0u;
+          }
+          uint32_t t1[1];
+          kth_largest<1, 2, LOW_BIT>(ck, T, t1);
+          const int need_eq = T - count_above<2>(ck[0], t1[0]);
+          int run_eq = 0, run_sel = 0;
+#pragma unroll
+          for (int w = 0; w < 2; ++w) {
+            const bool in = 64 * w + lane < n;
+            const bool eq = in && ck[0][w] == t1[0];
+            const unsigned long long beq = __ballot(eq);
+            const bool sel = (in && ck[0][w] > t1[0]) || (eq && run_eq + lanes_before(beq) < need_eq);
+            const unsigned long long bsel = __ballot(sel);
+            const int pos = run_sel + lanes_before(bsel);
+            if (sel && pos < T) {            // (pos < T always holds; the test keeps a wrong count from ever leaving the row)
+              if (lut64)
+                reinterpret_cast<long long*>(lut)[row * T + pos] = (int)idx[w];
+              else
+                reinterpret_cast<int*>(lut)[row * T + pos] = (int)idx[w];
+              if (mrow) lm[idx[w]] = 1;
+            }
+            run_eq += __popcll(beq);
+            run_sel += __popcll(bsel);
+          }
+          if (mrow) {
+            wave_lds_fence();
+            if (!(N & 3)) {
+#pragma unroll
+              for (int e = 0; e < EPL / 4; ++e)
+                if (4 * (64 * e + lane) < N) reinterpret_cast<uint32_t*>(mrow)[64 * e + lane] = reinterpret_cast<const uint32_t*>(lm)[64 * e + lane];
+            } else {
+#pragma unroll
+              for (int e = 0; e < EPL; ++e)
+                if (64 * e + lane < N) mrow[64 * e + lane] = lm[64 * e + lane];
+            }
+          }
+          wave_lds_fence();                  // (the next row's list goes over this one)
+          continue;
+        }
+        wave_lds_fence();
+        const uint32_t (&k1)[1][EPL] = reinterpret_cast<const uint32_t (&)[1][EPL]>(kx[x]);
+        uint32_t t1[1];
+        kth_largest<1, EPL, LOW_BIT>(k1, T, t1);
+        thr[x] = t1[0];
+      }
+    }
+    emit_row<EPL>(kx[x], thr[x], T - count_above<EPL>(kx[x], thr[x]), mrow, lut, lut64, row * T, N, T, lane);
+  }
+}
+
 // One wavefront per (bh, m) row (four rows per workgroup): find the T-th largest key, then emit
 // winners in ascending index order (ties at the threshold value go to the lowest indices).  Writes the int8 map row and the look-up-table row.
-// EPL > 0: the row's keys live in EPL registers per lane (N <= 64*EPL); EPL == 0: keys in LDS.
+// EPL > 0: the row's keys live in EPL registers per lane (N <= 64*EPL; select_rows); EPL == 0: keys in LDS.
 // LOW_BIT: lowest key bit that can differ (16 for 16-bit score dtypes, whose low bits are zero).
 template <typename IO, int EPL, int LOW_BIT>
 __global__ __launch_bounds__(256) void topk_kernel(const typename IO::raw* __restrict__ score,
                                                    int8_t* __restrict__ sparse_map, void* __restrict__ lut, int lut64, int N,
                                                    int T, size_t nrows) {
   extern __shared__ uint32_t lds_keys[];
-  // (the histograms are only used when the keys live in LDS: the register instances carry a token array)
-  __shared__ __attribute__((aligned(16))) uint32_t hist_all[EPL == 0 ? 4 : 1][EPL == 0 ? 256 : 1];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const size_t row = (size_t)blockIdx.x * 4 + wave;
   if (row >= nrows) return;
   const typename IO::raw* s = score + row * N;
-  constexpr int NR = EPL > 0 ? EPL : 1;
-  uint32_t kreg[NR];
-  uint32_t* keys = lds_keys + (size_t)wave * (EPL > 0 ? 0 : N);
-  const int nit = EPL > 0 ? EPL : (N + 63) / 64;
-  // out-of-range slots hold key 0, below every real key (a real key has bit 31 set or is > 0 ... except
-  // the most negative NaN pattern); they are excluded explicitly by the index test below.
-  if (EPL > 0) {
-#pragma unroll
-    for (int e = 0; e < NR; ++e) {
-      const int i = e * 64 + lane;
-      kreg[e] = i < N ? order_key<LOW_BIT>(IO::ld(s[i])) : 0u;
-    }
-  } else {
-    for (int i = lane; i < N; i += 64) keys[i] = order_key<LOW_BIT>(IO::ld(s[i]));
-  }
-  auto key_at = [&](int e) -> uint32_t {
-    if (EPL > 0) return kreg[e < NR ? e : 0];
-    const int i = e * 64 + lane;
-    return i < N ? keys[i] : 0u;
-  };
-  // Keys in LDS: radix select, eight key bits per pass (two passes for bf16 scores): the keys that agree with the digits found
-  // so far are counted per value of the next digit in a 256-bin histogram (LDS atomics of this wave on its own
-  // bins); lane l then owns the four highest undecided digits 255 - 4l .. 252 - 4l, a prefix sum over the lanes
-  // gives the number of keys above them, and the one lane whose digits straddle the wanted rank names the digit.
   if (T <= 0) {              // nothing to select (a ratio that rounds to no block at all): an all-zero map row, no table row
     if (sparse_map)
       for (int i = lane; i < N; i += 64) sparse_map[row * N + i] = 0;
     return;
   }
-  uint32_t thr = 0;          // digits decided so far
-  int need = T;              // rank of the threshold among the keys that agree with them
-  uint32_t* hist = hist_all[EPL == 0 ? wave : 0];
-  if (EPL > 0) {
-    // Keys in registers: the threshold is built bit by bit from the top, keeping a bit when at least T keys are at or
-    // above the value it gives (one compare per key and bit, counted through the wave's ballot: no memory traffic and no
-    // serialised atomics on the few histogram bins that the exponents of a row of scores fall into).  Slots past the
-    // end of the row hold key 0 and are never at or above a candidate, which has at least one bit set.
-    for (int b = 31; b >= LOW_BIT; --b) {
-      const uint32_t cand = thr | (1u << b);
-      int cnt = 0;
+  if constexpr (EPL > 0) {
+    __shared__ __attribute__((aligned(16))) uint32_t lists[4][2 * SELECT_CAND + 16 * EPL];
+    // (out-of-range slots hold key 0, below every real key but the most negative NaN pattern; the index tests exclude them)
+    uint32_t kx[1][EPL];
 #pragma unroll
-      for (int e = 0; e < NR; ++e) cnt += __popcll(__ballot(kreg[e] >= cand));
-      if (cnt >= T) thr = cand;
+    for (int e = 0; e < EPL; ++e) {
+      const int i = e * 64 + lane;
+      kx[0][e] = i < N ? order_key<LOW_BIT>(IO::ld(s[i])) : 0u;
     }
-    int above = 0;
-#pragma unroll
-    for (int e = 0; e < NR; ++e) above += __popcll(__ballot(kreg[e] > thr));
-    need = T - above;        // how many of the keys equal to the threshold are taken
-  }
-#pragma unroll
-  for (int hi = EPL > 0 ? LOW_BIT : 32; hi > LOW_BIT;) {
-    const int w = (hi - LOW_BIT) < 8 ? (hi - LOW_BIT) : 8;
-    const int shift = hi - w;
-    *reinterpret_cast<i32x4_t*>(&hist[4 * lane]) = i32x4_t{0, 0, 0, 0};
-    wave_lds_fence();
-    auto count_key = [&](int e, uint32_t kv) {
-      const bool in = e * 64 + lane < N;
-      const bool agrees = hi == 32 || ((kv ^ thr) >> (hi & 31)) == 0;
-      if (in && agrees) atomicAdd(&hist[(kv >> shift) & ((1u << w) - 1u)], 1u);
-    };
-    if (EPL > 0) {
-#pragma unroll
-      for (int e = 0; e < NR; ++e) count_key(e, kreg[e]);
-    } else {
-      for (int e = 0; e < nit; ++e) count_key(e, key_at(e));
-    }
-    wave_lds_fence();
-    const i32x4_t c4 = *reinterpret_cast<const i32x4_t*>(&hist[252 - 4 * lane]);    // digits 252 - 4l .. 255 - 4l
-    const int c[4] = {c4[3], c4[2], c4[1], c4[0]};                                   // in descending order of the digit
-    const int mine = c[0] + c[1] + c[2] + c[3];
-    const int incl = wave_inclusive_sum(mine, lane);
-    const int above = incl - mine;               // keys (among those that agree) whose digit is above all of this lane's
-    const bool here = above < need && need <= incl;
-    int digit = 0, rest = 0;
-#pragma unroll
-    for (int jj = 0; jj < 4; ++jj) {             // (at most one of the four digits straddles the rank)
-      int before = above;
-#pragma unroll
-      for (int t = 0; t < jj; ++t) before += c[t];
-      if (before < need && need <= before + c[jj]) {
-        digit = 255 - 4 * lane - jj;
-        rest = need - before;
-      }
-    }
-    const unsigned long long who = __ballot(here);
-    const int src = who ? (int)__builtin_ctzll(who) : 0;
-    digit = __builtin_amdgcn_readlane(digit, src);
-    need = __builtin_amdgcn_readlane(rest, src);
-    thr |= (uint32_t)digit << shift;
-    hi = shift;
-  }
-  const int need_eq = need;
-  int run_eq = 0, run_sel = 0;
-  const unsigned long long lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  int8_t* mrow = sparse_map + row * N;
-  auto emit = [&](int e, uint32_t kv) {
-    const int i = e * 64 + lane;
-    const bool in = i < N;
-    const bool gt = in && kv > thr;
-    const bool eq = in && kv == thr;
-    const unsigned long long beq = __ballot(eq);
-    const int eq_rank = run_eq + __popcll(beq & lt_mask);
-    const bool sel = gt || (eq && eq_rank < need_eq);
-    const unsigned long long bsel = __ballot(sel);
-    const int pos = run_sel + __popcll(bsel & lt_mask);
-    if (in && sparse_map) mrow[i] = sel ? 1 : 0;
-    if (sel && pos < T) {              // (pos < T always holds; the test keeps a wrong count from ever leaving the row)
-      if (lut64)
-        reinterpret_cast<long long*>(lut)[row * T + pos] = i;
-      else
-        reinterpret_cast<int*>(lut)[row * T + pos] = i;
-    }
-    run_eq += __popcll(beq);
-    run_sel += __popcll(bsel);
-  };
-  if (EPL > 0) {
-#pragma unroll
-    for (int e = 0; e < NR; ++e)
-      if (e * 64 < N) emit(e, kreg[e]);
+    select_rows<EPL, LOW_BIT, 1>(kx, lists[wave], sparse_map, lut, lut64, row, 1, N, T, lane);
   } else {
-    for (int e = 0; e < nit; ++e) emit(e, key_at(e));
+    // Keys in LDS: radix select, eight key bits per pass (two passes for bf16 scores): the keys that agree with the digits found
+    // so far are counted per value of the next digit in a 256-bin histogram (LDS atomics of this wave on its own
+    // bins); lane l then owns the four highest undecided digits 255 - 4l .. 252 - 4l, a prefix sum over the lanes
+    // gives the number of keys above them, and the one lane whose digits straddle the wanted rank names the digit.
+    __shared__ __attribute__((aligned(16))) uint32_t hist_all[4][256];
+    uint32_t* keys = lds_keys + (size_t)wave * N;
+    const int nit = (N + 63) / 64;
+    for (int i = lane; i < N; i += 64) keys[i] = order_key<LOW_BIT>(IO::ld(s[i]));
+    uint32_t thr = 0;          // digits decided so far
+    int need = T;              // rank of the threshold among the keys that agree with them
+    uint32_t* hist = hist_all[wave];
+#pragma unroll
+    for (int hi = 32; hi > LOW_BIT;) {
+      const int w = (hi - LOW_BIT) < 8 ? (hi - LOW_BIT) : 8;
+      const int shift = hi - w;
+      *reinterpret_cast<i32x4_t*>(&hist[4 * lane]) = i32x4_t{0, 0, 0, 0};
+      wave_lds_fence();
+      for (int e = 0; e < nit; ++e) {
+        const int i = e * 64 + lane;
+        const uint32_t kv = i < N ? keys[i] : 0u;
+        if (i < N && (hi == 32 || ((kv ^ thr) >> (hi & 31)) == 0)) atomicAdd(&hist[(kv >> shift) & ((1u << w) - 1u)], 1u);
+      }
+      wave_lds_fence();
+      const i32x4_t c4 = *reinterpret_cast<const i32x4_t*>(&hist[252 - 4 * lane]);    // digits 252 - 4l .. 255 - 4l
+      const int c[4] = {c4[3], c4[2], c4[1], c4[0]};                                   // in descending order of the digit
+      const int mine = c[0] + c[1] + c[2] + c[3];
+      const int incl = wave_inclusive_sum(mine, lane);
+      const int above = incl - mine;               // keys (among those that agree) whose digit is above all of this lane's
+      const bool here = above < need && need <= incl;
+      int digit = 0, rest = 0;
+#pragma unroll
+      for (int jj = 0; jj < 4; ++jj) {             // (at most one of the four digits straddles the rank)
+        int before = above;
+#pragma unroll
+        for (int t = 0; t < jj; ++t) before += c[t];
+        if (before < need && need <= before + c[jj]) {
+          digit = 255 - 4 * lane - jj;
+          rest = need - before;
+        }
+      }
+      const unsigned long long who = __ballot(here);
+      const int src = who ? (int)__builtin_ctzll(who) : 0;
+      digit = __builtin_amdgcn_readlane(digit, src);
+      need = __builtin_amdgcn_readlane(rest, src);
+      thr |= (uint32_t)digit << shift;
+      hi = shift;
+    }
+    int run_eq = 0, run_sel = 0;
+    for (int e = 0; e < nit; ++e) {
+      const int i = e * 64 + lane;
+      const bool in = i < N;
+      const uint32_t kv = in ? keys[i] : 0u;
+      const bool eq = in && kv == thr;
+      const unsigned long long beq = __ballot(eq);
+      const bool sel = (in && kv > thr) || (eq && run_eq + lanes_before(beq) < need);
+      const unsigned long long bsel = __ballot(sel);
+      const int pos = run_sel + lanes_before(bsel);
+      if (in && sparse_map) sparse_map[row * N + i] = sel ? 1 : 0;
+      if (sel && pos < T) {              // (pos < T always holds; the test keeps a wrong count from ever leaving the row)
+        if (lut64)
+          reinterpret_cast<long long*>(lut)[row * T + pos] = i;
+        else
+          reinterpret_cast<int*>(lut)[row * T + pos] = i;
+      }
+      run_eq += __popcll(beq);
+      run_sel += __popcll(bsel);
+    }
   }
+}
+
+// ---- scores and selection in one launch, rows of at most 128 key blocks ------------------------------------------------
+// One workgroup of eight waves per 32 query blocks of a head: the waves form the 32 x N scores (16-bit inputs: tiles of 32 x
+// 32 on the matrix cores; fp32 inputs: every product and sum rounded on the vector ALU as in score_kernel), keep them in LDS,
+// rounded, and then select for four rows each.  The scores never go to memory and a launch is saved: mask builder of 2
+// heads x 1024 x 64 in fp32 25.3 -> 19.6 us, of 32 x 7813 x 64 38.1 -> 35.0.  With longer rows the two kernels, spread over more
+// workgroups, are as fast or faster (12 heads x 9360 x 128, 128-row query blocks: 36.5 us against 39.0; 2 x 75600: 62 against 77).
+constexpr int SELECT_FUSED_N = 128;
+template <typename IO, int D>
+__global__ __launch_bounds__(512) void select_kernel(const typename IO::raw* __restrict__ pq, const typename IO::raw* __restrict__ pk,
+                                                     int8_t* __restrict__ sparse_map, void* __restrict__ lut, int lut64, int M,
+                                                     int N, int T) {
+  typedef typename IO::raw raw;
+  constexpr int EB = sizeof(raw), EPL = SELECT_FUSED_N / 64;
+  constexpr int OS = 64 * EPL + 4 / EB;     // scores between rows
+  constexpr int RS = D * 4 + 16;            // bytes between rows of an fp32 q tile
+  __shared__ __attribute__((aligned(16))) uint8_t sq[EB == 4 ? 32 * RS : 16];
+  __shared__ __attribute__((aligned(16))) raw ss[32 * OS];
+  const int bh = blockIdx.y, m0 = blockIdx.x * 32;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int r = lane & 31, h = lane >> 5;
+  if constexpr (EB == 2) {
+    if (wave * 32 < N) {                    // (at most four tiles)
+      ScoreFrags<IO, D> a, b;
+      a.load(pq, bh, M, blockIdx.x, lane);
+      b.load(pk, bh, N, wave, lane);
+      const f32x16_t acc = score_tile<IO, D>(a, b);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) ss[(8 * (i >> 2) + (i & 3) + 4 * h) * OS + 32 * wave + r] = IO::st(acc[i]);
+    }
+  } else {
+    constexpr int NC = D / 4;               // 16-byte pieces per row
+    const __amdgpu_buffer_rsrc_t qh = make_rsrc(pq + (size_t)bh * M * D, (uint32_t)M * D * EB);    // rows past the end read as zero
+    const __amdgpu_buffer_rsrc_t kh = make_rsrc(pk + (size_t)bh * N * D, (uint32_t)N * D * EB);
+    for (int p = tid; p < 32 * NC; p += 512) {
+      const int row = p / NC, pc = p % NC;
+      *reinterpret_cast<i16x8_t*>(sq + row * RS + pc * 16) = buf_load_b128(qh, (uint32_t)(m0 + row) * (D * EB) + 16 * pc);
+    }
+    __syncthreads();
+    // item = (tile of 32 key blocks, group of 8 rows): a lane forms four scores of its key block
+    for (int it = wave; (it >> 2) * 32 < N; it += 8) {
+      const int t = it >> 2, g8 = 8 * (it & 3) + 4 * h;
+      const uint32_t koff = (uint32_t)(32 * t + r) * (D * EB);
+      float acc[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+      for (int c = 0; c < NC; ++c) {
+        const f32x4_t b = __builtin_bit_cast(f32x4_t, buf_load_b128(kh, koff + 16 * c));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const f32x4_t a = *reinterpret_cast<const f32x4_t*>(sq + (g8 + i) * RS + c * 16);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const float prod = a[j] * b[j];
+            acc[i] = acc[i] + prod;
+          }
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) ss[(g8 + i) * OS + 32 * t + r] = IO::st(acc[i]);
+    }
+  }
+  __syncthreads();
+  const int mw = m0 + 4 * wave;                // this wave's four rows
+  if (mw >= M) return;
+  const size_t row0 = (size_t)bh * M + mw;
+  const int rows = min(4, M - mw);
+  if (T <= 0) {              // nothing to select: all-zero map rows, no table rows
+    if (sparse_map)
+      for (int x = 0; x < rows; ++x)
+        for (int i = lane; i < N; i += 64) sparse_map[(row0 + x) * N + i] = 0;
+    return;
+  }
+  uint32_t kx[4][EPL];
+#pragma unroll
+  for (int x = 0; x < 4; ++x)
+#pragma unroll
+    for (int e = 0; e < EPL; ++e)
+      kx[x][e] = 64 * e + lane < N ? order_key<IO::KEY_LOW_BIT>(IO::ld(ss[(4 * wave + x) * OS + 64 * e + lane])) : 0u;
+  select_rows<EPL, IO::KEY_LOW_BIT, 4>(kx, nullptr, sparse_map, lut, lut64, row0, rows, N, T, lane);
 }
 
 template <typename IO>
@@ -586,6 +812,22 @@ static void launch_topk(const typename IO::raw* score, int8_t* sparse_map, void*
     hipLaunchKernelGGL((topk_kernel<IO, 0, LOW>), grid, block, (size_t)N * 16, st, score, sparse_map, lut, lut64, N, T, nrows);
 }
 
+// scores and selection (map row, look-up row) of every query block from the block means (in tiles where score_takes_tiled)
+template <typename IO>
+static void launch_select(const typename IO::raw* pq, const typename IO::raw* pk, int tiled, typename IO::raw* score,
+                          int8_t* sparse_map, void* lut, int lut64, int BH, int M, int N, int D, int T, hipStream_t st) {
+  if (N <= SELECT_FUSED_N && (D == 64 || D == 128)) {
+    const dim3 grid(cdiv(M, 32), BH);
+    if (D == 128)
+      hipLaunchKernelGGL((select_kernel<IO, 128>), grid, dim3(512), 0, st, pq, pk, sparse_map, lut, lut64, M, N, T);
+    else
+      hipLaunchKernelGGL((select_kernel<IO, 64>), grid, dim3(512), 0, st, pq, pk, sparse_map, lut, lut64, M, N, T);
+    return;
+  }
+  launch_score<IO>(pq, pk, tiled, score, BH, M, N, D, st);
+  launch_topk<IO>(score, sparse_map, lut, lut64, N, T, (size_t)BH * M, st);
+}
+
 struct MapWs {
   size_t chunk_sums, group_sums, colmean, pq, pk, score, total;
 };
@@ -598,8 +840,9 @@ static MapWs map_ws(int dtype, int BH, int L, int D, int BLKQ, int BLKK) {
   w.chunk_sums = off; off += align_up((int64_t)BH * nchunk * D * 4, 256);
   w.group_sums = off; off += align_up((int64_t)BH * cdiv((int)nchunk, KMEAN_GROUP) * D * 4, 256);
   w.colmean = off;    off += align_up((int64_t)BH * D * eb, 256);
-  w.pq = off;         off += align_up((int64_t)BH * M * D * eb, 256);
-  w.pk = off;         off += align_up((int64_t)BH * N * D * eb, 256);
+  // (whole tiles of 32 rows per head, as the score kernels read them)
+  w.pq = off;         off += align_up((int64_t)BH * align_up(M, 32) * D * eb, 256);
+  w.pk = off;         off += align_up((int64_t)BH * align_up(N, 32) * D * eb, 256);
   w.score = off;      off += align_up((int64_t)BH * M * N * eb, 256);
   w.total = off;
   return w;
@@ -622,12 +865,12 @@ static int validate_pool(int dtype, int BH, int L, int D, int BLK) {
 
 template <typename IO, int MODE>
 static void launch_pool(const void* x, const RowLayout& lay, const void* colmean, void* out, int BH, int L, int D, int BLK,
-                        hipStream_t st) {
+                        hipStream_t st, int tiled = 0) {
   const int nblk = cdiv(L, BLK);
   const int bpw = 256 / (D / IO::VEC);
   dim3 grid(cdiv(nblk, bpw), BH);
   hipLaunchKernelGGL((pool_kernel<IO, MODE>), grid, dim3(256), 0, st, (const typename IO::raw*)x, lay,
-                     (const typename IO::raw*)colmean, out, L, D, BLK, nblk);
+                     (const typename IO::raw*)colmean, out, L, D, BLK, nblk, tiled);
 }
 
 // levels 2 and 3 of the K column mean from the chunk sums
@@ -661,19 +904,19 @@ static int block_map_impl(const void* q, const void* k, const RowLayout& lay, in
   typename IO::raw* pq = (typename IO::raw*)(ws + w.pq);
   typename IO::raw* pk = (typename IO::raw*)(ws + w.pk);
   typename IO::raw* score = (typename IO::raw*)(ws + w.score);
+  const int tiled = score_takes_tiled(dtype, D);
   {
     // k chunk sums and q block means share one launch
     const int nchunk = cdiv(L, KMEAN_CHUNK);
     const int bpw = 256 / (D / IO::VEC);
     dim3 grid(cdiv(max(nchunk, M), bpw), BH, 2);
     hipLaunchKernelGGL((pool_pair_kernel<IO>), grid, dim3(256), 0, st, (const typename IO::raw*)k, chunk_sums, nchunk,
-                       (const typename IO::raw*)q, lay, pq, BLKQ, M, L, D);
+                       (const typename IO::raw*)q, lay, pq, BLKQ, M, L, D, tiled);
   }
   launch_colmean_reduce<IO>(chunk_sums, (float*)(ws + w.group_sums), colmean, BH, L, D, st);
-  launch_pool<IO, 2>(k, lay, colmean, pk, BH, L, D, BLKK, st);
-  launch_score<IO>(pq, pk, score, BH, M, N, D, st);
-  // topk == 0 selects nothing: the kernel then only clears the map row.
-  launch_topk<IO>(score, sparse_map, lut, lut64, N, topk, (size_t)BH * M, st);
+  launch_pool<IO, 2>(k, lay, colmean, pk, BH, L, D, BLKK, st, tiled);
+  // (topk == 0 selects nothing: the map rows are cleared)
+  launch_select<IO>(pq, pk, tiled, score, sparse_map, lut, lut64, BH, M, N, D, topk, st);
   return check_launch("block map");
 }
 
@@ -697,15 +940,16 @@ void launch_k_colmean(const void* k, const RowLayout& lay, int dtype, int BH, in
 }
 
 // Scores and top-k selection from block means computed elsewhere (the quantisers of the SageSLA path
-// produce them on the way): pq (BH, M, D), pk (BH, N, D) in `dtype`; score: (BH, M, N) elements of `dtype`.
+// produce them on the way): pq (BH, M, D), pk (BH, N, D) in `dtype`, in tiles where score_takes_tiled says so; score:
+// (BH, M, N) elements of `dtype`.
 void launch_map_from_pooled(int dtype, const void* pq, const void* pk, void* score, int BH, int M, int N, int D, int topk,
                             int8_t* sparse_map, void* lut, int lut64, hipStream_t st) {
   if (dtype == SLA_BF16) {
-    launch_score<IoBf16>((const uint16_t*)pq, (const uint16_t*)pk, (uint16_t*)score, BH, M, N, D, st);
-    launch_topk<IoBf16>((const uint16_t*)score, sparse_map, lut, lut64, N, topk, (size_t)BH * M, st);
+    const int tiled = score_takes_tiled(dtype, D);
+    launch_select<IoBf16>((const uint16_t*)pq, (const uint16_t*)pk, tiled, (uint16_t*)score, sparse_map, lut, lut64, BH, M, N, D, topk, st);
   } else {
-    launch_score<IoF16>((const uint16_t*)pq, (const uint16_t*)pk, (uint16_t*)score, BH, M, N, D, st);
-    launch_topk<IoF16>((const uint16_t*)score, sparse_map, lut, lut64, N, topk, (size_t)BH * M, st);
+    const int tiled = score_takes_tiled(dtype, D);
+    launch_select<IoF16>((const uint16_t*)pq, (const uint16_t*)pk, tiled, (uint16_t*)score, sparse_map, lut, lut64, BH, M, N, D, topk, st);
   }
 }
 

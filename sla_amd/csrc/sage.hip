@@ -10,6 +10,7 @@
 //   S = (q_int8 . k_int8) * sq * sk * scale ; P = softmax numerators over the selected blocks ;
 //   O = (e4m3(c P) . v_fp8) * sv / sum(e4m3(c P)), c = 112 with P <= 4 (reference maximum lagging by <= 2).
 // The look-up table of the bf16 path is used as is (no delta encoding is needed here).
+#include "block_map.h"
 #include "common.h"
 #include "sage_steps.h"
 
@@ -30,7 +31,7 @@ template <typename Tag, int D, int BLK, bool SUB_MEAN, bool POOL>
 __global__ __launch_bounds__(256) void quant_int8_kernel(const uint16_t* __restrict__ x, const RowLayout lay,
                                                          const uint16_t* __restrict__ colmean, int8_t* __restrict__ xq,
                                                          float* __restrict__ scale, uint16_t* __restrict__ pooled, int L,
-                                                         int nblk) {
+                                                         int nblk, int tiled) {
   using E = Elem<Tag>;
   constexpr int CPR = D / 8;
   constexpr int RPP = 256 / CPR;
@@ -98,7 +99,8 @@ __global__ __launch_bounds__(256) void quant_int8_kernel(const uint16_t* __restr
       for (int i = 0; i < BATCH; ++i) acc = acc + E::to_float(t[i]);
     }
     for (; r < nrows; ++r) acc = acc + E::to_float(tile[r * TSTR + tid]);
-    pooled[((size_t)bh * nblk + blk) * D + tid] = E::from_float(acc / (float)nrows);
+    pooled[tiled ? tiled_head(bh, nblk, D) + tiled_pos(blk, tid, D) : ((size_t)bh * nblk + blk) * D + tid] =
+        E::from_float(acc / (float)nrows);
   }
 #pragma unroll
   for (int p = 0; p < NP; ++p) {
@@ -499,8 +501,8 @@ static SagePrepWs sage_prep_ws(int BH, int L, int D) {
   const int64_t M = cdiv(L, 128), N = cdiv(L, 64);
   SagePrepWs w;
   size_t off = sage_ws(BH, L, D).total;
-  w.pq = off;    off += align_up((int64_t)BH * M * D * 2, 256);
-  w.pk = off;    off += align_up((int64_t)BH * N * D * 2, 256);
+  w.pq = off;    off += align_up((int64_t)BH * align_up(M, 32) * D * 2, 256);      // (whole tiles of 32)
+  w.pk = off;    off += align_up((int64_t)BH * align_up(N, 32) * D * 2, 256);
   w.score = off; off += align_up((int64_t)BH * M * N * 2, 256);
   w.total = off;
   return w;
@@ -531,9 +533,9 @@ static int quant_qk_impl(const void* q, const void* k, int dtype, int BH, int L,
   const RowLayout lay = contiguous_layout(BH, L, D);
   launch_k_colmean(k, lay, dtype, BH, L, D, (float*)(ws + w.chunk_sums), ws + w.colmean, st);
   hipLaunchKernelGGL((quant_int8_kernel<Tag, D, 128, false, false>), dim3(M, BH), dim3(256), 0, st, (const uint16_t*)q, lay,
-                     nullptr, q8, qs, nullptr, L, M);
+                     nullptr, q8, qs, nullptr, L, M, 0);
   hipLaunchKernelGGL((quant_int8_kernel<Tag, D, 64, true, false>), dim3(N, BH), dim3(256), 0, st, (const uint16_t*)k, lay,
-                     (const uint16_t*)(ws + w.colmean), k8, ks, nullptr, L, N);
+                     (const uint16_t*)(ws + w.colmean), k8, ks, nullptr, L, N, 0);
   return check_launch("sage_quant_qk");
 }
 
@@ -555,11 +557,12 @@ static int prepare_impl(const void* q, const void* k, const void* v, const RowLa
   const int M = cdiv(L, 128), N = cdiv(L, 64);
   uint16_t* pq = (uint16_t*)(ws + p.pq);
   uint16_t* pk = (uint16_t*)(ws + p.pk);
+  const int tiled = score_takes_tiled(dtype, D);
   launch_k_colmean(k, lay, dtype, BH, L, D, (float*)(ws + w.chunk_sums), ws + w.colmean, st);
   hipLaunchKernelGGL((quant_int8_kernel<Tag, D, 128, false, true>), dim3(M, BH), dim3(256), 0, st, (const uint16_t*)q, lay,
-                     nullptr, q8, qs, pq, L, M);
+                     nullptr, q8, qs, pq, L, M, tiled);
   hipLaunchKernelGGL((quant_int8_kernel<Tag, D, 64, true, true>), dim3(N, BH), dim3(256), 0, st, (const uint16_t*)k, lay,
-                     (const uint16_t*)(ws + w.colmean), k8, ks, pk, L, N);
+                     (const uint16_t*)(ws + w.colmean), k8, ks, pk, L, N, tiled);
   launch_map_from_pooled(dtype, pq, pk, ws + p.score, BH, M, N, D, topk, sparse_map, lut, lut64, st);
   int rc = check_launch("sage_prepare");
   if (rc || !v) return rc;

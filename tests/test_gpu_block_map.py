@@ -120,3 +120,30 @@ def test_widest_supported_row(dev):
     with pytest.raises(AssertionError, match="4096"):
         get_block_map(torch.zeros(1, 1, L + 1, 32, dtype=torch.bfloat16, device=dev),
                       torch.zeros(1, 1, L + 1, 32, dtype=torch.bfloat16, device=dev), 0.01, 128, 64)
+
+
+@pytest.mark.parametrize("H,L,D,BLKQ,ratio,dtype", [
+    (2, 8192, 128, 64, 0.1, torch.bfloat16),     # 128 key blocks: the last size scored and selected in one launch
+    (2, 8193, 64, 128, 0.1, torch.float16),      # 129: two launches, short list from one maximum per lane (T = 12)
+    (1, 8150, 64, 64, 0.24, torch.float32),      # 128, fp32, a ragged last block
+    (1, 20000, 128, 128, 0.2, torch.bfloat16),   # 313 key blocks, T = 62: short list from two maxima per lane
+    (1, 20000, 64, 128, 0.4, torch.bfloat16),    # T = 125: the search over all keys
+    (1, 66000, 64, 128, 0.03, torch.float16)])   # 1032 key blocks, T = 30
+def test_selection_paths(dev, H, L, D, BLKQ, ratio, dtype):
+    """The ways a row is selected, by its length and by the number of selected blocks, at the sizes where they change."""
+    g = torch.Generator().manual_seed(L + D)
+    q, k = (torch.randn(1, H, L, D, generator=g).to(dtype) for _ in range(2))
+    m_ref, lut_ref, T = O.get_block_map(q, k, ratio, BLKQ, 64)
+    m, lut, T2 = get_block_map(q.to(dev), k.to(dev), ratio, BLKQ, 64)
+    assert T == T2 and torch.equal(m.cpu(), m_ref) and torch.equal(lut.cpu().long(), lut_ref.long())
+
+
+@pytest.mark.parametrize("L", [4096, 20000])
+def test_selection_among_equal_scores(dev, L):
+    """Most scores of a row equal: the short list overflows and the lowest indices win."""
+    q = torch.ones(1, 1, L, 64, dtype=torch.bfloat16)
+    k = torch.ones(1, 1, L, 64, dtype=torch.bfloat16)
+    k[:, :, 640:704] = 3.0
+    m_ref, lut_ref, T = O.get_block_map(q, k, 0.1, 64, 64)
+    m, lut, _ = get_block_map(q.to(dev), k.to(dev), 0.1, 64, 64)
+    assert torch.equal(m.cpu(), m_ref) and torch.equal(lut.cpu().long(), lut_ref.long())
