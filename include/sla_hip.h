@@ -57,6 +57,7 @@ extern "C" {
 #define SLA_WS_LINEAR_COMPLEMENT_BWD 8
 #define SLA_WS_MODULE_FWD 9    /* dtype: that of the inputs */
 #define SLA_WS_LINEAR_BWD_STATES_APART 10 /* linear_workspace of sla_module_bwd_states */
+#define SLA_WS_SAGE_MODULE_FWD 11
 
 /* flags of sla_linear_bwd */
 #define SLA_BWD_ACCUMULATE 1   /* dq, dk, dv already hold the sparse branch's gradients: add to them */
@@ -329,6 +330,18 @@ int sage_quant_v_strided(const void* v, const int64_t* v_strides, int dtype, int
 int sla_linear_out_fwd_strided(const void* q, const int64_t* q_strides, const float* bias, const void* residual, void* out,
                                const int64_t* out_strides, int dtype, int fmap, int B, int H, int L, int D,
                                void* workspace, int64_t workspace_bytes, void* stream);
+
+/* Forward of the whole quantised module in one call, q, k, v in `dtype`: the kernels of
+ * sla_linear_state_quant_v_fwd, sage_prepare (without v), sage_sparse_attn_fwd and sla_linear_out_fwd, bit-identical
+ * results; 128-row query blocks and 64-row key blocks.  qkv_strides / out_strides: both or neither (contiguous).
+ * side_stream (optional, same device, default priority): for large inputs the state build and the quantisation of v run
+ * on it beside the rest of the preparation; `stream` waits for it before the call returns.
+ * Workspace: SLA_WS_SAGE_MODULE_FWD.
+ * Replaces SageSparseLinearAttention.forward, SageSLA/core.py:75-163. */
+int sage_module_fwd(const void* q, const void* k, const void* v, const int64_t* qkv_strides, const float* weight,
+                    const float* bias, void* out, const int64_t* out_strides, int dtype, int fmap, int B, int H, int L,
+                    int D, int topk, float qk_scale, float v_range, void* workspace, int64_t workspace_bytes,
+                    void* stream, void* side_stream);
 
 #ifdef __cplusplus
 }

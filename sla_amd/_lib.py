@@ -20,7 +20,8 @@ SLA_MASK_GIVEN = -1
 _DTYPE_CODES = {torch.float32: SLA_F32, torch.bfloat16: SLA_BF16, torch.float16: SLA_F16}
 FMAP = {"elu": 0, "relu": 1, "softmax": 2}
 (WS_BLOCK_MAP, WS_SPARSE_BWD, WS_LINEAR_FWD, WS_LINEAR_BWD, WS_SAGE_QUANT, WS_LINEAR_COMPLEMENT, WS_SAGE_PREPARE,
- WS_LINEAR_STATES, WS_LINEAR_COMPLEMENT_BWD, WS_MODULE_FWD, WS_LINEAR_BWD_STATES_APART) = range(11)
+ WS_LINEAR_STATES, WS_LINEAR_COMPLEMENT_BWD, WS_MODULE_FWD, WS_LINEAR_BWD_STATES_APART,
+ WS_SAGE_MODULE_FWD) = range(12)
 BWD_ACCUMULATE, BWD_STATES_READY = 1, 2
 
 ERR_BAD_ARG, ERR_UNSUPPORTED, ERR_LAUNCH, ERR_WORKSPACE = -1, -2, -3, -4
@@ -66,6 +67,7 @@ SIGNATURES = {
                                    _I, _I, _I, _I, _F, _P, _I64, _P, _I64, _P, _P]),
     "sla_module_fwd": (_I, [_P, _P, _P, _P, _I, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _F,
                             _P, _I64, _P, _P]),
+    "sage_module_fwd": (_I, [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _F, _P, _I64, _P, _P]),
     "sage_quant_qk": (_I, [_P, _P, _I, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _I64, _P]),
     "sage_prepare": (_I, [_P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P, _P, _I, _P, _P, _P, _P, _P, _P, _F, _P, _I64, _P]),
     "sage_quant_v": (_I, [_P, _I, _I, _I, _I, _I, _P, _P, _F, _P, _I64, _P]),

@@ -83,6 +83,7 @@ int64_t sage_prepare_workspace_bytes(int BH, int L, int D);
 int64_t linear_states_bytes(int BH, int L, int D);
 int64_t linear_complement_workspace_bytes(int BH, int L, int D);
 int64_t linear_complement_bwd_workspace_bytes(int BH, int L, int D, int BLKQ);
+int64_t sage_module_workspace_bytes(int B, int H, int L, int D, int topk);
 int64_t linear_bwd_states_apart_bytes(int BH, int L, int D);
 int64_t module_fwd_workspace_bytes(int in_dtype, int BH, int L, int D, int BLKQ, int BLKK);
 
@@ -127,6 +128,9 @@ extern "C" int64_t sla_workspace_bytes(int op, int dtype, int B, int H, int L, i
       SLA_REQUIRE(BLKQ > 0 && BLKK > 0, SLA_ERR_BAD_ARG, "non-positive block size");
       SLA_REQUIRE(dtype == SLA_F32 || dtype == SLA_BF16 || dtype == SLA_F16, SLA_ERR_BAD_ARG, "unknown dtype %d", dtype);
       return module_fwd_workspace_bytes(dtype, BH, L, D, BLKQ, BLKK);
+    case SLA_WS_SAGE_MODULE_FWD:
+      SLA_REQUIRE(topk >= 0, SLA_ERR_BAD_ARG, "bad topk");
+      return sage_module_workspace_bytes(B, H, L, D, topk);
     default:
       set_error("unknown workspace op %d", op);
       return SLA_ERR_BAD_ARG;

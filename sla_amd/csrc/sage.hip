@@ -13,10 +13,12 @@
 #include "block_map.h"
 #include "common.h"
 #include "sage_steps.h"
+#include "side_events.h"
 
 namespace sla {
 
 int64_t k_colmean_scratch_floats(int BH, int L, int D);
+int64_t linear_fwd_workspace_bytes(int BH, int L, int D);
 void launch_k_colmean(const void* k, const RowLayout& lay, int dtype, int BH, int L, int D, float* scratch, void* colmean,
                       hipStream_t st);
 void launch_map_from_pooled(int dtype, const void* pq, const void* pk, void* score, int BH, int M, int N, int D, int topk,
@@ -627,7 +629,7 @@ extern "C" int sage_quant_qk(const void* q, const void* k, int dtype, int B, int
 static int prepare_entry(const void* q, const void* k, const void* v, const int64_t* qkv_strides, int dtype, int B, int H, int L,
                          int D, int BLKQ, int BLKK, int topk, int8_t* sparse_map, void* lut, int lut_elem_bytes, int8_t* q_int8,
                          float* q_scale, int8_t* k_int8, float* k_scale, uint8_t* v_fp8, float* v_scale, float v_range,
-                         void* workspace, int64_t workspace_bytes, void* stream) {
+                         void* workspace, int64_t workspace_bytes, void* stream, bool want_map = true) {
   int rc = validate_sage(dtype, B, H, L, D, BLKQ, BLKK);
   if (rc) return rc;
   rc = validate_v_range(v_range);
@@ -642,7 +644,7 @@ static int prepare_entry(const void* q, const void* k, const void* v, const int6
               lut_elem_bytes);
   // (v, v_fp8 and v_scale may all three be NULL: the caller then quantises v itself with sage_quant_v, e.g. on another
   //  stream)
-  SLA_REQUIRE(q && k && sparse_map && (lut || topk == 0) && q_int8 && q_scale && k_int8 && k_scale && workspace &&
+  SLA_REQUIRE(q && k && (sparse_map || !want_map) && (lut || topk == 0) && q_int8 && q_scale && k_int8 && k_scale && workspace &&
                   ((v && v_fp8 && v_scale) || (!v && !v_fp8 && !v_scale)),
               SLA_ERR_BAD_ARG, "null pointer");
   SLA_REQUIRE(((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)lut | (uintptr_t)q_int8 | (uintptr_t)k_int8 |
@@ -749,4 +751,96 @@ extern "C" int sage_sparse_attn_fwd(const int8_t* q_int8, const float* q_scale, 
   if (D == 128) { SAGE_CASE(f16_tag, 128); }
   SAGE_CASE(f16_tag, 64);
 #undef SAGE_CASE
+}
+
+// ---- the whole quantised forward in one call -----------------------------------------------------------------------
+namespace sla {
+struct SageModuleWs {
+  int64_t prep_bytes, linear_bytes;
+  size_t prep, linear, q8, k8, v8, qs, ks, vs, lut, o_s, total;
+};
+static SageModuleWs sage_module_ws(int B, int H, int L, int D, int topk) {
+  const int64_t BH = (int64_t)B * H, M = cdiv(L, 128), N = cdiv(L, 64), elems = BH * L * D;
+  SageModuleWs w;
+  w.prep_bytes = sage_prepare_workspace_bytes((int)BH, L, D);
+  w.linear_bytes = linear_fwd_workspace_bytes((int)BH, L, D);
+  size_t off = 0;
+  w.prep = off;   off += align_up(w.prep_bytes, 256);
+  w.linear = off; off += align_up(w.linear_bytes, 256);
+  w.q8 = off;     off += align_up(elems, 256);
+  w.k8 = off;     off += align_up(elems, 256);
+  w.v8 = off;     off += align_up(elems, 256);
+  w.qs = off;     off += align_up(BH * M * 4, 256);
+  w.ks = off;     off += align_up(BH * N * 4, 256);
+  w.vs = off;     off += align_up(BH * D * 4, 256);
+  w.lut = off;    off += align_up(BH * M * topk * 4, 256);
+  w.o_s = off;    off += align_up(elems * 2, 256);
+  w.total = off;
+  return w;
+}
+int64_t sage_module_workspace_bytes(int B, int H, int L, int D, int topk) {
+  return (int64_t)sage_module_ws(B, H, L, D, topk).total;
+}
+}  // namespace sla
+
+extern "C" int sage_module_fwd(const void* q, const void* k, const void* v, const int64_t* qkv_strides, const float* weight,
+                               const float* bias, void* out, const int64_t* out_strides, int dtype, int fmap, int B, int H, int L,
+                               int D, int topk, float qk_scale, float v_range, void* workspace, int64_t workspace_bytes,
+                               void* stream, void* side_stream) {
+  int rc = validate_sage(dtype, B, H, L, D, 128, 64);
+  if (rc) return rc;
+  SLA_REQUIRE((qkv_strides == nullptr) == (out_strides == nullptr), SLA_ERR_BAD_ARG, "pass both stride arrays or neither");
+  SLA_REQUIRE(topk >= 0 && topk <= cdiv(L, 64), SLA_ERR_BAD_ARG, "topk=%d outside [0, %d]", topk, cdiv(L, 64));
+  SLA_REQUIRE(fmap == SLA_FMAP_ELU || fmap == SLA_FMAP_RELU || fmap == SLA_FMAP_SOFTMAX, SLA_ERR_BAD_ARG,
+              "unknown feature map %d", fmap);
+  SLA_REQUIRE(q && k && v && weight && bias && out && workspace, SLA_ERR_BAD_ARG, "null pointer");
+  SLA_REQUIRE(((uintptr_t)workspace | (uintptr_t)weight | (uintptr_t)out) % 16 == 0, SLA_ERR_BAD_ARG,
+              "pointers must be 16-byte aligned");
+  const SageModuleWs w = sage_module_ws(B, H, L, D, topk);
+  SLA_REQUIRE(workspace_bytes >= (int64_t)w.total, SLA_ERR_WORKSPACE, "workspace of %lld bytes, need %lld",
+              (long long)workspace_bytes, (long long)w.total);
+  RowLayout lay;                       // (what the steps would find wrong with the strides, before the first launch)
+  if ((rc = make_layout(qkv_strides, B, H, L, D, 2, &lay))) return rc;
+  if ((rc = make_layout(out_strides, B, H, L, D, 2, &lay))) return rc;
+  char* ws = (char*)workspace;
+  hipStream_t st = (hipStream_t)stream, side = (hipStream_t)side_stream;
+  int8_t *q8 = (int8_t*)(ws + w.q8), *k8 = (int8_t*)(ws + w.k8);
+  uint8_t* v8 = (uint8_t*)(ws + w.v8);
+  float *qs = (float*)(ws + w.qs), *ks = (float*)(ws + w.ks), *vs = (float*)(ws + w.vs);
+  void *lut = ws + w.lut, *o_s = ws + w.o_s;
+  const auto state = [&](hipStream_t s) {
+    return qkv_strides ? sla_linear_state_quant_v_fwd_strided(k, v, qkv_strides, weight, dtype, fmap, B, H, L, D, ws + w.linear,
+                                                              w.linear_bytes, v8, vs, v_range, s)
+                       : sla_linear_state_quant_v_fwd(k, v, weight, dtype, fmap, B, H, L, D, ws + w.linear, w.linear_bytes, v8,
+                                                      vs, v_range, s);
+  };
+  const auto prepare = [&]() {
+    return prepare_entry(q, k, nullptr, qkv_strides, dtype, B, H, L, D, 128, 64, topk, nullptr, lut, 4, q8, qs, k8, ks, nullptr,
+                         nullptr, v_range, ws + w.prep, w.prep_bytes, stream, false);
+  };
+  const auto attention = [&]() -> int {
+    int r = sage_sparse_attn_fwd(q8, qs, k8, ks, v8, vs, lut, 4, o_s, dtype, B, H, L, D, 128, 64, topk, qk_scale, stream);
+    if (r) return r;
+    return qkv_strides ? sla_linear_out_fwd_strided(q, qkv_strides, bias, o_s, out, out_strides, dtype, fmap, B, H, L, D,
+                                                    ws + w.linear, w.linear_bytes, stream)
+                       : sla_linear_out_fwd(q, bias, o_s, out, dtype, fmap, B, H, L, D, ws + w.linear, w.linear_bytes, stream);
+  };
+  if (!side || side == st || !side_stream_pays(B, H, L, D)) {
+    if ((rc = state(st))) return rc;
+    if ((rc = prepare())) return rc;
+    return attention();
+  }
+  std::lock_guard<std::mutex> lock(side_events_mutex());
+  SideEvents* ev;
+  if ((rc = side_events_for_current_device(&ev))) return rc;
+  SLA_HIP_OK(hipEventRecord(ev->fork, st));
+  SLA_HIP_OK(hipStreamWaitEvent(side, ev->fork, 0));
+  // (once the second stream waits on `stream`, no path leaves without `stream` waiting for it in turn)
+  rc = state(side);
+  const int rc_prep = prepare();
+  SLA_HIP_OK(hipEventRecord(ev->first, side));
+  SLA_HIP_OK(hipStreamWaitEvent(st, ev->first, 0));
+  if (rc) return rc;
+  if (rc_prep) return rc_prep;
+  return attention();
 }

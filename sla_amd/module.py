@@ -9,7 +9,7 @@ import torch.nn as nn
 
 from . import _lib
 from .block_map import get_block_map, topk_count
-from .linear import linear_complement_bwd, linear_complement_fwd, linear_state_fwd, linear_state_quant_v_fwd
+from .linear import linear_complement_bwd, linear_complement_fwd, linear_state_fwd
 from .sparse_attn import sparse_attn_bwd, sparse_attn_fwd
 
 FEATURE_MAPS = ("elu", "relu", "softmax")
@@ -256,17 +256,11 @@ class _StateBuild:
 
     _side = {}
 
-    def __init__(self, k, v, weight, fmap, quant_v_range=None):
-        """``quant_v_range``: also quantise ``v`` to FP8 with that range in the same library call (``self.v_fp8``,
-        ``self.v_scale``, ready after ``join``)."""
+    def __init__(self, k, v, weight, fmap):
         dev = k.device
-        self.v_fp8 = self.v_scale = None
 
         def build():
-            if quant_v_range is None:
-                self.ws = linear_state_fwd(k, v, weight, fmap)
-            else:
-                self.ws, self.v_fp8, self.v_scale = linear_state_quant_v_fwd(k, v, weight, fmap, quant_v_range)
+            self.ws = linear_state_fwd(k, v, weight, fmap)
 
         cur = torch.cuda.current_stream(dev)
         if torch.cuda.is_current_stream_capturing():
@@ -282,19 +276,6 @@ class _StateBuild:
         side.wait_stream(cur)    # k, v and the weight were produced on the calling stream
         with torch.cuda.stream(side):
             build()
-        for t in (self.v_fp8, self.v_scale):
-            if t is not None:
-                t.record_stream(cur)         # allocated under the side stream, consumed on the calling one
-
-    def also(self, fn, *args):
-        """Runs ``fn(*args)`` behind the state build, on the same side stream; its results are ready after ``join``."""
-        if self.side is None:
-            return fn(*args)
-        with torch.cuda.stream(self.side):
-            res = fn(*args)
-        for t in (res if isinstance(res, tuple) else (res,)):
-            t.record_stream(torch.cuda.current_stream(t.device))
-        return res
 
     def join(self):
         if self.side is not None:

@@ -12,7 +12,7 @@ import torch.nn as nn
 from . import _lib
 from .block_map import get_block_map, topk_count
 from .linear import linear_out_fwd
-from .module import FEATURE_MAPS, _StateBuild
+from .module import FEATURE_MAPS, _side_stream, _StateBuild
 
 SAGE_BLKQ, SAGE_BLKK = 128, 64
 # Range of the e4m3 values v is quantised to.  The reference's call passes 2.25 (SageSLA/core.py:129), which keeps the
@@ -117,6 +117,29 @@ def sage_attn_fwd(q8, qs, k8, ks, v8, vs, lut, topk, out_dtype, qk_scale=None):
     return o
 
 
+def _sage_module_fwd(q, k, v, weight, bias, topk_ratio, fmap):
+    """The whole quantised forward as one library call (``sage_module_fwd``); q, k, v in the compute dtype, contiguous or
+    row-contiguous views with common strides (the output then has q's memory order)."""
+    B, H, L, D = q.shape
+    dev = q.device
+    dt = _lib.dtype_code(q.dtype)
+    T = topk_count(-(-L // SAGE_BLKK), topk_ratio)
+    n = _lib.workspace_bytes(_lib.WS_SAGE_MODULE_FWD, dt, B, H, L, D, SAGE_BLKQ, SAGE_BLKK, T)
+    ws = torch.empty(n, dtype=torch.uint8, device=dev)
+    if q.is_contiguous() and k.is_contiguous() and v.is_contiguous():
+        s_in = s_out = None
+        out = torch.empty((B, H, L, D), dtype=q.dtype, device=dev)
+    else:
+        assert _lib.row_strided(q, k, v), "q, k, v must be contiguous or share row-contiguous strides"
+        out = _lib.empty_like_rows(q)
+        s_in, s_out = _lib.strides_arg(q), _lib.strides_arg(out)
+    rc = _lib.load().sage_module_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), s_in, weight.data_ptr(), bias.data_ptr(),
+                                     out.data_ptr(), s_out, dt, _lib.FMAP[fmap], B, H, L, D, T, D ** -0.5, V_RANGE_E4M3,
+                                     ws.data_ptr(), n, _lib.stream_ptr(dev), _side_stream(dev))
+    _lib.check(rc)
+    return out
+
+
 class SageSparseLinearAttention(nn.Module):
     def __init__(self, head_dim, topk, feature_map="softmax", use_bf16=True, tie_feature_map_qk=True, BLKQ=SAGE_BLKQ,
                  BLKK=SAGE_BLKK):
@@ -157,27 +180,22 @@ class SageSparseLinearAttention(nn.Module):
             v = v.contiguous()
         headdim = q.size(-1)
         assert headdim in [64, 128], "headdim should be in [64, 128]. For other headdim, you can use padding and specify the softmax scale."
-        # The k/v half of the linear branch runs on a side stream beside the preparation and the attention
-        # kernel (measured best when started first: 0.570 against 0.593 ms serial at H12 L32760).
+        weight, bias = self.proj_l.weight.contiguous(), self.proj_l.bias.contiguous()
         if q.dtype == k.dtype == v.dtype == self.dtype:
-            # v, which neither the mask nor the q / k quantisers need, is quantised with the state build on the side
-            # stream: the state kernel streams v anyway and finds the column maxima the quantiser starts from
-            state = _StateBuild(k, v, self.proj_l.weight, self.feature_map, quant_v_range=V_RANGE_E4M3)
-            v8, vs = state.v_fp8, state.v_scale
-            # the mask sees the same values as the quantisers: one pass structure for both
-            sparse_map, lut, real_topk, q8, qs, k8, ks, _, _ = sage_prepare(q, k, None, self.topk)
-            state.join()
+            # the mask sees the same values as the quantisers: one library call for everything
+            o = _sage_module_fwd(q, k, v, weight, bias, self.topk, self.feature_map)
         else:
             # the mask is built from the inputs as given, the quantisers work in the compute dtype (core.py:96-100)
-            sparse_map, lut, real_topk = get_block_map(q, k, topk_ratio=self.topk, BLKQ=SAGE_BLKQ, BLKK=SAGE_BLKK)
+            _, lut, T = get_block_map(q, k, topk_ratio=self.topk, BLKQ=SAGE_BLKQ, BLKK=SAGE_BLKK)
             q = q.to(self.dtype)
             k = k.to(self.dtype)
             v = v.to(self.dtype)
-            state = _StateBuild(k, v, self.proj_l.weight, self.feature_map)
+            state = _StateBuild(k, v, weight, self.feature_map)
             q8, qs, k8, ks = quant_qk(q, k)
             v8, vs = quant_v(v)
-        o_s = sage_attn_fwd(q8, qs, k8, ks, v8, vs, lut, real_topk, self.dtype)
-        o = linear_out_fwd(q, self.proj_l.bias, o_s, state.join(), self.feature_map).to(dtype)
+            o_s = sage_attn_fwd(q8, qs, k8, ks, v8, vs, lut, T, self.dtype)
+            o = linear_out_fwd(q, bias, o_s, state.join(), self.feature_map).to(dtype)
         if return_sparsity:
-            return o, real_topk / sparse_map.shape[-1]
+            N = -(-q.shape[2] // SAGE_BLKK)
+            return o, topk_count(N, self.topk) / N
         return o

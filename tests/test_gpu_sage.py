@@ -106,6 +106,31 @@ def test_state_build_with_v_quantised_in_the_same_call(dev, L, D, dtype, fmap, v
     assert torch.equal(linear_out_fwd(qd, bd, None, ws2, fmap), out_ref)
 
 
+@pytest.mark.parametrize("H,L,D,half,fmap", [(3, 577, 128, False, "elu"), (2, 1001, 64, True, "softmax"), (2, 4097, 64, False, "relu"),
+                                             (12, 6001, 128, False, "softmax")])      # (the last one from 16 MiB per tensor on)
+@pytest.mark.parametrize("rows_in_place", [False, True])
+def test_module_in_one_call_equals_the_steps(dev, H, L, D, half, fmap, rows_in_place):
+    """The whole forward as one library call: bit for bit the preparation, attention and linear calls by themselves."""
+    from sla_amd.linear import linear_out_fwd, linear_state_quant_v_fwd
+    dtype = torch.float16 if half else torch.bfloat16
+    g = torch.Generator().manual_seed(L + D)
+    q, k, v = (torch.randn(1, L, H, D, generator=g).to(dtype).to(dev).transpose(1, 2) for _ in range(3))
+    if not rows_in_place:
+        q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
+    mod = SageSparseLinearAttention(D, 0.1, fmap, use_bf16=not half).to(dev)
+    with torch.no_grad():
+        for p, t in zip((mod.proj_l.weight, mod.proj_l.bias), make_proj(D)):
+            p.copy_(t)
+        for _ in range(2):                               # (twice: the events between the streams are used again)
+            out, density = mod(q, k, v, return_sparsity=True)
+        m, lut, T, q8, qs, k8, ks, _, _ = sage_prepare(q, k, None, 0.1)
+        ws, v8, vs = linear_state_quant_v_fwd(k, v, mod.proj_l.weight, fmap)
+        o_s = sage_attn_fwd(q8, qs, k8, ks, v8, vs, lut, T, dtype)
+        ref = linear_out_fwd(q, mod.proj_l.bias, o_s, ws, fmap)
+    assert torch.equal(out, ref) and out.dtype == dtype and density == T / m.shape[-1]
+    assert out.stride() == ref.stride()
+
+
 @pytest.mark.parametrize("L,D,ratio", [(512, 128, 0.5), (1000, 128, 0.3), (333, 64, 0.5), (2048, 128, 0.1)])
 def test_attention_vs_fp32_and_vs_quantised_oracle(dev, L, D, ratio):
     q, k, v = _qkv(L, D, L + 1)
