@@ -385,13 +385,31 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 // arithmetic it shares (S^T = K Q^T and dP^T = V dO^T, so that the log-sum-exp and delta of a query are per-lane
 // scalars and dS^T leaves the accumulator as the B operand of dQ^T += K^T dS^T).  What differs:
 //   * the wave owns all 64 query rows (two tiles of 32): Q^T and dO^T fragments and the dQ^T accumulators fill the
-//     accumulation registers, and every transposed K fragment read from LDS feeds two products;
-//   * K and V go from memory straight into LDS, 32 keys at a time, two generations each, swizzled like the Q / dO
-//     rows of bwd_dkdv_stream_kernel; the 32 keys after next are requested as soon as the current ones are used up
-//     (the transposed K fragments wait in registers), a unit and a half before they are wanted;
-//   * inside a unit of 32 keys the two query tiles are staggered: S, dP of tile 0 | S, dP of tile 1 beside the
-//     vector arithmetic of tile 0 | dQ of tile 0 beside the vector arithmetic of tile 1 | dQ of tile 1.
+//     accumulation registers, and every K or V fragment read from LDS feeds the products of both tiles;
+//   * K and V go from memory straight into LDS, 32 keys at a time, two generations each, swizzled; a generation takes the
+//     32 keys after next as soon as its fragments have been read (the transposed K fragments wait in registers);
+//   * the loop is rotated: S and dP of both tiles of unit u + 1 (32 products) run beside the vector arithmetic of unit u,
+//     then come dQ of unit u (16 products) beside the requests and the transposed fragments of unit u + 1.
+// A lone wave issues one instruction per four cycles at best, and every one of them takes its turn with the 48 products
+// (1536 cycles) of a unit, so instructions are what is saved: the accumulators of dP start from -delta instead of zero
+// (no subtraction per element), four requests share one M0, every LDS offset but eight is an instruction immediate: 272
+// instructions per unit where reading the row-wise fragments once per tile took 367.  Measured, that version against this:
+// B1 H12 L32760 with 25 key blocks per row 551 -> 485 us (matrix pipe busy 53 -> 61 % of the cycles, at a clock that the
+// power limit holds at 1.65 GHz), B2 H16 L32760 with 128-row blocks 1428 -> 1224 us, B2 H4 L4096 37.9 -> 33.2 us.
 constexpr int DQ_STREAM_MAX_T = 2048;          // look-up rows longer than this take bwd_dq_kernel
+
+// Four requests of 16 bytes per lane, memory -> LDS, REQ_PITCH bytes apart in LDS.  The instruction offset counts for both
+// addresses: off[j] is the memory offset less j * REQ_PITCH (never negative: REQ_SLACK bytes are part of it and of a
+// descriptor that starts as many bytes early).
+constexpr int REQ_PITCH = 1040;                // 4 rows of 256 bytes + 16 bytes of padding
+constexpr int REQ_SLACK = 64;
+template <int J>
+static __device__ __forceinline__ void lds_dma_row4(__amdgpu_buffer_rsrc_t rsrc, uint32_t off, uint32_t lds) {
+  if constexpr (J == 0)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds), "v"(off), "s"(rsrc) : "memory");
+  else
+    asm volatile("buffer_load_dwordx4 %0, %1, 0 offen offset:%2 lds" ::"v"(off), "s"(rsrc), "n"(J * REQ_PITCH) : "memory");
+}
 
 template <typename Tag>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void bwd_dq_stream_kernel(
@@ -403,7 +421,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
   using E = Elem<Tag>;
   constexpr int D = 128, DC = D / 16, DT = D / 32;
   constexpr int ROWB = D * 2;
-  constexpr int TILE = 32 * ROWB;                 // 32 rows of K or V
+  constexpr int TILE = 8 * REQ_PITCH;             // 32 rows of K or V
   __shared__ __attribute__((aligned(16))) uint8_t smem[4 * TILE];      // K generation 0, 1; V generation 0, 1
   __shared__ uint16_t entries[DQ_STREAM_MAX_T];                        // this block's look-up row
 
@@ -420,8 +438,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
   const uint32_t row_bytes = pitch * 2;
   const __amdgpu_buffer_rsrc_t qh = make_rsrc(q + head_off, lin.head_range_bytes(L, D));
   const __amdgpu_buffer_rsrc_t doh = make_rsrc(d_o + ldo.head(bh), ldo.head_range_bytes(L, D));
-  const __amdgpu_buffer_rsrc_t kh = make_rsrc(k + head_off, lin.head_range_bytes(L, D));
-  const __amdgpu_buffer_rsrc_t vh = make_rsrc(v + head_off, lin.head_range_bytes(L, D));
+  const __amdgpu_buffer_rsrc_t kh = make_rsrc(k + head_off - REQ_SLACK / 2, lin.head_range_bytes(L, D) + REQ_SLACK);
+  const __amdgpu_buffer_rsrc_t vh = make_rsrc(v + head_off - REQ_SLACK / 2, lin.head_range_bytes(L, D) + REQ_SLACK);
   const int qrow0 = mb * 64;
 
   // The first 64 entries of the look-up row are asked for before anything else: the first requests for K and V hang on
@@ -434,7 +452,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
   // The rows of the forward's output come the same way: delta = rowsum(dO * O) (reference kernel.py:282-286, the
   // preprocess step) is formed here, for this block's rows, and written out for the dK/dV kernel.
   i16x8_t qf[2][DC], dof[2][DC], of[2][DC];
-  float lse_q[2], delta_q[2];
+  float lse_q[2];
+  f32x16_t neg_delta[2];                          // sixteen copies of -delta: what the accumulators of dP start from
   const __amdgpu_buffer_rsrc_t oh = make_rsrc(o + (size_t)bh * L * D, (uint32_t)L * D * 2);      // (contiguous (B, H, L, D))
 #pragma unroll
   for (int qt = 0; qt < 2; ++qt) {
@@ -453,7 +472,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
   // key rows past L are never written into LDS: what LDS holds in their place has to be finite (their probabilities
   // are masked to exactly 0 below)
 #pragma unroll
-  for (int i = 0; i < 4 * TILE / 16 / 64; ++i) reinterpret_cast<i32x4_t*>(smem)[i * 64 + lane] = i32x4_t{0, 0, 0, 0};
+  for (int i = 0; i < (4 * TILE / 16 + 63) / 64; ++i)
+    if (i * 64 + lane < 4 * TILE / 16) reinterpret_cast<i32x4_t*>(smem)[i * 64 + lane] = i32x4_t{0, 0, 0, 0};
   wave_lds_fence();
 
   f32x16_t dqacc[DT][2];
@@ -464,151 +484,162 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
 #pragma unroll
       for (int i = 0; i < 16; ++i) dqacc[dt][qt][i] = 0.f;
 
-  // ---- addressing (see bwd_dkdv_stream_kernel) ----
-  auto swz = [](int row) __attribute__((always_inline)) { return ((row & 3) << 2) | ((row >> 2) & 3); };
+  // ---- addressing ----
+  // A request moves 4 rows (64 lanes x 16 bytes): lane -> row 4 j + lane / 16, 16-byte slot lane % 16, which receives
+  // piece (slot ^ 4 (row % 4)) of that row; requests are padded by one 16-byte slot.  For one piece the 16 rows of a
+  // row-wise read hit 16 different slots (row % 4 picks the group of four, row / 4 the slot in it), and so do the
+  // 4 rows x 4 pieces of a transposing read.
   const uint32_t smem_addr = __builtin_amdgcn_readfirstlane((uint32_t)(size_t)smem);
   const int lrow = lane >> 4, lslot = lane & 15;
-  uint32_t koff[4];                  // request j covers rows 4 j + lane / 16 of the 32: j % 4 here, 16 rows more for j >= 4
+  uint32_t koff[4];                  // rows 4 j + lane / 16; sixteen rows more for the second half of a tile
 #pragma unroll
-  for (int j = 0; j < 4; ++j) koff[j] = (uint32_t)(4 * j + lrow) * row_bytes + (uint32_t)(lslot ^ swz(4 * j + lrow)) * 16;
-  const int nunits = 2 * topk;
-  auto unit_rows = [&](int u) __attribute__((always_inline)) -> int {           // first key row of unit u; past the end: the last unit again
-    const int uc = min(u, nunits - 1);
-    return __builtin_amdgcn_readfirstlane((int)entries[uc >> 1]) * 64 + 32 * (uc & 1);
+  for (int j = 0; j < 4; ++j)
+    koff[j] = (uint32_t)(4 * j + lrow) * row_bytes + (uint32_t)(lslot ^ (4 * lrow)) * 16 + REQ_SLACK - j * REQ_PITCH;
+  const uint32_t half_bytes = 16 * row_bytes;
+  const int row_none = (L + 63) & ~63;            // past every head: such requests touch neither memory nor LDS
+  auto entry_row0 = [&](int e) __attribute__((always_inline)) -> int {
+    const int row0 = __builtin_amdgcn_readfirstlane((int)entries[min(e, topk - 1)]) * 64;
+    return e < topk ? row0 : row_none;
   };
-  auto request = [&](int key0, int GEN) __attribute__((always_inline)) {
-    const uint32_t rb = (uint32_t)key0 * row_bytes;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const uint32_t off = koff[j & 3] + rb + (uint32_t)(j >> 2) * 16 * row_bytes;
-      lds_dma_b128(kh, off, smem_addr, GEN * TILE + j * 1024);
-      lds_dma_b128(vh, off, smem_addr, (2 + GEN) * TILE + j * 1024);
-    }
-  };
-  int rfo[DC];
-#pragma unroll
-  for (int c = 0; c < DC; ++c) rfo[c] = r * ROWB + (((2 * c + g) ^ swz(r & 15)) * 16);
+  // request J (rows 4 J ..) of the 32 rows from key0 on, into the tile at LDS address `tile`
+#define SLA_DQ_REQUEST(RSRC, J, KEY0, TILE_AT)                                                                       \
+  lds_dma_row4<(J) & 3>(RSRC, koff[(J) & 3] + ((uint32_t)(KEY0) * row_bytes + ((J) >= 4 ? half_bytes : 0u)),          \
+                        smem_addr + (uint32_t)(TILE_AT) + ((J) >> 2) * 4 * REQ_PITCH)
+  // fragments: row-wise, row r, piece 2 c + g: one base per c / 2; transposed, rows tr_row and tr_row + 8 (and 16 further
+  // for the second half), 8 bytes at element 4 (lane % 4) of the 16-column strip 2 dt + (lane / 16) % 2: one base per dt
+  const uint8_t* rfp[4];
+  const uint8_t* tfp[DT];
   const int tr_row = 4 * g + ((lane & 15) >> 2);
-  int tfo[2][DT];
 #pragma unroll
-  for (int h = 0; h < 2; ++h)
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt) {
-      const int row = tr_row + 8 * h;
-      const int piece = 4 * dt + 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1);
-      tfo[h][dt] = row * ROWB + ((piece ^ swz(row & 15)) * 16) + (lane & 1) * 8;
+  for (int i = 0; i < 4; ++i) {
+    rfp[i] = smem + r * ROWB + (r >> 2) * 16 + ((4 * i + g) ^ (4 * (r & 3))) * 16;
+    tfp[i] = smem + tr_row * ROWB + (tr_row >> 2) * 16 +
+             ((4 * i + 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1)) ^ (4 * (tr_row & 3))) * 16 + (lane & 1) * 8;
+  }
+  i16x8_t af[3], bf[3];              // row-wise K and V fragments, two chunks ahead
+  i16x8_t trk[2][DT];                // transposed K fragments of the unit whose dQ products come next
+  auto row_frags = [&](int GEN, int c) __attribute__((always_inline)) {
+    af[c % 3] = *reinterpret_cast<const i16x8_t*>(rfp[c >> 1] + GEN * TILE + (c & 1) * 32);
+    bf[c % 3] = *reinterpret_cast<const i16x8_t*>(rfp[c >> 1] + (2 + GEN) * TILE + (c & 1) * 32);
+  };
+  auto tr_frag = [&](int GEN, int c2, int dt) __attribute__((always_inline)) {
+    const uint8_t* t0 = tfp[dt] + GEN * TILE + 4 * c2 * REQ_PITCH;
+    trk[c2][dt] = concat4(lds_read_tr16(reinterpret_cast<const uint16_t*>(t0)),
+                          lds_read_tr16(reinterpret_cast<const uint16_t*>(t0 + 2 * REQ_PITCH)));
+  };
+
+  struct Tiles {
+    f32x16_t s[2], dp[2];            // S^T and dP^T - delta of the two query tiles
+  };
+  Tiles ta, tb;
+  i32x4_t dsw[2][2];                 // dS^T of the two query tiles, packed: B operands of the dQ products
+  // element i of tile qt: P = exp2(S c - lse), then dS = P (dP - delta), two per packed word
+  auto prob = [&](Tiles& t, int qt, int i) __attribute__((always_inline)) {
+    float p = fast_exp2(__builtin_fmaf(t.s[qt][i], c_log2e, -lse_q[qt]));
+    asm volatile("" : "+v"(p));
+    t.s[qt][i] = p;
+  };
+  auto grad = [&](Tiles& t, int qt, int i) __attribute__((always_inline)) {
+    float ds = t.s[qt][i] * t.dp[qt][i];
+    asm volatile("" : "+v"(ds));
+    t.dp[qt][i] = ds;
+    if (i & 1) {
+      uint32_t a = E::pack2(t.dp[qt][i - 1], t.dp[qt][i]);
+      asm volatile("" : "+v"(a));
+      dsw[qt][i >> 3][(i >> 1) & 3] = (int)a;
     }
-  // One unit = 32 keys, 48 MFMAs.  GEN = u % 2.
-  f32x16_t s0, dp0, s1, dp1;
-  auto unit = [&](int GEN, int key0, int key0_next2) __attribute__((always_inline)) {
-    asm volatile("s_waitcnt vmcnt(16)" ::: "memory");          // this unit's rows have landed (the next unit's 16 requests may be out)
-    const uint8_t* kg = smem + GEN * TILE;
-    const uint8_t* vg = smem + (2 + GEN) * TILE;
-    const int valid = L - key0;                                // key rows of this unit that exist
-    i16x8_t af[4], bf[4];                                      // row-wise fragments, three products ahead
-    auto first_products = [&](f32x16_t& s, f32x16_t& dp, const i16x8_t (&qq)[DC], const i16x8_t (&dd)[DC], auto&& beside)
-        __attribute__((always_inline)) {
+  };
+  // product 4 c + {0, 1, 2, 3} of the 32: S and dP of tile 0, then of tile 1, chunk c of the head dimension
+  auto score_product = [&](Tiles& t, int c, int which) __attribute__((always_inline)) {
+    const int qt = which >> 1;
+    if (which & 1) {
+      if (c == 0) mfma_scores_first<Tag>(t.dp[qt], bf[0], dof[qt][0], neg_delta[qt]);
+      else mfma_scores<Tag>(t.dp[qt], bf[c % 3], dof[qt][c]);
+    } else {
+      if (c == 0) mfma_scores_first<Tag>(t.s[qt], af[0], qf[qt][0]);
+      else mfma_scores<Tag>(t.s[qt], af[c % 3], qf[qt][c]);
+    }
+  };
+  auto mask_tail = [&](Tiles& t, int valid) __attribute__((always_inline)) {   // key index of register i is 8 (i / 4) + i % 4 + 4 g
+    const int lim = valid - 4 * g;
 #pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        af[c] = *reinterpret_cast<const i16x8_t*>(kg + rfo[c]);
-        bf[c] = *reinterpret_cast<const i16x8_t*>(vg + rfo[c]);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int c = 0; c < DC; ++c) {
-        if (c + 3 < DC) {
-          af[(c + 3) & 3] = *reinterpret_cast<const i16x8_t*>(kg + rfo[c + 3]);
-          bf[(c + 3) & 3] = *reinterpret_cast<const i16x8_t*>(vg + rfo[c + 3]);
-        }
-        if (c == 0) mfma_scores_first<Tag>(s, af[0], qq[0]);
-        else mfma_scores<Tag>(s, af[c & 3], qq[c]);
-        beside(2 * c);
-        __builtin_amdgcn_sched_barrier(0);
-        if (c == 0) mfma_scores_first<Tag>(dp, bf[0], dd[0]);
-        else mfma_scores<Tag>(dp, bf[c & 3], dd[c]);
-        beside(2 * c + 1);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    };
-    // element i of a tile: dS^T = P^T (dP^T - delta), P = exp2(S c - lse); packed in pairs into the B operand
-    auto element = [&](f32x16_t& s, f32x16_t& dp, int qt, i32x4_t (&dsw)[2], int i) __attribute__((always_inline)) {
-      float p = fast_exp2(__builtin_fmaf(s[i], c_log2e, -lse_q[qt]));
-      float ds = p * (dp[i] - delta_q[qt]);
-      asm volatile("" : "+v"(ds));
-      s[i] = ds;
-      if (i & 1) {
-        uint32_t a = E::pack2(s[i - 1], s[i]);
-        asm volatile("" : "+v"(a));
-        dsw[i >> 3][(i >> 1) & 3] = (int)a;
-      }
-    };
-    auto mask_tail = [&](f32x16_t& s) __attribute__((always_inline)) {       // key index of register i is 8 (i / 4) + i % 4 + 4 g
-      const int lim = valid - 4 * g;
+    for (int qt = 0; qt < 2; ++qt)
 #pragma unroll
       for (int i = 0; i < 16; ++i)
-        if (8 * (i >> 2) + (i & 3) >= lim) s[i] = -INFINITY;
-    };
-    i32x4_t dsw0[2], dsw1[2];
-    first_products(s0, dp0, qf[0], dof[0], [](int) __attribute__((always_inline)) {});
-    // (the vector ALU keeps off a product's result for two products' time: the elements start in slot 2)
-    first_products(s1, dp1, qf[1], dof[1], [&](int sl) __attribute__((always_inline)) {
-      if (sl == 2 && __builtin_expect(valid < 32, 0)) mask_tail(s0);
-      if (sl >= 2) element(s0, dp0, 0, dsw0, sl - 2);
-      if (sl >= 14) element(s0, dp0, 0, dsw0, sl);             // sixteen elements in fourteen slots
-    });
-    // second products: transposed K fragments, fetched once and used by both query tiles
-    i16x8_t trk[2][DT];
-#pragma unroll
-    for (int c2 = 0; c2 < 2; ++c2)
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt) {
-        const uint8_t* t0 = kg + 16 * c2 * ROWB;
-        trk[c2][dt] = concat4(lds_read_tr16(reinterpret_cast<const uint16_t*>(t0 + tfo[0][dt])),
-                              lds_read_tr16(reinterpret_cast<const uint16_t*>(t0 + tfo[1][dt])));
-      }
+        if (8 * (i >> 2) + (i & 3) >= lim) t.s[qt][i] = -INFINITY;
+  };
+
+  // One iteration = unit u (generation GU = u % 2), 48 products:
+  //   slots  0..31  S and dP of unit u + 1 into `nxt`        beside: P and dS of unit u (in `cur`), K rows 16.. of unit u + 2
+  //   slots 32..47  dQ += K^T dS of unit u                    beside: V and K rows 0..15 of unit u + 3, and from unit u + 1
+  //                                                           the transposed K fragments, from u + 2 the first row-wise ones
+  // Requests are answered in order.  When the row-wise fragments of unit u + 2 are first read, only the eight requests for
+  // V of unit u + 3 may be out; a tile half is requested again only behind a product that waited for LDS reads issued after
+  // the last read of that half (LDS reads return in order).
+  auto iteration = [&](int GU, Tiles& cur, Tiles& nxt, int key_u, int key_u2, int key_u3) __attribute__((always_inline)) {
+    const int GN = GU ^ 1;
+    if (__builtin_expect(L - key_u < 32, 0)) mask_tail(cur, L - key_u);
     __builtin_amdgcn_sched_barrier(0);
-    if (__builtin_expect(valid < 32, 0)) {
-      asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
-      mask_tail(s1);
-    }
 #pragma unroll
-    for (int sl = 0; sl < 8; ++sl) {
-      const int c2 = sl >> 2, dt = sl & 3;
-      dqacc[dt][0] = E::mfma32(trk[c2][dt], __builtin_bit_cast(i16x8_t, dsw0[c2]), dqacc[dt][0]);
-      // This unit's V has been used up, its K is in registers (or on its way there): their generation takes the unit
-      // after next, a unit and a half before it is wanted.  One request per product: requests that follow each other
-      // closely wait for the compute unit's one vector-memory path, and a single wave waits with them.  V first.
-      {
-        const uint32_t off = koff[sl & 3] + (uint32_t)key0_next2 * row_bytes + (uint32_t)(sl >> 2) * 16 * row_bytes;
-        lds_dma_b128(vh, off, smem_addr, (2 + GEN) * TILE + sl * 1024);
-      }
-      if (sl >= 2) {
-        element(s1, dp1, 1, dsw1, 2 * (sl - 2));
-        element(s1, dp1, 1, dsw1, 2 * (sl - 2) + 1);
-      }
-      if (sl >= 6) {
-        element(s1, dp1, 1, dsw1, 12 + 2 * (sl - 6));
-        element(s1, dp1, 1, dsw1, 13 + 2 * (sl - 6));
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    }
+    for (int c = 0; c < DC; ++c) {
 #pragma unroll
-    for (int sl = 0; sl < 8; ++sl) {
-      const int c2 = sl >> 2, dt = sl & 3;
-      dqacc[dt][1] = E::mfma32(trk[c2][dt], __builtin_bit_cast(i16x8_t, dsw1[c2]), dqacc[dt][1]);
-      if (sl == 0) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");        // (every read of K has long returned)
-      const uint32_t off = koff[sl & 3] + (uint32_t)key0_next2 * row_bytes + (uint32_t)(sl >> 2) * 16 * row_bytes;
-      lds_dma_b128(kh, off, smem_addr, GEN * TILE + sl * 1024);
+      for (int which = 0; which < 4; ++which) {
+        const int sl = 4 * c + which;
+        score_product(nxt, c, which);
+        prob(cur, sl >> 4, sl & 15);
+        if (sl > 0) grad(cur, (sl - 1) >> 4, (sl - 1) & 15);
+        if (which == 1 && c + 2 < DC) row_frags(GN, c + 2);
+        if (sl == 12) SLA_DQ_REQUEST(kh, 4, key_u2, GU * TILE);
+        if (sl == 15) SLA_DQ_REQUEST(kh, 5, key_u2, GU * TILE);
+        if (sl == 18) SLA_DQ_REQUEST(kh, 6, key_u2, GU * TILE);
+        if (sl == 21) SLA_DQ_REQUEST(kh, 7, key_u2, GU * TILE);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    grad(cur, 1, 15);
+#pragma unroll
+    for (int sl = 0; sl < 16; ++sl) {
+      const int c2 = sl >> 3, dt = (sl >> 1) & 3, qt = sl & 1;
+      dqacc[dt][qt] = E::mfma32(trk[c2][dt], __builtin_bit_cast(i16x8_t, dsw[qt][c2]), dqacc[dt][qt]);
+      if (sl == 0) SLA_DQ_REQUEST(vh, 0, key_u3, (2 + GN) * TILE);
+      if (sl == 1) SLA_DQ_REQUEST(vh, 1, key_u3, (2 + GN) * TILE);
+      if (sl == 2) SLA_DQ_REQUEST(vh, 2, key_u3, (2 + GN) * TILE);
+      if (sl == 3) SLA_DQ_REQUEST(vh, 3, key_u3, (2 + GN) * TILE);
+      if (sl == 4) SLA_DQ_REQUEST(vh, 4, key_u3, (2 + GN) * TILE);
+      if (sl == 5) SLA_DQ_REQUEST(vh, 5, key_u3, (2 + GN) * TILE);
+      if (sl == 6) SLA_DQ_REQUEST(vh, 6, key_u3, (2 + GN) * TILE);
+      if (sl == 7) SLA_DQ_REQUEST(vh, 7, key_u3, (2 + GN) * TILE);
+      if (qt == 1) tr_frag(GN, c2, dt);
+      if (sl == 9) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+      if (sl == 10) row_frags(GU, 0);
+      if (sl == 12) row_frags(GU, 1);
+      if (sl == 12) {
+        asm volatile("s_waitcnt lgkmcnt(6)" ::: "memory");       // (K rows 0..15 of unit u + 1 have been read: eight reads came after)
+        SLA_DQ_REQUEST(kh, 0, key_u3, GN * TILE);
+      }
+      if (sl == 13) SLA_DQ_REQUEST(kh, 1, key_u3, GN * TILE);
+      if (sl == 14) SLA_DQ_REQUEST(kh, 2, key_u3, GN * TILE);
+      if (sl == 15) SLA_DQ_REQUEST(kh, 3, key_u3, GN * TILE);
       __builtin_amdgcn_sched_barrier(0);
     }
   };
 
-  int key_cur = 0, key_n1 = 0;
-  if (nunits > 0) {
-    key_cur = unit_rows(0);
-    key_n1 = unit_rows(1);
-    request(key_cur, 0);
-    request(key_n1, 1);
+  // first key rows of the listed blocks: E0 of the entry of units u and u + 1, E1 of the next one, E2 of the one after
+  int E0 = 0, E1 = 0, E2 = 0;
+  if (topk > 0) {
+    E0 = entry_row0(0);
+    E1 = entry_row0(1);
+    E2 = entry_row0(2);
+#define SLA_DQ_REQUEST8(RSRC, KEY0, TILE_AT)                                                                         \
+  SLA_DQ_REQUEST(RSRC, 0, KEY0, TILE_AT); SLA_DQ_REQUEST(RSRC, 1, KEY0, TILE_AT);                                    \
+  SLA_DQ_REQUEST(RSRC, 2, KEY0, TILE_AT); SLA_DQ_REQUEST(RSRC, 3, KEY0, TILE_AT);                                    \
+  SLA_DQ_REQUEST(RSRC, 4, KEY0, TILE_AT); SLA_DQ_REQUEST(RSRC, 5, KEY0, TILE_AT);                                    \
+  SLA_DQ_REQUEST(RSRC, 6, KEY0, TILE_AT); SLA_DQ_REQUEST(RSRC, 7, KEY0, TILE_AT)
+    SLA_DQ_REQUEST8(kh, E0, 0);
+    SLA_DQ_REQUEST8(vh, E0, 2 * TILE);
+    SLA_DQ_REQUEST8(kh, E0 + 32, TILE);
+    SLA_DQ_REQUEST8(vh, E0 + 32, 3 * TILE);
+#undef SLA_DQ_REQUEST8
   }
   // delta of this lane's two rows.  The sum runs in the order of bwd_delta_kernel, whose thread t adds the eight products
   // of columns 8t .. 8t+7 one after the other and then meets threads t^1, t^2, t^4, t^8: here t = 2c + g, so the first
@@ -627,7 +658,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
     for (int sh = 1; sh < DC; sh <<= 1)
 #pragma unroll
       for (int c = 0; c < DC; c += 2 * sh) part[c] = part[c] + part[c + sh];
-    delta_q[qt] = part[0];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) neg_delta[qt][i] = -part[0];
+    asm volatile("" : "+v"(neg_delta[qt]));
     const int qrow = qrow0 + 32 * qt + r;
     if (g == 0 && qrow < L) delta[(size_t)bh * L + qrow] = part[0];
   }
@@ -637,13 +670,55 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
   for (int qt = 0; qt < 2; ++qt)
 #pragma unroll
     for (int c = 0; c < DC; ++c) asm volatile("" : "+a"(qf[qt][c]), "+a"(dof[qt][c]));
-  for (int u = 0; u < nunits; u += 2) {
-    const int key_n2 = unit_rows(u + 2), key_n3 = unit_rows(u + 3);
-    unit(0, key_cur, key_n2);
-    unit(1, key_n1, key_n3);
-    key_cur = key_n2;
-    key_n1 = key_n3;
+  if (topk > 0) {
+    // (the two rows of delta written above count as memory operations too: two more may be out)
+    asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+    row_frags(0, 0);
+    row_frags(0, 1);
+#pragma unroll
+    for (int c = 0; c < DC; ++c) {
+#pragma unroll
+      for (int which = 0; which < 4; ++which) score_product(ta, c, which);
+      if (c + 2 < DC) row_frags(0, c + 2);
+    }
+#pragma unroll
+    for (int c2 = 0; c2 < 2; ++c2)
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) tr_frag(0, c2, dt);
+    // (the vector ALU reads the products' results next; every fragment of unit 0 has been read)
+    asm volatile("s_nop 15\n\ts_nop 15\n\ts_waitcnt lgkmcnt(0)" ::: "memory");
+    SLA_DQ_REQUEST(vh, 0, E1, 2 * TILE); SLA_DQ_REQUEST(vh, 1, E1, 2 * TILE); SLA_DQ_REQUEST(vh, 2, E1, 2 * TILE);
+    SLA_DQ_REQUEST(vh, 3, E1, 2 * TILE); SLA_DQ_REQUEST(vh, 4, E1, 2 * TILE); SLA_DQ_REQUEST(vh, 5, E1, 2 * TILE);
+    SLA_DQ_REQUEST(vh, 6, E1, 2 * TILE); SLA_DQ_REQUEST(vh, 7, E1, 2 * TILE);
+    SLA_DQ_REQUEST(kh, 0, E1, 0); SLA_DQ_REQUEST(kh, 1, E1, 0); SLA_DQ_REQUEST(kh, 2, E1, 0); SLA_DQ_REQUEST(kh, 3, E1, 0);
+    asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
+    row_frags(1, 0);
+    row_frags(1, 1);
+    for (int b = 0;; ++b) {
+      const int E3 = entry_row0(b + 3);                       // (looked up now, used two units from now)
+      iteration(0, ta, tb, E0, E1, E1 + 32);                  // unit 2 b
+      if (b + 1 >= topk) break;
+      iteration(1, tb, ta, E0 + 32, E1 + 32, E2);             // unit 2 b + 1
+      E0 = E1;
+      E1 = E2;
+      E2 = E3;
+    }
+    // the last unit: no scores left to form beside its arithmetic
+    if (__builtin_expect(L - (E0 + 32) < 32, 0)) mask_tail(tb, L - (E0 + 32));
+#pragma unroll
+    for (int qt = 0; qt < 2; ++qt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        prob(tb, qt, i);
+        grad(tb, qt, i);
+      }
+#pragma unroll
+    for (int sl = 0; sl < 16; ++sl) {
+      const int c2 = sl >> 3, dt = (sl >> 1) & 3, qt = sl & 1;
+      dqacc[dt][qt] = E::mfma32(trk[c2][dt], __builtin_bit_cast(i16x8_t, dsw[qt][c2]), dqacc[dt][qt]);
+    }
   }
+#undef SLA_DQ_REQUEST
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // (nothing of this workgroup is in flight when it ends)
 
   // The rounded rows go through LDS (the rings are free now) and leave as whole rows in streaming stores: they are not
