@@ -8,24 +8,39 @@
 //     the accumulators in the B-operand layout of dV^T += dO^T P and dK^T += Q^T dS.  Nothing is handed from wave
 //     to wave, and there is one barrier per 32 query rows;
 //   * Q and dO rows go from memory straight into LDS (buffer loads with the LDS bit), 32 rows at a time, into a
-//     ring of four generations; the rows of unit u + 3 are requested while unit u is worked on.  Rows are unpadded;
-//     the 16-byte pieces of a row are XOR-swizzled with the row index so that both the row-wise reads (A operands
-//     of S and dP) and the transposing reads (A operands of the second products) are free of bank conflicts;
+//     ring of four generations; a generation is requested two units of 32 rows before it is first read.  The
+//     16-byte pieces of a row are XOR-swizzled so that both the row-wise reads (A operands of S and dP) and the
+//     transposing reads (A operands of the second products) are free of bank conflicts;
 //   * the loop is rotated: the exponentials and the rest of the vector arithmetic of unit u run beside the first
-//     products of unit u + 1, then come the second products of unit u.
+//     products of unit u + 1, then come the second products of unit u;
+//   * a lone wave issues one instruction per four cycles at best, so instructions are what is saved: V^T is kept
+//     negated and the accumulators of -dP start from delta (no subtraction per element; dK comes out negated and is
+//     turned at the end), four requests share one M0, LDS offsets are instruction immediates: 225 instructions per
+//     unit of 32 products (1024 cycles of the matrix pipe) where 300 were needed without all that.  The barrier stands
+//     where the fragments of a unit have all been read, so that the first reads of the next unit and the requests for
+//     the unit after next run beside products.  Measured, before and after: B1 H12 L32760 with 25 key blocks per row
+//     840 -> 758 us (matrix pipe busy 45 -> 51 % of the cycles at 1.74 GHz, where the power limit holds it), B2 H16
+//     L32760 with 128-row query blocks 2272 -> 2065 us, B2 H4 L4096 48.5 -> 43.0 us.
 #pragma once
+#include <type_traits>
+
 #include "common.h"
 
 namespace sla {
 
-// 16 bytes per lane, memory -> LDS: lane l's piece lands at lds_base + lds_off + 16 l.  (Between a scalar write of M0
-// and a memory -> LDS load that reads it the hardware wants one wait state; the compiler adds it to its own code and
-// does not look into these instructions.)
-static __device__ __forceinline__ void lds_dma_b128(__amdgpu_buffer_rsrc_t rsrc, uint32_t byte_off, uint32_t lds_base,
-                                                    uint32_t lds_off) {
-  asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds_base), "v"(byte_off), "s"(rsrc),
-               "s"(lds_off)
-               : "memory", "scc");
+// One of four requests of 16 bytes per lane, memory -> LDS (lane l's piece lands 16 l bytes on), REQ_PITCH bytes apart in
+// LDS.  The instruction offset counts for both addresses: off is the memory offset less J * REQ_PITCH (never negative:
+// REQ_SLACK bytes are part of it and of a descriptor that starts as many bytes early).  J = 0 sets M0 for all four.
+// (Between a scalar write of M0 and a memory -> LDS load that reads it the hardware wants one wait state; the compiler
+// adds it to its own code and does not look into these instructions.)
+constexpr int REQ_PITCH = 1040;                // 4 rows of 256 bytes + 16 bytes of padding
+constexpr int REQ_SLACK = 64;
+template <int J>
+static __device__ __forceinline__ void lds_dma_row4(__amdgpu_buffer_rsrc_t rsrc, uint32_t off, uint32_t lds) {
+  if constexpr (J == 0)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds), "v"(off), "s"(rsrc) : "memory");
+  else
+    asm volatile("buffer_load_dwordx4 %0, %1, 0 offen offset:%2 lds" ::"v"(off), "s"(rsrc), "n"(J * REQ_PITCH) : "memory");
 }
 // 4 bytes per lane: lane l's word lands at lds_base + lds_off + 4 l
 static __device__ __forceinline__ void lds_dma_b32(__amdgpu_buffer_rsrc_t rsrc, uint32_t byte_off, uint32_t lds_base,
@@ -47,9 +62,9 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   // (wide = 1: the lists name 128-row query blocks; an entry is then walked as its two 64-row halves)
   using E = Elem<Tag>;
   constexpr int D = 128, DC = D / 16, DT = D / 32;
-  constexpr int ROWB = D * 2;               // bytes per row in LDS (unpadded)
-  constexpr int TILE = 32 * ROWB;           // 32 rows of Q or of dO
-  constexpr int GEN = 2 * TILE + 256;       // one generation: Q rows, dO rows, 32 log-sum-exps, 32 deltas
+  constexpr int ROWB = D * 2;               // bytes per row in LDS
+  constexpr int TILE = 8 * REQ_PITCH;       // 32 rows of Q or of dO
+  constexpr int GEN = 2 * TILE + 512;       // one generation: Q rows, dO rows, log-sum-exps, deltas (32 of 64 words used)
   constexpr int NG = 4;
   constexpr int NREQ = 9;                   // requests per wave and unit: 4 x Q, 4 x dO (its 16 rows), 1 x lse or delta
   __shared__ __attribute__((aligned(16))) uint8_t smem[NG * GEN];
@@ -75,8 +90,8 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 
   const size_t head_off = lin.head(bh);
   const uint32_t pitch = (uint32_t)lin.sl, pitch_do = (uint32_t)ldo.sl;
-  const __amdgpu_buffer_rsrc_t qh = make_rsrc(q + head_off, lin.head_range_bytes(L, D));
-  const __amdgpu_buffer_rsrc_t doh = make_rsrc(d_o + ldo.head(bh), ldo.head_range_bytes(L, D));
+  const __amdgpu_buffer_rsrc_t qh = make_rsrc(q + head_off - REQ_SLACK / 2, lin.head_range_bytes(L, D) + REQ_SLACK);
+  const __amdgpu_buffer_rsrc_t doh = make_rsrc(d_o + ldo.head(bh) - REQ_SLACK / 2, ldo.head_range_bytes(L, D) + REQ_SLACK);
   const __amdgpu_buffer_rsrc_t kb = make_rsrc(k + head_off, lin.head_range_bytes(L, D));
   const __amdgpu_buffer_rsrc_t vb = make_rsrc(v + head_off, lin.head_range_bytes(L, D));
   // wave 0 fetches the log-sum-exps of a unit, wave 1 its deltas
@@ -89,7 +104,7 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   const int e0 = sg * seg;
   const int count_lane = count[(size_t)bh * Nblk + nb];
   const int first_entry = mylist[min(e0 + (tid >> wide), Mblk - 1)];
-  // K^T and V^T fragments (B operands): this lane's key column, 8 adjacent d per chunk; parked in accumulation registers
+  // K^T and -V^T fragments (B operands): this lane's key column, 8 adjacent d per chunk; parked in accumulation registers
   const int krow = nb * 64 + w * 32 + r;
   const bool kok = krow < L;
   i16x8_t kf[DC], vf[DC];
@@ -116,219 +131,256 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   // this work item's part of the list, in units of 32 query rows (two per listed query block)
   const int e1 = min(__builtin_amdgcn_readfirstlane(count_lane), (sg + 1) * seg);
   const int nent = (e1 - e0) << wide;               // 64-row blocks this work item walks
-  const int nunits = 2 * nent;
-  auto entry_row0 = [&](int e) __attribute__((always_inline)) -> int {          // past the end: the last entry again (fetched, never used)
-    return __builtin_amdgcn_readfirstlane(entries[min(e, nent - 1)]) * 64;
+  const int row_none = (L + 63) & ~63;              // past every head: such requests touch neither memory nor LDS
+  auto entry_row0 = [&](int e) __attribute__((always_inline)) -> int {
+    const int row0 = __builtin_amdgcn_readfirstlane(entries[min(e, nent - 1)]) * 64;
+    return e < nent ? row0 : row_none;
   };
   if (tid < (seg << wide)) entries[tid] = (first_entry << wide) + (tid & wide);
   for (int i = 128 + tid; i < nent; i += 128) entries[i] = (mylist[e0 + (i >> wide)] << wide) + (i & wide);
 
   // ---- addressing ----
   // A request moves 4 rows (64 lanes x 16 bytes): lane -> row 4j + lane / 16 of this wave's 16 rows, 16-byte slot
-  // lane % 16, which receives piece (slot ^ swz(row)) of that row.  swz(row) = 4 (row % 4) + (row / 4) % 4: for one
-  // piece the 16 rows of a row-wise read hit 16 different slots, and the 4 rows x 4 pieces of a transposing read too.
-  auto swz = [](int row) __attribute__((always_inline)) { return ((row & 3) << 2) | ((row >> 2) & 3); };
+  // lane % 16, which receives piece (slot ^ 4 (row % 4)) of that row; requests are padded by one 16-byte slot.  For one
+  // piece the 16 rows of a row-wise read hit 16 different slots (row % 4 picks the group of four, row / 4 the slot in
+  // it), and so do the 4 rows x 4 pieces of a transposing read.
   const uint32_t smem_addr = (uint32_t)(size_t)smem;
   const int lrow = lane >> 4, lslot = lane & 15;
   uint32_t qoff[4], dooff[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    const int row = 16 * w + 4 * j + lrow;                     // row of the unit (16 w: a multiple of 16, no part in swz)
-    const uint32_t piece = (uint32_t)(lslot ^ swz(row & 15)) * 16;
-    qoff[j] = (uint32_t)row * pitch * 2 + piece;
-    dooff[j] = (uint32_t)row * pitch_do * 2 + piece;
+    const uint32_t row = 16 * w + 4 * j + lrow;                // row of the unit
+    const uint32_t piece = (uint32_t)(lslot ^ (4 * lrow)) * 16 + REQ_SLACK - j * REQ_PITCH;
+    qoff[j] = row * pitch * 2 + piece;
+    dooff[j] = row * pitch_do * 2 + piece;
   }
-  // LDS addresses of this wave's 16 rows inside a tile and of its 32 words (log-sum-exps or deltas) behind the tiles
-  const uint32_t rows_base = __builtin_amdgcn_readfirstlane(smem_addr + (uint32_t)(16 * w) * ROWB);
-  const uint32_t ld_base = __builtin_amdgcn_readfirstlane(smem_addr + (uint32_t)w * 128);
-  auto request = [&](int row0, int gen) __attribute__((always_inline)) {
-    const uint32_t base = (uint32_t)gen * GEN;
-    const uint32_t rq = (uint32_t)row0 * pitch * 2, rdo = (uint32_t)row0 * pitch_do * 2;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      lds_dma_b128(qh, qoff[j] + rq, rows_base, base + j * 1024);
-      lds_dma_b128(doh, dooff[j] + rdo, rows_base, base + TILE + j * 1024);
-    }
-    if (lane < 32) lds_dma_b32(ldh, (uint32_t)(row0 + lane) * 4, ld_base, base + 2 * TILE);
-  };
-  // row-wise fragment c of this lane: row r, piece 2c + g
-  int rfo[DC];
-#pragma unroll
-  for (int c = 0; c < DC; ++c) rfo[c] = r * ROWB + (((2 * c + g) ^ swz(r & 15)) * 16);
-  // transposed fragment (16 query rows x 32 d): rows 16 c2 + 4 g + (lane % 16) / 4 and 8 further on, 8 bytes at element
-  // 4 (lane % 4) of the 16-column strip 2 dt + (lane / 16) % 2
+  // LDS addresses of this wave's 16 rows inside a tile and of its words (log-sum-exps or deltas) behind the tiles
+  const uint32_t rows_base = __builtin_amdgcn_readfirstlane(smem_addr + (uint32_t)(4 * w) * REQ_PITCH);
+  const uint32_t ld_base = __builtin_amdgcn_readfirstlane(smem_addr + (uint32_t)w * 256);
+  const uint32_t lane4 = (uint32_t)lane * 4;
+#define SLA_DKDV_REQUEST_Q(J, ROW0, GENERATION) \
+  lds_dma_row4<J>(qh, qoff[J] + (uint32_t)(ROW0) * (pitch * 2), rows_base + (uint32_t)(GENERATION) * GEN)
+#define SLA_DKDV_REQUEST_DO(J, ROW0, GENERATION) \
+  lds_dma_row4<J>(doh, dooff[J] + (uint32_t)(ROW0) * (pitch_do * 2), rows_base + (uint32_t)(GENERATION) * GEN + TILE)
+#define SLA_DKDV_REQUEST_LD(ROW0, GENERATION) \
+  lds_dma_b32(ldh, lane4 + (uint32_t)(ROW0) * 4, ld_base, (uint32_t)(GENERATION) * GEN + 2 * TILE)
+  // fragments: row-wise, row r, piece 2c + g: one base per c / 2; transposed (16 query rows x 32 d), rows
+  // 16 c2 + 4 g + (lane % 16) / 4 and 8 further on, 8 bytes at element 4 (lane % 4) of the 16-column strip
+  // 2 dt + (lane / 16) % 2: one base per dt
+  const uint8_t* rfp[4];
+  const uint8_t* tfp[DT];
+  const uint8_t* const ldp = smem + 2 * TILE + 16 * g;       // log-sum-exps of rows 4g .. 4g + 3; deltas 256 bytes on
   const int tr_row = 4 * g + ((lane & 15) >> 2);
-  int tfo[2][DT];                    // [which of the two rows][dt], without the 16 c2 rows
 #pragma unroll
-  for (int h = 0; h < 2; ++h)
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt) {
-      const int row = tr_row + 8 * h;
-      const int piece = 4 * dt + 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1);
-      tfo[h][dt] = row * ROWB + ((piece ^ swz(row & 15)) * 16) + (lane & 1) * 8;
-    }
-
-  // ---- prologue: units 0, 1, 2 requested; S and dP of unit 0 ----
-  f32x16_t s_a, dp_a, s_b, dp_b;
-  __syncthreads();                                             // the zeros and the entries are in place before anything is requested
-  // first query rows of the listed blocks: E0 = of the entry of units u and u + 1, E1 = of the next one, E2 = of the one after
-  int E0 = 0, E1 = 0, E2 = 0;
-  if (nunits > 0) {
-    E0 = entry_row0(0);
-    E1 = entry_row0(1);
-    E2 = entry_row0(2);
-    request(E0, 0);
-    request(E0 + 32, 1);
-    request(E1, 2);
+  for (int i = 0; i < 4; ++i) {
+    rfp[i] = smem + r * ROWB + (r >> 2) * 16 + ((4 * i + g) ^ (4 * (r & 3))) * 16;
+    tfp[i] = smem + tr_row * ROWB + (tr_row >> 2) * 16 +
+             ((4 * i + 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1)) ^ (4 * (tr_row & 3))) * 16 + (lane & 1) * 8;
   }
-  // (the wait for the K^T and V^T fragments comes here, behind the first requests, which only needed the list)
-#pragma unroll
-  for (int c = 0; c < DC; ++c) asm volatile("" : "+a"(kf[c]), "+a"(vf[c]));
-  if (nunits > 0) {
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NREQ) : "memory");
-    __syncthreads();
-#pragma unroll
-    for (int c = 0; c < DC; ++c) {
-      const i16x8_t a = *reinterpret_cast<const i16x8_t*>(smem + rfo[c]);
-      const i16x8_t b = *reinterpret_cast<const i16x8_t*>(smem + TILE + rfo[c]);
-      if (c == 0) {
-        mfma_scores_first<Tag>(s_a, a, kf[c]);
-        mfma_scores_first<Tag>(dp_a, b, vf[c]);
-      } else {
-        mfma_scores<Tag>(s_a, a, kf[c]);
-        mfma_scores<Tag>(dp_a, b, vf[c]);
-      }
-    }
-    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");         // (the vector ALU reads these results next)
-  }
-
-  // What one iteration fetches from LDS for the next one (the data landed long before): the log-sum-exps and deltas of
-  // its 32 query rows (accumulator register 4 i4 + j of S / dP is query row 8 i4 + 4 g + j of the unit; this lane's
-  // column is its key) and the transposed fragments of its first two groups of second products.
-  f32x4_t l4[4], d4[4];
-  i16x8_t trd[4], trq[4];            // transposed dO / Q fragments of group grp in slot grp % 4, fetched two groups ahead
-  auto row_scalars = [&](const uint8_t* gen, int i4) __attribute__((always_inline)) {
-    l4[i4] = *reinterpret_cast<const f32x4_t*>(gen + 2 * TILE + (8 * i4 + 4 * g) * 4);
-    d4[i4] = *reinterpret_cast<const f32x4_t*>(gen + 2 * TILE + 128 + (8 * i4 + 4 * g) * 4);
+  i16x8_t af[3], bf[3];              // row-wise Q and dO fragments, two chunks ahead
+  i16x8_t trd[5], trq[5];            // transposed dO / Q fragments of group grp in slot grp % 5, four groups ahead
+  f32x4_t l4[4];                     // log-sum-exps of the unit whose elements come next: accumulator register
+                                     // 4 i4 + j of S / dP is query row 8 i4 + 4 g + j of the unit, this lane's column its key
+  auto row_frags = [&](int at, int c) __attribute__((always_inline)) {
+    af[c % 3] = *reinterpret_cast<const i16x8_t*>(rfp[c >> 1] + at + (c & 1) * 32);
+    bf[c % 3] = *reinterpret_cast<const i16x8_t*>(rfp[c >> 1] + at + TILE + (c & 1) * 32);
   };
-  auto tr_frags = [&](const uint8_t* gen, int grp) __attribute__((always_inline)) {
+  auto tr_frags = [&](int at, int grp) __attribute__((always_inline)) {
+    const uint8_t* t0 = tfp[grp & 3] + at + 4 * (grp >> 2) * REQ_PITCH;
+    trd[grp % 5] = concat4(lds_read_tr16(reinterpret_cast<const uint16_t*>(t0 + TILE)),
+                           lds_read_tr16(reinterpret_cast<const uint16_t*>(t0 + TILE + 2 * REQ_PITCH)));
+    trq[grp % 5] = concat4(lds_read_tr16(reinterpret_cast<const uint16_t*>(t0)),
+                           lds_read_tr16(reinterpret_cast<const uint16_t*>(t0 + 2 * REQ_PITCH)));
+  };
+  auto read_lse = [&](int at, int i4) __attribute__((always_inline)) {
+    l4[i4] = *reinterpret_cast<const f32x4_t*>(ldp + at + i4 * 32);
+  };
+  auto read_delta = [&](int at, f32x16_t& dp, int i4) __attribute__((always_inline)) {      // what the chain of -dP starts from
+    const f32x4_t d4 = *reinterpret_cast<const f32x4_t*>(ldp + at + 256 + i4 * 32);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) dp[4 * i4 + j] = d4[j];
+  };
+  // product 2 c + {0, 1} of the first sixteen: S, -dP + delta, chunk c of the head dimension
+  auto score_product = [&](f32x16_t& s, f32x16_t& dp, int c, int which) __attribute__((always_inline)) {
+    if (which) mfma_scores<Tag>(dp, bf[c % 3], vf[c]);
+    else if (c == 0) mfma_scores_first<Tag>(s, af[0], kf[0]);
+    else mfma_scores<Tag>(s, af[c % 3], kf[c]);
+  };
+  i32x4_t pw[2], dw[2];
+  // element i of a unit: P = exp2(S c - lse), then -dS = P (delta - dP); packed in pairs
+  auto prob = [&](f32x16_t& s, int i) __attribute__((always_inline)) {
+    float p = fast_exp2(__builtin_fmaf(s[i], c_log2e, -l4[i >> 2][i & 3]));
+    asm volatile("" : "+v"(p));
+    s[i] = p;
+  };
+  auto grad = [&](f32x16_t& s, f32x16_t& dp, int i) __attribute__((always_inline)) {
+    float ds = s[i] * dp[i];
+    asm volatile("" : "+v"(ds));
+    dp[i] = ds;
+    if (i & 1) {
+      uint32_t a = E::pack2(s[i - 1], s[i]), b = E::pack2(dp[i - 1], dp[i]);
+      asm volatile("" : "+v"(a), "+v"(b));
+      pw[i >> 3][(i >> 1) & 3] = (int)a;
+      dw[i >> 3][(i >> 1) & 3] = (int)b;
+    }
+  };
+  auto second_products = [&](int grp) __attribute__((always_inline)) {
     const int c2 = grp >> 2, dt = grp & 3;
-    const uint8_t* t0 = gen + 16 * c2 * ROWB;
-    trd[grp & 3] = concat4(lds_read_tr16(reinterpret_cast<const uint16_t*>(t0 + TILE + tfo[0][dt])),
-                           lds_read_tr16(reinterpret_cast<const uint16_t*>(t0 + TILE + tfo[1][dt])));
-    trq[grp & 3] = concat4(lds_read_tr16(reinterpret_cast<const uint16_t*>(t0 + tfo[0][dt])),
-                           lds_read_tr16(reinterpret_cast<const uint16_t*>(t0 + tfo[1][dt])));
+    dvacc[dt] = E::mfma32(trd[grp % 5], __builtin_bit_cast(i16x8_t, pw[c2]), dvacc[dt]);
+    dkacc[dt] = E::mfma32(trq[grp % 5], __builtin_bit_cast(i16x8_t, dw[c2]), dkacc[dt]);
   };
-  if (nunits > 0) {
+  auto mask_rows = [&](int row0) __attribute__((always_inline)) {      // rows past L: +inf makes every probability exactly 0
 #pragma unroll
-    for (int i4 = 0; i4 < 4; ++i4) row_scalars(smem, i4);
-    tr_frags(smem, 0);
-    tr_frags(smem, 1);
-  }
+    for (int i4 = 0; i4 < 4; ++i4)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (row0 + 8 * i4 + 4 * g + j >= L) l4[i4][j] = INFINITY;
+  };
 
-  // One iteration = unit u, 32 MFMAs:
-  //   slots  0..15  S and dP of unit u + 1 (two chains)      beside: P and dS of unit u
-  //   slots 16..31  dV^T += dO^T P, dK^T += Q^T dS of unit u  beside: the requests for unit u + 3, and what the next
-  //                                                            iteration wants from LDS first (see above)
-  // On entry: s_cur, dp_cur = Q K^T and dO V^T of unit u.  Before anything else: this wave's part of unit u + 1 has
-  // landed (all but the latest nine requests), one barrier (the partner's part too; everyone is done with unit u - 1,
-  // whose generation the requests for u + 3 overwrite).  A single wave per SIMD has nobody to hide its LDS latency:
-  // every fragment is fetched three products (row-wise) or two groups (transposed) before it is used, and the first
-  // four elements of the vector arithmetic run while the first row-wise fragments are on their way.
-  // GU = u % 4: the generation of unit u.  (Unrolling four iterations to make it a constant costs more registers
-  // than the kernel has: the compiler then spills the resident fragments.)
-  auto iteration = [&](int GU, f32x16_t& s_cur, f32x16_t& dp_cur, f32x16_t& s_nxt, f32x16_t& dp_nxt, int row0_u,
-                       int row0_req) __attribute__((always_inline)) {
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NREQ) : "memory");
-    __syncthreads();
-    const uint8_t* gu = smem + GU * GEN;                       // unit u: transposed reads
-    const uint8_t* gn = smem + ((GU + 1) & 3) * GEN;           // unit u + 1: row-wise reads, scalars, first transposed reads
-    i16x8_t af[4], bf[4];
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-      af[c] = *reinterpret_cast<const i16x8_t*>(gn + rfo[c]);
-      bf[c] = *reinterpret_cast<const i16x8_t*>(gn + TILE + rfo[c]);
-    }
-    if (__builtin_expect(row0_u + 32 > L, 0)) {                // rows past L: +inf makes every probability exactly 0
-#pragma unroll
-      for (int i4 = 0; i4 < 4; ++i4)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          if (row0_u + 8 * i4 + 4 * g + j >= L) {
-            l4[i4][j] = INFINITY;
-            d4[i4][j] = 0.f;
-          }
-    }
-    i32x4_t pw[2], dw[2];
-    // element i of unit u: P = exp2(S c - lse), dS = P (dP - delta); packed in pairs
-    auto element = [&](int i) __attribute__((always_inline)) {
-      float p = fast_exp2(__builtin_fmaf(s_cur[i], c_log2e, -l4[i >> 2][i & 3]));
-      float ds = p * (dp_cur[i] - d4[i >> 2][i & 3]);
-      asm volatile("" : "+v"(p), "+v"(ds));
-      s_cur[i] = p;
-      dp_cur[i] = ds;
-      if (i & 1) {
-        uint32_t a = E::pack2(s_cur[i - 1], s_cur[i]), b = E::pack2(dp_cur[i - 1], dp_cur[i]);
-        asm volatile("" : "+v"(a), "+v"(b));
-        pw[i >> 3][(i >> 1) & 3] = (int)a;
-        dw[i >> 3][(i >> 1) & 3] = (int)b;
-      }
-    };
-#pragma unroll
-    for (int i = 0; i < 4; ++i) element(i);
+  // One iteration = unit u in generation GU = u % 4, 32 products:
+  //   slots  0..15  S and dP of unit u + 1 (two chains)        beside: P and dS of unit u, the transposed fragments of its first
+  //                                                             four groups, the requests for dO and scalars of unit u + 3
+  //   slots 16..31  dV^T += dO^T P, dK^T += Q^T dS of unit u   beside: the other transposed fragments; then, from the barrier on,
+  //                                                             the requests for Q of unit u + 4 (into unit u's generation) and
+  //                                                             what the next iteration wants first from LDS
+  // The barrier stands where this wave has read all of unit u's generation and its part of unit u + 2 has landed (only
+  // the nine requests for unit u + 3 may be out): behind it everyone's has, and the generation may be overwritten.
+  // (A key row past L only ever feeds its own, never stored, column of dK^T / dV^T: no masking needed.)
+  f32x16_t s_a, dp_a, s_b, dp_b;
+  auto iteration = [&](auto gu, f32x16_t& s_cur, f32x16_t& dp_cur, f32x16_t& s_nxt, f32x16_t& dp_nxt, int row0_u, int row0_u3,
+                       int row0_u4) __attribute__((always_inline)) {
+    constexpr int GU = decltype(gu)::value, AT0 = GU * GEN, AT1 = ((GU + 1) & 3) * GEN, AT2 = ((GU + 2) & 3) * GEN;
+    if (__builtin_expect(row0_u + 32 > L, 0)) mask_rows(row0_u);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int c = 0; c < DC; ++c) {
-      if (c + 3 < DC) {
-        af[(c + 3) & 3] = *reinterpret_cast<const i16x8_t*>(gn + rfo[c + 3]);
-        bf[(c + 3) & 3] = *reinterpret_cast<const i16x8_t*>(gn + TILE + rfo[c + 3]);
-      }
 #pragma unroll
-      for (int half = 0; half < 2; ++half) {
-        if (half == 0) {
-          if (c == 0) mfma_scores_first<Tag>(s_nxt, af[c & 3], kf[c]);
-          else mfma_scores<Tag>(s_nxt, af[c & 3], kf[c]);
-        } else {
-          if (c == 0) mfma_scores_first<Tag>(dp_nxt, bf[c & 3], vf[c]);
-          else mfma_scores<Tag>(dp_nxt, bf[c & 3], vf[c]);
-        }
-        const int sl = 2 * c + half;                           // twelve elements left for sixteen slots
-        if (sl < 12) element(4 + sl);
+      for (int which = 0; which < 2; ++which) {
+        const int sl = 2 * c + which;
+        score_product(s_nxt, dp_nxt, c, which);
+        prob(s_cur, sl);
+        if (sl > 0) grad(s_cur, dp_cur, sl - 1);
+        if (which == 0 && c + 2 < DC) row_frags(AT1, c + 2);
+        if (sl == 1) SLA_DKDV_REQUEST_DO(0, row0_u3, (GU + 3) & 3);
+        if (sl == 2) SLA_DKDV_REQUEST_DO(1, row0_u3, (GU + 3) & 3);
+        if (sl == 3) SLA_DKDV_REQUEST_DO(2, row0_u3, (GU + 3) & 3);
+        if (sl == 4) SLA_DKDV_REQUEST_DO(3, row0_u3, (GU + 3) & 3);
+        if (sl == 5) SLA_DKDV_REQUEST_LD(row0_u3, (GU + 3) & 3);
+        if (sl == 9) tr_frags(AT0, 0);
+        if (sl == 11) tr_frags(AT0, 1);
+        if (sl == 13) tr_frags(AT0, 2);
+        if (sl == 15) tr_frags(AT0, 3);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
-    // (a key row past L only ever feeds its own, never stored, column of dK^T / dV^T: no masking needed)
-    const uint32_t req_base = (uint32_t)((GU + 3) & 3) * GEN;
-    const uint32_t rq = (uint32_t)row0_req * pitch * 2, rdo = (uint32_t)row0_req * pitch_do * 2;
-    // eight groups (c2, dt) of two products
+    grad(s_cur, dp_cur, 15);
 #pragma unroll
     for (int grp = 0; grp < 8; ++grp) {
-      const int c2 = grp >> 2, dt = grp & 3;
-      if (grp + 2 < 8) tr_frags(gu, grp + 2);
-      else tr_frags(gn, grp + 2 - 8);                          // the next unit's first two groups
-      if (grp >= 4) row_scalars(gn, grp - 4);                  // and its scalars
-      dvacc[dt] = E::mfma32(trd[grp & 3], __builtin_bit_cast(i16x8_t, pw[c2]), dvacc[dt]);
-      dkacc[dt] = E::mfma32(trq[grp & 3], __builtin_bit_cast(i16x8_t, dw[c2]), dkacc[dt]);
-      if (grp < 4) {
-        lds_dma_b128(qh, qoff[grp] + rq, rows_base, req_base + grp * 1024);
-        lds_dma_b128(doh, dooff[grp] + rdo, rows_base, req_base + TILE + grp * 1024);
-      } else if (grp == 4) {
-        if (lane < 32) lds_dma_b32(ldh, (uint32_t)(row0_req + lane) * 4, ld_base, req_base + 2 * TILE);
+      if (grp < 4) tr_frags(AT0, grp + 4);
+      if (grp == 5) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(NREQ) : "memory");
+      second_products(grp);
+      if (grp >= 5) {
+        if (grp == 5) SLA_DKDV_REQUEST_Q(0, row0_u4, GU);
+        if (grp == 5) row_frags(AT2, 0);
+        if (grp == 6) SLA_DKDV_REQUEST_Q(1, row0_u4, GU);
+        if (grp == 6) read_delta(AT2, dp_cur, 0);
+        if (grp == 6) read_delta(AT2, dp_cur, 1);
+        if (grp == 6) read_delta(AT2, dp_cur, 2);
+        if (grp == 6) read_delta(AT2, dp_cur, 3);
+        if (grp == 7) SLA_DKDV_REQUEST_Q(2, row0_u4, GU);
+        if (grp == 7) SLA_DKDV_REQUEST_Q(3, row0_u4, GU);
+        if (grp == 7) row_frags(AT2, 1);
       }
+      if (grp >= 3 && grp < 7) read_lse(AT1, grp - 3);
       __builtin_amdgcn_sched_barrier(0);
     }
   };
 
-  for (int u = 0; u < nunits; u += 2) {
-    const int E3 = entry_row0((u >> 1) + 3);                        // (looked up now, used two units from now)
-    iteration(u & 3, s_a, dp_a, s_b, dp_b, E0, E1 + 32);            // unit u; requests unit u + 3
-    iteration((u + 1) & 3, s_b, dp_b, s_a, dp_a, E0 + 32, E2);      // unit u + 1; requests u + 4
-    E0 = E1;
-    E1 = E2;
-    E2 = E3;
+  __syncthreads();                                             // the zeros and the entries are in place before anything is requested
+  // first query rows of the listed blocks: E0 = of the entry of units u and u + 1, E1 = of the next one, E2 = of the one after
+  int E0 = 0, E1 = 0, E2 = 0;
+  if (nent > 0) {
+    E0 = entry_row0(0);
+    E1 = entry_row0(1);
+    E2 = entry_row0(2);
+#define SLA_DKDV_REQUEST_UNIT(ROW0, G)                                                                                          \
+  SLA_DKDV_REQUEST_Q(0, ROW0, G); SLA_DKDV_REQUEST_Q(1, ROW0, G); SLA_DKDV_REQUEST_Q(2, ROW0, G); SLA_DKDV_REQUEST_Q(3, ROW0, G);     \
+  SLA_DKDV_REQUEST_DO(0, ROW0, G); SLA_DKDV_REQUEST_DO(1, ROW0, G); SLA_DKDV_REQUEST_DO(2, ROW0, G); SLA_DKDV_REQUEST_DO(3, ROW0, G); \
+  SLA_DKDV_REQUEST_LD(ROW0, G)
+    SLA_DKDV_REQUEST_UNIT(E0, 0);
+    SLA_DKDV_REQUEST_UNIT(E0 + 32, 1);
+    SLA_DKDV_REQUEST_UNIT(E1, 2);
+#undef SLA_DKDV_REQUEST_UNIT
   }
+  // (the wait for the K^T and V^T fragments comes here, behind the first requests, which only needed the list)
+#pragma unroll
+  for (int c = 0; c < DC; ++c) {
+    vf[c] ^= (short)0x8000;                                    // -V
+    asm volatile("" : "+a"(kf[c]), "+a"(vf[c]));
+  }
+  if (nent > 0) {
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * NREQ) : "memory");
+    row_frags(0, 0);
+    row_frags(0, 1);
+#pragma unroll
+    for (int i4 = 0; i4 < 4; ++i4) {
+      read_delta(0, dp_a, i4);
+      read_lse(0, i4);
+    }
+#pragma unroll
+    for (int c = 0; c < DC; ++c) {
+      score_product(s_a, dp_a, c, 0);
+      score_product(s_a, dp_a, c, 1);
+      if (c + 2 < DC) row_frags(0, c + 2);
+    }
+    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");         // (the vector ALU reads these results next)
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(NREQ) : "memory");
+    SLA_DKDV_REQUEST_Q(0, E1 + 32, 3); SLA_DKDV_REQUEST_Q(1, E1 + 32, 3);
+    SLA_DKDV_REQUEST_Q(2, E1 + 32, 3); SLA_DKDV_REQUEST_Q(3, E1 + 32, 3);
+    row_frags(GEN, 0);
+    row_frags(GEN, 1);
+#pragma unroll
+    for (int i4 = 0; i4 < 4; ++i4) read_delta(GEN, dp_b, i4);
+    int last_at;                                               // where the last unit lies (an odd one: generation 1 or 3)
+    for (int b = 0;; b += 2) {
+      int E3 = entry_row0(b + 3);                              // (looked up now, used two units from now)
+      iteration(std::integral_constant<int, 0>{}, s_a, dp_a, s_b, dp_b, E0, E1 + 32, E2);
+      last_at = GEN;
+      if (b + 1 >= nent) break;
+      iteration(std::integral_constant<int, 1>{}, s_b, dp_b, s_a, dp_a, E0 + 32, E2, E2 + 32);
+      E0 = E1;
+      E1 = E2;
+      E2 = E3;
+      E3 = entry_row0(b + 4);
+      iteration(std::integral_constant<int, 2>{}, s_a, dp_a, s_b, dp_b, E0, E1 + 32, E2);
+      last_at = 3 * GEN;
+      if (b + 2 >= nent) break;
+      iteration(std::integral_constant<int, 3>{}, s_b, dp_b, s_a, dp_a, E0 + 32, E2, E2 + 32);
+      E0 = E1;
+      E1 = E2;
+      E2 = E3;
+    }
+    // the last unit: no scores left to form beside its arithmetic
+    if (__builtin_expect(E0 + 64 > L, 0)) mask_rows(E0 + 32);
+#pragma unroll
+    for (int grp = 0; grp < 4; ++grp) tr_frags(last_at, grp);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      prob(s_b, i);
+      grad(s_b, dp_b, i);
+    }
+#pragma unroll
+    for (int grp = 0; grp < 8; ++grp) {
+      if (grp < 4) tr_frags(last_at, grp + 4);
+      second_products(grp);
+    }
+  }
+#undef SLA_DKDV_REQUEST_Q
+#undef SLA_DKDV_REQUEST_DO
+#undef SLA_DKDV_REQUEST_LD
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");    // (nothing of this workgroup is in flight when it ends)
 
+  const auto turned = [&](float x) __attribute__((always_inline)) { return __builtin_fmaf(x, -qk_scale, 0.f); };   // (+0 for an empty sum)
   if (slot >= 0) {
     // one segment of a long list: fp32 partial [dk | dv][64][D], added up by bwd_dkdv_reduce_kernel
     float* pk = part + (size_t)slot * (2 * 64 * D) + (size_t)(w * 32 + r) * D;
@@ -338,8 +390,8 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 #pragma unroll
       for (int i4 = 0; i4 < 4; ++i4) {
         const int d0 = 32 * dt + 8 * i4 + 4 * g;
-        *reinterpret_cast<f32x4_t*>(pk + d0) = f32x4_t{dkacc[dt][4 * i4 + 0] * qk_scale, dkacc[dt][4 * i4 + 1] * qk_scale,
-                                                       dkacc[dt][4 * i4 + 2] * qk_scale, dkacc[dt][4 * i4 + 3] * qk_scale};
+        *reinterpret_cast<f32x4_t*>(pk + d0) = f32x4_t{turned(dkacc[dt][4 * i4 + 0]), turned(dkacc[dt][4 * i4 + 1]),
+                                                       turned(dkacc[dt][4 * i4 + 2]), turned(dkacc[dt][4 * i4 + 3])};
         *reinterpret_cast<f32x4_t*>(pv + d0) =
             f32x4_t{dvacc[dt][4 * i4 + 0], dvacc[dt][4 * i4 + 1], dvacc[dt][4 * i4 + 2], dvacc[dt][4 * i4 + 3]};
       }
@@ -360,8 +412,8 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
       for (int i4 = 0; i4 < 4; ++i4) {
         i32x2_t wv;
         if (which == 0) {
-          wv[0] = (int)E::pack2(dkacc[dt][4 * i4 + 0] * qk_scale, dkacc[dt][4 * i4 + 1] * qk_scale);
-          wv[1] = (int)E::pack2(dkacc[dt][4 * i4 + 2] * qk_scale, dkacc[dt][4 * i4 + 3] * qk_scale);
+          wv[0] = (int)E::pack2(turned(dkacc[dt][4 * i4 + 0]), turned(dkacc[dt][4 * i4 + 1]));
+          wv[1] = (int)E::pack2(turned(dkacc[dt][4 * i4 + 2]), turned(dkacc[dt][4 * i4 + 3]));
         } else {
           wv[0] = (int)E::pack2(dvacc[dt][4 * i4 + 0], dvacc[dt][4 * i4 + 1]);
           wv[1] = (int)E::pack2(dvacc[dt][4 * i4 + 2], dvacc[dt][4 * i4 + 3]);
@@ -397,19 +449,6 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 // B1 H12 L32760 with 25 key blocks per row 551 -> 485 us (matrix pipe busy 53 -> 61 % of the cycles, at a clock that the
 // power limit holds at 1.65 GHz), B2 H16 L32760 with 128-row blocks 1428 -> 1224 us, B2 H4 L4096 37.9 -> 33.2 us.
 constexpr int DQ_STREAM_MAX_T = 2048;          // look-up rows longer than this take bwd_dq_kernel
-
-// Four requests of 16 bytes per lane, memory -> LDS, REQ_PITCH bytes apart in LDS.  The instruction offset counts for both
-// addresses: off[j] is the memory offset less j * REQ_PITCH (never negative: REQ_SLACK bytes are part of it and of a
-// descriptor that starts as many bytes early).
-constexpr int REQ_PITCH = 1040;                // 4 rows of 256 bytes + 16 bytes of padding
-constexpr int REQ_SLACK = 64;
-template <int J>
-static __device__ __forceinline__ void lds_dma_row4(__amdgpu_buffer_rsrc_t rsrc, uint32_t off, uint32_t lds) {
-  if constexpr (J == 0)
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds), "v"(off), "s"(rsrc) : "memory");
-  else
-    asm volatile("buffer_load_dwordx4 %0, %1, 0 offen offset:%2 lds" ::"v"(off), "s"(rsrc), "n"(J * REQ_PITCH) : "memory");
-}
 
 template <typename Tag>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void bwd_dq_stream_kernel(
