@@ -731,26 +731,27 @@ static int bwd_impl(const void* q, const void* k, const void* v, const void* o, 
                        w.seg, (int)w.max_items, (int)w.max_slots);
   const int total_q = BH * Mblk;
   const bool contig = lin.sl == D && ldo.sl == D;
-  // head dim 128 with 64-row query blocks has kernels of its own (32-bit byte offsets inside a head); a 128-row query
+  // The kernels of sparse_bwd_stream.h walk 64-row query blocks with 32-bit byte offsets inside a head; a 128-row query
   // block goes through them as its two halves (`wide`), which follow the block's row of the table and its list entries
   const int wide = BLKQ == 128;
   const int Mblk64 = cdiv(L, 64);
   const int total_q64 = BH * Mblk64;
-  const bool stream_dkdv = D == 128 && (BLKQ == 64 || BLKQ == 128) && (uint64_t)lin.sl * 2u * (uint64_t)L < (1ull << 31) &&
+  const bool stream_dkdv = (BLKQ == 64 || BLKQ == 128) && (uint64_t)lin.sl * 2u * (uint64_t)L < (1ull << 31) &&
                            (uint64_t)ldo.sl * 2u * (uint64_t)L < (1ull << 31);
   // (The stream kernel keeps a look-up row as 16-bit key block indices.  One wave of it walks a block that the general
   // kernel gives two waves, and it forms delta itself: with 64-row blocks it is ahead from a wave for every third SIMD on
   // (whole backward, 324 blocks 62.6 / 65.8 us, 512 blocks 87.2 / 91.8; 260 blocks 54.6 / 53.4); with 128-row blocks, to which
-  // the general kernel gives four waves sharing their tiles, only when every SIMD has one (390 blocks 94.6 / 93.0).)
+  // the general kernel gives four waves sharing their tiles, only when every SIMD has one (390 blocks 94.6 / 93.0).  Head
+  // dim 64 follows the same lines: 512 blocks 52.0 / 59.5, 1024 halves of 128-row blocks 60.1 / 74.2.)
   const bool stream_dq = stream_dkdv && topk <= DQ_STREAM_MAX_T && total_q64 >= (wide ? 1024 : 320) && Mblk64 <= 65535;
-  // delta = rowsum(dO * O): the dQ kernel of the common shape forms it for its own rows, the general one reads it
+  // delta = rowsum(dO * O): the stream dQ kernel forms it for its own rows, the general one reads it
   if ((steps & SB_DQ) && !stream_dq)
     hipLaunchKernelGGL((bwd_delta_kernel<Tag, D>), dim3((unsigned)((rows + RPB - 1) / RPB)), dim3(256), 0, st,
                        (const uint16_t*)o, (const uint16_t*)d_o, ldo, delta, rows, L);
 #define SLA_BWD_LAUNCH(CONTIG)                                                                                              \
   if (!(steps & SB_DQ)) {                                                                                                   \
   } else if (stream_dq)                                                                                                     \
-    hipLaunchKernelGGL((bwd_dq_stream_kernel<Tag>), dim3(xcd_grid(total_q64)), dim3(64), 0, st, (const uint16_t*)q,         \
+    hipLaunchKernelGGL((bwd_dq_stream_kernel<Tag, D>), dim3(xcd_grid(total_q64)), dim3(64), 0, st, (const uint16_t*)q,         \
                        (const uint16_t*)k, (const uint16_t*)v, (const uint16_t*)d_o, (const uint16_t*)o, lse, delta, lut,   \
                        lut64, (uint16_t*)dq, lin, ldo, L, Mblk64, topk, qk_scale, total_q64, wide);                        \
   else                                                                                                                      \
@@ -759,7 +760,7 @@ static int bwd_impl(const void* q, const void* k, const void* v, const void* o, 
                        lut64, (uint16_t*)dq, lin, ldo, L, Mblk, topk, qk_scale, total_q);                                  \
   if (!(steps & SB_DKDV)) {                                                                                                 \
   } else if (stream_dkdv)                                                                                                   \
-    hipLaunchKernelGGL((bwd_dkdv_stream_kernel<Tag>), dim3(xcd_grid(w.max_items)), dim3(128), 0, st, (const uint16_t*)q,    \
+    hipLaunchKernelGGL((bwd_dkdv_stream_kernel<Tag, D>), dim3(xcd_grid(w.max_items)), dim3(128), 0, st, (const uint16_t*)q,    \
                        (const uint16_t*)k, (const uint16_t*)v, (const uint16_t*)d_o, lse, delta, list, count, items,       \
                        totals, part, w.seg, (uint16_t*)dk, (uint16_t*)dv, lin, ldo, L, Mblk, Nblk, qk_scale, wide);       \
   else                                                                                                                      \

@@ -1,10 +1,11 @@
-// dK / dV of the block-sparse attention backward for 64-row query blocks at head dim 128: one workgroup of two
-// waves per key block (or per segment of a key block's list), one wave per SIMD.
+// dK / dV of the block-sparse attention backward for 64-row query blocks: one workgroup of two waves per key block (or
+// per segment of a key block's list), one wave per SIMD at head dim 128, two at head dim 64 (where everything a wave
+// keeps is half as large).
 //
 // Stands in for _attn_bwd_dkdv of the reference (sparse_linear_attention/kernel.py:160-237) like bwd_dkdv_kernel,
 // whose work items, lists and arithmetic it shares.  What differs:
 //   * a wave owns 32 keys and the whole head dimension: K^T and V^T fragments (B operands of S = Q K^T and
-//     dP = dO V^T) and the dK^T / dV^T accumulators (128 d x 32 keys each) stay in its registers, P and dS leave
+//     dP = dO V^T) and the dK^T / dV^T accumulators (D x 32 keys each) stay in its registers, P and dS leave
 //     the accumulators in the B-operand layout of dV^T += dO^T P and dK^T += Q^T dS.  Nothing is handed from wave
 //     to wave, and there is one barrier per 32 query rows;
 //   * Q and dO rows go from memory straight into LDS (buffer loads with the LDS bit), 32 rows at a time, into a
@@ -20,7 +21,8 @@
 //     where the fragments of a unit have all been read, so that the first reads of the next unit and the requests for
 //     the unit after next run beside products.  Measured, before and after: B1 H12 L32760 with 25 key blocks per row
 //     840 -> 758 us (matrix pipe busy 45 -> 51 % of the cycles at 1.74 GHz, where the power limit holds it), B2 H16
-//     L32760 with 128-row query blocks 2272 -> 2065 us, B2 H4 L4096 48.5 -> 43.0 us.
+//     L32760 with 128-row query blocks 2272 -> 2065 us, B2 H4 L4096 48.5 -> 43.0 us.  Head dim 64 against
+//     bwd_dkdv_kernel: B2 H8 L6001 with 9 key blocks per row 57.6 -> 44.2 us.
 #pragma once
 #include <type_traits>
 
@@ -28,20 +30,37 @@
 
 namespace sla {
 
+template <int N>
+using I = std::integral_constant<int, N>;
+
 // One of four requests of 16 bytes per lane, memory -> LDS (lane l's piece lands 16 l bytes on), REQ_PITCH bytes apart in
 // LDS.  The instruction offset counts for both addresses: off is the memory offset less J * REQ_PITCH (never negative:
-// REQ_SLACK bytes are part of it and of a descriptor that starts as many bytes early).  J = 0 sets M0 for all four.
+// REQ_SLACK bytes are part of it and of a descriptor that starts as many bytes early).  The first of a group sets M0.
 // (Between a scalar write of M0 and a memory -> LDS load that reads it the hardware wants one wait state; the compiler
 // adds it to its own code and does not look into these instructions.)
-constexpr int REQ_PITCH = 1040;                // 4 rows of 256 bytes + 16 bytes of padding
+constexpr int REQ_PITCH = 1040;                // 4 rows of 256 bytes (8 of 128) + 16 bytes of padding
 constexpr int REQ_SLACK = 64;
-template <int J>
+template <int J, bool SET = J == 0>
 static __device__ __forceinline__ void lds_dma_row4(__amdgpu_buffer_rsrc_t rsrc, uint32_t off, uint32_t lds) {
-  if constexpr (J == 0)
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds), "v"(off), "s"(rsrc) : "memory");
+  if constexpr (SET)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen offset:%3 lds" ::"s"(lds), "v"(off), "s"(rsrc),
+                 "n"(J * REQ_PITCH)
+                 : "memory");
   else
     asm volatile("buffer_load_dwordx4 %0, %1, 0 offen offset:%2 lds" ::"v"(off), "s"(rsrc), "n"(J * REQ_PITCH) : "memory");
 }
+// Where the 16-byte pieces of 32 rows lie: request j holds rows RPR j .., piece p of a row in slot p ^ swz(row).  For one piece
+// the 16 rows of a row-wise read hit 16 different slots of the 256 bytes LDS serves at a time, and so do the 4 rows x 4 pieces
+// of a transposing read.  (256-byte rows: row % 4 picks the group of four slots, the padding of a request the slot in it.
+// 128-byte rows: row % 2 and row / 2 % 2 pick the group, row / 4 % 2 a pair in it and the padding the slot of the pair.)
+template <int D>
+struct BwdTile {
+  static constexpr int ROWB = D * 2, RPR = 1024 / ROWB, NREQ = 32 / RPR, BYTES = NREQ * REQ_PITCH;
+  static __device__ __forceinline__ int swz(int row) { return D == 128 ? 4 * (row & 3) : 4 * ((row >> 1) & 1) + 2 * ((row >> 2) & 1); }
+  static __device__ __forceinline__ int piece_at(int row, int piece) {        // byte offset inside the tile
+    return row * ROWB + row / RPR * 16 + (piece ^ swz(row)) * 16;
+  }
+};
 // 4 bytes per lane: lane l's word lands at lds_base + lds_off + 4 l
 static __device__ __forceinline__ void lds_dma_b32(__amdgpu_buffer_rsrc_t rsrc, uint32_t byte_off, uint32_t lds_base,
                                                    uint32_t lds_off) {
@@ -52,8 +71,8 @@ static __device__ __forceinline__ void lds_dma_b32(__amdgpu_buffer_rsrc_t rsrc, 
 
 constexpr int DKDV_STREAM_MAX_SEG = 1024;      // list entries one work item may have (they are copied into LDS)
 
-template <typename Tag>
-__global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(1, 1))) void bwd_dkdv_stream_kernel(
+template <typename Tag, int D>
+__global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 ? 2 : 1))) void bwd_dkdv_stream_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
     const uint16_t* __restrict__ d_o, const float* __restrict__ lse, const float* __restrict__ delta,
     const int* __restrict__ list, const int* __restrict__ count, const i32x4_t* __restrict__ items,
@@ -61,12 +80,15 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     const RowLayout lin, const RowLayout ldo, int L, int Mblk, int Nblk, float qk_scale, int wide) {
   // (wide = 1: the lists name 128-row query blocks; an entry is then walked as its two 64-row halves)
   using E = Elem<Tag>;
-  constexpr int D = 128, DC = D / 16, DT = D / 32;
-  constexpr int ROWB = D * 2;               // bytes per row in LDS
-  constexpr int TILE = 8 * REQ_PITCH;       // 32 rows of Q or of dO
+  using T32 = BwdTile<D>;
+  constexpr int DC = D / 16, DT = D / 32;
+  constexpr int TILE = T32::BYTES;          // 32 rows of Q or of dO
   constexpr int GEN = 2 * TILE + 512;       // one generation: Q rows, dO rows, log-sum-exps, deltas (32 of 64 words used)
   constexpr int NG = 4;
-  constexpr int NREQ = 9;                   // requests per wave and unit: 4 x Q, 4 x dO (its 16 rows), 1 x lse or delta
+  constexpr int NR = T32::NREQ / 2;         // requests per wave (16 rows) and tile
+  constexpr int NREQ = 2 * NR + 1;          // requests per wave and unit: Q, dO, 1 x lse or delta
+  constexpr int NGRP = 2 * DT;              // groups (16 query rows x 32 d) of two second products
+  constexpr int ROWS8 = 8 / T32::RPR * REQ_PITCH;              // 8 rows further on in a tile
   __shared__ __attribute__((aligned(16))) uint8_t smem[NG * GEN];
   // This work item's list entries.  (Read from memory inside the loop they would be vector loads - the inline assembly
   // keeps the compiler from using the scalar path - and waiting for a vector load means waiting for every memory ->
@@ -140,22 +162,20 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   for (int i = 128 + tid; i < nent; i += 128) entries[i] = (mylist[e0 + (i >> wide)] << wide) + (i & wide);
 
   // ---- addressing ----
-  // A request moves 4 rows (64 lanes x 16 bytes): lane -> row 4j + lane / 16 of this wave's 16 rows, 16-byte slot
-  // lane % 16, which receives piece (slot ^ 4 (row % 4)) of that row; requests are padded by one 16-byte slot.  For one
-  // piece the 16 rows of a row-wise read hit 16 different slots (row % 4 picks the group of four, row / 4 the slot in
-  // it), and so do the 4 rows x 4 pieces of a transposing read.
+  // A request moves RPR rows (64 lanes x 16 bytes): lane -> row RPR j + lane / (D / 8) of this wave's 16 rows, 16-byte slot
+  // lane % (D / 8), which receives piece (slot ^ swz(row)) of that row.
   const uint32_t smem_addr = (uint32_t)(size_t)smem;
-  const int lrow = lane >> 4, lslot = lane & 15;
-  uint32_t qoff[4], dooff[4];
+  const int lrow = lane / (D / 8), lslot = lane % (D / 8);
+  uint32_t qoff[NR], dooff[NR];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const uint32_t row = 16 * w + 4 * j + lrow;                // row of the unit
-    const uint32_t piece = (uint32_t)(lslot ^ (4 * lrow)) * 16 + REQ_SLACK - j * REQ_PITCH;
+  for (int j = 0; j < NR; ++j) {
+    const uint32_t row = 16 * w + T32::RPR * j + lrow;         // row of the unit
+    const uint32_t piece = (uint32_t)(lslot ^ T32::swz(lrow)) * 16 + REQ_SLACK - j * REQ_PITCH;
     qoff[j] = row * pitch * 2 + piece;
     dooff[j] = row * pitch_do * 2 + piece;
   }
   // LDS addresses of this wave's 16 rows inside a tile and of its words (log-sum-exps or deltas) behind the tiles
-  const uint32_t rows_base = __builtin_amdgcn_readfirstlane(smem_addr + (uint32_t)(4 * w) * REQ_PITCH);
+  const uint32_t rows_base = __builtin_amdgcn_readfirstlane(smem_addr + (uint32_t)(NR * w) * REQ_PITCH);
   const uint32_t ld_base = __builtin_amdgcn_readfirstlane(smem_addr + (uint32_t)w * 256);
   const uint32_t lane4 = (uint32_t)lane * 4;
 #define SLA_DKDV_REQUEST_Q(J, ROW0, GENERATION) \
@@ -164,33 +184,34 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   lds_dma_row4<J>(doh, dooff[J] + (uint32_t)(ROW0) * (pitch_do * 2), rows_base + (uint32_t)(GENERATION) * GEN + TILE)
 #define SLA_DKDV_REQUEST_LD(ROW0, GENERATION) \
   lds_dma_b32(ldh, lane4 + (uint32_t)(ROW0) * 4, ld_base, (uint32_t)(GENERATION) * GEN + 2 * TILE)
-  // fragments: row-wise, row r, piece 2c + g: one base per c / 2; transposed (16 query rows x 32 d), rows
-  // 16 c2 + 4 g + (lane % 16) / 4 and 8 further on, 8 bytes at element 4 (lane % 4) of the 16-column strip
-  // 2 dt + (lane / 16) % 2: one base per dt
+  // fragments: row-wise, row r, piece 2c + g: four bases; transposed (16 query rows x 32 d), rows 16 c2 + 4 g +
+  // (lane % 16) / 4 and 8 further on, 8 bytes at element 4 (lane % 4) of the 16-column strip 2 dt + (lane / 16) % 2: one
+  // base per dt
   const uint8_t* rfp[4];
   const uint8_t* tfp[DT];
   const uint8_t* const ldp = smem + 2 * TILE + 16 * g;       // log-sum-exps of rows 4g .. 4g + 3; deltas 256 bytes on
   const int tr_row = 4 * g + ((lane & 15) >> 2);
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    rfp[i] = smem + r * ROWB + (r >> 2) * 16 + ((4 * i + g) ^ (4 * (r & 3))) * 16;
-    tfp[i] = smem + tr_row * ROWB + (tr_row >> 2) * 16 +
-             ((4 * i + 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1)) ^ (4 * (tr_row & 3))) * 16 + (lane & 1) * 8;
-  }
+  for (int i = 0; i < 4; ++i) rfp[i] = smem + T32::piece_at(r, 2 * (i * DC / 4) + g);
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+    tfp[dt] = smem + T32::piece_at(tr_row, 4 * dt + 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1)) + (lane & 1) * 8;
+  constexpr int TRS = D == 128 ? 5 : 4;
   i16x8_t af[3], bf[3];              // row-wise Q and dO fragments, two chunks ahead
-  i16x8_t trd[5], trq[5];            // transposed dO / Q fragments of group grp in slot grp % 5, four groups ahead
+  i16x8_t trd[TRS], trq[TRS];        // transposed dO / Q fragments of group grp in slot grp % TRS, four groups ahead
   f32x4_t l4[4];                     // log-sum-exps of the unit whose elements come next: accumulator register
                                      // 4 i4 + j of S / dP is query row 8 i4 + 4 g + j of the unit, this lane's column its key
   auto row_frags = [&](int at, int c) __attribute__((always_inline)) {
-    af[c % 3] = *reinterpret_cast<const i16x8_t*>(rfp[c >> 1] + at + (c & 1) * 32);
-    bf[c % 3] = *reinterpret_cast<const i16x8_t*>(rfp[c >> 1] + at + TILE + (c & 1) * 32);
+    const uint8_t* p = rfp[c * 4 / DC] + at + (D == 128 ? (c & 1) * 32 : 0);
+    af[c % 3] = *reinterpret_cast<const i16x8_t*>(p);
+    bf[c % 3] = *reinterpret_cast<const i16x8_t*>(p + TILE);
   };
   auto tr_frags = [&](int at, int grp) __attribute__((always_inline)) {
-    const uint8_t* t0 = tfp[grp & 3] + at + 4 * (grp >> 2) * REQ_PITCH;
-    trd[grp % 5] = concat4(lds_read_tr16(reinterpret_cast<const uint16_t*>(t0 + TILE)),
-                           lds_read_tr16(reinterpret_cast<const uint16_t*>(t0 + TILE + 2 * REQ_PITCH)));
-    trq[grp % 5] = concat4(lds_read_tr16(reinterpret_cast<const uint16_t*>(t0)),
-                           lds_read_tr16(reinterpret_cast<const uint16_t*>(t0 + 2 * REQ_PITCH)));
+    const uint8_t* t0 = tfp[grp % DT] + at + grp / DT * 2 * ROWS8;
+    trd[grp % TRS] = concat4(lds_read_tr16(reinterpret_cast<const uint16_t*>(t0 + TILE)),
+                             lds_read_tr16(reinterpret_cast<const uint16_t*>(t0 + TILE + ROWS8)));
+    trq[grp % TRS] = concat4(lds_read_tr16(reinterpret_cast<const uint16_t*>(t0)),
+                             lds_read_tr16(reinterpret_cast<const uint16_t*>(t0 + ROWS8)));
   };
   auto read_lse = [&](int at, int i4) __attribute__((always_inline)) {
     l4[i4] = *reinterpret_cast<const f32x4_t*>(ldp + at + i4 * 32);
@@ -225,9 +246,9 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     }
   };
   auto second_products = [&](int grp) __attribute__((always_inline)) {
-    const int c2 = grp >> 2, dt = grp & 3;
-    dvacc[dt] = E::mfma32(trd[grp % 5], __builtin_bit_cast(i16x8_t, pw[c2]), dvacc[dt]);
-    dkacc[dt] = E::mfma32(trq[grp % 5], __builtin_bit_cast(i16x8_t, dw[c2]), dkacc[dt]);
+    const int c2 = grp / DT, dt = grp % DT;
+    dvacc[dt] = E::mfma32(trd[grp % TRS], __builtin_bit_cast(i16x8_t, pw[c2]), dvacc[dt]);
+    dkacc[dt] = E::mfma32(trq[grp % TRS], __builtin_bit_cast(i16x8_t, dw[c2]), dkacc[dt]);
   };
   auto mask_rows = [&](int row0) __attribute__((always_inline)) {      // rows past L: +inf makes every probability exactly 0
 #pragma unroll
@@ -237,18 +258,21 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
         if (row0 + 8 * i4 + 4 * g + j >= L) l4[i4][j] = INFINITY;
   };
 
-  // One iteration = unit u in generation GU = u % 4, 32 products:
-  //   slots  0..15  S and dP of unit u + 1 (two chains)        beside: P and dS of unit u, the transposed fragments of its first
-  //                                                             four groups, the requests for dO and scalars of unit u + 3
-  //   slots 16..31  dV^T += dO^T P, dK^T += Q^T dS of unit u   beside: the other transposed fragments; then, from the barrier on,
-  //                                                             the requests for Q of unit u + 4 (into unit u's generation) and
-  //                                                             what the next iteration wants first from LDS
+  // One iteration = unit u in generation GU = u % 4, D / 4 products:
+  //   first half   S and dP of unit u + 1 (two chains)        beside: P and dS of unit u, the transposed fragments of its first
+  //                                                            four groups, the requests for dO and scalars of unit u + 3
+  //   second half  dV^T += dO^T P, dK^T += Q^T dS of unit u   beside: the other transposed fragments; then, from the barrier on,
+  //                                                            the requests for Q of unit u + 4 (into unit u's generation) and
+  //                                                            what the next iteration wants first from LDS
   // The barrier stands where this wave has read all of unit u's generation and its part of unit u + 2 has landed (only
-  // the nine requests for unit u + 3 may be out): behind it everyone's has, and the generation may be overwritten.
+  // the requests for unit u + 3 may be out): behind it everyone's has, and the generation may be overwritten.
+  // At head dim 64 a unit has half the products for the same vector arithmetic: two elements per product, the last four
+  // beside the first second products, which need the first eight only.
   // (A key row past L only ever feeds its own, never stored, column of dK^T / dV^T: no masking needed.)
   f32x16_t s_a, dp_a, s_b, dp_b;
   auto iteration = [&](auto gu, f32x16_t& s_cur, f32x16_t& dp_cur, f32x16_t& s_nxt, f32x16_t& dp_nxt, int row0_u, int row0_u3,
                        int row0_u4) __attribute__((always_inline)) {
+    constexpr int EA = D == 128 ? 16 : 12;                     // elements beside the first half
     constexpr int GU = decltype(gu)::value, AT0 = GU * GEN, AT1 = ((GU + 1) & 3) * GEN, AT2 = ((GU + 2) & 3) * GEN;
     if (__builtin_expect(row0_u + 32 > L, 0)) mask_rows(row0_u);
     __builtin_amdgcn_sched_barrier(0);
@@ -258,59 +282,91 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
       for (int which = 0; which < 2; ++which) {
         const int sl = 2 * c + which;
         score_product(s_nxt, dp_nxt, c, which);
-        prob(s_cur, sl);
-        if (sl > 0) grad(s_cur, dp_cur, sl - 1);
+#pragma unroll
+        for (int i = sl * EA / (2 * DC); i < (sl + 1) * EA / (2 * DC); ++i) {
+          prob(s_cur, i);
+          if (i > 0) grad(s_cur, dp_cur, i - 1);
+        }
         if (which == 0 && c + 2 < DC) row_frags(AT1, c + 2);
         if (sl == 1) SLA_DKDV_REQUEST_DO(0, row0_u3, (GU + 3) & 3);
         if (sl == 2) SLA_DKDV_REQUEST_DO(1, row0_u3, (GU + 3) & 3);
-        if (sl == 3) SLA_DKDV_REQUEST_DO(2, row0_u3, (GU + 3) & 3);
-        if (sl == 4) SLA_DKDV_REQUEST_DO(3, row0_u3, (GU + 3) & 3);
-        if (sl == 5) SLA_DKDV_REQUEST_LD(row0_u3, (GU + 3) & 3);
-        if (sl == 9) tr_frags(AT0, 0);
-        if (sl == 11) tr_frags(AT0, 1);
-        if (sl == 13) tr_frags(AT0, 2);
-        if (sl == 15) tr_frags(AT0, 3);
+        if constexpr (NR == 4) {
+          if (sl == 3) SLA_DKDV_REQUEST_DO(NR - 2, row0_u3, (GU + 3) & 3);
+          if (sl == 4) SLA_DKDV_REQUEST_DO(NR - 1, row0_u3, (GU + 3) & 3);
+        }
+        if (sl == NR + 1) SLA_DKDV_REQUEST_LD(row0_u3, (GU + 3) & 3);
+        if (D == 128 ? (sl >= 9 && (sl & 1)) : sl >= 4) tr_frags(AT0, D == 128 ? (sl - 9) >> 1 : sl - 4);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
-    grad(s_cur, dp_cur, 15);
+    if (EA == 16) grad(s_cur, dp_cur, 15);
 #pragma unroll
-    for (int grp = 0; grp < 8; ++grp) {
-      if (grp < 4) tr_frags(AT0, grp + 4);
-      if (grp == 5) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(NREQ) : "memory");
+    for (int grp = 0; grp < NGRP; ++grp) {
+      constexpr int BAR = D == 128 ? 5 : 2;                    // the group before which the barrier stands
+      if (grp + 4 < NGRP) tr_frags(AT0, grp + 4);
+      if (grp == BAR) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(NREQ) : "memory");
+      if (EA < 16 && grp == DT) grad(s_cur, dp_cur, 15);
       second_products(grp);
-      if (grp >= 5) {
-        if (grp == 5) SLA_DKDV_REQUEST_Q(0, row0_u4, GU);
-        if (grp == 5) row_frags(AT2, 0);
-        if (grp == 6) SLA_DKDV_REQUEST_Q(1, row0_u4, GU);
-        if (grp == 6) read_delta(AT2, dp_cur, 0);
-        if (grp == 6) read_delta(AT2, dp_cur, 1);
-        if (grp == 6) read_delta(AT2, dp_cur, 2);
-        if (grp == 6) read_delta(AT2, dp_cur, 3);
-        if (grp == 7) SLA_DKDV_REQUEST_Q(2, row0_u4, GU);
-        if (grp == 7) SLA_DKDV_REQUEST_Q(3, row0_u4, GU);
-        if (grp == 7) row_frags(AT2, 1);
+      if (EA < 16 && grp < DT) {
+        constexpr int PER = (16 - EA) / DT;
+#pragma unroll
+        for (int i = EA + grp * PER; i < EA + (grp + 1) * PER; ++i) {
+          prob(s_cur, i);
+          grad(s_cur, dp_cur, i - 1);
+        }
       }
-      if (grp >= 3 && grp < 7) read_lse(AT1, grp - 3);
+      if (grp == BAR) {
+        SLA_DKDV_REQUEST_Q(0, row0_u4, GU);
+        row_frags(AT2, 0);
+      }
+      if (grp == BAR + 1) {
+        SLA_DKDV_REQUEST_Q(1, row0_u4, GU);
+#pragma unroll
+        for (int i4 = 0; i4 < 4; ++i4) read_delta(AT2, dp_cur, i4);
+      }
+      if (grp == NGRP - 1) {
+        if constexpr (NR == 4) {
+          SLA_DKDV_REQUEST_Q(NR - 2, row0_u4, GU);
+          SLA_DKDV_REQUEST_Q(NR - 1, row0_u4, GU);
+        }
+        row_frags(AT2, 1);
+      }
+      if (D == 128 ? grp >= 3 && grp < 7 : grp >= 2) {
+        read_lse(AT1, D == 128 ? grp - 3 : 2 * grp - 4);
+        if (D == 64) read_lse(AT1, 2 * grp - 3);
+      }
       __builtin_amdgcn_sched_barrier(0);
     }
   };
 
   __syncthreads();                                             // the zeros and the entries are in place before anything is requested
+  const auto request_q = [&](int row0, int gen) __attribute__((always_inline)) {
+    SLA_DKDV_REQUEST_Q(0, row0, gen);
+    SLA_DKDV_REQUEST_Q(1, row0, gen);
+    if constexpr (NR == 4) {
+      SLA_DKDV_REQUEST_Q(NR - 2, row0, gen);
+      SLA_DKDV_REQUEST_Q(NR - 1, row0, gen);
+    }
+  };
+  const auto request_unit = [&](int row0, int gen) __attribute__((always_inline)) {
+    request_q(row0, gen);
+    SLA_DKDV_REQUEST_DO(0, row0, gen);
+    SLA_DKDV_REQUEST_DO(1, row0, gen);
+    if constexpr (NR == 4) {
+      SLA_DKDV_REQUEST_DO(NR - 2, row0, gen);
+      SLA_DKDV_REQUEST_DO(NR - 1, row0, gen);
+    }
+    SLA_DKDV_REQUEST_LD(row0, gen);
+  };
   // first query rows of the listed blocks: E0 = of the entry of units u and u + 1, E1 = of the next one, E2 = of the one after
   int E0 = 0, E1 = 0, E2 = 0;
   if (nent > 0) {
     E0 = entry_row0(0);
     E1 = entry_row0(1);
     E2 = entry_row0(2);
-#define SLA_DKDV_REQUEST_UNIT(ROW0, G)                                                                                          \
-  SLA_DKDV_REQUEST_Q(0, ROW0, G); SLA_DKDV_REQUEST_Q(1, ROW0, G); SLA_DKDV_REQUEST_Q(2, ROW0, G); SLA_DKDV_REQUEST_Q(3, ROW0, G);     \
-  SLA_DKDV_REQUEST_DO(0, ROW0, G); SLA_DKDV_REQUEST_DO(1, ROW0, G); SLA_DKDV_REQUEST_DO(2, ROW0, G); SLA_DKDV_REQUEST_DO(3, ROW0, G); \
-  SLA_DKDV_REQUEST_LD(ROW0, G)
-    SLA_DKDV_REQUEST_UNIT(E0, 0);
-    SLA_DKDV_REQUEST_UNIT(E0 + 32, 1);
-    SLA_DKDV_REQUEST_UNIT(E1, 2);
-#undef SLA_DKDV_REQUEST_UNIT
+    request_unit(E0, 0);
+    request_unit(E0 + 32, 1);
+    request_unit(E1, 2);
   }
   // (the wait for the K^T and V^T fragments comes here, behind the first requests, which only needed the list)
 #pragma unroll
@@ -335,8 +391,7 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     }
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");         // (the vector ALU reads these results next)
     asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(NREQ) : "memory");
-    SLA_DKDV_REQUEST_Q(0, E1 + 32, 3); SLA_DKDV_REQUEST_Q(1, E1 + 32, 3);
-    SLA_DKDV_REQUEST_Q(2, E1 + 32, 3); SLA_DKDV_REQUEST_Q(3, E1 + 32, 3);
+    request_q(E1 + 32, 3);
     row_frags(GEN, 0);
     row_frags(GEN, 1);
 #pragma unroll
@@ -344,18 +399,18 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     int last_at;                                               // where the last unit lies (an odd one: generation 1 or 3)
     for (int b = 0;; b += 2) {
       int E3 = entry_row0(b + 3);                              // (looked up now, used two units from now)
-      iteration(std::integral_constant<int, 0>{}, s_a, dp_a, s_b, dp_b, E0, E1 + 32, E2);
+      iteration(I<0>{}, s_a, dp_a, s_b, dp_b, E0, E1 + 32, E2);
       last_at = GEN;
       if (b + 1 >= nent) break;
-      iteration(std::integral_constant<int, 1>{}, s_b, dp_b, s_a, dp_a, E0 + 32, E2, E2 + 32);
+      iteration(I<1>{}, s_b, dp_b, s_a, dp_a, E0 + 32, E2, E2 + 32);
       E0 = E1;
       E1 = E2;
       E2 = E3;
       E3 = entry_row0(b + 4);
-      iteration(std::integral_constant<int, 2>{}, s_a, dp_a, s_b, dp_b, E0, E1 + 32, E2);
+      iteration(I<2>{}, s_a, dp_a, s_b, dp_b, E0, E1 + 32, E2);
       last_at = 3 * GEN;
       if (b + 2 >= nent) break;
-      iteration(std::integral_constant<int, 3>{}, s_b, dp_b, s_a, dp_a, E0 + 32, E2, E2 + 32);
+      iteration(I<3>{}, s_b, dp_b, s_a, dp_a, E0 + 32, E2, E2 + 32);
       E0 = E1;
       E1 = E2;
       E2 = E3;
@@ -370,8 +425,8 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
       grad(s_b, dp_b, i);
     }
 #pragma unroll
-    for (int grp = 0; grp < 8; ++grp) {
-      if (grp < 4) tr_frags(last_at, grp + 4);
+    for (int grp = 0; grp < NGRP; ++grp) {
+      if (grp + 4 < NGRP) tr_frags(last_at, grp + 4);
       second_products(grp);
     }
   }
@@ -430,8 +485,8 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 
 
 // ---- dQ ------------------------------------------------------------------------------------------------------------
-// dQ of the block-sparse attention backward for 64-row query blocks at head dim 128: one wave per query block, one wave
-// per SIMD, no barriers.
+// dQ of the block-sparse attention backward for 64-row query blocks: one wave per query block, one wave per SIMD, no
+// barriers.
 //
 // Stands in for _attn_bwd_dq of the reference (sparse_linear_attention/kernel.py:95-157) like bwd_dq_kernel, whose
 // arithmetic it shares (S^T = K Q^T and dP^T = V dO^T, so that the log-sum-exp and delta of a query are per-lane
@@ -448,9 +503,11 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 // instructions per unit where reading the row-wise fragments once per tile took 367.  Measured, that version against this:
 // B1 H12 L32760 with 25 key blocks per row 551 -> 485 us (matrix pipe busy 53 -> 61 % of the cycles, at a clock that the
 // power limit holds at 1.65 GHz), B2 H16 L32760 with 128-row blocks 1428 -> 1224 us, B2 H4 L4096 37.9 -> 33.2 us.
+// Head dim 64 against bwd_dq_kernel, whole backward: B1 H12 L32760 with 25 key blocks 891 -> 673 us, B1 H16 L16380 with
+// 128-row blocks 538 -> 442 us, B1 H16 L2000 59.5 -> 52.0 us.
 constexpr int DQ_STREAM_MAX_T = 2048;          // look-up rows longer than this take bwd_dq_kernel
 
-template <typename Tag>
+template <typename Tag, int D>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void bwd_dq_stream_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
     const uint16_t* __restrict__ d_o, const uint16_t* __restrict__ o, const float* __restrict__ lse, float* __restrict__ delta,
@@ -458,9 +515,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
     int Mblk, int topk, float qk_scale, int total, int wide) {
   // (Mblk: 64-row blocks per head.  wide = 1: the look-up table has one row per 128-row block, which both halves follow)
   using E = Elem<Tag>;
-  constexpr int D = 128, DC = D / 16, DT = D / 32;
-  constexpr int ROWB = D * 2;
-  constexpr int TILE = 8 * REQ_PITCH;             // 32 rows of K or V
+  using T32 = BwdTile<D>;
+  constexpr int DC = D / 16, DT = D / 32;
+  constexpr int TILE = T32::BYTES;                // 32 rows of K or V
+  constexpr int NR = T32::NREQ;                   // requests per tile
+  constexpr int ROWS8 = 8 / T32::RPR * REQ_PITCH; // 8 rows further on in a tile
   __shared__ __attribute__((aligned(16))) uint8_t smem[4 * TILE];      // K generation 0, 1; V generation 0, 1
   __shared__ uint16_t entries[DQ_STREAM_MAX_T];                        // this block's look-up row
 
@@ -524,47 +583,58 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
       for (int i = 0; i < 16; ++i) dqacc[dt][qt][i] = 0.f;
 
   // ---- addressing ----
-  // A request moves 4 rows (64 lanes x 16 bytes): lane -> row 4 j + lane / 16, 16-byte slot lane % 16, which receives
-  // piece (slot ^ 4 (row % 4)) of that row; requests are padded by one 16-byte slot.  For one piece the 16 rows of a
-  // row-wise read hit 16 different slots (row % 4 picks the group of four, row / 4 the slot in it), and so do the
-  // 4 rows x 4 pieces of a transposing read.
+  // A request moves RPR rows (64 lanes x 16 bytes): lane -> row RPR j + lane / (D / 8), 16-byte slot lane % (D / 8), which
+  // receives piece (slot ^ swz(row)) of that row.
   const uint32_t smem_addr = __builtin_amdgcn_readfirstlane((uint32_t)(size_t)smem);
-  const int lrow = lane >> 4, lslot = lane & 15;
-  uint32_t koff[4];                  // rows 4 j + lane / 16; sixteen rows more for the second half of a tile
+  const int lrow = lane / (D / 8), lslot = lane % (D / 8);
+  uint32_t koff[4];                  // requests 0 .. 3; head dim 128: sixteen rows more for requests 4 .. 7
 #pragma unroll
   for (int j = 0; j < 4; ++j)
-    koff[j] = (uint32_t)(4 * j + lrow) * row_bytes + (uint32_t)(lslot ^ (4 * lrow)) * 16 + REQ_SLACK - j * REQ_PITCH;
+    koff[j] = (uint32_t)(T32::RPR * j + lrow) * row_bytes + (uint32_t)(lslot ^ T32::swz(lrow)) * 16 + REQ_SLACK - j * REQ_PITCH;
   const uint32_t half_bytes = 16 * row_bytes;
   const int row_none = (L + 63) & ~63;            // past every head: such requests touch neither memory nor LDS
   auto entry_row0 = [&](int e) __attribute__((always_inline)) -> int {
     const int row0 = __builtin_amdgcn_readfirstlane((int)entries[min(e, topk - 1)]) * 64;
     return e < topk ? row0 : row_none;
   };
-  // request J (rows 4 J ..) of the 32 rows from key0 on, into the tile at LDS address `tile`
-#define SLA_DQ_REQUEST(RSRC, J, KEY0, TILE_AT)                                                                       \
-  lds_dma_row4<(J) & 3>(RSRC, koff[(J) & 3] + ((uint32_t)(KEY0) * row_bytes + ((J) >= 4 ? half_bytes : 0u)),          \
-                        smem_addr + (uint32_t)(TILE_AT) + ((J) >> 2) * 4 * REQ_PITCH)
-  // fragments: row-wise, row r, piece 2 c + g: one base per c / 2; transposed, rows tr_row and tr_row + 8 (and 16 further
-  // for the second half), 8 bytes at element 4 (lane % 4) of the 16-column strip 2 dt + (lane / 16) % 2: one base per dt
+  // request J (rows RPR J ..) of the 32 rows from key0 on, into the tile at LDS address `tile`; SET: the first of its group
+#define SLA_DQ_REQUEST(RSRC, J, SET, KEY0, TILE_AT)                                                                  \
+  lds_dma_row4<(J) & 3, SET>(RSRC, koff[(J) & 3] + ((uint32_t)(KEY0) * row_bytes + ((J) >= 4 ? half_bytes : 0u)),     \
+                             smem_addr + (uint32_t)(TILE_AT) + ((J) >> 2) * 4 * REQ_PITCH)
+  // the first (H = 0) or second sixteen rows of a tile, request i of them
+  auto request_half = [&](const __amdgpu_buffer_rsrc_t& rsrc, auto h, auto i, int key0, int tile_at) __attribute__((always_inline)) {
+    constexpr int J = decltype(h)::value * (NR / 2) + decltype(i)::value;
+    SLA_DQ_REQUEST(rsrc, J, decltype(i)::value == 0, key0, tile_at);
+  };
+  auto request_rows = [&](const __amdgpu_buffer_rsrc_t& rsrc, auto h, int key0, int tile_at) __attribute__((always_inline)) {
+    request_half(rsrc, h, I<0>{}, key0, tile_at);
+    request_half(rsrc, h, I<1>{}, key0, tile_at);
+    if constexpr (NR == 8) {
+      request_half(rsrc, h, I<2>{}, key0, tile_at);
+      request_half(rsrc, h, I<3>{}, key0, tile_at);
+    }
+  };
+  // fragments: row-wise, row r, piece 2 c + g: four bases; transposed, rows tr_row and tr_row + 8 (and 16 further for the
+  // second half), 8 bytes at element 4 (lane % 4) of the 16-column strip 2 dt + (lane / 16) % 2: one base per dt
   const uint8_t* rfp[4];
   const uint8_t* tfp[DT];
   const int tr_row = 4 * g + ((lane & 15) >> 2);
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    rfp[i] = smem + r * ROWB + (r >> 2) * 16 + ((4 * i + g) ^ (4 * (r & 3))) * 16;
-    tfp[i] = smem + tr_row * ROWB + (tr_row >> 2) * 16 +
-             ((4 * i + 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1)) ^ (4 * (tr_row & 3))) * 16 + (lane & 1) * 8;
-  }
+  for (int i = 0; i < 4; ++i) rfp[i] = smem + T32::piece_at(r, 2 * (i * DC / 4) + g);
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+    tfp[dt] = smem + T32::piece_at(tr_row, 4 * dt + 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1)) + (lane & 1) * 8;
   i16x8_t af[3], bf[3];              // row-wise K and V fragments, two chunks ahead
   i16x8_t trk[2][DT];                // transposed K fragments of the unit whose dQ products come next
   auto row_frags = [&](int GEN, int c) __attribute__((always_inline)) {
-    af[c % 3] = *reinterpret_cast<const i16x8_t*>(rfp[c >> 1] + GEN * TILE + (c & 1) * 32);
-    bf[c % 3] = *reinterpret_cast<const i16x8_t*>(rfp[c >> 1] + (2 + GEN) * TILE + (c & 1) * 32);
+    const uint8_t* p = rfp[c * 4 / DC] + GEN * TILE + (D == 128 ? (c & 1) * 32 : 0);
+    af[c % 3] = *reinterpret_cast<const i16x8_t*>(p);
+    bf[c % 3] = *reinterpret_cast<const i16x8_t*>(p + 2 * TILE);
   };
   auto tr_frag = [&](int GEN, int c2, int dt) __attribute__((always_inline)) {
-    const uint8_t* t0 = tfp[dt] + GEN * TILE + 4 * c2 * REQ_PITCH;
+    const uint8_t* t0 = tfp[dt] + GEN * TILE + 2 * c2 * ROWS8;
     trk[c2][dt] = concat4(lds_read_tr16(reinterpret_cast<const uint16_t*>(t0)),
-                          lds_read_tr16(reinterpret_cast<const uint16_t*>(t0 + 2 * REQ_PITCH)));
+                          lds_read_tr16(reinterpret_cast<const uint16_t*>(t0 + ROWS8)));
   };
 
   struct Tiles {
@@ -588,7 +658,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
       dsw[qt][i >> 3][(i >> 1) & 3] = (int)a;
     }
   };
-  // product 4 c + {0, 1, 2, 3} of the 32: S and dP of tile 0, then of tile 1, chunk c of the head dimension
+  // element e of the unit's 32 in the order the dQ products want them: the first eight registers of both tiles, then the others
+  auto element = [&](Tiles& t, int e) __attribute__((always_inline)) {
+    const auto qt = [](int n) __attribute__((always_inline)) { return (n >> 3) & 1; };
+    const auto at = [](int n) __attribute__((always_inline)) { return (n >> 4) * 8 + (n & 7); };
+    if (e < 32) prob(t, qt(e), at(e));
+    if (e > 0) grad(t, qt(e - 1), at(e - 1));
+  };
+  // product 4 c + {0, 1, 2, 3} of the first ones: S and dP of tile 0, then of tile 1, chunk c of the head dimension
   auto score_product = [&](Tiles& t, int c, int which) __attribute__((always_inline)) {
     const int qt = which >> 1;
     if (which & 1) {
@@ -608,15 +685,18 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
         if (8 * (i >> 2) + (i & 3) >= lim) t.s[qt][i] = -INFINITY;
   };
 
-  // One iteration = unit u (generation GU = u % 2), 48 products:
-  //   slots  0..31  S and dP of unit u + 1 into `nxt`        beside: P and dS of unit u (in `cur`), K rows 16.. of unit u + 2
-  //   slots 32..47  dQ += K^T dS of unit u                    beside: V and K rows 0..15 of unit u + 3, and from unit u + 1
-  //                                                           the transposed K fragments, from u + 2 the first row-wise ones
-  // Requests are answered in order.  When the row-wise fragments of unit u + 2 are first read, only the eight requests for
-  // V of unit u + 3 may be out; a tile half is requested again only behind a product that waited for LDS reads issued after
+  // One iteration = unit u (generation GU = u % 2), 3 D / 8 products:
+  //   first two thirds  S and dP of unit u + 1 into `nxt`     beside: P and dS of unit u (in `cur`), K rows 16.. of unit u + 2
+  //   last third        dQ += K^T dS of unit u                 beside: V and K rows 0..15 of unit u + 3, and from unit u + 1
+  //                                                            the transposed K fragments, from u + 2 the first row-wise ones
+  // Requests are answered in order.  When the row-wise fragments of unit u + 2 are first read, only the requests for V of
+  // unit u + 3 may be out; a tile half is requested again only behind a product that waited for LDS reads issued after
   // the last read of that half (LDS reads return in order).
-  auto iteration = [&](int GU, Tiles& cur, Tiles& nxt, int key_u, int key_u2, int key_u3) __attribute__((always_inline)) {
-    const int GN = GU ^ 1;
+  // At head dim 64 there are half the products for the same vector arithmetic: the last four elements come beside the first
+  // four dQ products, which need the first sixteen only.
+  auto iteration = [&](auto gu, Tiles& cur, Tiles& nxt, int key_u, int key_u2, int key_u3) __attribute__((always_inline)) {
+    constexpr int GU = decltype(gu)::value, GN = GU ^ 1;
+    constexpr int EA = D == 128 ? 32 : 28;                     // elements beside the first products
     if (__builtin_expect(L - key_u < 32, 0)) mask_tail(cur, L - key_u);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -625,40 +705,49 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
       for (int which = 0; which < 4; ++which) {
         const int sl = 4 * c + which;
         score_product(nxt, c, which);
-        prob(cur, sl >> 4, sl & 15);
-        if (sl > 0) grad(cur, (sl - 1) >> 4, (sl - 1) & 15);
+#pragma unroll
+        for (int e = sl * EA / (4 * DC); e < (sl + 1) * EA / (4 * DC); ++e) element(cur, e);
         if (which == 1 && c + 2 < DC) row_frags(GN, c + 2);
-        if (sl == 12) SLA_DQ_REQUEST(kh, 4, key_u2, GU * TILE);
-        if (sl == 15) SLA_DQ_REQUEST(kh, 5, key_u2, GU * TILE);
-        if (sl == 18) SLA_DQ_REQUEST(kh, 6, key_u2, GU * TILE);
-        if (sl == 21) SLA_DQ_REQUEST(kh, 7, key_u2, GU * TILE);
+        if (sl == 12) request_half(kh, I<1>{}, I<0>{}, key_u2, GU * TILE);
+        if (sl == (D == 128 ? 15 : 14)) request_half(kh, I<1>{}, I<1>{}, key_u2, GU * TILE);
+        if constexpr (NR == 8) {
+          if (sl == 18) request_half(kh, I<1>{}, I<2>{}, key_u2, GU * TILE);
+          if (sl == 21) request_half(kh, I<1>{}, I<3>{}, key_u2, GU * TILE);
+        }
         __builtin_amdgcn_sched_barrier(0);
       }
     }
-    grad(cur, 1, 15);
+    if (EA == 32) element(cur, 32);
 #pragma unroll
-    for (int sl = 0; sl < 16; ++sl) {
-      const int c2 = sl >> 3, dt = (sl >> 1) & 3, qt = sl & 1;
+    for (int sl = 0; sl < 4 * DT; ++sl) {
+      const int c2 = sl / (2 * DT), dt = (sl >> 1) % DT, qt = sl & 1;
+      if (EA < 32 && sl == 2 * DT) element(cur, 32);
       dqacc[dt][qt] = E::mfma32(trk[c2][dt], __builtin_bit_cast(i16x8_t, dsw[qt][c2]), dqacc[dt][qt]);
-      if (sl == 0) SLA_DQ_REQUEST(vh, 0, key_u3, (2 + GN) * TILE);
-      if (sl == 1) SLA_DQ_REQUEST(vh, 1, key_u3, (2 + GN) * TILE);
-      if (sl == 2) SLA_DQ_REQUEST(vh, 2, key_u3, (2 + GN) * TILE);
-      if (sl == 3) SLA_DQ_REQUEST(vh, 3, key_u3, (2 + GN) * TILE);
-      if (sl == 4) SLA_DQ_REQUEST(vh, 4, key_u3, (2 + GN) * TILE);
-      if (sl == 5) SLA_DQ_REQUEST(vh, 5, key_u3, (2 + GN) * TILE);
-      if (sl == 6) SLA_DQ_REQUEST(vh, 6, key_u3, (2 + GN) * TILE);
-      if (sl == 7) SLA_DQ_REQUEST(vh, 7, key_u3, (2 + GN) * TILE);
-      if (qt == 1) tr_frag(GN, c2, dt);
-      if (sl == 9) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-      if (sl == 10) row_frags(GU, 0);
-      if (sl == 12) row_frags(GU, 1);
-      if (sl == 12) {
-        asm volatile("s_waitcnt lgkmcnt(6)" ::: "memory");       // (K rows 0..15 of unit u + 1 have been read: eight reads came after)
-        SLA_DQ_REQUEST(kh, 0, key_u3, GN * TILE);
+      if (EA < 32 && sl < 32 - EA) element(cur, EA + sl);
+      if (sl == 0) request_half(vh, I<0>{}, I<0>{}, key_u3, (2 + GN) * TILE);
+      if (sl == 1) request_half(vh, I<0>{}, I<1>{}, key_u3, (2 + GN) * TILE);
+      if constexpr (NR == 8) {
+        if (sl == 2) request_half(vh, I<0>{}, I<2>{}, key_u3, (2 + GN) * TILE);
+        if (sl == 3) request_half(vh, I<0>{}, I<3>{}, key_u3, (2 + GN) * TILE);
+        if (sl == 6) request_half(vh, I<1>{}, I<2>{}, key_u3, (2 + GN) * TILE);
+        if (sl == 7) request_half(vh, I<1>{}, I<3>{}, key_u3, (2 + GN) * TILE);
       }
-      if (sl == 13) SLA_DQ_REQUEST(kh, 1, key_u3, GN * TILE);
-      if (sl == 14) SLA_DQ_REQUEST(kh, 2, key_u3, GN * TILE);
-      if (sl == 15) SLA_DQ_REQUEST(kh, 3, key_u3, GN * TILE);
+      if (sl == NR / 2) request_half(vh, I<1>{}, I<0>{}, key_u3, (2 + GN) * TILE);
+      if (sl == NR / 2 + 1) request_half(vh, I<1>{}, I<1>{}, key_u3, (2 + GN) * TILE);
+      if (qt == 1) tr_frag(GN, c2, dt);
+      constexpr int W = D == 128 ? 9 : 4;                      // unit u + 2 has landed from here on
+      if (sl == W) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NR) : "memory");
+      if (sl == W + 1) row_frags(GU, 0);
+      if (sl == (D == 128 ? 12 : 6)) {
+        row_frags(GU, 1);
+        asm volatile("s_waitcnt lgkmcnt(4)" ::: "memory");     // (K rows 0..15 of unit u + 1 have been read: six or more reads came after)
+        request_half(kh, I<0>{}, I<0>{}, key_u3, GN * TILE);
+      }
+      if (sl == (D == 128 ? 13 : 7)) request_half(kh, I<0>{}, I<1>{}, key_u3, GN * TILE);
+      if constexpr (NR == 8) {
+        if (sl == 14) request_half(kh, I<0>{}, I<2>{}, key_u3, GN * TILE);
+        if (sl == 15) request_half(kh, I<0>{}, I<3>{}, key_u3, GN * TILE);
+      }
       __builtin_amdgcn_sched_barrier(0);
     }
   };
@@ -669,16 +758,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
     E0 = entry_row0(0);
     E1 = entry_row0(1);
     E2 = entry_row0(2);
-#define SLA_DQ_REQUEST8(RSRC, KEY0, TILE_AT)                                                                         \
-  SLA_DQ_REQUEST(RSRC, 0, KEY0, TILE_AT); SLA_DQ_REQUEST(RSRC, 1, KEY0, TILE_AT);                                    \
-  SLA_DQ_REQUEST(RSRC, 2, KEY0, TILE_AT); SLA_DQ_REQUEST(RSRC, 3, KEY0, TILE_AT);                                    \
-  SLA_DQ_REQUEST(RSRC, 4, KEY0, TILE_AT); SLA_DQ_REQUEST(RSRC, 5, KEY0, TILE_AT);                                    \
-  SLA_DQ_REQUEST(RSRC, 6, KEY0, TILE_AT); SLA_DQ_REQUEST(RSRC, 7, KEY0, TILE_AT)
-    SLA_DQ_REQUEST8(kh, E0, 0);
-    SLA_DQ_REQUEST8(vh, E0, 2 * TILE);
-    SLA_DQ_REQUEST8(kh, E0 + 32, TILE);
-    SLA_DQ_REQUEST8(vh, E0 + 32, 3 * TILE);
-#undef SLA_DQ_REQUEST8
+    request_rows(kh, I<0>{}, E0, 0);
+    request_rows(kh, I<1>{}, E0, 0);
+    request_rows(vh, I<0>{}, E0, 2 * TILE);
+    request_rows(vh, I<1>{}, E0, 2 * TILE);
+    request_rows(kh, I<0>{}, E0 + 32, TILE);
+    request_rows(kh, I<1>{}, E0 + 32, TILE);
+    request_rows(vh, I<0>{}, E0 + 32, 3 * TILE);
+    request_rows(vh, I<1>{}, E0 + 32, 3 * TILE);
   }
   // delta of this lane's two rows.  The sum runs in the order of bwd_delta_kernel, whose thread t adds the eight products
   // of columns 8t .. 8t+7 one after the other and then meets threads t^1, t^2, t^4, t^8: here t = 2c + g, so the first
@@ -711,7 +798,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
     for (int c = 0; c < DC; ++c) asm volatile("" : "+a"(qf[qt][c]), "+a"(dof[qt][c]));
   if (topk > 0) {
     // (the two rows of delta written above count as memory operations too: two more may be out)
-    asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NR) : "memory");
     row_frags(0, 0);
     row_frags(0, 1);
 #pragma unroll
@@ -726,18 +813,17 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
       for (int dt = 0; dt < DT; ++dt) tr_frag(0, c2, dt);
     // (the vector ALU reads the products' results next; every fragment of unit 0 has been read)
     asm volatile("s_nop 15\n\ts_nop 15\n\ts_waitcnt lgkmcnt(0)" ::: "memory");
-    SLA_DQ_REQUEST(vh, 0, E1, 2 * TILE); SLA_DQ_REQUEST(vh, 1, E1, 2 * TILE); SLA_DQ_REQUEST(vh, 2, E1, 2 * TILE);
-    SLA_DQ_REQUEST(vh, 3, E1, 2 * TILE); SLA_DQ_REQUEST(vh, 4, E1, 2 * TILE); SLA_DQ_REQUEST(vh, 5, E1, 2 * TILE);
-    SLA_DQ_REQUEST(vh, 6, E1, 2 * TILE); SLA_DQ_REQUEST(vh, 7, E1, 2 * TILE);
-    SLA_DQ_REQUEST(kh, 0, E1, 0); SLA_DQ_REQUEST(kh, 1, E1, 0); SLA_DQ_REQUEST(kh, 2, E1, 0); SLA_DQ_REQUEST(kh, 3, E1, 0);
-    asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
+    request_rows(vh, I<0>{}, E1, 2 * TILE);
+    request_rows(vh, I<1>{}, E1, 2 * TILE);
+    request_rows(kh, I<0>{}, E1, 0);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NR + NR / 2) : "memory");
     row_frags(1, 0);
     row_frags(1, 1);
     for (int b = 0;; ++b) {
       const int E3 = entry_row0(b + 3);                       // (looked up now, used two units from now)
-      iteration(0, ta, tb, E0, E1, E1 + 32);                  // unit 2 b
+      iteration(I<0>{}, ta, tb, E0, E1, E1 + 32);                  // unit 2 b
       if (b + 1 >= topk) break;
-      iteration(1, tb, ta, E0 + 32, E1 + 32, E2);             // unit 2 b + 1
+      iteration(I<1>{}, tb, ta, E0 + 32, E1 + 32, E2);             // unit 2 b + 1
       E0 = E1;
       E1 = E2;
       E2 = E3;
@@ -745,15 +831,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
     // the last unit: no scores left to form beside its arithmetic
     if (__builtin_expect(L - (E0 + 32) < 32, 0)) mask_tail(tb, L - (E0 + 32));
 #pragma unroll
-    for (int qt = 0; qt < 2; ++qt)
+    for (int e = 0; e <= 32; ++e) element(tb, e);
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        prob(tb, qt, i);
-        grad(tb, qt, i);
-      }
-#pragma unroll
-    for (int sl = 0; sl < 16; ++sl) {
-      const int c2 = sl >> 3, dt = (sl >> 1) & 3, qt = sl & 1;
+    for (int sl = 0; sl < 4 * DT; ++sl) {
+      const int c2 = sl / (2 * DT), dt = (sl >> 1) % DT, qt = sl & 1;
       dqacc[dt][qt] = E::mfma32(trk[c2][dt], __builtin_bit_cast(i16x8_t, dsw[qt][c2]), dqacc[dt][qt]);
     }
   }

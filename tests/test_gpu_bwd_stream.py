@@ -1,4 +1,4 @@
-"""The head-dim-128 backward kernels at the edges of their loops: table rows of one to three key blocks (the rotated loop's
+"""The backward kernels at the edges of their loops: table rows of one to three key blocks (the rotated loop's
 prologue and tail meet), lists of none to many query blocks, last blocks whose halves of 32 rows are short, full or missing."""
 import pytest
 import torch
@@ -15,9 +15,10 @@ pytestmark = pytest.mark.gpu
                                                (28, 768, 12, 64, torch.bfloat16),    # every key block
                                                (80, 801, 1, 128, torch.bfloat16),    # 128-row blocks, the last without a second half
                                                (80, 831, 2, 128, torch.float16)])
-def test_short_rows_and_lists(dev, H, L, T, BLKQ, dtype):
+@pytest.mark.parametrize("D", [128, 64])
+def test_short_rows_and_lists(dev, H, L, T, BLKQ, dtype, D):
     g = torch.Generator().manual_seed(L + T)
-    q, k, v, do = (torch.randn(1, H, L, 128, generator=g).to(dtype) for _ in range(4))
+    q, k, v, do = (torch.randn(1, H, L, D, generator=g).to(dtype) for _ in range(4))
     M, N = -(-L // BLKQ), -(-L // 64)
     # the last key block in every third row, the others drawn from the first half of the rest: some lists stay empty
     lut = torch.stack([torch.randperm(N if T == N else max(N // 2, T), generator=g)[:T] for _ in range(H * M)])
