@@ -135,15 +135,16 @@ def _module_bwd_saved(saved, off, q_ptr, k_ptr, v_ptr, s_qkv, d_out, s_do, weigh
     n_l = _lib.workspace_bytes(_lib.WS_LINEAR_BWD_STATES_APART, dt, B, H, L, D, 64, 64, 0)
     n_s = -(-n_s // 256) * 256
     ws = torch.empty(n_s + n_l, dtype=torch.uint8, device=dev)
-    dwb = torch.empty(D * D + D, dtype=torch.float32, device=dev)
+    dw = torch.empty((D, D), dtype=torch.float32, device=dev)
+    db = torch.empty((D,), dtype=torch.float32, device=dev)
     base, w0 = saved.data_ptr(), ws.data_ptr()
     rc = _lib.load().sla_module_bwd_states(
         q_ptr, k_ptr, v_ptr, s_qkv, base + off["o_s"], d_out.data_ptr(), s_do, base + off["lse"], base + off["map"],
-        base + off["lut"], 4, weight.data_ptr(), bias.data_ptr(), base + off["states"], *grads, dwb.data_ptr(),
-        dwb.data_ptr() + D * D * 4, dt, _lib.FMAP[fmap], B, H, L, D, BLKQ, BLKK, T, D ** -0.5, w0, n_s, w0 + n_s, n_l,
+        base + off["lut"], 4, weight.data_ptr(), bias.data_ptr(), base + off["states"], *grads, dw.data_ptr(),
+        db.data_ptr(), dt, _lib.FMAP[fmap], B, H, L, D, BLKQ, BLKK, T, D ** -0.5, w0, n_s, w0 + n_s, n_l,
         _lib.stream_ptr(dev), _side_stream(dev))
     _lib.check(rc)
-    return dwb[:D * D].view(D, D), dwb[D * D:]
+    return dw, db
 
 
 class _sla_core(torch.autograd.Function):
@@ -172,16 +173,16 @@ class _sla_core(torch.autograd.Function):
         shape, in_dt, T, BLKQ, BLKK, fmap, dtype, in_dtype = ctx.cfg
         off = _plan(in_dt, _lib.dtype_code(dtype), *shape, BLKQ, BLKK, T, True)[2]
         d_out = d_out.contiguous().to(dtype)
-        g = torch.empty((3, *shape), dtype=dtype, device=d_out.device)
-        step = g.stride(0) * g.element_size()
-        g0 = g.data_ptr()
+        # (an allocation per gradient: a caller may keep one of them, or detach it in place, without the others)
+        grads = [torch.empty(shape, dtype=dtype, device=d_out.device) for _ in range(3)]
         if qkv:
             ptrs = [t.data_ptr() for t in qkv]
         else:
+            step = grads[0].numel() * grads[0].element_size()
             ptrs = [saved.data_ptr() + off["cast"] + i * step for i in range(3)]
-        dw, db = _module_bwd_saved(saved, off, *ptrs, None, d_out, None, weight, bias, (g0, g0 + step, g0 + 2 * step), shape,
+        dw, db = _module_bwd_saved(saved, off, *ptrs, None, d_out, None, weight, bias, [t.data_ptr() for t in grads], shape,
                                    dtype, T, BLKQ, BLKK, fmap)
-        return (*g.to(in_dtype).unbind(0), dw, db, None, None, None, None, None, None)
+        return (*(t.to(in_dtype) for t in grads), dw, db, None, None, None, None, None, None)
 
 
 class _sla_complement(torch.autograd.Function):

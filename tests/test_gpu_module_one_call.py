@@ -42,3 +42,14 @@ def test_one_call_equals_the_steps(dev, H, L, D, BLKQ, in_dtype, half):
         for name, t, r in zip(("dq", "dk", "dv"), (qg, kg, vg), ref):
             assert torch.equal(t.grad, r.to(in_dtype)), name
         assert torch.equal(mod.proj_l.weight.grad, dw) and torch.equal(mod.proj_l.bias.grad, db)
+
+
+@pytest.mark.parametrize("in_dtype", [torch.bfloat16, torch.float32])
+def test_gradients_own_their_memory(dev, in_dtype):
+    """What the backward returns can be detached in place and kept one without the others."""
+    mod = SparseLinearAttention(64, 0.5).to(dev)
+    x = [torch.randn(1, 2, 256, 64, device=dev, dtype=in_dtype, requires_grad=True) for _ in range(3)]
+    inputs = [*x, mod.proj_l.weight, mod.proj_l.bias]
+    for t, grad in zip(inputs, torch.autograd.grad(mod(*x).sum(), inputs)):
+        assert grad.shape == t.shape and not grad._is_view()
+        assert grad.untyped_storage().nbytes() == t.numel() * t.element_size()
