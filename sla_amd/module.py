@@ -349,8 +349,9 @@ class SparseLinearAttention(nn.Module):
         weight = self.proj_l.weight.contiguous()
         bias = self.proj_l.bias.contiguous()
         mask = None
-        if not (q.dtype == k.dtype == v.dtype and (dtype == self.dtype or dtype == torch.float32)):
-            # the mask is built from the inputs in their own dtype (reference core.py:83), the rest works on copies
+        if not (q.dtype == k.dtype == v.dtype and (dtype == self.dtype or (dtype == torch.float32 and v.data_ptr() % 16 == 0))):
+            # the mask is built from the inputs in their own dtype (reference core.py:83), the rest works on copies (which the
+            # library makes itself of fp32 tensors that lie on 16 bytes)
             with torch.no_grad():
                 mask = get_block_map(q, k, topk_ratio=self.topk, BLKQ=self.BLKQ, BLKK=self.BLKK)[:2]
             q, k, v = q.to(self.dtype), k.to(self.dtype), v.to(self.dtype)

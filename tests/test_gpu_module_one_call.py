@@ -53,3 +53,18 @@ def test_gradients_own_their_memory(dev, in_dtype):
     for t, grad in zip(inputs, torch.autograd.grad(mod(*x).sum(), inputs)):
         assert grad.shape == t.shape and not grad._is_view()
         assert grad.untyped_storage().nbytes() == t.numel() * t.element_size()
+
+
+def test_fp32_v_off_alignment(dev):
+    """An fp32 v that does not lie on 16 bytes is converted by the copy, as any other."""
+    q, k, v, do = (torch.randn(1, 2, 300, 64, device=dev) for _ in range(4))
+    mod = SparseLinearAttention(64, 0.5).to(dev)
+    off = torch.empty(v.numel() + 1, device=dev)[1:].view_as(v).copy_(v)
+    assert off.is_contiguous() and off.data_ptr() % 16
+    with torch.no_grad():
+        assert torch.equal(mod(q, k, off), mod(q, k, v))
+    grads = []
+    for t in (v, off):
+        x = [q.clone().requires_grad_(True), k.clone().requires_grad_(True), t.detach().requires_grad_(True)]
+        grads.append(torch.autograd.grad(mod(*x), x, do))
+    assert all(torch.equal(a, b) for a, b in zip(*grads))
