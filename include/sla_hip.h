@@ -58,6 +58,7 @@ extern "C" {
 #define SLA_WS_MODULE_FWD 9    /* dtype: that of the inputs */
 #define SLA_WS_LINEAR_BWD_STATES_APART 10 /* linear_workspace of sla_module_bwd_states */
 #define SLA_WS_SAGE_MODULE_FWD 11
+#define SLA_WS_LINEAR_COMPLEMENT_STATES 12 /* `states` of sla_linear_complement_fwd_states */
 
 /* flags of sla_linear_bwd */
 #define SLA_BWD_ACCUMULATE 1   /* dq, dk, dv already hold the sparse branch's gradients: add to them */
@@ -264,6 +265,20 @@ int sla_linear_complement_bwd(const void* q, const void* k, const void* v, const
                               void* dk, void* dv, float* d_weight, float* d_bias, int dtype, int fmap, int B, int H,
                               int L, int D, int BLKQ, int BLKK, int topk, int flags, void* workspace,
                               int64_t workspace_bytes, void* stream);
+
+/* The two calls above with the query blocks' states (SLA_WS_LINEAR_COMPLEMENT_STATES bytes, 16-byte aligned) in a buffer of
+ * the caller's: the forward writes them, the backward of the same q, k, v, lut and sizes reads them instead of forming them
+ * again.  The workspaces are smaller by that many bytes. */
+int sla_linear_complement_fwd_states(const void* q, const void* k, const void* v, const void* lut, int lut_elem_bytes,
+                                     const float* weight, const float* bias, const void* residual, void* out,
+                                     void* states, int dtype, int fmap, int B, int H, int L, int D, int BLKQ, int BLKK,
+                                     int topk, void* workspace, int64_t workspace_bytes, void* stream);
+int sla_linear_complement_bwd_states(const void* q, const void* k, const void* v, const int8_t* sparse_map,
+                                     const void* lut, int lut_elem_bytes, const float* weight, const float* bias,
+                                     const void* d_out, const void* states, void* dq, void* dk, void* dv,
+                                     float* d_weight, float* d_bias, int dtype, int fmap, int B, int H, int L, int D,
+                                     int BLKQ, int BLKK, int topk, int flags, void* workspace, int64_t workspace_bytes,
+                                     void* stream);
 
 /* Linear branch backward.  d_out is the gradient of `out` above.  Writes dq, dk, dv in `dtype`
  * (gradients of the linear branch only; the residual's gradient is d_out itself) and the

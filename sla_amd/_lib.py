@@ -21,7 +21,7 @@ _DTYPE_CODES = {torch.float32: SLA_F32, torch.bfloat16: SLA_BF16, torch.float16:
 FMAP = {"elu": 0, "relu": 1, "softmax": 2}
 (WS_BLOCK_MAP, WS_SPARSE_BWD, WS_LINEAR_FWD, WS_LINEAR_BWD, WS_SAGE_QUANT, WS_LINEAR_COMPLEMENT, WS_SAGE_PREPARE,
  WS_LINEAR_STATES, WS_LINEAR_COMPLEMENT_BWD, WS_MODULE_FWD, WS_LINEAR_BWD_STATES_APART,
- WS_SAGE_MODULE_FWD) = range(12)
+ WS_SAGE_MODULE_FWD, WS_LINEAR_COMPLEMENT_STATES) = range(13)
 BWD_ACCUMULATE, BWD_STATES_READY = 1, 2
 
 ERR_BAD_ARG, ERR_UNSUPPORTED, ERR_LAUNCH, ERR_WORKSPACE = -1, -2, -3, -4
@@ -58,6 +58,10 @@ SIGNATURES = {
     "sla_linear_out_fwd": (_I, [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _I64, _P]),
     "sla_linear_complement_fwd": (_I, [_P, _P, _P, _P, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P, _I64,
                                        _P]),
+    "sla_linear_complement_fwd_states": (_I, [_P, _P, _P, _P, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P,
+                                              _I64, _P]),
+    "sla_linear_complement_bwd_states": (_I, [_P, _P, _P, _P, _P, _I, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I,
+                                              _I, _I, _I, _I, _P, _I64, _P]),
     "sla_linear_complement_bwd": (_I, [_P, _P, _P, _P, _P, _I, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I,
                                        _I, _I, _I, _P, _I64, _P]),
     "sla_linear_bwd": (_I, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P, _I64, _P]),

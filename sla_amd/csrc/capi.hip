@@ -81,7 +81,8 @@ int64_t linear_bwd_workspace_bytes(int BH, int L, int D);
 int64_t sage_quant_workspace_bytes(int BH, int L, int D);
 int64_t sage_prepare_workspace_bytes(int BH, int L, int D);
 int64_t linear_states_bytes(int BH, int L, int D);
-int64_t linear_complement_workspace_bytes(int BH, int L, int D);
+int64_t linear_complement_workspace_bytes(int BH, int L, int D, int BLKQ);
+int64_t linear_complement_states_bytes(int BH, int L, int D, int BLKQ);
 int64_t linear_complement_bwd_workspace_bytes(int BH, int L, int D, int BLKQ);
 int64_t sage_module_workspace_bytes(int B, int H, int L, int D, int topk);
 int64_t linear_bwd_states_apart_bytes(int BH, int L, int D);
@@ -118,7 +119,10 @@ extern "C" int64_t sla_workspace_bytes(int op, int dtype, int B, int H, int L, i
     case SLA_WS_SAGE_PREPARE:
       return sage_prepare_workspace_bytes(BH, L, D);
     case SLA_WS_LINEAR_COMPLEMENT:
-      return linear_complement_workspace_bytes(BH, L, D);
+      return linear_complement_workspace_bytes(BH, L, D, BLKQ == 128 ? 128 : 64);
+    case SLA_WS_LINEAR_COMPLEMENT_STATES:
+      SLA_REQUIRE(BLKQ == 64 || BLKQ == 128, SLA_ERR_UNSUPPORTED, "BLKQ=%d (64 or 128)", BLKQ);
+      return linear_complement_states_bytes(BH, L, D, BLKQ);
     case SLA_WS_LINEAR_COMPLEMENT_BWD:
       SLA_REQUIRE(BLKQ == 64 || BLKQ == 128, SLA_ERR_UNSUPPORTED, "BLKQ=%d (64 or 128)", BLKQ);
       return linear_complement_bwd_workspace_bytes(BH, L, D, BLKQ);

@@ -12,10 +12,13 @@
 // Kernels:
 //   block states : linear_state_partial_kernel with one 64-row slice per workgroup, 16-bit h_j^T, fp32 z_j
 //   totals       : sum_j h_j, sum_j z_j in fp32 (groups of 16 blocks, then the groups)
-//   out          : one workgroup per query block: gathers and subtracts the T selected states from the total
-//                  (the same 32 KB-per-tile gather traffic as the sparse kernel's K/V tiles), rounds H_i^T
-//                  into LDS and runs N^T = H_i^T phi(Q)^T, OUT^T = W Y^T for its rows in the transposed
+//   gather       : H_i, z_i = totals - the T selected states, per query block (H_i rounded); the backward reads them again
+//   out          : N^T = H_i^T phi(Q)^T, OUT^T = W Y^T for the rows of a query block in the transposed
 //                  formulation of the global output kernel.
+// At 12 heads of 16380 rows, head dim 128, 12 of 256 blocks selected, with the gathers inside the kernels of the rows (a
+// workgroup per query or key block, the whole state in 64 fp32 registers per thread, two waves per SIMD): out 236 us,
+// rows 171 us, kv 171 us, and the backward formed the forward's states again (88 us).  With the
+// gathers in a kernel of their own: gather 124 us (twice), out 77 us, rows 110 us, kv 112 us.
 #include "linear_state.h"
 
 namespace sla {
@@ -82,259 +85,263 @@ __global__ __launch_bounds__(256) void complement_total_kernel(const float* __re
   }
 }
 
-// A D x D state held in fp32 registers: thread t of 256 owns the 16-byte chunks t + 256 c of the (row-major, 16-bit)
-// block states, and element t of the z vectors when t < D.
-template <int D>
-static __device__ __forceinline__ void state_from_total(float (&acc)[D * D / 8 / 256][8], float& zacc,
-                                                        const float* __restrict__ total, const float* __restrict__ ztotal,
-                                                        int tid) {
+// Rows' states: `total - sum of the listed block states` for every query block (its look-up row) or, in the backward, for
+// every key block (the query blocks that selected it); 16-bit result, z in fp32.
+//
+// Bound by the L2 traffic of the listed states (32 KB each at D = 128).  Neighbouring lists share most of their entries, so
+// a workgroup walks a run of GATHER_RUN consecutive rows with the state in fp32 registers: the first gathers
+// `total - its list`, a later one only applies the difference of its list against the previous one (adds back what dropped
+// out in that list's order, then subtracts what is new in its own order: results do not depend on scheduling) unless the
+// difference is the longer one.  A workgroup holds a slice of 8 KB of the state: 16 values per thread leave room for six
+// waves per SIMD, and all rows' slices of one head (2 MB at 256 blocks) fit an XCD's L2, which they would not in full; the
+// XCD-aware order therefore has the slice outside the run.  Lists longer than GATHER_TMAX are gathered in full.
+// A list that names every block gives exactly zero by definition, not the rounding residue of two fp32 sums formed in
+// different orders, which the 1e-5 of the divisor would otherwise turn into an arbitrary result.
+constexpr int GATHER_RUN = 8;
+constexpr int GATHER_TMAX = 256;
+
+// The signed difference list between the previous list (`tp` entries) and this one (`tc`), both in LDS:
+// out[0 .. ndrop) = ~j for the blocks j only the previous list names, out[ndrop .. ndrop + nnew) = j for the blocks
+// only this one names.  Returns ndrop + nnew; entries past GATHER_TMAX are not written.  One wave.
+static __device__ __forceinline__ int list_difference(const int* prev, int tp, const int* cur, int tc, int* out, int lane) {
+  int n = 0;
 #pragma unroll
-  for (int c = 0; c < D * D / 8 / 256; ++c) {
-    const int idx = (tid + 256 * c) * 8;
-    const f32x4_t a = *reinterpret_cast<const f32x4_t*>(total + idx);
-    const f32x4_t b = *reinterpret_cast<const f32x4_t*>(total + idx + 4);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      acc[c][e] = a[e];
-      acc[c][4 + e] = b[e];
+  for (int side = 0; side < 2; ++side) {
+    const int *mine = side ? cur : prev, *other = side ? prev : cur;
+    const int nm = side ? tc : tp, no = side ? tp : tc;
+    for (int i0 = 0; i0 < nm; i0 += 64) {
+      bool only = i0 + lane < nm;
+      const int j = only ? mine[i0 + lane] : 0;
+      for (int u = 0; u < no; ++u) only &= other[u] != j;
+      const unsigned long long m = __ballot(only);
+      const int pos = n + __popcll(m & ((1ull << lane) - 1));
+      if (only && pos < GATHER_TMAX) out[pos] = side ? j : ~j;
+      n += __popcll(m);
     }
   }
-  zacc = tid < D ? ztotal[tid] : 0.f;
+  return n;
 }
 
-// Adds or subtracts `count` listed block states, in list order.  `at(i)` is list entry i: a block index j >= 0 means
-// "subtract block j", ~j (negative) means "add block j".  Two listed states are in flight while a third is being
-// applied (the gather is latency-bound: bytes in flight per compute unit set its rate).
-template <typename Tag, int D, typename At>
-static __device__ __forceinline__ void apply_states(float (&acc)[D * D / 8 / 256][8], float& zacc,
-                                                    const uint16_t* __restrict__ blocks, const float* __restrict__ zblocks,
-                                                    int count, At at, int tid) {
+// list: row (head, r) starts `stride` entries after the previous one and has count[r] entries (`fixed` where count is null).
+// 1-D grid over (head, slice, run), 256 threads; thread t owns the 16-byte chunks t and t + 256 of its slice.
+template <typename Tag, int D>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void complement_gather_kernel(const uint16_t* __restrict__ blocks,
+                                                                const float* __restrict__ zblocks,
+                                                                const float* __restrict__ total,
+                                                                const float* __restrict__ ztotal,
+                                                                const void* __restrict__ list, int list64,
+                                                                const int* __restrict__ count, int fixed, int stride,
+                                                                uint16_t* __restrict__ states, float* __restrict__ zstates,
+                                                                int nrows, int nblk, int ntotal) {
   using E = Elem<Tag>;
   constexpr int DD = D * D;
-  constexpr int NCH = DD / 8 / 256;
-  i16x8_t ring[2][NCH];
-  float zring[2] = {0.f, 0.f};
-  float sgn[2] = {0.f, 0.f};
-  auto fetch = [&](int slot, int i) {
-    const int e = at(i);
-    const int nb = e < 0 ? ~e : e;
-    sgn[slot] = e < 0 ? 1.0f : -1.0f;
-    const uint16_t* p = blocks + (size_t)nb * DD;
-#pragma unroll
-    for (int c = 0; c < NCH; ++c) ring[slot][c] = *reinterpret_cast<const i16x8_t*>(p + (tid + 256 * c) * 8);
-    zring[slot] = tid < D ? zblocks[(size_t)nb * D + tid] : 0.f;
+  constexpr int SLICES = DD / 4096;
+  constexpr int BATCH = 4;               // listed states in flight
+  static_assert(DD % 4096 == 0, "slices of 4096 values");
+  __shared__ int sRow[GATHER_RUN][GATHER_TMAX], sDiff[GATHER_RUN][GATHER_TMAX];
+  __shared__ int sLen[GATHER_RUN];       // entries of the row's difference list, -1 where its own list is taken
+  const int logical = xcd_remap(blockIdx.x, gridDim.x, ntotal);
+  if (logical < 0) return;
+  const int runs = (nrows + GATHER_RUN - 1) / GATHER_RUN;
+  const int unit = logical / runs, row0 = (logical - unit * runs) * GATHER_RUN;
+  const int bh = unit / SLICES, slice = unit - bh * SLICES;
+  const int tid = threadIdx.x;
+  const bool has_z = slice == 0 && tid < D;
+  const size_t off = (size_t)slice * 4096 + tid * 8;
+  const uint16_t* hb = blocks + (size_t)bh * nblk * DD + off;
+  const float* zb = zblocks + (size_t)bh * nblk * D + (has_z ? tid : 0);
+  const float* tot = total + (size_t)bh * DD + off;
+
+  auto length = [&](int row) -> int { return count ? count[(size_t)bh * nrows + row] : fixed; };
+  auto entry = [&](int row, int i) -> int {
+    const size_t at = ((size_t)bh * nrows + row) * stride + i;
+    return list64 ? (int)reinterpret_cast<const long long*>(list)[at] : reinterpret_cast<const int*>(list)[at];
   };
-  if (count > 0) fetch(0, 0);
-  if (count > 1) fetch(1, 1);
-  int it = 0;
-  for (; it + 1 < count; it += 2) {       // slot parity is static inside the unrolled pair
-    i16x8_t x[NCH];
+  auto fits = [&](int cnt) { return cnt <= GATHER_TMAX && cnt < nblk; };
+  // all lists of the run, then all differences (a wave takes every fourth)
+  const int steps = min(GATHER_RUN, nrows - row0);
 #pragma unroll
-    for (int c = 0; c < NCH; ++c) x[c] = ring[0][c];
-    const float zx = zring[0], sx = sgn[0];
-    if (it + 2 < count) fetch(0, it + 2);
-#pragma unroll
-    for (int c = 0; c < NCH; ++c)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) acc[c][e] += sx * E::to_float((uint16_t)x[c][e]);
-    zacc += sx * zx;
-#pragma unroll
-    for (int c = 0; c < NCH; ++c) x[c] = ring[1][c];
-    const float zy = zring[1], sy = sgn[1];
-    if (it + 3 < count) fetch(1, it + 3);
-#pragma unroll
-    for (int c = 0; c < NCH; ++c)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) acc[c][e] += sy * E::to_float((uint16_t)x[c][e]);
-    zacc += sy * zy;
+  for (int step = 0; step < GATHER_RUN; ++step) {
+    const int cnt = step < steps ? length(row0 + step) : 0;
+    if (fits(cnt) && tid < cnt) sRow[step][tid] = entry(row0 + step, tid);
   }
-  if (it < count) {
-#pragma unroll
-    for (int c = 0; c < NCH; ++c)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) acc[c][e] += sgn[0] * E::to_float((uint16_t)ring[0][c][e]);
-    zacc += sgn[0] * zring[0];
-  }
-}
-
-// `total - sum of the listed blocks` (list entries are block indices, subtracted in list order).
-// When the list names every block (`count == nblocks`) the difference is exactly zero by definition; it is
-// returned as such instead of as the rounding residue of two fp32 sums formed in different orders, which the
-// 1e-5 of the divisor would otherwise turn into an arbitrary result.
-template <typename Tag, int D, typename At>
-static __device__ __forceinline__ void gather_complement(float (&acc)[D * D / 8 / 256][8], float& zacc,
-                                                         const float* __restrict__ total, const float* __restrict__ ztotal,
-                                                         const uint16_t* __restrict__ blocks, const float* __restrict__ zblocks,
-                                                         int count, int nblocks, At at, int tid) {
-  if (count >= nblocks) {                    // (uniform over the workgroup)
-#pragma unroll
-    for (int c = 0; c < D * D / 8 / 256; ++c)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) acc[c][e] = 0.f;
-    zacc = 0.f;
-    return;
-  }
-  state_from_total<D>(acc, zacc, total, ztotal, tid);
-  apply_states<Tag, D>(acc, zacc, blocks, zblocks, count, at, tid);
-}
-
-// The gathered state, rounded to 16 bit, into an LDS matrix of D rows with row stride STR (same row-major
-// order as the block states in memory).
-template <typename Tag, int D, int STR>
-static __device__ __forceinline__ void park_state(uint16_t* sH, const float (&acc)[D * D / 8 / 256][8], int tid) {
-  using E = Elem<Tag>;
-#pragma unroll
-  for (int c = 0; c < D * D / 8 / 256; ++c) {
-    const int idx = (tid + 256 * c) * 8;
-    const int row = idx / D, col = idx % D;
-    i32x4_t w;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) w[e] = (int)E::pack2(acc[c][2 * e], acc[c][2 * e + 1]);
-    *reinterpret_cast<i32x4_t*>(&sH[row * STR + col]) = w;
-  }
-}
-
-// Look-up rows of neighbouring query blocks share most of their entries, so a workgroup walks a run of COMPL_RUN
-// consecutive query blocks of one head and keeps H_i in fp32 registers: the first block of the run gathers
-// `total - its T selected states`, every later block only applies the difference of its look-up row against the
-// previous one (adds back the states that dropped out, subtracts the new ones).  The difference lists are formed in
-// a fixed order (dropped entries in the previous row's order, then new entries in this row's order), so results do
-// not depend on scheduling.  Rows longer than COMPL_TMAX fall back to the full gather for every block.
-constexpr int COMPL_RUN = 4;
-constexpr int COMPL_TMAX = 256;
-
-// The signed difference list between the previous look-up row (sPrev) and this one (sCur), both `T` entries in LDS:
-// sList[0 .. ndrop) = ~j for the blocks j only the previous row names, sList[ndrop .. ndrop + nnew) = j for the blocks
-// only this row names.  Returns ndrop + nnew.  All 256 threads call it; contains workgroup barriers.
-static __device__ __forceinline__ int lut_difference(const int* sPrev, const int* sCur, int* sList, int (*sCnt)[4], int T,
-                                                     int tid) {
+  __syncthreads();
   const int lane = tid & 63, wave = tid >> 6;
-  bool isdrop = false, isnew = false;
-  int p = 0, c = 0;
-  if (tid < T) {
-    p = sPrev[tid];
-    c = sCur[tid];
-    bool found_p = false, found_c = false;
-    for (int u = 0; u < T; ++u) {
-      found_p |= sCur[u] == p;
-      found_c |= sPrev[u] == c;
+  for (int step = wave; step < steps; step += 4) {
+    int n = -1;
+    if (step) {
+      const int tp = length(row0 + step - 1), tc = length(row0 + step);
+      if (fits(tp) && fits(tc)) {
+        n = list_difference(sRow[step - 1], tp, sRow[step], tc, sDiff[step], lane);
+        if (n >= tc) n = -1;
+      }
     }
-    isdrop = !found_p;
-    isnew = !found_c;
-  }
-  const unsigned long long bd = __ballot(isdrop), bn = __ballot(isnew);
-  if (lane == 0) {
-    sCnt[0][wave] = __popcll(bd);
-    sCnt[1][wave] = __popcll(bn);
+    if (lane == 0) sLen[step] = n;
   }
   __syncthreads();
-  int ndrop = 0, nnew = 0, before_d = 0, before_n = 0;
+
+  float acc[2][8], zacc = 0.f;
+#pragma nounroll
+  for (int step = 0; step < steps; ++step) {
+    const int row = row0 + step;
+    const size_t at_row = (size_t)bh * nrows + row;
+    const int cnt = __builtin_amdgcn_readfirstlane(length(row)), diff = __builtin_amdgcn_readfirstlane(sLen[step]);
+    const bool all = cnt >= nblk, full = diff < 0, kept = fits(cnt);      // (uniform over the workgroup)
+    const int* mine = full ? sRow[step] : sDiff[step];
+    int n = full ? cnt : diff;
+    if (all) {
+      n = 0;
+      zacc = 0.f;
 #pragma unroll
-  for (int w = 0; w < 4; ++w) {
-    before_d += w < wave ? sCnt[0][w] : 0;
-    before_n += w < wave ? sCnt[1][w] : 0;
-    ndrop += sCnt[0][w];
-    nnew += sCnt[1][w];
+      for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[c][e] = 0.f;
+    } else if (full) {
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const f32x4_t a = *reinterpret_cast<const f32x4_t*>(tot + 2048 * c);
+        const f32x4_t b = *reinterpret_cast<const f32x4_t*>(tot + 2048 * c + 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          acc[c][e] = a[e];
+          acc[c][4 + e] = b[e];
+        }
+      }
+      zacc = has_z ? ztotal[(size_t)bh * D + tid] : 0.f;
+    }
+    for (int i0 = 0; i0 < n; i0 += BATCH) {
+      i16x8_t x[BATCH][2];
+      float zx[BATCH], sgn[BATCH];
+#pragma unroll
+      for (int u = 0; u < BATCH; ++u) {
+        if (i0 + u >= n) continue;
+        const int e = __builtin_amdgcn_readfirstlane(kept ? mine[i0 + u] : entry(row, i0 + u));
+        const int j = e < 0 ? ~e : e;
+        sgn[u] = e < 0 ? 1.0f : -1.0f;
+        const uint16_t* p = hb + (size_t)j * DD;
+        x[u][0] = *reinterpret_cast<const i16x8_t*>(p);
+        x[u][1] = *reinterpret_cast<const i16x8_t*>(p + 2048);
+        zx[u] = has_z ? zb[(size_t)j * D] : 0.f;
+      }
+#pragma unroll
+      for (int u = 0; u < BATCH; ++u) {
+        if (i0 + u >= n) continue;
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) acc[c][e] += sgn[u] * E::to_float((uint16_t)x[u][c][e]);
+        zacc += sgn[u] * zx[u];
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      i32x4_t w;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) w[e] = (int)E::pack2(acc[c][2 * e], acc[c][2 * e + 1]);
+      *reinterpret_cast<i32x4_t*>(states + at_row * DD + off + 2048 * c) = w;
+    }
+    if (has_z) zstates[at_row * D + tid] = zacc;
   }
-  const unsigned long long lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  if (isdrop) sList[before_d + __popcll(bd & lt_mask)] = ~p;
-  if (isnew) sList[ndrop + before_n + __popcll(bn & lt_mask)] = c;
-  __syncthreads();
-  return ndrop + nnew;
 }
 
-// 1-D grid over (head, run of COMPL_RUN query blocks) with the XCD-aware remap of the attention kernels: neighbouring
-// runs select mostly the same key blocks, so their state reads hit the same XCD's L2.  256 threads.
+// A row's state on its way from memory into an LDS matrix of D rows with row stride STR.
+template <int D>
+struct StateRows {
+  static constexpr int NCH = D * D / 8 / 256;
+  static_assert(D * D / 8 % 256 == 0, "state does not divide among the threads");
+  i16x8_t x[NCH];
+  float z;
+  __device__ __forceinline__ void fetch(const uint16_t* states, const float* zstates, size_t row, int tid) {
+#pragma unroll
+    for (int c = 0; c < NCH; ++c) x[c] = *reinterpret_cast<const i16x8_t*>(states + row * D * D + (tid + 256 * c) * 8);
+    z = tid < D ? zstates[row * D + tid] : 0.f;
+  }
+  template <int STR>
+  __device__ __forceinline__ void park(uint16_t* sH, int tid) const {
+#pragma unroll
+    for (int c = 0; c < NCH; ++c) {
+      const int idx = (tid + 256 * c) * 8;
+      *reinterpret_cast<i16x8_t*>(&sH[idx / D * STR + idx % D]) = x[c];
+    }
+  }
+};
+
+// 1-D grid over (head, run of OUT_RUN query blocks: the projection weight is converted once per run), XCD-aware order, 256
+// threads; the next block's state is requested beside the products of the present one.
+constexpr int OUT_RUN = 4;
+
 template <typename Tag, int D, int BLKQ>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void complement_out_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ hblk,
-                                                             const float* __restrict__ zblk, const float* __restrict__ hall,
-                                                             const float* __restrict__ zall, const void* __restrict__ lut,
-                                                             int lut64, const float* __restrict__ weight,
-                                                             const float* __restrict__ bias, const uint16_t* __restrict__ residual,
-                                                             uint16_t* __restrict__ out, int L, int Mblk, int N, int topk,
-                                                             int fmap, int total) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void complement_out_kernel(
+    const uint16_t* __restrict__ q, const uint16_t* __restrict__ states, const float* __restrict__ zstates,
+    const float* __restrict__ weight, const float* __restrict__ bias, const uint16_t* __restrict__ residual,
+    uint16_t* __restrict__ out, int L, int Mblk, int fmap, int total) {
   using E = Elem<Tag>;
   constexpr int DC = D / 16;
   constexpr int DT = D / 32;
   constexpr int STR = D + 8;
   constexpr int DD = D * D;
-  constexpr int NCH = DD / 8 / 256;     // 16-byte chunks of the state per thread
-  static_assert(DD / 8 % 256 == 0, "state does not divide among the threads");
   __shared__ __attribute__((aligned(16))) uint16_t sH[D * STR];    // H_i^T [d2][d1]
   __shared__ __attribute__((aligned(16))) uint16_t sW[D * STR];    // W [e][d2 in accumulator slot order]
   __shared__ float sBias[D];
   __shared__ float sZ[D];
-  __shared__ int sPrev[COMPL_TMAX], sCur[COMPL_TMAX], sList[2 * COMPL_TMAX];
-  __shared__ int sCnt[2][4];
 
   const int logical = xcd_remap(blockIdx.x, gridDim.x, total);
   if (logical < 0) return;
-  const int runs = (Mblk + COMPL_RUN - 1) / COMPL_RUN;
-  const int bh = logical / runs, mb0 = (logical - bh * runs) * COMPL_RUN;
+  const int runs = (Mblk + OUT_RUN - 1) / OUT_RUN;
+  const int bh = logical / runs, mb0 = (logical - bh * runs) * OUT_RUN;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int g = lane >> 5, r = lane & 31;
 
+  StateRows<D> h;
+  h.fetch(states, zstates, (size_t)bh * Mblk + mb0, tid);
   // projection weight, 16 bit, columns in accumulator slot order; bias
-  for (int idx = tid; idx < DD; idx += 256) {
-    const int e = idx / D, d = idx % D;
-    sW[e * STR + slot_order_pos(d)] = E::from_float(weight[idx]);
+#pragma unroll
+  for (int i = 0; i < DD / 1024; ++i) {
+    const int idx = (tid + 256 * i) * 4, e = idx / D, d = idx % D;       // (four adjacent columns stay adjacent)
+    const f32x4_t x = *reinterpret_cast<const f32x4_t*>(weight + idx);
+    i32x2_t w;
+    w[0] = (int)E::pack2(x[0], x[1]);
+    w[1] = (int)E::pack2(x[2], x[3]);
+    *reinterpret_cast<i32x2_t*>(&sW[e * STR + slot_order_pos(d)]) = w;
   }
   if (tid < D) sBias[tid] = round16<Tag>(bias[tid]);
 
-  const uint16_t* hb = hblk + (size_t)bh * N * DD;
-  const float* zb = zblk + (size_t)bh * N * D;
-  const bool diffable = topk <= COMPL_TMAX && topk < N;
-  float acc[NCH][8];
-  float zacc;
+  // this wave's 32 queries of a block: rows in operand order
+  i16x8_t xq[DC];
+  auto fetch_q = [&](int mb) {
+    const int qrow = mb * BLKQ + wave * 32 + r;
+    const bool ok = wave < BLKQ / 32 && qrow < L;
+#pragma unroll
+    for (int c = 0; c < DC; ++c) {
+      xq[c] = i16x8_t{0, 0, 0, 0, 0, 0, 0, 0};
+      if (ok) xq[c] = *reinterpret_cast<const i16x8_t*>(q + ((size_t)bh * L + qrow) * D + 16 * c + 8 * g);
+    }
+  };
+  fetch_q(mb0);
+
 #pragma nounroll
-  for (int step = 0; step < COMPL_RUN; ++step) {
+  for (int step = 0; step < OUT_RUN; ++step) {
     const int mb = mb0 + step;
     if (mb >= Mblk) break;
-    const size_t lut_row = ((size_t)bh * Mblk + mb) * topk;
-    auto lut_at = [&](int i) -> int {
-      return lut64 ? (int)reinterpret_cast<const long long*>(lut)[lut_row + i]
-                   : reinterpret_cast<const int*>(lut)[lut_row + i];
-    };
-    // ---- H_i in fp32: total - selected for the first block of the run, the previous block's H plus the difference of
-    // the two look-up rows afterwards ----
-    const bool full = step == 0 || !diffable;          // (uniform over the workgroup)
-    int count = topk;
-    if (full) {
-      if (diffable && tid < topk) sPrev[tid] = lut_at(tid);       // (read after the barriers below)
-      if (topk >= N) {
-        count = 0;                                                // everything selected: exactly zero, see gather_complement
-#pragma unroll
-        for (int c = 0; c < NCH; ++c)
-#pragma unroll
-          for (int e = 0; e < 8; ++e) acc[c][e] = 0.f;
-        zacc = 0.f;
-      } else {
-        state_from_total<D>(acc, zacc, hall + (size_t)bh * DD, zall + (size_t)bh * D, tid);
-      }
-    } else {
-      if (tid < topk) sCur[tid] = lut_at(tid);
-      __syncthreads();
-      count = lut_difference(sPrev, sCur, sList, sCnt, topk, tid);
-      if (tid < topk) sPrev[tid] = sCur[tid];                     // (every thread has passed the barriers of lut_difference)
-    }
-    auto entry_at = [&](int i) -> int { return full ? lut_at(i) : sList[i]; };
-    apply_states<Tag, D>(acc, zacc, hb, zb, count, entry_at, tid);
-    park_state<Tag, D, STR>(sH, acc, tid);
-    if (tid < D) sZ[tid] = round16<Tag>(zacc);
+    h.template park<STR>(sH, tid);
+    if (tid < D) sZ[tid] = round16<Tag>(h.z);
     __syncthreads();
+    const bool more = step + 1 < OUT_RUN && mb + 1 < Mblk;
+    if (more) h.fetch(states, zstates, (size_t)bh * Mblk + mb + 1, tid);
     if (wave < BLKQ / 32) {
       // ---- this wave's 32 queries ----
       const int qrow = mb * BLKQ + wave * 32 + r;
       const bool ok = qrow < L;
       const size_t off = ((size_t)bh * L + qrow) * D;
-      i16x8_t xq[DC];
+      i32x2_t res[DT][4];
 #pragma unroll
-      for (int c = 0; c < DC; ++c) {
-        xq[c] = i16x8_t{0, 0, 0, 0, 0, 0, 0, 0};
-        if (ok) xq[c] = *reinterpret_cast<const i16x8_t*>(q + off + 16 * c + 8 * g);
-      }
+      for (int et = 0; et < DT; ++et)
+#pragma unroll
+        for (int i4 = 0; i4 < 4; ++i4)
+          if (residual && ok) res[et][i4] = *reinterpret_cast<const i32x2_t*>(residual + off + 32 * et + 8 * i4 + 4 * g);
       i16x8_t qf[DC];
       float den = phi_pack_den<Tag, DC>(fmap, xq, qf, [&](int c, int j) { return sZ[16 * c + 8 * g + j]; });
+      if (more) fetch_q(mb + 1);
       den += __shfl_xor(den, 32);
       den = round16<Tag>(1e-5f + round16<Tag>(den));
       const float inv_den = 1.0f / den;
@@ -381,8 +388,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
             for (int j = 0; j < 4; ++j) y[j] = round16<Tag>(oacc[4 * i4 + j] + sBias[e0 + j]);
             if (residual) {
-              const i32x2_t rv = *reinterpret_cast<const i32x2_t*>(residual + off + e0);
-              const uint16_t* rp = reinterpret_cast<const uint16_t*>(&rv);
+              const uint16_t* rp = reinterpret_cast<const uint16_t*>(&res[et][i4]);
 #pragma unroll
               for (int j = 0; j < 4; ++j) y[j] += E::to_float(rp[j]);
             }
@@ -407,25 +413,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 //   G_j = sum_{i : j not in S_i} dH_i = sum_i dH_i - sum_{i in C_j} dH_i  (C_j = query blocks that selected j), gz_j likewise
 //   dc = v G_j^T + gz_j ; dv = c G_j ; dk = phi'(k) dc                     (rows of key block j)
 // Kernels (the totals, the per-block products and dW / db reuse kernels of the forward and of the global backward):
-//   rows : one workgroup per query block: gathers H_i like the forward, then y, dy, dn, dden, da, dq for its rows on the
-//          MFMA in transposed form; writes dq and the row-wise temporaries dn, y (16 bit), dden
-//   kv   : one workgroup per key block: gathers G_j = total - listed dH_i, then dv, dc, dk for its 64 rows
+//   rows   : one workgroup per query block: y, dy, dn, dden, da, dq for its rows from the forward's H_i, z_i on the MFMA in
+//            transposed form; writes dq and the row-wise temporaries dn, y (16 bit), dden
+//   gather : the forward's kernel: G_j, gz_j = total - listed dH_i, dz_i
+//   kv     : one workgroup per key block: dv, dc, dk for its 64 rows
 
 // 1-D grid over (head, query block), XCD-aware order, 256 threads; waves 0 .. BLKQ/32-1 own 32 query rows each.
 template <typename Tag, int D, int BLKQ>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void complement_bwd_rows_kernel(
-    const uint16_t* __restrict__ q, const uint16_t* __restrict__ gout, const uint16_t* __restrict__ hblk,
-    const float* __restrict__ zblk, const float* __restrict__ hall, const float* __restrict__ zall, const void* __restrict__ lut,
-    int lut64, const uint16_t* __restrict__ wt, uint16_t* __restrict__ dq, uint16_t* __restrict__ dn_out,
-    uint16_t* __restrict__ y_out, float* __restrict__ dden_out, int L, int Mblk, int N, int topk, int fmap, int total,
-    int accumulate) {
+    const uint16_t* __restrict__ q, const uint16_t* __restrict__ gout, const uint16_t* __restrict__ states,
+    const float* __restrict__ zstates, const uint16_t* __restrict__ wt, uint16_t* __restrict__ dq, uint16_t* __restrict__ dn_out,
+    uint16_t* __restrict__ y_out, float* __restrict__ dden_out, int L, int Mblk, int fmap, int total, int accumulate) {
   using E = Elem<Tag>;
   constexpr int DC = D / 16;
   constexpr int DT = D / 32;
   constexpr int HSTR = D + 16;           // H_i^T is read row-wise (n^T = H^T a^T) and transposed (da^T = H dn^T)
   constexpr int XSTR = D + 8;
   constexpr int DD = D * D;
-  constexpr int NCH = DD / 8 / 256;
   constexpr int XROWS = D > BLKQ ? D : BLKQ;
   __shared__ __attribute__((aligned(16))) uint16_t sHT[D * HSTR];      // H_i^T [d2][d1]
   // first the waves' staging tiles (q, G in), then W^T [d][e] (A of dy^T = W^T G^T), then staging tiles again (out)
@@ -438,12 +442,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int bh = logical / Mblk, mb = logical - bh * Mblk;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int g = lane >> 5, r = lane & 31;
-  const size_t lut_row = ((size_t)bh * Mblk + mb) * topk;
-  auto lut_at = [&](int i) -> int {
-    return lut64 ? (int)reinterpret_cast<const long long*>(lut)[lut_row + i]
-                 : reinterpret_cast<const int*>(lut)[lut_row + i];
-  };
-
   const int row0 = mb * BLKQ + wave * 32;
   const bool active = wave < BLKQ / 32 && row0 < L;     // (uniform per wave)
   const int rows_valid = min(32, L - row0);
@@ -452,11 +450,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const size_t toff = ((size_t)bh * L + row0) * D;
   uint16_t* const stage = sX + wave * 32 * XSTR;
 
-  // This wave's q and G rows are parked in LDS before the gather (held in registers they would not fit beside its
-  // accumulators): q in the wave's staging tile, G in the still unused H_i^T buffer.
+  // This wave's q and G rows take their operand order through LDS: q in the wave's staging tile, G in the still unused
+  // H_i^T buffer.  The state is on its way meanwhile.
   constexpr bool G_IN_H = (BLKQ / 32) * 32 * XSTR <= D * HSTR;
   uint16_t* const gstage = G_IN_H ? sHT + wave * 32 * XSTR : stage;
   TileRows<D> gt;
+  StateRows<D> h;
+  h.fetch(states, zstates, (size_t)bh * Mblk + mb, tid);
   if (active) {
     TileRows<D> qt;
     qt.fetch(q + toff, rows_valid, lane);
@@ -464,10 +464,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     qt.park(stage, lane);
     if (G_IN_H) gt.park(gstage, lane);
   }
-  float acc[NCH][8];
-  float zacc;
-  gather_complement<Tag, D>(acc, zacc, hall + (size_t)bh * DD, zall + (size_t)bh * D, hblk + (size_t)bh * N * DD,
-                            zblk + (size_t)bh * N * D, topk, N, lut_at, tid);
   // G in B-operand order (d = 16c + 8g + j)
   i16x8_t gf[DC];
   if (active && G_IN_H) {
@@ -475,8 +471,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     for (int c = 0; c < DC; ++c) gf[c] = *reinterpret_cast<const i16x8_t*>(&gstage[r * XSTR + 16 * c + 8 * g]);
   }
   if (G_IN_H) __syncthreads();           // the G tiles have been read: the buffer takes H_i^T
-  park_state<Tag, D, HSTR>(sHT, acc, tid);
-  if (tid < D) sZ[tid] = round16<Tag>(zacc);
+  h.template park<HSTR>(sHT, tid);
+  if (tid < D) sZ[tid] = round16<Tag>(h.z);
   __syncthreads();                       // H_i^T, z_i visible
   // q in B-operand order (d = 16c + 8g + j) -> a = phi(q) as B operand and the divisor; raw q in accumulator order
   // (d = 32t + 8i4 + 4g + j) for the gradient through phi
@@ -614,20 +610,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 }
 
 // 1-D grid over (head, key block), XCD-aware order, 256 threads; waves 0 and 1 own 32 key rows each.
-// dhblk: per query block dH_i^T [d2][d1] (16 bit), dzblk: dz_i (fp32); gall / gzall: their sums over the query blocks.
+// states: per key block G_j^T [d2][d1] (16 bit), zstates: gz_j (fp32).
 template <typename Tag, int D>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void complement_bwd_kv_kernel(
-    const uint16_t* __restrict__ k, const uint16_t* __restrict__ v, const uint16_t* __restrict__ dhblk,
-    const float* __restrict__ dzblk, const float* __restrict__ gall, const float* __restrict__ gzall,
-    const int* __restrict__ list, const int* __restrict__ count, uint16_t* __restrict__ dk, uint16_t* __restrict__ dv, int L,
-    int Mblk, int N, int fmap, int total, int accumulate) {
+    const uint16_t* __restrict__ k, const uint16_t* __restrict__ v, const uint16_t* __restrict__ states,
+    const float* __restrict__ zstates, uint16_t* __restrict__ dk, uint16_t* __restrict__ dv, int L, int N, int fmap, int total,
+    int accumulate) {
   using E = Elem<Tag>;
   constexpr int DC = D / 16;
   constexpr int DT = D / 32;
   constexpr int GSTR = D + 16;           // G_j^T is read row-wise (dv^T = G^T c^T) and transposed (dc^T = G v^T)
   constexpr int SSTR = TileRows<D>::SSTR;
-  constexpr int DD = D * D;
-  constexpr int NCH = DD / 8 / 256;
   __shared__ __attribute__((aligned(16))) uint16_t sGT[D * GSTR];      // G_j^T [d2][d1]
   __shared__ __attribute__((aligned(16))) uint16_t sStage[2][32 * SSTR];
   __shared__ float sGZ[D];
@@ -637,18 +630,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int bh = logical / N, nb = logical - bh * N;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int g = lane >> 5, r = lane & 31;
-  const int* mylist = list + ((size_t)bh * N + nb) * Mblk;
-  auto list_at = [&](int i) -> int { return mylist[i]; };
-
   const int row0 = nb * 64 + wave * 32;
   const bool active = wave < 2 && row0 < L;
   const int rows_valid = min(32, L - row0);
   const size_t toff = ((size_t)bh * L + row0) * D;
-  // this wave's k and v rows are parked in LDS before the gather: k in the wave's staging tile, v in the still
-  // unused G_j^T buffer
+  // this wave's k and v rows take their operand order through LDS: k in the wave's staging tile, v in the still unused
+  // G_j^T buffer; the state is on its way meanwhile
   static_assert(2 * 32 * SSTR <= D * GSTR, "v tiles exceed the state buffer");
   uint16_t* const stage = sStage[wave & 1];
   uint16_t* const vstage = sGT + (wave & 1) * 32 * SSTR;
+  StateRows<D> h;
+  h.fetch(states, zstates, (size_t)bh * N + nb, tid);
   if (active) {
     TileRows<D> kt, vt;
     kt.fetch(k + toff, rows_valid, lane);
@@ -656,18 +648,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     kt.park(stage, lane);
     vt.park(vstage, lane);
   }
-  float acc[NCH][8];
-  float zacc;
-  gather_complement<Tag, D>(acc, zacc, gall + (size_t)bh * DD, gzall + (size_t)bh * D, dhblk + (size_t)bh * Mblk * DD,
-                            dzblk + (size_t)bh * Mblk * D, count[(size_t)bh * N + nb], Mblk, list_at, tid);
   i16x8_t vf[DC];
   if (active) {
 #pragma unroll
     for (int c = 0; c < DC; ++c) vf[c] = *reinterpret_cast<const i16x8_t*>(&vstage[r * SSTR + 16 * c + 8 * g]);
   }
   __syncthreads();                       // the v tiles have been read: the buffer takes G_j^T
-  park_state<Tag, D, GSTR>(sGT, acc, tid);
-  if (tid < D) sGZ[tid] = zacc;
+  h.template park<GSTR>(sGT, tid);
+  if (tid < D) sGZ[tid] = h.z;
   __syncthreads();
   if (!active) return;
 
@@ -750,8 +738,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // ---- host ---------------------------------------------------------------------------------
 struct ComplWs {
   int ngroup;
-  size_t hblk, zblk, hgrp, zgrp, hall, zall, total;
+  size_t hblk, zblk, hgrp, zgrp, hall, zall, total;      // total: without the query blocks' states, which follow
 };
+// The query blocks' states: what the backward reads of the forward.
+struct ComplStates {
+  size_t h, z, total;
+};
+static ComplStates compl_states(int BH, int L, int D, int BLKQ) {
+  const int64_t M = cdiv(L, BLKQ);
+  ComplStates w;
+  w.h = 0;
+  w.z = align_up((int64_t)BH * M * D * D * 2, 256);
+  w.total = w.z + align_up((int64_t)BH * M * D * 4, 256);
+  return w;
+}
+int64_t linear_complement_states_bytes(int BH, int L, int D, int BLKQ) { return (int64_t)compl_states(BH, L, D, BLKQ).total; }
 static ComplWs compl_ws(int BH, int L, int D) {
   const int64_t N = cdiv(L, 64);
   ComplWs w;
@@ -766,30 +767,54 @@ static ComplWs compl_ws(int BH, int L, int D) {
   w.total = off;
   return w;
 }
-int64_t linear_complement_workspace_bytes(int BH, int L, int D) { return (int64_t)compl_ws(BH, L, D).total; }
+int64_t linear_complement_workspace_bytes(int BH, int L, int D, int BLKQ) {
+  return (int64_t)(compl_ws(BH, L, D).total + compl_states(BH, L, D, BLKQ).total);
+}
 
-template <typename Tag, int D, int BLKQ>
-static int complement_impl(const void* q, const void* k, const void* v, const void* lut, int lut64, const float* weight,
-                           const float* bias, const void* residual, void* out, int fmap, int BH, int L, int topk, char* ws,
-                           hipStream_t st) {
+// `total - listed` for nrows rows of every head (see complement_gather_kernel)
+template <typename Tag, int D>
+static void launch_gather(const uint16_t* blocks, const float* zblocks, const float* total, const float* ztotal, const void* list,
+                          int list64, const int* count, int fixed, int stride, uint16_t* states, float* zstates, int BH, int nrows,
+                          int nblk, hipStream_t st) {
+  const int units = BH * (D * D / 4096) * cdiv(nrows, GATHER_RUN);
+  hipLaunchKernelGGL((complement_gather_kernel<Tag, D>), dim3(xcd_grid(units)), dim3(256), 0, st, blocks, zblocks, total, ztotal,
+                     list, list64, count, fixed, stride, states, zstates, nrows, nblk, units);
+}
+
+// Block states, their totals and the query blocks' states.
+template <typename Tag, int D>
+static void complement_states_run(const void* k, const void* v, const void* lut, int lut64, int fmap, int BH, int L, int BLKQ,
+                                  int topk, char* ws, char* states, hipStream_t st) {
   const ComplWs w = compl_ws(BH, L, D);
-  const int N = cdiv(L, 64), Mblk = cdiv(L, BLKQ);
+  const ComplStates s = compl_states(BH, L, D, BLKQ);
+  const int N = cdiv(L, 64);
   uint16_t* hblk = (uint16_t*)(ws + w.hblk);
   float* zblk = (float*)(ws + w.zblk);
   float* hall = (float*)(ws + w.hall);
   float* zall = (float*)(ws + w.zall);
-  hipLaunchKernelGGL((linear_state_partial_kernel<Tag, D, true>), dim3(N, BH), dim3(256), 0, st, (const uint16_t*)k,
-                     (const uint16_t*)v, contiguous_layout(BH, L, D), (void*)hblk, zblk, L, 64, fmap);
   float* hgrp = (float*)(ws + w.hgrp);
   float* zgrp = (float*)(ws + w.zgrp);
+  hipLaunchKernelGGL((linear_state_partial_kernel<Tag, D, true>), dim3(N, BH), dim3(256), 0, st, (const uint16_t*)k,
+                     (const uint16_t*)v, contiguous_layout(BH, L, D), (void*)hblk, zblk, L, 64, fmap, (const float*)nullptr);
   hipLaunchKernelGGL((complement_group_kernel<Tag>), dim3(cdiv(D * D / 8, 256), w.ngroup, BH), dim3(256), 0, st, hblk, zblk,
                      hgrp, zgrp, N, D);
   hipLaunchKernelGGL(complement_total_kernel, dim3(cdiv(D * D, 256), BH), dim3(256), 0, st, hgrp, zgrp, hall, zall, w.ngroup,
                      D);
-  const int total = BH * cdiv(Mblk, COMPL_RUN);
-  hipLaunchKernelGGL((complement_out_kernel<Tag, D, BLKQ>), dim3(xcd_grid(total)), dim3(256), 0, st, (const uint16_t*)q, hblk,
-                     zblk, hall, zall, lut, lut64, weight, bias, (const uint16_t*)residual, (uint16_t*)out, L, Mblk, N, topk,
-                     fmap, total);
+  launch_gather<Tag, D>(hblk, zblk, hall, zall, lut, lut64, nullptr, topk, topk, (uint16_t*)(states + s.h),
+                        (float*)(states + s.z), BH, cdiv(L, BLKQ), N, st);
+}
+
+template <typename Tag, int D, int BLKQ>
+static int complement_impl(const void* q, const void* k, const void* v, const void* lut, int lut64, const float* weight,
+                           const float* bias, const void* residual, void* out, int fmap, int BH, int L, int topk, char* ws,
+                           char* states, hipStream_t st) {
+  const ComplStates s = compl_states(BH, L, D, BLKQ);
+  const int Mblk = cdiv(L, BLKQ);
+  complement_states_run<Tag, D>(k, v, lut, lut64, fmap, BH, L, BLKQ, topk, ws, states, st);
+  const int total = BH * cdiv(Mblk, OUT_RUN);
+  hipLaunchKernelGGL((complement_out_kernel<Tag, D, BLKQ>), dim3(xcd_grid(total)), dim3(256), 0, st, (const uint16_t*)q,
+                     (const uint16_t*)(states + s.h), (const float*)(states + s.z), weight, bias, (const uint16_t*)residual,
+                     (uint16_t*)out, L, Mblk, fmap, total);
   return check_launch("linear_complement_fwd");
 }
 
@@ -822,21 +847,21 @@ static ComplBwdWs compl_bwd_ws(int BH, int L, int D, int BLKQ) {
   return w;
 }
 int64_t linear_complement_bwd_workspace_bytes(int BH, int L, int D, int BLKQ) {
-  return (int64_t)compl_bwd_ws(BH, L, D, BLKQ).total;
+  return (int64_t)(compl_bwd_ws(BH, L, D, BLKQ).total + compl_states(BH, L, D, BLKQ).total);
 }
 
 template <typename Tag, int D, int BLKQ>
 static int complement_bwd_impl(const void* q, const void* k, const void* v, const int8_t* sparse_map, const void* lut, int lut64,
                                const float* weight, const void* d_out, void* dq, void* dk, void* dv, float* d_weight,
                                float* d_bias, int dtype, int fmap, int BH, int L, int topk, int accumulate, char* ws,
-                               hipStream_t st) {
+                               const char* kept, hipStream_t st) {
   const ComplBwdWs w = compl_bwd_ws(BH, L, D, BLKQ);
   const int N = cdiv(L, 64), Mblk = cdiv(L, BLKQ);
   const RowLayout lay = contiguous_layout(BH, L, D);
-  uint16_t* hblk = (uint16_t*)(ws + w.fwd.hblk);
-  float* zblk = (float*)(ws + w.fwd.zblk);
-  float* hall = (float*)(ws + w.fwd.hall);
-  float* zall = (float*)(ws + w.fwd.zall);
+  const ComplStates s = compl_states(BH, L, D, BLKQ);
+  // (the forward's block states are done with when the key blocks' take their place)
+  uint16_t* gst = (uint16_t*)(ws + w.fwd.hblk);
+  float* gzst = (float*)(ws + w.fwd.zblk);
   uint16_t* wt = (uint16_t*)(ws + w.wt);
   uint16_t* dn = (uint16_t*)(ws + w.dn);
   uint16_t* y = (uint16_t*)(ws + w.y);
@@ -847,20 +872,17 @@ static int complement_bwd_impl(const void* q, const void* k, const void* v, cons
   float* gzall = (float*)(ws + w.gzall);
   int* count = (int*)(ws + w.count);
   int* list = (int*)(ws + w.list);
-  // the forward's states again: per key block, then their totals
-  hipLaunchKernelGGL((linear_state_partial_kernel<Tag, D, true>), dim3(N, BH), dim3(256), 0, st, (const uint16_t*)k,
-                     (const uint16_t*)v, lay, (void*)hblk, zblk, L, 64, fmap, (const float*)nullptr);
-  hipLaunchKernelGGL((complement_group_kernel<Tag>), dim3(cdiv(D * D / 8, 256), w.fwd.ngroup, BH), dim3(256), 0, st, hblk, zblk,
-                     (float*)(ws + w.fwd.hgrp), (float*)(ws + w.fwd.zgrp), N, D);
-  hipLaunchKernelGGL(complement_total_kernel, dim3(cdiv(D * D, 256), BH), dim3(256), 0, st, (const float*)(ws + w.fwd.hgrp),
-                     (const float*)(ws + w.fwd.zgrp), hall, zall, w.fwd.ngroup, D);
+  if (!kept) {
+    complement_states_run<Tag, D>(k, v, lut, lut64, fmap, BH, L, BLKQ, topk, ws, ws + w.total, st);
+    kept = ws + w.total;
+  }
   hipLaunchKernelGGL((linear_prep_weight_kernel<Tag>), dim3(cdiv(D * D, 256)), dim3(256), 0, st, weight, wt, D);
   launch_col_lists(sparse_map, list, count, BH, Mblk, N, st);
   // rows: dq and the row temporaries
   const int total_q = BH * Mblk;
   hipLaunchKernelGGL((complement_bwd_rows_kernel<Tag, D, BLKQ>), dim3(xcd_grid(total_q)), dim3(256), 0, st, (const uint16_t*)q,
-                     (const uint16_t*)d_out, hblk, zblk, hall, zall, lut, lut64, wt, (uint16_t*)dq, dn, y, dden, L, Mblk, N, topk,
-                     fmap, total_q, accumulate);
+                     (const uint16_t*)d_out, (const uint16_t*)(kept + s.h), (const float*)(kept + s.z), wt, (uint16_t*)dq, dn, y,
+                     dden, L, Mblk, fmap, total_q, accumulate);
   // per query block dH_i^T = (a_i^T dn_i)^T and dz_i = sum dden a (the state kernel with q, dn in the place of k, v),
   // then their totals
   hipLaunchKernelGGL((linear_state_partial_kernel<Tag, D, true, true>), dim3(Mblk, BH), dim3(256), 0, st, (const uint16_t*)q,
@@ -872,10 +894,10 @@ static int complement_bwd_impl(const void* q, const void* k, const void* v, cons
   // dW, db
   launch_weight_grads(dtype, D, q, dn, d_out, y, dden, BH, L, fmap, ws + w.wg, d_weight, d_bias, st);
   // dk, dv
+  launch_gather<Tag, D>(dhblk, dzblk, gall, gzall, list, 0, count, 0, Mblk, gst, gzst, BH, N, Mblk, st);
   const int total_k = BH * N;
   hipLaunchKernelGGL((complement_bwd_kv_kernel<Tag, D>), dim3(xcd_grid(total_k)), dim3(256), 0, st, (const uint16_t*)k,
-                     (const uint16_t*)v, dhblk, dzblk, gall, gzall, list, count, (uint16_t*)dk, (uint16_t*)dv, L, Mblk, N, fmap,
-                     total_k, accumulate);
+                     (const uint16_t*)v, gst, gzst, (uint16_t*)dk, (uint16_t*)dv, L, N, fmap, total_k, accumulate);
   return check_launch("linear_complement_bwd");
 }
 
@@ -883,11 +905,11 @@ static int complement_bwd_impl(const void* q, const void* k, const void* v, cons
 
 using namespace sla;
 
-extern "C" int sla_linear_complement_bwd(const void* q, const void* k, const void* v, const int8_t* sparse_map, const void* lut,
-                                         int lut_elem_bytes, const float* weight, const float* bias, const void* d_out, void* dq,
-                                         void* dk, void* dv, float* d_weight, float* d_bias, int dtype, int fmap, int B, int H,
-                                         int L, int D, int BLKQ, int BLKK, int topk, int flags, void* workspace,
-                                         int64_t workspace_bytes, void* stream) {
+static int complement_bwd_entry(const void* q, const void* k, const void* v, const int8_t* sparse_map, const void* lut,
+                                int lut_elem_bytes, const float* weight, const float* bias, const void* d_out, void* dq, void* dk,
+                                void* dv, float* d_weight, float* d_bias, int dtype, int fmap, int B, int H, int L, int D, int BLKQ,
+                                int BLKK, int topk, int flags, void* workspace, int64_t workspace_bytes,
+                                const char* states, bool apart, void* stream) {
   int rc = validate_linear(dtype, fmap, B, H, L, D);
   if (rc) return rc;
   rc = validate_attn_shape(dtype, B, H, L, D, BLKQ, BLKK, topk, lut_elem_bytes);
@@ -900,9 +922,11 @@ extern "C" int sla_linear_complement_bwd(const void* q, const void* k, const voi
   SLA_REQUIRE(((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)d_out | (uintptr_t)dq | (uintptr_t)dk | (uintptr_t)dv |
                (uintptr_t)weight | (uintptr_t)workspace) % 16 == 0,
               SLA_ERR_BAD_ARG, "pointers must be 16-byte aligned");
+  SLA_REQUIRE(!apart || (states && (uintptr_t)states % 16 == 0), SLA_ERR_BAD_ARG, "states null or not 16-byte aligned");
   SLA_REQUIRE((int64_t)H * B <= 65535, SLA_ERR_UNSUPPORTED, "B*H exceeds 65535");
   const int BH = B * H;
-  const int64_t need = linear_complement_bwd_workspace_bytes(BH, L, D, BLKQ);
+  const int64_t need = linear_complement_bwd_workspace_bytes(BH, L, D, BLKQ) -
+                       (apart ? linear_complement_states_bytes(BH, L, D, BLKQ) : 0);
   SLA_REQUIRE(workspace_bytes >= need, SLA_ERR_WORKSPACE, "workspace of %lld bytes, need %lld", (long long)workspace_bytes,
               (long long)need);
   hipStream_t st = (hipStream_t)stream;
@@ -912,7 +936,7 @@ extern "C" int sla_linear_complement_bwd(const void* q, const void* k, const voi
 #define SLA_CPLB_CASE(TAG, DD, BQ)                                                                                      \
   if (D == DD && BLKQ == BQ)                                                                                            \
   return complement_bwd_impl<TAG, DD, BQ>(q, k, v, sparse_map, lut, lut64, weight, d_out, dq, dk, dv, d_weight, d_bias, \
-                                          dtype, fmap, BH, L, topk, accumulate, ws, st)
+                                          dtype, fmap, BH, L, topk, accumulate, ws, states, st)
   if (dtype == SLA_BF16) {
     SLA_CPLB_CASE(bf16_tag, 128, 64);
     SLA_CPLB_CASE(bf16_tag, 128, 128);
@@ -929,10 +953,30 @@ extern "C" int sla_linear_complement_bwd(const void* q, const void* k, const voi
   return SLA_ERR_UNSUPPORTED;
 }
 
-extern "C" int sla_linear_complement_fwd(const void* q, const void* k, const void* v, const void* lut, int lut_elem_bytes,
-                                         const float* weight, const float* bias, const void* residual, void* out, int dtype,
-                                         int fmap, int B, int H, int L, int D, int BLKQ, int BLKK, int topk, void* workspace,
+extern "C" int sla_linear_complement_bwd(const void* q, const void* k, const void* v, const int8_t* sparse_map, const void* lut,
+                                         int lut_elem_bytes, const float* weight, const float* bias, const void* d_out, void* dq,
+                                         void* dk, void* dv, float* d_weight, float* d_bias, int dtype, int fmap, int B, int H,
+                                         int L, int D, int BLKQ, int BLKK, int topk, int flags, void* workspace,
                                          int64_t workspace_bytes, void* stream) {
+  return complement_bwd_entry(q, k, v, sparse_map, lut, lut_elem_bytes, weight, bias, d_out, dq, dk, dv, d_weight, d_bias, dtype,
+                              fmap, B, H, L, D, BLKQ, BLKK, topk, flags, workspace, workspace_bytes, nullptr, false, stream);
+}
+
+extern "C" int sla_linear_complement_bwd_states(const void* q, const void* k, const void* v, const int8_t* sparse_map,
+                                                const void* lut, int lut_elem_bytes, const float* weight, const float* bias,
+                                                const void* d_out, const void* states, void* dq, void* dk, void* dv,
+                                                float* d_weight, float* d_bias, int dtype, int fmap, int B, int H, int L, int D,
+                                                int BLKQ, int BLKK, int topk, int flags, void* workspace,
+                                                int64_t workspace_bytes, void* stream) {
+  return complement_bwd_entry(q, k, v, sparse_map, lut, lut_elem_bytes, weight, bias, d_out, dq, dk, dv, d_weight, d_bias, dtype,
+                              fmap, B, H, L, D, BLKQ, BLKK, topk, flags, workspace, workspace_bytes, (const char*)states, true,
+                              stream);
+}
+
+static int complement_fwd_entry(const void* q, const void* k, const void* v, const void* lut, int lut_elem_bytes,
+                                const float* weight, const float* bias, const void* residual, void* out, int dtype, int fmap,
+                                int B, int H, int L, int D, int BLKQ, int BLKK, int topk, void* workspace,
+                                int64_t workspace_bytes, char* states, bool apart, void* stream) {
   int rc = validate_linear(dtype, fmap, B, H, L, D);
   if (rc) return rc;
   rc = validate_attn_shape(dtype, B, H, L, D, BLKQ, BLKK, topk, lut_elem_bytes);
@@ -941,17 +985,20 @@ extern "C" int sla_linear_complement_fwd(const void* q, const void* k, const voi
   SLA_REQUIRE(((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)out | (uintptr_t)residual | (uintptr_t)weight |
                (uintptr_t)workspace) % 16 == 0,
               SLA_ERR_BAD_ARG, "pointers must be 16-byte aligned");
+  SLA_REQUIRE(!apart || (states && (uintptr_t)states % 16 == 0), SLA_ERR_BAD_ARG, "states null or not 16-byte aligned");
   SLA_REQUIRE((int64_t)H * B <= 65535 && cdiv(L, BLKQ) <= 65535 * 32, SLA_ERR_UNSUPPORTED, "grid too large");
   const int BH = B * H;
-  const int64_t need = linear_complement_workspace_bytes(BH, L, D);
+  const int64_t need = linear_complement_workspace_bytes(BH, L, D, BLKQ) -
+                       (apart ? linear_complement_states_bytes(BH, L, D, BLKQ) : 0);
   SLA_REQUIRE(workspace_bytes >= need, SLA_ERR_WORKSPACE, "workspace of %lld bytes, need %lld", (long long)workspace_bytes,
               (long long)need);
   hipStream_t st = (hipStream_t)stream;
   char* ws = (char*)workspace;
+  if (!apart) states = ws + compl_ws(BH, L, D).total;
   const int lut64 = lut_elem_bytes == 8;
 #define SLA_CPL_CASE(TAG, DD, BQ) \
   if (D == DD && BLKQ == BQ)      \
-  return complement_impl<TAG, DD, BQ>(q, k, v, lut, lut64, weight, bias, residual, out, fmap, BH, L, topk, ws, st)
+  return complement_impl<TAG, DD, BQ>(q, k, v, lut, lut64, weight, bias, residual, out, fmap, BH, L, topk, ws, states, st)
   if (dtype == SLA_BF16) {
     SLA_CPL_CASE(bf16_tag, 128, 64);
     SLA_CPL_CASE(bf16_tag, 128, 128);
@@ -966,4 +1013,20 @@ extern "C" int sla_linear_complement_fwd(const void* q, const void* k, const voi
 #undef SLA_CPL_CASE
   set_error("unsupported D=%d BLKQ=%d", D, BLKQ);
   return SLA_ERR_UNSUPPORTED;
+}
+
+extern "C" int sla_linear_complement_fwd(const void* q, const void* k, const void* v, const void* lut, int lut_elem_bytes,
+                                         const float* weight, const float* bias, const void* residual, void* out, int dtype,
+                                         int fmap, int B, int H, int L, int D, int BLKQ, int BLKK, int topk, void* workspace,
+                                         int64_t workspace_bytes, void* stream) {
+  return complement_fwd_entry(q, k, v, lut, lut_elem_bytes, weight, bias, residual, out, dtype, fmap, B, H, L, D, BLKQ, BLKK, topk,
+                              workspace, workspace_bytes, nullptr, false, stream);
+}
+
+extern "C" int sla_linear_complement_fwd_states(const void* q, const void* k, const void* v, const void* lut, int lut_elem_bytes,
+                                                const float* weight, const float* bias, const void* residual, void* out,
+                                                void* states, int dtype, int fmap, int B, int H, int L, int D, int BLKQ,
+                                                int BLKK, int topk, void* workspace, int64_t workspace_bytes, void* stream) {
+  return complement_fwd_entry(q, k, v, lut, lut_elem_bytes, weight, bias, residual, out, dtype, fmap, B, H, L, D, BLKQ, BLKK, topk,
+                              workspace, workspace_bytes, (char*)states, true, stream);
 }

@@ -92,33 +92,43 @@ def linear_out_fwd(q, bias, residual, state_ws, fmap: str):
     return out
 
 
-def linear_complement_fwd(q, k, v, lut, topk, weight, bias, residual, fmap: str, BLKQ: int = 64, BLKK: int = 64):
+def linear_complement_fwd(q, k, v, lut, topk, weight, bias, residual, fmap: str, BLKQ: int = 64, BLKK: int = 64,
+                          keep_states: bool = False):
     """Linear branch over the key blocks each query block did NOT select, + projection + ``residual``.
 
     Opt-in variant (the paper's formulation); the reference module computes the global branch
-    (``core.py:92-96``).  :func:`linear_complement_bwd` is its backward."""
+    (``core.py:92-96``).  :func:`linear_complement_bwd` is its backward.  With ``keep_states`` the result is
+    ``(out, states)``: the query blocks' states, which the backward then need not form again."""
     _lib.require_gpu(q, k, v, lut, weight, bias)
     B, H, L, D = q.shape
     dt = _lib.dtype_code(q.dtype)
     if lut.dtype not in (torch.int32, torch.int64):
         raise TypeError(f"lut must be int32 or int64, got {lut.dtype}")
-    ws = _lib.workspace(_lib.WS_LINEAR_COMPLEMENT, dt, B, H, L, D, BLKQ, BLKK, topk, q.device)
     out = torch.empty_like(q)
-    rc = _lib.load().sla_linear_complement_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), lut.data_ptr(),
-                                               lut.element_size(), weight.data_ptr(), bias.data_ptr(),
-                                               0 if residual is None else residual.data_ptr(), out.data_ptr(), dt,
-                                               _lib.FMAP[fmap], B, H, L, D, BLKQ, BLKK, topk, ws.data_ptr(),
-                                               ws.numel(), _lib.stream_ptr(q.device))
-    _lib.check(rc)
-    return out
+    sizes = (dt, B, H, L, D, BLKQ, BLKK, topk)
+    n = _lib.workspace_bytes(_lib.WS_LINEAR_COMPLEMENT, *sizes)
+    ins = (q.data_ptr(), k.data_ptr(), v.data_ptr(), lut.data_ptr(), lut.element_size(), weight.data_ptr(), bias.data_ptr(),
+           0 if residual is None else residual.data_ptr(), out.data_ptr())
+    tail = (dt, _lib.FMAP[fmap], B, H, L, D, BLKQ, BLKK, topk)
+    if not keep_states:
+        ws = torch.empty(n, dtype=torch.uint8, device=q.device)
+        _lib.check(_lib.load().sla_linear_complement_fwd(*ins, *tail, ws.data_ptr(), n, _lib.stream_ptr(q.device)))
+        return out
+    states = _lib.workspace(_lib.WS_LINEAR_COMPLEMENT_STATES, *sizes, q.device)
+    n -= states.numel()
+    ws = torch.empty(n, dtype=torch.uint8, device=q.device)
+    _lib.check(_lib.load().sla_linear_complement_fwd_states(*ins, states.data_ptr(), *tail, ws.data_ptr(), n,
+                                                            _lib.stream_ptr(q.device)))
+    return out, states
 
 
 def linear_complement_bwd(q, k, v, sparse_map, lut, topk, weight, bias, d_out, fmap: str, BLKQ: int = 64, BLKK: int = 64,
-                          accumulate_into=None):
+                          accumulate_into=None, states=None):
     """Gradients of :func:`linear_complement_fwd` (the linear branch only; the residual's gradient is ``d_out``).
 
     ``sparse_map`` and ``lut`` are the pair ``get_block_map`` returned.  ``accumulate_into=(dq, dk, dv)`` adds to
-    existing gradient tensors instead of allocating new ones.  Returns ``(dq, dk, dv, d_weight, d_bias)``."""
+    existing gradient tensors instead of allocating new ones; ``states`` is what the forward kept.  Returns
+    ``(dq, dk, dv, d_weight, d_bias)``."""
     _lib.require_gpu(q, k, v, sparse_map, lut, weight, bias, d_out)
     B, H, L, D = q.shape
     dt = _lib.dtype_code(q.dtype)
@@ -126,7 +136,10 @@ def linear_complement_bwd(q, k, v, sparse_map, lut, topk, weight, bias, d_out, f
         raise TypeError(f"lut must be int32 or int64, got {lut.dtype}")
     assert sparse_map.dtype == torch.int8 and sparse_map.is_contiguous() and lut.is_contiguous()
     assert q.is_contiguous() and k.is_contiguous() and v.is_contiguous() and d_out.is_contiguous()
-    ws = _lib.workspace(_lib.WS_LINEAR_COMPLEMENT_BWD, dt, B, H, L, D, BLKQ, BLKK, topk, q.device)
+    n = _lib.workspace_bytes(_lib.WS_LINEAR_COMPLEMENT_BWD, dt, B, H, L, D, BLKQ, BLKK, topk)
+    if states is not None:
+        n -= states.numel()
+    ws = torch.empty(n, dtype=torch.uint8, device=q.device)
     if accumulate_into is None:
         dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
         flags = 0
@@ -135,11 +148,14 @@ def linear_complement_bwd(q, k, v, sparse_map, lut, topk, weight, bias, d_out, f
         flags = _lib.BWD_ACCUMULATE
     dw = torch.empty((D, D), dtype=torch.float32, device=q.device)
     db = torch.empty((D,), dtype=torch.float32, device=q.device)
-    rc = _lib.load().sla_linear_complement_bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), sparse_map.data_ptr(),
-                                               lut.data_ptr(), lut.element_size(), weight.data_ptr(), bias.data_ptr(),
-                                               d_out.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
-                                               dw.data_ptr(), db.data_ptr(), dt, _lib.FMAP[fmap], B, H, L, D, BLKQ, BLKK,
-                                               topk, flags, ws.data_ptr(), ws.numel(), _lib.stream_ptr(q.device))
+    ins = (q.data_ptr(), k.data_ptr(), v.data_ptr(), sparse_map.data_ptr(), lut.data_ptr(), lut.element_size(),
+           weight.data_ptr(), bias.data_ptr(), d_out.data_ptr())
+    tail = (dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dw.data_ptr(), db.data_ptr(), dt, _lib.FMAP[fmap], B, H, L, D, BLKQ,
+            BLKK, topk, flags, ws.data_ptr(), n, _lib.stream_ptr(q.device))
+    if states is None:
+        rc = _lib.load().sla_linear_complement_bwd(*ins, *tail)
+    else:
+        rc = _lib.load().sla_linear_complement_bwd_states(*ins, states.data_ptr(), *tail)
     _lib.check(rc)
     return dq, dk, dv, dw, db
 

@@ -197,20 +197,22 @@ class _sla_complement(torch.autograd.Function):
         qk_scale = q.shape[-1] ** -0.5
         weight, bias = weight.contiguous(), bias.contiguous()
         o_s, lse = sparse_attn_fwd(q, k, v, lut, topk, BLKQ, BLKK, qk_scale)
-        out = linear_complement_fwd(q, k, v, lut, topk, weight, bias, o_s, fmap, BLKQ, BLKK)
-        if any(ctx.needs_input_grad[:5]):
-            ctx.save_for_backward(q, k, v, weight, bias, sparse_map, lut, lse, o_s)
+        keep = any(ctx.needs_input_grad[:5])
+        out = linear_complement_fwd(q, k, v, lut, topk, weight, bias, o_s, fmap, BLKQ, BLKK, keep_states=keep)
+        if keep:
+            out, states = out
+            ctx.save_for_backward(q, k, v, weight, bias, sparse_map, lut, lse, o_s, states)
             ctx.cfg = (topk, BLKQ, BLKK, fmap, qk_scale)
         return out
 
     @staticmethod
     def backward(ctx, d_out):
-        q, k, v, weight, bias, sparse_map, lut, lse, o_s = ctx.saved_tensors
+        q, k, v, weight, bias, sparse_map, lut, lse, o_s, states = ctx.saved_tensors
         topk, BLKQ, BLKK, fmap, qk_scale = ctx.cfg
         d_out = d_out.contiguous()
         dq, dk, dv = sparse_attn_bwd(q, k, v, o_s, d_out, lse, sparse_map, lut, topk, BLKQ, BLKK, qk_scale)
         _, _, _, dw, db = linear_complement_bwd(q, k, v, sparse_map, lut, topk, weight, bias, d_out, fmap, BLKQ, BLKK,
-                                                accumulate_into=(dq, dk, dv))
+                                                accumulate_into=(dq, dk, dv), states=states)
         return dq, dk, dv, dw, db, None, None, None, None, None, None
 
 

@@ -143,3 +143,46 @@ def test_everything_selected_leaves_the_bias_and_no_gradient(dev):
         for t in (dq, dk, dv, dw):
             assert int(torch.count_nonzero(t)) == 0
         assert max_abs(db.cpu(), g.float().sum((0, 1, 2)).cpu()) <= 1e-2 * float(g.float().sum((0, 1, 2)).abs().max())
+
+
+def _dense(q, k, v, lut, w, b, BLKQ):
+    """The definition in fp32 with the block states as matrices: H = (all - selected) @ h."""
+    L, D = q.shape[-2:]
+    M, N = lut.shape[2], -(-L // 64)
+    pad = lambda t, n: torch.nn.functional.pad(t, (0, 0, 0, n - L))  # noqa: E731
+    phi = lambda t: torch.nn.functional.elu(t) + 1  # noqa: E731
+    fk, vv = (pad(t, N * 64).unflatten(2, (N, 64)) for t in (phi(k), v))
+    fq = pad(phi(q), M * BLKQ).unflatten(2, (M, BLKQ))
+    rest = 1 - torch.zeros(*lut.shape[:2], M, N).scatter_(3, lut, 1.0)
+    H = (rest @ (fk.transpose(-1, -2) @ vv).flatten(3)).unflatten(3, (D, D))
+    z = rest @ fk.sum(3)
+    o = (fq @ H) / (1e-5 + fq @ z.unsqueeze(-1))
+    return o.flatten(2, 3)[:, :, :L] @ w.T + b
+
+
+@pytest.mark.parametrize("L,D,BLKQ,T", [
+    (300 * 64 - 17, 64, 64, 257),       # lists longer than what the difference of neighbouring lists is formed for
+    (263 * 64, 64, 128, 256),           # the longest it is formed for
+    (9 * 64 + 1, 128, 64, 1), (33 * 64 - 5, 128, 64, 7), (40 * 64, 128, 128, 30), (64, 128, 64, 0)])
+def test_gather_over_runs_of_lists(dev, L, D, BLKQ, T):
+    """Lists of random entries (every one names block 0, so that block's list of query blocks names all of them), runs that end
+    inside a row's eight; the states handed to the backward give the same bits as those it forms."""
+    gen = torch.Generator().manual_seed(L + T)
+    q, k, v, g = (torch.randn(1, 2, L, D, generator=gen).to(torch.bfloat16) for _ in range(4))
+    w, b = make_proj(D)
+    M, N = -(-L // BLKQ), -(-L // 64)
+    order = torch.rand(1, 2, M, N, generator=gen)
+    order[..., 0] = -1.0
+    lut = order.argsort(-1)[..., :T].sort(-1).values.contiguous()
+    m = torch.zeros(1, 2, M, N, dtype=torch.int8).scatter_(3, lut, 1)
+    leaves = [t.float().clone().requires_grad_(True) for t in (q, k, v, w, b)]
+    ref = _dense(*leaves[:3], lut, *leaves[3:], BLKQ)
+    ref.backward(g.float())
+    q, k, v, g, w, b, m, lut = (t.to(dev) for t in (q, k, v, g, w, b, m, lut))
+    out, states = linear_complement_fwd(q, k, v, lut, T, w, b, None, "elu", BLKQ, 64, keep_states=True)
+    assert torch.equal(out, linear_complement_fwd(q, k, v, lut.int(), T, w, b, None, "elu", BLKQ, 64))
+    assert max_abs(out.cpu(), ref.detach()) <= TOL_ABS and cos_sim(out.cpu(), ref.detach()) >= TOL_COS
+    got = linear_complement_bwd(q, k, v, m, lut, T, w, b, g, "elu", BLKQ, 64, states=states)
+    for a, c in zip(got, linear_complement_bwd(q, k, v, m, lut, T, w, b, g, "elu", BLKQ, 64)):
+        assert torch.equal(a, c)
+    _check_grads(got, [t.grad for t in leaves])
