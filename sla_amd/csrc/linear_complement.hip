@@ -18,7 +18,7 @@
 // At 12 heads of 16380 rows, head dim 128, 12 of 256 blocks selected, with the gathers inside the kernels of the rows (a
 // workgroup per query or key block, the whole state in 64 fp32 registers per thread, two waves per SIMD): out 236 us,
 // rows 171 us, kv 171 us, and the backward formed the forward's states again (88 us).  With the
-// gathers in a kernel of their own: gather 124 us (twice), out 77 us, rows 110 us, kv 112 us.
+// gathers in a kernel of their own: gather 101 us (twice), out 77 us, rows 110 us, kv 112 us.
 #include "linear_state.h"
 
 namespace sla {
@@ -88,159 +88,174 @@ __global__ __launch_bounds__(256) void complement_total_kernel(const float* __re
 // Rows' states: `total - sum of the listed block states` for every query block (its look-up row) or, in the backward, for
 // every key block (the query blocks that selected it); 16-bit result, z in fp32.
 //
-// Bound by the L2 traffic of the listed states (32 KB each at D = 128).  Neighbouring lists share most of their entries, so
-// a workgroup walks a run of GATHER_RUN consecutive rows with the state in fp32 registers: the first gathers
-// `total - its list`, a later one only applies the difference of its list against the previous one (adds back what dropped
-// out in that list's order, then subtracts what is new in its own order: results do not depend on scheduling) unless the
-// difference is the longer one.  A workgroup holds a slice of 8 KB of the state: 16 values per thread leave room for six
-// waves per SIMD, and all rows' slices of one head (2 MB at 256 blocks) fit an XCD's L2, which they would not in full; the
-// XCD-aware order therefore has the slice outside the run.  Lists longer than GATHER_TMAX are gathered in full.
-// A list that names every block gives exactly zero by definition, not the rounding residue of two fp32 sums formed in
-// different orders, which the 1e-5 of the divisor would otherwise turn into an arbitrary result.
-constexpr int GATHER_RUN = 8;
+// Bound by the traffic of the listed states (32 KB each at D = 128; a head's do not fit an XCD's L2).  Neighbouring lists
+// share many entries (6.8 of 12 between two rows at 12 heads x 16380 rows), so a workgroup takes GATHER_ROWS consecutive rows
+// at once: it walks the union of their lists and applies every block's state to all the rows that name it.  It holds a slice
+// of 4 KB of the state, 8 values per row and thread.  Applying the difference of a row's list against the previous one's
+// instead (one state in registers, 10.2 of 12 loads per row left) took 124 us there,
+// the union takes 101.
+// Every row's sum runs in the order of the union (the first row's list, what the second adds to it, ...).  Lists longer than
+// GATHER_TMAX are walked by themselves.  A list that names every block gives exactly zero by definition, not the rounding
+// residue of two fp32 sums formed in different orders, which the 1e-5 of the divisor would turn into an arbitrary result.
+constexpr int GATHER_ROWS = 8;
 constexpr int GATHER_TMAX = 256;
 
-// The signed difference list between the previous list (`tp` entries) and this one (`tc`), both in LDS:
-// out[0 .. ndrop) = ~j for the blocks j only the previous list names, out[ndrop .. ndrop + nnew) = j for the blocks
-// only this one names.  Returns ndrop + nnew; entries past GATHER_TMAX are not written.  One wave.
-static __device__ __forceinline__ int list_difference(const int* prev, int tp, const int* cur, int tc, int* out, int lane) {
-  int n = 0;
-#pragma unroll
-  for (int side = 0; side < 2; ++side) {
-    const int *mine = side ? cur : prev, *other = side ? prev : cur;
-    const int nm = side ? tc : tp, no = side ? tp : tc;
-    for (int i0 = 0; i0 < nm; i0 += 64) {
-      bool only = i0 + lane < nm;
-      const int j = only ? mine[i0 + lane] : 0;
-      for (int u = 0; u < no; ++u) only &= other[u] != j;
-      const unsigned long long m = __ballot(only);
-      const int pos = n + __popcll(m & ((1ull << lane) - 1));
-      if (only && pos < GATHER_TMAX) out[pos] = side ? j : ~j;
-      n += __popcll(m);
-    }
-  }
-  return n;
-}
-
 // list: row (head, r) starts `stride` entries after the previous one and has count[r] entries (`fixed` where count is null).
-// 1-D grid over (head, slice, run), 256 threads; thread t owns the 16-byte chunks t and t + 256 of its slice.
+// 1-D grid over (head, slice, group of rows), 256 threads; thread t owns 16-byte chunk t of its slice.
 template <typename Tag, int D>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void complement_gather_kernel(const uint16_t* __restrict__ blocks,
-                                                                const float* __restrict__ zblocks,
-                                                                const float* __restrict__ total,
-                                                                const float* __restrict__ ztotal,
-                                                                const void* __restrict__ list, int list64,
-                                                                const int* __restrict__ count, int fixed, int stride,
-                                                                uint16_t* __restrict__ states, float* __restrict__ zstates,
-                                                                int nrows, int nblk, int ntotal) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void complement_gather_kernel(
+    const uint16_t* __restrict__ blocks, const float* __restrict__ zblocks, const float* __restrict__ total,
+    const float* __restrict__ ztotal, const void* __restrict__ list, int list64, const int* __restrict__ count, int fixed,
+    int stride, uint16_t* __restrict__ states, float* __restrict__ zstates, int nrows, int nblk, int ntotal) {
   using E = Elem<Tag>;
   constexpr int DD = D * D;
-  constexpr int SLICES = DD / 4096;
-  constexpr int BATCH = 4;               // listed states in flight
-  static_assert(DD % 4096 == 0, "slices of 4096 values");
-  __shared__ int sRow[GATHER_RUN][GATHER_TMAX], sDiff[GATHER_RUN][GATHER_TMAX];
-  __shared__ int sLen[GATHER_RUN];       // entries of the row's difference list, -1 where its own list is taken
+  constexpr int SLICES = DD / 2048;
+  constexpr int R = GATHER_ROWS;
+  constexpr int BATCH = 8;               // listed states in flight
+  constexpr int CHUNKS = GATHER_TMAX / 64;
+  static_assert(DD % 2048 == 0, "slices of 2048 values");
+  static_assert(R == 8, "a wave builds the union's share of two rows");
+  __shared__ int sRow[R][GATHER_TMAX];
+  __shared__ uint32_t sUnion[R * GATHER_TMAX];       // block in the lower 24 bits, the rows that name it above
+  __shared__ int sCnt[R * CHUNKS];
   const int logical = xcd_remap(blockIdx.x, gridDim.x, ntotal);
   if (logical < 0) return;
-  const int runs = (nrows + GATHER_RUN - 1) / GATHER_RUN;
-  const int unit = logical / runs, row0 = (logical - unit * runs) * GATHER_RUN;
+  const int groups = (nrows + R - 1) / R;
+  const int unit = logical / groups, row0 = (logical - unit * groups) * R;
   const int bh = unit / SLICES, slice = unit - bh * SLICES;
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const bool has_z = slice == 0 && tid < D;
-  const size_t off = (size_t)slice * 4096 + tid * 8;
+  const size_t off = (size_t)slice * 2048 + tid * 8;
   const uint16_t* hb = blocks + (size_t)bh * nblk * DD + off;
   const float* zb = zblocks + (size_t)bh * nblk * D + (has_z ? tid : 0);
-  const float* tot = total + (size_t)bh * DD + off;
-
-  auto length = [&](int row) -> int { return count ? count[(size_t)bh * nrows + row] : fixed; };
   auto entry = [&](int row, int i) -> int {
     const size_t at = ((size_t)bh * nrows + row) * stride + i;
     return list64 ? (int)reinterpret_cast<const long long*>(list)[at] : reinterpret_cast<const int*>(list)[at];
   };
-  auto fits = [&](int cnt) { return cnt <= GATHER_TMAX && cnt < nblk; };
-  // all lists of the run, then all differences (a wave takes every fourth)
-  const int steps = min(GATHER_RUN, nrows - row0);
+
+  int cnt[R];                            // (uniform over the workgroup)
 #pragma unroll
-  for (int step = 0; step < GATHER_RUN; ++step) {
-    const int cnt = step < steps ? length(row0 + step) : 0;
-    if (fits(cnt) && tid < cnt) sRow[step][tid] = entry(row0 + step, tid);
+  for (int s = 0; s < R; ++s) {
+    cnt[s] = row0 + s < nrows ? __builtin_amdgcn_readfirstlane(count ? count[(size_t)bh * nrows + row0 + s] : fixed) : 0;
+    if (cnt[s] <= GATHER_TMAX && cnt[s] < nblk && tid < cnt[s]) sRow[s][tid] = entry(row0 + s, tid);
+  }
+  auto listed = [&](int s) { return cnt[s] <= GATHER_TMAX && cnt[s] < nblk ? cnt[s] : 0; };     // entries in LDS
+  __syncthreads();
+  // the union: wave w finds which entries of rows w and w + 4 no earlier row names, and who else names them
+  uint32_t word[2][CHUNKS];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int s = wave + 4 * h;
+    int mine = 0;
+#pragma unroll
+    for (int x = 0; x < R; ++x) mine = x == s ? listed(x) : mine;
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) {
+      word[h][c] = 0;
+      if (c * 64 < mine) {
+        const bool has = c * 64 + lane < mine;
+        const int j = has ? sRow[s][c * 64 + lane] : -1;
+        uint32_t rows = has ? 1u << s : 0u;
+#pragma unroll
+        for (int x = 0; x < R; ++x) {
+          bool hit = false;
+          if (x != s)
+            for (int u = 0, n = listed(x); u < n; ++u) hit |= sRow[x][u] == j;
+          rows |= hit ? 1u << x : 0u;
+        }
+        if (has && (rows & ((1u << s) - 1)) == 0) word[h][c] = (uint32_t)j | rows << 24;
+      }
+      const unsigned long long m = __ballot(word[h][c] != 0);
+      if (lane == 0) sCnt[s * CHUNKS + c] = __popcll(m);
+    }
   }
   __syncthreads();
-  const int lane = tid & 63, wave = tid >> 6;
-  for (int step = wave; step < steps; step += 4) {
-    int n = -1;
-    if (step) {
-      const int tp = length(row0 + step - 1), tc = length(row0 + step);
-      if (fits(tp) && fits(tc)) {
-        n = list_difference(sRow[step - 1], tp, sRow[step], tc, sDiff[step], lane);
-        if (n >= tc) n = -1;
-      }
+  int n = 0;
+  {
+    int before[2][CHUNKS];
+    for (int i = 0; i < R * CHUNKS; ++i) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int c = 0; c < CHUNKS; ++c)
+          if (i == (wave + 4 * h) * CHUNKS + c) before[h][c] = n;
+      n += sCnt[i];
     }
-    if (lane == 0) sLen[step] = n;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int c = 0; c < CHUNKS; ++c) {
+        const unsigned long long m = __ballot(word[h][c] != 0);
+        if (word[h][c] != 0) sUnion[before[h][c] + __popcll(m & ((1ull << lane) - 1))] = word[h][c];
+      }
+    n = __builtin_amdgcn_readfirstlane(n);
   }
   __syncthreads();
 
-  float acc[2][8], zacc = 0.f;
-#pragma nounroll
-  for (int step = 0; step < steps; ++step) {
-    const int row = row0 + step;
-    const size_t at_row = (size_t)bh * nrows + row;
-    const int cnt = __builtin_amdgcn_readfirstlane(length(row)), diff = __builtin_amdgcn_readfirstlane(sLen[step]);
-    const bool all = cnt >= nblk, full = diff < 0, kept = fits(cnt);      // (uniform over the workgroup)
-    const int* mine = full ? sRow[step] : sDiff[step];
-    int n = full ? cnt : diff;
-    if (all) {
-      n = 0;
-      zacc = 0.f;
+  float acc[R][8], zacc[R];
+  {
+    const float* tot = total + (size_t)bh * DD + off;
+    const f32x4_t a = *reinterpret_cast<const f32x4_t*>(tot), b = *reinterpret_cast<const f32x4_t*>(tot + 4);
+    const float z = has_z ? ztotal[(size_t)bh * D + tid] : 0.f;
 #pragma unroll
-      for (int c = 0; c < 2; ++c)
+    for (int s = 0; s < R; ++s) {
+      zacc[s] = z;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) acc[c][e] = 0.f;
-    } else if (full) {
-#pragma unroll
-      for (int c = 0; c < 2; ++c) {
-        const f32x4_t a = *reinterpret_cast<const f32x4_t*>(tot + 2048 * c);
-        const f32x4_t b = *reinterpret_cast<const f32x4_t*>(tot + 2048 * c + 4);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          acc[c][e] = a[e];
-          acc[c][4 + e] = b[e];
-        }
+      for (int e = 0; e < 4; ++e) {
+        acc[s][e] = a[e];
+        acc[s][4 + e] = b[e];
       }
-      zacc = has_z ? ztotal[(size_t)bh * D + tid] : 0.f;
     }
+  }
+  // subtracts the blocks of words at(0 .. n-1) from the rows they name
+  auto walk = [&](int n, auto at) {
     for (int i0 = 0; i0 < n; i0 += BATCH) {
-      i16x8_t x[BATCH][2];
-      float zx[BATCH], sgn[BATCH];
+      i16x8_t x[BATCH];
+      float zx[BATCH];
+      uint32_t rows[BATCH];
 #pragma unroll
       for (int u = 0; u < BATCH; ++u) {
+        rows[u] = 0;
         if (i0 + u >= n) continue;
-        const int e = __builtin_amdgcn_readfirstlane(kept ? mine[i0 + u] : entry(row, i0 + u));
-        const int j = e < 0 ? ~e : e;
-        sgn[u] = e < 0 ? 1.0f : -1.0f;
-        const uint16_t* p = hb + (size_t)j * DD;
-        x[u][0] = *reinterpret_cast<const i16x8_t*>(p);
-        x[u][1] = *reinterpret_cast<const i16x8_t*>(p + 2048);
+        const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane((int)at(i0 + u));
+        const uint32_t j = w & 0xffffffu;
+        rows[u] = w >> 24;
+        x[u] = *reinterpret_cast<const i16x8_t*>(hb + (size_t)j * DD);
         zx[u] = has_z ? zb[(size_t)j * D] : 0.f;
       }
 #pragma unroll
       for (int u = 0; u < BATCH; ++u) {
         if (i0 + u >= n) continue;
+        float f[8];
 #pragma unroll
-        for (int c = 0; c < 2; ++c)
+        for (int e = 0; e < 8; ++e) f[e] = E::to_float((uint16_t)x[u][e]);
 #pragma unroll
-          for (int e = 0; e < 8; ++e) acc[c][e] += sgn[u] * E::to_float((uint16_t)x[u][c][e]);
-        zacc += sgn[u] * zx[u];
+        for (int s = 0; s < R; ++s)
+          if (rows[u] >> s & 1) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) acc[s][e] -= f[e];
+            zacc[s] -= zx[u];
+          }
       }
     }
+  };
+  walk(n, [&](int i) { return sUnion[i]; });
+  for (int s = 0; s < R; ++s) {          // lists too long for the union, one at a time
+    int longer = 0;
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      i32x4_t w;
+    for (int x = 0; x < R; ++x) longer = x == s && cnt[x] > GATHER_TMAX && cnt[x] < nblk ? cnt[x] : longer;
+    if (longer) walk(longer, [&](int i) { return (uint32_t)entry(row0 + s, i) | (1u << s) << 24; });
+  }
 #pragma unroll
-      for (int e = 0; e < 4; ++e) w[e] = (int)E::pack2(acc[c][2 * e], acc[c][2 * e + 1]);
-      *reinterpret_cast<i32x4_t*>(states + at_row * DD + off + 2048 * c) = w;
-    }
-    if (has_z) zstates[at_row * D + tid] = zacc;
+  for (int s = 0; s < R; ++s) {
+    if (row0 + s >= nrows) break;
+    const bool all = cnt[s] >= nblk;
+    const size_t at_row = (size_t)bh * nrows + row0 + s;
+    i32x4_t w;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) w[e] = all ? 0 : (int)E::pack2(acc[s][2 * e], acc[s][2 * e + 1]);
+    *reinterpret_cast<i32x4_t*>(states + at_row * DD + off) = w;
+    if (has_z) zstates[at_row * D + tid] = all ? 0.f : zacc[s];
   }
 }
 
@@ -776,7 +791,7 @@ template <typename Tag, int D>
 static void launch_gather(const uint16_t* blocks, const float* zblocks, const float* total, const float* ztotal, const void* list,
                           int list64, const int* count, int fixed, int stride, uint16_t* states, float* zstates, int BH, int nrows,
                           int nblk, hipStream_t st) {
-  const int units = BH * (D * D / 4096) * cdiv(nrows, GATHER_RUN);
+  const int units = BH * (D * D / 2048) * cdiv(nrows, GATHER_ROWS);
   hipLaunchKernelGGL((complement_gather_kernel<Tag, D>), dim3(xcd_grid(units)), dim3(256), 0, st, blocks, zblocks, total, ztotal,
                      list, list64, count, fixed, stride, states, zstates, nrows, nblk, units);
 }

@@ -161,12 +161,12 @@ def _dense(q, k, v, lut, w, b, BLKQ):
 
 
 @pytest.mark.parametrize("L,D,BLKQ,T", [
-    (300 * 64 - 17, 64, 64, 257),       # lists longer than what the difference of neighbouring lists is formed for
-    (263 * 64, 64, 128, 256),           # the longest it is formed for
+    (300 * 64 - 17, 64, 64, 257),       # lists too long for the union of neighbouring lists
+    (263 * 64, 64, 128, 256),           # the longest it takes
     (9 * 64 + 1, 128, 64, 1), (33 * 64 - 5, 128, 64, 7), (40 * 64, 128, 128, 30), (64, 128, 64, 0)])
-def test_gather_over_runs_of_lists(dev, L, D, BLKQ, T):
-    """Lists of random entries (every one names block 0, so that block's list of query blocks names all of them), runs that end
-    inside a row's eight; the states handed to the backward give the same bits as those it forms."""
+def test_gather_over_groups_of_lists(dev, L, D, BLKQ, T):
+    """Lists of random entries (every one names block 0, so that block's list of query blocks names all of them), groups of
+    fewer than eight rows at the end; the states handed to the backward give the same bits as those it forms."""
     gen = torch.Generator().manual_seed(L + T)
     q, k, v, g = (torch.randn(1, 2, L, D, generator=gen).to(torch.bfloat16) for _ in range(4))
     w, b = make_proj(D)
