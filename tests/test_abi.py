@@ -211,3 +211,20 @@ def test_missing_library_fails_loudly(monkeypatch):
     monkeypatch.setattr(_lib, "LIB_PATH", "/nonexistent/libsla_hip.so")
     with pytest.raises(ImportError):
         _lib.load()
+
+
+def test_complement_states_entries_check_their_states():
+    """The variants that keep the query blocks' states ask for the buffer, aligned, and for a workspace smaller by it."""
+    lib = _lib.load()
+    ws = lambda op: lib.sla_workspace_bytes(op, 1, 1, 2, 128, 128, 64, 64, 1)  # noqa: E731
+    states = ws(_lib.WS_LINEAR_COMPLEMENT_STATES)
+    assert states >= 2 * 2 * (128 * 128 * 2 + 128 * 4)
+    fw = lambda st, n: lib.sla_linear_complement_fwd_states(  # noqa: E731
+        FAKE, FAKE, FAKE, FAKE, 8, FAKE, FAKE, None, FAKE, st, 1, 0, 1, 2, 128, 128, 64, 64, 1, FAKE, n, None)
+    bw = lambda st, n: lib.sla_linear_complement_bwd_states(  # noqa: E731
+        FAKE, FAKE, FAKE, FAKE, FAKE, 8, FAKE, FAKE, FAKE, st, FAKE, FAKE, FAKE, FAKE, FAKE, 1, 0, 1, 2, 128, 128, 64, 64, 1, 0,
+        FAKE, n, None)
+    for call, op in ((fw, _lib.WS_LINEAR_COMPLEMENT), (bw, _lib.WS_LINEAR_COMPLEMENT_BWD)):
+        assert call(None, 1 << 30) == _lib.ERR_BAD_ARG
+        assert call(FAKE + 8, 1 << 30) == _lib.ERR_BAD_ARG and "aligned" in _lib.last_error()
+        assert call(FAKE, ws(op) - states - 1) == _lib.ERR_WORKSPACE
