@@ -142,6 +142,16 @@ def require_gpu(*tensors) -> None:
             raise RuntimeError("sla_amd runs on the GPU only: got a tensor on " + str(t.device))
 
 
+def check_operands(x, *others) -> None:
+    """Everything a module's one library call reads through raw pointers lies on one GPU (the call itself cannot tell a host
+    pointer from a device pointer: a projection that was left on the CPU has to be refused here)."""
+    require_gpu(x, *others)
+    dev = x.device
+    for t in others:
+        if t.device != dev:
+            raise RuntimeError(f"sla_amd: operands on {dev} and {t.device}")
+
+
 def _significant_strides(t):
     """Strides of the batch, head and row dimensions; None where the dimension has one entry (its stride is never used)."""
     return tuple(st if n > 1 else None for n, st in zip(t.shape[:3], t.stride()[:3]))

@@ -330,10 +330,11 @@ class SparseLinearAttention(nn.Module):
             q, k, v: (B, H, L, D).
             return_sparsity: also return real_topk / n_key_blocks (reference core.py:102-103).
         """
-        _lib.require_gpu(q, k, v)          # no CPU path: refuse loudly before anything touches a stream
+        proj = self.proj_l
+        weight, bias = proj.weight, proj.bias
+        _lib.check_operands(q, k, v, weight, bias)      # no CPU path: refuse loudly before anything touches a stream
         dtype = q.dtype
-        needs_grad = torch.is_grad_enabled() and any(
-            t.requires_grad for t in (q, k, v, self.proj_l.weight, self.proj_l.bias))
+        needs_grad = torch.is_grad_enabled() and any(t.requires_grad for t in (q, k, v, weight, bias))
         # Inference on activations that are not laid out as (B, H, L, D) -- a (B, L, H, D) tensor or the slices
         # of a packed QKV projection, viewed as (B, H, L, D) -- reads them where they are and writes the output
         # in the same dimension order, instead of copying three tensors in and one out (the reference makes
@@ -348,8 +349,7 @@ class SparseLinearAttention(nn.Module):
 
         if self.linear_mode == "complement":
             return self._forward_complement(q, k, q.to(self.dtype), k.to(self.dtype), v.to(self.dtype), dtype, return_sparsity)
-        weight = self.proj_l.weight.contiguous()
-        bias = self.proj_l.bias.contiguous()
+        weight, bias = weight.contiguous(), bias.contiguous()
         mask = None
         if not (q.dtype == k.dtype == v.dtype and (dtype == self.dtype or (dtype == torch.float32 and v.data_ptr() % 16 == 0))):
             # the mask is built from the inputs in their own dtype (reference core.py:83), the rest works on copies (which the
@@ -382,8 +382,9 @@ class SparseLinearAttention(nn.Module):
             o = res[0] if return_sparsity else res
             o = o.permute(0, 2, 1, 3)
             return (o, res[1]) if return_sparsity else o
-        args = (qkv.contiguous(), self.proj_l.weight.contiguous(), self.proj_l.bias.contiguous(), self.topk, self.BLKQ, self.BLKK,
-                self.feature_map)
+        weight, bias = self.proj_l.weight, self.proj_l.bias
+        _lib.check_operands(qkv, weight, bias)
+        args = (qkv.contiguous(), weight.contiguous(), bias.contiguous(), self.topk, self.BLKQ, self.BLKK, self.feature_map)
         if torch.is_grad_enabled() and any(t.requires_grad for t in args[:3]):
             o = _sla_packed.apply(*args)
         else:

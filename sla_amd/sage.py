@@ -169,7 +169,8 @@ class SageSparseLinearAttention(nn.Module):
 
     @torch.no_grad()
     def forward(self, q, k, v, return_sparsity=False):
-        _lib.require_gpu(q, k, v)          # no CPU path: refuse loudly before anything touches a stream
+        weight, bias = self.proj_l.weight, self.proj_l.bias
+        _lib.check_operands(q, k, v, weight, bias)      # no CPU path: refuse loudly before anything touches a stream
         dtype = q.dtype
         # (B, L, H, D) activations or slices of a packed projection, viewed as (B, H, L, D), are read where they lie
         # and the output is written in the same order; anything else is copied as in the reference (core.py:85-87)
@@ -180,7 +181,7 @@ class SageSparseLinearAttention(nn.Module):
             v = v.contiguous()
         headdim = q.size(-1)
         assert headdim in [64, 128], "headdim should be in [64, 128]. For other headdim, you can use padding and specify the softmax scale."
-        weight, bias = self.proj_l.weight.contiguous(), self.proj_l.bias.contiguous()
+        weight, bias = weight.contiguous(), bias.contiguous()
         if q.dtype == k.dtype == v.dtype == self.dtype:
             # the mask sees the same values as the quantisers: one library call for everything
             o = _sage_module_fwd(q, k, v, weight, bias, self.topk, self.feature_map)

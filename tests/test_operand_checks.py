@@ -1,0 +1,93 @@
+"""What the modules hand to the library as raw pointers is checked before the library is entered.  Runs without a GPU: CPU
+tensors that say they are on one, and a library that records its calls."""
+import pytest
+import torch
+
+from sla_amd import SageSparseLinearAttention, SparseLinearAttention, _lib, module
+
+
+class _OnGpu(torch.Tensor):
+    """A CPU tensor that says it is on the GPU (the stub library never reads it)."""
+
+    is_cuda = property(lambda self: True)
+
+
+class _Library:
+    def __init__(self):
+        self.calls = []
+
+    def __getattr__(self, name):
+        if name == "sla_workspace_bytes":
+            return lambda *a: 4096
+
+        def entry(*args):
+            self.calls.append(name)
+            return 0
+        return entry
+
+
+@pytest.fixture
+def library(monkeypatch):
+    lib = _Library()
+    monkeypatch.setattr(_lib, "load", lambda: lib)
+    monkeypatch.setattr(_lib, "stream_ptr", lambda dev: 0)
+    for mod in ("sla_amd.module", "sla_amd.sage"):
+        monkeypatch.setattr(mod + "._side_stream", lambda dev: None)
+    _lib.workspace_bytes.cache_clear()
+    module._plan.cache_clear()
+    yield lib
+    _lib.workspace_bytes.cache_clear()
+    module._plan.cache_clear()
+
+
+def _operands(*shape, dtype=torch.bfloat16):
+    return [torch.zeros(shape, dtype=dtype).as_subclass(_OnGpu) for _ in range(3)]
+
+
+def _on_gpu(mod):
+    for name in ("weight", "bias"):
+        p = getattr(mod.proj_l, name)
+        del mod.proj_l._parameters[name]
+        setattr(mod.proj_l, name, p.detach().as_subclass(_OnGpu))
+    return mod
+
+
+def _modules():
+    return [SparseLinearAttention(64, 0.5), SparseLinearAttention(64, 0.5, linear_mode="complement"),
+            SageSparseLinearAttention(64, 0.5)]
+
+
+@pytest.mark.parametrize("which", [0, 2])
+def test_accepted_operands_reach_the_library(library, which):
+    mod = _on_gpu(_modules()[which])
+    with torch.no_grad():
+        mod(*_operands(1, 2, 128, 64))
+        if which == 0:
+            mod.forward_packed(torch.zeros(1, 128, 3, 2, 64, dtype=torch.bfloat16).as_subclass(_OnGpu))
+    assert library.calls
+
+
+@pytest.mark.parametrize("grad", [False, True])
+@pytest.mark.parametrize("which", range(3))
+@pytest.mark.parametrize("left", ["weight", "bias"])
+def test_a_projection_left_on_the_cpu_is_refused(library, which, grad, left):
+    mod = _on_gpu(_modules()[which])
+    setattr(mod.proj_l, left, torch.zeros(64, 64) if left == "weight" else torch.zeros(64))
+    ops = _operands(1, 2, 128, 64)
+    if grad:
+        ops = [t.requires_grad_(True) for t in ops]
+    with torch.set_grad_enabled(grad), pytest.raises(RuntimeError, match="on the GPU only"):
+        mod(*ops)
+    if which == 0:
+        packed = torch.zeros(1, 128, 3, 2, 64, dtype=torch.bfloat16).as_subclass(_OnGpu).requires_grad_(grad)
+        with torch.set_grad_enabled(grad), pytest.raises(RuntimeError, match="on the GPU only"):
+            mod.forward_packed(packed)
+    assert not library.calls
+
+
+@pytest.mark.parametrize("grad", [False, True])
+def test_packed_activations_on_the_cpu_are_refused(library, grad):
+    mod = _on_gpu(SparseLinearAttention(64, 0.5))
+    with torch.set_grad_enabled(grad), pytest.raises(RuntimeError, match="on the GPU only"):
+        mod.forward_packed(torch.zeros(1, 128, 3, 2, 64, dtype=torch.bfloat16).requires_grad_(grad))
+    assert not library.calls
