@@ -152,6 +152,19 @@ def check_operands(x, *others) -> None:
             raise RuntimeError(f"sla_amd: operands on {dev} and {t.device}")
 
 
+def check_shapes(q, k, v) -> None:
+    """The library takes every size from q: k and v of another shape would be read past their end."""
+    assert q.dim() == 4 and q.shape == k.shape == v.shape, (
+        f"q, k, v must have the same shape (B, H, L, D), got {tuple(q.shape)}, {tuple(k.shape)}, {tuple(v.shape)}")
+
+
+def check_projection(weight, bias, D) -> None:
+    """``proj_l``'s parameters are read as D x D and D values of 32 bits."""
+    if weight.dtype != torch.float32 or bias.dtype != torch.float32 or weight.shape != (D, D) or bias.shape != (D,):
+        raise ValueError(f"proj_l must be float32 of head dim {D}, got weight {tuple(weight.shape)} {weight.dtype}, bias "
+                         f"{tuple(bias.shape)} {bias.dtype}")
+
+
 def _significant_strides(t):
     """Strides of the batch, head and row dimensions; None where the dimension has one entry (its stride is never used)."""
     return tuple(st if n > 1 else None for n, st in zip(t.shape[:3], t.stride()[:3]))

@@ -333,6 +333,8 @@ class SparseLinearAttention(nn.Module):
         proj = self.proj_l
         weight, bias = proj.weight, proj.bias
         _lib.check_operands(q, k, v, weight, bias)      # no CPU path: refuse loudly before anything touches a stream
+        _lib.check_shapes(q, k, v)
+        _lib.check_projection(weight, bias, q.shape[3])
         dtype = q.dtype
         needs_grad = torch.is_grad_enabled() and any(t.requires_grad for t in (q, k, v, weight, bias))
         # Inference on activations that are not laid out as (B, H, L, D) -- a (B, L, H, D) tensor or the slices
@@ -384,6 +386,7 @@ class SparseLinearAttention(nn.Module):
             return (o, res[1]) if return_sparsity else o
         weight, bias = self.proj_l.weight, self.proj_l.bias
         _lib.check_operands(qkv, weight, bias)
+        _lib.check_projection(weight, bias, qkv.shape[-1])
         args = (qkv.contiguous(), weight.contiguous(), bias.contiguous(), self.topk, self.BLKQ, self.BLKK, self.feature_map)
         if torch.is_grad_enabled() and any(t.requires_grad for t in args[:3]):
             o = _sla_packed.apply(*args)

@@ -171,6 +171,8 @@ class SageSparseLinearAttention(nn.Module):
     def forward(self, q, k, v, return_sparsity=False):
         weight, bias = self.proj_l.weight, self.proj_l.bias
         _lib.check_operands(q, k, v, weight, bias)      # no CPU path: refuse loudly before anything touches a stream
+        _lib.check_shapes(q, k, v)
+        _lib.check_projection(weight, bias, q.shape[3])
         dtype = q.dtype
         # (B, L, H, D) activations or slices of a packed projection, viewed as (B, H, L, D), are read where they lie
         # and the output is written in the same order; anything else is copied as in the reference (core.py:85-87)

@@ -91,3 +91,35 @@ def test_packed_activations_on_the_cpu_are_refused(library, grad):
     with torch.set_grad_enabled(grad), pytest.raises(RuntimeError, match="on the GPU only"):
         mod.forward_packed(torch.zeros(1, 128, 3, 2, 64, dtype=torch.bfloat16).requires_grad_(grad))
     assert not library.calls
+
+
+@pytest.mark.parametrize("grad", [False, True])
+@pytest.mark.parametrize("which", range(3))
+@pytest.mark.parametrize("operand,shape", [(1, (1, 1, 128, 64)), (1, (1, 2, 64, 64)), (2, (1, 1, 128, 64)), (2, (1, 2, 64, 64)),
+                                           (1, (1, 2, 256, 64)), (2, (1, 2, 128, 128))])
+def test_operands_of_different_shapes_are_refused(library, which, grad, operand, shape):
+    """Fewer key heads, shorter or longer keys or values: every size is taken from q, so k and v would be read past their end."""
+    mod = _on_gpu(_modules()[which])
+    ops = _operands(1, 2, 128, 64)
+    ops[operand] = torch.zeros(shape, dtype=torch.bfloat16).as_subclass(_OnGpu)
+    if grad:
+        ops = [t.requires_grad_(True) for t in ops]
+    with torch.set_grad_enabled(grad), pytest.raises(AssertionError, match="same shape"):
+        mod(*ops)
+    assert not library.calls
+
+
+@pytest.mark.parametrize("which", range(3))
+@pytest.mark.parametrize("weight,bias", [(torch.zeros(64, 64, dtype=torch.bfloat16), torch.zeros(64)),
+                                         (torch.zeros(64, 64), torch.zeros(64, dtype=torch.float16)),
+                                         (torch.zeros(128, 128), torch.zeros(128)), (torch.zeros(64, 64), torch.zeros(32))])
+def test_a_projection_of_another_type_or_size_is_refused(library, which, weight, bias):
+    """The kernels read D x D and D values of 32 bits."""
+    mod = _on_gpu(_modules()[which])
+    mod.proj_l.weight, mod.proj_l.bias = weight.as_subclass(_OnGpu), bias.as_subclass(_OnGpu)
+    with torch.no_grad(), pytest.raises(ValueError, match="proj_l"):
+        mod(*_operands(1, 2, 128, 64))
+    if which == 0:
+        with torch.no_grad(), pytest.raises(ValueError, match="proj_l"):
+            mod.forward_packed(torch.zeros(1, 128, 3, 2, 64, dtype=torch.bfloat16).as_subclass(_OnGpu))
+    assert not library.calls
