@@ -384,6 +384,7 @@ class SparseLinearAttention(nn.Module):
             o = res[0] if return_sparsity else res
             o = o.permute(0, 2, 1, 3)
             return (o, res[1]) if return_sparsity else o
+        assert qkv.dim() == 5 and qkv.shape[2] == 3, f"the packed projection is (B, L, 3, H, D), got {tuple(qkv.shape)}"
         weight, bias = self.proj_l.weight, self.proj_l.bias
         _lib.check_operands(qkv, weight, bias)
         _lib.check_projection(weight, bias, qkv.shape[-1])

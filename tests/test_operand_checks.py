@@ -123,3 +123,14 @@ def test_a_projection_of_another_type_or_size_is_refused(library, which, weight,
         with torch.no_grad(), pytest.raises(ValueError, match="proj_l"):
             mod.forward_packed(torch.zeros(1, 128, 3, 2, 64, dtype=torch.bfloat16).as_subclass(_OnGpu))
     assert not library.calls
+
+
+@pytest.mark.parametrize("grad", [False, True])
+@pytest.mark.parametrize("shape", [(1, 128, 4, 2, 64), (1, 128, 2, 2, 64)])
+def test_a_packed_tensor_has_three_parts(library, grad, shape):
+    """Inference, which does not enter the autograd function, refuses what training refuses."""
+    mod = _on_gpu(SparseLinearAttention(shape[-1], 0.5))
+    packed = torch.zeros(shape, dtype=torch.bfloat16).as_subclass(_OnGpu).requires_grad_(grad)
+    with torch.set_grad_enabled(grad), pytest.raises(AssertionError, match="packed"):
+        mod.forward_packed(packed)
+    assert not library.calls
