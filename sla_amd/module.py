@@ -5,6 +5,7 @@ from __future__ import annotations
 import functools
 
 import torch
+import torch.autograd.forward_ad as forward_ad
 import torch.nn as nn
 
 from . import _lib
@@ -145,6 +146,12 @@ def _module_bwd_saved(saved, off, q_ptr, k_ptr, v_ptr, s_qkv, d_out, s_do, weigh
         _lib.stream_ptr(dev), _side_stream(dev))
     _lib.check(rc)
     return dw, db
+
+
+def _through_autograd(*tensors):
+    """Whether a call goes through its autograd function: where a gradient may be asked for, and inside a forward-mode level
+    (the function has no jvp and refuses dual tensors; the library call alone would drop their tangents)."""
+    return torch.is_grad_enabled() and any(t.requires_grad for t in tensors) or forward_ad._current_level >= 0
 
 
 class _sla_core(torch.autograd.Function):
@@ -336,7 +343,7 @@ class SparseLinearAttention(nn.Module):
         _lib.check_shapes(q, k, v)
         _lib.check_projection(weight, bias, q.shape[3])
         dtype = q.dtype
-        needs_grad = torch.is_grad_enabled() and any(t.requires_grad for t in (q, k, v, weight, bias))
+        needs_grad = _through_autograd(q, k, v, weight, bias)
         # Inference on activations that are not laid out as (B, H, L, D) -- a (B, L, H, D) tensor or the slices
         # of a packed QKV projection, viewed as (B, H, L, D) -- reads them where they are and writes the output
         # in the same dimension order, instead of copying three tensors in and one out (the reference makes
@@ -389,7 +396,7 @@ class SparseLinearAttention(nn.Module):
         _lib.check_operands(qkv, weight, bias)
         _lib.check_projection(weight, bias, qkv.shape[-1])
         args = (qkv.contiguous(), weight.contiguous(), bias.contiguous(), self.topk, self.BLKQ, self.BLKK, self.feature_map)
-        if torch.is_grad_enabled() and any(t.requires_grad for t in args[:3]):
+        if _through_autograd(*args[:3]):
             o = _sla_packed.apply(*args)
         else:
             q, k, v = (args[0][:, :, i].permute(0, 2, 1, 3) for i in range(3))

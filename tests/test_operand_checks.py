@@ -2,6 +2,7 @@
 tensors that say they are on one, and a library that records its calls."""
 import pytest
 import torch
+import torch.autograd.forward_ad as forward_ad
 
 from sla_amd import SageSparseLinearAttention, SparseLinearAttention, _lib, module
 
@@ -134,3 +135,20 @@ def test_a_packed_tensor_has_three_parts(library, grad, shape):
     with torch.set_grad_enabled(grad), pytest.raises(AssertionError, match="packed"):
         mod.forward_packed(packed)
     assert not library.calls
+
+
+@pytest.mark.parametrize("no_grad", [False, True])
+@pytest.mark.parametrize("packed", [False, True])
+def test_forward_mode_tangents_are_refused(library, monkeypatch, packed, no_grad):
+    """There is no jvp: dual inputs raise as with any such autograd function, also where nothing asks for a gradient, instead
+    of giving an output without its tangent."""
+    monkeypatch.setattr(_lib, "require_gpu", lambda *t: None)
+    mod = SparseLinearAttention(64, 0.5).requires_grad_(False)
+    shape = (1, 128, 3, 2, 64) if packed else (1, 2, 128, 64)
+    x, y, dx = (torch.randn(shape).bfloat16() for _ in range(3))
+    with torch.set_grad_enabled(not no_grad), forward_ad.dual_level():
+        dual = forward_ad.make_dual(x, dx)
+        with pytest.raises(NotImplementedError, match="jvp"):
+            mod.forward_packed(dual) if packed else mod(dual, y, y)
+        out = mod.forward_packed(x) if packed else mod(x, y, y)       # (no tangent: nothing to lose)
+    assert out.shape == ((1, 128, 2, 64) if packed else shape)
