@@ -149,9 +149,11 @@ def _module_bwd_saved(saved, off, q_ptr, k_ptr, v_ptr, s_qkv, d_out, s_do, weigh
 
 
 def _through_autograd(*tensors):
-    """Whether a call goes through its autograd function: where a gradient may be asked for, and inside a forward-mode level
-    (the function has no jvp and refuses dual tensors; the library call alone would drop their tangents)."""
-    return torch.is_grad_enabled() and any(t.requires_grad for t in tensors) or forward_ad._current_level >= 0
+    """Whether a call goes through its autograd function: where a gradient may be asked for, inside a forward-mode level
+    (the function has no jvp and refuses dual tensors; the library call alone would drop their tangents), and under a trace
+    (which records the function; of the library call alone it would record the allocations)."""
+    return (torch.is_grad_enabled() and any(t.requires_grad for t in tensors) or forward_ad._current_level >= 0
+            or torch.jit.is_tracing())
 
 
 class _sla_core(torch.autograd.Function):

@@ -152,3 +152,15 @@ def test_forward_mode_tangents_are_refused(library, monkeypatch, packed, no_grad
             mod.forward_packed(dual) if packed else mod(dual, y, y)
         out = mod.forward_packed(x) if packed else mod(x, y, y)       # (no tangent: nothing to lose)
     assert out.shape == ((1, 128, 2, 64) if packed else shape)
+
+
+@pytest.mark.parametrize("packed", [False, True])
+def test_a_trace_records_the_operator(library, monkeypatch, packed):
+    """A traced inference call runs the library again; recorded below the operator it would be its uninitialised buffers."""
+    monkeypatch.setattr(_lib, "require_gpu", lambda *t: None)
+    mod = SparseLinearAttention(64, 0.5).requires_grad_(False)
+    x = torch.randn((1, 128, 3, 2, 64) if packed else (1, 2, 128, 64)).bfloat16()
+    traced = torch.jit.trace(lambda x: mod.forward_packed(x) if packed else mod(x, x, x), (x,), check_trace=False)
+    library.calls.clear()
+    traced(x)
+    assert library.calls == ["sla_module_fwd"]
