@@ -89,8 +89,10 @@ int sla_block_map_fwd(const void* q, const void* k, int dtype, int B, int H, int
 /* sla_block_map_fwd for callers that cannot allocate device memory and have no workspace to lend (code under HIP
  * graph capture, serving loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  Same kernels
  * and results as sla_block_map_fwd; the workspace is a fixed array of SLA_STATIC_SCRATCH_BYTES in device memory that
- * every GPU the library runs on holds until the process ends.  Problems whose sla_workspace_bytes(SLA_WS_BLOCK_MAP,
- * ...) exceeds that size are refused with SLA_ERR_WORKSPACE (B1 H12 L32760 D128 64/64 in bf16 needs 12.7 MB and fits).
+ * every GPU the library runs on holds until the process ends.  Problems that need more are refused with
+ * SLA_ERR_WORKSPACE (B1 H12 L32760 D128 64/64 in bf16 needs 12.7 MB and fits).  Where whole tiles of block means do not
+ * fit (many short heads, for which sla_workspace_bytes(SLA_WS_BLOCK_MAP, ...) counts mostly padding) the means lie as
+ * rows: the same results, and the same holds for sla_block_map_fwd with a smaller workspace.
  * Calls no hipMalloc / hipFree.  The first call on a GPU looks up the array's device address (make it once outside a
  * graph capture); the GPU that `stream` belongs to must be the current device.  All calls on one GPU share the array:
  * calls that overlap in time on one GPU (different streams) race; nothing in it needs clearing between calls. */

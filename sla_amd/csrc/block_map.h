@@ -4,9 +4,13 @@
 
 namespace sla {
 
-// 16-bit dtypes, head dim 64 or 128: the means are written in the order the matrix products of the scores read them; other
-// dtypes and head dims take rows.
+// 16-bit dtypes, head dim 64 or 128: the means are written in the order the matrix products of the scores read them, in whole
+// tiles of 32 blocks per head; other dtypes and head dims take rows, and so does a workspace with no room for the tiles.
 static inline int score_takes_tiled(int dtype, int D) { return dtype != SLA_F32 && (D == 64 || D == 128); }
+
+// Rows of at most this many key blocks are scored and selected from in one launch (block_map.hip), the scores never in memory.
+constexpr int SELECT_FUSED_N = 128;
+static inline bool scores_in_memory(int N, int D) { return N > SELECT_FUSED_N || (D != 64 && D != 128); }
 
 // Operand order: tiles of 32 blocks; per tile and 16 columns a fragment of 64 lanes x 8 elements, lane (r, h) = (block % 32,
 // column % 2), element j = columns 16 c + 2 j + h: what lane r + 32 h feeds the 32x32x2 product chain, two columns a step.

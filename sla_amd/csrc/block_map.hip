@@ -316,22 +316,38 @@ __global__ __launch_bounds__(256) void score_kernel(const typename IO::raw* __re
 // product of two 16-bit values is exact in fp32, so fused or not makes no difference; values whose products fall
 // into the fp32 subnormal range aside), at twice the rate of the vector ALU.
 // The operands arrive in the order the products read them (tiled_pos, written by the pooling kernels): a fragment is one
-// coalesced load, straight into registers.
-template <typename IO, int D>
+// coalesced load, straight into registers.  TILED = false: the means lie as rows (a workspace with no room for whole tiles);
+// a lane then reads all columns of its block and keeps the odd or the even ones.  The same bits.
+template <typename IO, int D, bool TILED>
 struct ScoreFrags {
   static constexpr int NC = D / 16;              // fragments (16 d of 32 blocks) per tile
   i32x4_t w[NC];
   __device__ __forceinline__ void load(const typename IO::raw* p, int bh, int nblk, int tile, int lane) {
-    const i16x8_t* t = reinterpret_cast<const i16x8_t*>(p + tiled_head(bh, nblk, D)) + (size_t)tile * (NC * 64) + lane;
+    if constexpr (TILED) {
+      const i16x8_t* t = reinterpret_cast<const i16x8_t*>(p + tiled_head(bh, nblk, D)) + (size_t)tile * (NC * 64) + lane;
 #pragma unroll
-    for (int c = 0; c < NC; ++c) w[c] = __builtin_bit_cast(i32x4_t, t[c * 64]);
+      for (int c = 0; c < NC; ++c) w[c] = __builtin_bit_cast(i32x4_t, t[c * 64]);
+    } else {
+      const int blk = min(32 * tile + (lane & 31), nblk - 1);      // (blocks past the end: scores nobody looks at)
+      const int sh = 16 * (lane >> 5);
+      const i32x4_t* t = reinterpret_cast<const i32x4_t*>(p + ((size_t)bh * nblk + blk) * D);
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        const i32x4_t a = t[2 * c], b = t[2 * c + 1];
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+          const uint32_t lo = (uint32_t)(x < 2 ? a[2 * x] : b[2 * x - 4]), hi = (uint32_t)(x < 2 ? a[2 * x + 1] : b[2 * x - 3]);
+          w[c][x] = (int)(((lo >> sh) & 0xffffu) | (hi >> sh) << 16);
+        }
+      }
+    }
   }
   __device__ __forceinline__ float at(int c, int j) const {      // column 16 c + 2 j + lane / 32 of the lane's block
     return IO::ld((typename IO::raw)((uint32_t)w[c][j >> 1] >> (16 * (j & 1))));
   }
 };
-template <typename IO, int D>
-static __device__ __forceinline__ f32x16_t score_tile(const ScoreFrags<IO, D>& a, const ScoreFrags<IO, D>& b) {
+template <typename IO, int D, bool TILED>
+static __device__ __forceinline__ f32x16_t score_tile(const ScoreFrags<IO, D, TILED>& a, const ScoreFrags<IO, D, TILED>& b) {
   __builtin_amdgcn_sched_barrier(0);             // (every load of both tiles first)
   f32x16_t acc;
 #pragma unroll
@@ -346,7 +362,7 @@ static __device__ __forceinline__ f32x16_t score_tile(const ScoreFrags<IO, D>& a
 // 64 x 64 scores per workgroup, one wave per 32 x 32 part; the rounded scores go through LDS and leave in 128-byte runs.
 // Bound by the fp32 matrix rate (40 heads x 1182 x 1182: 91 us at the nominal rate); with both operand tiles through LDS
 // 158 us, now 140.
-template <typename IO, int D>
+template <typename IO, int D, bool TILED>
 __global__ __launch_bounds__(256) void score_mfma_kernel(const typename IO::raw* __restrict__ pq,
                                                          const typename IO::raw* __restrict__ pk,
                                                          typename IO::raw* __restrict__ score, int M, int N) {
@@ -358,10 +374,10 @@ __global__ __launch_bounds__(256) void score_mfma_kernel(const typename IO::raw*
   const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
   const int wm = wave >> 1, wn = wave & 1;
   if (m0 + 32 * wm < M && n0 + 32 * wn < N) {
-    ScoreFrags<IO, D> a, b;
+    ScoreFrags<IO, D, TILED> a, b;
     a.load(pq, bh, M, (m0 >> 5) + wm, lane);
     b.load(pk, bh, N, (n0 >> 5) + wn, lane);
-    const f32x16_t acc = score_tile<IO, D>(a, b);
+    const f32x16_t acc = score_tile<IO, D, TILED>(a, b);
 #pragma unroll
     for (int i = 0; i < 16; ++i) sm[(wm * 32 + 8 * (i >> 2) + (i & 3) + 4 * h) * OS + wn * 32 + r] = IO::st(acc[i]);
   }
@@ -388,11 +404,16 @@ static void launch_score(const typename IO::raw* pq, const typename IO::raw* pk,
                          int N, int D, hipStream_t st) {
   const dim3 grid(cdiv(N, 64), cdiv(M, 64), BH);
   if constexpr (sizeof(typename IO::raw) == 2) {
-    if (tiled) {
-      if (D == 128) hipLaunchKernelGGL((score_mfma_kernel<IO, 128>), grid, dim3(256), 0, st, pq, pk, score, M, N);
-      else hipLaunchKernelGGL((score_mfma_kernel<IO, 64>), grid, dim3(256), 0, st, pq, pk, score, M, N);
-      return;
-    }
+#define SLA_SCORE_CASE(DD, TILED)                                                                                  \
+  if (D == DD && (tiled != 0) == TILED) {                                                                          \
+    hipLaunchKernelGGL((score_mfma_kernel<IO, DD, TILED>), grid, dim3(256), 0, st, pq, pk, score, M, N);            \
+    return;                                                                                                        \
+  }
+    SLA_SCORE_CASE(128, true)
+    SLA_SCORE_CASE(64, true)
+    SLA_SCORE_CASE(128, false)
+    SLA_SCORE_CASE(64, false)
+#undef SLA_SCORE_CASE
   }
   if (D % 32 == 0)
     hipLaunchKernelGGL((score_kernel<IO, true>), grid, dim3(256), 0, st, pq, pk, score, M, N, D);
@@ -723,8 +744,7 @@ __global__ __launch_bounds__(256) void topk_kernel(const typename IO::raw* __res
 // rounded, and then select for four rows each.  The scores never go to memory and a launch is saved: mask builder of 2
 // heads x 1024 x 64 in fp32 25.3 -> 19.6 us, of 32 x 7813 x 64 38.1 -> 35.0.  With longer rows the two kernels, spread over more
 // workgroups, are as fast or faster (12 heads x 9360 x 128, 128-row query blocks: 36.5 us against 39.0; 2 x 75600: 62 against 77).
-constexpr int SELECT_FUSED_N = 128;
-template <typename IO, int D>
+template <typename IO, int D, bool TILED>
 __global__ __launch_bounds__(512) void select_kernel(const typename IO::raw* __restrict__ pq, const typename IO::raw* __restrict__ pk,
                                                      int8_t* __restrict__ sparse_map, void* __restrict__ lut, int lut64, int M,
                                                      int N, int T) {
@@ -739,10 +759,10 @@ __global__ __launch_bounds__(512) void select_kernel(const typename IO::raw* __r
   const int r = lane & 31, h = lane >> 5;
   if constexpr (EB == 2) {
     if (wave * 32 < N) {                    // (at most four tiles)
-      ScoreFrags<IO, D> a, b;
+      ScoreFrags<IO, D, TILED> a, b;
       a.load(pq, bh, M, blockIdx.x, lane);
       b.load(pk, bh, N, wave, lane);
-      const f32x16_t acc = score_tile<IO, D>(a, b);
+      const f32x16_t acc = score_tile<IO, D, TILED>(a, b);
 #pragma unroll
       for (int i = 0; i < 16; ++i) ss[(8 * (i >> 2) + (i & 3) + 4 * h) * OS + 32 * wave + r] = IO::st(acc[i]);
     }
@@ -816,12 +836,18 @@ static void launch_topk(const typename IO::raw* score, int8_t* sparse_map, void*
 template <typename IO>
 static void launch_select(const typename IO::raw* pq, const typename IO::raw* pk, int tiled, typename IO::raw* score,
                           int8_t* sparse_map, void* lut, int lut64, int BH, int M, int N, int D, int T, hipStream_t st) {
-  if (N <= SELECT_FUSED_N && (D == 64 || D == 128)) {
+  if (!scores_in_memory(N, D)) {
     const dim3 grid(cdiv(M, 32), BH);
-    if (D == 128)
-      hipLaunchKernelGGL((select_kernel<IO, 128>), grid, dim3(512), 0, st, pq, pk, sparse_map, lut, lut64, M, N, T);
-    else
-      hipLaunchKernelGGL((select_kernel<IO, 64>), grid, dim3(512), 0, st, pq, pk, sparse_map, lut, lut64, M, N, T);
+#define SLA_SELECT_CASE(DD, TILED)                                                                                             \
+  if (D == DD && (tiled != 0) == TILED)                                                                                        \
+    hipLaunchKernelGGL((select_kernel<IO, DD, TILED>), grid, dim3(512), 0, st, pq, pk, sparse_map, lut, lut64, M, N, T);
+    if constexpr (sizeof(typename IO::raw) == 2) {
+      SLA_SELECT_CASE(128, true)
+      SLA_SELECT_CASE(64, true)
+    }
+    SLA_SELECT_CASE(128, false)
+    SLA_SELECT_CASE(64, false)
+#undef SLA_SELECT_CASE
     return;
   }
   launch_score<IO>(pq, pk, tiled, score, BH, M, N, D, st);
@@ -832,24 +858,29 @@ struct MapWs {
   size_t chunk_sums, group_sums, colmean, pq, pk, score, total;
 };
 
-static MapWs map_ws(int dtype, int BH, int L, int D, int BLKQ, int BLKK) {
+// tiled: the block means in whole tiles of 32 blocks per head; otherwise as rows
+static MapWs map_ws(int dtype, int BH, int L, int D, int BLKQ, int BLKK, bool tiled) {
   const int64_t M = cdiv(L, BLKQ), N = cdiv(L, BLKK), nchunk = cdiv(L, KMEAN_CHUNK);
+  const int unit = tiled ? 32 : 1;
   const int64_t eb = elem_bytes(dtype);
   MapWs w;
   size_t off = 0;
   w.chunk_sums = off; off += align_up((int64_t)BH * nchunk * D * 4, 256);
   w.group_sums = off; off += align_up((int64_t)BH * cdiv((int)nchunk, KMEAN_GROUP) * D * 4, 256);
   w.colmean = off;    off += align_up((int64_t)BH * D * eb, 256);
-  // (whole tiles of 32 rows per head, as the score kernels read them)
-  w.pq = off;         off += align_up((int64_t)BH * align_up(M, 32) * D * eb, 256);
-  w.pk = off;         off += align_up((int64_t)BH * align_up(N, 32) * D * eb, 256);
-  w.score = off;      off += align_up((int64_t)BH * M * N * eb, 256);
+  w.pq = off;         off += align_up((int64_t)BH * align_up(M, unit) * D * eb, 256);
+  w.pk = off;         off += align_up((int64_t)BH * align_up(N, unit) * D * eb, 256);
+  w.score = off;      off += scores_in_memory((int)N, D) ? align_up((int64_t)BH * M * N * eb, 256) : 0;
   w.total = off;
   return w;
 }
 
 int64_t block_map_workspace_bytes(int dtype, int BH, int L, int D, int BLKQ, int BLKK) {
-  return (int64_t)map_ws(dtype, BH, L, D, BLKQ, BLKK).total;
+  return (int64_t)map_ws(dtype, BH, L, D, BLKQ, BLKK, score_takes_tiled(dtype, D)).total;
+}
+// What a call can make do with: many short heads are mostly padding in tiles (1024 heads of 640 x 128: 21.0 MiB against 10.3).
+static int64_t block_map_least_bytes(int dtype, int BH, int L, int D, int BLKQ, int BLKK) {
+  return (int64_t)map_ws(dtype, BH, L, D, BLKQ, BLKK, false).total;
 }
 
 static int validate_pool(int dtype, int BH, int L, int D, int BLK) {
@@ -896,15 +927,15 @@ static void launch_k_colmean_t(const void* k, const RowLayout& lay, int BH, int 
 
 template <typename IO>
 static int block_map_impl(const void* q, const void* k, const RowLayout& lay, int dtype, int BH, int L, int D, int BLKQ,
-                          int BLKK, int topk, char* ws, int8_t* sparse_map, void* lut, int lut64, hipStream_t st) {
-  const MapWs w = map_ws(dtype, BH, L, D, BLKQ, BLKK);
+                          int BLKK, int topk, char* ws, bool tiled, int8_t* sparse_map, void* lut, int lut64,
+                          hipStream_t st) {
+  const MapWs w = map_ws(dtype, BH, L, D, BLKQ, BLKK, tiled);
   const int M = cdiv(L, BLKQ), N = cdiv(L, BLKK);
   float* chunk_sums = (float*)(ws + w.chunk_sums);
   typename IO::raw* colmean = (typename IO::raw*)(ws + w.colmean);
   typename IO::raw* pq = (typename IO::raw*)(ws + w.pq);
   typename IO::raw* pk = (typename IO::raw*)(ws + w.pk);
   typename IO::raw* score = (typename IO::raw*)(ws + w.score);
-  const int tiled = score_takes_tiled(dtype, D);
   {
     // k chunk sums and q block means share one launch
     const int nchunk = cdiv(L, KMEAN_CHUNK);
@@ -976,9 +1007,11 @@ int block_map_entry(const void* q, const void* k, const int64_t* strides, int dt
   SLA_REQUIRE(q && k && workspace && (sparse_map || !want_map) && (lut || topk == 0), SLA_ERR_BAD_ARG, "null pointer");
   SLA_REQUIRE(((uintptr_t)q | (uintptr_t)k | (uintptr_t)workspace | (uintptr_t)lut) % 16 == 0, SLA_ERR_BAD_ARG,
               "pointers must be 16-byte aligned");
-  const int64_t need = block_map_workspace_bytes(dtype, BH, L, D, BLKQ, BLKK);
+  const int64_t need = block_map_least_bytes(dtype, BH, L, D, BLKQ, BLKK);
   SLA_REQUIRE(workspace_bytes >= need, SLA_ERR_WORKSPACE, "workspace of %lld bytes, need %lld", (long long)workspace_bytes,
               (long long)need);
+  // (rows cost the score kernels twice the loads: only where the tiles do not fit)
+  const bool tiled = score_takes_tiled(dtype, D) && workspace_bytes >= block_map_workspace_bytes(dtype, BH, L, D, BLKQ, BLKK);
   RowLayout lay;
   rc = make_layout(strides, B, H, L, D, dtype == SLA_F32 ? 4 : 2, &lay);
   if (rc) return rc;
@@ -986,10 +1019,10 @@ int block_map_entry(const void* q, const void* k, const int64_t* strides, int dt
   char* ws = (char*)workspace;
   const int lut64 = lut_elem_bytes == 8;
   if (dtype == SLA_F32)
-    return block_map_impl<IoF32>(q, k, lay, dtype, BH, L, D, BLKQ, BLKK, topk, ws, sparse_map, lut, lut64, st);
+    return block_map_impl<IoF32>(q, k, lay, dtype, BH, L, D, BLKQ, BLKK, topk, ws, tiled, sparse_map, lut, lut64, st);
   if (dtype == SLA_BF16)
-    return block_map_impl<IoBf16>(q, k, lay, dtype, BH, L, D, BLKQ, BLKK, topk, ws, sparse_map, lut, lut64, st);
-  return block_map_impl<IoF16>(q, k, lay, dtype, BH, L, D, BLKQ, BLKK, topk, ws, sparse_map, lut, lut64, st);
+    return block_map_impl<IoBf16>(q, k, lay, dtype, BH, L, D, BLKQ, BLKK, topk, ws, tiled, sparse_map, lut, lut64, st);
+  return block_map_impl<IoF16>(q, k, lay, dtype, BH, L, D, BLKQ, BLKK, topk, ws, tiled, sparse_map, lut, lut64, st);
 }
 
 }  // namespace sla
@@ -1052,7 +1085,7 @@ extern "C" int sla_block_map_fwd_static(const void* q, const void* k, int dtype,
   SLA_REQUIRE(B > 0 && H > 0 && L > 0 && D > 0 && BLKQ > 0 && BLKK > 0 && (int64_t)B * H <= 65535, SLA_ERR_BAD_ARG,
               "bad size (B=%d H=%d L=%d D=%d BLKQ=%d BLKK=%d)", B, H, L, D, BLKQ, BLKK);
   SLA_REQUIRE(dtype == SLA_F32 || dtype == SLA_BF16 || dtype == SLA_F16, SLA_ERR_BAD_ARG, "unknown dtype %d", dtype);
-  const int64_t need = block_map_workspace_bytes(dtype, B * H, L, D, BLKQ, BLKK);
+  const int64_t need = block_map_least_bytes(dtype, B * H, L, D, BLKQ, BLKK);
   SLA_REQUIRE(need <= (int64_t)SLA_STATIC_SCRATCH_BYTES, SLA_ERR_WORKSPACE,
               "this problem needs %lld bytes of scratch, the static buffer holds %lld: use sla_block_map_fwd with a "
               "workspace of the caller's",

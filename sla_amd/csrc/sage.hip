@@ -505,7 +505,7 @@ static SagePrepWs sage_prep_ws(int BH, int L, int D) {
   size_t off = sage_ws(BH, L, D).total;
   w.pq = off;    off += align_up((int64_t)BH * align_up(M, 32) * D * 2, 256);      // (whole tiles of 32)
   w.pk = off;    off += align_up((int64_t)BH * align_up(N, 32) * D * 2, 256);
-  w.score = off; off += align_up((int64_t)BH * M * N * 2, 256);
+  w.score = off; off += scores_in_memory((int)N, D) ? align_up((int64_t)BH * M * N * 2, 256) : 0;
   w.total = off;
   return w;
 }
