@@ -615,7 +615,7 @@ static __device__ __forceinline__ void select_rows(const uint32_t (&kx)[R][EPL],
           }
           if (mrow) {
             wave_lds_fence();
-            if (!(N & 3)) {
+            if (!(((uintptr_t)mrow | (uint32_t)N) & 3)) {        // (a map may start at any byte)
 #pragma unroll
               for (int e = 0; e < EPL / 4; ++e)
                 if (4 * (64 * e + lane) < N) reinterpret_cast<uint32_t*>(mrow)[64 * e + lane] = reinterpret_cast<const uint32_t*>(lm)[64 * e + lane];

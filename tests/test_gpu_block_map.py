@@ -147,3 +147,20 @@ def test_selection_among_equal_scores(dev, L):
     m_ref, lut_ref, T = O.get_block_map(q, k, 0.1, 64, 64)
     m, lut, _ = get_block_map(q.to(dev), k.to(dev), 0.1, 64, 64)
     assert torch.equal(m.cpu(), m_ref) and torch.equal(lut.cpu().long(), lut_ref.long())
+
+
+@pytest.mark.parametrize("offset", [1, 2, 3])
+def test_a_map_that_starts_at_any_byte(dev, offset):
+    """The int8 map has no alignment to keep, also where its rows are a multiple of four long."""
+    from sla_amd import _lib, get_block_map
+    H, L, D, ratio = 2, 256 * 64, 64, 0.05
+    g = torch.Generator(device=dev).manual_seed(offset)
+    q, k = (torch.randn(1, H, L, D, generator=g, device=dev).bfloat16() for _ in range(2))
+    m_ref, lut_ref, T = get_block_map(q, k, ratio, 64, 64)
+    buf = torch.full((m_ref.numel() + 8,), 7, dtype=torch.int8, device=dev)
+    lut = torch.empty_like(lut_ref)
+    ws = _lib.workspace(_lib.WS_BLOCK_MAP, _lib.SLA_BF16, 1, H, L, D, 64, 64, T, dev)
+    _lib.check(_lib.load().sla_block_map_fwd(q.data_ptr(), k.data_ptr(), _lib.SLA_BF16, 1, H, L, D, 64, 64, T, ws.data_ptr(),
+                                             ws.numel(), buf.data_ptr() + offset, lut.data_ptr(), 8, _lib.stream_ptr(dev)))
+    assert torch.equal(buf[offset:offset + m_ref.numel()].view_as(m_ref), m_ref) and torch.equal(lut, lut_ref)
+    assert bool((buf[:offset] == 7).all()) and bool((buf[offset + m_ref.numel():] == 7).all())
