@@ -984,10 +984,11 @@ void launch_map_from_pooled(int dtype, const void* pq, const void* pk, void* sco
   }
 }
 
-// (want_map = false: the caller needs the look-up table only, sparse_map may be null)
-int block_map_entry(const void* q, const void* k, const int64_t* strides, int dtype, int B, int H, int L, int D, int BLKQ,
-                    int BLKK, int topk, void* workspace, int64_t workspace_bytes, int8_t* sparse_map, bool want_map, void* lut,
-                    int lut_elem_bytes, void* stream) {
+// Everything block_map_entry asks of its arguments, for a caller that launches something else before it; `lay` receives the
+// layout of q and k.  (want_map = false: the caller needs the look-up table only, sparse_map may be null)
+int block_map_check(const void* q, const void* k, const int64_t* strides, int dtype, int B, int H, int L, int D, int BLKQ,
+                    int BLKK, int topk, const void* workspace, int64_t workspace_bytes, const int8_t* sparse_map, bool want_map,
+                    const void* lut, int lut_elem_bytes, RowLayout* lay) {
   SLA_REQUIRE(B > 0 && H > 0, SLA_ERR_BAD_ARG, "non-positive batch/head count (B=%d H=%d)", B, H);
   const int64_t BH64 = (int64_t)B * H;
   SLA_REQUIRE(BH64 <= 65535, SLA_ERR_UNSUPPORTED, "B*H=%lld exceeds 65535", (long long)BH64);
@@ -1010,11 +1011,19 @@ int block_map_entry(const void* q, const void* k, const int64_t* strides, int dt
   const int64_t need = block_map_least_bytes(dtype, BH, L, D, BLKQ, BLKK);
   SLA_REQUIRE(workspace_bytes >= need, SLA_ERR_WORKSPACE, "workspace of %lld bytes, need %lld", (long long)workspace_bytes,
               (long long)need);
+  return make_layout(strides, B, H, L, D, dtype == SLA_F32 ? 4 : 2, lay);
+}
+
+int block_map_entry(const void* q, const void* k, const int64_t* strides, int dtype, int B, int H, int L, int D, int BLKQ,
+                    int BLKK, int topk, void* workspace, int64_t workspace_bytes, int8_t* sparse_map, bool want_map, void* lut,
+                    int lut_elem_bytes, void* stream) {
+  RowLayout lay;
+  const int rc = block_map_check(q, k, strides, dtype, B, H, L, D, BLKQ, BLKK, topk, workspace, workspace_bytes, sparse_map,
+                                 want_map, lut, lut_elem_bytes, &lay);
+  if (rc) return rc;
+  const int BH = B * H;
   // (rows cost the score kernels twice the loads: only where the tiles do not fit)
   const bool tiled = score_takes_tiled(dtype, D) && workspace_bytes >= block_map_workspace_bytes(dtype, BH, L, D, BLKQ, BLKK);
-  RowLayout lay;
-  rc = make_layout(strides, B, H, L, D, dtype == SLA_F32 ? 4 : 2, &lay);
-  if (rc) return rc;
   hipStream_t st = (hipStream_t)stream;
   char* ws = (char*)workspace;
   const int lut64 = lut_elem_bytes == 8;

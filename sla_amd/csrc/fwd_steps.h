@@ -7,6 +7,9 @@ namespace sla {
 
 // mask builder (block_map.hip); sparse_map may be null where only the look-up table is wanted
 int64_t block_map_workspace_bytes(int dtype, int BH, int L, int D, int BLKQ, int BLKK);
+int block_map_check(const void* q, const void* k, const int64_t* strides, int dtype, int B, int H, int L, int D, int BLKQ,
+                    int BLKK, int topk, const void* workspace, int64_t workspace_bytes, const int8_t* sparse_map, bool want_map,
+                    const void* lut, int lut_elem_bytes, RowLayout* lay);
 int block_map_entry(const void* q, const void* k, const int64_t* strides, int dtype, int B, int H, int L, int D, int BLKQ,
                     int BLKK, int topk, void* workspace, int64_t workspace_bytes, int8_t* sparse_map, bool want_map, void* lut,
                     int lut_elem_bytes, void* stream);

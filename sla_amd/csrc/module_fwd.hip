@@ -62,6 +62,12 @@ extern "C" int sla_module_fwd(const void* q, const void* k, const void* v, const
   char* const map_part = (char*)workspace;
   const int64_t map_bytes = align_up(block_map_workspace_bytes(in_dtype, BH, L, D, BLKQ, BLKK), 256);
   char* const parts = map_part + map_bytes;
+  if (!mask_given) {                   // (the mask builder's own checks too, before the first launch)
+    RowLayout unused;
+    rc = block_map_check(q, k, qkv_strides, in_dtype, B, H, L, D, BLKQ, BLKK, topk, map_part, map_bytes, sparse_map,
+                         sparse_map != nullptr, lut, lut_elem_bytes, &unused);
+    if (rc) return rc;
+  }
 
   const void *qc = q, *kc = k, *vc = v;
   if (casts) {

@@ -626,16 +626,17 @@ extern "C" int sage_quant_qk(const void* q, const void* k, int dtype, int B, int
   return quant_qk_impl<f16_tag, 64>(q, k, dtype, BH, L, q_int8, q_scale, k_int8, k_scale, ws, st);
 }
 
-static int prepare_entry(const void* q, const void* k, const void* v, const int64_t* qkv_strides, int dtype, int B, int H, int L,
-                         int D, int BLKQ, int BLKK, int topk, int8_t* sparse_map, void* lut, int lut_elem_bytes, int8_t* q_int8,
-                         float* q_scale, int8_t* k_int8, float* k_scale, uint8_t* v_fp8, float* v_scale, float v_range,
-                         void* workspace, int64_t workspace_bytes, void* stream, bool want_map = true) {
+// Everything prepare_entry asks of its arguments, for a caller that launches something else before it.
+static int prepare_check(const void* q, const void* k, const void* v, const int64_t* qkv_strides, int dtype, int B, int H, int L,
+                         int D, int BLKQ, int BLKK, int topk, const int8_t* sparse_map, const void* lut, int lut_elem_bytes,
+                         const int8_t* q_int8, const float* q_scale, const int8_t* k_int8, const float* k_scale,
+                         const uint8_t* v_fp8, const float* v_scale, float v_range, const void* workspace,
+                         int64_t workspace_bytes, bool want_map, RowLayout* lay) {
   int rc = validate_sage(dtype, B, H, L, D, BLKQ, BLKK);
   if (rc) return rc;
   rc = validate_v_range(v_range);
   if (rc) return rc;
-  RowLayout lay;
-  rc = make_layout(qkv_strides, B, H, L, D, 2, &lay);
+  rc = make_layout(qkv_strides, B, H, L, D, 2, lay);
   if (rc) return rc;
   const int N = cdiv(L, 64);
   SLA_REQUIRE(topk >= 0 && topk <= N, SLA_ERR_BAD_ARG, "topk=%d outside [0, %d]", topk, N);
@@ -653,6 +654,18 @@ static int prepare_entry(const void* q, const void* k, const void* v, const int6
   const int BH = B * H;
   SLA_REQUIRE(workspace_bytes >= sage_prepare_workspace_bytes(BH, L, D), SLA_ERR_WORKSPACE, "workspace of %lld bytes, need %lld",
               (long long)workspace_bytes, (long long)sage_prepare_workspace_bytes(BH, L, D));
+  return SLA_OK;
+}
+
+static int prepare_entry(const void* q, const void* k, const void* v, const int64_t* qkv_strides, int dtype, int B, int H, int L,
+                         int D, int BLKQ, int BLKK, int topk, int8_t* sparse_map, void* lut, int lut_elem_bytes, int8_t* q_int8,
+                         float* q_scale, int8_t* k_int8, float* k_scale, uint8_t* v_fp8, float* v_scale, float v_range,
+                         void* workspace, int64_t workspace_bytes, void* stream, bool want_map = true) {
+  RowLayout lay;
+  const int rc = prepare_check(q, k, v, qkv_strides, dtype, B, H, L, D, BLKQ, BLKK, topk, sparse_map, lut, lut_elem_bytes, q_int8,
+                               q_scale, k_int8, k_scale, v_fp8, v_scale, v_range, workspace, workspace_bytes, want_map, &lay);
+  if (rc) return rc;
+  const int BH = B * H;
   hipStream_t st = (hipStream_t)stream;
   char* ws = (char*)workspace;
   const int lut64 = lut_elem_bytes == 8;
@@ -794,13 +807,12 @@ extern "C" int sage_module_fwd(const void* q, const void* k, const void* v, cons
   SLA_REQUIRE(fmap == SLA_FMAP_ELU || fmap == SLA_FMAP_RELU || fmap == SLA_FMAP_SOFTMAX, SLA_ERR_BAD_ARG,
               "unknown feature map %d", fmap);
   SLA_REQUIRE(q && k && v && weight && bias && out && workspace, SLA_ERR_BAD_ARG, "null pointer");
-  SLA_REQUIRE(((uintptr_t)workspace | (uintptr_t)weight | (uintptr_t)out) % 16 == 0, SLA_ERR_BAD_ARG,
-              "pointers must be 16-byte aligned");
+  SLA_REQUIRE(((uintptr_t)k | (uintptr_t)v | (uintptr_t)workspace | (uintptr_t)weight | (uintptr_t)out) % 16 == 0,
+              SLA_ERR_BAD_ARG, "pointers must be 16-byte aligned");
   const SageModuleWs w = sage_module_ws(B, H, L, D, topk);
   SLA_REQUIRE(workspace_bytes >= (int64_t)w.total, SLA_ERR_WORKSPACE, "workspace of %lld bytes, need %lld",
               (long long)workspace_bytes, (long long)w.total);
-  RowLayout lay;                       // (what the steps would find wrong with the strides, before the first launch)
-  if ((rc = make_layout(qkv_strides, B, H, L, D, 2, &lay))) return rc;
+  RowLayout lay;
   if ((rc = make_layout(out_strides, B, H, L, D, 2, &lay))) return rc;
   char* ws = (char*)workspace;
   hipStream_t st = (hipStream_t)stream, side = (hipStream_t)side_stream;
@@ -808,6 +820,10 @@ extern "C" int sage_module_fwd(const void* q, const void* k, const void* v, cons
   uint8_t* v8 = (uint8_t*)(ws + w.v8);
   float *qs = (float*)(ws + w.qs), *ks = (float*)(ws + w.ks), *vs = (float*)(ws + w.vs);
   void *lut = ws + w.lut, *o_s = ws + w.o_s;
+  // (what the later steps would find wrong, before the first launch)
+  rc = prepare_check(q, k, nullptr, qkv_strides, dtype, B, H, L, D, 128, 64, topk, nullptr, lut, 4, q8, qs, k8, ks, nullptr,
+                     nullptr, v_range, ws + w.prep, w.prep_bytes, false, &lay);
+  if (rc) return rc;
   const auto state = [&](hipStream_t s) {
     return qkv_strides ? sla_linear_state_quant_v_fwd_strided(k, v, qkv_strides, weight, dtype, fmap, B, H, L, D, ws + w.linear,
                                                               w.linear_bytes, v8, vs, v_range, s)

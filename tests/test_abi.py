@@ -228,3 +228,21 @@ def test_complement_states_entries_check_their_states():
         assert call(None, 1 << 30) == _lib.ERR_BAD_ARG
         assert call(FAKE + 8, 1 << 30) == _lib.ERR_BAD_ARG and "aligned" in _lib.last_error()
         assert call(FAKE, ws(op) - states - 1) == _lib.ERR_WORKSPACE
+
+
+def test_one_call_forwards_check_everything_before_the_first_launch():
+    """What a later step of the one-call forwards would refuse is refused before the first of them is launched (here, without a
+    GPU, a launch that came first would be reported instead)."""
+    lib = _lib.load()
+    big = 64 * 4097                                  # one key block more than the mask builder takes
+    n = 1 << 40
+    for in_dtype, cast in ((_lib.SLA_BF16, None), (_lib.SLA_F32, FAKE)):
+        rc = lib.sla_module_fwd(FAKE, FAKE, FAKE, None, in_dtype, cast, FAKE, FAKE, FAKE, None, None, FAKE, None, FAKE, 4, FAKE,
+                                _lib.SLA_BF16, 0, 1, 1, big, 64, 64, 64, 3, 0.1, FAKE, n, None, None)
+        assert rc == _lib.ERR_UNSUPPORTED and "4096 key blocks" in _lib.last_error()
+    sage = lambda L=256, q=FAKE, v=FAKE, v_range=448.0: lib.sage_module_fwd(  # noqa: E731
+        q, FAKE, v, None, FAKE, FAKE, FAKE, None, _lib.SLA_BF16, 0, 1, 1, L, 64, 3, 0.1, v_range, FAKE, n, None, None)
+    assert sage(L=big) == _lib.ERR_UNSUPPORTED and "4096 key blocks" in _lib.last_error()
+    assert sage(q=FAKE + 2) == _lib.ERR_BAD_ARG and "aligned" in _lib.last_error()
+    assert sage(v=FAKE + 2) == _lib.ERR_BAD_ARG and "aligned" in _lib.last_error()
+    assert sage(v_range=500.0) == _lib.ERR_BAD_ARG and "v_range" in _lib.last_error()
