@@ -59,6 +59,8 @@ extern "C" {
 #define SLA_WS_LINEAR_BWD_STATES_APART 10 /* linear_workspace of sla_module_bwd_states */
 #define SLA_WS_SAGE_MODULE_FWD 11
 #define SLA_WS_LINEAR_COMPLEMENT_STATES 12 /* `states` of sla_linear_complement_fwd_states */
+#define SLA_WS_LINEAR_COMPLEMENT_APART 13 /* workspace of sla_linear_complement_fwd_states */
+#define SLA_WS_LINEAR_COMPLEMENT_BWD_APART 14 /* workspace of sla_linear_complement_bwd_states */
 
 /* flags of sla_linear_bwd */
 #define SLA_BWD_ACCUMULATE 1   /* dq, dk, dv already hold the sparse branch's gradients: add to them */
@@ -270,7 +272,7 @@ int sla_linear_complement_bwd(const void* q, const void* k, const void* v, const
 
 /* The two calls above with the query blocks' states (SLA_WS_LINEAR_COMPLEMENT_STATES bytes, 16-byte aligned) in a buffer of
  * the caller's: the forward writes them, the backward of the same q, k, v, lut and sizes reads them instead of forming them
- * again.  The workspaces are smaller by that many bytes. */
+ * again.  Workspaces: SLA_WS_LINEAR_COMPLEMENT_APART and SLA_WS_LINEAR_COMPLEMENT_BWD_APART. */
 int sla_linear_complement_fwd_states(const void* q, const void* k, const void* v, const void* lut, int lut_elem_bytes,
                                      const float* weight, const float* bias, const void* residual, void* out,
                                      void* states, int dtype, int fmap, int B, int H, int L, int D, int BLKQ, int BLKK,

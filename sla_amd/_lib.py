@@ -21,7 +21,7 @@ _DTYPE_CODES = {torch.float32: SLA_F32, torch.bfloat16: SLA_BF16, torch.float16:
 FMAP = {"elu": 0, "relu": 1, "softmax": 2}
 (WS_BLOCK_MAP, WS_SPARSE_BWD, WS_LINEAR_FWD, WS_LINEAR_BWD, WS_SAGE_QUANT, WS_LINEAR_COMPLEMENT, WS_SAGE_PREPARE,
  WS_LINEAR_STATES, WS_LINEAR_COMPLEMENT_BWD, WS_MODULE_FWD, WS_LINEAR_BWD_STATES_APART,
- WS_SAGE_MODULE_FWD, WS_LINEAR_COMPLEMENT_STATES) = range(13)
+ WS_SAGE_MODULE_FWD, WS_LINEAR_COMPLEMENT_STATES, WS_LINEAR_COMPLEMENT_APART, WS_LINEAR_COMPLEMENT_BWD_APART) = range(15)
 BWD_ACCUMULATE, BWD_STATES_READY = 1, 2
 
 ERR_BAD_ARG, ERR_UNSUPPORTED, ERR_LAUNCH, ERR_WORKSPACE = -1, -2, -3, -4

@@ -84,6 +84,8 @@ int64_t linear_states_bytes(int BH, int L, int D);
 int64_t linear_complement_workspace_bytes(int BH, int L, int D, int BLKQ);
 int64_t linear_complement_states_bytes(int BH, int L, int D, int BLKQ);
 int64_t linear_complement_bwd_workspace_bytes(int BH, int L, int D, int BLKQ);
+int64_t linear_complement_apart_bytes(int BH, int L, int D);
+int64_t linear_complement_bwd_apart_bytes(int BH, int L, int D, int BLKQ);
 int64_t sage_module_workspace_bytes(int B, int H, int L, int D, int topk);
 int64_t linear_bwd_states_apart_bytes(int BH, int L, int D);
 int64_t module_fwd_workspace_bytes(int in_dtype, int BH, int L, int D, int BLKQ, int BLKK);
@@ -126,6 +128,11 @@ extern "C" int64_t sla_workspace_bytes(int op, int dtype, int B, int H, int L, i
     case SLA_WS_LINEAR_COMPLEMENT_BWD:
       SLA_REQUIRE(BLKQ == 64 || BLKQ == 128, SLA_ERR_UNSUPPORTED, "BLKQ=%d (64 or 128)", BLKQ);
       return linear_complement_bwd_workspace_bytes(BH, L, D, BLKQ);
+    case SLA_WS_LINEAR_COMPLEMENT_APART:
+      return linear_complement_apart_bytes(BH, L, D);
+    case SLA_WS_LINEAR_COMPLEMENT_BWD_APART:
+      SLA_REQUIRE(BLKQ == 64 || BLKQ == 128, SLA_ERR_UNSUPPORTED, "BLKQ=%d (64 or 128)", BLKQ);
+      return linear_complement_bwd_apart_bytes(BH, L, D, BLKQ);
     case SLA_WS_LINEAR_BWD_STATES_APART:
       return linear_bwd_states_apart_bytes(BH, L, D);
     case SLA_WS_MODULE_FWD:

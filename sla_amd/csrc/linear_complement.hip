@@ -753,7 +753,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // ---- host ---------------------------------------------------------------------------------
 struct ComplWs {
   int ngroup;
-  size_t hblk, zblk, hgrp, zgrp, hall, zall, total;      // total: without the query blocks' states, which follow
+  size_t hblk, zblk, hgrp, zgrp, hall, zall, total;      // total: without the query blocks' states
 };
 // The query blocks' states: what the backward reads of the forward.
 struct ComplStates {
@@ -782,8 +782,31 @@ static ComplWs compl_ws(int BH, int L, int D) {
   w.total = off;
   return w;
 }
+// A call that does not keep the query blocks' states (twice the bytes of q at 64-row blocks and head dim 128) forms them for a
+// few heads at a time: in the place of the groups' sums, which nobody reads any more (an eighth of the block states), or,
+// where those hold less, in up to CPL_STATES_AT_ONCE bytes of their own, so that short problems stay one launch.
+// 40 heads x 75600 x 128: 1.65 GiB of workspace (all at once 3.1), in 10 groups.
+constexpr int64_t CPL_STATES_AT_ONCE = 64ll << 20;
+struct ComplGroups {
+  int heads;             // per group
+  size_t at, extra;      // where the states lie; bytes they add behind `end`, the end of the rest of the workspace
+};
+static ComplGroups compl_groups(int BH, int L, int D, int BLKQ, size_t end) {
+  const ComplWs w = compl_ws(BH, L, D);
+  const size_t sums = w.zgrp - w.hgrp, one = compl_states(1, L, D, BLKQ).total;
+  const size_t room = sums > (size_t)CPL_STATES_AT_ONCE ? sums : (size_t)CPL_STATES_AT_ONCE;
+  ComplGroups g;
+  g.heads = (int)(room / one < 1 ? 1 : room / one > (size_t)BH ? BH : room / one);
+  g.heads = cdiv(BH, cdiv(BH, g.heads));                    // (even groups)
+  const size_t bytes = compl_states(g.heads, L, D, BLKQ).total;
+  g.extra = bytes <= sums ? 0 : bytes;
+  g.at = bytes <= sums ? w.hgrp : end;
+  return g;
+}
+int64_t linear_complement_apart_bytes(int BH, int L, int D) { return (int64_t)compl_ws(BH, L, D).total; }
 int64_t linear_complement_workspace_bytes(int BH, int L, int D, int BLKQ) {
-  return (int64_t)(compl_ws(BH, L, D).total + compl_states(BH, L, D, BLKQ).total);
+  const size_t end = compl_ws(BH, L, D).total;
+  return (int64_t)(end + compl_groups(BH, L, D, BLKQ, end).extra);
 }
 
 // `total - listed` for nrows rows of every head (see complement_gather_kernel)
@@ -796,40 +819,57 @@ static void launch_gather(const uint16_t* blocks, const float* zblocks, const fl
                      list, list64, count, fixed, stride, states, zstates, nrows, nblk, units);
 }
 
-// Block states, their totals and the query blocks' states.
+// Block states and their totals.
 template <typename Tag, int D>
-static void complement_states_run(const void* k, const void* v, const void* lut, int lut64, int fmap, int BH, int L, int BLKQ,
-                                  int topk, char* ws, char* states, hipStream_t st) {
+static void complement_totals_run(const void* k, const void* v, int fmap, int BH, int L, char* ws, hipStream_t st) {
   const ComplWs w = compl_ws(BH, L, D);
-  const ComplStates s = compl_states(BH, L, D, BLKQ);
   const int N = cdiv(L, 64);
   uint16_t* hblk = (uint16_t*)(ws + w.hblk);
   float* zblk = (float*)(ws + w.zblk);
-  float* hall = (float*)(ws + w.hall);
-  float* zall = (float*)(ws + w.zall);
   float* hgrp = (float*)(ws + w.hgrp);
   float* zgrp = (float*)(ws + w.zgrp);
   hipLaunchKernelGGL((linear_state_partial_kernel<Tag, D, true>), dim3(N, BH), dim3(256), 0, st, (const uint16_t*)k,
                      (const uint16_t*)v, contiguous_layout(BH, L, D), (void*)hblk, zblk, L, 64, fmap, (const float*)nullptr);
   hipLaunchKernelGGL((complement_group_kernel<Tag>), dim3(cdiv(D * D / 8, 256), w.ngroup, BH), dim3(256), 0, st, hblk, zblk,
                      hgrp, zgrp, N, D);
-  hipLaunchKernelGGL(complement_total_kernel, dim3(cdiv(D * D, 256), BH), dim3(256), 0, st, hgrp, zgrp, hall, zall, w.ngroup,
-                     D);
-  launch_gather<Tag, D>(hblk, zblk, hall, zall, lut, lut64, nullptr, topk, topk, (uint16_t*)(states + s.h),
-                        (float*)(states + s.z), BH, cdiv(L, BLKQ), N, st);
+  hipLaunchKernelGGL(complement_total_kernel, dim3(cdiv(D * D, 256), BH), dim3(256), 0, st, hgrp, zgrp, (float*)(ws + w.hall),
+                     (float*)(ws + w.zall), w.ngroup, D);
 }
 
+// The query blocks' states of `heads` heads from head h0 on, laid out as compl_states(heads, ..) says.
+template <typename Tag, int D>
+static void complement_gather_run(const void* lut, int lut64, int BH, int L, int BLKQ, int topk, const char* ws, int h0, int heads,
+                                  char* states, hipStream_t st) {
+  const ComplWs w = compl_ws(BH, L, D);
+  const ComplStates s = compl_states(heads, L, D, BLKQ);
+  const int N = cdiv(L, 64), M = cdiv(L, BLKQ);
+  const size_t head = h0;
+  launch_gather<Tag, D>((const uint16_t*)(ws + w.hblk) + head * N * D * D, (const float*)(ws + w.zblk) + head * N * D,
+                        (const float*)(ws + w.hall) + head * D * D, (const float*)(ws + w.zall) + head * D,
+                        lut ? (const char*)lut + head * M * topk * (lut64 ? 8 : 4) : nullptr, lut64, nullptr, topk, topk,
+                        (uint16_t*)(states + s.h), (float*)(states + s.z), heads, M, N, st);
+}
+
+// (kept: where the caller wants every head's states; null: they are formed in the workspace, a group of heads at a time)
 template <typename Tag, int D, int BLKQ>
 static int complement_impl(const void* q, const void* k, const void* v, const void* lut, int lut64, const float* weight,
                            const float* bias, const void* residual, void* out, int fmap, int BH, int L, int topk, char* ws,
-                           char* states, hipStream_t st) {
-  const ComplStates s = compl_states(BH, L, D, BLKQ);
+                           char* kept, hipStream_t st) {
   const int Mblk = cdiv(L, BLKQ);
-  complement_states_run<Tag, D>(k, v, lut, lut64, fmap, BH, L, BLKQ, topk, ws, states, st);
-  const int total = BH * cdiv(Mblk, OUT_RUN);
-  hipLaunchKernelGGL((complement_out_kernel<Tag, D, BLKQ>), dim3(xcd_grid(total)), dim3(256), 0, st, (const uint16_t*)q,
-                     (const uint16_t*)(states + s.h), (const float*)(states + s.z), weight, bias, (const uint16_t*)residual,
-                     (uint16_t*)out, L, Mblk, fmap, total);
+  complement_totals_run<Tag, D>(k, v, fmap, BH, L, ws, st);
+  const ComplGroups g = compl_groups(BH, L, D, BLKQ, compl_ws(BH, L, D).total);
+  const int step = kept ? BH : g.heads;
+  char* const states = kept ? kept : ws + g.at;
+  for (int h0 = 0; h0 < BH; h0 += step) {
+    const int heads = BH - h0 < step ? BH - h0 : step;
+    const ComplStates s = compl_states(heads, L, D, BLKQ);
+    const size_t rows = (size_t)h0 * L * D;
+    complement_gather_run<Tag, D>(lut, lut64, BH, L, BLKQ, topk, ws, h0, heads, states, st);
+    const int total = heads * cdiv(Mblk, OUT_RUN);
+    hipLaunchKernelGGL((complement_out_kernel<Tag, D, BLKQ>), dim3(xcd_grid(total)), dim3(256), 0, st, (const uint16_t*)q + rows,
+                       (const uint16_t*)(states + s.h), (const float*)(states + s.z), weight, bias,
+                       residual ? (const uint16_t*)residual + rows : nullptr, (uint16_t*)out + rows, L, Mblk, fmap, total);
+  }
   return check_launch("linear_complement_fwd");
 }
 
@@ -861,8 +901,10 @@ static ComplBwdWs compl_bwd_ws(int BH, int L, int D, int BLKQ) {
   w.total = off;
   return w;
 }
+int64_t linear_complement_bwd_apart_bytes(int BH, int L, int D, int BLKQ) { return (int64_t)compl_bwd_ws(BH, L, D, BLKQ).total; }
 int64_t linear_complement_bwd_workspace_bytes(int BH, int L, int D, int BLKQ) {
-  return (int64_t)(compl_bwd_ws(BH, L, D, BLKQ).total + compl_states(BH, L, D, BLKQ).total);
+  const size_t end = compl_bwd_ws(BH, L, D, BLKQ).total;
+  return (int64_t)(end + compl_groups(BH, L, D, BLKQ, end).extra);
 }
 
 template <typename Tag, int D, int BLKQ>
@@ -873,7 +915,6 @@ static int complement_bwd_impl(const void* q, const void* k, const void* v, cons
   const ComplBwdWs w = compl_bwd_ws(BH, L, D, BLKQ);
   const int N = cdiv(L, 64), Mblk = cdiv(L, BLKQ);
   const RowLayout lay = contiguous_layout(BH, L, D);
-  const ComplStates s = compl_states(BH, L, D, BLKQ);
   // (the forward's block states are done with when the key blocks' take their place)
   uint16_t* gst = (uint16_t*)(ws + w.fwd.hblk);
   float* gzst = (float*)(ws + w.fwd.zblk);
@@ -887,17 +928,24 @@ static int complement_bwd_impl(const void* q, const void* k, const void* v, cons
   float* gzall = (float*)(ws + w.gzall);
   int* count = (int*)(ws + w.count);
   int* list = (int*)(ws + w.list);
-  if (!kept) {
-    complement_states_run<Tag, D>(k, v, lut, lut64, fmap, BH, L, BLKQ, topk, ws, ws + w.total, st);
-    kept = ws + w.total;
-  }
   hipLaunchKernelGGL((linear_prep_weight_kernel<Tag>), dim3(cdiv(D * D, 256)), dim3(256), 0, st, weight, wt, D);
   launch_col_lists(sparse_map, list, count, BH, Mblk, N, st);
-  // rows: dq and the row temporaries
-  const int total_q = BH * Mblk;
-  hipLaunchKernelGGL((complement_bwd_rows_kernel<Tag, D, BLKQ>), dim3(xcd_grid(total_q)), dim3(256), 0, st, (const uint16_t*)q,
-                     (const uint16_t*)d_out, (const uint16_t*)(kept + s.h), (const float*)(kept + s.z), wt, (uint16_t*)dq, dn, y,
-                     dden, L, Mblk, fmap, total_q, accumulate);
+  // rows: dq and the row temporaries (with the forward's states, kept or formed again)
+  if (!kept) complement_totals_run<Tag, D>(k, v, fmap, BH, L, ws, st);
+  const ComplGroups g = compl_groups(BH, L, D, BLKQ, w.total);
+  const int step = kept ? BH : g.heads;
+  for (int h0 = 0; h0 < BH; h0 += step) {
+    const int heads = BH - h0 < step ? BH - h0 : step;
+    const ComplStates s = compl_states(heads, L, D, BLKQ);
+    const size_t rows = (size_t)h0 * L * D;
+    if (!kept) complement_gather_run<Tag, D>(lut, lut64, BH, L, BLKQ, topk, ws, h0, heads, ws + g.at, st);
+    const char* const states = kept ? kept : ws + g.at;
+    const int total_q = heads * Mblk;
+    hipLaunchKernelGGL((complement_bwd_rows_kernel<Tag, D, BLKQ>), dim3(xcd_grid(total_q)), dim3(256), 0, st,
+                       (const uint16_t*)q + rows, (const uint16_t*)d_out + rows, (const uint16_t*)(states + s.h),
+                       (const float*)(states + s.z), wt, (uint16_t*)dq + rows, dn + rows, y + rows, dden + (size_t)h0 * L, L, Mblk,
+                       fmap, total_q, accumulate);
+  }
   // per query block dH_i^T = (a_i^T dn_i)^T and dz_i = sum dden a (the state kernel with q, dn in the place of k, v),
   // then their totals
   hipLaunchKernelGGL((linear_state_partial_kernel<Tag, D, true, true>), dim3(Mblk, BH), dim3(256), 0, st, (const uint16_t*)q,
@@ -940,8 +988,7 @@ static int complement_bwd_entry(const void* q, const void* k, const void* v, con
   SLA_REQUIRE(!apart || (states && (uintptr_t)states % 16 == 0), SLA_ERR_BAD_ARG, "states null or not 16-byte aligned");
   SLA_REQUIRE((int64_t)H * B <= 65535, SLA_ERR_UNSUPPORTED, "B*H exceeds 65535");
   const int BH = B * H;
-  const int64_t need = linear_complement_bwd_workspace_bytes(BH, L, D, BLKQ) -
-                       (apart ? linear_complement_states_bytes(BH, L, D, BLKQ) : 0);
+  const int64_t need = apart ? linear_complement_bwd_apart_bytes(BH, L, D, BLKQ) : linear_complement_bwd_workspace_bytes(BH, L, D, BLKQ);
   SLA_REQUIRE(workspace_bytes >= need, SLA_ERR_WORKSPACE, "workspace of %lld bytes, need %lld", (long long)workspace_bytes,
               (long long)need);
   hipStream_t st = (hipStream_t)stream;
@@ -1003,13 +1050,11 @@ static int complement_fwd_entry(const void* q, const void* k, const void* v, con
   SLA_REQUIRE(!apart || (states && (uintptr_t)states % 16 == 0), SLA_ERR_BAD_ARG, "states null or not 16-byte aligned");
   SLA_REQUIRE((int64_t)H * B <= 65535 && cdiv(L, BLKQ) <= 65535 * 32, SLA_ERR_UNSUPPORTED, "grid too large");
   const int BH = B * H;
-  const int64_t need = linear_complement_workspace_bytes(BH, L, D, BLKQ) -
-                       (apart ? linear_complement_states_bytes(BH, L, D, BLKQ) : 0);
+  const int64_t need = apart ? linear_complement_apart_bytes(BH, L, D) : linear_complement_workspace_bytes(BH, L, D, BLKQ);
   SLA_REQUIRE(workspace_bytes >= need, SLA_ERR_WORKSPACE, "workspace of %lld bytes, need %lld", (long long)workspace_bytes,
               (long long)need);
   hipStream_t st = (hipStream_t)stream;
   char* ws = (char*)workspace;
-  if (!apart) states = ws + compl_ws(BH, L, D).total;
   const int lut64 = lut_elem_bytes == 8;
 #define SLA_CPL_CASE(TAG, DD, BQ) \
   if (D == DD && BLKQ == BQ)      \

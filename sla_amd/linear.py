@@ -106,17 +106,15 @@ def linear_complement_fwd(q, k, v, lut, topk, weight, bias, residual, fmap: str,
         raise TypeError(f"lut must be int32 or int64, got {lut.dtype}")
     out = torch.empty_like(q)
     sizes = (dt, B, H, L, D, BLKQ, BLKK, topk)
-    n = _lib.workspace_bytes(_lib.WS_LINEAR_COMPLEMENT, *sizes)
+    n = _lib.workspace_bytes(_lib.WS_LINEAR_COMPLEMENT_APART if keep_states else _lib.WS_LINEAR_COMPLEMENT, *sizes)
     ins = (q.data_ptr(), k.data_ptr(), v.data_ptr(), lut.data_ptr(), lut.element_size(), weight.data_ptr(), bias.data_ptr(),
            0 if residual is None else residual.data_ptr(), out.data_ptr())
     tail = (dt, _lib.FMAP[fmap], B, H, L, D, BLKQ, BLKK, topk)
+    ws = torch.empty(n, dtype=torch.uint8, device=q.device)
     if not keep_states:
-        ws = torch.empty(n, dtype=torch.uint8, device=q.device)
         _lib.check(_lib.load().sla_linear_complement_fwd(*ins, *tail, ws.data_ptr(), n, _lib.stream_ptr(q.device)))
         return out
     states = _lib.workspace(_lib.WS_LINEAR_COMPLEMENT_STATES, *sizes, q.device)
-    n -= states.numel()
-    ws = torch.empty(n, dtype=torch.uint8, device=q.device)
     _lib.check(_lib.load().sla_linear_complement_fwd_states(*ins, states.data_ptr(), *tail, ws.data_ptr(), n,
                                                             _lib.stream_ptr(q.device)))
     return out, states
@@ -136,9 +134,8 @@ def linear_complement_bwd(q, k, v, sparse_map, lut, topk, weight, bias, d_out, f
         raise TypeError(f"lut must be int32 or int64, got {lut.dtype}")
     assert sparse_map.dtype == torch.int8 and sparse_map.is_contiguous() and lut.is_contiguous()
     assert q.is_contiguous() and k.is_contiguous() and v.is_contiguous() and d_out.is_contiguous()
-    n = _lib.workspace_bytes(_lib.WS_LINEAR_COMPLEMENT_BWD, dt, B, H, L, D, BLKQ, BLKK, topk)
-    if states is not None:
-        n -= states.numel()
+    n = _lib.workspace_bytes(_lib.WS_LINEAR_COMPLEMENT_BWD if states is None else _lib.WS_LINEAR_COMPLEMENT_BWD_APART, dt, B, H, L,
+                             D, BLKQ, BLKK, topk)
     ws = torch.empty(n, dtype=torch.uint8, device=q.device)
     if accumulate_into is None:
         dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)

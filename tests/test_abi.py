@@ -246,3 +246,20 @@ def test_one_call_forwards_check_everything_before_the_first_launch():
     assert sage(q=FAKE + 2) == _lib.ERR_BAD_ARG and "aligned" in _lib.last_error()
     assert sage(v=FAKE + 2) == _lib.ERR_BAD_ARG and "aligned" in _lib.last_error()
     assert sage(v_range=500.0) == _lib.ERR_BAD_ARG and "v_range" in _lib.last_error()
+
+
+@pytest.mark.parametrize("H,L,D,BLKQ", [(40, 75600, 128, 64), (40, 75600, 128, 128), (12, 16380, 128, 64), (2, 4096, 128, 64),
+                                        (1, 262144, 64, 64), (24, 1024, 64, 128)])
+def test_complement_workspace_holds_a_few_heads_states(H, L, D, BLKQ):
+    """Without keeping them, the query blocks' states (M D x D matrices per head) are never all in the workspace: it exceeds
+    what the key blocks' states and their sums take by at most 64 MiB, or one head's."""
+    lib = _lib.load()
+    ws = lambda op: lib.sla_workspace_bytes(op, 1, 1, H, L, D, BLKQ, 64, 1)  # noqa: E731
+    M, N = -(-L // BLKQ), -(-L // 64)
+    up = lambda n: -(-n // 256) * 256  # noqa: E731
+    rest = sum(up(H * n * D * 2 * (D + 2)) for n in (N,)) + sum(up(H * n * D * 4 * (D + 1)) for n in (-(-N // 16), 1)) + 6 * 256
+    room = max(64 << 20, up(M * D * D * 2) + up(M * D * 4))
+    assert ws(_lib.WS_LINEAR_COMPLEMENT) <= rest + room
+    apart, bwd_apart = (ws(op) for op in (_lib.WS_LINEAR_COMPLEMENT_APART, _lib.WS_LINEAR_COMPLEMENT_BWD_APART))
+    assert apart <= rest and 0 <= ws(_lib.WS_LINEAR_COMPLEMENT) - apart <= room
+    assert 0 <= ws(_lib.WS_LINEAR_COMPLEMENT_BWD) - bwd_apart <= room

@@ -186,3 +186,24 @@ def test_gather_over_groups_of_lists(dev, L, D, BLKQ, T):
     for a, c in zip(got, linear_complement_bwd(q, k, v, m, lut, T, w, b, g, "elu", BLKQ, 64)):
         assert torch.equal(a, c)
     _check_grads(got, [t.grad for t in leaves])
+
+
+@pytest.mark.parametrize("H,L,D,BLKQ,T", [
+    (9, 16333, 128, 64, 3),             # two groups of heads, five and four, in a place of their own
+    (40, 32760, 128, 64, 2),            # ten groups, in the place of the groups' sums
+    (13, 66000, 64, 64, 4), (7, 75600, 128, 128, 2)])
+def test_states_of_a_few_heads_at_a_time(dev, H, L, D, BLKQ, T):
+    """Forward and backward that do not keep the query blocks' states form them for a group of heads at a time: the bits of
+    the calls that hold all of them."""
+    g = torch.Generator(device=dev).manual_seed(L)
+    q, k, v, do = (torch.randn(1, H, L, D, generator=g, device=dev).bfloat16() for _ in range(4))
+    w, b = (t.to(dev) for t in make_proj(D))
+    M, N = -(-L // BLKQ), -(-L // 64)
+    lut = torch.rand(1, H, M, N, generator=g, device=dev).topk(T, -1).indices.sort(-1).values.contiguous()
+    m = torch.zeros(1, H, M, N, dtype=torch.int8, device=dev).scatter_(3, lut, 1)
+    out, states = linear_complement_fwd(q, k, v, lut, T, w, b, v, "softmax", BLKQ, 64, keep_states=True)
+    for table in (lut, lut.int()):
+        assert torch.equal(out, linear_complement_fwd(q, k, v, table, T, w, b, v, "softmax", BLKQ, 64))
+    ref = linear_complement_bwd(q, k, v, m, lut, T, w, b, do, "softmax", BLKQ, 64, states=states)
+    for a, c in zip(linear_complement_bwd(q, k, v, m, lut, T, w, b, do, "softmax", BLKQ, 64), ref):
+        assert torch.equal(a, c)
