@@ -199,14 +199,14 @@ class _sla_complement(torch.autograd.Function):
     + sum.  The reference has no such variant; the definition is ``linear_complement_fwd``'s."""
 
     @staticmethod
-    def forward(ctx, q, k, v, weight, bias, sparse_map, lut, topk, BLKQ, BLKK, fmap):
+    def forward(ctx, q, k, v, weight, bias, sparse_map, lut, topk, BLKQ, BLKK, fmap, keep):
+        # (keep: a backward may follow.  ctx.needs_input_grad also says so of a parameter under no_grad)
         assert q.is_contiguous() and k.is_contiguous() and v.is_contiguous()
         assert sparse_map.is_contiguous() and lut.is_contiguous()
         assert BLKQ in (64, 128) and BLKK == 64
         qk_scale = q.shape[-1] ** -0.5
         weight, bias = weight.contiguous(), bias.contiguous()
         o_s, lse = sparse_attn_fwd(q, k, v, lut, topk, BLKQ, BLKK, qk_scale)
-        keep = any(ctx.needs_input_grad[:5])
         out = linear_complement_fwd(q, k, v, lut, topk, weight, bias, o_s, fmap, BLKQ, BLKK, keep_states=keep)
         if keep:
             out, states = out
@@ -222,7 +222,7 @@ class _sla_complement(torch.autograd.Function):
         dq, dk, dv = sparse_attn_bwd(q, k, v, o_s, d_out, lse, sparse_map, lut, topk, BLKQ, BLKK, qk_scale)
         _, _, _, dw, db = linear_complement_bwd(q, k, v, sparse_map, lut, topk, weight, bias, d_out, fmap, BLKQ, BLKK,
                                                 accumulate_into=(dq, dk, dv), states=states)
-        return dq, dk, dv, dw, db, None, None, None, None, None, None
+        return dq, dk, dv, dw, db, None, None, None, None, None, None, None
 
 
 class _sla_packed(torch.autograd.Function):
@@ -359,7 +359,8 @@ class SparseLinearAttention(nn.Module):
             v = v.contiguous()
 
         if self.linear_mode == "complement":
-            return self._forward_complement(q, k, q.to(self.dtype), k.to(self.dtype), v.to(self.dtype), dtype, return_sparsity)
+            return self._forward_complement(q, k, q.to(self.dtype), k.to(self.dtype), v.to(self.dtype), dtype, return_sparsity,
+                                            needs_grad)
         weight, bias = weight.contiguous(), bias.contiguous()
         mask = None
         if not (q.dtype == k.dtype == v.dtype and (dtype == self.dtype or (dtype == torch.float32 and v.data_ptr() % 16 == 0))):
@@ -408,10 +409,10 @@ class SparseLinearAttention(nn.Module):
             return o, min(N, int(self.topk * N)) / N
         return o
 
-    def _forward_complement(self, q, k, qc, kc, vc, dtype, return_sparsity):
+    def _forward_complement(self, q, k, qc, kc, vc, dtype, return_sparsity, needs_grad):
         sparse_map, lut, real_topk = get_block_map(q, k, topk_ratio=self.topk, BLKQ=self.BLKQ, BLKK=self.BLKK)
         o = _sla_complement.apply(qc, kc, vc, self.proj_l.weight, self.proj_l.bias, sparse_map, lut, real_topk, self.BLKQ,
-                                  self.BLKK, self.feature_map).to(dtype)
+                                  self.BLKK, self.feature_map, needs_grad).to(dtype)
         if return_sparsity:
             return o, real_topk / sparse_map.shape[-1]
         return o

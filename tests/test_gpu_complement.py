@@ -4,7 +4,7 @@ import torch
 
 from conftest import cos_sim, max_abs
 from oracle import sla_oracle as O
-from sla_amd import SparseLinearAttention
+from sla_amd import SparseLinearAttention, _lib
 from sla_amd.inputs import CONFIGS, make_inputs, make_proj
 from sla_amd.linear import linear_bwd, linear_complement_bwd, linear_complement_fwd, linear_fwd
 
@@ -207,3 +207,22 @@ def test_states_of_a_few_heads_at_a_time(dev, H, L, D, BLKQ, T):
     ref = linear_complement_bwd(q, k, v, m, lut, T, w, b, do, "softmax", BLKQ, 64, states=states)
     for a, c in zip(linear_complement_bwd(q, k, v, m, lut, T, w, b, do, "softmax", BLKQ, 64), ref):
         assert torch.equal(a, c)
+
+
+def test_inference_does_not_keep_the_states(dev):
+    """Under no_grad, with parameters that could have a gradient, a forward takes no memory for the query blocks' states
+    beyond what it holds at a time."""
+    H, L, D = 16, 32760, 128
+    q, k, v = (torch.randn(1, H, L, D, device=dev).bfloat16() for _ in range(3))
+    mod = SparseLinearAttention(D, 0.02, "elu", linear_mode="complement").to(dev)
+    size = lambda op: _lib.workspace_bytes(op, _lib.SLA_BF16, 1, H, L, D, 64, 64, 10)  # noqa: E731
+    with torch.no_grad():
+        ref = mod(q, k, v)
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        assert torch.equal(mod(q, k, v), ref)
+    used = torch.cuda.max_memory_allocated() - before
+    tensors = 2 * q.numel() * 2 + H * L * 4 + (H * 512 * (512 + 10 * 8))          # attention output and result, lse, map, table
+    assert used <= tensors + size(_lib.WS_LINEAR_COMPLEMENT) + (16 << 20), used
+    assert size(_lib.WS_LINEAR_COMPLEMENT_STATES) > (128 << 20)
