@@ -785,8 +785,9 @@ static ComplWs compl_ws(int BH, int L, int D) {
 // A call that does not keep the query blocks' states (twice the bytes of q at 64-row blocks and head dim 128) forms them for a
 // few heads at a time: in the place of the groups' sums, which nobody reads any more (an eighth of the block states), or,
 // where those hold less, in up to CPL_STATES_AT_ONCE bytes of their own, so that short problems stay one launch.
-// 40 heads x 75600 x 128: 1.65 GiB of workspace (all at once 3.1), in 10 groups.
-constexpr int64_t CPL_STATES_AT_ONCE = 64ll << 20;
+// 40 heads x 75600 x 128: 1.65 GiB of workspace (all at once 3.1), in 10 groups, inference 17.3 ms (16.5).  12 heads x 32760
+// x 128, in us: 64 MiB at once 1222, 128 MiB 1118, all (201 MiB) 1090; up to 12 heads x 16380 are one group.
+constexpr int64_t CPL_STATES_AT_ONCE = 128ll << 20;
 struct ComplGroups {
   int heads;             // per group
   size_t at, extra;      // where the states lie; bytes they add behind `end`, the end of the rest of the workspace

@@ -252,13 +252,13 @@ def test_one_call_forwards_check_everything_before_the_first_launch():
                                         (1, 262144, 64, 64), (24, 1024, 64, 128)])
 def test_complement_workspace_holds_a_few_heads_states(H, L, D, BLKQ):
     """Without keeping them, the query blocks' states (M D x D matrices per head) are never all in the workspace: it exceeds
-    what the key blocks' states and their sums take by at most 64 MiB, or one head's."""
+    what the key blocks' states and their sums take by at most 128 MiB, or one head's."""
     lib = _lib.load()
     ws = lambda op: lib.sla_workspace_bytes(op, 1, 1, H, L, D, BLKQ, 64, 1)  # noqa: E731
     M, N = -(-L // BLKQ), -(-L // 64)
     up = lambda n: -(-n // 256) * 256  # noqa: E731
     rest = sum(up(H * n * D * 2 * (D + 2)) for n in (N,)) + sum(up(H * n * D * 4 * (D + 1)) for n in (-(-N // 16), 1)) + 6 * 256
-    room = max(64 << 20, up(M * D * D * 2) + up(M * D * 4))
+    room = max(128 << 20, up(M * D * D * 2) + up(M * D * 4))
     assert ws(_lib.WS_LINEAR_COMPLEMENT) <= rest + room
     apart, bwd_apart = (ws(op) for op in (_lib.WS_LINEAR_COMPLEMENT_APART, _lib.WS_LINEAR_COMPLEMENT_BWD_APART))
     assert apart <= rest and 0 <= ws(_lib.WS_LINEAR_COMPLEMENT) - apart <= room

@@ -189,9 +189,9 @@ def test_gather_over_groups_of_lists(dev, L, D, BLKQ, T):
 
 
 @pytest.mark.parametrize("H,L,D,BLKQ,T", [
-    (9, 16333, 128, 64, 3),             # two groups of heads, five and four, in a place of their own
-    (40, 32760, 128, 64, 2),            # ten groups, in the place of the groups' sums
-    (13, 66000, 64, 64, 4), (7, 75600, 128, 128, 2)])
+    (20, 16333, 128, 64, 3),            # two groups of heads in a place of their own
+    (36, 65000, 128, 64, 2),            # ten groups, in the place of the groups' sums
+    (19, 66000, 64, 64, 4), (7, 75600, 128, 128, 2)])
 def test_states_of_a_few_heads_at_a_time(dev, H, L, D, BLKQ, T):
     """Forward and backward that do not keep the query blocks' states form them for a group of heads at a time: the bits of
     the calls that hold all of them."""
