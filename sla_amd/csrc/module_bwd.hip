@@ -38,7 +38,7 @@ static int module_bwd_run(const void* q, const void* k, const void* v, const int
   // every argument of both calls is checked before the first kernel of either is launched
   if ((rc = sparse(st, 0))) return rc;
   if ((rc = linear(st, 0))) return rc;
-  if (!side || side == st || !side_stream_pays(B, H, L, D)) {
+  if (!side || side == st || !side_stream_pays(B, H, L, D, topk)) {
     // one stream: the same order, the short kernels in between
     if ((rc = sparse(st, SB_ALL))) return rc;
     return linear(st, LB_ALL);

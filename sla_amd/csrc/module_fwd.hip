@@ -95,7 +95,7 @@ extern "C" int sla_module_fwd(const void* q, const void* k, const void* v, const
     return attn_linear_run(qc, kc, vc, lin, lut, lut_elem_bytes, (const char*)states, bias, o_s, out, lout, lse, dtype, fmap, BH,
                            L, D, BLKQ, topk, qk_scale, st);
   };
-  if (!side || side == st || !side_stream_pays(B, H, L, D)) {
+  if (!side || side == st || !side_stream_pays(B, H, L, D, topk)) {
     if ((rc = state(st))) return rc;
     if ((rc = mask())) return rc;
     return attention();

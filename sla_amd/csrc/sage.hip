@@ -841,7 +841,7 @@ extern "C" int sage_module_fwd(const void* q, const void* k, const void* v, cons
                                                     ws + w.linear, w.linear_bytes, stream)
                        : sla_linear_out_fwd(q, bias, o_s, out, dtype, fmap, B, H, L, D, ws + w.linear, w.linear_bytes, stream);
   };
-  if (!side || side == st || !side_stream_pays(B, H, L, D)) {
+  if (!side || side == st || !side_stream_pays(B, H, L, D, topk)) {
     if ((rc = state(st))) return rc;
     if ((rc = prepare())) return rc;
     return attention();

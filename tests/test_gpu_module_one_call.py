@@ -1,5 +1,6 @@
 """sla_module_fwd / sla_module_bwd_states (what SparseLinearAttention runs) against the single-step entry points they string
-together: the same bits, below and above the size from which a second stream is used (16 MiB per tensor)."""
+together: the same bits, below and above the size (16 MiB per tensor) and the work (few heads, long sequences) from which a
+second stream is used."""
 import pytest
 import torch
 
@@ -14,7 +15,8 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("H,L,D,BLKQ,in_dtype,half", [
     (3, 2100, 128, 64, torch.bfloat16, False), (2, 1000, 64, 128, torch.float32, False), (2, 777, 128, 64, torch.float32, True),
     (2, 640, 64, 64, torch.float16, False),          # a mask from half precision, bf16 compute
-    (12, 6001, 128, 64, torch.bfloat16, False), (24, 6001, 64, 64, torch.float32, True)])
+    (12, 6001, 128, 64, torch.bfloat16, False), (24, 6001, 64, 64, torch.float32, True),
+    (2, 30001, 64, 64, torch.bfloat16, False)])
 def test_one_call_equals_the_steps(dev, H, L, D, BLKQ, in_dtype, half):
     ratio, fmap, dtype = 0.1, "elu" if not half else "softmax", torch.float16 if half else torch.bfloat16
     g = torch.Generator().manual_seed(L + D)
