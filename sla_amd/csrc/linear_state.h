@@ -265,13 +265,52 @@ static __device__ __forceinline__ void sum_slices(const float* __restrict__ p, i
   }
 }
 
+// The same sums in a launch of their own, left in the place of every head's first slice, with the same bits.  The kernel
+// below has D / 16 workgroups per head: few heads with many slices leave it reading on a few compute units.  Here a workgroup
+// of 512 threads takes 256 elements, its halves one half of the slices each, 32 loads in flight; the last one of a head takes z.
+// Bound by latency.  State build in us without this launch and with it: 1 head x 75600 x 128 (295 slices) 88.6 / 35.8, 2 heads
+// x 75600 x 128 (256) 78.4 / 41.4, 4 heads x 32760 x 128 (128) 53.9 / 37.9, 8 heads x 16384 x 64 (64) 23.2 / 19.9, 12 heads x
+// 24576 x 128 (42) 62.3 / 58.9, 16 heads x 16384 x 128 (32) 53.0 / 53.6, 2 heads x 4096 x 64 (16) 14.2 / 15.7.
+template <int D>
+__global__ __launch_bounds__(512) void linear_state_presum_kernel(float* __restrict__ kv_part, float* __restrict__ z_part,
+                                                                  int nsplit) {
+  constexpr int DD = D * D, BATCH = 32;
+  __shared__ float s_half[256];
+  const int bh = blockIdx.y, tid = threadIdx.x & 255, half = threadIdx.x >> 8;
+  const auto sum = [](const float* p, int n, size_t stride) __attribute__((always_inline)) {
+    float acc = 0.f;
+    for (int sp = 0; sp < n; sp += BATCH) {
+      float x[BATCH];
+#pragma unroll
+      for (int i = 0; i < BATCH; ++i) x[i] = p[(size_t)min(sp + i, n - 1) * stride];
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < BATCH; ++i)
+        if (sp + i < n) acc += x[i];
+    }
+    return acc;
+  };
+  if (blockIdx.x == DD / 256) {
+    float* p = z_part + (size_t)bh * nsplit * D + threadIdx.x;
+    if (threadIdx.x < D) *p = sum(p, nsplit, D);
+    return;
+  }
+  float* p = kv_part + (size_t)bh * nsplit * DD + blockIdx.x * 256 + tid;
+  const int n0 = (nsplit + 1) >> 1;
+  const float acc = half ? sum(p + (size_t)n0 * DD, nsplit - n0, DD) : sum(p, n0, DD);
+  if (half) s_half[tid] = acc;
+  __syncthreads();
+  if (!half) *p = acc + s_half[tid];
+}
+
+// (nsum: the slices to add up, all nsplit of a head or the first one alone, which then holds the sums)
 template <typename Tag, int D>
 __global__ __launch_bounds__(512) void linear_state_finish_kernel(const float* __restrict__ kv_part,
                                                                   const float* __restrict__ z_part,
                                                                   const float* __restrict__ weight, uint16_t* __restrict__ kvt,
                                                                   uint16_t* __restrict__ kvp, uint16_t* __restrict__ kvwt,
                                                                   uint16_t* __restrict__ z, uint16_t* __restrict__ wt, int nsplit,
-                                                                  int total) {
+                                                                  int nsum, int total) {
   using E = Elem<Tag>;
   constexpr int DD = D * D;
   constexpr int STR = D + 8;               // row pitch of the strip in LDS
@@ -297,7 +336,7 @@ __global__ __launch_bounds__(512) void linear_state_finish_kernel(const float* _
   f32x4_t acc[NR];
 #pragma unroll
   for (int i = 0; i < NR; ++i) acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  const int n0 = (nsplit + 1) >> 1, first = half ? n0 : 0, n = half ? nsplit - n0 : n0;
+  const int n0 = (nsum + 1) >> 1, first = half ? n0 : 0, n = half ? nsum - n0 : n0;
   sum_slices<NR>(kv_part + ((size_t)bh * nsplit + first) * DD + (size_t)dr * D + d1_0 + dc, n, DD, (size_t)64 * D, acc);
   if (half) {
 #pragma unroll
@@ -306,7 +345,7 @@ __global__ __launch_bounds__(512) void linear_state_finish_kernel(const float* _
       const float* pz = z_part + (size_t)bh * nsplit * D + d1_0 + tid;
       float sum = 0.f;
 #pragma unroll 8
-      for (int sp = 0; sp < nsplit; ++sp) sum += pz[(size_t)sp * D];
+      for (int sp = 0; sp < nsum; ++sp) sum += pz[(size_t)sp * D];
       z[(size_t)bh * D + d1_0 + tid] = E::from_float(sum);
     }
     if (bh == 0)
@@ -389,13 +428,20 @@ static inline LinWs lin_ws(int BH, int L, int D) {
 }
 
 
+constexpr int PRESUM_MIN_SLICES = 40;       // (measured at linear_state_presum_kernel)
+
 // (ws: where the states go; parts: where the slices' partial sums lie, the offsets of `w` past states_end)
 template <typename Tag, int D>
 static inline void launch_state_finish(const float* weight, int BH, char* ws, char* parts, const LinWs& w, hipStream_t st) {
+  float* const kv_part = (float*)(parts + (w.kv_part - w.states_end));
+  float* const z_part = (float*)(parts + (w.z_part - w.states_end));
+  const bool presum = w.nsplit >= PRESUM_MIN_SLICES;
+  if (presum)
+    hipLaunchKernelGGL((linear_state_presum_kernel<D>), dim3(D * D / 256 + 1, BH), dim3(512), 0, st, kv_part, z_part, w.nsplit);
   hipLaunchKernelGGL((linear_state_finish_kernel<Tag, D>), dim3(xcd_grid((int64_t)BH * (D / 16))), dim3(512), 0, st,
-                     (const float*)(parts + (w.kv_part - w.states_end)), (const float*)(parts + (w.z_part - w.states_end)), weight,
+                     (const float*)kv_part, (const float*)z_part, weight,
                      (uint16_t*)(ws + w.kvt), (uint16_t*)(ws + w.kvp), (uint16_t*)(ws + w.kvwt), (uint16_t*)(ws + w.z),
-                     (uint16_t*)(ws + w.wt), w.nsplit, BH * (D / 16));
+                     (uint16_t*)(ws + w.wt), w.nsplit, presum ? 1 : w.nsplit, BH * (D / 16));
 }
 
 // Streams K and V once and leaves the finished states and the 16-bit transposed weight.

@@ -153,3 +153,22 @@ def test_backward_with_the_forward_states_handed_over(dev, fmap, D):
     acc = linear_bwd(q, k, v, w, b, do, fmap, accumulate_into=tuple(t.clone() for t in base), states=states)
     for a, r in zip(acc, acc_ref):
         assert torch.equal(a, r)
+
+
+@pytest.mark.parametrize("H,L,D", [(1, 39 * 256, 128), (1, 40 * 256, 128), (1, 40 * 256 + 1, 64), (2, 66 * 256 - 3, 64), (3, 45000, 128),
+                                   (12, 12 * 1024, 64), (13, 11000, 128)])
+def test_states_over_many_slices(dev, H, L, D):
+    """The slices' sums on either side of the count from which they have a launch of their own (40), odd counts, a last slice
+    that is not full.  With the relu map phi(k) is exact: what is left is the fp32 sum and one rounding to bf16 (8 significant bits: 2^-8)."""
+    from sla_amd.linear import linear_state_fwd, saved_states
+    g = torch.Generator(device=dev).manual_seed(L)
+    k, v = (torch.randn(1, H, L, D, generator=g, device=dev).bfloat16() for _ in range(2))
+    w, _ = (t.to(dev) for t in make_proj(D))
+    st = saved_states(linear_state_fwd(k, v, w, "relu"), k)
+    part = -(-H * D * D * 2 // 256) * 256
+    kvt = st[:H * D * D * 2].view(torch.bfloat16).view(H, D, D).double()                     # [d2][d1]
+    z = st[3 * part:3 * part + H * D * 2].view(torch.bfloat16).view(H, D).double()
+    fk, vd = torch.relu(k[0]).double(), v[0].double()
+    for got, ref, mag in ((kvt, vd.transpose(1, 2) @ fk, vd.abs().transpose(1, 2) @ fk), (z, fk.sum(1), fk.sum(1))):
+        bound = ref.abs() * 2.0 ** -8 + mag * L * 2.0 ** -24
+        assert bool(((got - ref).abs() <= bound).all())
