@@ -587,8 +587,7 @@ struct LinBwdWs {
   LinSplit ss;   // slices of the stream kernel (one workgroup per compute unit, 128 rows per step): never more than st's
   size_t dn, y, dden, ds_part, dw_part, dz_part, db_part, ds, dst, dz, dw_head, db_head, total;
 };
-// (own_states = false: the forward's states lie elsewhere, the workspace holds none.  Head dim 128 never takes the path with
-//  row-wise temporaries.)
+// (own_states = false: the forward's states lie elsewhere, the workspace holds none.  Head dim 128 has no row-wise temporaries.)
 static LinBwdWs lin_bwd_ws(int BH, int L, int D, bool own_states) {
   LinBwdWs w;
   w.fwd = lin_ws(BH, L, D);
@@ -619,6 +618,10 @@ template <typename Tag, int D>
 static int linear_bwd_impl(const void* q, const void* k, const void* v, const float* weight, const void* d_out, void* dq,
                            void* dk, void* dv, const RowLayout& lin, const RowLayout& ldo, float* d_weight, float* d_bias,
                            int fmap, int BH, int L, int flags, const char* states, char* ws, hipStream_t st, int steps) {
+  // (the kernels of head dim 128 address a head's rows through 32-bit buffer offsets; make_layout asks for more)
+  const auto fits32 = [&](const RowLayout& lay) { return ((int64_t)(L - 1) * lay.sl + D) * 2 < ((int64_t)1 << 32); };
+  if constexpr (D == 128)
+    SLA_REQUIRE(fits32(lin) && fits32(ldo), SLA_ERR_UNSUPPORTED, "one head spans 4 GiB or more");
   if (steps == 0) return SLA_OK;        // (arguments checked, nothing asked for)
   const LinBwdWs w = lin_bwd_ws(BH, L, D, !states);
   const int accumulate = flags & SLA_BWD_ACCUMULATE;
@@ -630,12 +633,7 @@ static int linear_bwd_impl(const void* q, const void* k, const void* v, const fl
   const uint16_t* kvt = (const uint16_t*)(states + w.fwd.kvt);
   const uint16_t* z = (const uint16_t*)(states + w.fwd.z);
   constexpr int NW_ROWS = 4, NW_KV = 8;   // one workgroup per compute unit either way (LDS)
-  const int tiles_kv = balanced_tiles(cdiv(L, 32 * NW_KV), BH, 1);
-  // (the stream kernel addresses a head's rows through 32-bit buffer offsets)
-  const auto fits32 = [&](const RowLayout& lay) { return ((int64_t)(L - 1) * lay.sl + D) * 2 < ((int64_t)1 << 32); };
-  bool streamed = false;
-  if constexpr (D == 128) streamed = fits32(lin) && fits32(ldo);
-  if constexpr (D == 128) if (streamed) {
+  if constexpr (D == 128) {
     // q and G once: dq, and the partial sums M^T, dz, db of every slice (M^T's take the place of the general path's ds_part)
     float* m_part = (float*)(ws + w.ds_part);
     if (steps & LB_QUERY) {
@@ -658,8 +656,7 @@ static int linear_bwd_impl(const void* q, const void* k, const void* v, const fl
     else SLA_LBF_LAUNCH(2);
 #undef SLA_LBF_LAUNCH
     }
-  }
-  if (!streamed) {
+  } else {
   uint16_t* dn = (uint16_t*)(ws + w.dn);
   uint16_t* y = (uint16_t*)(ws + w.y);
   float* dden = (float*)(ws + w.dden);
@@ -682,7 +679,7 @@ static int linear_bwd_impl(const void* q, const void* k, const void* v, const fl
     hipLaunchKernelGGL(linear_bwd_reduce_heads_kernel, dim3(cdiv(D * D, 256)), dim3(256), 0, st,
                        (const float*)(ws + w.dw_head), (const float*)(ws + w.db_head), d_weight, d_bias, BH, D);
   if (!(steps & LB_KEYS)) return check_launch("linear_bwd");
-  if constexpr (D == 128) if (streamed) {
+  if constexpr (D == 128) {
 #define SLA_LBK_LAUNCH(FM)                                                                                                \
   hipLaunchKernelGGL((linear_bwd_keys_kernel<Tag, FM>), dim3(w.ss.nsplit, BH), dim3(512), 0, st, (const uint16_t*)k,        \
                      (const uint16_t*)v, (const uint16_t*)(ws + w.ds), (const uint16_t*)(ws + w.dst),                       \
@@ -691,8 +688,8 @@ static int linear_bwd_impl(const void* q, const void* k, const void* v, const fl
     else if (fmap == SLA_FMAP_RELU) SLA_LBK_LAUNCH(SLA_FMAP_RELU);
     else SLA_LBK_LAUNCH(SLA_FMAP_SOFTMAX);
 #undef SLA_LBK_LAUNCH
-    return check_launch("linear_bwd");
-  }
+  } else {
+  const int tiles_kv = balanced_tiles(cdiv(L, 32 * NW_KV), BH, 1);
   if (lin.sl == D)
     hipLaunchKernelGGL((linear_bwd_kv_kernel<Tag, D, NW_KV, true>), dim3(cdiv(L, 32 * NW_KV * tiles_kv), BH), dim3(64 * NW_KV),
                        0, st, (const uint16_t*)k, (const uint16_t*)v, (const uint16_t*)(ws + w.ds),
@@ -703,6 +700,7 @@ static int linear_bwd_impl(const void* q, const void* k, const void* v, const fl
                        0, st, (const uint16_t*)k, (const uint16_t*)v, (const uint16_t*)(ws + w.ds),
                        (const uint16_t*)(ws + w.dst), (const float*)(ws + w.dz), (uint16_t*)dk, (uint16_t*)dv, lin, L, fmap,
                        tiles_kv, accumulate);
+  }
   return check_launch("linear_bwd");
 }
 
