@@ -736,6 +736,9 @@ static int bwd_impl(const void* q, const void* k, const void* v, const void* o, 
   const int wide = BLKQ == 128;
   const int Mblk64 = cdiv(L, 64);
   const int total_q64 = BH * Mblk64;
+  // (dK/dV at head dim 64 is ahead of the general kernel down to the smallest launches: kernel in us, stream / general, 2 heads
+  //  x 1024 rows with 1 key block per row 7.5 / 8.3, 1 x 2000 with 3 10.0 / 11.7, 4 x 2000 14.7 / 16.2, 16 x 1500 with 2 11.6 /
+  //  14.8, 1 x 32760 with 51 86 / 121)
   const bool stream_dkdv = (BLKQ == 64 || BLKQ == 128) && (uint64_t)lin.sl * 2u * (uint64_t)L < (1ull << 31) &&
                            (uint64_t)ldo.sl * 2u * (uint64_t)L < (1ull << 31);
   // (The stream kernel keeps a look-up row as 16-bit key block indices.  One wave of it walks a block that the general

@@ -70,3 +70,39 @@ def test_fp32_v_off_alignment(dev):
         x = [q.clone().requires_grad_(True), k.clone().requires_grad_(True), t.detach().requires_grad_(True)]
         grads.append(torch.autograd.grad(mod(*x), x, do))
     assert all(torch.equal(a, b) for a, b in zip(*grads))
+
+
+@pytest.mark.parametrize("H,L,D,BLKQ,half", [(3, 2100, 128, 64, False), (2, 1000, 64, 128, True), (12, 6001, 128, 128, True),
+                                             (24, 6001, 64, 64, False)])
+def test_packed_one_call_equals_the_steps(dev, monkeypatch, H, L, D, BLKQ, half):
+    """forward_packed, whose calls read q, k, v and write their gradients where the packed tensors hold them, against the
+    single-step entry points on the views: the same bits, with the second stream as the size has it and without one."""
+    ratio, fmap, dtype = 0.1, "elu" if not half else "softmax", torch.float16 if half else torch.bfloat16
+    g = torch.Generator().manual_seed(L + D)
+    qkv = torch.randn(1, L, 3, H, D, generator=g).to(dtype).to(dev)
+    do = torch.randn(1, L, H, D, generator=g).to(dtype).to(dev)
+    w, b = (t.to(dev) for t in make_proj(D))
+    mod = SparseLinearAttention(D, ratio, fmap, BLKQ, 64, use_bf16=not half).to(dev)
+    with torch.no_grad():
+        mod.proj_l.weight.copy_(w)
+        mod.proj_l.bias.copy_(b)
+    q, k, v = (qkv[:, :, i].permute(0, 2, 1, 3) for i in range(3))
+    dv = do.permute(0, 2, 1, 3)
+    sparse_map, lut, T = get_block_map(q, k, ratio, BLKQ, 64)
+    state = linear_state_fwd(k, v, w, fmap)
+    out, o_s, lse = sparse_attn_linear_fwd(q, k, v, lut, T, BLKQ, 64, D ** -0.5, state, b, fmap, want_o_s=True)
+    ref = torch.empty_like(qkv)
+    grads = tuple(ref[:, :, i].permute(0, 2, 1, 3) for i in range(3))
+    sparse_attn_bwd(q, k, v, o_s, dv, lse, sparse_map, lut, T, BLKQ, 64, D ** -0.5, grads=grads)
+    _, _, _, dw, db = linear_bwd(q, k, v, w, b, dv, fmap, accumulate_into=grads)
+    for streams in (2, 2, 1):
+        if streams == 1:
+            monkeypatch.setattr("sla_amd.module._side_stream", lambda dev: None)
+        x = qkv.clone().requires_grad_(True)
+        mod.zero_grad()
+        o = mod.forward_packed(x)
+        o.backward(do)
+        assert torch.equal(o.detach(), out.permute(0, 2, 1, 3)) and torch.equal(x.grad, ref), streams
+        assert torch.equal(mod.proj_l.weight.grad, dw) and torch.equal(mod.proj_l.bias.grad, db)
+        with torch.no_grad():
+            assert torch.equal(mod.forward_packed(qkv), o)
