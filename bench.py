@@ -391,8 +391,9 @@ def main():
         return sparse_attn_linear_fwd(q, k, v, lut, T, cfg.BLKQ, cfg.BLKK, scale, state_ws, bdev, cfg.feature_map, False)
     ms_sparse, ms_sparse_mean = time_steps(torch, attention, args.steps, args.warmup)
     ms_sparse_cold, _ = time_steps(torch, attention, max(args.steps // 2, 5), 2, preheat_s=0.05, flush=flush_buf)
-    # the same launch where the module makes it: behind the mask builder on this stream and the state build on the
-    # module's second stream, caches as those kernels leave them
+    # the same launch behind the kernels that come before it in the module: mask builder on this stream, state build on the
+    # second one, caches as those kernels leave them.  The module enqueues these kernels in one library call, inside which
+    # no event of the caller's can stand; here the step functions enqueue them (the mask builder also writes the map)
     from sla_amd.module import _StateBuild
     in_module = []
     with torch.no_grad():

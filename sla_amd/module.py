@@ -21,6 +21,8 @@ def module_bwd(q, k, v, o_s, d_out, lse, sparse_map, lut, topk, BLKQ, BLKK, qk_s
     """Backward of the whole operator in one library call (``sla_module_bwd``): the kernels of
     :func:`sparse_attn_bwd` and of :func:`linear_bwd` accumulating into the same gradients, bit for bit, with the
     short kernels on ``side_stream`` beside the long ones when one is given.  Returns ``(dq, dk, dv, d_weight, d_bias)``.
+    For callers that hold the forward's parts in tensors of their own; the operators below keep them in one allocation and
+    take :func:`_module_bwd_saved`.
 
     q, k, v (and ``grads=(dq, dk, dv)`` when given) may be row-contiguous views sharing their strides, ``d_out`` a
     row-contiguous view of its own; ``o_s`` and ``lse`` are contiguous.  ``states`` as in :func:`linear_bwd`."""
