@@ -20,7 +20,7 @@
 //     unit of 32 products (1024 cycles of the matrix pipe) where 300 were needed without all that.  The barrier stands
 //     where the fragments of a unit have all been read, so that the first reads of the next unit and the requests for
 //     the unit after next run beside products.  Measured, before and after: B1 H12 L32760 with 25 key blocks per row
-//     840 -> 758 us (matrix pipe busy 45 -> 51 % of the cycles at 1.74 GHz, where the power limit holds it), B2 H16
+//     840 -> 758 us (matrix pipe busy 44 -> 52 % of the cycles, at 1.7 to 1.9 GHz, where the power limit holds it), B2 H16
 //     L32760 with 128-row query blocks 2272 -> 2065 us, B2 H4 L4096 48.5 -> 43.0 us.  Head dim 64 against
 //     bwd_dkdv_kernel: B2 H8 L6001 with 9 key blocks per row 57.6 -> 44.2 us.
 #pragma once
@@ -501,8 +501,8 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
 // (1536 cycles) of a unit, so instructions are what is saved: the accumulators of dP start from -delta instead of zero
 // (no subtraction per element), four requests share one M0, every LDS offset but eight is an instruction immediate: 272
 // instructions per unit where reading the row-wise fragments once per tile took 367.  Measured, that version against this:
-// B1 H12 L32760 with 25 key blocks per row 551 -> 485 us (matrix pipe busy 53 -> 61 % of the cycles, at a clock that the
-// power limit holds at 1.65 GHz), B2 H16 L32760 with 128-row blocks 1428 -> 1224 us, B2 H4 L4096 37.9 -> 33.2 us.
+// B1 H12 L32760 with 25 key blocks per row 551 -> 485 us (matrix pipe busy 49 -> 59 % of the cycles, at a clock that the
+// power limit holds near 1.7 GHz), B2 H16 L32760 with 128-row blocks 1428 -> 1224 us, B2 H4 L4096 37.9 -> 33.2 us.
 // Head dim 64 against bwd_dq_kernel, whole backward: B1 H12 L32760 with 25 key blocks 891 -> 673 us, B1 H16 L16380 with
 // 128-row blocks 538 -> 442 us, B1 H16 L2000 59.5 -> 52.0 us.
 constexpr int DQ_STREAM_MAX_T = 2048;          // look-up rows longer than this take bwd_dq_kernel
