@@ -7,204 +7,17 @@
 //   da = dn S^T + dden z ; dS = a^T dn ; dz = sum_l dden a
 //   dc = v dS^T + dz ; dv = c dS ; dq = phi'(q) da ; dk = phi'(k) dc
 //
-// Kernels:
+// Kernels (linear_bwd_stream.h, linear_state.h):
 //   state build (shared with the forward) : S and z again from k, v
-//   rows   : per 32 queries on one wave: y^T, dy^T, dn^T, da^T on the MFMA in transposed form (per-query
-//            scalars stay per-lane), writes dq and the row-wise temporaries dn, y (16 bit) and dden
-//   states : streams q, dn, G, y once; dS and dW on the MFMA (operands read transposed from LDS),
-//            dz and db on the vector ALU; fp32 partials
-//   reduce : fixed-order sums of the partials -> dS (16 bit, both orientations), dz, per-head dW, db;
-//            a second small kernel adds the heads
-//   kv     : per 32 keys on one wave: dc^T = dS v^T + dz, dv^T = dS^T c^T, dk = phi'(k) dc
+//   stream : q and G once: dq, and per slice of the sequence the partial sums M^T, dz, db
+//   finish : those sums added up -> dS (16 bit, both orientations), dz, per-head dW, db
+//   heads  : the heads' dW and db added up
+//   keys   : k and v once: dk, dv
+// The complement-mode branch forms dW and db with the states / reduce kernels below, from row-wise temporaries.
 #include "bwd_steps.h"
 #include "linear_bwd_stream.h"
 
 namespace sla {
-
-// ---- rows ---------------------------------------------------------------------------------
-// grid (ceil(L / (32*NW*tiles)), BH), NW waves of 32 queries each.  Inputs and outputs move through a
-// wave-private LDS staging tile so that global traffic is whole 256-byte rows; the next tile's q and G
-// rows are fetched into registers while the current tile is computed.
-template <typename Tag, int D, int NW>
-__global__ __launch_bounds__(64 * NW) void linear_bwd_rows_kernel(
-    const uint16_t* __restrict__ q, const uint16_t* __restrict__ gout, const uint16_t* __restrict__ kvt,
-    const uint16_t* __restrict__ kvp, const uint16_t* __restrict__ z, const uint16_t* __restrict__ wt,
-    uint16_t* __restrict__ dq, const RowLayout lin, const RowLayout ldo, uint16_t* __restrict__ dn_out,
-    uint16_t* __restrict__ y_out, float* __restrict__ dden_out, int L, int fmap, int tiles_per_wg, int accumulate) {
-  using E = Elem<Tag>;
-  constexpr int DC = D / 16;
-  constexpr int DT = D / 32;
-  constexpr int STR = D + 8;
-  __shared__ __attribute__((aligned(16))) uint16_t sKVT[D * STR];  // [d2][d1]          A of n^T = KVT a^T
-  __shared__ __attribute__((aligned(16))) uint16_t sKVP[D * STR];  // [d1][perm d2]     A of da^T = S dn^T
-  __shared__ __attribute__((aligned(16))) uint16_t sWT[D * STR];   // [d][e]            A of dy^T = W^T G^T
-  __shared__ __attribute__((aligned(16))) uint16_t sStage[NW][32 * STR];
-  __shared__ __attribute__((aligned(16))) float sZ[D];
-
-  const int bh = blockIdx.y;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int g = lane >> 5, r = lane & 31;
-
-  {
-    // all three operand matrices arrive in 16 bit and in the layout their MFMA reads want
-    const uint16_t* src = kvt + (size_t)bh * D * D;
-    const uint16_t* srcp = kvp + (size_t)bh * D * D;
-    for (int idx = tid; idx < D * D / 8; idx += 64 * NW) {
-      const int row = idx / (D / 8), col = (idx % (D / 8)) * 8;
-      *reinterpret_cast<i16x8_t*>(&sKVT[row * STR + col]) = *reinterpret_cast<const i16x8_t*>(src + (size_t)row * D + col);
-      *reinterpret_cast<i16x8_t*>(&sKVP[row * STR + col]) = *reinterpret_cast<const i16x8_t*>(srcp + (size_t)row * D + col);
-      *reinterpret_cast<i16x8_t*>(&sWT[row * STR + col]) = *reinterpret_cast<const i16x8_t*>(wt + (size_t)row * D + col);
-    }
-    if (tid < D) sZ[tid] = E::to_float(z[(size_t)bh * D + tid]);
-  }
-  __syncthreads();
-
-  // q and dq rows lie lin.sl elements apart, the rows of G ldo.sl; the temporaries dn, y are contiguous
-  const size_t head_off = (size_t)bh * L * D;
-  const size_t head_in = lin.head(bh), head_g = ldo.head(bh);
-  const size_t pitch = (size_t)lin.sl, pitch_g = (size_t)ldo.sl;
-  uint16_t* stage = sStage[wave];
-  constexpr int STEP = 32 * NW;
-  const int first_row = blockIdx.x * tiles_per_wg * STEP + wave * 32;
-  TileRows<D> qt, gt;                  // q and G rows of the tile about to be processed
-  if (first_row < L) {
-    qt.fetch(q + head_in + (size_t)first_row * pitch, min(32, L - first_row), lane, pitch);
-    gt.fetch(gout + head_g + (size_t)first_row * pitch_g, min(32, L - first_row), lane, pitch_g);
-  }
-  for (int tt = 0; tt < tiles_per_wg; ++tt) {
-    const int row0 = first_row + tt * STEP;
-    if (row0 >= L) break;
-    const int rows_valid = min(32, L - row0);
-    const int qrow = row0 + r;
-    const bool ok = qrow < L;
-    const size_t toff = head_off + (size_t)row0 * D;
-    const size_t toff_in = head_in + (size_t)row0 * pitch;
-
-    // q in B-operand order (d = 16c + 8g + j) and in accumulator order (d = 32t + 8i4 + 4g + j)
-    qt.park(stage, lane);
-    float f[DC][8];
-#pragma unroll
-    for (int c = 0; c < DC; ++c) {
-      const i16x8_t x = *reinterpret_cast<const i16x8_t*>(&stage[r * STR + 16 * c + 8 * g]);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) f[c][j] = E::to_float((uint16_t)x[j]);
-    }
-    i32x2_t xraw[DT][4];
-#pragma unroll
-    for (int t1 = 0; t1 < DT; ++t1)
-#pragma unroll
-      for (int i4 = 0; i4 < 4; ++i4)
-        xraw[t1][i4] = *reinterpret_cast<const i32x2_t*>(&stage[r * STR + 32 * t1 + 8 * i4 + 4 * g]);
-    wave_lds_fence();
-    gt.park(stage, lane);
-    i16x8_t gf[DC];
-#pragma unroll
-    for (int c = 0; c < DC; ++c) gf[c] = *reinterpret_cast<const i16x8_t*>(&stage[r * STR + 16 * c + 8 * g]);
-    wave_lds_fence();
-    TileRows<D> dq_old;
-    if (accumulate) dq_old.fetch(dq + toff_in, rows_valid, lane, pitch);
-    if (tt + 1 < tiles_per_wg && row0 + STEP < L) {
-      qt.fetch(q + toff_in + (size_t)STEP * pitch, min(32, L - row0 - STEP), lane, pitch);
-      gt.fetch(gout + head_g + (size_t)(row0 + STEP) * pitch_g, min(32, L - row0 - STEP), lane, pitch_g);
-    }
-
-    float row_mx, row_inv;
-    phi_row_pair<Tag, DC>(fmap, f, row_mx, row_inv);
-    float den = 0.f;
-    i16x8_t af[DC];
-#pragma unroll
-    for (int c = 0; c < DC; ++c) {
-      i32x4_t pw;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) den += f[c][j] * sZ[16 * c + 8 * g + j];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) pw[j] = (int)E::pack2(f[c][2 * j], f[c][2 * j + 1]);
-      af[c] = __builtin_bit_cast(i16x8_t, pw);
-    }
-    den += __shfl_xor(den, 32);
-    den += 1e-5f;
-    const float inv_den = 1.0f / den;
-
-    // y^T = (KVT a^T) / den ; dy^T = W^T G^T
-    float yv[DT][16], dnv[DT][16];
-#pragma unroll
-    for (int t = 0; t < DT; ++t) {
-      f32x16_t yacc, dyacc;
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        yacc[i] = 0.f;
-        dyacc[i] = 0.f;
-      }
-#pragma unroll
-      for (int c = 0; c < DC; ++c) {
-        const i16x8_t a1 = *reinterpret_cast<const i16x8_t*>(&sKVT[(32 * t + r) * STR + 16 * c + 8 * g]);
-        yacc = E::mfma32(a1, af[c], yacc);
-        const i16x8_t a2 = *reinterpret_cast<const i16x8_t*>(&sWT[(32 * t + r) * STR + 16 * c + 8 * g]);
-        dyacc = E::mfma32(a2, gf[c], dyacc);
-      }
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        yv[t][i] = yacc[i];
-        dnv[t][i] = dyacc[i];
-      }
-    }
-    float dden = 0.f;
-#pragma unroll
-    for (int t = 0; t < DT; ++t)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        yv[t][i] *= inv_den;
-        dden += dnv[t][i] * yv[t][i];
-        dnv[t][i] *= inv_den;          // dn^T
-      }
-    dden += __shfl_xor(dden, 32);
-    dden = -dden * inv_den;
-    if (ok && g == 0) dden_out[(size_t)bh * L + qrow] = dden;
-
-    // dn^T as B operand (register 8c2+j of tile t is d2 = 32t + 8*((8c2+j)/4) + 4g + j%4, the order sKVP's
-    // columns are stored in); dn and y go to memory for the state kernel
-    i16x8_t dnf[DT][2];
-#pragma unroll
-    for (int t = 0; t < DT; ++t)
-#pragma unroll
-      for (int c2 = 0; c2 < 2; ++c2) {
-        i32x4_t pw;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) pw[j] = (int)E::pack2(dnv[t][8 * c2 + 2 * j], dnv[t][8 * c2 + 2 * j + 1]);
-        dnf[t][c2] = __builtin_bit_cast(i16x8_t, pw);
-      }
-    store_acc_tile<E, D>(stage, dnv, dn_out + toff, nullptr, rows_valid, lane);
-    store_acc_tile<E, D>(stage, yv, y_out + toff, nullptr, rows_valid, lane);
-
-    // da^T = S dn^T + z dden
-    float da[DT][16], xq[DT][16];
-#pragma unroll
-    for (int t1 = 0; t1 < DT; ++t1) {
-      f32x16_t acc;
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc[i] = 0.f;
-#pragma unroll
-      for (int t = 0; t < DT; ++t)
-#pragma unroll
-        for (int c2 = 0; c2 < 2; ++c2) {
-          const i16x8_t a = *reinterpret_cast<const i16x8_t*>(&sKVP[(32 * t1 + r) * STR + 16 * (2 * t + c2) + 8 * g]);
-          acc = E::mfma32(a, dnf[t][c2], acc);
-        }
-#pragma unroll
-      for (int i4 = 0; i4 < 4; ++i4) {
-        const int d0 = 32 * t1 + 8 * i4 + 4 * g;
-        const uint16_t* xp = reinterpret_cast<const uint16_t*>(&xraw[t1][i4]);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          da[t1][4 * i4 + j] = acc[4 * i4 + j] + sZ[d0 + j] * dden;
-          xq[t1][4 * i4 + j] = E::to_float(xp[j]);
-        }
-      }
-    }
-    phi_backward<DT>(fmap, xq, da, row_mx, row_inv);
-    store_acc_tile<E, D>(stage, da, dq + toff_in, accumulate ? &dq_old : nullptr, rows_valid, lane, pitch);
-  }
-}
 
 // ---- states -------------------------------------------------------------------------------
 // grid (nsplit, BH).  dS^T partial [d2][d1] per (bh, split); dW^T partial [d][e] per (bh, split).
@@ -450,157 +263,20 @@ __global__ __launch_bounds__(256) void linear_bwd_reduce_heads_kernel(const floa
   }
 }
 
-// ---- kv -----------------------------------------------------------------------------------
-// Same tile traffic as the rows kernel: NW waves of 32 keys, whole-row global accesses through a
-// wave-private staging tile.
-// CONTIG: k, v, dk, dv are contiguous (B, H, L, D): the row pitch is the compile-time D.
-template <typename Tag, int D, int NW, bool CONTIG>
-__global__ __launch_bounds__(64 * NW) void linear_bwd_kv_kernel(const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
-                                                                const uint16_t* __restrict__ ds,
-                                                                const uint16_t* __restrict__ dst, const float* __restrict__ dz,
-                                                                uint16_t* __restrict__ dk, uint16_t* __restrict__ dv,
-                                                                const RowLayout lin, int L, int fmap, int tiles_per_wg,
-                                                                int accumulate) {
-  using E = Elem<Tag>;
-  constexpr int DC = D / 16;
-  constexpr int DT = D / 32;
-  constexpr int STR = D + 8;
-  __shared__ __attribute__((aligned(16))) uint16_t sDS[D * STR];   // [d1][d2]  A of dc^T = dS v^T
-  __shared__ __attribute__((aligned(16))) uint16_t sDST[D * STR];  // [d2][d1]  A of dv^T = dS^T c^T
-  __shared__ __attribute__((aligned(16))) uint16_t sStage[NW][32 * STR];
-  __shared__ __attribute__((aligned(16))) float sDZ[D];
-
-  const int bh = blockIdx.y;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int g = lane >> 5, r = lane & 31;
-  for (int idx = tid; idx < D * D / 8; idx += 64 * NW) {
-    const int row = idx / (D / 8), col = (idx % (D / 8)) * 8;
-    *reinterpret_cast<i16x8_t*>(&sDS[row * STR + col]) =
-        *reinterpret_cast<const i16x8_t*>(ds + (size_t)bh * D * D + (size_t)row * D + col);
-    *reinterpret_cast<i16x8_t*>(&sDST[row * STR + col]) =
-        *reinterpret_cast<const i16x8_t*>(dst + (size_t)bh * D * D + (size_t)row * D + col);
-  }
-  if (tid < D) sDZ[tid] = dz[(size_t)bh * D + tid];
-  __syncthreads();
-
-  const size_t head_off = lin.head(bh);   // k, v, dk, dv rows: lin.sl elements apart
-  const size_t pitch = CONTIG ? (size_t)D : (size_t)lin.sl;
-  uint16_t* stage = sStage[wave];
-  constexpr int STEP = 32 * NW;
-  const int first_row = blockIdx.x * tiles_per_wg * STEP + wave * 32;
-  for (int tt = 0; tt < tiles_per_wg; ++tt) {
-    const int row0 = first_row + tt * STEP;
-    if (row0 >= L) break;
-    const int rows_valid = min(32, L - row0);
-    const size_t toff = head_off + (size_t)row0 * pitch;
-
-    // two waves share a SIMD and cover each other's load latency; registers are too scarce to fetch ahead
-    TileRows<D> kt, vt;
-    kt.fetch(k + toff, rows_valid, lane, pitch);
-    vt.fetch(v + toff, rows_valid, lane, pitch);
-    kt.park(stage, lane);
-    float f[DC][8];
-#pragma unroll
-    for (int c = 0; c < DC; ++c) {
-      const i16x8_t x = *reinterpret_cast<const i16x8_t*>(&stage[r * STR + 16 * c + 8 * g]);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) f[c][j] = E::to_float((uint16_t)x[j]);
-    }
-    i32x2_t xraw[DT][4];
-#pragma unroll
-    for (int t = 0; t < DT; ++t)
-#pragma unroll
-      for (int i4 = 0; i4 < 4; ++i4)
-        xraw[t][i4] = *reinterpret_cast<const i32x2_t*>(&stage[r * STR + 32 * t + 8 * i4 + 4 * g]);
-    wave_lds_fence();
-    vt.park(stage, lane);
-    i16x8_t vf[DC];
-#pragma unroll
-    for (int c = 0; c < DC; ++c) vf[c] = *reinterpret_cast<const i16x8_t*>(&stage[r * STR + 16 * c + 8 * g]);
-    wave_lds_fence();
-    float row_mx, row_inv;
-    phi_row_pair<Tag, DC>(fmap, f, row_mx, row_inv);
-    {
-      // dv^T = dS^T c^T
-      i16x8_t cf[DC];
-#pragma unroll
-      for (int c = 0; c < DC; ++c) {
-        i32x4_t pw;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) pw[j] = (int)E::pack2(f[c][2 * j], f[c][2 * j + 1]);
-        cf[c] = __builtin_bit_cast(i16x8_t, pw);
-      }
-      float dvv[DT][16];
-#pragma unroll
-      for (int t = 0; t < DT; ++t) {
-        f32x16_t vacc;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) vacc[i] = 0.f;
-#pragma unroll
-        for (int c = 0; c < DC; ++c) {
-          const i16x8_t a2 = *reinterpret_cast<const i16x8_t*>(&sDST[(32 * t + r) * STR + 16 * c + 8 * g]);
-          vacc = E::mfma32(a2, cf[c], vacc);
-        }
-#pragma unroll
-        for (int i = 0; i < 16; ++i) dvv[t][i] = vacc[i];
-      }
-      if (accumulate)
-        store_acc_tile<E, D, true>(stage, dvv, dv + toff, nullptr, rows_valid, lane, pitch);
-      else
-        store_acc_tile<E, D, false>(stage, dvv, dv + toff, nullptr, rows_valid, lane, pitch);
-    }
-    // dc^T = dS v^T + dz ; dk = phi'(k) dc
-    float dc[DT][16], xk[DT][16];
-#pragma unroll
-    for (int t = 0; t < DT; ++t) {
-      f32x16_t acc;
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc[i] = 0.f;
-#pragma unroll
-      for (int c = 0; c < DC; ++c) {
-        const i16x8_t a1 = *reinterpret_cast<const i16x8_t*>(&sDS[(32 * t + r) * STR + 16 * c + 8 * g]);
-        acc = E::mfma32(a1, vf[c], acc);
-      }
-#pragma unroll
-      for (int i4 = 0; i4 < 4; ++i4) {
-        const int d0 = 32 * t + 8 * i4 + 4 * g;
-        const uint16_t* xp = reinterpret_cast<const uint16_t*>(&xraw[t][i4]);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          dc[t][4 * i4 + j] = acc[4 * i4 + j] + sDZ[d0 + j];
-          xk[t][4 * i4 + j] = E::to_float(xp[j]);
-        }
-      }
-    }
-    phi_backward<DT>(fmap, xk, dc, row_mx, row_inv);
-    if (accumulate)
-      store_acc_tile<E, D, true>(stage, dc, dk + toff, nullptr, rows_valid, lane, pitch);
-    else
-      store_acc_tile<E, D, false>(stage, dc, dk + toff, nullptr, rows_valid, lane, pitch);
-  }
-}
-
 // ---- host ---------------------------------------------------------------------------------
 struct LinBwdWs {
   LinWs fwd;
-  LinSplit st;   // slices of the states kernel (two workgroups per compute unit)
-  LinSplit ss;   // slices of the stream kernel (one workgroup per compute unit, 128 rows per step): never more than st's
-  size_t dn, y, dden, ds_part, dw_part, dz_part, db_part, ds, dst, dz, dw_head, db_head, total;
+  LinSplit sp;   // slices of the stream and keys kernels (128 rows per step)
+  size_t m_part, dz_part, db_part, ds, dst, dz, dw_head, db_head, total;
 };
-// (own_states = false: the forward's states lie elsewhere, the workspace holds none.  Head dim 128 has no row-wise temporaries.)
+// (own_states = false: the forward's states lie elsewhere, the workspace holds none)
 static LinBwdWs lin_bwd_ws(int BH, int L, int D, bool own_states) {
   LinBwdWs w;
   w.fwd = lin_ws(BH, L, D);
-  w.st = lin_split(BH, L, 512);
-  w.ss = lin_split(BH, L, 256, LBS_TR);
-  const int64_t np = (int64_t)BH * w.st.nsplit;
+  w.sp = lin_split(BH, L, D == 128 ? 256 : 512, LBS_TR);       // (one workgroup per compute unit at head dim 128, two at 64)
+  const int64_t np = (int64_t)BH * w.sp.nsplit;
   size_t off = own_states ? w.fwd.total : 0;
-  const int64_t rows = D == 128 ? 0 : (int64_t)BH * L;
-  w.dn = off;      off += align_up(rows * D * 2, 256);
-  w.y = off;       off += align_up(rows * D * 2, 256);
-  w.dden = off;    off += align_up(rows * 4, 256);
-  w.ds_part = off; off += align_up(np * D * D * 4, 256);
-  w.dw_part = off; off += align_up(D == 128 ? 0 : np * D * D * 4, 256);
+  w.m_part = off;  off += align_up(np * D * D * 4, 256);
   w.dz_part = off; off += align_up(np * D * 4, 256);
   w.db_part = off; off += align_up(np * D * 4, 256);
   w.ds = off;      off += align_up((int64_t)BH * D * D * 2, 256);
@@ -618,88 +294,48 @@ template <typename Tag, int D>
 static int linear_bwd_impl(const void* q, const void* k, const void* v, const float* weight, const void* d_out, void* dq,
                            void* dk, void* dv, const RowLayout& lin, const RowLayout& ldo, float* d_weight, float* d_bias,
                            int fmap, int BH, int L, int flags, const char* states, char* ws, hipStream_t st, int steps) {
-  // (the kernels of head dim 128 address a head's rows through 32-bit buffer offsets; make_layout asks for more)
-  const auto fits32 = [&](const RowLayout& lay) { return ((int64_t)(L - 1) * lay.sl + D) * 2 < ((int64_t)1 << 32); };
-  if constexpr (D == 128)
-    SLA_REQUIRE(fits32(lin) && fits32(ldo), SLA_ERR_UNSUPPORTED, "one head spans 4 GiB or more");
   if (steps == 0) return SLA_OK;        // (arguments checked, nothing asked for)
   const LinBwdWs w = lin_bwd_ws(BH, L, D, !states);
   const int accumulate = flags & SLA_BWD_ACCUMULATE;
   if ((steps & LB_STATES) && !states && !(flags & SLA_BWD_STATES_READY)) {
-    // everything the forward's state build leaves: transposed state, z, and (fold) the folded state + 16-bit weight
+    // everything the forward's state build leaves: transposed state, z, and (fold) the folded state
     launch_state_build<Tag, D>(k, v, lin, weight, fmap, BH, L, ws, ws + w.fwd.states_end, w.fwd, st);
   }
   if (!states) states = ws;
   const uint16_t* kvt = (const uint16_t*)(states + w.fwd.kvt);
   const uint16_t* z = (const uint16_t*)(states + w.fwd.z);
-  constexpr int NW_ROWS = 4, NW_KV = 8;   // one workgroup per compute unit either way (LDS)
-  if constexpr (D == 128) {
-    // q and G once: dq, and the partial sums M^T, dz, db of every slice (M^T's take the place of the general path's ds_part)
-    float* m_part = (float*)(ws + w.ds_part);
-    if (steps & LB_QUERY) {
+  float* m_part = (float*)(ws + w.m_part);
+  if (steps & LB_QUERY) {
 #define SLA_LBS_LAUNCH(FM)                                                                                                  \
-  hipLaunchKernelGGL((linear_bwd_stream_kernel<Tag, FM>), dim3(w.ss.nsplit, BH), dim3(512), 0, st, (const uint16_t*)q,        \
-                     (const uint16_t*)d_out, (const uint16_t*)(states + w.fwd.kvwt), z, (uint16_t*)dq, lin, ldo, m_part,          \
-                     (float*)(ws + w.dz_part), (float*)(ws + w.db_part), L, w.ss.rows_per_split, accumulate)
+  hipLaunchKernelGGL((linear_bwd_stream_kernel<Tag, D, FM>), dim3(w.sp.nsplit, BH), dim3(512), 0, st, (const uint16_t*)q,     \
+                     (const uint16_t*)d_out, (const uint16_t*)(states + w.fwd.kvw), z, (uint16_t*)dq, lin, ldo, m_part,          \
+                     (float*)(ws + w.dz_part), (float*)(ws + w.db_part), L, w.sp.rows_per_split, accumulate)
     if (fmap == SLA_FMAP_ELU) SLA_LBS_LAUNCH(SLA_FMAP_ELU);
     else if (fmap == SLA_FMAP_RELU) SLA_LBS_LAUNCH(SLA_FMAP_RELU);
     else SLA_LBS_LAUNCH(SLA_FMAP_SOFTMAX);
 #undef SLA_LBS_LAUNCH
-    }
-    if (steps & LB_REDUCE) {
+  }
+  if (steps & LB_REDUCE) {
 #define SLA_LBF_LAUNCH(HALVES)                                                                                               \
   hipLaunchKernelGGL((linear_bwd_finish_kernel<Tag, D, HALVES>), dim3(xcd_grid((int64_t)BH * (D / 8))), dim3(256 * HALVES), 0, \
                      st, (const float*)m_part, (const float*)(ws + w.dz_part), (const float*)(ws + w.db_part), weight, kvt,   \
                      (uint16_t*)(ws + w.ds), (uint16_t*)(ws + w.dst), (float*)(ws + w.dz), (float*)(ws + w.dw_head),           \
-                     (float*)(ws + w.db_head), w.ss.nsplit, BH * (D / 8))
+                     (float*)(ws + w.db_head), w.sp.nsplit, BH * (D / 8))
     if (steps & LB_BESIDE) SLA_LBF_LAUNCH(1);
     else SLA_LBF_LAUNCH(2);
 #undef SLA_LBF_LAUNCH
-    }
-  } else {
-  uint16_t* dn = (uint16_t*)(ws + w.dn);
-  uint16_t* y = (uint16_t*)(ws + w.y);
-  float* dden = (float*)(ws + w.dden);
-  const int tiles_rows = balanced_tiles(cdiv(L, 32 * NW_ROWS), BH, 1);
-  if (steps & LB_QUERY) {
-  hipLaunchKernelGGL((linear_bwd_rows_kernel<Tag, D, NW_ROWS>), dim3(cdiv(L, 32 * NW_ROWS * tiles_rows), BH), dim3(64 * NW_ROWS), 0, st, (const uint16_t*)q,
-                     (const uint16_t*)d_out, kvt, (const uint16_t*)(states + w.fwd.kvp), z, (const uint16_t*)(states + w.fwd.wt), (uint16_t*)dq, lin, ldo, dn, y,
-                     dden, L, fmap, tiles_rows, accumulate);
-  hipLaunchKernelGGL((linear_bwd_states_kernel<Tag, D>), dim3(w.st.nsplit, BH), dim3(256), 0, st, (const uint16_t*)q, dn,
-                     (const uint16_t*)d_out, y, dden, lin, ldo, (float*)(ws + w.ds_part), (float*)(ws + w.dw_part),
-                     (float*)(ws + w.dz_part), (float*)(ws + w.db_part), L, w.st.rows_per_split, fmap);
-  }
-  if (steps & LB_REDUCE)
-  hipLaunchKernelGGL((linear_bwd_reduce_kernel<Tag>), dim3(cdiv(D * D, 256), BH), dim3(256), 0, st,
-                     (const float*)(ws + w.ds_part), (const float*)(ws + w.dw_part), (const float*)(ws + w.dz_part),
-                     (const float*)(ws + w.db_part), (uint16_t*)(ws + w.ds), (uint16_t*)(ws + w.dst), (float*)(ws + w.dz),
-                     (float*)(ws + w.dw_head), (float*)(ws + w.db_head), w.st.nsplit, D);
-  }
-  if (steps & LB_REDUCE)
     hipLaunchKernelGGL(linear_bwd_reduce_heads_kernel, dim3(cdiv(D * D, 256)), dim3(256), 0, st,
                        (const float*)(ws + w.dw_head), (const float*)(ws + w.db_head), d_weight, d_bias, BH, D);
-  if (!(steps & LB_KEYS)) return check_launch("linear_bwd");
-  if constexpr (D == 128) {
+  }
+  if (steps & LB_KEYS) {
 #define SLA_LBK_LAUNCH(FM)                                                                                                \
-  hipLaunchKernelGGL((linear_bwd_keys_kernel<Tag, FM>), dim3(w.ss.nsplit, BH), dim3(512), 0, st, (const uint16_t*)k,        \
+  hipLaunchKernelGGL((linear_bwd_keys_kernel<Tag, D, FM>), dim3(w.sp.nsplit, BH), dim3(512), 0, st, (const uint16_t*)k,     \
                      (const uint16_t*)v, (const uint16_t*)(ws + w.ds), (const uint16_t*)(ws + w.dst),                       \
-                     (const float*)(ws + w.dz), (uint16_t*)dk, (uint16_t*)dv, lin, L, w.ss.rows_per_split, accumulate)
+                     (const float*)(ws + w.dz), (uint16_t*)dk, (uint16_t*)dv, lin, L, w.sp.rows_per_split, accumulate)
     if (fmap == SLA_FMAP_ELU) SLA_LBK_LAUNCH(SLA_FMAP_ELU);
     else if (fmap == SLA_FMAP_RELU) SLA_LBK_LAUNCH(SLA_FMAP_RELU);
     else SLA_LBK_LAUNCH(SLA_FMAP_SOFTMAX);
 #undef SLA_LBK_LAUNCH
-  } else {
-  const int tiles_kv = balanced_tiles(cdiv(L, 32 * NW_KV), BH, 1);
-  if (lin.sl == D)
-    hipLaunchKernelGGL((linear_bwd_kv_kernel<Tag, D, NW_KV, true>), dim3(cdiv(L, 32 * NW_KV * tiles_kv), BH), dim3(64 * NW_KV),
-                       0, st, (const uint16_t*)k, (const uint16_t*)v, (const uint16_t*)(ws + w.ds),
-                       (const uint16_t*)(ws + w.dst), (const float*)(ws + w.dz), (uint16_t*)dk, (uint16_t*)dv, lin, L, fmap,
-                       tiles_kv, accumulate);
-  else
-    hipLaunchKernelGGL((linear_bwd_kv_kernel<Tag, D, NW_KV, false>), dim3(cdiv(L, 32 * NW_KV * tiles_kv), BH), dim3(64 * NW_KV),
-                       0, st, (const uint16_t*)k, (const uint16_t*)v, (const uint16_t*)(ws + w.ds),
-                       (const uint16_t*)(ws + w.dst), (const float*)(ws + w.dz), (uint16_t*)dk, (uint16_t*)dv, lin, L, fmap,
-                       tiles_kv, accumulate);
   }
   return check_launch("linear_bwd");
 }

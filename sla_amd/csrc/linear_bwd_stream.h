@@ -1,4 +1,4 @@
-// Backward of the linear-attention branch + projection, query side, for head dim 128: one pass over q and G = d(out).
+// Backward of the linear-attention branch + projection, query side: one pass over q and G = d(out).
 //
 // With a = phi(q), S = phi(k)^T v, z = sum phi(k), den = 1e-5 + a.z, P = S W^T (the folded state of the forward,
 // core.py:90-99 of the reference) the branch is out = a P / den + b, so per query row
@@ -6,14 +6,16 @@
 //   dden = -(a.t) / den^2
 //   da   = t / den + dden z ;  dq = phi'(q) da
 // and the sums over the rows reduce to ONE D x D matrix and two vectors:
-//   M  = sum_l (a_l / den_l)^T G_l       ->  dS = M W,  dW = M^T S     (small products per head, formed afterwards)
+//   M  = sum_l a_l^T G_l / den_l         ->  dS = M W,  dW = M^T S     (small products per head, formed afterwards)
 //   dz = sum_l dden_l a_l ;  db = sum_l G_l
 // No row-wise temporary goes to memory: q and G are read once, dq is read (when accumulating) and written once.
 //
 //   stream   : grid (slices of L, heads), 8 waves.  Per 128 rows: every wave takes 16 rows through t, dden, da, dq
-//              (16x16x32 products, the row spread over 4 lanes), leaves a/den and dq in LDS; then the workgroup adds the
-//              tile's (a/den)^T G to M (32x32x16 products, both operands read transposed from LDS), dz and db on the
-//              vector ALU, and writes the dq rows whole.
+//              (16x16x32 products, the row spread over 4 lanes), leaves the weighted rows and dq in LDS; then the workgroup
+//              adds the tile's product to M (both operands read transposed from LDS), dz and db on the vector ALU, and
+//              writes the dq rows whole.
+//   The factor 1/den goes, with one rounding to 16 bit, to a at head dim 128 and to G at head dim 64: there a stays the 16-bit
+//   value it is, and in half precision G / den keeps its bits on long sequences, where a / den falls below the format's normal range.
 //   finish   : fixed-order sums of the slices' partials -> M^T (fp32), dz, db per head, and from them
 //              dS = M W (16 bit, both orientations) and this head's dW = M^T S (fp32)
 #pragma once
@@ -23,65 +25,57 @@ namespace sla {
 
 // LDS tiles of 256-byte rows without padding: 16-byte piece p of row r sits at piece slot p ^ swz(r).  Row-wise
 // 16-byte / 8-byte reads by 16 consecutive rows and transposing reads of 4 rows x 4 pieces both touch every bank once.
-static __device__ __forceinline__ int lbs_swz(int row) { return ((row & 3) << 2) | ((row >> 2) & 3); }
+// Rows of 128 bytes (head dim 64): a line of all banks holds two of them, so the swizzle counts pairs of rows.
+template <int D>
+static __device__ __forceinline__ int lbs_swz(int row) {
+  return D == 128 ? ((row & 3) << 2) | ((row >> 2) & 3) : ((row & 2) << 1) | ((row >> 2) & 3);
+}
+template <int D>
 static __device__ __forceinline__ uint32_t lbs_off(int row, int col) {
-  return (uint32_t)row * 256u + (uint32_t)(((col >> 3) ^ lbs_swz(row & 15)) << 4) + (uint32_t)(col & 7) * 2u;
+  return (uint32_t)row * (2u * D) + (uint32_t)(((col >> 3) ^ lbs_swz<D>(row & 15)) << 4) + (uint32_t)(col & 7) * 2u;
 }
 
 constexpr int LBS_TR = 128;   // rows per step of the stream kernel
 
-template <typename Tag, int FMAP>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void linear_bwd_stream_kernel(
-    const uint16_t* __restrict__ q, const uint16_t* __restrict__ gout, const uint16_t* __restrict__ kvwt,
+// Head dim 64 keeps half the registers and 60 KB of LDS, so two workgroups share a compute unit.  Against kernels with
+// row-wise temporaries (dn, y, dden) in memory, the backward of 16 heads x 6001 x 64, softmax map in half precision: rows 20.8 +
+// states 16.3 + sums 14.1 + heads 5.4 + keys 21.2 us; now stream 20.5 + finish 5.8 + heads 5.1 + keys 16.4.
+template <typename Tag, int D, int FMAP>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 128 ? 2 : 4, D == 128 ? 2 : 4))) void linear_bwd_stream_kernel(
+    const uint16_t* __restrict__ q, const uint16_t* __restrict__ gout, const uint16_t* __restrict__ kvw,
     const uint16_t* __restrict__ z, uint16_t* __restrict__ dq, const RowLayout lin, const RowLayout ldo,
     float* __restrict__ m_part, float* __restrict__ dz_part, float* __restrict__ db_part, int L, int rows_per_split,
     int accumulate) {
   // (the feature map is a template argument: as a run-time value every element's phi sits behind its own branch)
   using E = Elem<Tag>;
   constexpr int fmap = FMAP;
-  constexpr int D = 128, TR = LBS_TR;
+  constexpr int TR = LBS_TR;
   constexpr int TILE = TR * D * 2;               // bytes of one swizzled tile of rows
+  constexpr int CPR = D / 8;                     // 16-byte pieces per row
+  constexpr int RPP = 512 / CPR, NP = TR / RPP;  // rows per pass of the workgroup, passes per tile
+  constexpr int NF = CPR / 4;                    // passes of a wave over its own 16 rows
+  constexpr int NT = D / 16, NC = D / 32;        // 16-column tiles of a row, 32-column fragments
+  constexpr bool WEIGHT_G = D == 64;             // 1 / den goes to G, not to a
   constexpr int PSTR = D * 2 + 16;               // row pitch of sP: 16 rows x 16 bytes of a row-wise read cover every bank
-  __shared__ __attribute__((aligned(16))) char smem[3 * TILE + D * PSTR + 2 * D * 4];
-  char* const sQ = smem;                         // raw q rows, then a/den of the same rows
-  char* const sG = smem + TILE;                  // G rows
+  __shared__ __attribute__((aligned(16))) char smem[3 * TILE + D * PSTR + 2 * TR * 4];
+  char* const sQ = smem;                         // raw q rows, then a (/ den) of the same rows
+  char* const sG = smem + TILE;                  // G rows (then G / den)
   char* const sO = smem + 2 * TILE;              // dq rows of this step (16 bit)
   char* const sP = smem + 3 * TILE;              // folded state, P[d1][e]
   float* const sZ = reinterpret_cast<float*>(smem + 3 * TILE + D * PSTR);   // z[d1]
-  float* const sDD = sZ + D;                                                // dden * den per row of the step
-  float (*sRed)[32][D] = reinterpret_cast<float (*)[32][D]>(smem);          // final cross-thread sums (over sQ)
+  float* const sDD = sZ + TR;                                               // weight in dz of the row that sQ then holds
+  float (*sRed)[RPP][D] = reinterpret_cast<float (*)[RPP][D]>(smem);        // final cross-thread sums (over the tiles)
+  static_assert(2 * RPP * D * 4 <= 3 * TILE, "the final sums do not fit the tiles they reuse");
 
   const int split = blockIdx.x, bh = blockIdx.y, nsplit = gridDim.x;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int row_begin = split * rows_per_split;
   const int row_end = min(L, row_begin + rows_per_split);
-  // loader layout: thread = (row lrow + 32 p, 16-byte piece lp); + 8 KiB per p in a tile
-  const int lrow = tid >> 4, lp = tid & 15;
-  const uint32_t ld_off = lbs_off(lrow, 8 * lp);
+  // loader layout: thread = (row lrow + RPP p, 16-byte piece lp); + 8 KiB per p in a tile
+  const int lrow = tid / CPR, lp = tid % CPR;
+  const uint32_t ld_off = lbs_off<D>(lrow, 8 * lp);
   // row phase: lane = (row l of the wave's 16, quarter h): d1 = 16 T + 4 h + j
   const int l = lane & 15, h = lane >> 4;
-
-  {
-    // The folded state arrives as kvwt[e][d1]; the row phase wants rows of P[d1][e].  Through sQ: wave T turns the
-    // 16 columns d1 = 16 T .. of the staged copy into rows by transposing reads.
-    const uint16_t* src = kvwt + (size_t)bh * D * D;
-#pragma unroll
-    for (int p = 0; p < D / 32; ++p)
-      *reinterpret_cast<i16x8_t*>(sQ + ld_off + p * 8192) =
-          *reinterpret_cast<const i16x8_t*>(src + (size_t)(lrow + 32 * p) * D + 8 * lp);
-    if (tid < D) sZ[tid] = E::to_float(z[(size_t)bh * D + tid]);
-    __syncthreads();
-    const int pe = 8 * h + (l >> 2);      // rows e = 32 c + pe .. + 3 and + 4 .. + 7, columns 16 wave + 4 (l % 4) ..
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const uint16_t* p0 = reinterpret_cast<const uint16_t*>(sQ + lbs_off(32 * c + pe, 16 * wave + 4 * (l & 3)));
-      const uint16_t* p1 = reinterpret_cast<const uint16_t*>(sQ + lbs_off(32 * c + pe + 4, 16 * wave + 4 * (l & 3)));
-      // lane (l, h) now holds P[16 wave + l][32 c + 8 h .. + 7]
-      *reinterpret_cast<i16x8_t*>(sP + (16 * wave + l) * PSTR + (32 * c + 8 * h) * 2) =
-          concat4(lds_read_tr16(p0), lds_read_tr16(p1));
-    }
-    __syncthreads();
-  }
 
   const __amdgpu_buffer_rsrc_t q_rs = make_rsrc(q + lin.head(bh), lin.head_range_bytes(L, D));
   const __amdgpu_buffer_rsrc_t g_rs = make_rsrc(gout + ldo.head(bh), ldo.head_range_bytes(L, D));
@@ -91,23 +85,37 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const uint32_t pitch_b = (uint32_t)lin.sl * 2u, pitch_gb = (uint32_t)ldo.sl * 2u;
 
   // (rows past L lie outside the descriptors and read as zero: phi(0) meets G = 0 there and adds nothing)
-  i16x8_t rq[4], rg[4];
+  i16x8_t rq[NP], rg[NP];
   auto fetch_qg = [&](int r0) __attribute__((always_inline)) {
 #pragma unroll
-    for (int p = 0; p < 4; ++p) {
-      const uint32_t grow = (uint32_t)(r0 + lrow + 32 * p);
+    for (int p = 0; p < NP; ++p) {
+      const uint32_t grow = (uint32_t)(r0 + lrow + RPP * p);
       rq[p] = buf_load_b128(q_rs, grow * pitch_b + 16 * lp);
       rg[p] = buf_load_b128(g_rs, grow * pitch_gb + 16 * lp);
     }
   };
 
-  // M tiles of this wave: rows d1 = 32 mt .., columns e = 32 nt0 .. and 32 (nt0 + 1) ..
+  fetch_qg(row_begin);      // (on their way while the state is staged)
+  {
+    const uint16_t* src = kvw + (size_t)bh * D * D;
+#pragma unroll
+    for (int p = 0; p < D / RPP; ++p)
+      *reinterpret_cast<i16x8_t*>(sP + (lrow + RPP * p) * PSTR + 16 * lp) =
+          *reinterpret_cast<const i16x8_t*>(src + (size_t)(lrow + RPP * p) * D + 8 * lp);
+    if (tid < D) sZ[tid] = E::to_float(z[(size_t)bh * D + tid]);
+    // (the first step's barrier stands before the first read of either)
+  }
+
+  // M tiles of this wave, MW x MW: rows d1 = MW mt .., columns e = MW nt0 .. and MW (nt0 + 1) .. (32x32x16 products at head dim
+  // 128, 16x16x32 at 64)
+  constexpr int MW = D / 4, MR = MW * MW / 64;
+  typedef __attribute__((__vector_size__(MR * sizeof(float)))) float macc_t;
   const int mt = wave >> 1, nt0 = 2 * (wave & 1);
-  f32x16_t macc[2];
+  macc_t macc[2];
 #pragma unroll
   for (int t = 0; t < 2; ++t)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) macc[t][i] = 0.f;
+    for (int i = 0; i < MR; ++i) macc[t][i] = 0.f;
   float zacc[8], bacc[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
@@ -116,37 +124,39 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   }
 
   const int prow = 16 * wave + l;
-  uint32_t acc_off[8];        // (prow, 16 T + 4 h) in a row tile
+  uint32_t acc_off[NT];       // (prow, 16 T + 4 h) in a row tile
 #pragma unroll
-  for (int T = 0; T < 8; ++T) acc_off[T] = lbs_off(prow, 16 * T + 4 * h);
-  uint32_t g_off[4];          // (prow, 32 c + 8 h): G in B-operand order
+  for (int T = 0; T < NT; ++T) acc_off[T] = lbs_off<D>(prow, 16 * T + 4 * h);
+  uint32_t g_off[NC];         // (prow, 32 c + 8 h): G in B-operand order
 #pragma unroll
-  for (int c = 0; c < 4; ++c) g_off[c] = lbs_off(prow, 32 * c + 8 * h);
+  for (int c = 0; c < NC; ++c) g_off[c] = lbs_off<D>(prow, 32 * c + 8 * h);
   // A operand of t^T = P G^T: row d1 = 16 T + l of sP, e = 32 c + 8 h ..: + 16 PSTR per T, + 64 bytes per c
   const char* const p_base = sP + l * PSTR + h * 16;
-  // transposing reads of the M phase: rows 16 c + 8 g + (lane % 16) / 4 (+ 4), columns 32 tile + tr_col; + 4 KiB per c
+  // transposing reads of the M phase, KM rows per product: rows KM c + tr_row (+ 4), columns MW tile + tr_col; + 4 KiB per c
+  constexpr int KM = D == 128 ? 16 : 32;
   const int g2 = lane >> 5;
-  const int tr_row = 8 * g2 + ((lane & 15) >> 2);
-  const int tr_col = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+  const int tr_row = 8 * (D == 128 ? g2 : h) + ((lane & 15) >> 2);
+  const int tr_col = (D == 128 ? 16 * ((lane >> 4) & 1) : 0) + 4 * (lane & 3);
   uint32_t ma_off[2], mb_off[2][2];
 #pragma unroll
   for (int hf = 0; hf < 2; ++hf) {
-    ma_off[hf] = lbs_off(tr_row + 4 * hf, 32 * mt + tr_col);
+    ma_off[hf] = lbs_off<D>(tr_row + 4 * hf, MW * mt + tr_col);
 #pragma unroll
-    for (int t2 = 0; t2 < 2; ++t2) mb_off[hf][t2] = lbs_off(tr_row + 4 * hf, 32 * (nt0 + t2) + tr_col);
+    for (int t2 = 0; t2 < 2; ++t2) mb_off[hf][t2] = lbs_off<D>(tr_row + 4 * hf, MW * (nt0 + t2) + tr_col);
   }
 
-  // dq rows leave a step late, every wave writing the 16 rows it computed (4 rows x 256 bytes per instruction), so
+  // dq rows leave a step late, every wave writing the 16 rows it computed (whole rows, 1 KiB per instruction), so
   // that only the wave's own order of LDS accesses matters.
-  const int frow = 16 * wave + (lane >> 4);           // + 4 p
-  uint32_t f_off[4];
+  constexpr int FR = 64 / CPR;
+  const int frow = 16 * wave + lane / CPR;            // + FR p
+  uint32_t f_off[NF];
 #pragma unroll
-  for (int p = 0; p < 4; ++p) f_off[p] = lbs_off(frow + 4 * p, 8 * lp);
-  i16x8_t rdq[4];
+  for (int p = 0; p < NF; ++p) f_off[p] = lbs_off<D>(frow + FR * p, 8 * lp);
+  i16x8_t rdq[NF];
   auto flush_dq = [&](int r0) __attribute__((always_inline)) {
 #pragma unroll
-    for (int p = 0; p < 4; ++p) {
-      const int grow = r0 + frow + 4 * p;
+    for (int p = 0; p < NF; ++p) {
+      const int grow = r0 + frow + FR * p;
       const i16x8_t o16 = *reinterpret_cast<const i16x8_t*>(sO + f_off[p]);
       // (not accumulating: the descriptor is empty and rdq reads as zero; x + 0 keeps the 16-bit value)
       i32x4_t w;
@@ -159,11 +169,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     wave_lds_fence();     // the row phase rewrites these rows of sO
   };
 
-  fetch_qg(row_begin);
   for (int r0 = row_begin; r0 < row_end; r0 += TR) {
     // ---- tiles into LDS; db ----
 #pragma unroll
-    for (int p = 0; p < 4; ++p) {
+    for (int p = 0; p < NP; ++p) {
       const uint32_t o = ld_off + p * 8192;
       *reinterpret_cast<i16x8_t*>(sQ + o) = rq[p];
       *reinterpret_cast<i16x8_t*>(sG + o) = rg[p];
@@ -178,25 +187,25 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     // ---- row phase ----
     {
       // (the raw rows stay packed until phi' needs them again)
-      i16x4_t xraw[8];
+      i16x4_t xraw[NT];
 #pragma unroll
-      for (int T = 0; T < 8; ++T) xraw[T] = *reinterpret_cast<const i16x4_t*>(sQ + acc_off[T]);
+      for (int T = 0; T < NT; ++T) xraw[T] = *reinterpret_cast<const i16x4_t*>(sQ + acc_off[T]);
       auto xv = [&](int T, int j) __attribute__((always_inline)) { return E::to_float((uint16_t)xraw[T][j]); };
       float mx = 0.f, inv = 1.f, inv_den;
-      i32x2_t apk[8];         // a = phi(q), 16 bit (it is a 16-bit tensor in the reference)
+      i32x2_t apk[NT];         // a = phi(q), 16 bit (it is a 16-bit tensor in the reference)
       {
-        float a[8][4];
+        float a[NT][4];
         if (fmap == SLA_FMAP_SOFTMAX) {
           mx = xv(0, 0);
 #pragma unroll
-          for (int T = 0; T < 8; ++T)
+          for (int T = 0; T < NT; ++T)
 #pragma unroll
             for (int j = 0; j < 4; ++j) mx = fmaxf(mx, xv(T, j));
           mx = fmaxf(mx, __shfl_xor(mx, 16));
           mx = fmaxf(mx, __shfl_xor(mx, 32));
           float sum = 0.f;
 #pragma unroll
-          for (int T = 0; T < 8; ++T)
+          for (int T = 0; T < NT; ++T)
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
               a[T][j] = __expf(xv(T, j) - mx);
@@ -206,18 +215,18 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
           sum += __shfl_xor(sum, 32);
           inv = 1.0f / sum;
 #pragma unroll
-          for (int T = 0; T < 8; ++T)
+          for (int T = 0; T < NT; ++T)
 #pragma unroll
             for (int j = 0; j < 4; ++j) a[T][j] = round16<Tag>(a[T][j] * inv);
         } else {
 #pragma unroll
-          for (int T = 0; T < 8; ++T)
+          for (int T = 0; T < NT; ++T)
 #pragma unroll
             for (int j = 0; j < 4; ++j) a[T][j] = fmap_pointwise<Tag>(fmap, xv(T, j));
         }
         float den = 0.f;
 #pragma unroll
-        for (int T = 0; T < 8; ++T) {
+        for (int T = 0; T < NT; ++T) {
           const f32x4_t zz = *reinterpret_cast<const f32x4_t*>(sZ + 16 * T + 4 * h);
 #pragma unroll
           for (int j = 0; j < 4; ++j) den += a[T][j] * zz[j];
@@ -226,32 +235,40 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         den += __shfl_xor(den, 32);
         den += 1e-5f;
         inv_den = 1.0f / den;
-        // a/den takes the place of the raw row (this lane's own places)
+        // a or a/den takes the place of the raw row (this lane's own places)
+        const float aw = WEIGHT_G ? 1.0f : inv_den;
 #pragma unroll
-        for (int T = 0; T < 8; ++T) {
+        for (int T = 0; T < NT; ++T) {
           i32x2_t w;
-          w[0] = (int)E::pack2(a[T][0] * inv_den, a[T][1] * inv_den);
-          w[1] = (int)E::pack2(a[T][2] * inv_den, a[T][3] * inv_den);
+          w[0] = (int)E::pack2(a[T][0] * aw, a[T][1] * aw);
+          w[1] = (int)E::pack2(a[T][2] * aw, a[T][3] * aw);
           *reinterpret_cast<i32x2_t*>(sQ + acc_off[T]) = w;
           apk[T][0] = (int)E::pack2(a[T][0], a[T][1]);
           apk[T][1] = (int)E::pack2(a[T][2], a[T][3]);
         }
       }
 
-      // t^T = P G^T: 8 tiles of 16 d1 x 16 rows
-      f32x4_t t[8];
+      // t^T = P G^T: tiles of 16 d1 x 16 rows
+      f32x4_t t[NT];
 #pragma unroll
-      for (int T = 0; T < 8; ++T) t[T] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      for (int T = 0; T < NT; ++T) t[T] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
+      for (int c = 0; c < NC; ++c) {
         const i16x8_t b = *reinterpret_cast<const i16x8_t*>(sG + g_off[c]);
 #pragma unroll
-        for (int T = 0; T < 8; ++T)
+        for (int T = 0; T < NT; ++T)
           t[T] = E::mfma16(*reinterpret_cast<const i16x8_t*>(p_base + T * 16 * PSTR + c * 64), b, t[T]);
+        if (WEIGHT_G) {              // G / den over the same places (the row's four lanes hold all of it)
+          i32x4_t w;
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            w[j] = (int)E::pack2(E::to_float((uint16_t)b[2 * j]) * inv_den, E::to_float((uint16_t)b[2 * j + 1]) * inv_den);
+          *reinterpret_cast<i32x4_t*>(sG + g_off[c]) = w;
+        }
       }
       float s = 0.f;
 #pragma unroll
-      for (int T = 0; T < 8; ++T)
+      for (int T = 0; T < NT; ++T)
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const uint32_t w = (uint32_t)apk[T][j >> 1];
@@ -260,40 +277,40 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       s += __shfl_xor(s, 16);
       s += __shfl_xor(s, 32);
       const float dden = -s * inv_den * inv_den;
-      if (h == 0) sDD[prow] = -s * inv_den;     // dden * den: the weight of a/den in dz
+      if (h == 0) sDD[prow] = WEIGHT_G ? dden : -s * inv_den;     // the weight of what sQ holds (a, or a/den) in dz
 
       // da = t / den + dden z (in place), then dq = phi'(q) da
 #pragma unroll
-      for (int T = 0; T < 8; ++T) {
+      for (int T = 0; T < NT; ++T) {
         const f32x4_t zz = *reinterpret_cast<const f32x4_t*>(sZ + 16 * T + 4 * h);
 #pragma unroll
         for (int j = 0; j < 4; ++j) t[T][j] = __builtin_fmaf(t[T][j], inv_den, dden * zz[j]);
       }
       if (fmap == SLA_FMAP_RELU) {
 #pragma unroll
-        for (int T = 0; T < 8; ++T)
+        for (int T = 0; T < NT; ++T)
 #pragma unroll
           for (int j = 0; j < 4; ++j) t[T][j] = xv(T, j) > 0.f ? t[T][j] : 0.f;
       } else if (fmap == SLA_FMAP_ELU) {
 #pragma unroll
-        for (int T = 0; T < 8; ++T)
+        for (int T = 0; T < NT; ++T)
 #pragma unroll
           for (int j = 0; j < 4; ++j) t[T][j] = xv(T, j) > 0.f ? t[T][j] : t[T][j] * __expf(xv(T, j));
       } else {
         float dot = 0.f;
 #pragma unroll
-        for (int T = 0; T < 8; ++T)
+        for (int T = 0; T < NT; ++T)
 #pragma unroll
           for (int j = 0; j < 4; ++j) dot += __expf(xv(T, j) - mx) * inv * t[T][j];       // the unrounded softmax
         dot += __shfl_xor(dot, 16);
         dot += __shfl_xor(dot, 32);
 #pragma unroll
-        for (int T = 0; T < 8; ++T)
+        for (int T = 0; T < NT; ++T)
 #pragma unroll
           for (int j = 0; j < 4; ++j) t[T][j] = __expf(xv(T, j) - mx) * inv * (t[T][j] - dot);
       }
 #pragma unroll
-      for (int T = 0; T < 8; ++T) {
+      for (int T = 0; T < NT; ++T) {
         i32x2_t w;
         w[0] = (int)E::pack2(t[T][0], t[T][1]);
         w[1] = (int)E::pack2(t[T][2], t[T][3]);
@@ -302,13 +319,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
     __syncthreads();
 
-    // ---- M += (a/den)^T G ; dz ----
+    // ---- M += a^T G / den ; dz ----
     // (what dq holds so far is asked for here, where the row phase's registers are free, and used in the next step)
 #pragma unroll
-    for (int p = 0; p < 4; ++p) rdq[p] = buf_load_b128(dq_rs, (uint32_t)(r0 + frow + 4 * p) * pitch_b + 16 * lp);
+    for (int p = 0; p < NF; ++p) rdq[p] = buf_load_b128(dq_rs, (uint32_t)(r0 + frow + FR * p) * pitch_b + 16 * lp);
     __builtin_amdgcn_sched_barrier(0);      // (asked for first: the loop's next wait on memory covers these too)
 #pragma unroll
-    for (int c = 0; c < TR / 16; ++c) {
+    for (int c = 0; c < TR / KM; ++c) {
       const uint16_t* pa0 = reinterpret_cast<const uint16_t*>(sQ + ma_off[0] + c * 4096);
       const uint16_t* pa1 = reinterpret_cast<const uint16_t*>(sQ + ma_off[1] + c * 4096);
       const i16x8_t af = concat4(lds_read_tr16(pa0), lds_read_tr16(pa1));
@@ -316,12 +333,14 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       for (int t2 = 0; t2 < 2; ++t2) {
         const uint16_t* pb0 = reinterpret_cast<const uint16_t*>(sG + mb_off[0][t2] + c * 4096);
         const uint16_t* pb1 = reinterpret_cast<const uint16_t*>(sG + mb_off[1][t2] + c * 4096);
-        macc[t2] = E::mfma32(af, concat4(lds_read_tr16(pb0), lds_read_tr16(pb1)), macc[t2]);
+        const i16x8_t bf = concat4(lds_read_tr16(pb0), lds_read_tr16(pb1));
+        if constexpr (D == 128) macc[t2] = E::mfma32(af, bf, macc[t2]);
+        else macc[t2] = E::mfma16(af, bf, macc[t2]);
       }
     }
 #pragma unroll
-    for (int p = 0; p < 4; ++p) {
-      const int row = lrow + 32 * p;
+    for (int p = 0; p < NP; ++p) {
+      const int row = lrow + RPP * p;
       const uint32_t o = ld_off + p * 8192;
       const i16x8_t an = *reinterpret_cast<const i16x8_t*>(sQ + o);
       const float dd = sDD[row];
@@ -337,11 +356,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   float* mo = m_part + pidx * D * D;
 #pragma unroll
   for (int t2 = 0; t2 < 2; ++t2) {
-    const int col = 32 * (nt0 + t2) + (lane & 31);
+    const int col = MW * (nt0 + t2) + (lane & (MW - 1));
 #pragma unroll
-    for (int i4 = 0; i4 < 4; ++i4) {
+    for (int i4 = 0; i4 < MR / 4; ++i4) {
       const f32x4_t v4 = {macc[t2][4 * i4], macc[t2][4 * i4 + 1], macc[t2][4 * i4 + 2], macc[t2][4 * i4 + 3]};
-      *reinterpret_cast<f32x4_t*>(mo + (size_t)col * D + 32 * mt + 8 * i4 + 4 * g2) = v4;
+      *reinterpret_cast<f32x4_t*>(mo + (size_t)col * D + MW * mt + 8 * i4 + 4 * (D == 128 ? g2 : h)) = v4;
     }
   }
   // (the loop's last barrier has passed: sQ is free)
@@ -354,7 +373,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   if (tid < D) {
     float s0 = 0.f, s1 = 0.f;
 #pragma unroll 8
-    for (int rr = 0; rr < 32; ++rr) {
+    for (int rr = 0; rr < RPP; ++rr) {
       s0 += sRed[0][rr][tid];
       s1 += sRed[1][rr][tid];
     }
@@ -363,21 +382,23 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   }
 }
 
-// Key side of the same backward, head dim 128: dv = c dS, dc = v dS^T + dz, dk = phi'(k) dc with c = phi(k).
+// Key side of the same backward: dv = c dS, dc = v dS^T + dz, dk = phi'(k) dc with c = phi(k).
 // grid (slices of L, heads), 8 waves; dS [d1][d2] and dS^T [d2][d1] (16 bit, rows padded by 16 bytes) and dz stay in LDS,
 // every wave walks its own 16-key tiles of the slice and never meets another wave after the staging barrier:
-//   rows of k, v (fetched a tile ahead) -> two wave-private swizzled 4 KB tiles; phi(k) takes the place of k;
+//   rows of k, v (fetched a tile ahead) -> two wave-private swizzled tiles; phi(k) takes the place of k;
 //   dv^T = dS^T c^T and dc^T = dS v^T as 16x16x32 products (a key's row spread over 4 lanes, B operands read row-wise
 //   from the wave's tiles); dk, dv go back over the tiles and leave as whole rows, added to what dk, dv held (asked
 //   for at the start of the tile) when accumulating.
-template <typename Tag, int FMAP>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void linear_bwd_keys_kernel(
+template <typename Tag, int D, int FMAP>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 128 ? 2 : 4, D == 128 ? 2 : 4))) void linear_bwd_keys_kernel(
     const uint16_t* __restrict__ k, const uint16_t* __restrict__ v, const uint16_t* __restrict__ ds,
     const uint16_t* __restrict__ dst, const float* __restrict__ dz, uint16_t* __restrict__ dk, uint16_t* __restrict__ dv,
     const RowLayout lin, int L, int rows_per_split, int accumulate) {
   using E = Elem<Tag>;
   constexpr int fmap = FMAP;
-  constexpr int D = 128;
+  constexpr int CPR = D / 8;                     // 16-byte pieces per row
+  constexpr int NF = CPR / 4, FR = 64 / CPR;     // passes over a wave's 16 rows, rows per pass
+  constexpr int NT = D / 16, NC = D / 32;        // 16-column tiles of a row, 32-column fragments
   constexpr int PSTR = D * 2 + 16;               // row pitch of the staged matrices
   constexpr int WT = 16 * D * 2;                 // bytes of a wave's tile
   __shared__ __attribute__((aligned(16))) char smem[2 * D * PSTR + D * 4 + 8 * 2 * WT];
@@ -413,26 +434,26 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const size_t pitch = (size_t)lin.sl;
   const uint32_t pitch_b = (uint32_t)lin.sl * 2u;
 
-  // loader / writer layout of a wave's tile: lane -> row lane / 16 + 4 p, 16-byte piece lane % 16
-  const int frow = lane >> 4, lp = lane & 15;
-  uint32_t f_off[4];
+  // loader / writer layout of a wave's tile: lane -> row lane / CPR + FR p, 16-byte piece lane % CPR
+  const int frow = lane / CPR, lp = lane % CPR;
+  uint32_t f_off[NF];
 #pragma unroll
-  for (int p = 0; p < 4; ++p) f_off[p] = lbs_off(frow + 4 * p, 8 * lp);
+  for (int p = 0; p < NF; ++p) f_off[p] = lbs_off<D>(frow + FR * p, 8 * lp);
   // product layout: lane = (key l of the tile's 16, quarter h): d = 16 T + 4 h + j
   const int l = lane & 15, h = lane >> 4;
-  uint32_t acc_off[8];        // (l, 16 T + 4 h)
+  uint32_t acc_off[NT];        // (l, 16 T + 4 h)
 #pragma unroll
-  for (int T = 0; T < 8; ++T) acc_off[T] = lbs_off(l, 16 * T + 4 * h);
-  uint32_t b_off[4];          // (l, 32 c + 8 h): B-operand order
+  for (int T = 0; T < NT; ++T) acc_off[T] = lbs_off<D>(l, 16 * T + 4 * h);
+  uint32_t b_off[NC];          // (l, 32 c + 8 h): B-operand order
 #pragma unroll
-  for (int c = 0; c < 4; ++c) b_off[c] = lbs_off(l, 32 * c + 8 * h);
+  for (int c = 0; c < NC; ++c) b_off[c] = lbs_off<D>(l, 32 * c + 8 * h);
   const uint32_t a_base = (uint32_t)l * PSTR + (uint32_t)h * 16u;     // row 16 T + l of a staged matrix: + 16 PSTR per T, + 64 per c
 
-  i16x8_t rk[4], rv[4];
+  i16x8_t rk[NF], rv[NF];
   auto fetch_kv = [&](int r0) __attribute__((always_inline)) {
 #pragma unroll
-    for (int p = 0; p < 4; ++p) {
-      const uint32_t o = (uint32_t)(r0 + frow + 4 * p) * pitch_b + 16 * lp;      // rows past L read as zero
+    for (int p = 0; p < NF; ++p) {
+      const uint32_t o = (uint32_t)(r0 + frow + FR * p) * pitch_b + 16 * lp;      // rows past L read as zero
       rk[p] = buf_load_b128(k_rs, o);
       rv[p] = buf_load_b128(v_rs, o);
     }
@@ -441,39 +462,39 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   if (first < row_end) fetch_kv(first);
   for (int r0 = first; r0 < row_end; r0 += 128) {
 #pragma unroll
-    for (int p = 0; p < 4; ++p) {
+    for (int p = 0; p < NF; ++p) {
       *reinterpret_cast<i16x8_t*>(tK + f_off[p]) = rk[p];
       *reinterpret_cast<i16x8_t*>(tV + f_off[p]) = rv[p];
     }
     wave_lds_fence();
     // what dk, dv hold (for this tile) and the next tile's rows: both have the whole tile to arrive
-    i16x8_t rdk[4], rdv[4];
+    i16x8_t rdk[NF], rdv[NF];
 #pragma unroll
-    for (int p = 0; p < 4; ++p) {
-      const uint32_t o = (uint32_t)(r0 + frow + 4 * p) * pitch_b + 16 * lp;
+    for (int p = 0; p < NF; ++p) {
+      const uint32_t o = (uint32_t)(r0 + frow + FR * p) * pitch_b + 16 * lp;
       rdk[p] = buf_load_b128(dk_rs, o);
       rdv[p] = buf_load_b128(dv_rs, o);
     }
     if (r0 + 128 < row_end) fetch_kv(r0 + 128);
 
-    i16x4_t xraw[8];
+    i16x4_t xraw[NT];
 #pragma unroll
-    for (int T = 0; T < 8; ++T) xraw[T] = *reinterpret_cast<const i16x4_t*>(tK + acc_off[T]);
+    for (int T = 0; T < NT; ++T) xraw[T] = *reinterpret_cast<const i16x4_t*>(tK + acc_off[T]);
     auto xv = [&](int T, int j) __attribute__((always_inline)) { return E::to_float((uint16_t)xraw[T][j]); };
     float mx = 0.f, inv = 1.f;
     {
-      float a[8][4];
+      float a[NT][4];
       if (fmap == SLA_FMAP_SOFTMAX) {
         mx = xv(0, 0);
 #pragma unroll
-        for (int T = 0; T < 8; ++T)
+        for (int T = 0; T < NT; ++T)
 #pragma unroll
           for (int j = 0; j < 4; ++j) mx = fmaxf(mx, xv(T, j));
         mx = fmaxf(mx, __shfl_xor(mx, 16));
         mx = fmaxf(mx, __shfl_xor(mx, 32));
         float sum = 0.f;
 #pragma unroll
-        for (int T = 0; T < 8; ++T)
+        for (int T = 0; T < NT; ++T)
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
             a[T][j] = __expf(xv(T, j) - mx);
@@ -483,19 +504,19 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         sum += __shfl_xor(sum, 32);
         inv = 1.0f / sum;
 #pragma unroll
-        for (int T = 0; T < 8; ++T)
+        for (int T = 0; T < NT; ++T)
 #pragma unroll
           for (int j = 0; j < 4; ++j) a[T][j] = round16<Tag>(a[T][j] * inv);
       } else {
 #pragma unroll
-        for (int T = 0; T < 8; ++T)
+        for (int T = 0; T < NT; ++T)
 #pragma unroll
           for (int j = 0; j < 4; ++j) a[T][j] = fmap_pointwise<Tag>(fmap, xv(T, j));
       }
       // c = phi(k) over the raw rows (this lane's own places; a key's gradients depend on its own row only, so rows
       // past the end, which are never written, need no care)
 #pragma unroll
-      for (int T = 0; T < 8; ++T) {
+      for (int T = 0; T < NT; ++T) {
         i32x2_t w;
         w[0] = (int)E::pack2(a[T][0], a[T][1]);
         w[1] = (int)E::pack2(a[T][2], a[T][3]);
@@ -504,18 +525,18 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
     wave_lds_fence();
     // dv^T = dS^T c^T ; dc^T = dS v^T
-    f32x4_t dva[8], dca[8];
+    f32x4_t dva[NT], dca[NT];
 #pragma unroll
-    for (int T = 0; T < 8; ++T) {
+    for (int T = 0; T < NT; ++T) {
       dva[T] = f32x4_t{0.f, 0.f, 0.f, 0.f};
       dca[T] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     }
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
+    for (int c = 0; c < NC; ++c) {
       const i16x8_t cf = *reinterpret_cast<const i16x8_t*>(tK + b_off[c]);
       const i16x8_t vf = *reinterpret_cast<const i16x8_t*>(tV + b_off[c]);
 #pragma unroll
-      for (int T = 0; T < 8; ++T) {
+      for (int T = 0; T < NT; ++T) {
         dva[T] = E::mfma16(*reinterpret_cast<const i16x8_t*>(sDST + a_base + T * 16 * PSTR + c * 64), cf, dva[T]);
         dca[T] = E::mfma16(*reinterpret_cast<const i16x8_t*>(sDS + a_base + T * 16 * PSTR + c * 64), vf, dca[T]);
       }
@@ -523,36 +544,36 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     wave_lds_fence();      // (the tiles are rewritten below: every read of them above comes first)
     // dc += dz ; dk = phi'(k) dc
 #pragma unroll
-    for (int T = 0; T < 8; ++T) {
+    for (int T = 0; T < NT; ++T) {
       const f32x4_t zz = *reinterpret_cast<const f32x4_t*>(sDZ + 16 * T + 4 * h);
 #pragma unroll
       for (int j = 0; j < 4; ++j) dca[T][j] += zz[j];
     }
     if (fmap == SLA_FMAP_RELU) {
 #pragma unroll
-      for (int T = 0; T < 8; ++T)
+      for (int T = 0; T < NT; ++T)
 #pragma unroll
         for (int j = 0; j < 4; ++j) dca[T][j] = xv(T, j) > 0.f ? dca[T][j] : 0.f;
     } else if (fmap == SLA_FMAP_ELU) {
 #pragma unroll
-      for (int T = 0; T < 8; ++T)
+      for (int T = 0; T < NT; ++T)
 #pragma unroll
         for (int j = 0; j < 4; ++j) dca[T][j] = xv(T, j) > 0.f ? dca[T][j] : dca[T][j] * __expf(xv(T, j));
     } else {
       float dot = 0.f;
 #pragma unroll
-      for (int T = 0; T < 8; ++T)
+      for (int T = 0; T < NT; ++T)
 #pragma unroll
         for (int j = 0; j < 4; ++j) dot += __expf(xv(T, j) - mx) * inv * dca[T][j];       // the unrounded softmax
       dot += __shfl_xor(dot, 16);
       dot += __shfl_xor(dot, 32);
 #pragma unroll
-      for (int T = 0; T < 8; ++T)
+      for (int T = 0; T < NT; ++T)
 #pragma unroll
         for (int j = 0; j < 4; ++j) dca[T][j] = __expf(xv(T, j) - mx) * inv * (dca[T][j] - dot);
     }
 #pragma unroll
-    for (int T = 0; T < 8; ++T) {
+    for (int T = 0; T < NT; ++T) {
       i32x2_t wk, wv;
       wk[0] = (int)E::pack2(dca[T][0], dca[T][1]);
       wk[1] = (int)E::pack2(dca[T][2], dca[T][3]);
@@ -564,8 +585,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     wave_lds_fence();
     // whole rows out: 16-bit value + what the tensor held, one rounded add (nothing held when not accumulating)
 #pragma unroll
-    for (int p = 0; p < 4; ++p) {
-      const int grow = r0 + frow + 4 * p;
+    for (int p = 0; p < NF; ++p) {
+      const int grow = r0 + frow + FR * p;
       const i16x8_t k16 = *reinterpret_cast<const i16x8_t*>(tK + f_off[p]);
       const i16x8_t v16 = *reinterpret_cast<const i16x8_t*>(tV + f_off[p]);
       i32x4_t wk, wv;

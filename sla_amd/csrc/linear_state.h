@@ -221,14 +221,15 @@ __global__ void linear_prep_weight_kernel(const float* __restrict__ weight, uint
 
 // ---- kernel 2 (forward, and a backward that has to rebuild the states): finish the states ----------------------------
 // From the slices' partial states of a head: their sums in ascending slice order, rounded to 16 bit (kvt, the transposed
-// state; kvp, its transpose in slot order, which only the head-dim-64 backward reads; z), and with the projection folded in
+// state; z), and with the projection folded in
 //   kvwt[bh][e][d1] = round16( sum_d2 round16(W[e][d2]) * KVT[d2][d1] ), fp32 accumulation:
-// (phi(Q) KV / den) W^T = (phi(Q) (KV W^T)) / den, so the output kernel needs one product per query tile.
+// (phi(Q) KV / den) W^T = (phi(Q) (KV W^T)) / den, so the output kernel needs one product per query tile.  kvw[d1][e] is that
+// matrix for the backward, from the sums before their rounding (fp32 products): dq's relative error against 64 bits 4.13e-3
+// where twice rounded sums leave 4.66e-3 (softmax map, 4 heads x 6001 x 64 in bf16).
 // One workgroup of 512 threads per head and 16 columns d1 (neighbouring workgroups on one XCD, so that the two halves of a
 // 128-byte line meet in its L2): the two halves of the workgroup sum one half of the slices each, over every row d2, and meet
 // in LDS; holding all a row of kvwt needs of the state, the workgroup then multiplies by W on the matrix cores.  Bound by
-// latency: the loads of eight slices and the workgroup's rows of W are in flight at once.  The workgroups of head 0 also
-// leave the 16-bit transposed weight wt[d][e] that a backward reads.
+// latency: the loads of eight slices and the workgroup's rows of W are in flight at once.
 // Against a summing and a folding kernel (the latter on the vector ALU), B1 H12 L9360 D128: 16.3 against 10.1 + 8.5 us and one
 // launch less; state build of 40 heads x 32760 x 128: 159 against 172 us, of 16 heads x 6001 x 64: 17.5 against 20.9.
 template <int NV, int BATCH = 8>
@@ -308,15 +309,16 @@ template <typename Tag, int D>
 __global__ __launch_bounds__(512) void linear_state_finish_kernel(const float* __restrict__ kv_part,
                                                                   const float* __restrict__ z_part,
                                                                   const float* __restrict__ weight, uint16_t* __restrict__ kvt,
-                                                                  uint16_t* __restrict__ kvp, uint16_t* __restrict__ kvwt,
-                                                                  uint16_t* __restrict__ z, uint16_t* __restrict__ wt, int nsplit,
-                                                                  int nsum, int total) {
+                                                                  uint16_t* __restrict__ kvw, uint16_t* __restrict__ kvwt,
+                                                                  uint16_t* __restrict__ z, int nsplit, int nsum, int total) {
   using E = Elem<Tag>;
   constexpr int DD = D * D;
   constexpr int STR = D + 8;               // row pitch of the strip in LDS
   constexpr int NR = D / 64;               // rows d2 per thread
   __shared__ __attribute__((aligned(16))) float s_half[NR * 256 * 4];     // sums of the upper half of the slices
   __shared__ __attribute__((aligned(16))) uint16_t s_kv[16 * STR];        // [d1][d2]
+  constexpr int STR32 = D + 4;
+  __shared__ __attribute__((aligned(16))) float s_kv32[16 * STR32];       // the same before rounding
   const int logical = xcd_remap(blockIdx.x, gridDim.x, total);
   if (logical < 0) return;
   const int bh = logical / (D / 16), d1_0 = 16 * (logical % (D / 16));
@@ -348,11 +350,6 @@ __global__ __launch_bounds__(512) void linear_state_finish_kernel(const float* _
       for (int sp = 0; sp < nsum; ++sp) sum += pz[(size_t)sp * D];
       z[(size_t)bh * D + d1_0 + tid] = E::from_float(sum);
     }
-    if (bh == 0)
-      for (int i = tid; i < 16 * D; i += 256) {
-        const int d = d1_0 + i / D, e = i % D;
-        wt[d * D + e] = E::from_float(weight[(size_t)e * D + d]);
-      }
   }
   __syncthreads();
   if (!half) {
@@ -365,19 +362,13 @@ __global__ __launch_bounds__(512) void linear_state_finish_kernel(const float* _
       w[1] = (int)E::pack2(acc[i][2], acc[i][3]);
       *reinterpret_cast<i32x2_t*>(kvt + (size_t)bh * DD + (size_t)d2 * D + d1_0 + dc) = w;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) s_kv[(dc + j) * STR + d2] = (uint16_t)((uint32_t)w[j >> 1] >> (16 * (j & 1)));
+      for (int j = 0; j < 4; ++j) {
+        s_kv[(dc + j) * STR + d2] = (uint16_t)((uint32_t)w[j >> 1] >> (16 * (j & 1)));
+        s_kv32[(dc + j) * STR32 + d2] = acc[i][j];
+      }
     }
   }
   __syncthreads();
-  if constexpr (D == 64) {
-    // slots 8 piece .. of a row hold d2 = 16 c + 4 gg .. + 3 and 8 further on (piece = 2 c + gg)
-    if (half && tid < 16 * (D / 8)) {
-      const int row = tid / (D / 8), piece = tid % (D / 8);
-      const uint16_t* src = s_kv + row * STR + 16 * (piece >> 1) + 4 * (piece & 1);
-      const i16x8_t v8 = concat4(*reinterpret_cast<const i16x4_t*>(src), *reinterpret_cast<const i16x4_t*>(src + 8));
-      *reinterpret_cast<i16x8_t*>(kvp + (size_t)bh * DD + (size_t)(d1_0 + row) * D + 8 * piece) = v8;
-    }
-  }
   if (wave >= D / 16) return;
   f32x4_t o = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -392,14 +383,25 @@ __global__ __launch_bounds__(512) void linear_state_finish_kernel(const float* _
   w[0] = (int)E::pack2(o[0], o[1]);
   w[1] = (int)E::pack2(o[2], o[3]);
   *reinterpret_cast<i32x2_t*>(kvwt + (size_t)bh * DD + (size_t)(16 * tile + l) * D + d1_0 + 4 * h) = w;
+  f32x4_t p = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int c = 0; c < D / 32; ++c)
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+      const f32x4_t a = *reinterpret_cast<const f32x4_t*>(s_kv32 + l * STR32 + 32 * c + 8 * h + 4 * x);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) p = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], round16<Tag>(wraw[c][x][j]), p, 0, 0, 0);
+    }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) kvw[(size_t)bh * DD + (size_t)(d1_0 + 4 * h + i) * D + 16 * tile + l] = E::from_float(p[i]);
 }
 
 // ---- workspace layout of the state build -----------------------------------------------------
-// The finished states (kvt .. wt) come first: `states_end` bytes that a caller may copy aside after the
+// The finished states (kvt .. z) come first: `states_end` bytes that a caller may copy aside after the
 // forward and put back at the start of the backward's workspace instead of having them rebuilt.
 struct LinWs {
   int nsplit, rows_per_split;
-  size_t kvt, kvp, kvwt, z, wt, states_end, kv_part, z_part, vmax_part, total;
+  size_t kvt, kvw, kvwt, z, states_end, kv_part, z_part, vmax_part, total;
 };
 
 static inline LinWs lin_ws(int BH, int L, int D) {
@@ -415,10 +417,9 @@ static inline LinWs lin_ws(int BH, int L, int D) {
   w.rows_per_split = sp.rows_per_split;
   size_t off = 0;
   w.kvt = off;     off += align_up((int64_t)BH * D * D * 2, 256);
-  w.kvp = off;     off += align_up((int64_t)BH * D * D * 2, 256);
+  w.kvw = off;     off += align_up((int64_t)BH * D * D * 2, 256);
   w.kvwt = off;    off += align_up((int64_t)BH * D * D * 2, 256);
   w.z = off;       off += align_up((int64_t)BH * D * 2, 256);
-  w.wt = off;      off += align_up((int64_t)D * D * 2, 256);
   w.states_end = off;
   w.kv_part = off; off += align_up((int64_t)BH * w.nsplit * D * D * 4, 256);
   w.z_part = off;  off += align_up((int64_t)BH * w.nsplit * D * 4, 256);
@@ -440,11 +441,11 @@ static inline void launch_state_finish(const float* weight, int BH, char* ws, ch
     hipLaunchKernelGGL((linear_state_presum_kernel<D>), dim3(D * D / 256 + 1, BH), dim3(512), 0, st, kv_part, z_part, w.nsplit);
   hipLaunchKernelGGL((linear_state_finish_kernel<Tag, D>), dim3(xcd_grid((int64_t)BH * (D / 16))), dim3(512), 0, st,
                      (const float*)kv_part, (const float*)z_part, weight,
-                     (uint16_t*)(ws + w.kvt), (uint16_t*)(ws + w.kvp), (uint16_t*)(ws + w.kvwt), (uint16_t*)(ws + w.z),
-                     (uint16_t*)(ws + w.wt), w.nsplit, presum ? 1 : w.nsplit, BH * (D / 16));
+                     (uint16_t*)(ws + w.kvt), (uint16_t*)(ws + w.kvw), (uint16_t*)(ws + w.kvwt), (uint16_t*)(ws + w.z),
+                     w.nsplit, presum ? 1 : w.nsplit, BH * (D / 16));
 }
 
-// Streams K and V once and leaves the finished states and the 16-bit transposed weight.
+// Streams K and V once and leaves the finished states.
 template <typename Tag, int D>
 static inline void launch_state_build(const void* k, const void* v, const RowLayout& lay, const float* weight, int fmap,
                                       int BH, int L, char* ws, char* parts, const LinWs& w, hipStream_t st) {
