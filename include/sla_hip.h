@@ -204,15 +204,11 @@ int sla_sparse_attn_linear_fwd_strided(const void* q, const void* k, const void*
 
 /* Backward of the whole module in one call: the kernels of sla_sparse_attn_bwd(_strided) followed by those of
  * sla_linear_bwd(_strided) with SLA_BWD_ACCUMULATE (the linear branch adds into dq, dk, dv), results equal to those two
- * calls bit for bit.  The only flag is SLA_BWD_STATES_READY.  qkv_strides / do_strides: both NULL for contiguous
+ * calls bit for bit (the linear branch's kernels come first, and the attention kernels add).  The only flag is SLA_BWD_STATES_READY.  qkv_strides / do_strides: both NULL for contiguous
  * (B, H, L, D) tensors, else as in the strided calls.  o_s is the attention output the forward saved.  The two workspaces
  * are those of the two calls (SLA_WS_SPARSE_BWD, SLA_WS_LINEAR_BWD).
- * side_stream (may be NULL or equal to stream: then everything runs on `stream`) takes the short kernels - the
- * per-key-block lists of the map, and the per-head reductions and small products of the linear branch - so that they run
- * beside the long dQ and dK/dV kernels instead of between them; `stream` waits for all of it before the call's last
- * kernel, so later work needs ordering against `stream` only.  The streams must belong to the current device and have the
- * same (default) priority.  The first call with a second stream on a device creates four events (no device memory), kept
- * for later calls; calls from several host threads take turns enqueueing.
+ * Everything runs on `stream`: the short kernels share the launches of longer ones.  side_stream is accepted for callers that
+ * hand one over and not used.
  * Replaces autograd through SparseLinearAttention.forward, sparse_linear_attention/core.py:88-100 with
  * kernel.py:277-320. */
 int sla_module_bwd(const void* q, const void* k, const void* v, const int64_t* qkv_strides, const void* o_s,

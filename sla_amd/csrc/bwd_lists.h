@@ -1,0 +1,188 @@
+// Short jobs of the backward that ride in other kernels' launches: the per-key-block lists of the map, the work items of the
+// dK/dV kernel, and the sum of the heads' weight gradients.  Each is a few workgroups bound by latency; a launch of its own
+// costs what it computes once more (10 + 6 + 5 us of a 207 us forward and backward of 8 heads x 4096 x 128).
+#pragma once
+#include "common.h"
+
+namespace sla {
+
+// ---- per-key-block lists ------------------------------------------------------------------
+// One workgroup of COL_NW wavefronts per strip of 64 key blocks.  Every wavefront takes its own chunk of
+// 64 map rows (query blocks): it reads them with coalesced 16-byte loads and transposes them through its
+// private LDS tile; lane c counts the ones of column c in that chunk.  After a barrier every wave knows
+// how many entries the chunks before its own contribute to each column and writes its matches at that
+// offset, walking the chunk in row order, so list[bh][n][0..count) holds the selecting query blocks in
+// ascending order.  Capacity Mblk per list (only `count` entries are ever touched).
+constexpr int COL_NW = 8;
+constexpr int COL_TILE = 64 * 80;                                    // bytes of a wave's tile
+constexpr int COL_LDS = COL_NW * (COL_TILE + 64 * 4);
+struct ColLists {
+  const int8_t* map;
+  int *list, *count;
+  int Mblk, Nblk, vec_ok, strips, wgs;                                // wgs = strips of 64 key blocks x heads; 0: nothing to do
+};
+static inline ColLists col_lists_job(const int8_t* map, int* list, int* count, int BH, int Mblk, int Nblk) {
+  // 16-byte loads of map rows need 16-byte aligned rows
+  const int strips = cdiv(Nblk, 64);
+  return ColLists{map, list, count, Mblk, Nblk, (Nblk % 16 == 0) && ((uintptr_t)map % 16 == 0), strips, strips * BH};
+}
+// (64 * COL_NW threads; smem: COL_LDS bytes, 16-byte aligned)
+static __device__ __forceinline__ void col_lists_body(const ColLists& j, int wg, char* smem) {
+  int8_t (*tile)[64][80] = reinterpret_cast<int8_t (*)[64][80]>(smem);
+  int (*cnt)[64] = reinterpret_cast<int (*)[64]>(smem + COL_NW * COL_TILE);
+  const int Mblk = j.Mblk, Nblk = j.Nblk;
+  const int bh = wg / j.strips;
+  const int n0 = (wg - bh * j.strips) * 64;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int n = n0 + lane;
+  const int8_t* base = j.map + (size_t)bh * Mblk * Nblk;
+  int* out = j.list + ((size_t)bh * Nblk + (n < Nblk ? n : 0)) * Mblk;
+  // lane -> (row lr + 16j, 16-byte chunk lc) of the tile
+  const int lr = lane >> 2, lc = (lane & 3) * 16;
+  int done = 0;              // entries of column `lane` written by earlier rounds
+  for (int r0 = 0; r0 < Mblk; r0 += 64 * COL_NW) {
+    const int m0 = r0 + 64 * wave;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int m = m0 + lr + 16 * i;
+      i32x4_t x = {0, 0, 0, 0};
+      if (m < Mblk) {
+        if (j.vec_ok && n0 + lc + 16 <= Nblk) {
+          x = *reinterpret_cast<const i32x4_t*>(base + (size_t)m * Nblk + n0 + lc);
+        } else {
+          int8_t* b = reinterpret_cast<int8_t*>(&x);
+          for (int e = 0; e < 16; ++e)
+            if (n0 + lc + e < Nblk) b[e] = base[(size_t)m * Nblk + n0 + lc + e];
+        }
+      }
+      *reinterpret_cast<i32x4_t*>(&tile[wave][lr + 16 * i][lc]) = x;
+    }
+    wave_lds_fence();
+    int mine = 0;
+#pragma unroll 16
+    for (int r = 0; r < 64; ++r) mine += tile[wave][r][lane] == 1;
+    cnt[wave][lane] = mine;
+    __syncthreads();
+    int before = 0, all = 0;
+#pragma unroll
+    for (int w = 0; w < COL_NW; ++w) {
+      const int cw = cnt[w][lane];
+      before += w < wave ? cw : 0;
+      all += cw;
+    }
+    if (n < Nblk) {
+      int c = done + before;
+#pragma unroll 16
+      for (int r = 0; r < 64; ++r)
+        if (tile[wave][r][lane] == 1) out[c++] = m0 + r;
+    }
+    done += all;
+    __syncthreads();         // cnt and the tiles are rewritten by the next round
+  }
+  if (wave == 0 && n < Nblk) j.count[(size_t)bh * Nblk + n] = done;
+}
+
+// ---- work items of the dK/dV kernel --------------------------------------------------------
+// A key block that very many query blocks selected (an attention "sink") would make one workgroup walk a list
+// many times the average length.  Lists longer than `seg` entries are therefore cut into segments of `seg`; every
+// segment is one work item.  item = {bh, key block, segment, slot}: slot < 0 for a key block with a single segment
+// (the workgroup writes dK / dV itself), otherwise the index of the fp32 partial this segment writes; the partials
+// of a key block occupy consecutive slots and are added in segment order.
+// One wave per 512 (head, key block) pairs: it counts the items of all pairs before its own (no other wave is waited for),
+// then numbers its own, 64 adjacent pairs at a time.  (One workgroup for all pairs, with eight adjacent ones per thread and
+// therefore scattered stores, took 38 us for 32 heads x 512.)
+constexpr int SEG_PAIRS = 512;
+struct Segments {
+  const int* count;
+  int *nseg, *slot0, *done;                                            // done: segments finished so far, cleared here
+  i32x4_t* items;
+  int* totals;
+  int nblocks, Nblk, seg, max_items, max_slots, wgs;                   // nblocks = heads x key blocks; wgs 0: nothing to do
+};
+static __device__ __forceinline__ void segments_body(const Segments& s, int wg) {
+  const int lane = threadIdx.x & 63;
+  const int first = wg * SEG_PAIRS;
+  const auto nsegs = [&](int c) { return c <= s.seg ? 1 : (c + s.seg - 1) / s.seg; };
+  int item0 = 0, slot = 0;
+  for (int i = lane; i < first; i += SEG_PAIRS) {
+    int c[SEG_PAIRS / 64];
+#pragma unroll
+    for (int x = 0; x < SEG_PAIRS / 64; ++x) c[x] = s.count[i + 64 * x];
+#pragma unroll
+    for (int x = 0; x < SEG_PAIRS / 64; ++x) {
+      const int n = nsegs(c[x]);
+      item0 += n;
+      slot += n > 1 ? n : 0;
+    }
+  }
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    item0 += __shfl_xor(item0, o);
+    slot += __shfl_xor(slot, o);
+  }
+  int c[SEG_PAIRS / 64];
+#pragma unroll
+  for (int x = 0; x < SEG_PAIRS / 64; ++x) {
+    const int i = first + 64 * x + lane;
+    c[x] = i < s.nblocks ? s.count[i] : 0;
+  }
+#pragma unroll
+  for (int x = 0; x < SEG_PAIRS / 64; ++x) {
+    const int i = first + 64 * x + lane;
+    const int n = i < s.nblocks ? nsegs(c[x]) : 0, m = n > 1 ? n : 0;
+    int a = n, b = m;                          // inclusive scans
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int ta = __shfl_up(a, o), tb = __shfl_up(b, o);
+      if (lane >= o) {
+        a += ta;
+        b += tb;
+      }
+    }
+    if (i < s.nblocks) {
+      const int fi = item0 + a - n, fs = slot + b - m;
+      s.nseg[i] = n;
+      s.slot0[i] = fs;
+      s.done[i] = 0;
+      const int bh = i / s.Nblk, nb = i - bh * s.Nblk;
+      // (a map whose rows hold more ones than the topk the workspace was sized for cannot overrun the tables: its
+      //  surplus items are dropped)
+      for (int sg = 0; sg < n; ++sg)
+        if (fi + sg < s.max_items)
+          s.items[fi + sg] = i32x4_t{bh, nb, sg, fs + m > s.max_slots ? -2 : n > 1 ? fs + sg : -1};
+    }
+    item0 += __shfl(a, 63);
+    slot += __shfl(b, 63);
+  }
+  if (first + SEG_PAIRS >= s.nblocks && lane == 0) {
+    s.totals[0] = min(item0, s.max_items);
+    s.totals[1] = min(slot, s.max_slots);
+  }
+}
+
+// ---- the heads' weight gradients added up, in ascending head order ----------------------------
+// dw_head [head][d][e], db_head [head][e] (fp32) -> d_weight [e][d], d_bias [e].  One wave per 256 elements.
+struct HeadSums {
+  const float *dw_head, *db_head;
+  float *d_weight, *d_bias;
+  int BH, D, wgs;                                                       // wgs = D * D / 256; 0: nothing to do
+};
+static __device__ __forceinline__ void head_sums_body(const HeadSums& s, int wg) {
+  const int lane = threadIdx.x & 63, DD = s.D * s.D;
+  const int i = wg * 256 + lane * 4;
+  f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+  for (int h = 0; h < s.BH; ++h) acc += *reinterpret_cast<const f32x4_t*>(s.dw_head + (size_t)h * DD + i);
+  const int d = i / s.D, e = i % s.D;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) s.d_weight[(e + j) * s.D + d] = acc[j];
+  if (wg == 0)
+    for (int x = lane; x < s.D; x += 64) {
+      float b = 0.f;
+#pragma unroll 8
+      for (int h = 0; h < s.BH; ++h) b += s.db_head[(size_t)h * s.D + x];
+      s.d_bias[x] = b;
+    }
+}
+
+}  // namespace sla

@@ -123,6 +123,14 @@ static __device__ __forceinline__ void wave_lds_fence() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// Workgroup barrier for data exchanged through LDS alone: loads and stores to memory stay in flight across it.  (__syncthreads
+// waits for every one of them, which takes away what was fetched ahead.)
+static __device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // ---- row-contiguous output of a tile held in MFMA accumulator layout ---------------------------
 // In the transposed formulations a lane owns one row (query / key) of a 32-row tile and, per 32-column
 // tile dt and register group i4, the 4 adjacent columns 32dt + 8i4 + 4g.. of that row.  Storing those

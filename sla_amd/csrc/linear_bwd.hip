@@ -202,7 +202,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // ---- reduce -------------------------------------------------------------------------------
 // Stage 1, grid (cdiv(D*D,256), BH): per head, add the split partials in ascending order:
 //   dS (16 bit, both orientations), dz, and this head's dW^T / db (fp32).
-// Stage 2, grid (cdiv(D*D,256)): add the per-head dW^T / db in ascending head order.
+// Stage 2 (head_sums_body): add the per-head dW^T / db in ascending head order.
 template <typename Tag>
 __global__ __launch_bounds__(256) void linear_bwd_reduce_kernel(const float* __restrict__ ds_part,
                                                                 const float* __restrict__ dw_part,
@@ -243,26 +243,6 @@ __global__ __launch_bounds__(256) void linear_bwd_reduce_kernel(const float* __r
   }
 }
 
-__global__ __launch_bounds__(256) void linear_bwd_reduce_heads_kernel(const float* __restrict__ dw_head,
-                                                                      const float* __restrict__ db_head,
-                                                                      float* __restrict__ d_weight, float* __restrict__ d_bias,
-                                                                      int BH, int D) {
-  const int DD = D * D;
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < DD) {
-    float s = 0.f;
-#pragma unroll 4
-    for (int h = 0; h < BH; ++h) s += dw_head[(size_t)h * DD + i];
-    const int d = i / D, e = i % D;      // layout [d][e]
-    d_weight[e * D + d] = s;
-  }
-  if (i < D) {
-    float s = 0.f;
-    for (int h = 0; h < BH; ++h) s += db_head[(size_t)h * D + i];
-    d_bias[i] = s;
-  }
-}
-
 // ---- host ---------------------------------------------------------------------------------
 struct LinBwdWs {
   LinWs fwd;
@@ -293,9 +273,12 @@ int64_t linear_bwd_states_apart_bytes(int BH, int L, int D) { return (int64_t)li
 template <typename Tag, int D>
 static int linear_bwd_impl(const void* q, const void* k, const void* v, const float* weight, const void* d_out, void* dq,
                            void* dk, void* dv, const RowLayout& lin, const RowLayout& ldo, float* d_weight, float* d_bias,
-                           int fmap, int BH, int L, int flags, const char* states, char* ws, hipStream_t st, int steps) {
-  if (steps == 0) return SLA_OK;        // (arguments checked, nothing asked for)
+                           int fmap, int BH, int L, int flags, const char* states, char* ws, hipStream_t st, int steps,
+                           const ColLists& lists, HeadSums* heads) {
   const LinBwdWs w = lin_bwd_ws(BH, L, D, !states);
+  const HeadSums hs = {(const float*)(ws + w.dw_head), (const float*)(ws + w.db_head), d_weight, d_bias, BH, D, D * D / 256};
+  if (heads) *heads = hs;
+  if (steps == 0) return SLA_OK;        // (arguments checked, nothing asked for)
   const int accumulate = flags & SLA_BWD_ACCUMULATE;
   if ((steps & LB_STATES) && !states && !(flags & SLA_BWD_STATES_READY)) {
     // everything the forward's state build leaves: transposed state, z, and (fold) the folded state
@@ -306,36 +289,37 @@ static int linear_bwd_impl(const void* q, const void* k, const void* v, const fl
   const uint16_t* z = (const uint16_t*)(states + w.fwd.z);
   float* m_part = (float*)(ws + w.m_part);
   if (steps & LB_QUERY) {
-#define SLA_LBS_LAUNCH(FM)                                                                                                  \
-  hipLaunchKernelGGL((linear_bwd_stream_kernel<Tag, D, FM>), dim3(w.sp.nsplit, BH), dim3(512), 0, st, (const uint16_t*)q,     \
-                     (const uint16_t*)d_out, (const uint16_t*)(states + w.fwd.kvw), z, (uint16_t*)dq, lin, ldo, m_part,          \
-                     (float*)(ws + w.dz_part), (float*)(ws + w.db_part), L, w.sp.rows_per_split, accumulate)
-    if (fmap == SLA_FMAP_ELU) SLA_LBS_LAUNCH(SLA_FMAP_ELU);
-    else if (fmap == SLA_FMAP_RELU) SLA_LBS_LAUNCH(SLA_FMAP_RELU);
-    else SLA_LBS_LAUNCH(SLA_FMAP_SOFTMAX);
+#define SLA_LBS_LAUNCH(FM, ACC)                                                                                            \
+  hipLaunchKernelGGL((linear_bwd_stream_kernel<Tag, D, FM, ACC>), dim3(w.sp.nsplit, BH), dim3(512), 0, st, (const uint16_t*)q, \
+                     (const uint16_t*)d_out, (const uint16_t*)(states + w.fwd.kvw), z, (uint16_t*)dq, lin, ldo, m_part,      \
+                     (float*)(ws + w.dz_part), (float*)(ws + w.db_part), L, w.sp.rows_per_split)
+#define SLA_LB_FMAPS(LAUNCH)                                          \
+  if (accumulate) {                                                   \
+    if (fmap == SLA_FMAP_ELU) LAUNCH(SLA_FMAP_ELU, true);             \
+    else if (fmap == SLA_FMAP_RELU) LAUNCH(SLA_FMAP_RELU, true);      \
+    else LAUNCH(SLA_FMAP_SOFTMAX, true);                              \
+  } else {                                                            \
+    if (fmap == SLA_FMAP_ELU) LAUNCH(SLA_FMAP_ELU, false);            \
+    else if (fmap == SLA_FMAP_RELU) LAUNCH(SLA_FMAP_RELU, false);     \
+    else LAUNCH(SLA_FMAP_SOFTMAX, false);                             \
+  }
+    SLA_LB_FMAPS(SLA_LBS_LAUNCH)
 #undef SLA_LBS_LAUNCH
   }
-  if (steps & LB_REDUCE) {
-#define SLA_LBF_LAUNCH(HALVES)                                                                                               \
-  hipLaunchKernelGGL((linear_bwd_finish_kernel<Tag, D, HALVES>), dim3(xcd_grid((int64_t)BH * (D / 8))), dim3(256 * HALVES), 0, \
-                     st, (const float*)m_part, (const float*)(ws + w.dz_part), (const float*)(ws + w.db_part), weight, kvt,   \
-                     (uint16_t*)(ws + w.ds), (uint16_t*)(ws + w.dst), (float*)(ws + w.dz), (float*)(ws + w.dw_head),           \
-                     (float*)(ws + w.db_head), w.sp.nsplit, BH * (D / 8))
-    if (steps & LB_BESIDE) SLA_LBF_LAUNCH(1);
-    else SLA_LBF_LAUNCH(2);
-#undef SLA_LBF_LAUNCH
-    hipLaunchKernelGGL(linear_bwd_reduce_heads_kernel, dim3(cdiv(D * D, 256)), dim3(256), 0, st,
-                       (const float*)(ws + w.dw_head), (const float*)(ws + w.db_head), d_weight, d_bias, BH, D);
-  }
+  if (steps & LB_REDUCE)
+    hipLaunchKernelGGL((linear_bwd_finish_kernel<Tag, D>), dim3(xcd_grid(lists.wgs) + xcd_grid((int64_t)BH * (D / 8))), dim3(512),
+                       0, st, (const float*)m_part, (const float*)(ws + w.dz_part), (const float*)(ws + w.db_part), weight, kvt,
+                       (uint16_t*)(ws + w.ds), (uint16_t*)(ws + w.dst), (float*)(ws + w.dz), (float*)(ws + w.dw_head),
+                       (float*)(ws + w.db_head), w.sp.nsplit, BH * (D / 8), xcd_grid(lists.wgs), lists);
+  if (steps & LB_HEADS) launch_head_sums(hs, st);
   if (steps & LB_KEYS) {
-#define SLA_LBK_LAUNCH(FM)                                                                                                \
-  hipLaunchKernelGGL((linear_bwd_keys_kernel<Tag, D, FM>), dim3(w.sp.nsplit, BH), dim3(512), 0, st, (const uint16_t*)k,     \
-                     (const uint16_t*)v, (const uint16_t*)(ws + w.ds), (const uint16_t*)(ws + w.dst),                       \
-                     (const float*)(ws + w.dz), (uint16_t*)dk, (uint16_t*)dv, lin, L, w.sp.rows_per_split, accumulate)
-    if (fmap == SLA_FMAP_ELU) SLA_LBK_LAUNCH(SLA_FMAP_ELU);
-    else if (fmap == SLA_FMAP_RELU) SLA_LBK_LAUNCH(SLA_FMAP_RELU);
-    else SLA_LBK_LAUNCH(SLA_FMAP_SOFTMAX);
+#define SLA_LBK_LAUNCH(FM, ACC)                                                                                          \
+  hipLaunchKernelGGL((linear_bwd_keys_kernel<Tag, D, FM, ACC>), dim3(w.sp.nsplit, BH), dim3(512), 0, st, (const uint16_t*)k, \
+                     (const uint16_t*)v, (const uint16_t*)(ws + w.ds), (const uint16_t*)(ws + w.dst),                      \
+                     (const float*)(ws + w.dz), (uint16_t*)dk, (uint16_t*)dv, lin, L, w.sp.rows_per_split)
+    SLA_LB_FMAPS(SLA_LBK_LAUNCH)
 #undef SLA_LBK_LAUNCH
+#undef SLA_LB_FMAPS
   }
   return check_launch("linear_bwd");
 }
@@ -378,8 +362,8 @@ static void weight_grads_impl(const void* q, const void* dn, const void* gout, c
                      (const float*)(ws + w.ds_part), (const float*)(ws + w.dw_part), (const float*)(ws + w.dz_part),
                      (const float*)(ws + w.db_part), (uint16_t*)(ws + w.ds), (uint16_t*)(ws + w.dst), (float*)(ws + w.dz),
                      (float*)(ws + w.dw_head), (float*)(ws + w.db_head), w.st.nsplit, D);
-  hipLaunchKernelGGL(linear_bwd_reduce_heads_kernel, dim3(cdiv(D * D, 256)), dim3(256), 0, st,
-                     (const float*)(ws + w.dw_head), (const float*)(ws + w.db_head), d_weight, d_bias, BH, D);
+  launch_head_sums(HeadSums{(const float*)(ws + w.dw_head), (const float*)(ws + w.db_head), d_weight, d_bias, BH, D, D * D / 256},
+                   st);
 }
 void launch_weight_grads(int dtype, int D, const void* q, const void* dn, const void* gout, const void* y, const float* dden,
                          int BH, int L, int fmap, char* ws, float* d_weight, float* d_bias, hipStream_t st) {
@@ -395,7 +379,8 @@ void launch_weight_grads(int dtype, int D, const void* q, const void* dn, const 
 int linear_bwd_steps(const void* q, const void* k, const void* v, const int64_t* qkv_strides, const float* weight,
                      const float* bias, const void* d_out, const int64_t* do_strides, void* dq, void* dk, void* dv,
                      float* d_weight, float* d_bias, int dtype, int fmap, int B, int H, int L, int D, int flags,
-                     const void* states, void* workspace, int64_t workspace_bytes, void* stream, int steps) {
+                     const void* states, void* workspace, int64_t workspace_bytes, void* stream, int steps, const ColLists* lists,
+                     HeadSums* heads) {
   int rc = validate_linear(dtype, fmap, B, H, L, D);
   if (rc) return rc;
   SLA_REQUIRE((flags & ~(SLA_BWD_ACCUMULATE | SLA_BWD_STATES_READY)) == 0, SLA_ERR_BAD_ARG, "unknown flag bits in %d", flags);
@@ -418,7 +403,7 @@ int linear_bwd_steps(const void* q, const void* k, const void* v, const int64_t*
   char* ws = (char*)workspace;
 #define SLA_LINB_CASE(TAG, DD) \
   return linear_bwd_impl<TAG, DD>(q, k, v, weight, d_out, dq, dk, dv, lin, ldo, d_weight, d_bias, fmap, BH, L, flags, (const char*)states, ws, st, \
-                                  steps)
+                                  steps, lists ? *lists : ColLists{}, heads)
   if (dtype == SLA_BF16) {
     if (D == 128) SLA_LINB_CASE(bf16_tag, 128);
     SLA_LINB_CASE(bf16_tag, 64);

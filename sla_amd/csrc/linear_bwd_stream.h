@@ -19,6 +19,7 @@
 //   finish   : fixed-order sums of the slices' partials -> M^T (fp32), dz, db per head, and from them
 //              dS = M W (16 bit, both orientations) and this head's dW = M^T S (fp32)
 #pragma once
+#include "bwd_lists.h"
 #include "linear_state.h"
 
 namespace sla {
@@ -39,16 +40,18 @@ constexpr int LBS_TR = 128;   // rows per step of the stream kernel
 
 // Head dim 64 keeps half the registers and 60 KB of LDS, so two workgroups share a compute unit.  Against kernels with
 // row-wise temporaries (dn, y, dden) in memory, the backward of 16 heads x 6001 x 64, softmax map in half precision: rows 20.8 +
-// states 16.3 + sums 14.1 + heads 5.4 + keys 21.2 us; now stream 20.5 + finish 5.8 + heads 5.1 + keys 16.4.
-template <typename Tag, int D, int FMAP>
+// states 16.3 + sums 14.1 + heads 5.4 + keys 21.2 us; now stream 19.8 + finish 5.8 + keys 12.8.
+// Bound by the vector ALU in the row phase (30 instructions per element) with one workgroup per compute unit in step between
+// barriers: 12 heads x 32760 x 128, elu map: 137 us with the floats of a row carried along (the compiler then spills what was
+// fetched ahead, waiting for it) and each product waiting for its fragment, now 112.
+template <typename Tag, int D, int FMAP, bool ACC>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 128 ? 2 : 4, D == 128 ? 2 : 4))) void linear_bwd_stream_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ gout, const uint16_t* __restrict__ kvw,
     const uint16_t* __restrict__ z, uint16_t* __restrict__ dq, const RowLayout lin, const RowLayout ldo,
-    float* __restrict__ m_part, float* __restrict__ dz_part, float* __restrict__ db_part, int L, int rows_per_split,
-    int accumulate) {
-  // (the feature map is a template argument: as a run-time value every element's phi sits behind its own branch)
+    float* __restrict__ m_part, float* __restrict__ dz_part, float* __restrict__ db_part, int L, int rows_per_split) {
+  // (the feature map is a template argument: as a run-time value every element's phi sits behind its own branch; ACC: dq is
+  //  added to what the tensor holds)
   using E = Elem<Tag>;
-  constexpr int fmap = FMAP;
   constexpr int TR = LBS_TR;
   constexpr int TILE = TR * D * 2;               // bytes of one swizzled tile of rows
   constexpr int CPR = D / 8;                     // 16-byte pieces per row
@@ -57,15 +60,15 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 128 ? 
   constexpr int NT = D / 16, NC = D / 32;        // 16-column tiles of a row, 32-column fragments
   constexpr bool WEIGHT_G = D == 64;             // 1 / den goes to G, not to a
   constexpr int PSTR = D * 2 + 16;               // row pitch of sP: 16 rows x 16 bytes of a row-wise read cover every bank
-  __shared__ __attribute__((aligned(16))) char smem[3 * TILE + D * PSTR + 2 * TR * 4];
+  __shared__ __attribute__((aligned(16))) char smem[3 * TILE + D * PSTR + D * 4 + D * 2 + TR * 4];
   char* const sQ = smem;                         // raw q rows, then a (/ den) of the same rows
   char* const sG = smem + TILE;                  // G rows (then G / den)
   char* const sO = smem + 2 * TILE;              // dq rows of this step (16 bit)
   char* const sP = smem + 3 * TILE;              // folded state, P[d1][e]
   float* const sZ = reinterpret_cast<float*>(smem + 3 * TILE + D * PSTR);   // z[d1]
-  float* const sDD = sZ + TR;                                               // weight in dz of the row that sQ then holds
-  float (*sRed)[RPP][D] = reinterpret_cast<float (*)[RPP][D]>(smem);        // final cross-thread sums (over the tiles)
-  static_assert(2 * RPP * D * 4 <= 3 * TILE, "the final sums do not fit the tiles they reuse");
+  uint16_t* const sZ16 = reinterpret_cast<uint16_t*>(sZ + D);               // the same, as stored
+  float* const sDD = reinterpret_cast<float*>(sZ16 + D);                    // weight in dz of the row that sQ then holds
+  float (*sRed)[8][D] = reinterpret_cast<float (*)[8][D]>(smem);            // final sums over the waves (over the tiles)
 
   const int split = blockIdx.x, bh = blockIdx.y, nsplit = gridDim.x;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -79,7 +82,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 128 ? 
 
   const __amdgpu_buffer_rsrc_t q_rs = make_rsrc(q + lin.head(bh), lin.head_range_bytes(L, D));
   const __amdgpu_buffer_rsrc_t g_rs = make_rsrc(gout + ldo.head(bh), ldo.head_range_bytes(L, D));
-  const __amdgpu_buffer_rsrc_t dq_rs = make_rsrc(dq + lin.head(bh), accumulate ? lin.head_range_bytes(L, D) : 0u);
+  const __amdgpu_buffer_rsrc_t dq_rs = make_rsrc(dq + lin.head(bh), lin.head_range_bytes(L, D));
   uint16_t* const dqh = dq + lin.head(bh);
   const size_t pitch = (size_t)lin.sl;
   const uint32_t pitch_b = (uint32_t)lin.sl * 2u, pitch_gb = (uint32_t)ldo.sl * 2u;
@@ -102,7 +105,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 128 ? 
     for (int p = 0; p < D / RPP; ++p)
       *reinterpret_cast<i16x8_t*>(sP + (lrow + RPP * p) * PSTR + 16 * lp) =
           *reinterpret_cast<const i16x8_t*>(src + (size_t)(lrow + RPP * p) * D + 8 * lp);
-    if (tid < D) sZ[tid] = E::to_float(z[(size_t)bh * D + tid]);
+    if (tid < D) {
+      const uint16_t zz = z[(size_t)bh * D + tid];
+      sZ[tid] = E::to_float(zz);
+      sZ16[tid] = zz;
+    }
     // (the first step's barrier stands before the first read of either)
   }
 
@@ -116,7 +123,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 128 ? 
   for (int t = 0; t < 2; ++t)
 #pragma unroll
     for (int i = 0; i < MR; ++i) macc[t][i] = 0.f;
-  float zacc[8], bacc[8];
+  float zacc[8], bacc[8];                        // dz and db of the loader's eight columns
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
     zacc[e] = 0.f;
@@ -124,12 +131,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 128 ? 
   }
 
   const int prow = 16 * wave + l;
-  uint32_t acc_off[NT];       // (prow, 16 T + 4 h) in a row tile
-#pragma unroll
-  for (int T = 0; T < NT; ++T) acc_off[T] = lbs_off<D>(prow, 16 * T + 4 * h);
-  uint32_t g_off[NC];         // (prow, 32 c + 8 h): G in B-operand order
-#pragma unroll
-  for (int c = 0; c < NC; ++c) g_off[c] = lbs_off<D>(prow, 32 * c + 8 * h);
+  // (prow, 16 T + 4 h) in a row tile, and (prow, 32 c + 8 h), G in B-operand order: pieces of a row are exclusive-ored
+  const uint32_t acc_off0 = lbs_off<D>(prow, 4 * h), g_off0 = lbs_off<D>(prow, 8 * h);
+  const auto acc_off = [&](int T) __attribute__((always_inline)) { return acc_off0 ^ (uint32_t)(T * 32); };
+  const auto g_off = [&](int c) __attribute__((always_inline)) { return g_off0 ^ (uint32_t)(c * 64); };
   // A operand of t^T = P G^T: row d1 = 16 T + l of sP, e = 32 c + 8 h ..: + 16 PSTR per T, + 64 bytes per c
   const char* const p_base = sP + l * PSTR + h * 16;
   // transposing reads of the M phase, KM rows per product: rows KM c + tr_row (+ 4), columns MW tile + tr_col; + 4 KiB per c
@@ -158,12 +163,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 128 ? 
     for (int p = 0; p < NF; ++p) {
       const int grow = r0 + frow + FR * p;
       const i16x8_t o16 = *reinterpret_cast<const i16x8_t*>(sO + f_off[p]);
-      // (not accumulating: the descriptor is empty and rdq reads as zero; x + 0 keeps the 16-bit value)
-      i32x4_t w;
+      i32x4_t w = __builtin_bit_cast(i32x4_t, o16);
+      if (ACC)
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-        w[j] = (int)E::pack2(E::to_float((uint16_t)o16[2 * j]) + E::to_float((uint16_t)rdq[p][2 * j]),
-                             E::to_float((uint16_t)o16[2 * j + 1]) + E::to_float((uint16_t)rdq[p][2 * j + 1]));
+        for (int j = 0; j < 4; ++j)
+          w[j] = (int)E::pack2(E::to_float((uint16_t)o16[2 * j]) + E::to_float((uint16_t)rdq[p][2 * j]),
+                               E::to_float((uint16_t)o16[2 * j + 1]) + E::to_float((uint16_t)rdq[p][2 * j + 1]));
       if (grow < row_end) *reinterpret_cast<i32x4_t*>(dqh + (size_t)grow * pitch + 8 * lp) = w;
     }
     wave_lds_fence();     // the row phase rewrites these rows of sO
@@ -179,148 +184,113 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 128 ? 
 #pragma unroll
       for (int e = 0; e < 8; ++e) bacc[e] += E::to_float((uint16_t)rg[p][e]);
     }
-    __syncthreads();
+    lds_barrier();
     if (r0 + TR < row_end) fetch_qg(r0 + TR);
     // the previous step's dq rows leave now: what dq held was asked for a phase ago and has had time to arrive
     if (r0 > row_begin) flush_dq(r0 - TR);
 
     // ---- row phase ----
     {
-      // (the raw rows stay packed until phi' needs them again)
+      // (The raw rows stay packed until phi' needs them again, and what is formed from them is formed again: with the row's
+      //  floats carried along, the rows fetched ahead were what the compiler spilled, and waited for.)
       i16x4_t xraw[NT];
 #pragma unroll
-      for (int T = 0; T < NT; ++T) xraw[T] = *reinterpret_cast<const i16x4_t*>(sQ + acc_off[T]);
-      auto xv = [&](int T, int j) __attribute__((always_inline)) { return E::to_float((uint16_t)xraw[T][j]); };
-      float mx = 0.f, inv = 1.f, inv_den;
-      i32x2_t apk[NT];         // a = phi(q), 16 bit (it is a 16-bit tensor in the reference)
-      {
-        float a[NT][4];
-        if (fmap == SLA_FMAP_SOFTMAX) {
-          mx = xv(0, 0);
+      for (int T = 0; T < NT; ++T) xraw[T] = *reinterpret_cast<const i16x4_t*>(sQ + acc_off(T));
+      i16x8_t gf[NC];
 #pragma unroll
-          for (int T = 0; T < NT; ++T)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) mx = fmaxf(mx, xv(T, j));
-          mx = fmaxf(mx, __shfl_xor(mx, 16));
-          mx = fmaxf(mx, __shfl_xor(mx, 32));
-          float sum = 0.f;
-#pragma unroll
-          for (int T = 0; T < NT; ++T)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              a[T][j] = __expf(xv(T, j) - mx);
-              sum += a[T][j];
-            }
-          sum += __shfl_xor(sum, 16);
-          sum += __shfl_xor(sum, 32);
-          inv = 1.0f / sum;
-#pragma unroll
-          for (int T = 0; T < NT; ++T)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) a[T][j] = round16<Tag>(a[T][j] * inv);
-        } else {
-#pragma unroll
-          for (int T = 0; T < NT; ++T)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) a[T][j] = fmap_pointwise<Tag>(fmap, xv(T, j));
-        }
-        float den = 0.f;
-#pragma unroll
-        for (int T = 0; T < NT; ++T) {
-          const f32x4_t zz = *reinterpret_cast<const f32x4_t*>(sZ + 16 * T + 4 * h);
-#pragma unroll
-          for (int j = 0; j < 4; ++j) den += a[T][j] * zz[j];
-        }
-        den += __shfl_xor(den, 16);
-        den += __shfl_xor(den, 32);
-        den += 1e-5f;
-        inv_den = 1.0f / den;
-        // a or a/den takes the place of the raw row (this lane's own places)
-        const float aw = WEIGHT_G ? 1.0f : inv_den;
-#pragma unroll
-        for (int T = 0; T < NT; ++T) {
-          i32x2_t w;
-          w[0] = (int)E::pack2(a[T][0] * aw, a[T][1] * aw);
-          w[1] = (int)E::pack2(a[T][2] * aw, a[T][3] * aw);
-          *reinterpret_cast<i32x2_t*>(sQ + acc_off[T]) = w;
-          apk[T][0] = (int)E::pack2(a[T][0], a[T][1]);
-          apk[T][1] = (int)E::pack2(a[T][2], a[T][3]);
-        }
-      }
-
-      // t^T = P G^T: tiles of 16 d1 x 16 rows
+      for (int c = 0; c < NC; ++c) gf[c] = *reinterpret_cast<const i16x8_t*>(sG + g_off(c));
+      __builtin_amdgcn_sched_barrier(0);
+      // t^T = P G^T (tiles of 16 d1 x 16 rows) beside a = phi(q): a product's fragment is read some products ahead
       f32x4_t t[NT];
 #pragma unroll
       for (int T = 0; T < NT; ++T) t[T] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int c = 0; c < NC; ++c) {
-        const i16x8_t b = *reinterpret_cast<const i16x8_t*>(sG + g_off[c]);
+      for (int c = 0; c < NC; ++c)
 #pragma unroll
         for (int T = 0; T < NT; ++T)
-          t[T] = E::mfma16(*reinterpret_cast<const i16x8_t*>(p_base + T * 16 * PSTR + c * 64), b, t[T]);
-        if (WEIGHT_G) {              // G / den over the same places (the row's four lanes hold all of it)
-          i32x4_t w;
+          t[T] = E::mfma16(*reinterpret_cast<const i16x8_t*>(p_base + T * 16 * PSTR + c * 64), gf[c], t[T]);
+      i32x2_t apk[NT];         // a = phi(q), 16 bit (it is a 16-bit tensor in the reference)
+      float mx = 0.f, inv = 1.f;
+      phi_quarters<Tag, FMAP, NT>(xraw, apk, mx, inv);
+      constexpr int AHEAD = D == 128 ? 4 : 2;
+      __builtin_amdgcn_sched_group_barrier(0x100, AHEAD, 0);
 #pragma unroll
-          for (int j = 0; j < 4; ++j)
-            w[j] = (int)E::pack2(E::to_float((uint16_t)b[2 * j]) * inv_den, E::to_float((uint16_t)b[2 * j + 1]) * inv_den);
-          *reinterpret_cast<i32x4_t*>(sG + g_off[c]) = w;
-        }
+      for (int i = 0; i < NC * NT - AHEAD; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x002, FMAP == SLA_FMAP_RELU ? 4 : 10, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      }
+      __builtin_amdgcn_sched_group_barrier(0x008, AHEAD, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      // den: z as an A operand with sixteen equal rows, the summed index in the order a row's four lanes hold a
+      i16x8_t zf[NC];
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        const uint16_t* zp = sZ16 + 32 * c + 4 * h;
+        zf[c] = concat4(*reinterpret_cast<const i16x4_t*>(zp), *reinterpret_cast<const i16x4_t*>(zp + 16));
+      }
+      f32x4_t dsum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        const i32x4_t w = {apk[2 * c][0], apk[2 * c][1], apk[2 * c + 1][0], apk[2 * c + 1][1]};
+        dsum = E::mfma16(zf[c], __builtin_bit_cast(i16x8_t, w), dsum);
       }
       float s = 0.f;
 #pragma unroll
       for (int T = 0; T < NT; ++T)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const uint32_t w = (uint32_t)apk[T][j >> 1];
-          s += E::to_float((uint16_t)((j & 1) ? (w >> 16) : (w & 0xffff))) * t[T][j];
-        }
-      s += __shfl_xor(s, 16);
-      s += __shfl_xor(s, 32);
+        for (int j = 0; j < 4; ++j) s += unpack_quarter<Tag>(apk[T], j) * t[T][j];
+      __builtin_amdgcn_sched_group_barrier(0x100, 2 * NC, 0);
+      __builtin_amdgcn_sched_group_barrier(0x008, NC, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      const float inv_den = 1.0f / (dsum[0] + 1e-5f);
+      s = sum_quarters(s);
       const float dden = -s * inv_den * inv_den;
       if (h == 0) sDD[prow] = WEIGHT_G ? dden : -s * inv_den;     // the weight of what sQ holds (a, or a/den) in dz
-
-      // da = t / den + dden z (in place), then dq = phi'(q) da
+      f32x4_t zz[NT];
+#pragma unroll
+      for (int T = 0; T < NT; ++T) zz[T] = *reinterpret_cast<const f32x4_t*>(sZ + 16 * T + 4 * h);
+      __builtin_amdgcn_sched_barrier(0);
+      // a or a/den takes the place of the raw row, G/den that of G (this lane's own places)
 #pragma unroll
       for (int T = 0; T < NT; ++T) {
-        const f32x4_t zz = *reinterpret_cast<const f32x4_t*>(sZ + 16 * T + 4 * h);
+        i32x2_t w = apk[T];
+        if (!WEIGHT_G)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) t[T][j] = __builtin_fmaf(t[T][j], inv_den, dden * zz[j]);
+          for (int j2 = 0; j2 < 2; ++j2)
+            w[j2] = (int)E::pack2(unpack_quarter<Tag>(apk[T], 2 * j2) * inv_den, unpack_quarter<Tag>(apk[T], 2 * j2 + 1) * inv_den);
+        *reinterpret_cast<i32x2_t*>(sQ + acc_off(T)) = w;
       }
-      if (fmap == SLA_FMAP_RELU) {
+      if (WEIGHT_G)
 #pragma unroll
-        for (int T = 0; T < NT; ++T)
+        for (int c = 0; c < NC; ++c) {
+          const i16x8_t gr = *reinterpret_cast<const i16x8_t*>(sG + g_off(c));
+          i32x4_t w;
 #pragma unroll
-          for (int j = 0; j < 4; ++j) t[T][j] = xv(T, j) > 0.f ? t[T][j] : 0.f;
-      } else if (fmap == SLA_FMAP_ELU) {
+          for (int j = 0; j < 4; ++j)
+            w[j] = (int)E::pack2(E::to_float((uint16_t)gr[2 * j]) * inv_den, E::to_float((uint16_t)gr[2 * j + 1]) * inv_den);
+          *reinterpret_cast<i32x4_t*>(sG + g_off(c)) = w;
+        }
+      // da = t / den + dden z (in place), then dq = phi'(q) da
 #pragma unroll
-        for (int T = 0; T < NT; ++T)
+      for (int T = 0; T < NT; ++T)
 #pragma unroll
-          for (int j = 0; j < 4; ++j) t[T][j] = xv(T, j) > 0.f ? t[T][j] : t[T][j] * __expf(xv(T, j));
-      } else {
-        float dot = 0.f;
-#pragma unroll
-        for (int T = 0; T < NT; ++T)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) dot += __expf(xv(T, j) - mx) * inv * t[T][j];       // the unrounded softmax
-        dot += __shfl_xor(dot, 16);
-        dot += __shfl_xor(dot, 32);
-#pragma unroll
-        for (int T = 0; T < NT; ++T)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) t[T][j] = __expf(xv(T, j) - mx) * inv * (t[T][j] - dot);
-      }
+        for (int j = 0; j < 4; ++j) t[T][j] = __builtin_fmaf(t[T][j], inv_den, dden * zz[T][j]);
+      forget_floats<NT>(xraw);
+      phi_quarters_backward<Tag, FMAP, NT>(xraw, mx, inv, t);
 #pragma unroll
       for (int T = 0; T < NT; ++T) {
         i32x2_t w;
         w[0] = (int)E::pack2(t[T][0], t[T][1]);
         w[1] = (int)E::pack2(t[T][2], t[T][3]);
-        *reinterpret_cast<i32x2_t*>(sO + acc_off[T]) = w;
+        *reinterpret_cast<i32x2_t*>(sO + acc_off(T)) = w;
       }
     }
-    __syncthreads();
+    lds_barrier();
 
-    // ---- M += a^T G / den ; dz ----
+    // ---- M += a^T G / den ----
     // (what dq holds so far is asked for here, where the row phase's registers are free, and used in the next step)
+    if (ACC)
 #pragma unroll
     for (int p = 0; p < NF; ++p) rdq[p] = buf_load_b128(dq_rs, (uint32_t)(r0 + frow + FR * p) * pitch_b + 16 * lp);
     __builtin_amdgcn_sched_barrier(0);      // (asked for first: the loop's next wait on memory covers these too)
@@ -340,14 +310,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 128 ? 
     }
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
-      const int row = lrow + RPP * p;
-      const uint32_t o = ld_off + p * 8192;
-      const i16x8_t an = *reinterpret_cast<const i16x8_t*>(sQ + o);
-      const float dd = sDD[row];
+      const i16x8_t an = *reinterpret_cast<const i16x8_t*>(sQ + ld_off + p * 8192);
+      const float dd = sDD[lrow + RPP * p];
 #pragma unroll
       for (int e = 0; e < 8; ++e) zacc[e] = __builtin_fmaf(dd, E::to_float((uint16_t)an[e]), zacc[e]);
     }
-    __syncthreads();
+    lds_barrier();
   }
   flush_dq(row_begin + (row_end - 1 - row_begin) / TR * TR);
 
@@ -363,22 +331,30 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 128 ? 
       *reinterpret_cast<f32x4_t*>(mo + (size_t)col * D + MW * mt + 8 * i4 + 4 * (D == 128 ? g2 : h)) = v4;
     }
   }
-  // (the loop's last barrier has passed: sQ is free)
+  lds_barrier();           // (the last dq rows have left sO)
+  // the lanes of a wave that hold the same columns; then the waves
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    sRed[0][lrow][8 * lp + e] = zacc[e];
-    sRed[1][lrow][8 * lp + e] = bacc[e];
-  }
-  __syncthreads();
-  if (tid < D) {
-    float s0 = 0.f, s1 = 0.f;
-#pragma unroll 8
-    for (int rr = 0; rr < RPP; ++rr) {
-      s0 += sRed[0][rr][tid];
-      s1 += sRed[1][rr][tid];
+  for (int which = 0; which < 2; ++which) {
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      v[e] = which ? bacc[e] : zacc[e];
+      if (CPR == 8)          // lane ^ 8
+        v[e] += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v[e]), 0x128, 0xf, 0xf, true));
+      v[e] = sum_quarters(v[e]);
     }
-    dz_part[pidx * D + tid] = s0;
-    db_part[pidx * D + tid] = s1;
+    if (lane < CPR)
+#pragma unroll
+      for (int x = 0; x < 2; ++x)
+        *reinterpret_cast<f32x4_t*>(&sRed[which][wave][8 * lp + 4 * x]) = f32x4_t{v[4 * x], v[4 * x + 1], v[4 * x + 2], v[4 * x + 3]};
+  }
+  lds_barrier();
+  if (tid < 2 * D) {
+    const int which = tid / D, col = tid % D;
+    float sum = 0.f;
+#pragma unroll
+    for (int w = 0; w < 8; ++w) sum += sRed[which][w][col];
+    (which ? db_part : dz_part)[pidx * D + col] = sum;
   }
 }
 
@@ -389,13 +365,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 128 ? 
 //   dv^T = dS^T c^T and dc^T = dS v^T as 16x16x32 products (a key's row spread over 4 lanes, B operands read row-wise
 //   from the wave's tiles); dk, dv go back over the tiles and leave as whole rows, added to what dk, dv held (asked
 //   for at the start of the tile) when accumulating.
-template <typename Tag, int D, int FMAP>
+template <typename Tag, int D, int FMAP, bool ACC>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 128 ? 2 : 4, D == 128 ? 2 : 4))) void linear_bwd_keys_kernel(
     const uint16_t* __restrict__ k, const uint16_t* __restrict__ v, const uint16_t* __restrict__ ds,
     const uint16_t* __restrict__ dst, const float* __restrict__ dz, uint16_t* __restrict__ dk, uint16_t* __restrict__ dv,
-    const RowLayout lin, int L, int rows_per_split, int accumulate) {
+    const RowLayout lin, int L, int rows_per_split) {
   using E = Elem<Tag>;
-  constexpr int fmap = FMAP;
   constexpr int CPR = D / 8;                     // 16-byte pieces per row
   constexpr int NF = CPR / 4, FR = 64 / CPR;     // passes over a wave's 16 rows, rows per pass
   constexpr int NT = D / 16, NC = D / 32;        // 16-column tiles of a row, 32-column fragments
@@ -422,13 +397,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 128 ? 
     }
     if (tid < D) sDZ[tid] = dz[(size_t)bh * D + tid];
   }
-  __syncthreads();
+  lds_barrier();
 
   const uint32_t range = lin.head_range_bytes(L, D);
   const __amdgpu_buffer_rsrc_t k_rs = make_rsrc(k + lin.head(bh), range);
   const __amdgpu_buffer_rsrc_t v_rs = make_rsrc(v + lin.head(bh), range);
-  const __amdgpu_buffer_rsrc_t dk_rs = make_rsrc(dk + lin.head(bh), accumulate ? range : 0u);
-  const __amdgpu_buffer_rsrc_t dv_rs = make_rsrc(dv + lin.head(bh), accumulate ? range : 0u);
+  const __amdgpu_buffer_rsrc_t dk_rs = make_rsrc(dk + lin.head(bh), range);
+  const __amdgpu_buffer_rsrc_t dv_rs = make_rsrc(dv + lin.head(bh), range);
   uint16_t* const dkh = dk + lin.head(bh);
   uint16_t* const dvh = dv + lin.head(bh);
   const size_t pitch = (size_t)lin.sl;
@@ -469,6 +444,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 128 ? 
     wave_lds_fence();
     // what dk, dv hold (for this tile) and the next tile's rows: both have the whole tile to arrive
     i16x8_t rdk[NF], rdv[NF];
+    if (ACC)
 #pragma unroll
     for (int p = 0; p < NF; ++p) {
       const uint32_t o = (uint32_t)(r0 + frow + FR * p) * pitch_b + 16 * lp;
@@ -480,49 +456,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 128 ? 
     i16x4_t xraw[NT];
 #pragma unroll
     for (int T = 0; T < NT; ++T) xraw[T] = *reinterpret_cast<const i16x4_t*>(tK + acc_off[T]);
-    auto xv = [&](int T, int j) __attribute__((always_inline)) { return E::to_float((uint16_t)xraw[T][j]); };
+    i32x2_t apk[NT];
     float mx = 0.f, inv = 1.f;
-    {
-      float a[NT][4];
-      if (fmap == SLA_FMAP_SOFTMAX) {
-        mx = xv(0, 0);
+    phi_quarters<Tag, FMAP, NT>(xraw, apk, mx, inv);
+    // c = phi(k) over the raw rows (this lane's own places; a key's gradients depend on its own row only, so rows
+    // past the end, which are never written, need no care)
 #pragma unroll
-        for (int T = 0; T < NT; ++T)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) mx = fmaxf(mx, xv(T, j));
-        mx = fmaxf(mx, __shfl_xor(mx, 16));
-        mx = fmaxf(mx, __shfl_xor(mx, 32));
-        float sum = 0.f;
-#pragma unroll
-        for (int T = 0; T < NT; ++T)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            a[T][j] = __expf(xv(T, j) - mx);
-            sum += a[T][j];
-          }
-        sum += __shfl_xor(sum, 16);
-        sum += __shfl_xor(sum, 32);
-        inv = 1.0f / sum;
-#pragma unroll
-        for (int T = 0; T < NT; ++T)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) a[T][j] = round16<Tag>(a[T][j] * inv);
-      } else {
-#pragma unroll
-        for (int T = 0; T < NT; ++T)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) a[T][j] = fmap_pointwise<Tag>(fmap, xv(T, j));
-      }
-      // c = phi(k) over the raw rows (this lane's own places; a key's gradients depend on its own row only, so rows
-      // past the end, which are never written, need no care)
-#pragma unroll
-      for (int T = 0; T < NT; ++T) {
-        i32x2_t w;
-        w[0] = (int)E::pack2(a[T][0], a[T][1]);
-        w[1] = (int)E::pack2(a[T][2], a[T][3]);
-        *reinterpret_cast<i32x2_t*>(tK + acc_off[T]) = w;
-      }
-    }
+    for (int T = 0; T < NT; ++T) *reinterpret_cast<i32x2_t*>(tK + acc_off[T]) = apk[T];
     wave_lds_fence();
     // dv^T = dS^T c^T ; dc^T = dS v^T
     f32x4_t dva[NT], dca[NT];
@@ -549,29 +489,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 128 ? 
 #pragma unroll
       for (int j = 0; j < 4; ++j) dca[T][j] += zz[j];
     }
-    if (fmap == SLA_FMAP_RELU) {
-#pragma unroll
-      for (int T = 0; T < NT; ++T)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) dca[T][j] = xv(T, j) > 0.f ? dca[T][j] : 0.f;
-    } else if (fmap == SLA_FMAP_ELU) {
-#pragma unroll
-      for (int T = 0; T < NT; ++T)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) dca[T][j] = xv(T, j) > 0.f ? dca[T][j] : dca[T][j] * __expf(xv(T, j));
-    } else {
-      float dot = 0.f;
-#pragma unroll
-      for (int T = 0; T < NT; ++T)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) dot += __expf(xv(T, j) - mx) * inv * dca[T][j];       // the unrounded softmax
-      dot += __shfl_xor(dot, 16);
-      dot += __shfl_xor(dot, 32);
-#pragma unroll
-      for (int T = 0; T < NT; ++T)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) dca[T][j] = __expf(xv(T, j) - mx) * inv * (dca[T][j] - dot);
-    }
+    phi_quarters_backward<Tag, FMAP, NT>(xraw, mx, inv, dca);
 #pragma unroll
     for (int T = 0; T < NT; ++T) {
       i32x2_t wk, wv;
@@ -583,13 +501,14 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 128 ? 
       *reinterpret_cast<i32x2_t*>(tV + acc_off[T]) = wv;
     }
     wave_lds_fence();
-    // whole rows out: 16-bit value + what the tensor held, one rounded add (nothing held when not accumulating)
+    // whole rows out; ACC: 16-bit value + what the tensor held, one rounded add
 #pragma unroll
     for (int p = 0; p < NF; ++p) {
       const int grow = r0 + frow + FR * p;
       const i16x8_t k16 = *reinterpret_cast<const i16x8_t*>(tK + f_off[p]);
       const i16x8_t v16 = *reinterpret_cast<const i16x8_t*>(tV + f_off[p]);
-      i32x4_t wk, wv;
+      i32x4_t wk = __builtin_bit_cast(i32x4_t, k16), wv = __builtin_bit_cast(i32x4_t, v16);
+      if (ACC)
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         wk[j] = (int)E::pack2(E::to_float((uint16_t)k16[2 * j]) + E::to_float((uint16_t)rdk[p][2 * j]),
@@ -614,28 +533,31 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 128 ? 
 //   kind 0: sums the columns d1 = i0 .. + 15 of every row e and forms 16 rows of dS;
 //   kind 1: sums the rows e = i0 .. + 15 and forms 16 columns of dW^T.
 // Either way it holds all its products need of M after one hand-over through LDS; the partials are read twice, from the
-// caches.  The slices are summed in two halves, whose sums are then added:
-//   HALVES 2: 512 threads, the halves side by side, eight slices' loads in flight: for a launch that has the chip to itself;
-//   HALVES 1: 256 threads, one half after the other, at most 72 registers per lane: what the dK/dV kernel of head dim 128
-//             leaves free beside its two workgroups on a compute unit (with more the launch would only get its turn when
-//             dK/dV is done).  The same bits.
+// caches.  The slices are summed in two halves side by side, whose sums are then added, eight slices' loads in flight.
 // Against a kernel for the sums and one for the products (on the vector ALU, M through memory in both orientations): 9.3
-// against 12.8 + 10.5 us (B2 H4 L4096), beside dK/dV 18 against 14 + 37 us (B1 H12 L9360) and 25 against 19 + 46 (L32760).
-template <typename Tag, int D, int HALVES>
-__global__ __launch_bounds__(256 * HALVES) __attribute__((amdgpu_waves_per_eu(HALVES == 2 ? 4 : 7))) void linear_bwd_finish_kernel(
+// against 12.8 + 10.5 us (B2 H4 L4096).  The first `first_wg` workgroups, a multiple of eight, build the lists of the map for
+// the attention backward: both are short and bound by latency.
+template <typename Tag, int D>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void linear_bwd_finish_kernel(
     const float* __restrict__ m_part, const float* __restrict__ dz_part, const float* __restrict__ db_part,
     const float* __restrict__ weight, const uint16_t* __restrict__ kvt, uint16_t* __restrict__ ds, uint16_t* __restrict__ dst,
-    float* __restrict__ dz, float* __restrict__ dw_head, float* __restrict__ db_head, int nsplit, int total) {
+    float* __restrict__ dz, float* __restrict__ dw_head, float* __restrict__ db_head, int nsplit, int total, int first_wg,
+    const ColLists lists) {
   using E = Elem<Tag>;
   constexpr int DD = D * D;
   constexpr int NR = D / 64;               // f32x4 sums per thread
   constexpr int KQ = D / 4;                // products per tile: four summed indices each
   constexpr int EP = D + 1;                // row pitch of the strip of rows
-  constexpr int NT = HALVES == 2 ? 1 : NR; // 16-wide tiles per wave
-  constexpr int BATCH = HALVES == 2 ? 8 : 4;
-  __shared__ __attribute__((aligned(16))) float s_half[HALVES == 2 ? NR * 256 * 4 : 4];
-  __shared__ __attribute__((aligned(16))) float sm[16 * EP];
-  const int logical = xcd_remap(blockIdx.x, gridDim.x, total);
+  constexpr int S_HALF = NR * 256 * 4;
+  constexpr int LDS = 4 * (S_HALF + 16 * EP) > COL_LDS ? 4 * (S_HALF + 16 * EP) : COL_LDS;
+  __shared__ __attribute__((aligned(16))) char smem[LDS];
+  float* const s_half = reinterpret_cast<float*>(smem);
+  float* const sm = s_half + S_HALF;
+  if ((int)blockIdx.x < first_wg) {
+    if ((int)blockIdx.x < lists.wgs) col_lists_body(lists, blockIdx.x, smem);
+    return;
+  }
+  const int logical = xcd_remap((int)blockIdx.x - first_wg, (int)gridDim.x - first_wg, total);
   if (logical < 0) return;
   const int bh = logical / (D / 8), rest = logical % (D / 8), kind = rest / (D / 16), i0 = 16 * (rest % (D / 16));
   const int tid = threadIdx.x & 255, half = threadIdx.x >> 8, lane = tid & 63, wave = threadIdx.x >> 6;
@@ -645,34 +567,25 @@ __global__ __launch_bounds__(256 * HALVES) __attribute__((amdgpu_waves_per_eu(HA
   const int er = kind == 0 ? tid >> 2 : tid >> 4, dc = kind == 0 ? 4 * (tid & 3) : 4 * (tid & 15);
   mp += kind == 0 ? (size_t)er * D + i0 + dc : (size_t)(i0 + er) * D + dc;
   const size_t vec = kind == 0 ? (size_t)64 * D : 64;
-  f32x4_t acc[NR], acc2[NR];
+  f32x4_t acc[NR];
 #pragma unroll
-  for (int i = 0; i < NR; ++i) {
-    acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    acc2[i] = acc[i];
-  }
-  if (HALVES == 2) {
-    sum_slices<NR, BATCH>(mp + (half ? (size_t)n0 * DD : 0), half ? nsplit - n0 : n0, DD, vec, acc);
-    if (half)
+  for (int i = 0; i < NR; ++i) acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  sum_slices<NR>(mp + (half ? (size_t)n0 * DD : 0), half ? nsplit - n0 : n0, DD, vec, acc);
+  if (half)
 #pragma unroll
-      for (int i = 0; i < NR; ++i) *reinterpret_cast<f32x4_t*>(s_half + (i * 256 + tid) * 4) = acc[i];
-  } else {
-    sum_slices<NR, BATCH>(mp, n0, DD, vec, acc);
-    sum_slices<NR, BATCH>(mp + (size_t)n0 * DD, nsplit - n0, DD, vec, acc2);
-  }
-  if (kind == 0 && half == HALVES - 1 && tid < 32) {
+    for (int i = 0; i < NR; ++i) *reinterpret_cast<f32x4_t*>(s_half + (i * 256 + tid) * 4) = acc[i];
+  if (kind == 0 && half && tid < 32) {
     const float* q = (tid < 16 ? dz_part : db_part) + (size_t)bh * nsplit * D + i0 + (tid & 15);
     float sum = 0.f;
 #pragma unroll 8
     for (int sp = 0; sp < nsplit; ++sp) sum += q[(size_t)sp * D];
     (tid < 16 ? dz : db_head)[(size_t)bh * D + i0 + (tid & 15)] = sum;
   }
-  if (HALVES == 2) __syncthreads();
+  __syncthreads();
   if (!half)
 #pragma unroll
     for (int i = 0; i < NR; ++i) {
-      if (HALVES == 2) acc2[i] = *reinterpret_cast<const f32x4_t*>(s_half + (i * 256 + tid) * 4);
-      acc[i] += acc2[i];
+      acc[i] += *reinterpret_cast<const f32x4_t*>(s_half + (i * 256 + tid) * 4);
       if (kind == 0) {
         *reinterpret_cast<f32x4_t*>(sm + (er + 64 * i) * 16 + dc) = acc[i];                    // [e][d1]
       } else {
@@ -681,45 +594,42 @@ __global__ __launch_bounds__(256 * HALVES) __attribute__((amdgpu_waves_per_eu(HA
       }
     }
   __syncthreads();
+  const int tile = wave;                   // 16 wide; head dim 64: four of the eight waves
+  if (tile >= D / 16) return;
+  f32x4_t o = {0.f, 0.f, 0.f, 0.f};
+  if (kind == 0) {
+    // row d1 = l of M, column d2 = 16 tile + l of W; summed index e = 4 kk + h
+    const int d2 = 16 * tile + l;
 #pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    const int tile = NT * wave + t;
-    if (tile >= D / 16) break;
-    f32x4_t o = {0.f, 0.f, 0.f, 0.f};
-    if (kind == 0) {
-      // row d1 = l of M, column d2 = 16 tile + l of W; summed index e = 4 kk + h
-      const int d2 = 16 * tile + l;
+    for (int k0 = 0; k0 < KQ; k0 += 16) {
+      float wb[16];
 #pragma unroll
-      for (int k0 = 0; k0 < KQ; k0 += 16) {
-        float wb[16];
+      for (int x = 0; x < 16; ++x) wb[x] = weight[(size_t)(4 * (k0 + x) + h) * D + d2];
 #pragma unroll
-        for (int x = 0; x < 16; ++x) wb[x] = weight[(size_t)(4 * (k0 + x) + h) * D + d2];
-#pragma unroll
-        for (int x = 0; x < 16; ++x)
-          o = __builtin_amdgcn_mfma_f32_16x16x4f32(sm[(4 * (k0 + x) + h) * 16 + l], round16<Tag>(wb[x]), o, 0, 0, 0);
-      }
-      // rows d1 = 4 h + i, column d2
-      i32x2_t w;
-      w[0] = (int)E::pack2(o[0], o[1]);
-      w[1] = (int)E::pack2(o[2], o[3]);
-      *reinterpret_cast<i32x2_t*>(dst + (size_t)bh * DD + (size_t)d2 * D + i0 + 4 * h) = w;
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        ds[(size_t)bh * DD + (size_t)(i0 + 4 * h + i) * D + d2] = (uint16_t)((uint32_t)w[i >> 1] >> (16 * (i & 1)));
-    } else {
-      // row d2 = 16 tile + l of S^T, column e = l of M; summed index d1 = KQ h + kk (adjacent per lane)
-      const uint16_t* st = kvt + (size_t)bh * DD + (size_t)(16 * tile + l) * D + KQ * h;
-#pragma unroll
-      for (int c = 0; c < KQ / 8; ++c) {
-        const i16x8_t sf = *reinterpret_cast<const i16x8_t*>(st + 8 * c);
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-          o = __builtin_amdgcn_mfma_f32_16x16x4f32(E::to_float((uint16_t)sf[j]), sm[l * EP + KQ * h + 8 * c + j], o, 0, 0, 0);
-      }
-      // rows d2 = 16 tile + 4 h + i, column e: the layout linear_bwd_reduce_heads_kernel adds up
-#pragma unroll
-      for (int i = 0; i < 4; ++i) dw_head[(size_t)bh * DD + (size_t)(16 * tile + 4 * h + i) * D + i0 + l] = o[i];
+      for (int x = 0; x < 16; ++x)
+        o = __builtin_amdgcn_mfma_f32_16x16x4f32(sm[(4 * (k0 + x) + h) * 16 + l], round16<Tag>(wb[x]), o, 0, 0, 0);
     }
+    // rows d1 = 4 h + i, column d2
+    i32x2_t w;
+    w[0] = (int)E::pack2(o[0], o[1]);
+    w[1] = (int)E::pack2(o[2], o[3]);
+    *reinterpret_cast<i32x2_t*>(dst + (size_t)bh * DD + (size_t)d2 * D + i0 + 4 * h) = w;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      ds[(size_t)bh * DD + (size_t)(i0 + 4 * h + i) * D + d2] = (uint16_t)((uint32_t)w[i >> 1] >> (16 * (i & 1)));
+  } else {
+    // row d2 = 16 tile + l of S^T, column e = l of M; summed index d1 = KQ h + kk (adjacent per lane)
+    const uint16_t* st = kvt + (size_t)bh * DD + (size_t)(16 * tile + l) * D + KQ * h;
+#pragma unroll
+    for (int c = 0; c < KQ / 8; ++c) {
+      const i16x8_t sf = *reinterpret_cast<const i16x8_t*>(st + 8 * c);
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        o = __builtin_amdgcn_mfma_f32_16x16x4f32(E::to_float((uint16_t)sf[j]), sm[l * EP + KQ * h + 8 * c + j], o, 0, 0, 0);
+    }
+    // rows d2 = 16 tile + 4 h + i, column e: the layout linear_bwd_reduce_heads_kernel adds up
+#pragma unroll
+    for (int i = 0; i < 4; ++i) dw_head[(size_t)bh * DD + (size_t)(16 * tile + 4 * h + i) * D + i0 + l] = o[i];
   }
 }
 

@@ -163,6 +163,102 @@ static __device__ __forceinline__ void phi_backward(int fmap, const float (&x)[D
   }
 }
 
+// ---- rows spread over four lanes: lane (l, h) of a wave holds elements 16 T + 4 h + j of row l, T < NT, j < 4 ---------------
+// Sum (maximum) over the four lanes l, l + 16, l + 32, l + 48, in all of them.
+template <typename Op>
+static __device__ __forceinline__ float over_quarters(float x, Op op) {
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  x = op(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return op(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+static __device__ __forceinline__ float sum_quarters(float x) {
+  return over_quarters(x, [](float a, float b) { return a + b; });
+}
+// phi of such rows, packed (the values are rounded where the reference holds 16 bit, two at a time); softmax: the row's
+// maximum and 1 / sum, from which phi_quarters_backward forms the unrounded values again.  Nothing of a row is kept as floats.
+template <typename Tag, int FMAP, int NT>
+static __device__ __forceinline__ void phi_quarters(const i16x4_t (&x)[NT], i32x2_t (&apk)[NT], float& mx, float& inv) {
+  using E = Elem<Tag>;
+  const auto xv = [&](int T, int j) __attribute__((always_inline)) { return E::to_float((uint16_t)x[T][j]); };
+  float ex[FMAP == SLA_FMAP_SOFTMAX ? NT : 1][4];
+  if (FMAP == SLA_FMAP_SOFTMAX) {
+    mx = xv(0, 0);
+#pragma unroll
+    for (int T = 0; T < NT; ++T)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) mx = fmaxf(mx, xv(T, j));
+    mx = over_quarters(mx, [](float u, float v) { return fmaxf(u, v); });
+    float sum = 0.f;
+#pragma unroll
+    for (int T = 0; T < NT; ++T)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        ex[T][j] = __expf(xv(T, j) - mx);
+        sum += ex[T][j];
+      }
+    inv = 1.0f / sum_quarters(sum);
+  }
+#pragma unroll
+  for (int T = 0; T < NT; ++T)
+#pragma unroll
+    for (int j2 = 0; j2 < 2; ++j2) {
+      float v[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int j = 2 * j2 + i;
+        if constexpr (FMAP == SLA_FMAP_SOFTMAX) v[i] = ex[T][j] * inv;
+        else if constexpr (FMAP == SLA_FMAP_RELU) v[i] = fmaxf(xv(T, j), 0.f);
+        else v[i] = xv(T, j) > 0.f ? xv(T, j) : __expf(xv(T, j)) - 1.0f;
+      }
+      if (FMAP == SLA_FMAP_ELU) {              // (elu rounded, then + 1 rounded)
+        float r0, r1;
+        round16_pair<Tag>(v[0], v[1], r0, r1);
+        v[0] = r0 + 1.0f;
+        v[1] = r1 + 1.0f;
+      }
+      apk[T][j2] = (int)E::pack2(v[0], v[1]);
+    }
+}
+// element j of a packed group of four
+template <typename Tag>
+static __device__ __forceinline__ float unpack_quarter(const i32x2_t& w, int j) {
+  const uint32_t p = (uint32_t)w[j >> 1];
+  return Elem<Tag>::to_float((uint16_t)((j & 1) ? (p >> 16) : (p & 0xffffu)));
+}
+// g = phi'(x) g
+template <typename Tag, int FMAP, int NT>
+static __device__ __forceinline__ void phi_quarters_backward(const i16x4_t (&x)[NT], float mx, float inv, f32x4_t (&g)[NT]) {
+  using E = Elem<Tag>;
+  const auto xv = [&](int T, int j) __attribute__((always_inline)) { return E::to_float((uint16_t)x[T][j]); };
+  float dot = 0.f;
+  if (FMAP == SLA_FMAP_SOFTMAX) {
+#pragma unroll
+    for (int T = 0; T < NT; ++T)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) dot += __expf(xv(T, j) - mx) * inv * g[T][j];
+    dot = sum_quarters(dot);
+  }
+#pragma unroll
+  for (int T = 0; T < NT; ++T)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (FMAP == SLA_FMAP_SOFTMAX) g[T][j] = __expf(xv(T, j) - mx) * inv * (g[T][j] - dot);
+      else if (FMAP == SLA_FMAP_ELU) g[T][j] = xv(T, j) > 0.f ? g[T][j] : g[T][j] * __expf(xv(T, j));
+      else g[T][j] = xv(T, j) > 0.f ? g[T][j] : 0.f;
+    }
+}
+// Keeps the compiler from carrying floats formed from the row's values from one use of them to the next: it sees new values.
+template <int NT>
+static __device__ __forceinline__ void forget_floats(i16x4_t (&x)[NT]) {
+#pragma unroll
+  for (int T = 0; T < NT; ++T) {
+    i32x2_t w = __builtin_bit_cast(i32x2_t, x[T]);
+    asm volatile("" : "+v"(w));
+    x[T] = __builtin_bit_cast(i16x4_t, w);
+  }
+}
+
 // Split of L among workgroups for the streaming state kernels.
 struct LinSplit {
   int nsplit, rows_per_split;

@@ -1,4 +1,4 @@
-// Ordering of a caller's second stream against its main one (module_fwd.hip, module_bwd.hip).
+// Ordering of a caller's second stream against its main one (module_fwd.hip, sage.hip).
 #pragma once
 #include "common.h"
 

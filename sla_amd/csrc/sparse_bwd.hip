@@ -7,7 +7,7 @@
 //   dQ = scale * dS K ; dK = scale * dS^T Q ; dV = P^T dO
 //
 // Four kernels.
-//   delta      : one pass over o and do.
+//   delta      : one pass over o and do (the streaming dQ kernel forms it itself).
 //   col_lists  : the reference scans the dense int8 map column in the dK/dV kernel (about
 //                1/density wasted iterations); here the map is turned once into per-key-block
 //                lists of the query blocks that selected it.
@@ -19,11 +19,30 @@
 //                in registers as B operands; P and dS leave the accumulators in B-operand layout
 //                for dV^T += dO^T P and dK^T += Q^T dS (Q^T, dO^T via transposing LDS reads).
 //                Four waves: two key halves x two halves of the head dimension.
+#include "bwd_lists.h"
 #include "bwd_steps.h"
 
 namespace sla {
 
 int validate_attn_shape(int dtype, int B, int H, int L, int D, int BLKQ, int BLKK, int topk, int lut_elem_bytes);
+
+// Four values rounded to 16 bit; `add`: then added, with one more rounding, to what the four places hold.
+template <typename E>
+static __device__ __forceinline__ void store_4(uint16_t* dst, float a, float b, float c, float d, int add) {
+  i32x2_t w;
+  w[0] = (int)E::pack2(a, b);
+  w[1] = (int)E::pack2(c, d);
+  if (add) {
+    const i32x2_t old = *reinterpret_cast<const i32x2_t*>(dst);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const uint32_t x = (uint32_t)w[j], y = (uint32_t)old[j];
+      w[j] = (int)E::pack2(E::to_float((uint16_t)(x & 0xffffu)) + E::to_float((uint16_t)(y & 0xffffu)),
+                           E::to_float((uint16_t)(x >> 16)) + E::to_float((uint16_t)(y >> 16)));
+    }
+  }
+  *reinterpret_cast<i32x2_t*>(dst) = w;
+}
 
 // ---- delta ------------------------------------------------------------------------------
 template <typename Tag, int D>
@@ -47,160 +66,25 @@ __global__ __launch_bounds__(256) void bwd_delta_kernel(const uint16_t* __restri
   if (row < rows && col == 0) delta[row] = s;
 }
 
-// ---- per-key-block lists ------------------------------------------------------------------
-// One workgroup of COL_NW wavefronts per strip of 64 key blocks.  Every wavefront takes its own chunk of
-// 64 map rows (query blocks): it reads them with coalesced 16-byte loads and transposes them through its
-// private LDS tile; lane c counts the ones of column c in that chunk.  After a barrier every wave knows
-// how many entries the chunks before its own contribute to each column and writes its matches at that
-// offset, walking the chunk in row order, so list[bh][n][0..count) holds the selecting query blocks in
-// ascending order.  Capacity Mblk per list (only `count` entries are ever touched).
-constexpr int COL_NW = 8;
-__global__ __launch_bounds__(64 * COL_NW) void bwd_col_lists_kernel(const int8_t* __restrict__ sparse_map,
-                                                                    int* __restrict__ list, int* __restrict__ count,
-                                                                    int Mblk, int Nblk, int vec_ok) {
-  __shared__ __attribute__((aligned(16))) int8_t tile[COL_NW][64][80];
-  __shared__ int cnt[COL_NW][64];
-  const int bh = blockIdx.y;
-  const int n0 = blockIdx.x * 64;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int n = n0 + lane;
-  const int8_t* base = sparse_map + (size_t)bh * Mblk * Nblk;
-  int* out = list + ((size_t)bh * Nblk + (n < Nblk ? n : 0)) * Mblk;
-  // lane -> (row lr + 16j, 16-byte chunk lc) of the tile
-  const int lr = lane >> 2, lc = (lane & 3) * 16;
-  int done = 0;              // entries of column `lane` written by earlier rounds
-  for (int r0 = 0; r0 < Mblk; r0 += 64 * COL_NW) {
-    const int m0 = r0 + 64 * wave;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int m = m0 + lr + 16 * j;
-      i32x4_t x = {0, 0, 0, 0};
-      if (m < Mblk) {
-        if (vec_ok && n0 + lc + 16 <= Nblk) {
-          x = *reinterpret_cast<const i32x4_t*>(base + (size_t)m * Nblk + n0 + lc);
-        } else {
-          int8_t* b = reinterpret_cast<int8_t*>(&x);
-          for (int e = 0; e < 16; ++e)
-            if (n0 + lc + e < Nblk) b[e] = base[(size_t)m * Nblk + n0 + lc + e];
-        }
-      }
-      *reinterpret_cast<i32x4_t*>(&tile[wave][lr + 16 * j][lc]) = x;
-    }
-    wave_lds_fence();
-    int mine = 0;
-#pragma unroll 16
-    for (int r = 0; r < 64; ++r) mine += tile[wave][r][lane] == 1;
-    cnt[wave][lane] = mine;
-    __syncthreads();
-    int before = 0, all = 0;
-#pragma unroll
-    for (int w = 0; w < COL_NW; ++w) {
-      const int cw = cnt[w][lane];
-      before += w < wave ? cw : 0;
-      all += cw;
-    }
-    if (n < Nblk) {
-      int c = done + before;
-#pragma unroll 16
-      for (int r = 0; r < 64; ++r)
-        if (tile[wave][r][lane] == 1) out[c++] = m0 + r;
-    }
-    done += all;
-    __syncthreads();         // cnt and the tiles are rewritten by the next round
-  }
-  if (wave == 0 && n < Nblk) count[(size_t)bh * Nblk + n] = done;
+// ---- lists of the map; short jobs -------------------------------------------------------------
+__global__ __launch_bounds__(64 * COL_NW) void bwd_col_lists_kernel(const ColLists job) {
+  __shared__ __attribute__((aligned(16))) char smem[COL_LDS];
+  col_lists_body(job, blockIdx.x, smem);
 }
 
-// ---- work items of the dK/dV kernel --------------------------------------------------------
-// A key block that very many query blocks selected (an attention "sink") would make one workgroup walk a list
-// many times the average length.  Lists longer than `seg` entries are therefore cut into segments of `seg`; every
-// segment is one work item.  item = {bh, key block, segment, slot}: slot < 0 for a key block with a single segment
-// (the workgroup writes dK / dV itself), otherwise the index of the fp32 partial this segment writes; the partials
-// of a key block occupy consecutive slots and are added in segment order by bwd_dkdv_reduce_kernel.
-// One workgroup of 1024 threads walks all (head, key block) pairs in order, eight per thread and round, with a running
-// prefix sum.
-__global__ __launch_bounds__(1024) void bwd_segments_kernel(const int* __restrict__ count, int* __restrict__ nseg,
-                                                            int* __restrict__ slot0, i32x4_t* __restrict__ items,
-                                                            int* __restrict__ totals, int nblocks, int Nblk, int seg,
-                                                            int max_items, int max_slots) {
-  constexpr int EPT = 8;                      // consecutive (head, key block) pairs per thread and round
-  __shared__ int wsum[2][16];
-  __shared__ int base[2];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  if (tid == 0) base[0] = base[1] = 0;
-  __syncthreads();
-  for (int i0 = 0; i0 < nblocks; i0 += 1024 * EPT) {
-    const int first = i0 + tid * EPT;
-    int ns[EPT];
-    int own_a = 0, own_b = 0;
-#pragma unroll
-    for (int e = 0; e < EPT; ++e) {
-      ns[e] = first + e < nblocks ? max(1, (count[first + e] + seg - 1) / seg) : 0;
-      own_a += ns[e];
-      own_b += ns[e] > 1 ? ns[e] : 0;
-    }
-    int a = own_a, b = own_b;                 // inclusive scans inside the wave
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int ta = __shfl_up(a, o), tb = __shfl_up(b, o);
-      if (lane >= o) {
-        a += ta;
-        b += tb;
-      }
-    }
-    if (lane == 63) {
-      wsum[0][wave] = a;
-      wsum[1][wave] = b;
-    }
-    __syncthreads();
-    int pa = 0, pb = 0, ta = 0, tb = 0;
-#pragma unroll
-    for (int w = 0; w < 16; ++w) {
-      pa += w < wave ? wsum[0][w] : 0;
-      pb += w < wave ? wsum[1][w] : 0;
-      ta += wsum[0][w];
-      tb += wsum[1][w];
-    }
-    int first_item = base[0] + pa + a - own_a, first_slot = base[1] + pb + b - own_b;
-#pragma unroll
-    for (int e = 0; e < EPT; ++e) {
-      const int i = first + e;
-      if (i < nblocks) {
-        const int ms = ns[e] > 1 ? ns[e] : 0;
-        nseg[i] = ns[e];
-        slot0[i] = first_slot;
-        const int bh = i / Nblk, nb = i - bh * Nblk;
-        // (a map whose rows hold more ones than the topk the workspace was sized for cannot overrun the tables: its
-        //  surplus items are dropped)
-        for (int sg = 0; sg < ns[e]; ++sg)
-          if (first_item + sg < max_items && first_slot + ms <= max_slots)
-            items[first_item + sg] = i32x4_t{bh, nb, sg, ns[e] > 1 ? first_slot + sg : -1};
-          else if (first_item + sg < max_items)
-            items[first_item + sg] = i32x4_t{bh, nb, sg, -2};
-        first_item += ns[e];
-        first_slot += ms;
-      }
-    }
-    __syncthreads();
-    if (tid == 0) {
-      base[0] += ta;
-      base[1] += tb;
-    }
-    __syncthreads();
-  }
-  if (tid == 0) {
-    totals[0] = min(base[0], max_items);
-    totals[1] = min(base[1], max_slots);
-  }
+// the work items and the sum of the heads where no dQ launch takes them along
+__global__ __launch_bounds__(64) void bwd_short_jobs_kernel(const Segments segs, const HeadSums heads) {
+  if ((int)blockIdx.x < segs.wgs) segments_body(segs, blockIdx.x);
+  else head_sums_body(heads, (int)blockIdx.x - segs.wgs);
 }
 
 // grid (Nblk, BH), 256 threads: key blocks whose list was cut add their partials (fp32, [slot][dk | dv][64][D]) in
-// segment order and write dK, dV; all others leave at once.
+// segment order and write dK, dV (`add`: added to what is there); all others leave at once.  (Behind bwd_dkdv_kernel only.)
 template <typename Tag, int D>
 __global__ __launch_bounds__(256) void bwd_dkdv_reduce_kernel(const int* __restrict__ nseg, const int* __restrict__ slot0,
                                                               const float* __restrict__ part, uint16_t* __restrict__ dk,
                                                               uint16_t* __restrict__ dv, const RowLayout lin, int L, int Nblk,
-                                                              int max_slots) {
+                                                              int max_slots, int add) {
   using E = Elem<Tag>;
   const int nb = blockIdx.x, bh = blockIdx.y;
   const int ns = nseg[(size_t)bh * Nblk + nb];
@@ -212,11 +96,8 @@ __global__ __launch_bounds__(256) void bwd_dkdv_reduce_kernel(const int* __restr
     const int which = idx / (64 * D), rem = idx - which * (64 * D);
     const int row = nb * 64 + rem / D, col = rem % D;
     if (row < L) {
-      i32x2_t w;
-      w[0] = (int)E::pack2(acc[0], acc[1]);
-      w[1] = (int)E::pack2(acc[2], acc[3]);
       uint16_t* dst = (which ? dv : dk) + lin.head(bh) + (size_t)row * (size_t)lin.sl + col;
-      *reinterpret_cast<i32x2_t*>(dst) = w;
+      store_4<E>(dst, acc[0], acc[1], acc[2], acc[3], add);
     }
   }
 }
@@ -232,7 +113,7 @@ __global__ __launch_bounds__(BLKQ * 2) __attribute__((amdgpu_waves_per_eu(D == 6
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
     const uint16_t* __restrict__ d_o, const float* __restrict__ lse, const float* __restrict__ delta,
     const void* __restrict__ lut, int lut64, uint16_t* __restrict__ dq, const RowLayout lin, const RowLayout ldo, int L,
-    int Mblk, int topk, float qk_scale, int total) {
+    int Mblk, int topk, float qk_scale, int total, int add) {
   using E = Elem<Tag>;
   constexpr int BLKK = 64;
   constexpr int NT = BLKQ * 2;
@@ -398,12 +279,9 @@ __global__ __launch_bounds__(BLKQ * 2) __attribute__((amdgpu_waves_per_eu(D == 6
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-      for (int i4 = 0; i4 < 4; ++i4) {
-        i32x2_t w;
-        w[0] = (int)E::pack2(dqacc[dt][4 * i4 + 0] * qk_scale, dqacc[dt][4 * i4 + 1] * qk_scale);
-        w[1] = (int)E::pack2(dqacc[dt][4 * i4 + 2] * qk_scale, dqacc[dt][4 * i4 + 3] * qk_scale);
-        *reinterpret_cast<i32x2_t*>(orow + 32 * dt + 8 * i4 + 4 * g) = w;
-      }
+      for (int i4 = 0; i4 < 4; ++i4)
+        store_4<E>(orow + 32 * dt + 8 * i4 + 4 * g, dqacc[dt][4 * i4 + 0] * qk_scale, dqacc[dt][4 * i4 + 1] * qk_scale,
+                   dqacc[dt][4 * i4 + 2] * qk_scale, dqacc[dt][4 * i4 + 3] * qk_scale, add);
   }
 }
 
@@ -421,7 +299,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 3
     const uint16_t* __restrict__ d_o, const float* __restrict__ lse, const float* __restrict__ delta,
     const int* __restrict__ list, const int* __restrict__ count, const i32x4_t* __restrict__ items,
     const int* __restrict__ totals, float* __restrict__ part, int seg, uint16_t* __restrict__ dk, uint16_t* __restrict__ dv,
-    const RowLayout lin, const RowLayout ldo, int L, int Mblk, int Nblk, float qk_scale) {
+    const RowLayout lin, const RowLayout ldo, int L, int Mblk, int Nblk, float qk_scale, int add) {
   using E = Elem<Tag>;
   constexpr int TQ = 64;                  // query rows per LDS tile
   constexpr int SUB = BLKQ / TQ;          // tiles per listed query block
@@ -646,13 +524,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 3
 #pragma unroll
       for (int i4 = 0; i4 < 4; ++i4) {
         const int d0 = 32 * (DH * dh + dt) + 8 * i4 + 4 * g;
-        i32x2_t w;
-        w[0] = (int)E::pack2(dkacc[dt][4 * i4 + 0] * qk_scale, dkacc[dt][4 * i4 + 1] * qk_scale);
-        w[1] = (int)E::pack2(dkacc[dt][4 * i4 + 2] * qk_scale, dkacc[dt][4 * i4 + 3] * qk_scale);
-        *reinterpret_cast<i32x2_t*>(dkrow + d0) = w;
-        w[0] = (int)E::pack2(dvacc[dt][4 * i4 + 0], dvacc[dt][4 * i4 + 1]);
-        w[1] = (int)E::pack2(dvacc[dt][4 * i4 + 2], dvacc[dt][4 * i4 + 3]);
-        *reinterpret_cast<i32x2_t*>(dvrow + d0) = w;
+        store_4<E>(dkrow + d0, dkacc[dt][4 * i4 + 0] * qk_scale, dkacc[dt][4 * i4 + 1] * qk_scale,
+                   dkacc[dt][4 * i4 + 2] * qk_scale, dkacc[dt][4 * i4 + 3] * qk_scale, add);
+        store_4<E>(dvrow + d0, dvacc[dt][4 * i4 + 0], dvacc[dt][4 * i4 + 1], dvacc[dt][4 * i4 + 2], dvacc[dt][4 * i4 + 3], add);
       }
   }
 }
@@ -661,10 +535,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 3
 // list[bh][n][0..count[bh][n]) = the query blocks that selected key block n, ascending; capacity Mblk per list
 // (also used by the backward of the complement-mode linear branch)
 void launch_col_lists(const int8_t* sparse_map, int* list, int* count, int BH, int Mblk, int Nblk, hipStream_t st) {
-  // 16-byte loads of map rows need 16-byte aligned rows
-  const int vec_ok = (Nblk % 16 == 0) && ((uintptr_t)sparse_map % 16 == 0);
-  hipLaunchKernelGGL(bwd_col_lists_kernel, dim3(cdiv(Nblk, 64), BH), dim3(64 * COL_NW), 0, st, sparse_map, list, count, Mblk, Nblk,
-                     vec_ok);
+  const ColLists job = col_lists_job(sparse_map, list, count, BH, Mblk, Nblk);
+  hipLaunchKernelGGL(bwd_col_lists_kernel, dim3(job.wgs), dim3(64 * COL_NW), 0, st, job);
+}
+void launch_head_sums(const HeadSums& heads, hipStream_t st) {
+  hipLaunchKernelGGL(bwd_short_jobs_kernel, dim3(heads.wgs), dim3(64), 0, st, Segments{}, heads);
 }
 
 }  // namespace sla
@@ -674,7 +549,7 @@ namespace sla {
 struct BwdWs {
   int seg;                  // longest stretch of a key block's list one workgroup walks
   int64_t max_items, max_slots;
-  size_t delta, count, list, nseg, slot0, items, totals, part, total;
+  size_t delta, count, list, nseg, slot0, done, items, totals, part, total;
 };
 static BwdWs bwd_ws(int BH, int L, int D, int BLKQ, int BLKK, int topk) {
   const int64_t M = cdiv(L, BLKQ), N = cdiv(L, BLKK);
@@ -697,6 +572,7 @@ static BwdWs bwd_ws(int BH, int L, int D, int BLKQ, int BLKK, int topk) {
   w.list = off;   off += align_up((int64_t)BH * N * M * 4, 256);
   w.nseg = off;   off += align_up((int64_t)BH * N * 4, 256);
   w.slot0 = off;  off += align_up((int64_t)BH * N * 4, 256);
+  w.done = off;   off += align_up((int64_t)BH * N * 4, 256);
   w.items = off;  off += align_up(w.max_items * 16, 256);
   w.totals = off; off += 256;
   w.part = off;   off += align_up(w.max_slots * 2 * 64 * D * 4, 256);
@@ -711,8 +587,8 @@ template <typename Tag, int D, int BLKQ>
 static int bwd_impl(const void* q, const void* k, const void* v, const void* o, const void* d_o, const float* lse,
                     const int8_t* sparse_map, const void* lut, int lut64, void* dq, void* dk, void* dv,
                     const RowLayout& lin, const RowLayout& ldo, int BH, int L, int topk, float qk_scale, char* ws,
-                    hipStream_t st, int steps) {
-  if (steps == 0) return SLA_OK;        // (arguments checked, nothing asked for)
+                    hipStream_t st, int steps, const HeadSums& heads) {
+  const int add = (steps & SB_ADD) != 0;
   const BwdWs w = bwd_ws(BH, L, D, BLKQ, 64, topk);
   const int Mblk = cdiv(L, BLKQ), Nblk = cdiv(L, 64);
   float* delta = (float*)(ws + w.delta);
@@ -723,12 +599,13 @@ static int bwd_impl(const void* q, const void* k, const void* v, const void* o, 
   if (steps & SB_LISTS) launch_col_lists(sparse_map, list, count, BH, Mblk, Nblk, st);
   int* nseg = (int*)(ws + w.nseg);
   int* slot0 = (int*)(ws + w.slot0);
+  int* done = (int*)(ws + w.done);
   i32x4_t* items = (i32x4_t*)(ws + w.items);
   int* totals = (int*)(ws + w.totals);
   float* part = (float*)(ws + w.part);
-  if (steps & SB_LISTS)
-    hipLaunchKernelGGL(bwd_segments_kernel, dim3(1), dim3(1024), 0, st, count, nseg, slot0, items, totals, BH * Nblk, Nblk,
-                       w.seg, (int)w.max_items, (int)w.max_slots);
+  const Segments segs = {count, nseg, slot0, done, items, totals, BH * Nblk, Nblk, w.seg, (int)w.max_items, (int)w.max_slots,
+                         cdiv(BH * Nblk, SEG_PAIRS)};
+  const int jobs = segs.wgs + heads.wgs;
   const int total_q = BH * Mblk;
   const bool contig = lin.sl == D && ldo.sl == D;
   // The kernels of sparse_bwd_stream.h walk 64-row query blocks with 32-bit byte offsets inside a head; a 128-row query
@@ -751,41 +628,47 @@ static int bwd_impl(const void* q, const void* k, const void* v, const void* o, 
   if ((steps & SB_DQ) && !stream_dq)
     hipLaunchKernelGGL((bwd_delta_kernel<Tag, D>), dim3((unsigned)((rows + RPB - 1) / RPB)), dim3(256), 0, st,
                        (const uint16_t*)o, (const uint16_t*)d_o, ldo, delta, rows, L);
+  if ((steps & SB_DQ) && !stream_dq)
+    hipLaunchKernelGGL(bwd_short_jobs_kernel, dim3(jobs), dim3(64), 0, st, segs, heads);
 #define SLA_BWD_LAUNCH(CONTIG)                                                                                              \
   if (!(steps & SB_DQ)) {                                                                                                   \
   } else if (stream_dq)                                                                                                     \
-    hipLaunchKernelGGL((bwd_dq_stream_kernel<Tag, D>), dim3(xcd_grid(total_q64)), dim3(64), 0, st, (const uint16_t*)q,         \
-                       (const uint16_t*)k, (const uint16_t*)v, (const uint16_t*)d_o, (const uint16_t*)o, lse, delta, lut,   \
-                       lut64, (uint16_t*)dq, lin, ldo, L, Mblk64, topk, qk_scale, total_q64, wide);                        \
+    hipLaunchKernelGGL((bwd_dq_stream_kernel<Tag, D>), dim3(xcd_grid(jobs) + xcd_grid(total_q64)), dim3(64), 0, st,           \
+                       (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, (const uint16_t*)d_o, (const uint16_t*)o, \
+                       lse, delta, lut, lut64, (uint16_t*)dq, lin, ldo, L, Mblk64, topk, qk_scale, total_q64, wide, add,     \
+                       xcd_grid(jobs), segs, heads);                                                                        \
   else                                                                                                                      \
     hipLaunchKernelGGL((bwd_dq_kernel<Tag, D, BLKQ, CONTIG>), dim3(xcd_grid(total_q)), dim3(BLKQ * 2), 0, st,               \
                        (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, (const uint16_t*)d_o, lse, delta, lut,   \
-                       lut64, (uint16_t*)dq, lin, ldo, L, Mblk, topk, qk_scale, total_q);                                  \
+                       lut64, (uint16_t*)dq, lin, ldo, L, Mblk, topk, qk_scale, total_q, add);                                \
   if (!(steps & SB_DKDV)) {                                                                                                 \
   } else if (stream_dkdv)                                                                                                   \
     hipLaunchKernelGGL((bwd_dkdv_stream_kernel<Tag, D>), dim3(xcd_grid(w.max_items)), dim3(128), 0, st, (const uint16_t*)q,    \
                        (const uint16_t*)k, (const uint16_t*)v, (const uint16_t*)d_o, lse, delta, list, count, items,       \
-                       totals, part, w.seg, (uint16_t*)dk, (uint16_t*)dv, lin, ldo, L, Mblk, Nblk, qk_scale, wide);       \
+                       totals, part, w.seg, (uint16_t*)dk, (uint16_t*)dv, lin, ldo, L, Mblk, Nblk, qk_scale, wide, add,    \
+                       nseg, done);                                                                                        \
   else                                                                                                                      \
     hipLaunchKernelGGL((bwd_dkdv_kernel<Tag, D, BLKQ, CONTIG>), dim3(xcd_grid(w.max_items)), dim3(256), 0, st,             \
                        (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, (const uint16_t*)d_o, lse, delta, list,  \
-                       count, items, totals, part, w.seg, (uint16_t*)dk, (uint16_t*)dv, lin, ldo, L, Mblk, Nblk, qk_scale);
+                       count, items, totals, part, w.seg, (uint16_t*)dk, (uint16_t*)dv, lin, ldo, L, Mblk, Nblk, qk_scale,  \
+                       add);
   if (contig) {
     SLA_BWD_LAUNCH(true)
   } else {
     SLA_BWD_LAUNCH(false)
   }
 #undef SLA_BWD_LAUNCH
-  if (steps & SB_DKDV)
+  if ((steps & SB_DKDV) && !stream_dkdv)
     hipLaunchKernelGGL((bwd_dkdv_reduce_kernel<Tag, D>), dim3(Nblk, BH), dim3(256), 0, st, nseg, slot0, part, (uint16_t*)dk,
-                       (uint16_t*)dv, lin, L, Nblk, (int)w.max_slots);
+                       (uint16_t*)dv, lin, L, Nblk, (int)w.max_slots, add);
   return check_launch("sparse_attn_bwd");
 }
 
 int attn_bwd_steps(const void* q, const void* k, const void* v, const int64_t* qkv_strides, const void* o, const void* d_o,
                    const int64_t* do_strides, const float* lse, const int8_t* sparse_map, const void* lut, int lut_elem_bytes,
                    void* dq, void* dk, void* dv, int dtype, int B, int H, int L, int D, int BLKQ, int BLKK, int topk,
-                   float qk_scale, void* workspace, int64_t workspace_bytes, void* stream, int steps) {
+                   float qk_scale, void* workspace, int64_t workspace_bytes, void* stream, int steps, const HeadSums* heads,
+                   ColLists* lists) {
   int rc = validate_attn_shape(dtype, B, H, L, D, BLKQ, BLKK, topk, lut_elem_bytes);
   if (rc) return rc;
   SLA_REQUIRE(q && k && v && o && d_o && lse && sparse_map && dq && dk && dv && workspace && (lut || topk == 0),
@@ -807,10 +690,16 @@ int attn_bwd_steps(const void* q, const void* k, const void* v, const int64_t* q
   hipStream_t st = (hipStream_t)stream;
   char* ws = (char*)workspace;
   const int lut64 = lut_elem_bytes == 8;
+  if (lists) {
+    const BwdWs w = bwd_ws(BH, L, D, BLKQ, 64, topk);
+    *lists = col_lists_job(sparse_map, (int*)(ws + w.list), (int*)(ws + w.count), BH, cdiv(L, BLKQ), cdiv(L, 64));
+  }
+  if (steps == 0) return SLA_OK;        // (arguments checked, nothing asked for)
+  const HeadSums none{}, &hs = heads ? *heads : none;
 #define SLA_BWD_CASE(TAG, DD, BQ)                                                                                          \
   if (D == DD && BLKQ == BQ)                                                                                               \
   return bwd_impl<TAG, DD, BQ>(q, k, v, o, d_o, lse, sparse_map, lut, lut64, dq, dk, dv, lin, ldo, BH, L, topk, qk_scale, \
-                               ws, st, steps)
+                               ws, st, steps, hs)
   if (dtype == SLA_BF16) {
     SLA_BWD_CASE(bf16_tag, 128, 64);
     SLA_BWD_CASE(bf16_tag, 128, 128);

@@ -77,8 +77,10 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
     const uint16_t* __restrict__ d_o, const float* __restrict__ lse, const float* __restrict__ delta,
     const int* __restrict__ list, const int* __restrict__ count, const i32x4_t* __restrict__ items,
     const int* __restrict__ totals, float* __restrict__ part, int seg, uint16_t* __restrict__ dk, uint16_t* __restrict__ dv,
-    const RowLayout lin, const RowLayout ldo, int L, int Mblk, int Nblk, float qk_scale, int wide) {
-  // (wide = 1: the lists name 128-row query blocks; an entry is then walked as its two 64-row halves)
+    const RowLayout lin, const RowLayout ldo, int L, int Mblk, int Nblk, float qk_scale, int wide, int add,
+    const int* __restrict__ nseg, int* __restrict__ done) {
+  // (wide = 1: the lists name 128-row query blocks; an entry is then walked as its two 64-row halves.  add: the gradients are
+  //  added, rounded, to what dk and dv hold)
   using E = Elem<Tag>;
   using T32 = BwdTile<D>;
   constexpr int DC = D / 16, DT = D / 32;
@@ -140,6 +142,15 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
 #pragma unroll
   for (int i = 0; i < (NG * GEN / 16 + 127) / 128; ++i)
     if (i * 128 + tid < NG * GEN / 16) reinterpret_cast<i32x4_t*>(smem)[i * 128 + tid] = i32x4_t{0, 0, 0, 0};
+
+  // what dk and dv hold, asked for before the last unit's arithmetic
+  const int krow0 = nb * 64 + w * 32;
+  TileRows<D> old[2];
+  const auto fetch_old = [&]() __attribute__((always_inline)) {
+    if (!add || slot >= 0) return;
+    old[0].fetch(dk + head_off + (size_t)krow0 * pitch, L - krow0, lane, pitch);
+    old[1].fetch(dv + head_off + (size_t)krow0 * pitch, L - krow0, lane, pitch);
+  };
 
   f32x16_t dkacc[DT], dvacc[DT];
 #pragma unroll
@@ -416,6 +427,7 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
       E2 = E3;
     }
     // the last unit: no scores left to form beside its arithmetic
+    fetch_old();
     if (__builtin_expect(E0 + 64 > L, 0)) mask_rows(E0 + 32);
 #pragma unroll
     for (int grp = 0; grp < 4; ++grp) tr_frags(last_at, grp);
@@ -430,6 +442,7 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
       second_products(grp);
     }
   }
+  if (nent <= 0) fetch_old();
 #undef SLA_DKDV_REQUEST_Q
 #undef SLA_DKDV_REQUEST_DO
 #undef SLA_DKDV_REQUEST_LD
@@ -437,7 +450,8 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
 
   const auto turned = [&](float x) __attribute__((always_inline)) { return __builtin_fmaf(x, -qk_scale, 0.f); };   // (+0 for an empty sum)
   if (slot >= 0) {
-    // one segment of a long list: fp32 partial [dk | dv][64][D], added up by bwd_dkdv_reduce_kernel
+    // One segment of a long list: fp32 partial [dk | dv][64][D].  The workgroup that finishes a key block's last segment adds
+    // all of them up, in segment order: its count is raised only when a workgroup's whole partial is visible to the others.
     float* pk = part + (size_t)slot * (2 * 64 * D) + (size_t)(w * 32 + r) * D;
     float* pv = pk + 64 * D;
 #pragma unroll
@@ -450,6 +464,22 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
         *reinterpret_cast<f32x4_t*>(pv + d0) =
             f32x4_t{dvacc[dt][4 * i4 + 0], dvacc[dt][4 * i4 + 1], dvacc[dt][4 * i4 + 2], dvacc[dt][4 * i4 + 3]};
       }
+    __threadfence();
+    __syncthreads();
+    const int ns = nseg[(size_t)bh * Nblk + nb];
+    if (tid == 0) entries[0] = atomicAdd(&done[(size_t)bh * Nblk + nb], 1);
+    __syncthreads();
+    if (entries[0] != ns - 1) return;
+    __threadfence();
+    const float* p0 = part + (size_t)(slot - sg) * (2 * 64 * D);
+    for (int idx = tid * 4; idx < 2 * 64 * D; idx += 128 * 4) {
+      f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+      for (int x = 0; x < ns; ++x) acc += *reinterpret_cast<const f32x4_t*>(p0 + (size_t)x * (2 * 64 * D) + idx);
+      const int which = idx / (64 * D), rem = idx - which * (64 * D);
+      const int row = nb * 64 + rem / D, col = rem % D;
+      if (row < L) store_4<E>((which ? dv : dk) + head_off + (size_t)row * pitch + col, acc[0], acc[1], acc[2], acc[3], add);
+    }
     return;
   }
   // The rounded rows go through LDS (both waves are done with the generations) and leave as whole rows in streaming
@@ -457,7 +487,6 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
   // back when the kernel ends.
   __syncthreads();
   uint16_t* const stage = reinterpret_cast<uint16_t*>(smem) + w * (32 * TileRows<D>::SSTR);
-  const int krow0 = nb * 64 + w * 32;
 #pragma unroll
   for (int which = 0; which < 2; ++which) {
     constexpr int SSTR = TileRows<D>::SSTR;
@@ -478,6 +507,7 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
     wave_lds_fence();
     TileRows<D> t;
     t.unpark(stage, lane);
+    if (add) t.template add<E>(old[which]);
     t.store_streaming((which == 0 ? dk : dv) + head_off + (size_t)krow0 * pitch, L - krow0, lane, pitch);
     wave_lds_fence();
   }
@@ -512,8 +542,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
     const uint16_t* __restrict__ d_o, const uint16_t* __restrict__ o, const float* __restrict__ lse, float* __restrict__ delta,
     const void* __restrict__ lut, int lut64, uint16_t* __restrict__ dq, const RowLayout lin, const RowLayout ldo, int L,
-    int Mblk, int topk, float qk_scale, int total, int wide) {
-  // (Mblk: 64-row blocks per head.  wide = 1: the look-up table has one row per 128-row block, which both halves follow)
+    int Mblk, int topk, float qk_scale, int total, int wide, int add, int first_wg, const Segments segs, const HeadSums heads) {
+  // (Mblk: 64-row blocks per head.  wide = 1: the look-up table has one row per 128-row block, which both halves follow.  add:
+  //  dQ is added, rounded, to what dq holds.  The first `first_wg` workgroups, a multiple of eight, take the short jobs along
+  //  that dK/dV and the caller wait for: they are done long before the rest.)
   using E = Elem<Tag>;
   using T32 = BwdTile<D>;
   constexpr int DC = D / 16, DT = D / 32;
@@ -523,7 +555,13 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
   __shared__ __attribute__((aligned(16))) uint8_t smem[4 * TILE];      // K generation 0, 1; V generation 0, 1
   __shared__ uint16_t entries[DQ_STREAM_MAX_T];                        // this block's look-up row
 
-  const int logical = xcd_remap(blockIdx.x, gridDim.x, total);
+  if ((int)blockIdx.x < first_wg) {
+    const int job = blockIdx.x;
+    if (job < segs.wgs) segments_body(segs, job);
+    else if (job < segs.wgs + heads.wgs) head_sums_body(heads, job - segs.wgs);
+    return;
+  }
+  const int logical = xcd_remap((int)blockIdx.x - first_wg, (int)gridDim.x - first_wg, total);
   if (logical < 0) return;
   const int bh = logical / Mblk;
   const int mb = logical - bh * Mblk;
@@ -573,6 +611,15 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
   for (int i = 0; i < (4 * TILE / 16 + 63) / 64; ++i)
     if (i * 64 + lane < 4 * TILE / 16) reinterpret_cast<i32x4_t*>(smem)[i * 64 + lane] = i32x4_t{0, 0, 0, 0};
   wave_lds_fence();
+
+  // what dq holds, asked for before the last unit's arithmetic
+  TileRows<D> old[2];
+  const auto fetch_old = [&]() __attribute__((always_inline)) {
+    if (!add) return;
+#pragma unroll
+    for (int qt = 0; qt < 2; ++qt)
+      old[qt].fetch(dq + head_off + (size_t)(qrow0 + 32 * qt) * pitch, L - qrow0 - 32 * qt, lane, pitch);
+  };
 
   f32x16_t dqacc[DT][2];
 #pragma unroll
@@ -829,6 +876,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
       E2 = E3;
     }
     // the last unit: no scores left to form beside its arithmetic
+    fetch_old();
     if (__builtin_expect(L - (E0 + 32) < 32, 0)) mask_tail(tb, L - (E0 + 32));
 #pragma unroll
     for (int e = 0; e <= 32; ++e) element(tb, e);
@@ -838,6 +886,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
       dqacc[dt][qt] = E::mfma32(trk[c2][dt], __builtin_bit_cast(i16x8_t, dsw[qt][c2]), dqacc[dt][qt]);
     }
   }
+  if (topk <= 0) fetch_old();
 #undef SLA_DQ_REQUEST
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // (nothing of this workgroup is in flight when it ends)
 
@@ -859,6 +908,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
     wave_lds_fence();
     TileRows<D> t;
     t.unpark(stage, lane);
+    if (add) t.template add<E>(old[qt]);
     t.store_streaming(dq + head_off + (size_t)(qrow0 + 32 * qt) * pitch, L - qrow0 - 32 * qt, lane, pitch);
     wave_lds_fence();
   }

@@ -19,8 +19,8 @@ FEATURE_MAPS = ("elu", "relu", "softmax")
 def module_bwd(q, k, v, o_s, d_out, lse, sparse_map, lut, topk, BLKQ, BLKK, qk_scale, weight, bias, fmap, states=None,
                grads=None, side_stream=None):
     """Backward of the whole operator in one library call (``sla_module_bwd``): the kernels of
-    :func:`sparse_attn_bwd` and of :func:`linear_bwd` accumulating into the same gradients, bit for bit, with the
-    short kernels on ``side_stream`` beside the long ones when one is given.  Returns ``(dq, dk, dv, d_weight, d_bias)``.
+    :func:`sparse_attn_bwd` and of :func:`linear_bwd` accumulating into the same gradients, bit for bit, the short kernels
+    in the launches of longer ones (``side_stream`` is accepted and not used).  Returns ``(dq, dk, dv, d_weight, d_bias)``.
     For callers that hold the forward's parts in tensors of their own; the operators below keep them in one allocation and
     take :func:`_module_bwd_saved`.
 
@@ -145,7 +145,7 @@ def _module_bwd_saved(saved, off, q_ptr, k_ptr, v_ptr, s_qkv, d_out, s_do, weigh
         q_ptr, k_ptr, v_ptr, s_qkv, base + off["o_s"], d_out.data_ptr(), s_do, base + off["lse"], base + off["map"],
         base + off["lut"], 4, weight.data_ptr(), bias.data_ptr(), base + off["states"], *grads, dw.data_ptr(),
         db.data_ptr(), dt, _lib.FMAP[fmap], B, H, L, D, BLKQ, BLKK, T, D ** -0.5, w0, n_s, w0 + n_s, n_l,
-        _lib.stream_ptr(dev), _side_stream(dev))
+        _lib.stream_ptr(dev), None)
     _lib.check(rc)
     return dw, db
 

@@ -1,0 +1,62 @@
+"""Work items of the dK/dV kernel: counts of (head, key block) pairs around the 512 one wave numbers, and key blocks that every
+query block selects, whose lists are cut into segments that the last workgroup to finish adds up; alone and added to what the
+gradients hold."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def dev():
+    return torch.device("cuda:0")
+
+
+@pytest.mark.parametrize("H,N,T", [(511, 1, 1), (512, 1, 1), (171, 3, 2), (342, 3, 2), (8, 130, 3), (3, 171, 4)])
+def test_gradients_over_all_pairs(dev, H, N, T):
+    from sla_amd.sparse_attn import sparse_attn_bwd, sparse_attn_fwd
+    D, L = 64, 64 * N - 5
+    g = torch.Generator(device=dev).manual_seed(H)
+    q, k, v, do = (torch.randn(1, H, L, D, device=dev, generator=g).bfloat16() for _ in range(4))
+    # every row selects key block 0 (a list of N entries, several segments from 65 on) and T - 1 blocks after it
+    i = torch.arange(N, device=dev)[:, None]
+    lut = torch.cat([torch.zeros(N, 1, dtype=torch.long, device=dev), 1 + (i + torch.arange(T - 1, device=dev)) % max(N - 1, 1)], 1)
+    lut = lut.sort(1).values.expand(1, H, N, T).contiguous()
+    smap = torch.zeros(1, H, N, N, dtype=torch.int8, device=dev).scatter_(3, lut, 1)
+    lut = lut.int()
+    scale = D ** -0.5
+    o, lse = sparse_attn_fwd(q, k, v, lut, T, 64, 64, scale)
+    got = sparse_attn_bwd(q, k, v, o, do, lse, smap, lut, T, 64, 64, scale)
+    mask = smap[0, 0].bool().repeat_interleave(64, 0).repeat_interleave(64, 1)[:L, :L]
+    for h0 in range(0, H, 64 if N < 8 else 1):
+        hs = slice(h0, h0 + (64 if N < 8 else 1))
+        qf, kf, vf = (t[0, hs].float().requires_grad_(True) for t in (q, k, v))
+        s = (torch.bmm(qf, kf.transpose(1, 2).contiguous()) * scale).masked_fill(~mask, float("-inf"))
+        ref = torch.autograd.grad(torch.bmm(torch.softmax(s, -1), vf), (qf, kf, vf), do[0, hs].float())
+        for name, a, r in zip("qkv", got, ref):
+            # (probabilities, dS and the result are rounded to bf16, u = 2^-9 each: within 4 u of the largest 2-norm of a head)
+            err = (a[0, hs].float() - r).flatten(1).norm(dim=1)
+            assert bool((err <= 4 * 2.0 ** -9 * r.flatten(1).norm(dim=1).clamp_min(1e-3) + 1e-3).all()), (name, h0, err.max().item())
+
+
+@pytest.mark.parametrize("H,L", [(2, 8320), (1, 4161)])
+def test_added_to_what_the_gradients_hold(dev, H, L):
+    """A whole backward over lists in segments equals the attention's gradients plus the linear branch's, bit for bit."""
+    from sla_amd.inputs import make_proj
+    from sla_amd.linear import linear_bwd
+    from sla_amd.module import module_bwd
+    from sla_amd.sparse_attn import sparse_attn_bwd, sparse_attn_fwd
+    D, T, N = 128, 2, -(-L // 64)
+    g = torch.Generator(device=dev).manual_seed(L)
+    q, k, v, do = (torch.randn(1, H, L, D, device=dev, generator=g).bfloat16() for _ in range(4))
+    w, b = (t.to(dev) for t in make_proj(D))
+    lut = torch.stack([torch.zeros(N, dtype=torch.long), 1 + torch.arange(N) % (N - 1)], 1).to(dev).expand(1, H, N, T).contiguous()
+    smap = torch.zeros(1, H, N, N, dtype=torch.int8, device=dev).scatter_(3, lut, 1)
+    lut = lut.int()
+    o, lse = sparse_attn_fwd(q, k, v, lut, T, 64, 64, D ** -0.5)
+    grads = sparse_attn_bwd(q, k, v, o, do, lse, smap, lut, T, 64, 64, D ** -0.5)
+    ref = linear_bwd(q, k, v, w, b, do, "elu", accumulate_into=grads)
+    for _ in range(2):
+        got = module_bwd(q, k, v, o, do, lse, smap, lut, T, 64, 64, D ** -0.5, w, b, "elu")
+        for a, r in zip(got, ref):
+            assert torch.equal(a, r)
