@@ -12,6 +12,7 @@
 //   score      : acc = acc + (a_d * b_d), d ascending, no fused multiply-add.
 // Selection is by (score descending, index ascending); -0.0 == +0.0.
 #include "block_map.h"
+#include "block_pool.h"
 #include "fwd_steps.h"
 
 #include <mutex>
@@ -20,138 +21,20 @@
 
 namespace sla {
 
-constexpr int KMEAN_CHUNK = 64;   // rows per level-1 sum
-constexpr int KMEAN_GROUP = 32;   // level-1 sums per level-2 sum
-
-// KEY_LOW_BIT: lowest bit of the fp32 image of a value of this type that can be non-zero.
-struct IoF32 {
-  typedef float raw;
-  static constexpr int VEC = 4;
-  static constexpr int KEY_LOW_BIT = 0;
-  static __device__ __forceinline__ float ld(raw x) { return x; }
-  static __device__ __forceinline__ raw st(float x) { return x; }
-};
-struct IoBf16 {
-  typedef uint16_t raw;
-  static constexpr int VEC = 8;
-  static constexpr int KEY_LOW_BIT = 16;
-  static __device__ __forceinline__ float ld(raw x) { return Elem<bf16_tag>::to_float(x); }
-  static __device__ __forceinline__ raw st(float x) { return Elem<bf16_tag>::from_float(x); }
-};
-struct IoF16 {
-  typedef uint16_t raw;
-  static constexpr int VEC = 8;
-  static constexpr int KEY_LOW_BIT = 13;
-  static __device__ __forceinline__ float ld(raw x) { return Elem<f16_tag>::to_float(x); }
-  static __device__ __forceinline__ raw st(float x) { return Elem<f16_tag>::from_float(x); }
-};
-
-template <typename IO>
-struct alignas(16) Vec16 {
-  typename IO::raw e[IO::VEC];
-};
-
-// MODE 0: fp32 block sums (no division)        -> out_f32 (BH, nblk, D)
-// MODE 1: block mean in the input dtype        -> out     (BH, nblk, D)
-// MODE 2: block mean of round(x - colmean)     -> out     (BH, nblk, D)
-// One thread owns VEC adjacent columns of one block and walks its rows in order.
-// tiled: the means go out in operand order (16-bit dtypes; tiled_pos) instead of as rows.
-template <typename IO, int MODE>
-static __device__ __forceinline__ void pool_body(const typename IO::raw* __restrict__ x, const RowLayout lay,
-                                                 const typename IO::raw* __restrict__ colmean, void* __restrict__ out, int L,
-                                                 int D, int BLK, int nblk, int tiled, int bx, int bh) {
-  constexpr int VEC = IO::VEC;
-  const int tpr = D / VEC;
-  const int bpw = 256 / tpr;
-  const int sub = threadIdx.x / tpr;
-  const int blk = bx * bpw + sub;
-  const int c = (threadIdx.x - sub * tpr) * VEC;
-  if (sub >= bpw || blk >= nblk) return;
-  const int row0 = blk * BLK;
-  const int nrows = min(BLK, L - row0);
-  float acc[VEC];
-  float cm[VEC];
-#pragma unroll
-  for (int e = 0; e < VEC; ++e) acc[e] = 0.f;
-  if (MODE == 2) {
-    Vec16<IO> m = *reinterpret_cast<const Vec16<IO>*>(colmean + (size_t)bh * D + c);
-#pragma unroll
-    for (int e = 0; e < VEC; ++e) cm[e] = IO::ld(m.e[e]);
-  }
-  const size_t pitch = (size_t)lay.sl;
-  const typename IO::raw* p = x + lay.head(bh) + (size_t)row0 * pitch + c;
-  // rows are fetched sixteen at a time (all loads of a batch in flight together), then added in row order
-  constexpr int BATCH = 16;
-  int r = 0;
-  for (; r + BATCH <= nrows; r += BATCH) {
-    Vec16<IO> v[BATCH];
-#pragma unroll
-    for (int i = 0; i < BATCH; ++i) v[i] = *reinterpret_cast<const Vec16<IO>*>(p + (size_t)(r + i) * pitch);
-#pragma unroll
-    for (int i = 0; i < BATCH; ++i)
-#pragma unroll
-      for (int e = 0; e < VEC; ++e) {
-        float f = IO::ld(v[i].e[e]);
-        if (MODE == 2) f = IO::ld(IO::st(f - cm[e]));
-        acc[e] = acc[e] + f;
-      }
-  }
-  for (; r < nrows; ++r) {
-    Vec16<IO> v = *reinterpret_cast<const Vec16<IO>*>(p + (size_t)r * pitch);
-#pragma unroll
-    for (int e = 0; e < VEC; ++e) {
-      float f = IO::ld(v.e[e]);
-      if (MODE == 2) f = IO::ld(IO::st(f - cm[e]));
-      acc[e] = acc[e] + f;
-    }
-  }
-  const size_t o = ((size_t)bh * nblk + blk) * D + c;
-  if (MODE == 0) {
-    float* of = reinterpret_cast<float*>(out) + o;
-#pragma unroll
-    for (int e = 0; e < VEC; ++e) of[e] = acc[e];
-  } else {
-    const float cnt = (float)nrows;
-    Vec16<IO> r;
-#pragma unroll
-    for (int e = 0; e < VEC; ++e) r.e[e] = IO::st(acc[e] / cnt);
-    if constexpr (VEC == 8) {
-      if (tiled) {             // four even and four odd columns, adjacent in their places
-        uint16_t* t = reinterpret_cast<uint16_t*>(out) + tiled_head(bh, nblk, D);
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          i16x4_t w;
-#pragma unroll
-          for (int j = 0; j < 4; ++j) w[j] = (short)r.e[2 * j + h];
-          *reinterpret_cast<i16x4_t*>(t + tiled_pos(blk, c + h, D)) = w;
-        }
-        return;
-      }
-    }
-    *reinterpret_cast<Vec16<IO>*>(reinterpret_cast<typename IO::raw*>(out) + o) = r;
-  }
-}
-
 template <typename IO, int MODE>
 __global__ __launch_bounds__(256) void pool_kernel(const typename IO::raw* __restrict__ x, const RowLayout lay,
                                                    const typename IO::raw* __restrict__ colmean,
                                                    void* __restrict__ out, int L, int D, int BLK, int nblk, int tiled) {
-  pool_body<IO, MODE>(x, lay, colmean, out, L, D, BLK, nblk, tiled, blockIdx.x, blockIdx.y);
+  pool_body<IO, MODE, IO::VEC, 256>(x, lay, colmean, out, L, D, BLK, nblk, tiled, blockIdx.x, blockIdx.y);
 }
 
-// The two independent first passes of the mask builder in one launch (neither fills the memory system alone):
-// blockIdx.z == 0: block means of q (MODE 1); z == 1: fp32 chunk sums of k (MODE 0, chunks of KMEAN_CHUNK rows).  K comes
-// second because the next pass reads it again: what of it is still in the memory-side cache then is the part read last
-// (module forward at B1 H12 L32760: 0.493 against 0.498 ms with k first).
+// The two independent first passes of the mask builder in one launch (neither fills the memory system alone).
 template <typename IO>
 __global__ __launch_bounds__(256) void pool_pair_kernel(const typename IO::raw* __restrict__ k, float* __restrict__ chunk_sums,
                                                         int nchunk, const typename IO::raw* __restrict__ q,
                                                         const RowLayout lay, typename IO::raw* __restrict__ pq, int BLKQ,
                                                         int nblkq, int L, int D, int tiled) {
-  if (blockIdx.z == 1)
-    pool_body<IO, 0>(k, lay, nullptr, chunk_sums, L, D, KMEAN_CHUNK, nchunk, 0, blockIdx.x, blockIdx.y);
-  else
-    pool_body<IO, 1>(q, lay, nullptr, pq, L, D, BLKQ, nblkq, tiled, blockIdx.x, blockIdx.y);
+  pool_pair_body<IO, IO::VEC>(k, chunk_sums, nchunk, q, lay, pq, BLKQ, nblkq, L, D, tiled, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 
 // Column mean of K, levels 2 and 3 of the fixed summation order:
@@ -184,40 +67,13 @@ __global__ __launch_bounds__(128) void colmean_kernel(const float* __restrict__ 
   colmean[(size_t)bh * D + d] = IO::st(acc / (float)L);
 }
 
-// Levels 2 and 3 in one launch when the group sums of a column slab fit in LDS: one workgroup per (head, slab of
-// COLMEAN_SLAB columns), thread (gi, c) = (tid / COLMEAN_SLAB, tid % COLMEAN_SLAB) forms group sums gi, gi + 16, ...
-// of its column; the first COLMEAN_SLAB threads then add the groups in ascending order.  (Small workgroups: the
-// launch has to find room beside the memory-bound kernels that run on other streams at the same time.)
-constexpr int COLMEAN_SLAB = 16;
-constexpr int COLMEAN_MAX_GROUPS = 256;
+// Levels 2 and 3 in one launch when the group sums of a column slab fit in LDS.
 template <typename IO>
 __global__ __launch_bounds__(256) void colmean_fused_kernel(const float* __restrict__ chunk_sums,
                                                             typename IO::raw* __restrict__ colmean, int nchunk, int ngroup,
                                                             int D, int L) {
   __shared__ float gs[COLMEAN_MAX_GROUPS * COLMEAN_SLAB];
-  const int bh = blockIdx.y, tid = threadIdx.x;
-  const int c = tid % COLMEAN_SLAB, d = blockIdx.x * COLMEAN_SLAB + c;
-  for (int g = tid / COLMEAN_SLAB; g < ngroup; g += 256 / COLMEAN_SLAB) {
-    const int c0 = g * KMEAN_GROUP;
-    const int n = min(KMEAN_GROUP, nchunk - c0);
-    // (a group's loads all in flight, then added in order: mask builder of 16 heads x 6001 x 64 25.3 -> 23.2 us, of 40 x 75600 x 128 656 -> 652)
-    const float* p = chunk_sums + ((size_t)bh * nchunk + c0) * D + d;
-    float x[KMEAN_GROUP];
-#pragma unroll
-    for (int i = 0; i < KMEAN_GROUP; ++i) x[i] = p[(size_t)min(i, n - 1) * D];
-    __builtin_amdgcn_sched_barrier(0);
-    float acc = 0.f;
-#pragma unroll
-    for (int i = 0; i < KMEAN_GROUP; ++i)
-      if (i < n) acc = acc + x[i];
-    gs[g * COLMEAN_SLAB + c] = acc;
-  }
-  __syncthreads();
-  if (tid < COLMEAN_SLAB) {
-    float acc = 0.f;
-    for (int g = 0; g < ngroup; ++g) acc = acc + gs[g * COLMEAN_SLAB + tid];
-    colmean[(size_t)bh * D + d] = IO::st(acc / (float)L);
-  }
+  colmean_body<IO>(chunk_sums, colmean, nchunk, ngroup, D, L, blockIdx.x, blockIdx.y, gs);
 }
 
 // score[bh][m][n] = round_dtype( sum_d pq[m][d]*pk[n][d] ), d ascending, every product and every sum rounded to fp32.
@@ -883,6 +739,15 @@ static int64_t block_map_least_bytes(int dtype, int BH, int L, int D, int BLKQ, 
   return (int64_t)map_ws(dtype, BH, L, D, BLKQ, BLKK, false).total;
 }
 
+MapParts block_map_parts(int dtype, int BH, int L, int D, int BLKQ, int BLKK, void* workspace, int64_t workspace_bytes) {
+  // (rows cost the score kernels twice the loads: only where the tiles do not fit)
+  const bool tiled = score_takes_tiled(dtype, D) && workspace_bytes >= block_map_workspace_bytes(dtype, BH, L, D, BLKQ, BLKK);
+  const MapWs w = map_ws(dtype, BH, L, D, BLKQ, BLKK, tiled);
+  char* const ws = (char*)workspace;
+  return MapParts{(float*)(ws + w.chunk_sums), (float*)(ws + w.group_sums), ws + w.colmean, ws + w.pq, ws + w.pk, ws + w.score,
+                  tiled, cdiv(L, BLKQ), cdiv(L, BLKK), cdiv(L, KMEAN_CHUNK)};
+}
+
 static int validate_pool(int dtype, int BH, int L, int D, int BLK) {
   SLA_REQUIRE(dtype == SLA_F32 || dtype == SLA_BF16 || dtype == SLA_F16, SLA_ERR_BAD_ARG, "unknown dtype %d", dtype);
   SLA_REQUIRE(BH > 0 && L > 0 && D > 0 && BLK > 0, SLA_ERR_BAD_ARG, "non-positive size (BH=%d L=%d D=%d BLK=%d)", BH, L,
@@ -925,30 +790,31 @@ static void launch_k_colmean_t(const void* k, const RowLayout& lay, int BH, int 
   launch_colmean_reduce<IO>(chunk_sums, group_sums, colmean, BH, L, D, st);
 }
 
+// scores and selection from the block means in `m` (topk == 0 selects nothing: the map rows are cleared)
+void block_map_select(int dtype, const MapParts& m, int BH, int D, int topk, int8_t* sparse_map, void* lut, int lut64,
+                      hipStream_t st) {
+  if (dtype == SLA_F32)
+    launch_select<IoF32>((const float*)m.pq, (const float*)m.pk, m.tiled, (float*)m.score, sparse_map, lut, lut64, BH, m.M, m.N, D, topk, st);
+  else if (dtype == SLA_BF16)
+    launch_select<IoBf16>((const uint16_t*)m.pq, (const uint16_t*)m.pk, m.tiled, (uint16_t*)m.score, sparse_map, lut, lut64, BH, m.M, m.N, D, topk, st);
+  else
+    launch_select<IoF16>((const uint16_t*)m.pq, (const uint16_t*)m.pk, m.tiled, (uint16_t*)m.score, sparse_map, lut, lut64, BH, m.M, m.N, D, topk, st);
+}
+
+// first_pass = false: the chunk sums of k and the block means of q are there already
 template <typename IO>
-static int block_map_impl(const void* q, const void* k, const RowLayout& lay, int dtype, int BH, int L, int D, int BLKQ,
-                          int BLKK, int topk, char* ws, bool tiled, int8_t* sparse_map, void* lut, int lut64,
-                          hipStream_t st) {
-  const MapWs w = map_ws(dtype, BH, L, D, BLKQ, BLKK, tiled);
-  const int M = cdiv(L, BLKQ), N = cdiv(L, BLKK);
-  float* chunk_sums = (float*)(ws + w.chunk_sums);
-  typename IO::raw* colmean = (typename IO::raw*)(ws + w.colmean);
-  typename IO::raw* pq = (typename IO::raw*)(ws + w.pq);
-  typename IO::raw* pk = (typename IO::raw*)(ws + w.pk);
-  typename IO::raw* score = (typename IO::raw*)(ws + w.score);
-  {
+static void block_map_pool(const void* q, const void* k, const RowLayout& lay, const MapParts& m, int BH, int L, int D, int BLKQ,
+                           int BLKK, bool first_pass, hipStream_t st) {
+  typename IO::raw* colmean = (typename IO::raw*)m.colmean;
+  if (first_pass) {
     // k chunk sums and q block means share one launch
-    const int nchunk = cdiv(L, KMEAN_CHUNK);
     const int bpw = 256 / (D / IO::VEC);
-    dim3 grid(cdiv(max(nchunk, M), bpw), BH, 2);
-    hipLaunchKernelGGL((pool_pair_kernel<IO>), grid, dim3(256), 0, st, (const typename IO::raw*)k, chunk_sums, nchunk,
-                       (const typename IO::raw*)q, lay, pq, BLKQ, M, L, D, tiled);
+    hipLaunchKernelGGL((pool_pair_kernel<IO>), dim3(cdiv(max(m.nchunk, m.M), bpw), BH, 2), dim3(256), 0, st,
+                       (const typename IO::raw*)k, m.chunk_sums, m.nchunk, (const typename IO::raw*)q, lay,
+                       (typename IO::raw*)m.pq, BLKQ, m.M, L, D, m.tiled);
   }
-  launch_colmean_reduce<IO>(chunk_sums, (float*)(ws + w.group_sums), colmean, BH, L, D, st);
-  launch_pool<IO, 2>(k, lay, colmean, pk, BH, L, D, BLKK, st, tiled);
-  // (topk == 0 selects nothing: the map rows are cleared)
-  launch_select<IO>(pq, pk, tiled, score, sparse_map, lut, lut64, BH, M, N, D, topk, st);
-  return check_launch("block map");
+  launch_colmean_reduce<IO>(m.chunk_sums, m.group_sums, colmean, BH, L, D, st);
+  launch_pool<IO, 2>(k, lay, colmean, m.pk, BH, L, D, BLKK, st, m.tiled);
 }
 
 // Column mean of k over L in the fixed order, rounded to `dtype`.  scratch: fp32, at least
@@ -1014,6 +880,15 @@ int block_map_check(const void* q, const void* k, const int64_t* strides, int dt
   return make_layout(strides, B, H, L, D, dtype == SLA_F32 ? 4 : 2, lay);
 }
 
+int block_map_run(const void* q, const void* k, const RowLayout& lay, int dtype, const MapParts& m, int BH, int L, int D, int BLKQ,
+                  int BLKK, int topk, int8_t* sparse_map, void* lut, int lut64, bool first_pass, hipStream_t st) {
+  if (dtype == SLA_F32) block_map_pool<IoF32>(q, k, lay, m, BH, L, D, BLKQ, BLKK, first_pass, st);
+  else if (dtype == SLA_BF16) block_map_pool<IoBf16>(q, k, lay, m, BH, L, D, BLKQ, BLKK, first_pass, st);
+  else block_map_pool<IoF16>(q, k, lay, m, BH, L, D, BLKQ, BLKK, first_pass, st);
+  block_map_select(dtype, m, BH, D, topk, sparse_map, lut, lut64, st);
+  return check_launch("block map");
+}
+
 int block_map_entry(const void* q, const void* k, const int64_t* strides, int dtype, int B, int H, int L, int D, int BLKQ,
                     int BLKK, int topk, void* workspace, int64_t workspace_bytes, int8_t* sparse_map, bool want_map, void* lut,
                     int lut_elem_bytes, void* stream) {
@@ -1021,17 +896,9 @@ int block_map_entry(const void* q, const void* k, const int64_t* strides, int dt
   const int rc = block_map_check(q, k, strides, dtype, B, H, L, D, BLKQ, BLKK, topk, workspace, workspace_bytes, sparse_map,
                                  want_map, lut, lut_elem_bytes, &lay);
   if (rc) return rc;
-  const int BH = B * H;
-  // (rows cost the score kernels twice the loads: only where the tiles do not fit)
-  const bool tiled = score_takes_tiled(dtype, D) && workspace_bytes >= block_map_workspace_bytes(dtype, BH, L, D, BLKQ, BLKK);
-  hipStream_t st = (hipStream_t)stream;
-  char* ws = (char*)workspace;
-  const int lut64 = lut_elem_bytes == 8;
-  if (dtype == SLA_F32)
-    return block_map_impl<IoF32>(q, k, lay, dtype, BH, L, D, BLKQ, BLKK, topk, ws, tiled, sparse_map, lut, lut64, st);
-  if (dtype == SLA_BF16)
-    return block_map_impl<IoBf16>(q, k, lay, dtype, BH, L, D, BLKQ, BLKK, topk, ws, tiled, sparse_map, lut, lut64, st);
-  return block_map_impl<IoF16>(q, k, lay, dtype, BH, L, D, BLKQ, BLKK, topk, ws, tiled, sparse_map, lut, lut64, st);
+  const MapParts m = block_map_parts(dtype, B * H, L, D, BLKQ, BLKK, workspace, workspace_bytes);
+  return block_map_run(q, k, lay, dtype, m, B * H, L, D, BLKQ, BLKK, topk, sparse_map, lut, lut_elem_bytes == 8, true,
+                       (hipStream_t)stream);
 }
 
 }  // namespace sla

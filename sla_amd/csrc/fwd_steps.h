@@ -10,6 +10,17 @@ int64_t block_map_workspace_bytes(int dtype, int BH, int L, int D, int BLKQ, int
 int block_map_check(const void* q, const void* k, const int64_t* strides, int dtype, int B, int H, int L, int D, int BLKQ,
                     int BLKK, int topk, const void* workspace, int64_t workspace_bytes, const int8_t* sparse_map, bool want_map,
                     const void* lut, int lut_elem_bytes, RowLayout* lay);
+// Where the parts of its workspace lie: chunk sums and column mean of k, block means of q and k (tiled: in operand order), scores.
+struct MapParts {
+  float *chunk_sums, *group_sums;
+  void *colmean, *pq, *pk, *score;
+  int tiled, M, N, nchunk;
+};
+MapParts block_map_parts(int dtype, int BH, int L, int D, int BLKQ, int BLKK, void* workspace, int64_t workspace_bytes);
+void block_map_select(int dtype, const MapParts& m, int BH, int D, int topk, int8_t* sparse_map, void* lut, int lut64,
+                      hipStream_t st);
+int block_map_run(const void* q, const void* k, const RowLayout& lay, int dtype, const MapParts& m, int BH, int L, int D, int BLKQ,
+                  int BLKK, int topk, int8_t* sparse_map, void* lut, int lut64, bool first_pass, hipStream_t st);
 int block_map_entry(const void* q, const void* k, const int64_t* strides, int dtype, int B, int H, int L, int D, int BLKQ,
                     int BLKK, int topk, void* workspace, int64_t workspace_bytes, int8_t* sparse_map, bool want_map, void* lut,
                     int lut_elem_bytes, void* stream);

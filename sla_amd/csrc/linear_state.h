@@ -11,13 +11,16 @@ namespace sla {
 // instead of sum_rows phi(k) (used by the complement backward, where "k" is q and "v" a row gradient).
 // VMAX: the largest |v| of every column over the slice goes to vmax_part[bh][split][D] (what the FP8 quantiser of v
 // needs of v before it can start: v is streamed here anyway).
-template <typename Tag, int D, bool OUT16 = false, bool ZW = false, bool VMAX = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void linear_state_partial_kernel(const uint16_t* __restrict__ k,
-                                                                   const uint16_t* __restrict__ v, const RowLayout lay,
-                                                                   void* __restrict__ kv_part_, float* __restrict__ z_part,
-                                                                   int L, int rows_per_split, int fmap,
-                                                                   const float* __restrict__ zweight = nullptr,
-                                                                   float* __restrict__ vmax_part = nullptr) {
+template <int D>
+constexpr int state_partial_lds() { return 2 * 64 * (D + 16) * 2 + 2048 * 4; }       // bytes
+// DEPTH: tiles in flight in registers beside the one in LDS.  Two where a launch does not fill the chip and a slice is a chain of
+// tile latencies; one where memory is the bound and the registers buy a third workgroup per compute unit.
+template <typename Tag, int D, bool OUT16, bool ZW, bool VMAX, int DEPTH>
+static __device__ __forceinline__ void state_partial_body(const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
+                                                          const RowLayout lay, void* __restrict__ kv_part_,
+                                                          float* __restrict__ z_part, int L, int rows_per_split, int fmap,
+                                                          const float* __restrict__ zweight, float* __restrict__ vmax_part,
+                                                          int split, int bh, int nsplit, char* smem) {
   using E = Elem<Tag>;
   constexpr int TR = 64;                 // rows per LDS tile
   constexpr int STR = D + 16;            // LDS row stride: transposed reads of 4 rows hit disjoint banks
@@ -28,11 +31,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
   constexpr int WPT = (DT * DT) / 4;     // output tiles per wave (4 waves)
   static_assert(DT * DT % 4 == 0, "state tiles must divide among 4 waves");
 
-  __shared__ __attribute__((aligned(16))) uint16_t sK[TR * STR];
-  __shared__ __attribute__((aligned(16))) uint16_t sV[TR * STR];
-  __shared__ float sZ[RPP][D];
+  uint16_t* const sK = reinterpret_cast<uint16_t*>(smem);
+  uint16_t* const sV = sK + TR * STR;
+  float (*sZ)[D] = reinterpret_cast<float (*)[D]>(smem + 2 * TR * STR * 2);
+  static_assert(RPP * D == 2048, "a pass of the workgroup is 2048 columns");
 
-  const int split = blockIdx.x, bh = blockIdx.y, nsplit = gridDim.x;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int g = lane >> 5;
   const int row_begin = split * rows_per_split;
@@ -62,31 +65,33 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
   const int tr_row = (lane & 15) >> 2;
   const int tr_col = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
 
-  // rows of the next tile are fetched into registers while the current tile is multiplied
-  i16x8_t kreg[NP], vreg[NP];
-  float wreg[NP];
-  auto fetch = [&](int r0) {
+  // rows of the next tiles are fetched into registers while the current tile is multiplied
+  i16x8_t kreg[DEPTH][NP], vreg[DEPTH][NP];
+  float wreg[DEPTH][NP];
+  auto fetch = [&](int r0, int s) __attribute__((always_inline)) {
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
       const int grow = r0 + lrow + p * RPP;
-      kreg[p] = i16x8_t{0, 0, 0, 0, 0, 0, 0, 0};
-      vreg[p] = i16x8_t{0, 0, 0, 0, 0, 0, 0, 0};
-      wreg[p] = 1.0f;
+      kreg[s][p] = i16x8_t{0, 0, 0, 0, 0, 0, 0, 0};
+      vreg[s][p] = i16x8_t{0, 0, 0, 0, 0, 0, 0, 0};
+      wreg[s][p] = 1.0f;
       if (grow < row_end) {
-        kreg[p] = *reinterpret_cast<const i16x8_t*>(kh + (size_t)grow * pitch + lcol);
-        vreg[p] = *reinterpret_cast<const i16x8_t*>(vh + (size_t)grow * pitch + lcol);
-        if (ZW) wreg[p] = zweight[(size_t)bh * L + grow];
+        kreg[s][p] = *reinterpret_cast<const i16x8_t*>(kh + (size_t)grow * pitch + lcol);
+        vreg[s][p] = *reinterpret_cast<const i16x8_t*>(vh + (size_t)grow * pitch + lcol);
+        if (ZW) wreg[s][p] = zweight[(size_t)bh * L + grow];
       }
     }
   };
-  if (row_begin < row_end) fetch(row_begin);
-  for (int r0 = row_begin; r0 < row_end; r0 += TR) {
-    __syncthreads();
+  if (row_begin < row_end)
+#pragma unroll
+    for (int s = 0; s < DEPTH; ++s) fetch(row_begin + s * TR, s);
+  const auto tile = [&](int r0, int s) __attribute__((always_inline)) {
+    lds_barrier();
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
       const int row = lrow + p * RPP;
       const int grow = r0 + row;
-      const i16x8_t kk = kreg[p], vv = vreg[p];
+      const i16x8_t kk = kreg[s][p], vv = vreg[s][p];
       const bool ok = grow < row_end;
       float f[8];
 #pragma unroll
@@ -120,7 +125,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         if (!ok) f[e] = 0.f;              // rows past the end take no part (phi(0) is not 0 for elu/softmax)
-        zacc[e] += ZW ? wreg[p] * f[e] : f[e];
+        zacc[e] += ZW ? wreg[s][p] * f[e] : f[e];
         fk[e] = (short)E::from_float(f[e]);
       }
       *reinterpret_cast<i16x8_t*>(&sK[row * STR + lcol]) = fk;
@@ -132,15 +137,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
           vmx[j] = __builtin_elementwise_max(vmx[j], __builtin_bit_cast(u16x2_t, vw[j] & 0x7fff7fff));
       }
     }
-    __syncthreads();
-    if (r0 + TR < row_end) fetch(r0 + TR);     // after the barrier: its fence would wait for these loads
+    lds_barrier();
+    if (r0 + DEPTH * TR < row_end) fetch(r0 + DEPTH * TR, s);
 #pragma unroll
     for (int c = 0; c < TR / 16; ++c) {
       const int l0 = 16 * c + 8 * g + tr_row;
 #pragma unroll
       for (int t = 0; t < WPT; ++t) {
-        const int tile = wave * WPT + t;
-        const int d1t = tile / DT, d2t = tile % DT;
+        const int d1t = (wave * WPT + t) / DT, d2t = (wave * WPT + t) % DT;
         const uint16_t* pa = &sK[l0 * STR + 32 * d1t + tr_col];
         const uint16_t* pb = &sV[l0 * STR + 32 * d2t + tr_col];
         const i16x8_t a = concat4(lds_read_tr16(pa), lds_read_tr16(pa + 4 * STR));
@@ -148,7 +152,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
         acc[t] = E::mfma32(a, b, acc[t]);
       }
     }
-  }
+  };
+  for (int r0 = row_begin; r0 < row_end; r0 += DEPTH * TR)
+#pragma unroll
+    for (int s = 0; s < DEPTH; ++s)
+      if (s == 0 || r0 + s * TR < row_end) tile(r0 + s * TR, s);
 
   // partial KV, stored transposed: kv_part[bh][split][d2][d1]
   const size_t part_off = ((size_t)bh * nsplit + split) * D * D;
@@ -197,6 +205,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
       vmax_part[((size_t)bh * nsplit + split) * D + tid] = a;
     }
   }
+}
+
+template <typename Tag, int D, bool OUT16 = false, bool ZW = false, bool VMAX = false>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void linear_state_partial_kernel(
+    const uint16_t* __restrict__ k, const uint16_t* __restrict__ v, const RowLayout lay, void* __restrict__ kv_part,
+    float* __restrict__ z_part, int L, int rows_per_split, int fmap, const float* __restrict__ zweight = nullptr,
+    float* __restrict__ vmax_part = nullptr) {
+  __shared__ __attribute__((aligned(16))) char smem[state_partial_lds<D>()];
+  state_partial_body<Tag, D, OUT16, ZW, VMAX, 1>(k, v, lay, kv_part, z_part, L, rows_per_split, fmap, zweight, vmax_part, blockIdx.x,
+                                              blockIdx.y, gridDim.x, smem);
 }
 
 // Position of column d2 inside a row whose columns are re-ordered to the accumulator slot order of the
@@ -305,22 +323,26 @@ __global__ __launch_bounds__(512) void linear_state_presum_kernel(float* __restr
 }
 
 // (nsum: the slices to add up, all nsplit of a head or the first one alone, which then holds the sums)
+struct StateFinish {
+  const float *kv_part, *z_part, *weight;
+  uint16_t *kvt, *kvw, *kvwt, *z;
+  int nsplit, nsum, total;                 // total = heads x D / 16 workgroups
+};
+template <int D>
+constexpr int state_finish_lds() { return D / 64 * 256 * 16 + 16 * (D + 4) * 4 + 16 * (D + 8) * 2; }       // bytes
 template <typename Tag, int D>
-__global__ __launch_bounds__(512) void linear_state_finish_kernel(const float* __restrict__ kv_part,
-                                                                  const float* __restrict__ z_part,
-                                                                  const float* __restrict__ weight, uint16_t* __restrict__ kvt,
-                                                                  uint16_t* __restrict__ kvw, uint16_t* __restrict__ kvwt,
-                                                                  uint16_t* __restrict__ z, int nsplit, int nsum, int total) {
+static __device__ __forceinline__ void state_finish_body(const StateFinish& job, int logical, char* smem) {
+  const float *kv_part = job.kv_part, *z_part = job.z_part, *weight = job.weight;
+  uint16_t *kvt = job.kvt, *kvw = job.kvw, *kvwt = job.kvwt, *z = job.z;
+  const int nsplit = job.nsplit, nsum = job.nsum;
   using E = Elem<Tag>;
   constexpr int DD = D * D;
   constexpr int STR = D + 8;               // row pitch of the strip in LDS
   constexpr int NR = D / 64;               // rows d2 per thread
-  __shared__ __attribute__((aligned(16))) float s_half[NR * 256 * 4];     // sums of the upper half of the slices
-  __shared__ __attribute__((aligned(16))) uint16_t s_kv[16 * STR];        // [d1][d2]
   constexpr int STR32 = D + 4;
-  __shared__ __attribute__((aligned(16))) float s_kv32[16 * STR32];       // the same before rounding
-  const int logical = xcd_remap(blockIdx.x, gridDim.x, total);
-  if (logical < 0) return;
+  float* const s_half = reinterpret_cast<float*>(smem);                   // sums of the upper half of the slices
+  float* const s_kv32 = s_half + NR * 256 * 4;                            // [d1][d2] before rounding
+  uint16_t* const s_kv = reinterpret_cast<uint16_t*>(s_kv32 + 16 * STR32); // [d1][d2]
   const int bh = logical / (D / 16), d1_0 = 16 * (logical % (D / 16));
   const int tid = threadIdx.x & 255, half = threadIdx.x >> 8, lane = tid & 63, wave = threadIdx.x >> 6;
   const int l = lane & 15, h = lane >> 4;
@@ -429,20 +451,34 @@ static inline LinWs lin_ws(int BH, int L, int D) {
 }
 
 
+template <typename Tag, int D>
+__global__ __launch_bounds__(512) void linear_state_finish_kernel(const StateFinish job) {
+  __shared__ __attribute__((aligned(16))) char smem[state_finish_lds<D>()];
+  const int logical = xcd_remap(blockIdx.x, gridDim.x, job.total);
+  if (logical >= 0) state_finish_body<Tag, D>(job, logical, smem);
+}
+
 constexpr int PRESUM_MIN_SLICES = 40;       // (measured at linear_state_presum_kernel)
 
-// (ws: where the states go; parts: where the slices' partial sums lie, the offsets of `w` past states_end)
+// What is left to do behind the partial states (and, with many slices, behind the launch that adds them up first).  ws: where
+// the states go; parts: where the slices' partial sums lie, the offsets of `w` past states_end.
+template <int D>
+static inline StateFinish state_finish_job(const float* weight, int BH, char* ws, char* parts, const LinWs& w) {
+  return StateFinish{(const float*)(parts + (w.kv_part - w.states_end)), (const float*)(parts + (w.z_part - w.states_end)), weight,
+                     (uint16_t*)(ws + w.kvt), (uint16_t*)(ws + w.kvw), (uint16_t*)(ws + w.kvwt), (uint16_t*)(ws + w.z), w.nsplit,
+                     w.nsplit >= PRESUM_MIN_SLICES ? 1 : w.nsplit, BH * (D / 16)};
+}
+template <int D>
+static inline void launch_state_presum(int BH, char* parts, const LinWs& w, hipStream_t st) {
+  if (w.nsplit >= PRESUM_MIN_SLICES)
+    hipLaunchKernelGGL((linear_state_presum_kernel<D>), dim3(D * D / 256 + 1, BH), dim3(512), 0, st,
+                       (float*)(parts + (w.kv_part - w.states_end)), (float*)(parts + (w.z_part - w.states_end)), w.nsplit);
+}
 template <typename Tag, int D>
 static inline void launch_state_finish(const float* weight, int BH, char* ws, char* parts, const LinWs& w, hipStream_t st) {
-  float* const kv_part = (float*)(parts + (w.kv_part - w.states_end));
-  float* const z_part = (float*)(parts + (w.z_part - w.states_end));
-  const bool presum = w.nsplit >= PRESUM_MIN_SLICES;
-  if (presum)
-    hipLaunchKernelGGL((linear_state_presum_kernel<D>), dim3(D * D / 256 + 1, BH), dim3(512), 0, st, kv_part, z_part, w.nsplit);
-  hipLaunchKernelGGL((linear_state_finish_kernel<Tag, D>), dim3(xcd_grid((int64_t)BH * (D / 16))), dim3(512), 0, st,
-                     (const float*)kv_part, (const float*)z_part, weight,
-                     (uint16_t*)(ws + w.kvt), (uint16_t*)(ws + w.kvw), (uint16_t*)(ws + w.kvwt), (uint16_t*)(ws + w.z),
-                     w.nsplit, presum ? 1 : w.nsplit, BH * (D / 16));
+  launch_state_presum<D>(BH, parts, w, st);
+  const StateFinish job = state_finish_job<D>(weight, BH, ws, parts, w);
+  hipLaunchKernelGGL((linear_state_finish_kernel<Tag, D>), dim3(xcd_grid(job.total)), dim3(512), 0, st, job);
 }
 
 // Streams K and V once and leaves the finished states.

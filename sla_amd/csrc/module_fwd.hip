@@ -1,28 +1,119 @@
 // Forward of the whole module (mask builder, linear branch's states, attention with the linear branch in its epilogue) as
 // one call.
 //
-// Stands in for SparseLinearAttention.forward of the reference (sparse_linear_attention/core.py:69-105).  On `stream`:
-//     [16-bit copies of fp32 inputs] | mask builder | attention
-// with the state build (k, v only) on the caller's second stream beside the mask builder where that pays.
+// Stands in for SparseLinearAttention.forward of the reference (sparse_linear_attention/core.py:69-105).  On `stream`, launches
+// that need nothing of each other in one:
+//     block means of q, chunk sums of k [fp32 inputs: and the 16-bit copies] | slices' partial states, column mean of k |
+//     states finished, block means of k | scores and selection | attention
+// (five launches; in eight of their own, and seven with 16-bit inputs, everything before the attention took 34 us for 2 heads x
+// 1024 x 64 in fp32, 57 for 8 x 4096 x 128: now 25 and 43.)
+// From 16 MiB per tensor on the state build (k, v only) runs on the caller's second stream beside the mask builder instead.
+#include "block_pool.h"
 #include "fwd_steps.h"
+#include "linear_state.h"
 #include "side_events.h"
 
 namespace sla {
 
-// 16-bit copies of three fp32 tensors of n elements each, one after the other in `dst` (n a multiple of 8).
-template <typename Tag>
-__global__ __launch_bounds__(256) void cast3_kernel(const float* __restrict__ a, const float* __restrict__ b,
-                                                    const float* __restrict__ c, uint16_t* __restrict__ dst, int64_t n) {
-  const float* src = blockIdx.y == 0 ? a : blockIdx.y == 1 ? b : c;
-  const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 8;
-  if (i >= n) return;
-  const f32x4_t x = *reinterpret_cast<const f32x4_t*>(src + i), y = *reinterpret_cast<const f32x4_t*>(src + i + 4);
-  i32x4_t w;
-  w[0] = (int)Elem<Tag>::pack2(x[0], x[1]);
-  w[1] = (int)Elem<Tag>::pack2(x[2], x[3]);
-  w[2] = (int)Elem<Tag>::pack2(y[0], y[1]);
-  w[3] = (int)Elem<Tag>::pack2(y[2], y[3]);
-  *reinterpret_cast<i32x4_t*>(dst + (int64_t)blockIdx.y * n + i) = w;
+// First pass over q and k (pool_pair_body); grid (., heads, 2).  Cast: fp32 inputs, whose 16-bit copies leave on the way (n
+// elements each, one after the other in `cast`); blockIdx.z == 2 copies v.
+template <typename IO, int W, typename Cast>
+__global__ __launch_bounds__(256) void prefix_pool_kernel(const typename IO::raw* __restrict__ q, const typename IO::raw* __restrict__ k,
+                                                          const typename IO::raw* __restrict__ v, const RowLayout lay,
+                                                          const MapParts m, int BLKQ, int L, int D, uint16_t* __restrict__ cast,
+                                                          int64_t n) {
+  if (!__is_same(Cast, NoCast) && blockIdx.z == 2) {
+    if constexpr (!__is_same(Cast, NoCast)) {
+      const int64_t stride = (int64_t)gridDim.x * gridDim.y * 256 * 8;
+      for (int64_t i = (((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * 256 + threadIdx.x) * 8; i < n; i += stride) {
+        const f32x4_t x = *reinterpret_cast<const f32x4_t*>(v + i), y = *reinterpret_cast<const f32x4_t*>(v + i + 4);
+        i32x4_t w;
+        w[0] = (int)Elem<Cast>::pack2(x[0], x[1]);
+        w[1] = (int)Elem<Cast>::pack2(x[2], x[3]);
+        w[2] = (int)Elem<Cast>::pack2(y[0], y[1]);
+        w[3] = (int)Elem<Cast>::pack2(y[2], y[3]);
+        *reinterpret_cast<i32x4_t*>(cast + 2 * n + i) = w;
+      }
+    }
+    return;
+  }
+  pool_pair_body<IO, W, Cast>(k, m.chunk_sums, m.nchunk, q, lay, (typename IO::raw*)m.pq, BLKQ, m.M, L, D, m.tiled, blockIdx.x,
+                              blockIdx.y, blockIdx.z, cast, n);
+}
+
+// The slices' partial states and, in the first `first_wg` workgroups, the column mean of k; one head's slices are adjacent.
+template <typename Tag, int D, typename IO>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void prefix_state_kernel(
+    const uint16_t* __restrict__ k, const uint16_t* __restrict__ v, const RowLayout lay, float* __restrict__ kv_part,
+    float* __restrict__ z_part, int L, int rows_per_split, int nsplit, int fmap, const MapParts m, int first_wg) {
+  constexpr int LDS = state_partial_lds<D>() > COLMEAN_MAX_GROUPS * COLMEAN_SLAB * 4 ? state_partial_lds<D>() : COLMEAN_MAX_GROUPS * COLMEAN_SLAB * 4;
+  __shared__ __attribute__((aligned(16))) char smem[LDS];
+  const int wg = blockIdx.x;
+  if (wg < first_wg) {
+    colmean_body<IO>(m.chunk_sums, (typename IO::raw*)m.colmean, m.nchunk, (m.nchunk + KMEAN_GROUP - 1) / KMEAN_GROUP, D, L,
+                     wg % (D / COLMEAN_SLAB), wg / (D / COLMEAN_SLAB), reinterpret_cast<float*>(smem));
+    return;
+  }
+  const int bh = (wg - first_wg) / nsplit;
+  state_partial_body<Tag, D, false, false, false, 2>(k, v, lay, kv_part, z_part, L, rows_per_split, fmap, nullptr, nullptr,
+                                                  wg - first_wg - bh * nsplit, bh, nsplit, smem);
+}
+
+// The states finished and, in the workgroups from `first_pool` on (`per_head` for each head), the block means of k.
+template <typename Tag, int D, typename IO, int W>
+__global__ __launch_bounds__(512) void prefix_finish_kernel(const StateFinish job, int first_pool, const typename IO::raw* __restrict__ k,
+                                                            const RowLayout lay, const MapParts m, int L, int per_head) {
+  __shared__ __attribute__((aligned(16))) char smem[state_finish_lds<D>()];
+  const int wg = blockIdx.x;
+  if (wg < first_pool) {
+    const int logical = xcd_remap(wg, first_pool, job.total);
+    if (logical >= 0) state_finish_body<Tag, D>(job, logical, smem);
+    return;
+  }
+  const int bh = (wg - first_pool) / per_head;
+  pool_body<IO, 2, W, 512>(k, lay, (const typename IO::raw*)m.colmean, m.pk, L, D, 64, m.N, m.tiled, wg - first_pool - bh * per_head, bh);
+}
+
+// One thread per 4 bytes of a block's columns while the first pass of the wide form would not put a wave on every SIMD.
+static inline bool narrow_pools(int in_dtype, const MapParts& m, int BH, int D) {
+  return (int64_t)BH * m.nchunk * D * elem_bytes(in_dtype) / 16 < 1024 * 64;
+}
+
+template <typename IO, typename Cast>
+static void launch_prefix_pool(const void* q, const void* k, const void* v, const RowLayout& lay, const MapParts& m, int in_dtype,
+                               int BLKQ, int BH, int L, int D, void* cast, hipStream_t st) {
+  typedef typename IO::raw raw;
+  const int64_t n = (int64_t)BH * L * D;
+  const int z = __is_same(Cast, NoCast) ? 2 : 3;
+#define SLA_POOL_CASE(W)                                                                                                      \
+  hipLaunchKernelGGL((prefix_pool_kernel<IO, W, Cast>), dim3(cdiv(max(m.nchunk, m.M), 256 / (D / (W))), BH, z), dim3(256), 0, st, \
+                     (const raw*)q, (const raw*)k, (const raw*)v, lay, m, BLKQ, L, D, (uint16_t*)cast, n)
+  if (narrow_pools(in_dtype, m, BH, D)) SLA_POOL_CASE(IO::VEC / 4);
+  else SLA_POOL_CASE(IO::VEC);
+#undef SLA_POOL_CASE
+}
+
+// partial states | column mean; states finished | block means of k
+template <typename IO, typename Tag, int D>
+static void launch_prefix_rest(const void* k, const RowLayout& lin, const void* kc, const void* vc, const RowLayout& lay, const MapParts& m,
+                               int in_dtype, const float* weight, int fmap, int BH, int L, char* states, char* parts, hipStream_t st) {
+  typedef typename IO::raw raw;
+  const LinWs w = lin_ws(BH, L, D);
+  const int first_wg = BH * (D / COLMEAN_SLAB);
+  hipLaunchKernelGGL((prefix_state_kernel<Tag, D, IO>), dim3(first_wg + BH * w.nsplit), dim3(256), 0, st, (const uint16_t*)kc,
+                     (const uint16_t*)vc, lay, (float*)(parts + (w.kv_part - w.states_end)),
+                     (float*)(parts + (w.z_part - w.states_end)), L, w.rows_per_split, w.nsplit, fmap, m, first_wg);
+  launch_state_presum<D>(BH, parts, w, st);
+  const StateFinish job = state_finish_job<D>(weight, BH, states, parts, w);
+#define SLA_FINISH_CASE(W)                                                                                                   \
+  {                                                                                                                          \
+    const int per_head = cdiv(m.N, 512 / (D / (W)));                                                                         \
+    hipLaunchKernelGGL((prefix_finish_kernel<Tag, D, IO, W>), dim3(xcd_grid(job.total) + BH * per_head), dim3(512), 0, st, job, \
+                       xcd_grid(job.total), (const raw*)k, lin, m, L, per_head);                                             \
+  }
+  if (narrow_pools(in_dtype, m, BH, D)) SLA_FINISH_CASE(IO::VEC / 4)
+  else SLA_FINISH_CASE(IO::VEC)
+#undef SLA_FINISH_CASE
 }
 
 int64_t module_fwd_workspace_bytes(int in_dtype, int BH, int L, int D, int BLKQ, int BLKK) {
@@ -70,34 +161,46 @@ extern "C" int sla_module_fwd(const void* q, const void* k, const void* v, const
   }
 
   const void *qc = q, *kc = k, *vc = v;
+  MapParts m{};
+  RowLayout lmap = lin;                // (q and k as the mask builder reads them: the inputs themselves)
+  if (!mask_given) m = block_map_parts(in_dtype, BH, L, D, BLKQ, BLKK, map_part, map_bytes);
   if (casts) {
     const int64_t n = (int64_t)BH * L * D;
-    const dim3 grid((unsigned)((n / 8 + 255) / 256), 3);
-    if (dtype == SLA_BF16)
-      hipLaunchKernelGGL((cast3_kernel<bf16_tag>), grid, dim3(256), 0, st, (const float*)q, (const float*)k, (const float*)v,
-                         (uint16_t*)cast, n);
-    else
-      hipLaunchKernelGGL((cast3_kernel<f16_tag>), grid, dim3(256), 0, st, (const float*)q, (const float*)k, (const float*)v,
-                         (uint16_t*)cast, n);
+    if (dtype == SLA_BF16) launch_prefix_pool<IoF32, bf16_tag>(q, k, v, lmap, m, in_dtype, BLKQ, BH, L, D, cast, st);
+    else launch_prefix_pool<IoF32, f16_tag>(q, k, v, lmap, m, in_dtype, BLKQ, BH, L, D, cast, st);
     qc = cast;
     kc = (uint16_t*)cast + n;
     vc = (uint16_t*)cast + 2 * n;
   }
-  const auto state = [&](hipStream_t s) {
-    return linear_state_run(kc, vc, lin, weight, dtype, fmap, BH, L, D, (char*)states, parts, s);
-  };
-  const auto mask = [&]() -> int {
-    if (mask_given) return SLA_OK;
-    return block_map_entry(q, k, qkv_strides, in_dtype, B, H, L, D, BLKQ, BLKK, topk, map_part, map_bytes, sparse_map,
-                           sparse_map != nullptr, lut, lut_elem_bytes, st);
-  };
+  const int lut64 = lut_elem_bytes == 8;
   const auto attention = [&]() {
     return attn_linear_run(qc, kc, vc, lin, lut, lut_elem_bytes, (const char*)states, bias, o_s, out, lout, lse, dtype, fmap, BH,
                            L, D, BLKQ, topk, qk_scale, st);
   };
-  if (!side || side == st || !side_stream_pays(B, H, L, D, topk)) {
-    if ((rc = state(st))) return rc;
-    if ((rc = mask())) return rc;
+  const bool two = side && side != st && side_stream_pays(B, H, L, D, topk);
+  if (!two) {
+    if (mask_given) {
+      if ((rc = linear_state_run(kc, vc, lin, weight, dtype, fmap, BH, L, D, (char*)states, parts, st))) return rc;
+      return attention();
+    }
+    if (in_dtype == SLA_BF16) launch_prefix_pool<IoBf16, NoCast>(q, k, v, lmap, m, in_dtype, BLKQ, BH, L, D, nullptr, st);
+    else if (in_dtype == SLA_F16) launch_prefix_pool<IoF16, NoCast>(q, k, v, lmap, m, in_dtype, BLKQ, BH, L, D, nullptr, st);
+#define SLA_REST_CASE(IO, TAG)                                                                                                  \
+  if (D == 128)                                                                                                                 \
+    launch_prefix_rest<IO, TAG, 128>(k, lmap, kc, vc, lin, m, in_dtype, weight, fmap, BH, L, (char*)states, parts, st);         \
+  else                                                                                                                          \
+    launch_prefix_rest<IO, TAG, 64>(k, lmap, kc, vc, lin, m, in_dtype, weight, fmap, BH, L, (char*)states, parts, st)
+    if (casts && dtype == SLA_BF16) {
+      SLA_REST_CASE(IoF32, bf16_tag);
+    } else if (casts) {
+      SLA_REST_CASE(IoF32, f16_tag);
+    } else if (dtype == SLA_BF16) {
+      SLA_REST_CASE(IoBf16, bf16_tag);
+    } else {
+      SLA_REST_CASE(IoF16, f16_tag);
+    }
+#undef SLA_REST_CASE
+    block_map_select(in_dtype, m, BH, D, topk, sparse_map, lut, lut64, st);
     return attention();
   }
   std::lock_guard<std::mutex> lock(side_events_mutex());
@@ -106,8 +209,9 @@ extern "C" int sla_module_fwd(const void* q, const void* k, const void* v, const
   SLA_HIP_OK(hipEventRecord(ev->fork, st));
   SLA_HIP_OK(hipStreamWaitEvent(side, ev->fork, 0));
   // (once the second stream waits on `stream`, no path leaves without `stream` waiting for it in turn)
-  rc = state(side);
-  const int rc_mask = mask();
+  rc = linear_state_run(kc, vc, lin, weight, dtype, fmap, BH, L, D, (char*)states, parts, side);
+  const int rc_mask = mask_given ? (int)SLA_OK
+                                 : block_map_run(q, k, lmap, in_dtype, m, BH, L, D, BLKQ, BLKK, topk, sparse_map, lut, lut64, !casts, st);
   SLA_HIP_OK(hipEventRecord(ev->first, side));
   SLA_HIP_OK(hipStreamWaitEvent(st, ev->first, 0));
   if (rc) return rc;
