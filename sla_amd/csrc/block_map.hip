@@ -73,7 +73,7 @@ __global__ __launch_bounds__(256) void colmean_fused_kernel(const float* __restr
                                                             typename IO::raw* __restrict__ colmean, int nchunk, int ngroup,
                                                             int D, int L) {
   __shared__ float gs[COLMEAN_MAX_GROUPS * COLMEAN_SLAB];
-  colmean_body<IO>(chunk_sums, colmean, nchunk, ngroup, D, L, blockIdx.x, blockIdx.y, gs);
+  colmean_body<IO, 256>(chunk_sums, colmean, nchunk, ngroup, D, L, blockIdx.x, blockIdx.y, gs);
 }
 
 // score[bh][m][n] = round_dtype( sum_d pq[m][d]*pk[n][d] ), d ascending, every product and every sum rounded to fp32.

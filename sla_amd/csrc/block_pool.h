@@ -157,18 +157,18 @@ static __device__ __forceinline__ void pool_pair_body(const typename IO::raw* __
     pool_body<IO, 1, W, 256, Cast>(q, lay, nullptr, pq, L, D, BLKQ, nblkq, tiled, bx, bh, cast);
 }
 
-// Column mean of K, levels 2 and 3 of the summation order: one workgroup of 256 threads per (head, slab of COLMEAN_SLAB
-// columns), thread (gi, c) = (tid / COLMEAN_SLAB, tid % COLMEAN_SLAB) forms group sums gi, gi + 16, ...
+// Column mean of K, levels 2 and 3 of the summation order: one workgroup of NT threads per (head, slab of COLMEAN_SLAB
+// columns), thread (gi, c) = (tid / COLMEAN_SLAB, tid % COLMEAN_SLAB) forms group sums gi, gi + NT / COLMEAN_SLAB, ...
 // of its column; the first COLMEAN_SLAB threads then add the groups in ascending order.  (Small workgroups: the
 // launch has to find room beside the memory-bound kernels that run on other streams at the same time.)
 constexpr int COLMEAN_SLAB = 16;
 constexpr int COLMEAN_MAX_GROUPS = 256;
-template <typename IO>
+template <typename IO, int NT>
 static __device__ __forceinline__ void colmean_body(const float* __restrict__ chunk_sums, typename IO::raw* __restrict__ colmean,
                                                     int nchunk, int ngroup, int D, int L, int slab, int bh, float* gs) {
   const int tid = threadIdx.x;
   const int c = tid % COLMEAN_SLAB, d = slab * COLMEAN_SLAB + c;
-  for (int g = tid / COLMEAN_SLAB; g < ngroup; g += 256 / COLMEAN_SLAB) {
+  for (int g = tid / COLMEAN_SLAB; g < ngroup; g += NT / COLMEAN_SLAB) {
     const int c0 = g * KMEAN_GROUP;
     const int n = min(KMEAN_GROUP, nchunk - c0);
     // (a group's loads all in flight, then added in order: mask builder of 16 heads x 6001 x 64 25.3 -> 23.2 us, of 40 x 75600 x 128 656 -> 652)

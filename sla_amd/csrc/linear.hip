@@ -143,7 +143,7 @@ template <typename Tag, int D>
 static int linear_state_quant_v_impl(const void* k, const void* v, const RowLayout& lay, const float* weight, int dtype, int fmap,
                                      int BH, int L, char* ws, uint8_t* v_fp8, float* v_scale, float v_range, hipStream_t st) {
   const LinWs w = lin_ws(BH, L, D);
-  hipLaunchKernelGGL((linear_state_partial_kernel<Tag, D, false, false, true>), dim3(w.nsplit, BH), dim3(256), 0, st,
+  hipLaunchKernelGGL((linear_state_partial_kernel<Tag, D, false, false, true>), dim3(w.nsplit, BH), dim3(StateTile<D, false>::NTH), 0, st,
                      (const uint16_t*)k, (const uint16_t*)v, lay, (float*)(ws + w.kv_part), (float*)(ws + w.z_part), L,
                      w.rows_per_split, fmap, (const float*)nullptr, (float*)(ws + w.vmax_part));
   int rc = quant_v_from_partial_amax(v, lay, dtype, BH, L, D, (const float*)(ws + w.vmax_part), w.nsplit, v_fp8, v_scale,

@@ -259,6 +259,18 @@ static __device__ __forceinline__ void forget_floats(i16x4_t (&x)[NT]) {
   }
 }
 
+// Reduction over N = 8 or 16 adjacent lanes, in all of them, without LDS: the same tree as shuffles by 1, 2, 4 (, 8) give.
+template <int N, typename Op>
+static __device__ __forceinline__ float over_lanes(float x, Op op) {
+#define SLA_DPP(CTRL) __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, true))
+  x = op(x, SLA_DPP(0xB1));                    // lane ^ 1
+  x = op(x, SLA_DPP(0x4E));                    // lane ^ 2
+  x = op(x, SLA_DPP(0x141));                   // mirrored within eight: the other four, which agree by now
+  if (N == 16) x = op(x, SLA_DPP(0x140));      // mirrored within sixteen
+#undef SLA_DPP
+  return x;
+}
+
 // Split of L among workgroups for the streaming state kernels.
 struct LinSplit {
   int nsplit, rows_per_split;

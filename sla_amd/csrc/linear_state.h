@@ -5,48 +5,63 @@
 namespace sla {
 
 // ---- kernel 1: partial states -----------------------------------------------------------
-// grid (nsplit, BH), 256 threads.  Thread t moves 16-byte chunk (t%CPR) of rows t/CPR + i*RPP.
+// grid (nsplit, BH).  Thread t moves 16-byte chunk (t%CPR) of rows t/CPR + i*RPP.
+// A slice is a chain of tiles, each a memory latency, the feature map and the products' reads of LDS: two tiles are in flight in
+// registers beside the one in LDS, and eight waves share a tile (head dim 128: 64 rows, two 32 x 32 parts of the state per wave;
+// head dim 64: 128 rows, one part per wave and half of the rows, the halves added at the end).  Against four waves per 64 rows
+// with one tile in flight, each row's sums through LDS: 8 heads x 4096 x 128, softmax map 19.8 -> 14.3 us, 16 heads x 6001 x 64
+// 13.6 -> 11.8, 12 heads x 32760 x 128 beside the mask builder 79.5 -> 76.5.
+// OUT16 (one tile of 64 rows per workgroup): four waves.
 // OUT16: the D x D partial is written rounded to 16 bit (per-key-block states of the complement mode).
 // ZW: zweight holds one fp32 per row of the head, (BH, L), and the z partial becomes sum_rows zweight * phi(k)
 // instead of sum_rows phi(k) (used by the complement backward, where "k" is q and "v" a row gradient).
 // VMAX: the largest |v| of every column over the slice goes to vmax_part[bh][split][D] (what the FP8 quantiser of v
 // needs of v before it can start: v is streamed here anyway).
-template <int D>
-constexpr int state_partial_lds() { return 2 * 64 * (D + 16) * 2 + 2048 * 4; }       // bytes
-// DEPTH: tiles in flight in registers beside the one in LDS.  Two where a launch does not fill the chip and a slice is a chain of
-// tile latencies; one where memory is the bound and the registers buy a third workgroup per compute unit.
-template <typename Tag, int D, bool OUT16, bool ZW, bool VMAX, int DEPTH>
+template <int D, bool OUT16>
+struct StateTile {
+  static constexpr int NTH = OUT16 ? 256 : 512;                    // threads
+  static constexpr int GROUPS = D == 64 && !OUT16 ? 2 : 1;         // groups of 64 rows, each with its own waves
+  static constexpr int TR = 64 * GROUPS;                           // rows per LDS tile
+  static constexpr int DEPTH = OUT16 ? 1 : 2;                      // tiles in flight in registers
+  static constexpr int STR = D + 16;                               // LDS row stride: transposed reads of 4 rows hit disjoint banks
+  static constexpr int LDS = 2 * TR * STR * 2;                     // bytes; the final sums reuse it
+};
+template <typename Tag, int D, bool OUT16, bool ZW, bool VMAX>
 static __device__ __forceinline__ void state_partial_body(const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
                                                           const RowLayout lay, void* __restrict__ kv_part_,
                                                           float* __restrict__ z_part, int L, int rows_per_split, int fmap,
                                                           const float* __restrict__ zweight, float* __restrict__ vmax_part,
                                                           int split, int bh, int nsplit, char* smem) {
   using E = Elem<Tag>;
-  constexpr int TR = 64;                 // rows per LDS tile
-  constexpr int STR = D + 16;            // LDS row stride: transposed reads of 4 rows hit disjoint banks
+  using T = StateTile<D, OUT16>;
+  constexpr int TR = T::TR, STR = T::STR, NTH = T::NTH, DEPTH = T::DEPTH;
   constexpr int CPR = D / 8;             // 16-byte chunks per row
-  constexpr int RPP = 256 / CPR;         // rows covered by one pass of the 256 threads
+  constexpr int RPP = NTH / CPR;         // rows covered by one pass of the workgroup
   constexpr int NP = TR / RPP;           // passes per tile
-  constexpr int DT = D / 32;             // 32-wide tiles along either state dimension
-  constexpr int WPT = (DT * DT) / 4;     // output tiles per wave (4 waves)
-  static_assert(DT * DT % 4 == 0, "state tiles must divide among 4 waves");
+  constexpr int DT = D / 32;             // 32-wide parts of the state along either dimension
+  constexpr int NWG = NTH / 64 / T::GROUPS;    // waves per group of rows
+  constexpr int WPT = (DT * DT) / NWG;   // parts per wave
+  static_assert(DT * DT % NWG == 0, "the parts of the state must divide among the waves");
 
   uint16_t* const sK = reinterpret_cast<uint16_t*>(smem);
   uint16_t* const sV = sK + TR * STR;
-  float (*sZ)[D] = reinterpret_cast<float (*)[D]>(smem + 2 * TR * STR * 2);
-  static_assert(RPP * D == 2048, "a pass of the workgroup is 2048 columns");
+  float (*sZ)[D] = reinterpret_cast<float (*)[D]>(smem);
+  static_assert(RPP * D * 4 <= T::LDS && (T::GROUPS == 1 || NWG * 64 * 16 * 4 <= T::LDS), "the final sums do not fit the tiles");
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int g = lane >> 5;
   const int row_begin = split * rows_per_split;
   const int row_end = min(L, row_begin + rows_per_split);
-  const uint16_t* kh = k + lay.head(bh);
-  const uint16_t* vh = v + lay.head(bh);
-  const size_t pitch = (size_t)lay.sl;
+  // (slices are whole tiles but for the last of a head: rows past it lie outside the descriptors and read as zero)
+  const __amdgpu_buffer_rsrc_t k_rs = make_rsrc(k + lay.head(bh), lay.head_range_bytes(L, D));
+  const __amdgpu_buffer_rsrc_t v_rs = make_rsrc(v + lay.head(bh), lay.head_range_bytes(L, D));
+  const __amdgpu_buffer_rsrc_t w_rs = make_rsrc(ZW ? zweight + (size_t)bh * L : nullptr, ZW ? (uint32_t)L * 4u : 0u);
+  const uint32_t pitch_b = (uint32_t)lay.sl * 2u;
 
   const int lrow = tid / CPR, lcol = (tid % CPR) * 8;
 
-  // wave w owns output tiles w*WPT .. w*WPT+WPT-1; tile id = d1tile*DT + d2tile
+  // wave w of its group owns parts w*WPT .. w*WPT+WPT-1; part = d1part*DT + d2part
+  const int gw = wave % NWG, group = wave / NWG;
   f32x16_t acc[WPT];
 #pragma unroll
   for (int t = 0; t < WPT; ++t)
@@ -71,15 +86,10 @@ static __device__ __forceinline__ void state_partial_body(const uint16_t* __rest
   auto fetch = [&](int r0, int s) __attribute__((always_inline)) {
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
-      const int grow = r0 + lrow + p * RPP;
-      kreg[s][p] = i16x8_t{0, 0, 0, 0, 0, 0, 0, 0};
-      vreg[s][p] = i16x8_t{0, 0, 0, 0, 0, 0, 0, 0};
-      wreg[s][p] = 1.0f;
-      if (grow < row_end) {
-        kreg[s][p] = *reinterpret_cast<const i16x8_t*>(kh + (size_t)grow * pitch + lcol);
-        vreg[s][p] = *reinterpret_cast<const i16x8_t*>(vh + (size_t)grow * pitch + lcol);
-        if (ZW) wreg[s][p] = zweight[(size_t)bh * L + grow];
-      }
+      const uint32_t grow = (uint32_t)(r0 + lrow + p * RPP);
+      kreg[s][p] = buf_load_b128(k_rs, grow * pitch_b + 2u * (uint32_t)lcol);
+      vreg[s][p] = buf_load_b128(v_rs, grow * pitch_b + 2u * (uint32_t)lcol);
+      wreg[s][p] = ZW ? __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(w_rs, (int)(grow * 4u), 0, 0)) : 1.0f;
     }
   };
   if (row_begin < row_end)
@@ -101,16 +111,14 @@ static __device__ __forceinline__ void state_partial_body(const uint16_t* __rest
         float mx = f[0];
 #pragma unroll
         for (int e = 1; e < 8; ++e) mx = fmaxf(mx, f[e]);
-#pragma unroll
-        for (int s = 1; s < CPR; s <<= 1) mx = fmaxf(mx, __shfl_xor(mx, s));
+        mx = over_lanes<CPR>(mx, [](float a, float b) { return fmaxf(a, b); });
         float sum = 0.f;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           f[e] = __expf(f[e] - mx);
           sum += f[e];
         }
-#pragma unroll
-        for (int s = 1; s < CPR; s <<= 1) sum += __shfl_xor(sum, s);
+        sum = over_lanes<CPR>(sum, [](float a, float b) { return a + b; });
         const float inv = 1.0f / sum;
 #pragma unroll
         for (int e = 0; e < 8; ++e) f[e] = round16<Tag>(f[e] * inv);
@@ -140,11 +148,11 @@ static __device__ __forceinline__ void state_partial_body(const uint16_t* __rest
     lds_barrier();
     if (r0 + DEPTH * TR < row_end) fetch(r0 + DEPTH * TR, s);
 #pragma unroll
-    for (int c = 0; c < TR / 16; ++c) {
-      const int l0 = 16 * c + 8 * g + tr_row;
+    for (int c = 0; c < 4; ++c) {
+      const int l0 = 64 * group + 16 * c + 8 * g + tr_row;
 #pragma unroll
       for (int t = 0; t < WPT; ++t) {
-        const int d1t = (wave * WPT + t) / DT, d2t = (wave * WPT + t) % DT;
+        const int d1t = (gw * WPT + t) / DT, d2t = (gw * WPT + t) % DT;
         const uint16_t* pa = &sK[l0 * STR + 32 * d1t + tr_col];
         const uint16_t* pb = &sV[l0 * STR + 32 * d2t + tr_col];
         const i16x8_t a = concat4(lds_read_tr16(pa), lds_read_tr16(pa + 4 * STR));
@@ -158,12 +166,21 @@ static __device__ __forceinline__ void state_partial_body(const uint16_t* __rest
     for (int s = 0; s < DEPTH; ++s)
       if (s == 0 || r0 + s * TR < row_end) tile(r0 + s * TR, s);
 
+  lds_barrier();             // (the tiles are free)
+  if constexpr (T::GROUPS == 2) {
+    static_assert(WPT == 1, "one part per wave");
+    f32x16_t* const other = reinterpret_cast<f32x16_t*>(smem) + (size_t)gw * 64 + lane;
+    if (group) *other = acc[0];
+    lds_barrier();
+    if (!group) acc[0] += *other;
+    lds_barrier();
+  }
   // partial KV, stored transposed: kv_part[bh][split][d2][d1]
   const size_t part_off = ((size_t)bh * nsplit + split) * D * D;
 #pragma unroll
   for (int t = 0; t < WPT; ++t) {
-    const int tile = wave * WPT + t;
-    const int d1t = tile / DT, d2t = tile % DT;
+    if (group) break;
+    const int d1t = (gw * WPT + t) / DT, d2t = (gw * WPT + t) % DT;
     const int d2 = 32 * d2t + (lane & 31);
 #pragma unroll
     for (int i4 = 0; i4 < 4; ++i4) {
@@ -180,10 +197,10 @@ static __device__ __forceinline__ void state_partial_body(const uint16_t* __rest
     }
   }
   // partial z: reduce the RPP row groups through LDS
-  __syncthreads();
 #pragma unroll
-  for (int e = 0; e < 8; ++e) sZ[lrow][lcol + e] = zacc[e];
-  __syncthreads();
+  for (int x = 0; x < 2; ++x)
+    *reinterpret_cast<f32x4_t*>(&sZ[lrow][lcol + 4 * x]) = f32x4_t{zacc[4 * x], zacc[4 * x + 1], zacc[4 * x + 2], zacc[4 * x + 3]};
+  lds_barrier();
   if (tid < D) {
     float s = 0.f;
 #pragma unroll
@@ -191,13 +208,13 @@ static __device__ __forceinline__ void state_partial_body(const uint16_t* __rest
     z_part[((size_t)bh * nsplit + split) * D + tid] = s;
   }
   if (VMAX) {
-    __syncthreads();
+    lds_barrier();
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       sZ[lrow][lcol + 2 * j] = E::to_float(vmx[j][0]);
       sZ[lrow][lcol + 2 * j + 1] = E::to_float(vmx[j][1]);
     }
-    __syncthreads();
+    lds_barrier();
     if (tid < D) {
       float a = 0.f;
 #pragma unroll
@@ -208,12 +225,12 @@ static __device__ __forceinline__ void state_partial_body(const uint16_t* __rest
 }
 
 template <typename Tag, int D, bool OUT16 = false, bool ZW = false, bool VMAX = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void linear_state_partial_kernel(
+__global__ __launch_bounds__((StateTile<D, OUT16>::NTH)) __attribute__((amdgpu_waves_per_eu(OUT16 ? 3 : 4, OUT16 ? 3 : 4))) void linear_state_partial_kernel(
     const uint16_t* __restrict__ k, const uint16_t* __restrict__ v, const RowLayout lay, void* __restrict__ kv_part,
     float* __restrict__ z_part, int L, int rows_per_split, int fmap, const float* __restrict__ zweight = nullptr,
     float* __restrict__ vmax_part = nullptr) {
-  __shared__ __attribute__((aligned(16))) char smem[state_partial_lds<D>()];
-  state_partial_body<Tag, D, OUT16, ZW, VMAX, 1>(k, v, lay, kv_part, z_part, L, rows_per_split, fmap, zweight, vmax_part, blockIdx.x,
+  __shared__ __attribute__((aligned(16))) char smem[StateTile<D, OUT16>::LDS];
+  state_partial_body<Tag, D, OUT16, ZW, VMAX>(k, v, lay, kv_part, z_part, L, rows_per_split, fmap, zweight, vmax_part, blockIdx.x,
                                               blockIdx.y, gridDim.x, smem);
 }
 
@@ -434,7 +451,7 @@ static inline LinWs lin_ws(int BH, int L, int D) {
   // rows; more only lengthen the chain that adds them up (state build of 8 heads x 4096 rows x 128: 64 slices 34.6 us, 16
   // slices 23.8; 4 heads x 7813 x 64: 123 slices 23.5, 31 slices 15.3; with 1024 rows 16 slices of 64 rows 14.7, 4 of 256 19.4).
   const int min_rows = L >= 4096 ? 256 : cdiv(L, 16);
-  const LinSplit sp = lin_split(BH, L, 512, 64, min_rows);
+  const LinSplit sp = lin_split(BH, L, 512, D == 64 ? StateTile<64, false>::TR : StateTile<128, false>::TR, min_rows);
   w.nsplit = sp.nsplit;
   w.rows_per_split = sp.rows_per_split;
   size_t off = 0;
@@ -485,7 +502,7 @@ static inline void launch_state_finish(const float* weight, int BH, char* ws, ch
 template <typename Tag, int D>
 static inline void launch_state_build(const void* k, const void* v, const RowLayout& lay, const float* weight, int fmap,
                                       int BH, int L, char* ws, char* parts, const LinWs& w, hipStream_t st) {
-  hipLaunchKernelGGL((linear_state_partial_kernel<Tag, D>), dim3(w.nsplit, BH), dim3(256), 0, st, (const uint16_t*)k,
+  hipLaunchKernelGGL((linear_state_partial_kernel<Tag, D>), dim3(w.nsplit, BH), dim3(StateTile<D, false>::NTH), 0, st, (const uint16_t*)k,
                      (const uint16_t*)v, lay, (void*)(parts + (w.kv_part - w.states_end)),
                      (float*)(parts + (w.z_part - w.states_end)), L, w.rows_per_split, fmap);
   launch_state_finish<Tag, D>(weight, BH, ws, parts, w, st);

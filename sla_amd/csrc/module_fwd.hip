@@ -43,19 +43,19 @@ __global__ __launch_bounds__(256) void prefix_pool_kernel(const typename IO::raw
 
 // The slices' partial states and, in the first `first_wg` workgroups, the column mean of k; one head's slices are adjacent.
 template <typename Tag, int D, typename IO>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void prefix_state_kernel(
+__global__ __launch_bounds__((StateTile<D, false>::NTH)) __attribute__((amdgpu_waves_per_eu(4, 4))) void prefix_state_kernel(
     const uint16_t* __restrict__ k, const uint16_t* __restrict__ v, const RowLayout lay, float* __restrict__ kv_part,
     float* __restrict__ z_part, int L, int rows_per_split, int nsplit, int fmap, const MapParts m, int first_wg) {
-  constexpr int LDS = state_partial_lds<D>() > COLMEAN_MAX_GROUPS * COLMEAN_SLAB * 4 ? state_partial_lds<D>() : COLMEAN_MAX_GROUPS * COLMEAN_SLAB * 4;
-  __shared__ __attribute__((aligned(16))) char smem[LDS];
+  static_assert(COLMEAN_MAX_GROUPS * COLMEAN_SLAB * 4 <= StateTile<D, false>::LDS, "the column mean's sums fit the tiles");
+  __shared__ __attribute__((aligned(16))) char smem[StateTile<D, false>::LDS];
   const int wg = blockIdx.x;
   if (wg < first_wg) {
-    colmean_body<IO>(m.chunk_sums, (typename IO::raw*)m.colmean, m.nchunk, (m.nchunk + KMEAN_GROUP - 1) / KMEAN_GROUP, D, L,
+    colmean_body<IO, StateTile<D, false>::NTH>(m.chunk_sums, (typename IO::raw*)m.colmean, m.nchunk, (m.nchunk + KMEAN_GROUP - 1) / KMEAN_GROUP, D, L,
                      wg % (D / COLMEAN_SLAB), wg / (D / COLMEAN_SLAB), reinterpret_cast<float*>(smem));
     return;
   }
   const int bh = (wg - first_wg) / nsplit;
-  state_partial_body<Tag, D, false, false, false, 2>(k, v, lay, kv_part, z_part, L, rows_per_split, fmap, nullptr, nullptr,
+  state_partial_body<Tag, D, false, false, false>(k, v, lay, kv_part, z_part, L, rows_per_split, fmap, nullptr, nullptr,
                                                   wg - first_wg - bh * nsplit, bh, nsplit, smem);
 }
 
@@ -100,7 +100,7 @@ static void launch_prefix_rest(const void* k, const RowLayout& lin, const void* 
   typedef typename IO::raw raw;
   const LinWs w = lin_ws(BH, L, D);
   const int first_wg = BH * (D / COLMEAN_SLAB);
-  hipLaunchKernelGGL((prefix_state_kernel<Tag, D, IO>), dim3(first_wg + BH * w.nsplit), dim3(256), 0, st, (const uint16_t*)kc,
+  hipLaunchKernelGGL((prefix_state_kernel<Tag, D, IO>), dim3(first_wg + BH * w.nsplit), dim3(StateTile<D, false>::NTH), 0, st, (const uint16_t*)kc,
                      (const uint16_t*)vc, lay, (float*)(parts + (w.kv_part - w.states_end)),
                      (float*)(parts + (w.z_part - w.states_end)), L, w.rows_per_split, w.nsplit, fmap, m, first_wg);
   launch_state_presum<D>(BH, parts, w, st);
