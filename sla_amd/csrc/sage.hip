@@ -11,7 +11,9 @@
 //   O = (e4m3(c P) . v_fp8) * sv / sum(e4m3(c P)), c = 112 with P <= 4 (reference maximum lagging by <= 2).
 // The look-up table of the bf16 path is used as is (no delta encoding is needed here).
 #include "block_map.h"
+#include "block_pool.h"
 #include "common.h"
+#include "linear_state.h"
 #include "sage_steps.h"
 #include "side_events.h"
 
@@ -29,20 +31,22 @@ void launch_map_from_pooled(int dtype, const void* pq, const void* pk, void* sco
 // POOL: also write the block mean the mask builder needs (of x, or of x - colmean rounded to 16 bit, as
 // get_block_map pools it: utils.py:55-58 of the reference), summed row by row in fp32 and divided once,
 // exactly as the pooling kernel of the mask builder does, so the block is read from memory once for both.
+template <int D, int BLK, bool POOL>
+constexpr int quant_int8_lds() { return 16 + (POOL ? BLK * (D + 8) * 2 : 0); }       // bytes
+// (tid: this thread among the 256 of the block; a workgroup may hold several blocks, of which some are not `active`)
 template <typename Tag, int D, int BLK, bool SUB_MEAN, bool POOL>
-__global__ __launch_bounds__(256) void quant_int8_kernel(const uint16_t* __restrict__ x, const RowLayout lay,
-                                                         const uint16_t* __restrict__ colmean, int8_t* __restrict__ xq,
-                                                         float* __restrict__ scale, uint16_t* __restrict__ pooled, int L,
-                                                         int nblk, int tiled) {
+static __device__ __forceinline__ void quant_int8_body(const uint16_t* __restrict__ x, const RowLayout lay,
+                                                       const uint16_t* __restrict__ colmean, int8_t* __restrict__ xq,
+                                                       float* __restrict__ scale, uint16_t* __restrict__ pooled, int L,
+                                                       int nblk, int tiled, int blk, int bh, int tid, bool active, char* smem) {
   using E = Elem<Tag>;
   constexpr int CPR = D / 8;
   constexpr int RPP = 256 / CPR;
   constexpr int NP = BLK / RPP;
   constexpr int TSTR = D + 8;
-  __shared__ float sred[4];
-  __shared__ __attribute__((aligned(16))) uint16_t tile[POOL ? BLK * TSTR : 8];
-  const int blk = blockIdx.x, bh = blockIdx.y;
-  const int tid = threadIdx.x;
+  float* const sred = reinterpret_cast<float*>(smem);
+  uint16_t* const tile = reinterpret_cast<uint16_t*>(smem + 16);
+  if (!active) blk = nblk;                 // (every row of it lies past the end)
   const int lrow = tid / CPR, lcol = (tid % CPR) * 8;
   float cm[8];
 #pragma unroll
@@ -83,6 +87,7 @@ __global__ __launch_bounds__(256) void quant_int8_kernel(const uint16_t* __restr
   for (int s = 1; s < 64; s <<= 1) amax = fmaxf(amax, __shfl_xor(amax, s));
   if ((tid & 63) == 0) sred[tid >> 6] = amax;
   __syncthreads();
+  if (!active) return;
   amax = fmaxf(fmaxf(sred[0], sred[1]), fmaxf(sred[2], sred[3]));
   const float sc = fmaxf(amax, 1e-30f) / 127.0f;
   if (tid == 0) scale[(size_t)bh * nblk + blk] = sc;
@@ -123,6 +128,16 @@ __global__ __launch_bounds__(256) void quant_int8_kernel(const uint16_t* __restr
     }
     *reinterpret_cast<i32x2_t*>(xq + ((size_t)bh * L + grow) * D + lcol) = w;
   }
+}
+
+template <typename Tag, int D, int BLK, bool SUB_MEAN, bool POOL>
+__global__ __launch_bounds__(256) void quant_int8_kernel(const uint16_t* __restrict__ x, const RowLayout lay,
+                                                         const uint16_t* __restrict__ colmean, int8_t* __restrict__ xq,
+                                                         float* __restrict__ scale, uint16_t* __restrict__ pooled, int L,
+                                                         int nblk, int tiled) {
+  __shared__ __attribute__((aligned(16))) char smem[quant_int8_lds<D, BLK, POOL>()];
+  quant_int8_body<Tag, D, BLK, SUB_MEAN, POOL>(x, lay, colmean, xq, scale, pooled, L, nblk, tiled, blockIdx.x, blockIdx.y,
+                                               threadIdx.x, true, smem);
 }
 
 // ---- FP8 per-channel quantisation of V ------------------------------------------------------
@@ -766,6 +781,140 @@ extern "C" int sage_sparse_attn_fwd(const int8_t* q_int8, const float* q_scale, 
 #undef SAGE_CASE
 }
 
+// ---- the preparation of small inputs in four launches -----------------------------------------------------------------
+// The same work as sage_prepare and sla_linear_state_quant_v_fwd, launches that need nothing of each other in one:
+//   q quantised (with its block means), chunk sums of k | slices' partial states (with the maxima of |v|), column mean of k |
+//   states finished, k quantised (with its block means), v quantised | scores and selection
+// Eleven launches of 2 to 12 us were what a call on 16 heads x 5003 x 64 consisted of besides its attention: 54 us in eight, now 36 in three.
+namespace sla {
+
+template <typename Tag>
+struct IoOf;
+template <>
+struct IoOf<bf16_tag> {
+  typedef IoBf16 type;
+};
+template <>
+struct IoOf<f16_tag> {
+  typedef IoF16 type;
+};
+
+template <typename Tag, int D>
+__global__ __launch_bounds__(256) void sage_first_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
+                                                         const RowLayout lay, int8_t* __restrict__ q8, float* __restrict__ qs,
+                                                         uint16_t* __restrict__ pq, int M, int tiled, float* __restrict__ chunk_sums,
+                                                         int nchunk, int L, int quant_wgs, int per_head) {
+  __shared__ __attribute__((aligned(16))) char smem[quant_int8_lds<D, 128, true>()];
+  const int wg = blockIdx.x;
+  if (wg < quant_wgs) {
+    quant_int8_body<Tag, D, 128, false, true>(q, lay, nullptr, q8, qs, pq, L, M, tiled, wg % M, wg / M, threadIdx.x, true, smem);
+  } else {
+    const int i = wg - quant_wgs, bh = i / per_head;
+    pool_body<typename IoOf<Tag>::type, 0, 2, 256>(k, lay, nullptr, chunk_sums, L, D, KMEAN_CHUNK, nchunk, 0, i - bh * per_head, bh);
+  }
+}
+
+template <typename Tag, int D>
+__global__ __launch_bounds__((StateTile<D, false>::NTH)) __attribute__((amdgpu_waves_per_eu(4, 4))) void sage_state_kernel(
+    const uint16_t* __restrict__ k, const uint16_t* __restrict__ v, const RowLayout lay, float* __restrict__ kv_part,
+    float* __restrict__ z_part, float* __restrict__ vmax_part, int L, int rows_per_split, int nsplit, int fmap,
+    const float* __restrict__ chunk_sums, uint16_t* __restrict__ colmean, int nchunk, int first_wg) {
+  static_assert(COLMEAN_MAX_GROUPS * COLMEAN_SLAB * 4 <= StateTile<D, false>::LDS, "the column mean's sums fit the tiles");
+  __shared__ __attribute__((aligned(16))) char smem[StateTile<D, false>::LDS];
+  const int wg = blockIdx.x;
+  if (wg < first_wg) {
+    colmean_body<typename IoOf<Tag>::type, StateTile<D, false>::NTH>(chunk_sums, colmean, nchunk, (nchunk + KMEAN_GROUP - 1) / KMEAN_GROUP,
+                                                                     D, L, wg % (D / COLMEAN_SLAB), wg / (D / COLMEAN_SLAB),
+                                                                     reinterpret_cast<float*>(smem));
+    return;
+  }
+  const int bh = (wg - first_wg) / nsplit;
+  state_partial_body<Tag, D, false, false, true>(k, v, lay, kv_part, z_part, L, rows_per_split, fmap, nullptr, vmax_part,
+                                                 wg - first_wg - bh * nsplit, bh, nsplit, smem);
+}
+
+// first `finish_wgs` workgroups: the states; then two key blocks per workgroup; then 512 * 8 values of v per workgroup, whose
+// scales it forms from the slices' maxima itself (the first one of a head leaves them for the attention).
+template <typename Tag, int D>
+__global__ __launch_bounds__(512) void sage_finish_kernel(const StateFinish job, int finish_wgs, const uint16_t* __restrict__ k,
+                                                          const uint16_t* __restrict__ v, const RowLayout lay,
+                                                          const uint16_t* __restrict__ colmean, int8_t* __restrict__ k8,
+                                                          float* __restrict__ ks, uint16_t* __restrict__ pk, int N, int tiled,
+                                                          int quant_wgs, const float* __restrict__ vmax_part, uint8_t* __restrict__ v8,
+                                                          float* __restrict__ vs, float v_range, int L, int v_wgs) {
+  constexpr int QLDS = (quant_int8_lds<D, 64, true>() + 15) / 16 * 16;
+  constexpr int LDS = state_finish_lds<D>() > 2 * QLDS ? state_finish_lds<D>() : 2 * QLDS;
+  __shared__ __attribute__((aligned(16))) char smem[LDS];
+  int wg = blockIdx.x;
+  if (wg < finish_wgs) {
+    const int logical = xcd_remap(wg, finish_wgs, job.total);
+    if (logical >= 0) state_finish_body<Tag, D>(job, logical, smem);
+    return;
+  }
+  wg -= finish_wgs;
+  const int tid = threadIdx.x;
+  if (wg < quant_wgs) {
+    const int per_head = (N + 1) / 2, bh = wg / per_head, half = tid >> 8, blk = 2 * (wg - bh * per_head) + half;
+    quant_int8_body<Tag, D, 64, true, true>(k, lay, colmean, k8, ks, pk, L, N, tiled, blk, bh, tid & 255, blk < N, smem + half * QLDS);
+    return;
+  }
+  wg -= quant_wgs;
+  using E = Elem<Tag>;
+  constexpr int CPR = D / 8, RPP = 512 / CPR;
+  const int bh = wg / v_wgs, part = wg - bh * v_wgs;
+  float* const s_scale = reinterpret_cast<float*>(smem);
+  if (tid < D) {
+    const float* p = vmax_part + (size_t)bh * job.nsplit * D + tid;
+    float a = 0.f;
+#pragma unroll 16
+    for (int c = 0; c < job.nsplit; ++c) a = fmaxf(a, p[(size_t)c * D]);
+    a = fmaxf(a, 1e-30f) / v_range;
+    s_scale[tid] = a;
+    if (part == 0) vs[(size_t)bh * D + tid] = a;
+  }
+  const int row = part * RPP + tid / CPR, lcol = (tid % CPR) * 8;
+  i16x8_t x = {0, 0, 0, 0, 0, 0, 0, 0};
+  if (row < L) x = *reinterpret_cast<const i16x8_t*>(v + lay.head(bh) + (size_t)row * (size_t)lay.sl + lcol);
+  lds_barrier();
+  if (row >= L) return;
+  float f[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) f[e] = E::to_float((uint16_t)x[e]) / s_scale[lcol + e];
+  i32x2_t w;
+  w[0] = (int)cvt4_fp8(f[0], f[1], f[2], f[3]);
+  w[1] = (int)cvt4_fp8(f[4], f[5], f[6], f[7]);
+  *reinterpret_cast<i32x2_t*>(v8 + ((size_t)bh * L + row) * D + lcol) = w;
+}
+
+template <typename Tag, int D>
+static void launch_small_preparation(const void* q, const void* k, const void* v, const RowLayout& lay, int dtype, const float* weight,
+                                     int fmap, int BH, int L, int topk, void* lut, int8_t* q8, float* qs, int8_t* k8, float* ks,
+                                     uint8_t* v8, float* vs, float v_range, char* prep, char* linear, hipStream_t st) {
+  const SageWs w = sage_ws(BH, L, D);
+  const SagePrepWs p = sage_prep_ws(BH, L, D);
+  const LinWs lw = lin_ws(BH, L, D);
+  const int M = cdiv(L, 128), N = cdiv(L, 64), tiled = score_takes_tiled(dtype, D);
+  float* const chunk_sums = (float*)(prep + w.chunk_sums);
+  uint16_t *const colmean = (uint16_t*)(prep + w.colmean), *const pq = (uint16_t*)(prep + p.pq), *const pk = (uint16_t*)(prep + p.pk);
+  const int per_head = cdiv(N, 256 / (D / 2));               // (chunks of KMEAN_CHUNK = 64 rows)
+  hipLaunchKernelGGL((sage_first_kernel<Tag, D>), dim3(BH * M + BH * per_head), dim3(256), 0, st, (const uint16_t*)q,
+                     (const uint16_t*)k, lay, q8, qs, pq, M, tiled, chunk_sums, N, L, BH * M, per_head);
+  const int first_wg = BH * (D / COLMEAN_SLAB);
+  hipLaunchKernelGGL((sage_state_kernel<Tag, D>), dim3(first_wg + BH * lw.nsplit), dim3(StateTile<D, false>::NTH), 0, st,
+                     (const uint16_t*)k, (const uint16_t*)v, lay, (float*)(linear + lw.kv_part), (float*)(linear + lw.z_part),
+                     (float*)(linear + lw.vmax_part), L, lw.rows_per_split, lw.nsplit, fmap, (const float*)chunk_sums, colmean, N,
+                     first_wg);
+  launch_state_presum<D>(BH, linear + lw.states_end, lw, st);
+  const StateFinish job = state_finish_job<D>(weight, BH, linear, linear + lw.states_end, lw);
+  const int finish_wgs = xcd_grid(job.total), quant_wgs = BH * cdiv(N, 2), v_wgs = cdiv(L, 512 / (D / 8));
+  hipLaunchKernelGGL((sage_finish_kernel<Tag, D>), dim3(finish_wgs + quant_wgs + BH * v_wgs), dim3(512), 0, st, job, finish_wgs,
+                     (const uint16_t*)k, (const uint16_t*)v, lay, (const uint16_t*)colmean, k8, ks, pk, N, tiled, quant_wgs,
+                     (const float*)(linear + lw.vmax_part), v8, vs, v_range, L, v_wgs);
+  launch_map_from_pooled(dtype, pq, pk, prep + p.score, BH, M, N, D, topk, nullptr, lut, 0, st);
+}
+
+}  // namespace sla
+
 // ---- the whole quantised forward in one call -----------------------------------------------------------------------
 namespace sla {
 struct SageModuleWs {
@@ -842,8 +991,20 @@ extern "C" int sage_module_fwd(const void* q, const void* k, const void* v, cons
                        : sla_linear_out_fwd(q, bias, o_s, out, dtype, fmap, B, H, L, D, ws + w.linear, w.linear_bytes, stream);
   };
   if (!side || side == st || !side_stream_pays(B, H, L, D, topk)) {
-    if ((rc = state(st))) return rc;
-    if ((rc = prepare())) return rc;
+    if ((rc = make_layout(qkv_strides, B, H, L, D, 2, &lay))) return rc;
+    SLA_REQUIRE(w.linear_bytes >= linear_fwd_workspace_bytes(B * H, L, D), SLA_ERR_WORKSPACE, "workspace too small");
+#define SAGE_SMALL_CASE(TAG, DD)                                                                                              \
+  launch_small_preparation<TAG, DD>(q, k, v, lay, dtype, weight, fmap, B * H, L, topk, lut, q8, qs, k8, ks, v8, vs, v_range, \
+                                    ws + w.prep, ws + w.linear, st)
+    if (dtype == SLA_BF16) {
+      if (D == 128) SAGE_SMALL_CASE(bf16_tag, 128);
+      else SAGE_SMALL_CASE(bf16_tag, 64);
+    } else {
+      if (D == 128) SAGE_SMALL_CASE(f16_tag, 128);
+      else SAGE_SMALL_CASE(f16_tag, 64);
+    }
+#undef SAGE_SMALL_CASE
+    if ((rc = check_launch("sage_module_fwd"))) return rc;
     return attention();
   }
   std::lock_guard<std::mutex> lock(side_events_mutex());

@@ -37,3 +37,23 @@ def test_forward_equals_the_steps(dev, B, H, L, D, BLKQ, in_dtype, fmap, half):
         if in_dtype == dtype:                  # (B, L, H, D) activations read where they lie
             rows = [t.transpose(1, 2).contiguous().transpose(1, 2) for t in (q, k, v)]
             assert torch.equal(mod(*rows), out)
+
+
+@pytest.mark.parametrize("H,L,D,fmap,half", [(1, 1, 64, "softmax", False), (2, 63, 128, "elu", True), (3, 129, 64, "relu", False),
+                                             (5, 2049, 128, "softmax", False), (1, 10500, 64, "elu", False)])
+def test_quantised_forward_equals_the_steps(dev, H, L, D, fmap, half):
+    """The quantised module's preparation likewise: an odd number of key blocks, less than a block, a state build of many slices."""
+    from sla_amd import SageSparseLinearAttention
+    from sla_amd.linear import linear_out_fwd, linear_state_quant_v_fwd
+    from sla_amd.sage import sage_attn_fwd, sage_prepare
+    dtype, ratio = torch.float16 if half else torch.bfloat16, 1.0 if L < 256 else 0.2
+    g = torch.Generator().manual_seed(L + D)
+    q, k, v = (torch.randn(1, H, L, D, generator=g).to(dtype).to(dev) for _ in range(3))
+    mod = SageSparseLinearAttention(D, ratio, fmap, use_bf16=not half).to(dev)
+    with torch.no_grad():
+        for p, t in zip((mod.proj_l.weight, mod.proj_l.bias), make_proj(D)):
+            p.copy_(t)
+        _, lut, T, q8, qs, k8, ks, _, _ = sage_prepare(q, k, None, ratio)
+        ws, v8, vs = linear_state_quant_v_fwd(k, v, mod.proj_l.weight, fmap)
+        o_s = sage_attn_fwd(q8, qs, k8, ks, v8, vs, lut, T, dtype)
+        assert torch.equal(mod(q, k, v), linear_out_fwd(q, mod.proj_l.bias, o_s, ws, fmap))
