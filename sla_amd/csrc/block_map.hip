@@ -21,20 +21,20 @@
 
 namespace sla {
 
-template <typename IO, int MODE>
+template <typename IO, int MODE, int W>
 __global__ __launch_bounds__(256) void pool_kernel(const typename IO::raw* __restrict__ x, const RowLayout lay,
                                                    const typename IO::raw* __restrict__ colmean,
                                                    void* __restrict__ out, int L, int D, int BLK, int nblk, int tiled) {
-  pool_body<IO, MODE, IO::VEC, 256>(x, lay, colmean, out, L, D, BLK, nblk, tiled, blockIdx.x, blockIdx.y);
+  pool_body<IO, MODE, W, 256>(x, lay, colmean, out, L, D, BLK, nblk, tiled, blockIdx.x, blockIdx.y);
 }
 
 // The two independent first passes of the mask builder in one launch (neither fills the memory system alone).
-template <typename IO>
+template <typename IO, int W>
 __global__ __launch_bounds__(256) void pool_pair_kernel(const typename IO::raw* __restrict__ k, float* __restrict__ chunk_sums,
                                                         int nchunk, const typename IO::raw* __restrict__ q,
                                                         const RowLayout lay, typename IO::raw* __restrict__ pq, int BLKQ,
                                                         int nblkq, int L, int D, int tiled) {
-  pool_pair_body<IO, IO::VEC>(k, chunk_sums, nchunk, q, lay, pq, BLKQ, nblkq, L, D, tiled, blockIdx.x, blockIdx.y, blockIdx.z);
+  pool_pair_body<IO, W>(k, chunk_sums, nchunk, q, lay, pq, BLKQ, nblkq, L, D, tiled, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 
 // Column mean of K, levels 2 and 3 of the fixed summation order:
@@ -763,10 +763,13 @@ template <typename IO, int MODE>
 static void launch_pool(const void* x, const RowLayout& lay, const void* colmean, void* out, int BH, int L, int D, int BLK,
                         hipStream_t st, int tiled = 0) {
   const int nblk = cdiv(L, BLK);
-  const int bpw = 256 / (D / IO::VEC);
-  dim3 grid(cdiv(nblk, bpw), BH);
-  hipLaunchKernelGGL((pool_kernel<IO, MODE>), grid, dim3(256), 0, st, (const typename IO::raw*)x, lay,
-                     (const typename IO::raw*)colmean, out, L, D, BLK, nblk, tiled);
+  typedef typename IO::raw raw;
+  if (narrow_pools(sizeof(raw) == 4 ? SLA_F32 : SLA_BF16, BH, L, D) && D / (IO::VEC / 4) <= 256)
+    hipLaunchKernelGGL((pool_kernel<IO, MODE, IO::VEC / 4>), dim3(cdiv(nblk, 256 / (D / (IO::VEC / 4))), BH), dim3(256), 0, st,
+                       (const raw*)x, lay, (const raw*)colmean, out, L, D, BLK, nblk, tiled);
+  else
+    hipLaunchKernelGGL((pool_kernel<IO, MODE, IO::VEC>), dim3(cdiv(nblk, 256 / (D / IO::VEC)), BH), dim3(256), 0, st, (const raw*)x,
+                       lay, (const raw*)colmean, out, L, D, BLK, nblk, tiled);
 }
 
 // levels 2 and 3 of the K column mean from the chunk sums
@@ -808,10 +811,13 @@ static void block_map_pool(const void* q, const void* k, const RowLayout& lay, c
   typename IO::raw* colmean = (typename IO::raw*)m.colmean;
   if (first_pass) {
     // k chunk sums and q block means share one launch
-    const int bpw = 256 / (D / IO::VEC);
-    hipLaunchKernelGGL((pool_pair_kernel<IO>), dim3(cdiv(max(m.nchunk, m.M), bpw), BH, 2), dim3(256), 0, st,
-                       (const typename IO::raw*)k, m.chunk_sums, m.nchunk, (const typename IO::raw*)q, lay,
-                       (typename IO::raw*)m.pq, BLKQ, m.M, L, D, m.tiled);
+    typedef typename IO::raw raw;
+#define SLA_PAIR_CASE(W)                                                                                                     \
+  hipLaunchKernelGGL((pool_pair_kernel<IO, W>), dim3(cdiv(max(m.nchunk, m.M), 256 / (D / (W))), BH, 2), dim3(256), 0, st,   \
+                     (const raw*)k, m.chunk_sums, m.nchunk, (const raw*)q, lay, (raw*)m.pq, BLKQ, m.M, L, D, m.tiled)
+    if (narrow_pools(sizeof(raw) == 4 ? SLA_F32 : SLA_BF16, BH, L, D) && D / (IO::VEC / 4) <= 256) SLA_PAIR_CASE(IO::VEC / 4);
+    else SLA_PAIR_CASE(IO::VEC);
+#undef SLA_PAIR_CASE
   }
   launch_colmean_reduce<IO>(m.chunk_sums, m.group_sums, colmean, BH, L, D, st);
   launch_pool<IO, 2>(k, lay, colmean, m.pk, BH, L, D, BLKK, st, m.tiled);

@@ -157,6 +157,11 @@ static __device__ __forceinline__ void pool_pair_body(const typename IO::raw* __
     pool_body<IO, 1, W, 256, Cast>(q, lay, nullptr, pq, L, D, BLKQ, nblkq, tiled, bx, bh, cast);
 }
 
+// One thread per 4 bytes of a block's columns while the first pass of the wide form would not put a wave on every SIMD.
+static inline bool narrow_pools(int dtype, int BH, int L, int D) {
+  return (int64_t)BH * cdiv(L, KMEAN_CHUNK) * D * elem_bytes(dtype) / 16 < 1024 * 64;
+}
+
 // Column mean of K, levels 2 and 3 of the summation order: one workgroup of NT threads per (head, slab of COLMEAN_SLAB
 // columns), thread (gi, c) = (tid / COLMEAN_SLAB, tid % COLMEAN_SLAB) forms group sums gi, gi + NT / COLMEAN_SLAB, ...
 // of its column; the first COLMEAN_SLAB threads then add the groups in ascending order.  (Small workgroups: the

@@ -7,7 +7,7 @@
 //     states finished, block means of k | scores and selection | attention
 // (five launches; in eight of their own, and seven with 16-bit inputs, everything before the attention took 34 us for 2 heads x
 // 1024 x 64 in fp32, 57 for 8 x 4096 x 128: now 25 and 43.)
-// From 16 MiB per tensor on the state build (k, v only) runs on the caller's second stream beside the mask builder instead.
+// From 64 MiB per tensor on the state build (k, v only) runs on the caller's second stream beside the mask builder instead.
 #include "block_pool.h"
 #include "fwd_steps.h"
 #include "linear_state.h"
@@ -74,11 +74,6 @@ __global__ __launch_bounds__(512) void prefix_finish_kernel(const StateFinish jo
   pool_body<IO, 2, W, 512>(k, lay, (const typename IO::raw*)m.colmean, m.pk, L, D, 64, m.N, m.tiled, wg - first_pool - bh * per_head, bh);
 }
 
-// One thread per 4 bytes of a block's columns while the first pass of the wide form would not put a wave on every SIMD.
-static inline bool narrow_pools(int in_dtype, const MapParts& m, int BH, int D) {
-  return (int64_t)BH * m.nchunk * D * elem_bytes(in_dtype) / 16 < 1024 * 64;
-}
-
 template <typename IO, typename Cast>
 static void launch_prefix_pool(const void* q, const void* k, const void* v, const RowLayout& lay, const MapParts& m, int in_dtype,
                                int BLKQ, int BH, int L, int D, void* cast, hipStream_t st) {
@@ -88,7 +83,7 @@ static void launch_prefix_pool(const void* q, const void* k, const void* v, cons
 #define SLA_POOL_CASE(W)                                                                                                      \
   hipLaunchKernelGGL((prefix_pool_kernel<IO, W, Cast>), dim3(cdiv(max(m.nchunk, m.M), 256 / (D / (W))), BH, z), dim3(256), 0, st, \
                      (const raw*)q, (const raw*)k, (const raw*)v, lay, m, BLKQ, L, D, (uint16_t*)cast, n)
-  if (narrow_pools(in_dtype, m, BH, D)) SLA_POOL_CASE(IO::VEC / 4);
+  if (narrow_pools(in_dtype, BH, L, D)) SLA_POOL_CASE(IO::VEC / 4);
   else SLA_POOL_CASE(IO::VEC);
 #undef SLA_POOL_CASE
 }
@@ -111,7 +106,7 @@ static void launch_prefix_rest(const void* k, const RowLayout& lin, const void* 
     hipLaunchKernelGGL((prefix_finish_kernel<Tag, D, IO, W>), dim3(xcd_grid(job.total) + BH * per_head), dim3(512), 0, st, job, \
                        xcd_grid(job.total), (const raw*)k, lin, m, L, per_head);                                             \
   }
-  if (narrow_pools(in_dtype, m, BH, D)) SLA_FINISH_CASE(IO::VEC / 4)
+  if (narrow_pools(in_dtype, BH, L, D)) SLA_FINISH_CASE(IO::VEC / 4)
   else SLA_FINISH_CASE(IO::VEC)
 #undef SLA_FINISH_CASE
 }
@@ -177,7 +172,7 @@ extern "C" int sla_module_fwd(const void* q, const void* k, const void* v, const
     return attn_linear_run(qc, kc, vc, lin, lut, lut_elem_bytes, (const char*)states, bias, o_s, out, lout, lse, dtype, fmap, BH,
                            L, D, BLKQ, topk, qk_scale, st);
   };
-  const bool two = side && side != st && side_stream_pays(B, H, L, D, topk);
+  const bool two = side && side != st && side_stream_pays_fwd(B, H, L, D);
   if (!two) {
     if (mask_given) {
       if ((rc = linear_state_run(kc, vc, lin, weight, dtype, fmap, BH, L, D, (char*)states, parts, st))) return rc;

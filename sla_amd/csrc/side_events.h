@@ -14,18 +14,18 @@ struct SideEvents {
 std::mutex& side_events_mutex();
 int side_events_for_current_device(SideEvents** out);      // (with the lock held)
 
-// A call uses the second stream only from this size of one of q, k, v on, or from this many operations of one product over the
-// selected tiles on (few heads with long sequences, whose short kernels are few workgroups with long chains).  Handing work to
-// it and back costs 25 us of host time in the forward, 30 in the quantised one and 80 in the backward, which the GPU has to
-// be busy for: the line is where the pass on one stream takes as long as the host needs to enqueue it on two.
-// Measured, two streams against one, over 2 to 40 heads, both head dims, 4 to 64 MiB (forward + backward in us):
-//   by size, rows of 64 values: 24 heads x 4096 (12 MiB) 314 / 202, x 5461 (16 MiB) 320 / 269, x 8192 (24 MiB) 329 / 337;
-//     40 heads x 2457 329 / 243, x 3276 337 / 330, x 6553 398 / 424; rows of 128: 8 heads x 6144 (12 MiB) 296 / 206, x 8192
-//     294 / 245, x 12288 337 / 352; 40 heads x 1228 246 / 223, x 1638 (16 MiB) 248 / 271; 24 heads x 2730 274 / 294.  The forward
-//     and the quantised forward gain 2 to 11 % from 16 MiB on (24 heads x 5461 x 64: 72 / 76 and 100.6 / 101.4).
-//   by operations, below 16 MiB: 2 heads x 40000 x 64, 62 blocks per row (41 GFLOP) 633 / 722, forward 171 / 180, quantised 191 /
-//     198; 16 heads x 4096 x 64, 32 blocks (17 GFLOP) 301 / 302, 86 / 89, 90 / 95; 4 heads x 16000 x 64, 25 blocks (13 GFLOP) 288 /
-//     317, 85 / 89, 109 / 99; 24 heads x 2700 x 64, 21 blocks (11 GFLOP) 342 / 302, 87 / 89, 98 / 107.
+// The module's forward uses the second stream from this size of one of q, k, v on.  Handing work to it and back costs 15 to 40 us
+// where a call is waited for, and on one stream the independent launches are merged anyway.  Measured, two streams / one, us per
+// call among others (and waited for): 12 heads x 6500 x 128 (19 MiB) 103 / 103 (137 / 124), 40 x 6500 x 64 (32 MiB) 122 / 126 (156 / 147),
+// 12 x 16000 x 128 (47 MiB) 265 / 263 (302 / 286), 8 x 32000 x 128 (63 MiB) 548 / 546 (581 / 566), 2 x 75600 x 128 (37 MiB) 751 / 760
+// (800 / 782); 12 x 32760 x 128 (96 MiB) 484 / 500.
+constexpr int64_t SIDE_MIN_BYTES_FWD = 64ll << 20;
+static inline bool side_stream_pays_fwd(int B, int H, int L, int D) { return (int64_t)B * H * L * D * 2 >= SIDE_MIN_BYTES_FWD; }
+
+// The quantised forward, whose preparation is mostly passes over memory, from this size on, or from this many operations of one
+// product over the selected tiles on (few heads with long sequences).  Two / one: 12 heads x 6500 x 128 (19 MiB) 122 / 128 (164 /
+// 157), 24 x 6500 x 64 106 / 104 (153 / 135), 16 x 8000 x 128 (31 MiB) 155 / 154 (196 / 184), 40 x 6500 x 64 (32 MiB) 145 / 161 (192 /
+// 191), 12 x 16000 x 128 257 / 282, 4 x 40000 x 128 359 / 390.
 constexpr int64_t SIDE_MIN_BYTES = 16ll << 20;
 constexpr int64_t SIDE_MIN_OPS = 16000000000ll;
 static inline bool side_stream_pays(int B, int H, int L, int D, int topk) {
