@@ -11,252 +11,278 @@
 //
 // Kernels:
 //   block states : linear_state_partial_kernel with one 64-row slice per workgroup, 16-bit h_j^T, fp32 z_j
-//   totals       : sum_j h_j, sum_j z_j in fp32 (groups of 16 blocks, then the groups)
-//   gather       : H_i, z_i = totals - the T selected states, per query block (H_i rounded); the backward reads them again
+//   weights      : one row of bits per query block, set for the key blocks its look-up row does not name
+//   states       : H_i, z_i = weights times block states, per query block (H_i rounded); the backward reads them again
 //   out          : N^T = H_i^T phi(Q)^T, OUT^T = W Y^T for the rows of a query block in the transposed
 //                  formulation of the global output kernel.
-// At 12 heads of 16380 rows, head dim 128, 12 of 256 blocks selected, with the gathers inside the kernels of the rows (a
+// At 12 heads of 16380 rows, head dim 128, 12 of 256 blocks selected, with the states formed inside the kernels of the rows (a
 // workgroup per query or key block, the whole state in 64 fp32 registers per thread, two waves per SIMD): out 236 us,
-// rows 171 us, kv 171 us, and the backward formed the forward's states again (88 us).  With the
-// gathers in a kernel of their own: gather 101 us (twice), out 77 us, rows 110 us, kv 112 us.
+// rows 171 us, kv 171 us.  With the states in a kernel of their own: out 77 us, rows 110 us, kv 112 us.
 #include "linear_state.h"
 
 namespace sla {
 
 int validate_attn_shape(int dtype, int B, int H, int L, int D, int BLKQ, int BLKK, int topk, int lut_elem_bytes);
-void launch_col_lists(const int8_t* sparse_map, int* list, int* count, int BH, int Mblk, int Nblk, hipStream_t st);
 int64_t weight_grads_workspace_bytes(int BH, int L, int D);
 void launch_weight_grads(int dtype, int D, const void* q, const void* dn, const void* gout, const void* y, const float* dden,
                          int BH, int L, int fmap, char* ws, float* d_weight, float* d_bias, hipStream_t st);
 
-// Totals in two fixed-order levels: groups of TOTAL_GROUP consecutive key blocks, then the groups in order.
-// level 1: grid (cdiv(D*D/8, 256), ngroup, BH), thread owns 8 adjacent elements of one group's D x D sum;
-// level 2: grid (cdiv(D*D, 256), BH), thread owns one element.
-constexpr int TOTAL_GROUP = 16;
+// Weights of the states: one bit per row and block state, 1 where the state takes part; zero from the table's end on.
+// all[head][row] says that the row leaves every block out.  A lane of the matrix instruction holds one row and eight of sixteen
+// columns; a word is what it needs of 64 columns, the even ones' bits in the lower half and the odd ones' in the upper, so that
+// a shift and a mask leave the operand's pairs with the pattern of 2.0 (one bit in either 16-bit format, and in fp32) where the
+// bit is set.  Words of a head: [32 rows][64 columns][lane].
+constexpr int WEIGHT_STEP = 64;
+static inline int64_t weight_words(int nrows, int nblk) { return (int64_t)cdiv(nrows, 32) * cdiv(nblk, WEIGHT_STEP) * 64; }
+static __device__ __forceinline__ int weight_bit(int c) { return (c >> 2 & 12) + (c >> 1 & 3) + 16 * (c & 1); }
 
-template <typename Tag>
-__global__ __launch_bounds__(256) void complement_group_kernel(const uint16_t* __restrict__ hblk,
-                                                               const float* __restrict__ zblk, float* __restrict__ hgrp,
-                                                               float* __restrict__ zgrp, int N, int D) {
-  using E = Elem<Tag>;
-  const int DD = D * D;
-  const int grp = blockIdx.y, ngroup = gridDim.y, bh = blockIdx.z;
-  const int j0 = grp * TOTAL_GROUP, j1 = min(N, j0 + TOTAL_GROUP);
-  const int i = (blockIdx.x * 256 + threadIdx.x) * 8;
-  if (i < DD) {
-    float acc[8];
+// Rows of a look-up table (query blocks): the blocks the row does not name.  grid (nrows, heads).
+__global__ __launch_bounds__(64) void complement_row_weights_kernel(const void* __restrict__ lut, int lut64, int topk,
+                                                                    uint32_t* __restrict__ w, int* __restrict__ all, int nblk) {
+  constexpr int SPAN = 1024;             // words at a time (32768 blocks)
+  __shared__ uint32_t word[SPAN];
+  const int row = blockIdx.x, nrows = gridDim.x, steps = (nblk + WEIGHT_STEP - 1) / WEIGHT_STEP, tid = threadIdx.x;
+  const size_t at = (size_t)blockIdx.y * nrows + row;
+  w += ((size_t)blockIdx.y * ((nrows + 31) >> 5) + (row >> 5)) * steps * 64;
+  for (int w0 = 0; w0 < 2 * steps; w0 += SPAN) {
+    const int span = min(SPAN, 2 * steps - w0);
+    for (int i = tid; i < span; i += 64) {
+      const int c0 = ((w0 + i) >> 1) * WEIGHT_STEP + 8 * (i & 1);
+      uint32_t x = 0;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) acc[e] = 0.f;
-    const uint16_t* p = hblk + (size_t)bh * N * DD + i;
-#pragma unroll 8
-    for (int j = j0; j < j1; ++j) {
-      const i16x8_t x = *reinterpret_cast<const i16x8_t*>(p + (size_t)j * DD);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) acc[e] += E::to_float((uint16_t)x[e]);
+      for (int e = 0; e < 32; ++e) {
+        const int c = 16 * (e >> 3) + (e & 7);
+        x |= c0 + c < nblk ? 1u << weight_bit(c) : 0u;
+      }
+      word[i] = x;
     }
-    float* o = hgrp + ((size_t)bh * ngroup + grp) * DD + i;
-    *reinterpret_cast<f32x4_t*>(o) = f32x4_t{acc[0], acc[1], acc[2], acc[3]};
-    *reinterpret_cast<f32x4_t*>(o + 4) = f32x4_t{acc[4], acc[5], acc[6], acc[7]};
+    __syncthreads();
+    for (int t = tid; t < topk; t += 64) {
+      const int j = lut64 ? (int)reinterpret_cast<const long long*>(lut)[at * topk + t] : reinterpret_cast<const int*>(lut)[at * topk + t];
+      const int i = (j >> 6) * 2 + (j >> 3 & 1) - w0;
+      if (j >= 0 && i >= 0 && i < span) atomicAnd(&word[i], ~(1u << weight_bit(j & 63)));
+    }
+    __syncthreads();
+    for (int i = tid; i < span; i += 64) w[(w0 + i) * 32 + (row & 31)] = word[i];
+    __syncthreads();
   }
-  const int d = blockIdx.x * 256 + threadIdx.x;
-  if (d < D) {
-    float s = 0.f;
-    for (int j = j0; j < j1; ++j) s += zblk[((size_t)bh * N + j) * D + d];
-    zgrp[((size_t)bh * ngroup + grp) * D + d] = s;
-  }
+  if (tid == 0) all[at] = topk >= nblk;
 }
 
-__global__ __launch_bounds__(256) void complement_total_kernel(const float* __restrict__ hgrp, const float* __restrict__ zgrp,
-                                                               float* __restrict__ hall, float* __restrict__ zall, int ngroup,
-                                                               int D) {
-  const int DD = D * D;
-  const int bh = blockIdx.y;
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i < DD) {
-    float s = 0.f;
-#pragma unroll 4
-    for (int gi = 0; gi < ngroup; ++gi) s += hgrp[((size_t)bh * ngroup + gi) * DD + i];
-    hall[(size_t)bh * DD + i] = s;
+// Columns of the map (key blocks): the query blocks that did not select it.  grid (cdiv(Nblk, 64), heads), a lane per key block,
+// a word per wave and pass.
+__global__ __launch_bounds__(512) void complement_column_weights_kernel(const int8_t* __restrict__ map, uint32_t* __restrict__ w,
+                                                                        int* __restrict__ all, int Mblk, int Nblk) {
+  __shared__ uint32_t any[64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n = blockIdx.x * 64 + lane;
+  const int steps = (Mblk + WEIGHT_STEP - 1) / WEIGHT_STEP;
+  const size_t bh = blockIdx.y;
+  if (wave == 0) any[lane] = 0;
+  __syncthreads();
+  if (n < Nblk) {
+    const int8_t* const col = map + bh * Mblk * Nblk + n;
+    w += (bh * ((Nblk + 31) >> 5) + (n >> 5)) * steps * 64;
+    uint32_t seen = 0;
+    for (int i = wave; i < 2 * steps; i += 8) {
+      const int m0 = (i >> 1) * WEIGHT_STEP + 8 * (i & 1);
+      int8_t sel[32];
+#pragma unroll
+      for (int e = 0; e < 32; ++e) sel[e] = col[(size_t)min(m0 + 16 * (e >> 3) + (e & 7), Mblk - 1) * Nblk];
+      uint32_t x = 0;
+#pragma unroll
+      for (int e = 0; e < 32; ++e) {
+        const int c = 16 * (e >> 3) + (e & 7);
+        x |= m0 + c < Mblk && sel[e] != 1 ? 1u << weight_bit(c) : 0u;
+      }
+      w[i * 32 + (n & 31)] = x;
+      seen |= x;
+    }
+    if (seen) atomicOr(&any[lane], 1u);
   }
-  if (i < D) {
-    float s = 0.f;
-    for (int gi = 0; gi < ngroup; ++gi) s += zgrp[((size_t)bh * ngroup + gi) * D + i];
-    zall[(size_t)bh * D + i] = s;
-  }
+  __syncthreads();
+  if (wave == 0 && n < Nblk) all[bh * Nblk + n] = any[lane] == 0;
 }
 
-// Rows' states: `total - sum of the listed block states` for every query block (its look-up row) or, in the backward, for
-// every key block (the query blocks that selected it); 16-bit result, z in fp32.
+// Rows' states, states[r] = the sum of the block states whose bit is set in row r (16-bit result), z in fp32: for every query
+// block in the forward, for every key block in the backward.
 //
-// Bound by the traffic of the listed states (32 KB each at D = 128; a head's do not fit an XCD's L2).  Neighbouring lists
-// share many entries (6.8 of 12 between two rows at 12 heads x 16380 rows), so a workgroup takes GATHER_ROWS consecutive rows
-// at once: it walks the union of their lists and applies every block's state to all the rows that name it.  It holds a slice
-// of 4 KB of the state, 8 values per row and thread.  Applying the difference of a row's list against the previous one's
-// instead (one state in registers, 10.2 of 12 loads per row left) took 124 us there,
-// the union takes 101.
-// Every row's sum runs in the order of the union (the first row's list, what the second adds to it, ...).  Lists longer than
-// GATHER_TMAX are walked by themselves.  A list that names every block gives exactly zero by definition, not the rounding
-// residue of two fp32 sums formed in different orders, which the 1e-5 of the divisor would turn into an arbitrary result.
-constexpr int GATHER_ROWS = 8;
-constexpr int GATHER_TMAX = 256;
-
-// list: row (head, r) starts `stride` entries after the previous one and has count[r] entries (`fixed` where count is null).
-// 1-D grid over (head, slice, group of rows), 256 threads; thread t owns 16-byte chunk t of its slice.
+// A matrix product of the weights (nrows x nblk) with the block states (nblk x D*D) on the matrix cores, whose products are
+// exact (weights 0 and 2, the sum halved at the end), accumulated in fp32.  Bound by memory up to some 400 blocks (every block
+// state is read once and every state written once: 2 x 32 KB per row at D = 128), by the matrix cores above.  A workgroup of
+// four waves takes 128 rows x 256 values, a wave 128 x 64 as eight 32 x 32 accumulators (parts of 32 rows that the head does
+// not have are left out): eight products for every four transposed LDS reads.  Tiles of 64 blocks go through registers, two tiles ahead, into one of two LDS buffers.  Even and odd values of a
+// row are parked apart, so that a lane's two column tiles hold neighbouring values and 32 lanes store whole 128-byte lines.
+// z: workgroups of their own (the first ones of a head), 128 rows x 32 values, fp32 matrix products.
+// Against `total - sum of the listed states` on the vector ALU, the union of eight rows' lists at a time, and its totals in two
+// launches: 12 heads x 16380 x 128, 12 of 256 blocks selected 70 us where that took 101 + 23 + 8; forward and backward of 12 heads
+// x 75600 x 128 with 5 % selected 12.2 ms (15.5), 10.7 (11.8) where neighbouring rows select alike, 6.6 (6.8) with 2 %; 8 heads x
+// 4096 x 128 with 20 % 309 us (382).  64 x 64 values per wave: the same up to 256 blocks, 7.0 ms for the one with 2 %.
+// A row that leaves every block out is exactly zero, whatever the block states hold.
 template <typename Tag, int D>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void complement_gather_kernel(
-    const uint16_t* __restrict__ blocks, const float* __restrict__ zblocks, const float* __restrict__ total,
-    const float* __restrict__ ztotal, const void* __restrict__ list, int list64, const int* __restrict__ count, int fixed,
-    int stride, uint16_t* __restrict__ states, float* __restrict__ zstates, int nrows, int nblk, int ntotal) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void complement_states_kernel(
+    const uint16_t* __restrict__ blocks, const float* __restrict__ zblocks, const uint32_t* __restrict__ w,
+    const int* __restrict__ all, uint16_t* __restrict__ states, float* __restrict__ zstates, int nrows, int nblk, int ntotal) {
   using E = Elem<Tag>;
   constexpr int DD = D * D;
-  constexpr int SLICES = DD / 2048;
-  constexpr int R = GATHER_ROWS;
-  constexpr int BATCH = 8;               // listed states in flight
-  constexpr int CHUNKS = GATHER_TMAX / 64;
-  static_assert(DD % 2048 == 0, "slices of 2048 values");
-  static_assert(R == 8, "a wave builds the union's share of two rows");
-  __shared__ int sRow[R][GATHER_TMAX];
-  __shared__ uint32_t sUnion[R * GATHER_TMAX];       // block in the lower 24 bits, the rows that name it above
-  __shared__ int sCnt[R * CHUNKS];
+  constexpr int BM = 128, BN = 256, KS = WEIGHT_STEP, MI = BM / 32;
+  constexpr int CPR = BN / 8, NP = KS * CPR / 256;   // 16-byte pieces of a row; pieces per thread and tile
+  constexpr int STR = BN + 16;                       // transposed reads of 4 rows hit disjoint banks
+  constexpr int ZT = D / 32, CT = DD / BN;
+  __shared__ __attribute__((aligned(16))) uint16_t sB[2][KS * STR];
+  __shared__ int sAll[BM];
   const int logical = xcd_remap(blockIdx.x, gridDim.x, ntotal);
   if (logical < 0) return;
-  const int groups = (nrows + R - 1) / R;
-  const int unit = logical / groups, row0 = (logical - unit * groups) * R;
-  const int bh = unit / SLICES, slice = unit - bh * SLICES;
+  const int rtiles = (nrows + BM - 1) / BM, per_head = (ZT + CT) * rtiles;
+  const int bh = logical / per_head, rest = logical - bh * per_head;
+  const int ct = rest / rtiles, row0 = (rest - ct * rtiles) * BM;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const bool has_z = slice == 0 && tid < D;
-  const size_t off = (size_t)slice * 2048 + tid * 8;
-  const uint16_t* hb = blocks + (size_t)bh * nblk * DD + off;
-  const float* zb = zblocks + (size_t)bh * nblk * D + (has_z ? tid : 0);
-  auto entry = [&](int row, int i) -> int {
-    const size_t at = ((size_t)bh * nrows + row) * stride + i;
-    return list64 ? (int)reinterpret_cast<const long long*>(list)[at] : reinterpret_cast<const int*>(list)[at];
-  };
-
-  int cnt[R];                            // (uniform over the workgroup)
-#pragma unroll
-  for (int s = 0; s < R; ++s) {
-    cnt[s] = row0 + s < nrows ? __builtin_amdgcn_readfirstlane(count ? count[(size_t)bh * nrows + row0 + s] : fixed) : 0;
-    if (cnt[s] <= GATHER_TMAX && cnt[s] < nblk && tid < cnt[s]) sRow[s][tid] = entry(row0 + s, tid);
-  }
-  auto listed = [&](int s) { return cnt[s] <= GATHER_TMAX && cnt[s] < nblk ? cnt[s] : 0; };     // entries in LDS
+  const int g = lane >> 5, r = lane & 31;
+  const int steps = (nblk + KS - 1) / KS;
+  const uint32_t* const wb = w + (size_t)bh * ((nrows + 31) >> 5) * steps * 64 + lane;
+  if (tid < BM) sAll[tid] = all[(size_t)bh * nrows + min(row0 + tid, nrows - 1)];
   __syncthreads();
-  // the union: wave w finds which entries of rows w and w + 4 no earlier row names, and who else names them
-  uint32_t word[2][CHUNKS];
+
+  if (ct < ZT) {
+    // ---- z: rows row0 + 32 wave .., values 32 ct .. ----
+    const int base = row0 + 32 * wave;
+    if (base >= nrows) return;
+    const uint32_t* wr = wb + (size_t)(base >> 5) * steps * 64;
+    const float* zb = zblocks + (size_t)bh * nblk * D;
+    f32x16_t acc;
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int s = wave + 4 * h;
-    int mine = 0;
+    for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+    uint32_t a[2];
+    float z[2][32];
+    // (lane group g holds blocks 16 c + 8 g + u of a step)
+    const auto fetch = [&](int st, int s) __attribute__((always_inline)) {
+      const __amdgpu_buffer_rsrc_t rs = make_rsrc(zb + (size_t)st * KS * D, (uint32_t)min(nblk - st * KS, KS) * D * 4u);
+      a[s] = wr[st * 64];
 #pragma unroll
-    for (int x = 0; x < R; ++x) mine = x == s ? listed(x) : mine;
+      for (int u = 0; u < 32; ++u)
+        z[s][u] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+            rs, (int)(((16 * (u >> 3) + 8 * g + (u & 7)) * D + 32 * ct + r) * 4), 0, 0));
+    };
+    fetch(0, 0);
+    for (int s0 = 0; s0 < steps; s0 += 2)
 #pragma unroll
-    for (int c = 0; c < CHUNKS; ++c) {
-      word[h][c] = 0;
-      if (c * 64 < mine) {
-        const bool has = c * 64 + lane < mine;
-        const int j = has ? sRow[s][c * 64 + lane] : -1;
-        uint32_t rows = has ? 1u << s : 0u;
+      for (int s = 0; s < 2; ++s) {
+        if (s0 + s >= steps) break;
+        if (s0 + s + 1 < steps) fetch(s0 + s + 1, s ^ 1);
 #pragma unroll
-        for (int x = 0; x < R; ++x) {
-          bool hit = false;
-          if (x != s)
-            for (int u = 0, n = listed(x); u < n; ++u) hit |= sRow[x][u] == j;
-          rows |= hit ? 1u << x : 0u;
+        for (int u = 0; u < 32; ++u) {
+          const int bit = (u >> 1) + 16 * (u & 1);             // (u = 8 c + e: weight_bit(16 c + e))
+          const float x = __uint_as_float((bit <= 30 ? a[s] << (30 - bit) : a[s] >> 1) & 0x40000000u);
+          acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x, z[s][u], acc, 0, 0, 0);
         }
-        if (has && (rows & ((1u << s) - 1)) == 0) word[h][c] = (uint32_t)j | rows << 24;
       }
-      const unsigned long long m = __ballot(word[h][c] != 0);
-      if (lane == 0) sCnt[s * CHUNKS + c] = __popcll(m);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int row = 8 * (i >> 2) + 4 * g + (i & 3);
+      if (base + row < nrows)
+        zstates[((size_t)bh * nrows + base + row) * D + 32 * ct + r] = sAll[32 * wave + row] ? 0.f : 0.5f * acc[i];
     }
+    return;
   }
-  __syncthreads();
-  int n = 0;
-  {
-    int before[2][CHUNKS];
-    for (int i = 0; i < R * CHUNKS; ++i) {
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int c = 0; c < CHUNKS; ++c)
-          if (i == (wave + 4 * h) * CHUNKS + c) before[h][c] = n;
-      n += sCnt[i];
-    }
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-      for (int c = 0; c < CHUNKS; ++c) {
-        const unsigned long long m = __ballot(word[h][c] != 0);
-        if (word[h][c] != 0) sUnion[before[h][c] + __popcll(m & ((1ull << lane) - 1))] = word[h][c];
-      }
-    n = __builtin_amdgcn_readfirstlane(n);
-  }
-  __syncthreads();
 
-  float acc[R][8], zacc[R];
-  {
-    const float* tot = total + (size_t)bh * DD + off;
-    const f32x4_t a = *reinterpret_cast<const f32x4_t*>(tot), b = *reinterpret_cast<const f32x4_t*>(tot + 4);
-    const float z = has_z ? ztotal[(size_t)bh * D + tid] : 0.f;
+  const int col0 = (ct - ZT) * BN;
+  const int tr_row = (lane & 15) >> 2, tr_col = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+  const int brow = tid / CPR, bch = tid % CPR;       // this thread's piece of rows brow + 256 / CPR p
+  const uint16_t* const hb = blocks + (size_t)bh * nblk * DD + col0;
+  const int mine = min(MI, (nrows - row0 + 31) / 32);            // 32-row parts with rows
+  const uint32_t* wp[MI];                             // (a part without rows reads the last one with rows, to no end)
 #pragma unroll
-    for (int s = 0; s < R; ++s) {
-      zacc[s] = z;
+  for (int m = 0; m < MI; ++m) wp[m] = wb + (size_t)(min(row0 + 32 * m, nrows - 1) >> 5) * steps * 64;
+
+  f32x16_t acc[MI][2];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        acc[s][e] = a[e];
-        acc[s][4 + e] = b[e];
+  for (int m = 0; m < MI; ++m)
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[m][t][i] = 0.f;
+  i16x8_t breg[2][NP];
+  uint32_t areg[2][MI];
+  const auto fetch_b = [&](int k0, int s) __attribute__((always_inline)) {
+    const int rows = min(KS, nblk - k0);             // (rows past the last block read as zero)
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc(hb + (size_t)k0 * DD, rows > 0 ? ((uint32_t)(rows - 1) * DD + BN) * 2u : 0u);
+#pragma unroll
+    for (int p = 0; p < NP; ++p) breg[s][p] = buf_load_b128(rs, ((uint32_t)(brow + 256 / CPR * p) * DD + 8u * (uint32_t)bch) * 2u);
+  };
+  const auto park_b = [&](int s) __attribute__((always_inline)) {
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+      const i32x4_t x = __builtin_bit_cast(i32x4_t, breg[s][p]);
+      i32x2_t even, odd;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        even[h] = (int)__builtin_amdgcn_perm((uint32_t)x[2 * h + 1], (uint32_t)x[2 * h], 0x05040100u);
+        odd[h] = (int)__builtin_amdgcn_perm((uint32_t)x[2 * h + 1], (uint32_t)x[2 * h], 0x07060302u);
       }
-    }
-  }
-  // subtracts the blocks of words at(0 .. n-1) from the rows they name
-  auto walk = [&](int n, auto at) {
-    for (int i0 = 0; i0 < n; i0 += BATCH) {
-      i16x8_t x[BATCH];
-      float zx[BATCH];
-      uint32_t rows[BATCH];
-#pragma unroll
-      for (int u = 0; u < BATCH; ++u) {
-        rows[u] = 0;
-        if (i0 + u >= n) continue;
-        const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane((int)at(i0 + u));
-        const uint32_t j = w & 0xffffffu;
-        rows[u] = w >> 24;
-        x[u] = *reinterpret_cast<const i16x8_t*>(hb + (size_t)j * DD);
-        zx[u] = has_z ? zb[(size_t)j * D] : 0.f;
-      }
-#pragma unroll
-      for (int u = 0; u < BATCH; ++u) {
-        if (i0 + u >= n) continue;
-        float f[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) f[e] = E::to_float((uint16_t)x[u][e]);
-#pragma unroll
-        for (int s = 0; s < R; ++s)
-          if (rows[u] >> s & 1) {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) acc[s][e] -= f[e];
-            zacc[s] -= zx[u];
-          }
-      }
+      uint16_t* at = &sB[s][(brow + 256 / CPR * p) * STR + 4 * bch];
+      *reinterpret_cast<i32x2_t*>(at) = even;
+      *reinterpret_cast<i32x2_t*>(at + BN / 2) = odd;
     }
   };
-  walk(n, [&](int i) { return sUnion[i]; });
-  for (int s = 0; s < R; ++s) {          // lists too long for the union, one at a time
-    int longer = 0;
+  const auto fetch_a = [&](int k0, int s) __attribute__((always_inline)) {
 #pragma unroll
-    for (int x = 0; x < R; ++x) longer = x == s && cnt[x] > GATHER_TMAX && cnt[x] < nblk ? cnt[x] : longer;
-    if (longer) walk(longer, [&](int i) { return (uint32_t)entry(row0 + s, i) | (1u << s) << 24; });
-  }
+    for (int m = 0; m < MI; ++m) areg[s][m] = wp[m][k0];
+  };
+  const auto operand = [](uint32_t x, int c) __attribute__((always_inline)) {
+    i32x4_t a;
 #pragma unroll
-  for (int s = 0; s < R; ++s) {
-    if (row0 + s >= nrows) break;
-    const bool all = cnt[s] >= nblk;
-    const size_t at_row = (size_t)bh * nrows + row0 + s;
-    i32x4_t w;
+    for (int i = 0; i < 4; ++i) {
+      const int d = 4 * c + i;
+      a[i] = (int)((d <= 14 ? x << (14 - d) : x >> 1) & 0x40004000u);
+    }
+    return __builtin_bit_cast(i16x8_t, a);
+  };
+  fetch_b(0, 0);
+  fetch_b(KS, 1);
+  fetch_a(0, 0);
+  park_b(0);
+  fetch_b(2 * KS, 0);
+  lds_barrier();
+  const auto step = [&](int k0, int s) __attribute__((always_inline)) {
+    if (k0 + KS < nblk) fetch_a(k0 + KS, s ^ 1);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) w[e] = all ? 0 : (int)E::pack2(acc[s][2 * e], acc[s][2 * e + 1]);
-    *reinterpret_cast<i32x4_t*>(states + at_row * DD + off) = w;
-    if (has_z) zstates[at_row * D + tid] = all ? 0.f : zacc[s];
-  }
+    for (int c = 0; c < 4; ++c) {
+      if (k0 + 16 * c >= nblk) break;
+      i16x8_t b[2];
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const uint16_t* p = &sB[s][(16 * c + 8 * g + tr_row) * STR + (BN / 2) * t + 32 * wave + tr_col];
+        b[t] = concat4(lds_read_tr16(p), lds_read_tr16(p + 4 * STR));
+      }
+#pragma unroll
+      for (int m = 0; m < MI; ++m)
+        if (m < mine) {
+          const i16x8_t a = operand(areg[s][m], c);
+#pragma unroll
+          for (int t = 0; t < 2; ++t) acc[m][t] = E::mfma32(a, b[t], acc[m][t]);
+        }
+    }
+    if (k0 + KS < nblk) {
+      park_b(s ^ 1);
+      fetch_b(k0 + 3 * KS, s ^ 1);
+      lds_barrier();
+    }
+  };
+  for (int k0 = 0; k0 < nblk; k0 += 2 * KS)
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+      if (s == 0 || k0 + KS < nblk) step(k0 + s * KS, s);
+
+#pragma unroll
+  for (int m = 0; m < MI; ++m)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int row = 32 * m + 8 * (i >> 2) + 4 * g + (i & 3);
+      if (row0 + row < nrows) {
+        uint32_t v = E::pack2(0.5f * acc[m][0][i], 0.5f * acc[m][1][i]);
+        if (sAll[row]) v = 0u;
+        *reinterpret_cast<uint32_t*>(states + ((size_t)bh * nrows + row0 + row) * DD + col0 + 64 * wave + 2 * r) = v;
+      }
+    }
 }
 
 // A row's state on its way from memory into an LDS matrix of D rows with row stride STR.
@@ -427,10 +453,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 //   dH_i = a_i^T dn_i (rows of query block i), dz_i = sum_rows dden a
 //   G_j = sum_{i : j not in S_i} dH_i = sum_i dH_i - sum_{i in C_j} dH_i  (C_j = query blocks that selected j), gz_j likewise
 //   dc = v G_j^T + gz_j ; dv = c G_j ; dk = phi'(k) dc                     (rows of key block j)
-// Kernels (the totals, the per-block products and dW / db reuse kernels of the forward and of the global backward):
+// Kernels (the per-block products and dW / db reuse kernels of the forward and of the global backward):
 //   rows   : one workgroup per query block: y, dy, dn, dden, da, dq for its rows from the forward's H_i, z_i on the MFMA in
 //            transposed form; writes dq and the row-wise temporaries dn, y (16 bit), dden
-//   gather : the forward's kernel: G_j, gz_j = total - listed dH_i, dz_i
+//   states : the forward's kernel, with the map's columns as weights: G_j, gz_j
 //   kv     : one workgroup per key block: dv, dc, dk for its 64 rows
 
 // 1-D grid over (head, query block), XCD-aware order, 256 threads; waves 0 .. BLKQ/32-1 own 32 query rows each.
@@ -752,8 +778,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
 // ---- host ---------------------------------------------------------------------------------
 struct ComplWs {
-  int ngroup;
-  size_t hblk, zblk, hgrp, zgrp, hall, zall, total;      // total: without the query blocks' states
+  size_t hblk, zblk, w, all, total;                      // total: without the query blocks' states
 };
 // The query blocks' states: what the backward reads of the forward.
 struct ComplStates {
@@ -774,80 +799,64 @@ static ComplWs compl_ws(int BH, int L, int D) {
   size_t off = 0;
   w.hblk = off; off += align_up((int64_t)BH * N * D * D * 2, 256);
   w.zblk = off; off += align_up((int64_t)BH * N * D * 4, 256);
-  w.ngroup = cdiv((int)N, TOTAL_GROUP);
-  w.hgrp = off; off += align_up((int64_t)BH * w.ngroup * D * D * 4, 256);
-  w.zgrp = off; off += align_up((int64_t)BH * w.ngroup * D * 4, 256);
-  w.hall = off; off += align_up((int64_t)BH * D * D * 4, 256);
-  w.zall = off; off += align_up((int64_t)BH * D * 4, 256);
+  // (weights of up to N rows over up to N blocks: the backward's take the place of the forward's)
+  w.w = off;    off += align_up(BH * weight_words((int)N, (int)N) * 4, 256);
+  w.all = off;  off += align_up((int64_t)BH * N * 4, 256);
   w.total = off;
   return w;
 }
 // A call that does not keep the query blocks' states (twice the bytes of q at 64-row blocks and head dim 128) forms them for a
-// few heads at a time: in the place of the groups' sums, which nobody reads any more (an eighth of the block states), or,
-// where those hold less, in up to CPL_STATES_AT_ONCE bytes of their own, so that short problems stay one launch.
-// 40 heads x 75600 x 128: 1.65 GiB of workspace (all at once 3.1), in 10 groups, inference 17.3 ms (16.5).  12 heads x 32760
-// x 128, in us: 64 MiB at once 1222, 128 MiB 1118, all (201 MiB) 1090; up to 12 heads x 16380 are one group.
+// few heads at a time, in up to CPL_STATES_AT_ONCE bytes, so that short problems stay one launch.
+// 40 heads x 75600 x 128: 1.57 GiB of workspace (all at once 3.0), in 14 groups.
 constexpr int64_t CPL_STATES_AT_ONCE = 128ll << 20;
 struct ComplGroups {
   int heads;             // per group
-  size_t at, extra;      // where the states lie; bytes they add behind `end`, the end of the rest of the workspace
+  size_t extra;          // bytes their states add behind the rest of the workspace
 };
-static ComplGroups compl_groups(int BH, int L, int D, int BLKQ, size_t end) {
-  const ComplWs w = compl_ws(BH, L, D);
-  const size_t sums = w.zgrp - w.hgrp, one = compl_states(1, L, D, BLKQ).total;
-  const size_t room = sums > (size_t)CPL_STATES_AT_ONCE ? sums : (size_t)CPL_STATES_AT_ONCE;
+static ComplGroups compl_groups(int BH, int L, int D, int BLKQ) {
+  const size_t room = (size_t)CPL_STATES_AT_ONCE, one = compl_states(1, L, D, BLKQ).total;
   ComplGroups g;
   g.heads = (int)(room / one < 1 ? 1 : room / one > (size_t)BH ? BH : room / one);
   g.heads = cdiv(BH, cdiv(BH, g.heads));                    // (even groups)
-  const size_t bytes = compl_states(g.heads, L, D, BLKQ).total;
-  g.extra = bytes <= sums ? 0 : bytes;
-  g.at = bytes <= sums ? w.hgrp : end;
+  g.extra = compl_states(g.heads, L, D, BLKQ).total;
   return g;
 }
 int64_t linear_complement_apart_bytes(int BH, int L, int D) { return (int64_t)compl_ws(BH, L, D).total; }
 int64_t linear_complement_workspace_bytes(int BH, int L, int D, int BLKQ) {
-  const size_t end = compl_ws(BH, L, D).total;
-  return (int64_t)(end + compl_groups(BH, L, D, BLKQ, end).extra);
+  return (int64_t)(compl_ws(BH, L, D).total + compl_groups(BH, L, D, BLKQ).extra);
 }
 
-// `total - listed` for nrows rows of every head (see complement_gather_kernel)
+// The states of nrows rows of every head from its nblk block states (see complement_states_kernel)
 template <typename Tag, int D>
-static void launch_gather(const uint16_t* blocks, const float* zblocks, const float* total, const float* ztotal, const void* list,
-                          int list64, const int* count, int fixed, int stride, uint16_t* states, float* zstates, int BH, int nrows,
-                          int nblk, hipStream_t st) {
-  const int units = BH * (D * D / 2048) * cdiv(nrows, GATHER_ROWS);
-  hipLaunchKernelGGL((complement_gather_kernel<Tag, D>), dim3(xcd_grid(units)), dim3(256), 0, st, blocks, zblocks, total, ztotal,
-                     list, list64, count, fixed, stride, states, zstates, nrows, nblk, units);
+static void launch_states(const uint16_t* blocks, const float* zblocks, const uint32_t* w, const int* all, uint16_t* states,
+                          float* zstates, int BH, int nrows, int nblk, hipStream_t st) {
+  const int units = BH * (D / 32 + D * D / 256) * cdiv(nrows, 128);
+  hipLaunchKernelGGL((complement_states_kernel<Tag, D>), dim3(xcd_grid(units)), dim3(256), 0, st, blocks, zblocks, w, all, states,
+                     zstates, nrows, nblk, units);
 }
 
-// Block states and their totals.
+// Block states.
 template <typename Tag, int D>
-static void complement_totals_run(const void* k, const void* v, int fmap, int BH, int L, char* ws, hipStream_t st) {
+static void complement_blocks_run(const void* k, const void* v, int fmap, int BH, int L, char* ws, hipStream_t st) {
   const ComplWs w = compl_ws(BH, L, D);
-  const int N = cdiv(L, 64);
-  uint16_t* hblk = (uint16_t*)(ws + w.hblk);
-  float* zblk = (float*)(ws + w.zblk);
-  float* hgrp = (float*)(ws + w.hgrp);
-  float* zgrp = (float*)(ws + w.zgrp);
-  hipLaunchKernelGGL((linear_state_partial_kernel<Tag, D, true>), dim3(N, BH), dim3(256), 0, st, (const uint16_t*)k,
-                     (const uint16_t*)v, contiguous_layout(BH, L, D), (void*)hblk, zblk, L, 64, fmap, (const float*)nullptr);
-  hipLaunchKernelGGL((complement_group_kernel<Tag>), dim3(cdiv(D * D / 8, 256), w.ngroup, BH), dim3(256), 0, st, hblk, zblk,
-                     hgrp, zgrp, N, D);
-  hipLaunchKernelGGL(complement_total_kernel, dim3(cdiv(D * D, 256), BH), dim3(256), 0, st, hgrp, zgrp, (float*)(ws + w.hall),
-                     (float*)(ws + w.zall), w.ngroup, D);
+  hipLaunchKernelGGL((linear_state_partial_kernel<Tag, D, true>), dim3(cdiv(L, 64), BH), dim3(256), 0, st, (const uint16_t*)k,
+                     (const uint16_t*)v, contiguous_layout(BH, L, D), (void*)(ws + w.hblk), (float*)(ws + w.zblk), L, 64, fmap,
+                     (const float*)nullptr);
 }
 
 // The query blocks' states of `heads` heads from head h0 on, laid out as compl_states(heads, ..) says.
 template <typename Tag, int D>
-static void complement_gather_run(const void* lut, int lut64, int BH, int L, int BLKQ, int topk, const char* ws, int h0, int heads,
+static void complement_states_run(const void* lut, int lut64, int BH, int L, int BLKQ, int topk, char* ws, int h0, int heads,
                                   char* states, hipStream_t st) {
   const ComplWs w = compl_ws(BH, L, D);
   const ComplStates s = compl_states(heads, L, D, BLKQ);
   const int N = cdiv(L, 64), M = cdiv(L, BLKQ);
   const size_t head = h0;
-  launch_gather<Tag, D>((const uint16_t*)(ws + w.hblk) + head * N * D * D, (const float*)(ws + w.zblk) + head * N * D,
-                        (const float*)(ws + w.hall) + head * D * D, (const float*)(ws + w.zall) + head * D,
-                        lut ? (const char*)lut + head * M * topk * (lut64 ? 8 : 4) : nullptr, lut64, nullptr, topk, topk,
+  uint32_t* const wt = (uint32_t*)(ws + w.w);
+  int* const all = (int*)(ws + w.all);
+  hipLaunchKernelGGL(complement_row_weights_kernel, dim3(M, heads), dim3(64), 0, st,
+                     lut ? (const char*)lut + head * M * topk * (lut64 ? 8 : 4) : nullptr, lut64, topk, wt, all, N);
+  launch_states<Tag, D>((const uint16_t*)(ws + w.hblk) + head * N * D * D, (const float*)(ws + w.zblk) + head * N * D, wt, all,
                         (uint16_t*)(states + s.h), (float*)(states + s.z), heads, M, N, st);
 }
 
@@ -857,15 +866,15 @@ static int complement_impl(const void* q, const void* k, const void* v, const vo
                            const float* bias, const void* residual, void* out, int fmap, int BH, int L, int topk, char* ws,
                            char* kept, hipStream_t st) {
   const int Mblk = cdiv(L, BLKQ);
-  complement_totals_run<Tag, D>(k, v, fmap, BH, L, ws, st);
-  const ComplGroups g = compl_groups(BH, L, D, BLKQ, compl_ws(BH, L, D).total);
+  complement_blocks_run<Tag, D>(k, v, fmap, BH, L, ws, st);
+  const ComplGroups g = compl_groups(BH, L, D, BLKQ);
   const int step = kept ? BH : g.heads;
-  char* const states = kept ? kept : ws + g.at;
+  char* const states = kept ? kept : ws + compl_ws(BH, L, D).total;
   for (int h0 = 0; h0 < BH; h0 += step) {
     const int heads = BH - h0 < step ? BH - h0 : step;
     const ComplStates s = compl_states(heads, L, D, BLKQ);
     const size_t rows = (size_t)h0 * L * D;
-    complement_gather_run<Tag, D>(lut, lut64, BH, L, BLKQ, topk, ws, h0, heads, states, st);
+    complement_states_run<Tag, D>(lut, lut64, BH, L, BLKQ, topk, ws, h0, heads, states, st);
     const int total = heads * cdiv(Mblk, OUT_RUN);
     hipLaunchKernelGGL((complement_out_kernel<Tag, D, BLKQ>), dim3(xcd_grid(total)), dim3(256), 0, st, (const uint16_t*)q + rows,
                        (const uint16_t*)(states + s.h), (const float*)(states + s.z), weight, bias,
@@ -877,14 +886,12 @@ static int complement_impl(const void* q, const void* k, const void* v, const vo
 // ---- backward, host -------------------------------------------------------------------------
 struct ComplBwdWs {
   ComplWs fwd;
-  int ngroup_q;
-  size_t wt, dn, y, dden, dhblk, dzblk, dgrp, dzgrp, gall, gzall, wg, count, list, total;
+  size_t wt, dn, y, dden, dhblk, dzblk, wg, total;
 };
 static ComplBwdWs compl_bwd_ws(int BH, int L, int D, int BLKQ) {
-  const int64_t N = cdiv(L, 64), M = cdiv(L, BLKQ);
+  const int64_t M = cdiv(L, BLKQ);
   ComplBwdWs w;
   w.fwd = compl_ws(BH, L, D);
-  w.ngroup_q = cdiv((int)M, TOTAL_GROUP);
   size_t off = w.fwd.total;
   w.wt = off;    off += align_up((int64_t)D * D * 2, 256);
   w.dn = off;    off += align_up((int64_t)BH * L * D * 2, 256);
@@ -892,20 +899,13 @@ static ComplBwdWs compl_bwd_ws(int BH, int L, int D, int BLKQ) {
   w.dden = off;  off += align_up((int64_t)BH * L * 4, 256);
   w.dhblk = off; off += align_up((int64_t)BH * M * D * D * 2, 256);
   w.dzblk = off; off += align_up((int64_t)BH * M * D * 4, 256);
-  w.dgrp = off;  off += align_up((int64_t)BH * w.ngroup_q * D * D * 4, 256);
-  w.dzgrp = off; off += align_up((int64_t)BH * w.ngroup_q * D * 4, 256);
-  w.gall = off;  off += align_up((int64_t)BH * D * D * 4, 256);
-  w.gzall = off; off += align_up((int64_t)BH * D * 4, 256);
   w.wg = off;    off += align_up(weight_grads_workspace_bytes(BH, L, D), 256);
-  w.count = off; off += align_up((int64_t)BH * N * 4, 256);
-  w.list = off;  off += align_up((int64_t)BH * N * M * 4, 256);
   w.total = off;
   return w;
 }
 int64_t linear_complement_bwd_apart_bytes(int BH, int L, int D, int BLKQ) { return (int64_t)compl_bwd_ws(BH, L, D, BLKQ).total; }
 int64_t linear_complement_bwd_workspace_bytes(int BH, int L, int D, int BLKQ) {
-  const size_t end = compl_bwd_ws(BH, L, D, BLKQ).total;
-  return (int64_t)(end + compl_groups(BH, L, D, BLKQ, end).extra);
+  return (int64_t)(compl_bwd_ws(BH, L, D, BLKQ).total + compl_groups(BH, L, D, BLKQ).extra);
 }
 
 template <typename Tag, int D, int BLKQ>
@@ -925,40 +925,33 @@ static int complement_bwd_impl(const void* q, const void* k, const void* v, cons
   float* dden = (float*)(ws + w.dden);
   uint16_t* dhblk = (uint16_t*)(ws + w.dhblk);
   float* dzblk = (float*)(ws + w.dzblk);
-  float* gall = (float*)(ws + w.gall);
-  float* gzall = (float*)(ws + w.gzall);
-  int* count = (int*)(ws + w.count);
-  int* list = (int*)(ws + w.list);
   hipLaunchKernelGGL((linear_prep_weight_kernel<Tag>), dim3(cdiv(D * D, 256)), dim3(256), 0, st, weight, wt, D);
-  launch_col_lists(sparse_map, list, count, BH, Mblk, N, st);
   // rows: dq and the row temporaries (with the forward's states, kept or formed again)
-  if (!kept) complement_totals_run<Tag, D>(k, v, fmap, BH, L, ws, st);
-  const ComplGroups g = compl_groups(BH, L, D, BLKQ, w.total);
+  if (!kept) complement_blocks_run<Tag, D>(k, v, fmap, BH, L, ws, st);
+  const ComplGroups g = compl_groups(BH, L, D, BLKQ);
   const int step = kept ? BH : g.heads;
   for (int h0 = 0; h0 < BH; h0 += step) {
     const int heads = BH - h0 < step ? BH - h0 : step;
     const ComplStates s = compl_states(heads, L, D, BLKQ);
     const size_t rows = (size_t)h0 * L * D;
-    if (!kept) complement_gather_run<Tag, D>(lut, lut64, BH, L, BLKQ, topk, ws, h0, heads, ws + g.at, st);
-    const char* const states = kept ? kept : ws + g.at;
+    if (!kept) complement_states_run<Tag, D>(lut, lut64, BH, L, BLKQ, topk, ws, h0, heads, ws + w.total, st);
+    const char* const states = kept ? kept : ws + w.total;
     const int total_q = heads * Mblk;
     hipLaunchKernelGGL((complement_bwd_rows_kernel<Tag, D, BLKQ>), dim3(xcd_grid(total_q)), dim3(256), 0, st,
                        (const uint16_t*)q + rows, (const uint16_t*)d_out + rows, (const uint16_t*)(states + s.h),
                        (const float*)(states + s.z), wt, (uint16_t*)dq + rows, dn + rows, y + rows, dden + (size_t)h0 * L, L, Mblk,
                        fmap, total_q, accumulate);
   }
-  // per query block dH_i^T = (a_i^T dn_i)^T and dz_i = sum dden a (the state kernel with q, dn in the place of k, v),
-  // then their totals
+  // per query block dH_i^T = (a_i^T dn_i)^T and dz_i = sum dden a (the state kernel with q, dn in the place of k, v)
   hipLaunchKernelGGL((linear_state_partial_kernel<Tag, D, true, true>), dim3(Mblk, BH), dim3(256), 0, st, (const uint16_t*)q,
                      (const uint16_t*)dn, lay, (void*)dhblk, dzblk, L, BLKQ, fmap, (const float*)dden);
-  hipLaunchKernelGGL((complement_group_kernel<Tag>), dim3(cdiv(D * D / 8, 256), w.ngroup_q, BH), dim3(256), 0, st, dhblk, dzblk,
-                     (float*)(ws + w.dgrp), (float*)(ws + w.dzgrp), Mblk, D);
-  hipLaunchKernelGGL(complement_total_kernel, dim3(cdiv(D * D, 256), BH), dim3(256), 0, st, (const float*)(ws + w.dgrp),
-                     (const float*)(ws + w.dzgrp), gall, gzall, w.ngroup_q, D);
   // dW, db
   launch_weight_grads(dtype, D, q, dn, d_out, y, dden, BH, L, fmap, ws + w.wg, d_weight, d_bias, st);
   // dk, dv
-  launch_gather<Tag, D>(dhblk, dzblk, gall, gzall, list, 0, count, 0, Mblk, gst, gzst, BH, N, Mblk, st);
+  uint32_t* const wk = (uint32_t*)(ws + w.fwd.w);
+  int* const all = (int*)(ws + w.fwd.all);
+  hipLaunchKernelGGL(complement_column_weights_kernel, dim3(cdiv(N, 64), BH), dim3(512), 0, st, sparse_map, wk, all, Mblk, N);
+  launch_states<Tag, D>(dhblk, dzblk, wk, all, gst, gzst, BH, N, Mblk, st);
   const int total_k = BH * N;
   hipLaunchKernelGGL((complement_bwd_kv_kernel<Tag, D>), dim3(xcd_grid(total_k)), dim3(256), 0, st, (const uint16_t*)k,
                      (const uint16_t*)v, gst, gzst, (uint16_t*)dk, (uint16_t*)dv, L, N, fmap, total_k, accumulate);

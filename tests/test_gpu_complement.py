@@ -226,3 +226,29 @@ def test_inference_does_not_keep_the_states(dev):
     tensors = 2 * q.numel() * 2 + H * L * 4 + (H * 512 * (512 + 10 * 8))          # attention output and result, lse, map, table
     assert used <= tensors + size(_lib.WS_LINEAR_COMPLEMENT) + (16 << 20), used
     assert size(_lib.WS_LINEAR_COMPLEMENT_STATES) > (128 << 20)
+
+
+@pytest.mark.parametrize("L,D,BLKQ,T", [
+    (129 * 64 - 3, 128, 64, 5),         # one row, and one step of 64 block states, past a tile of 128 rows
+    (128 * 64, 64, 64, 127), (65 * 64, 128, 128, 64),
+    (31 * 64 + 1, 64, 128, 2), (191 * 64, 128, 64, 190)])
+def test_states_at_the_edges_of_their_tiles(dev, L, D, BLKQ, T):
+    """The states H_i, z_i that a forward keeps, against the sums over the non-selected blocks in 64 bits.  Integers throughout
+    (relu, small k and v): the block states are exact in 16 bits, z and the sums exact in 32, so H is the one rounding of the
+    exact sum and z exact."""
+    gen = torch.Generator().manual_seed(L + T)
+    q, k, v = (torch.randint(lo, 2, (1, 2, L, D), generator=gen).to(torch.bfloat16) for lo in (0, 0, -1))
+    w, b = make_proj(D)
+    M, N = -(-L // BLKQ), -(-L // 64)
+    lut = torch.rand(1, 2, M, N, generator=gen).argsort(-1)[..., :T].sort(-1).values.contiguous()
+    _, states = linear_complement_fwd(*(t.to(dev) for t in (q, k, v, lut)), T, w.to(dev), b.to(dev), None, "relu", BLKQ, 64,
+                                      keep_states=True)
+    raw, n = states.cpu().view(torch.uint8).flatten(), 2 * M * D * D * 2
+    H = raw[:n].view(torch.bfloat16).view(2, M, D, D)
+    at = -(-n // 256) * 256
+    z = raw[at:at + 2 * M * D * 4].view(torch.float32).view(2, M, D)
+    kb, vb = (torch.nn.functional.pad(t[0].double(), (0, 0, 0, N * 64 - L)).unflatten(1, (N, 64)) for t in (k, v))
+    rest = 1 - torch.zeros(2, M, N, dtype=torch.float64).scatter_(2, lut[0], 1.0)
+    want_h = (rest @ (vb.transpose(-1, -2) @ kb).flatten(2)).unflatten(2, (D, D))          # (transposed: [d2][d1])
+    assert torch.equal(H, want_h.to(torch.bfloat16))
+    assert torch.equal(z.double(), rest @ kb.sum(2))
