@@ -10,6 +10,7 @@
 //   S = (q_int8 . k_int8) * sq * sk * scale ; P = softmax numerators over the selected blocks ;
 //   O = (e4m3(c P) . v_fp8) * sv / sum(e4m3(c P)), c = 112 with P <= 4 (reference maximum lagging by <= 2).
 // The look-up table of the bf16 path is used as is (no delta encoding is needed here).
+#include <type_traits>
 #include "block_map.h"
 #include "block_pool.h"
 #include "common.h"
@@ -230,12 +231,23 @@ typedef __attribute__((address_space(3))) i32x2_t lds_i32x2_t;
 // probabilities are at most 4; they are scaled by 112 = 448/4 to use the e4m3 range.
 // K/V tiles: global -> registers -> LDS, double-buffered in LDS: the next tile is in flight during the whole
 // current one and there is one barrier per tile.
-template <typename OutTag, int D, int BLKQ>
+// LINEAR: the linear branch of the same rows, projection, bias and sum in the epilogue (bit for bit what the attention and
+// linear_out_kernel behind it leave): the per-head state (32 KB) is read straight from L2 in operand order, as in the 16-bit
+// kernel's epilogue, so that no barrier holds the other workgroup of the compute unit.  It costs this kernel 55 us at 40 heads x
+// 32760 x 128, softmax map, where the launch of its own, bound by memory (o_s written and read again), took 203.  q's rows are
+// loaded behind the last product: beside it they cost spills (1.66 ms for 1.62).
+struct SageLinear {
+  const uint16_t *q, *kvwt, *z;
+  const float* bias;
+  RowLayout lq, lout;
+  int fmap;
+};
+template <typename OutTag, int D, int BLKQ, bool LINEAR>
 __global__ __launch_bounds__(BLKQ * 2) __attribute__((amdgpu_waves_per_eu(2, 2))) void sage_fwd_kernel(
     const int8_t* __restrict__ q8, const float* __restrict__ q_scale, const int8_t* __restrict__ k8,
     const float* __restrict__ k_scale, const uint8_t* __restrict__ v8, const float* __restrict__ v_scale,
     const void* __restrict__ lut, int lut64, uint16_t* __restrict__ o, int L, int Mblk, int Nblk, int topk,
-    float scale_log2e, int total) {
+    float scale_log2e, int total, const SageLinear lin) {
   using EO = Elem<OutTag>;
   constexpr int BLKK = 64;
   constexpr int NT = BLKQ * 2;
@@ -243,7 +255,8 @@ __global__ __launch_bounds__(BLKQ * 2) __attribute__((amdgpu_waves_per_eu(2, 2))
   constexpr int DT = D / 32;                // 32-row tiles of O^T
   constexpr int STR = D + 16;               // bytes per LDS row
   constexpr int CPR = D / 16;               // 16-byte chunks per row
-  constexpr int NLD = (BLKK * CPR + NT - 1) / NT;
+  constexpr int NLD = BLKK * CPR / NT;
+  static_assert(BLKK * CPR % NT == 0, "a tile divides among the threads");
   constexpr float TAU = 2.0f;
   // probabilities are scaled by 112 = 448 / 2^TAU, applied as an offset of the exponent
   constexpr float LOG2_P_SCALE = 6.807354922057604f;
@@ -272,9 +285,19 @@ __global__ __launch_bounds__(BLKQ * 2) __attribute__((amdgpu_waves_per_eu(2, 2))
   const float* ksc = k_scale + (size_t)bh * Nblk;
 
   const size_t lut_row = ((size_t)bh * Mblk + mb) * topk;
-  auto lut_at = [&](int i) -> int {
-    return lut64 ? (int)reinterpret_cast<const long long*>(lut)[lut_row + i]
-                 : reinterpret_cast<const int*>(lut)[lut_row + i];
+  // 64 entries of the list at a time in the wave's lanes, with the tiles' dequantisation factors (as scalar loads, two per
+  // tile, they share their counter with the LDS reads: 1 % of the kernel).
+  int list_nb = 0;
+  float list_sc = 0.f;
+  auto entry = [&](int i, float& sc) -> int {                  // (i ascending by one)
+    if ((i & 63) == 0) {
+      const int at = min(i + lane, topk - 1);
+      list_nb = lut64 ? (int)reinterpret_cast<const long long*>(lut)[lut_row + at] : reinterpret_cast<const int*>(lut)[lut_row + at];
+      // an all-zero block has scale 1e-30/127; the floor keeps -inf * sc = -inf (never NaN) for masked rows
+      list_sc = fmaxf(qs * ksc[list_nb], 1e-37f);
+    }
+    sc = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(list_sc), i & 63));
+    return __builtin_amdgcn_readlane(list_nb, i & 63);
   };
   i16x8_t kreg[NLD], vreg[NLD];
   auto load_tile = [&](int nb) {
@@ -282,8 +305,7 @@ __global__ __launch_bounds__(BLKQ * 2) __attribute__((amdgpu_waves_per_eu(2, 2))
     for (int i = 0; i < NLD; ++i) {
       const int idx = tid + i * NT;
       const int row = idx / CPR, col = (idx % CPR) * 16;
-      // chunks past the tile (when the tile does not divide among the threads) and rows past L read as zero
-      const uint32_t off = idx < BLKK * CPR ? (uint32_t)(nb * BLKK + row) * D + col : 0xfffffff0u;
+      const uint32_t off = (uint32_t)(nb * BLKK + row) * D + col;      // (rows past L read as zero)
       kreg[i] = buf_load_b128(kh, off);
       vreg[i] = buf_load_b128(vh, off);
     }
@@ -292,11 +314,9 @@ __global__ __launch_bounds__(BLKQ * 2) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
     for (int i = 0; i < NLD; ++i) {
       const int idx = tid + i * NT;
-      if (idx < BLKK * CPR) {
-        const int row = idx / CPR, col = (idx % CPR) * 16;
-        *reinterpret_cast<i16x8_t*>(&sK[kslot][row * STR + col]) = kreg[i];
-        *reinterpret_cast<i16x8_t*>(&sV[vslot][row * STR + col]) = vreg[i];
-      }
+      const int row = idx / CPR, col = (idx % CPR) * 16;
+      *reinterpret_cast<i16x8_t*>(&sK[kslot][row * STR + col]) = kreg[i];
+      *reinterpret_cast<i16x8_t*>(&sV[vslot][row * STR + col]) = vreg[i];
     }
   };
 
@@ -334,40 +354,37 @@ __global__ __launch_bounds__(BLKQ * 2) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
   for (int i = 0; i < 16; ++i) magic[i] = MAGIC;
   // S^T of one tile: MAGIC + raw int32 products of both 32-key halves
-  auto scores = [&](int kslot, i32x16_t (&acc)[2]) {
+  auto scores = [&](int kslot, i32x16_t (&acc)[2]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
+    for (int c = 0; c < QC; ++c) {
 #pragma unroll
-      for (int c = 0; c < QC; ++c) {
+      for (int t = 0; t < 2; ++t) {
         const i32x4_t a = *reinterpret_cast<const i32x4_t*>(&sK[kslot][(32 * t + r) * STR + 32 * c + 16 * g]);
         acc[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, qf[c], c == 0 ? magic : acc[t], 0, 0, 0);
       }
     }
   };
-  // softmax numerators of one tile (scores acc, dequantisation factor sc, kv_valid existing key rows),
-  // packed to e4m3 in the B-operand order of the 64-key product
-  auto probabilities = [&](const i32x16_t (&acc)[2], float sc, int kv_valid) -> i32x8_t {
-    float s[2][16];
+  // ragged last key block (kv_valid existing key rows): missing rows take no part
+  auto mask = [&](i32x16_t (&acc)[2], int kv_valid) __attribute__((always_inline)) {
+    const int lim = kv_valid - 4 * g;      // key index of register i is 32t + 8(i/4) + i%4 + 4g
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) s[t][i] = __int_as_float(acc[t][i]);         // = 12582912 + score
-    if (kv_valid < BLKK) {                 // ragged last key block: missing rows take no part
-      const int lim = kv_valid - 4 * g;    // key index of register i is 32t + 8(i/4) + i%4 + 4g
-#pragma unroll
-      for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int i = 0; i < 16; ++i)
-          if (32 * t + 8 * (i >> 2) + (i & 3) >= lim) s[t][i] = -INFINITY;
-    }
-    // raw maximum of this lane's 32 scores (sc > 0, so the maximum commutes with the scaling)
-    float mx = s[0][0];
+      for (int i = 0; i < 16; ++i)
+        if (32 * t + 8 * (i >> 2) + (i & 3) >= lim) acc[t][i] = (int)0xff800000u;      // -inf
+  };
+  // raw maximum of this lane's 32 scores (sc > 0, so the maximum commutes with the scaling)
+  auto maximum = [&](const i32x16_t (&acc)[2]) __attribute__((always_inline)) {
+    float mx = __int_as_float(acc[0][0]);                                              // = 12582912 + score
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[t][i]);
-    mx -= MAGIC_F;                         // (exact: both are integers below 2^24)
-    if (__any(mx * sc > m_used + TAU)) {   // rare: move the reference and rescale what is accumulated
+      for (int i = 0; i < 16; ++i) mx = fmaxf(mx, __int_as_float(acc[t][i]));
+    return mx - MAGIC_F;                   // (exact: both are integers below 2^24)
+  };
+  // rare: moves the reference and rescales what is accumulated
+  auto raise_reference = [&](float mx, float sc) __attribute__((always_inline)) {
+    if (__any(mx * sc > m_used + TAU)) {
       float m_new = fmaxf(mx, __shfl_xor(mx, 32)) * sc;
       m_new = fmaxf(m_used, m_new);
       const float f = fast_exp2(m_used - m_new);     // 0 on the first tile
@@ -379,6 +396,10 @@ __global__ __launch_bounds__(BLKQ * 2) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
         for (int i = 0; i < 16; ++i) oacc[dt][i] *= f;
     }
+  };
+  // softmax numerators of one tile (scores acc, dequantisation factor sc), packed to e4m3 in the B-operand order of the
+  // 64-key product
+  auto probabilities = [&](const i32x16_t (&acc)[2], float sc) __attribute__((always_inline)) -> i32x8_t {
     // 112 p = exp2(s*sc - (m_used - log2 112)); -inf scores give exactly 0
     const float m_off = __builtin_fmaf(MAGIC_F, sc, m_used - LOG2_P_SCALE);
     i32x8_t pb;
@@ -388,13 +409,13 @@ __global__ __launch_bounds__(BLKQ * 2) __attribute__((amdgpu_waves_per_eu(2, 2))
       for (int i4 = 0; i4 < 4; ++i4) {
         float pv[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) pv[j] = fast_exp2(__builtin_fmaf(s[t][4 * i4 + j], sc, -m_off));
+        for (int j = 0; j < 4; ++j) pv[j] = fast_exp2(__builtin_fmaf(__int_as_float(acc[t][4 * i4 + j]), sc, -m_off));
         pb[4 * t + i4] = (int)cvt4_fp8(pv[0], pv[1], pv[2], pv[3]);
       }
     return pb;
   };
   // l += sum_keys P ; O^T += V8^T P^T: one 64-key product per 32 output channels
-  auto accumulate = [&](int vslot, const i32x8_t& pb) {
+  auto accumulate = [&](int vslot, const i32x8_t& pb) __attribute__((always_inline)) {
     // formats 0/0 = e4m3 for both operands, block scales 2^0
     lacc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(ones, pb, lacc, 0, 0, 0, 0x7f7f7f7f, 0, 0x7f7f7f7f);
 #pragma unroll
@@ -413,55 +434,78 @@ __global__ __launch_bounds__(BLKQ * 2) __attribute__((amdgpu_waves_per_eu(2, 2))
     }
   };
 
-  // Software pipeline over the selected tiles: step i issues the int8 products of tile i, then does the
-  // exponentials of tile i-1 on the vector ALU while the matrix core works, then issues the fp8 products
-  // of tile i-1.  Tile i+1 is in flight from global memory during the whole step.
-  int nb = topk > 0 ? lut_at(0) : 0;
-  int nb_next = topk > 1 ? lut_at(1) : 0;
-  if (topk > 0) {
-    load_tile(nb);
-    store_tile(0, 0);
-  }
-  __syncthreads();
-  i32x16_t acc_a[2], acc_b[2];              // scores of even / odd steps (ping-pong, no copies)
-  float sc_prev = 0.f;
-  int valid_prev = BLKK;
+  // Software pipeline over the selected tiles: step i issues the int8 products of tile i beside the exponentials of tile i-1,
+  // then the fp8 products of tile i-1 beside the maxima of tile i; between the two only the rare branches.  Tile i+1
+  // is in flight from global memory during the whole step.  Bound by the vector ALU (58 % of the cycles, the matrix cores 34;
+  // 1.40 ms at 51 tiles per row where a head's k and v fit an XCD's L2, 1.60 where not); the exponentials' order against the
+  // products, pinned one by one or left to the compiler inside the two halves, makes no difference beyond 2 %.
+  int nb = 0;
+  float sc = 0.f, sc_prev = 0.f, mx_prev = 0.f;
   int vslot_prev = 0, vslot = 0;
-  auto step = [&](int it, i32x16_t (&acc)[2], const i32x16_t (&acc_prev)[2]) {
+  i32x16_t acc_a[2], acc_b[2];              // scores of even / odd steps (ping-pong, no copies)
+  auto step = [&](int it, i32x16_t (&acc)[2], const i32x16_t (&acc_prev)[2], auto first) __attribute__((always_inline)) {
     const int kv_valid = L - nb * BLKK;
-    // an all-zero block has scale 1e-30/127; the floor keeps -inf * sc = -inf (never NaN) for masked rows
-    const float sc = fmaxf(qs * ksc[nb], 1e-37f);
+    const float sc_here = sc;
     const bool more = it + 1 < topk;
     if (more) {
-      nb = nb_next;
-      nb_next = it + 2 < topk ? lut_at(it + 2) : 0;
+      nb = entry(it + 1, sc);
       load_tile(nb);
     }
-    scores(it & 1, acc);
-    if (it > 0) {
-      const i32x8_t pb = probabilities(acc_prev, sc_prev, valid_prev);
+    i32x8_t pb;
+    if constexpr (first) {
+      scores(it & 1, acc);
+    } else {
+      raise_reference(mx_prev, sc_prev);
+      __builtin_amdgcn_sched_barrier(0);
+      scores(it & 1, acc);
+      pb = probabilities(acc_prev, sc_prev);
+      asm volatile("" :: "v"(pb));          // (formed here, not where the products below read them)
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (kv_valid < BLKK) mask(acc, kv_valid);
+    if constexpr (!first) {
+      __builtin_amdgcn_sched_barrier(0);
       accumulate(vslot_prev, pb);
     }
-    sc_prev = sc;
-    valid_prev = kv_valid;
+    mx_prev = maximum(acc);
+    sc_prev = sc_here;
     vslot_prev = vslot;
     vslot = vslot == 2 ? 0 : vslot + 1;
     if (more) store_tile((it + 1) & 1, vslot);
-    __syncthreads();                       // next tile visible; K of this step and V of the previous one consumed
+    lds_barrier();                         // next tile visible; K of this step and V of the previous one consumed
   };
-  int it = 0;
+  if (topk > 0) {
+    nb = entry(0, sc);
+    load_tile(nb);
+    store_tile(0, 0);
+    lds_barrier();
+    step(0, acc_a, acc_b, std::true_type{});
+  }
+  int it = 1;
   for (; it + 1 < topk; it += 2) {
-    step(it, acc_a, acc_b);
-    step(it + 1, acc_b, acc_a);
+    step(it, acc_b, acc_a, std::false_type{});
+    step(it + 1, acc_a, acc_b, std::false_type{});
   }
-  if (it < topk) {                         // odd count: one more step, its scores land in acc_a
-    step(it, acc_a, acc_b);
-    const i32x8_t pb = probabilities(acc_a, sc_prev, valid_prev);
-    accumulate(vslot_prev, pb);
+  const auto last = [&](const i32x16_t (&acc)[2]) __attribute__((always_inline)) {
+    raise_reference(mx_prev, sc_prev);
+    accumulate(vslot_prev, probabilities(acc, sc_prev));
+  };
+  constexpr int DC = D / 16;
+  i16x8_t xq[DC];                          // q as it is: this lane holds d = 16c + 8g + j of its row
+  const auto fetch_q = [&]() __attribute__((always_inline)) {
+    if constexpr (LINEAR) {
+      const uint16_t* p = lin.q + lin.lq.head(bh) + (size_t)min(qrow, L - 1) * (size_t)lin.lq.sl + 8 * g;
+#pragma unroll
+      for (int c = 0; c < DC; ++c) xq[c] = *reinterpret_cast<const i16x8_t*>(p + 16 * c);
+    }
+  };
+  if (it < topk) {                         // an even count: one more step, its scores land in acc_b
+    step(it, acc_b, acc_a, std::false_type{});
+    last(acc_b);
   } else if (topk > 0) {
-    const i32x8_t pb = probabilities(acc_b, sc_prev, valid_prev);
-    accumulate(vslot_prev, pb);
+    last(acc_a);
   }
+  fetch_q();
   const float inv = 1.0f / lacc[0];        // P_SCALE cancels: numerator and l carry the same factor
   // The rounded rows go through LDS (every wave is done with the tiles) and leave as whole rows in streaming stores:
   // they are not read again here, and what does not stay behind as modified lines in L2 need not be written back when
@@ -473,22 +517,65 @@ __global__ __launch_bounds__(BLKQ * 2) __attribute__((amdgpu_waves_per_eu(2, 2))
     uint16_t* const stage = wave < 3 ? reinterpret_cast<uint16_t*>(&sV[0][0]) + wave * (32 * SSTR)
                                      : reinterpret_cast<uint16_t*>(&sK[0][0]);
     const float* vs = v_scale + (size_t)bh * D;
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-      for (int i4 = 0; i4 < 4; ++i4) {
-        const int d0 = 32 * dt + 8 * i4 + 4 * g;
-        const f32x4_t sv = *reinterpret_cast<const f32x4_t*>(vs + d0);
-        i32x2_t w;
-        w[0] = (int)EO::pack2(oacc[dt][4 * i4 + 0] * inv * sv[0], oacc[dt][4 * i4 + 1] * inv * sv[1]);
-        w[1] = (int)EO::pack2(oacc[dt][4 * i4 + 2] * inv * sv[2], oacc[dt][4 * i4 + 3] * inv * sv[3]);
-        *reinterpret_cast<i32x2_t*>(&stage[r * SSTR + d0]) = w;
-      }
-    wave_lds_fence();
     const int row0 = mb * BLKQ + wave * 32;
+    // the attention's values of registers 4 i4 .. of tile dt, in 16 bit
+    const auto attention = [&](int dt, int i4) __attribute__((always_inline)) -> i32x2_t {
+      const f32x4_t sv = *reinterpret_cast<const f32x4_t*>(vs + 32 * dt + 8 * i4 + 4 * g);
+      i32x2_t w;
+      w[0] = (int)EO::pack2(oacc[dt][4 * i4 + 0] * inv * sv[0], oacc[dt][4 * i4 + 1] * inv * sv[1]);
+      w[1] = (int)EO::pack2(oacc[dt][4 * i4 + 2] * inv * sv[2], oacc[dt][4 * i4 + 3] * inv * sv[3]);
+      return w;
+    };
+    if constexpr (!LINEAR) {
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int i4 = 0; i4 < 4; ++i4)
+          *reinterpret_cast<i32x2_t*>(&stage[r * SSTR + 32 * dt + 8 * i4 + 4 * g]) = attention(dt, i4);
+    } else {
+      const uint16_t* const state = lin.kvwt + (size_t)bh * D * D;
+      const uint16_t* const z = lin.z + (size_t)bh * D;
+      i16x8_t zc[DC];
+#pragma unroll
+      for (int c = 0; c < DC; ++c) zc[c] = *reinterpret_cast<const i16x8_t*>(z + 16 * c + 8 * g);
+      i16x8_t fq[DC];
+      float den = phi_pack_den<OutTag, DC>(lin.fmap, xq, fq, [&](int c, int j) { return EO::to_float((uint16_t)zc[c][j]); });
+      den += __shfl_xor(den, 32);
+      den = round16<OutTag>(1e-5f + round16<OutTag>(den));
+      const float inv_den = 1.0f / den;
+#pragma unroll
+      for (int et = 0; et < DT; ++et) {
+        i16x8_t a[DC];
+#pragma unroll
+        for (int c = 0; c < DC; ++c) a[c] = *reinterpret_cast<const i16x8_t*>(state + (size_t)(32 * et + r) * D + 16 * c + 8 * g);
+        f32x16_t acc;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+#pragma unroll
+        for (int c = 0; c < DC; ++c) acc = EO::mfma32(a[c], fq[c], acc);
+#pragma unroll
+        for (int i4 = 0; i4 < 4; ++i4) {
+          const int e0 = 32 * et + 8 * i4 + 4 * g;
+          const i32x2_t o_s = attention(et, i4);
+          i32x2_t w;
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {    // (both summands in 16 bit, one rounded sum, as tensors)
+            const uint32_t x = (uint32_t)o_s[h];
+            float l[2];
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+              l[j] = round16<OutTag>(pin_f32(__builtin_fmaf(acc[4 * i4 + 2 * h + j], inv_den, round16<OutTag>(lin.bias[e0 + 2 * h + j]))));
+            w[h] = (int)EO::pack2(EO::to_float((uint16_t)(x & 0xffff)) + l[0], EO::to_float((uint16_t)(x >> 16)) + l[1]);
+          }
+          *reinterpret_cast<i32x2_t*>(&stage[r * SSTR + e0]) = w;
+        }
+      }
+    }
+    wave_lds_fence();
     TileRows<D> t;
     t.unpark(stage, lane);
-    t.store_streaming(o + head_off + (size_t)row0 * D, L - row0, lane, D);
+    const size_t pitch = LINEAR ? (size_t)lin.lout.sl : (size_t)D;
+    t.store_streaming(o + (LINEAR ? lin.lout.head(bh) : head_off) + (size_t)row0 * pitch, L - row0, lane, pitch);
   }
 }
 
@@ -750,35 +837,47 @@ extern "C" int sage_quant_v_strided(const void* v, const int64_t* v_strides, int
   return quant_v_entry(v, v_strides, dtype, B, H, L, D, v_fp8, v_scale, v_range, workspace, workspace_bytes, stream);
 }
 
+namespace sla {
+// (lin null: the attention alone, contiguous rows)
+static int sage_attention_run(const int8_t* q8, const float* qs, const int8_t* k8, const float* ks, const uint8_t* v8, const float* vs,
+                              const void* lut, int lut64, void* o, int dtype, int BH, int L, int D, int topk, float qk_scale,
+                              const SageLinear* lin, hipStream_t st) {
+  const int Mblk = cdiv(L, 128), Nblk = cdiv(L, 64), total = BH * Mblk;
+  const float c = qk_scale * 1.4426950408889634f;
+#define SAGE_CASE(TAG, DD)                                                                                                  \
+  if (lin)                                                                                                                  \
+    hipLaunchKernelGGL((sage_fwd_kernel<TAG, DD, 128, true>), dim3(xcd_grid(total)), dim3(256), 0, st, q8, qs, k8, ks, v8, vs, \
+                       lut, lut64, (uint16_t*)o, L, Mblk, Nblk, topk, c, total, *lin);                                      \
+  else                                                                                                                      \
+    hipLaunchKernelGGL((sage_fwd_kernel<TAG, DD, 128, false>), dim3(xcd_grid(total)), dim3(256), 0, st, q8, qs, k8, ks, v8, vs, \
+                       lut, lut64, (uint16_t*)o, L, Mblk, Nblk, topk, c, total, SageLinear{})
+  if (dtype == SLA_BF16) {
+    if (D == 128) { SAGE_CASE(bf16_tag, 128); }
+    else { SAGE_CASE(bf16_tag, 64); }
+  } else {
+    if (D == 128) { SAGE_CASE(f16_tag, 128); }
+    else { SAGE_CASE(f16_tag, 64); }
+  }
+#undef SAGE_CASE
+  return check_launch("sage_sparse_attn_fwd");
+}
+}  // namespace sla
+
 extern "C" int sage_sparse_attn_fwd(const int8_t* q_int8, const float* q_scale, const int8_t* k_int8,
                                     const float* k_scale, const uint8_t* v_fp8, const float* v_scale, const void* lut,
                                     int lut_elem_bytes, void* o, int out_dtype, int B, int H, int L, int D, int BLKQ,
                                     int BLKK, int topk, float qk_scale, void* stream) {
   int rc = validate_sage(out_dtype, B, H, L, D, BLKQ, BLKK);
   if (rc) return rc;
-  const int Mblk = cdiv(L, BLKQ), Nblk = cdiv(L, BLKK);
+  const int Nblk = cdiv(L, BLKK);
   SLA_REQUIRE(topk >= 0 && topk <= Nblk, SLA_ERR_BAD_ARG, "topk=%d outside [0, %d]", topk, Nblk);
   SLA_REQUIRE(lut_elem_bytes == 4 || lut_elem_bytes == 8, SLA_ERR_BAD_ARG, "lut_elem_bytes must be 4 or 8");
   SLA_REQUIRE(q_int8 && q_scale && k_int8 && k_scale && v_fp8 && v_scale && o && (lut || topk == 0), SLA_ERR_BAD_ARG,
               "null pointer");
   SLA_REQUIRE(((uintptr_t)q_int8 | (uintptr_t)k_int8 | (uintptr_t)v_fp8 | (uintptr_t)o | (uintptr_t)v_scale) % 16 == 0,
               SLA_ERR_BAD_ARG, "pointers must be 16-byte aligned");
-  hipStream_t st = (hipStream_t)stream;
-  const int BH = B * H;
-  const int total = BH * Mblk;
-  const float c = qk_scale * 1.4426950408889634f;
-  const int lut64 = lut_elem_bytes == 8;
-#define SAGE_CASE(TAG, DD)                                                                                              \
-  hipLaunchKernelGGL((sage_fwd_kernel<TAG, DD, 128>), dim3(xcd_grid(total)), dim3(256), 0, st, q_int8, q_scale, k_int8, \
-                     k_scale, v_fp8, v_scale, lut, lut64, (uint16_t*)o, L, Mblk, Nblk, topk, c, total);                 \
-  return check_launch("sage_sparse_attn_fwd")
-  if (out_dtype == SLA_BF16) {
-    if (D == 128) { SAGE_CASE(bf16_tag, 128); }
-    SAGE_CASE(bf16_tag, 64);
-  }
-  if (D == 128) { SAGE_CASE(f16_tag, 128); }
-  SAGE_CASE(f16_tag, 64);
-#undef SAGE_CASE
+  return sage_attention_run(q_int8, q_scale, k_int8, k_scale, v_fp8, v_scale, lut, lut_elem_bytes == 8, o, out_dtype, B * H, L, D,
+                            topk, qk_scale, nullptr, (hipStream_t)stream);
 }
 
 // ---- the preparation of small inputs in four launches -----------------------------------------------------------------
@@ -919,7 +1018,7 @@ static void launch_small_preparation(const void* q, const void* k, const void* v
 namespace sla {
 struct SageModuleWs {
   int64_t prep_bytes, linear_bytes;
-  size_t prep, linear, q8, k8, v8, qs, ks, vs, lut, o_s, total;
+  size_t prep, linear, q8, k8, v8, qs, ks, vs, lut, total;
 };
 static SageModuleWs sage_module_ws(int B, int H, int L, int D, int topk) {
   const int64_t BH = (int64_t)B * H, M = cdiv(L, 128), N = cdiv(L, 64), elems = BH * L * D;
@@ -936,7 +1035,6 @@ static SageModuleWs sage_module_ws(int B, int H, int L, int D, int topk) {
   w.ks = off;     off += align_up(BH * N * 4, 256);
   w.vs = off;     off += align_up(BH * D * 4, 256);
   w.lut = off;    off += align_up(BH * M * topk * 4, 256);
-  w.o_s = off;    off += align_up(elems * 2, 256);
   w.total = off;
   return w;
 }
@@ -961,14 +1059,14 @@ extern "C" int sage_module_fwd(const void* q, const void* k, const void* v, cons
   const SageModuleWs w = sage_module_ws(B, H, L, D, topk);
   SLA_REQUIRE(workspace_bytes >= (int64_t)w.total, SLA_ERR_WORKSPACE, "workspace of %lld bytes, need %lld",
               (long long)workspace_bytes, (long long)w.total);
-  RowLayout lay;
-  if ((rc = make_layout(out_strides, B, H, L, D, 2, &lay))) return rc;
+  RowLayout lay, lout;
+  if ((rc = make_layout(out_strides, B, H, L, D, 2, &lout))) return rc;
   char* ws = (char*)workspace;
   hipStream_t st = (hipStream_t)stream, side = (hipStream_t)side_stream;
   int8_t *q8 = (int8_t*)(ws + w.q8), *k8 = (int8_t*)(ws + w.k8);
   uint8_t* v8 = (uint8_t*)(ws + w.v8);
   float *qs = (float*)(ws + w.qs), *ks = (float*)(ws + w.ks), *vs = (float*)(ws + w.vs);
-  void *lut = ws + w.lut, *o_s = ws + w.o_s;
+  void* lut = ws + w.lut;
   // (what the later steps would find wrong, before the first launch)
   rc = prepare_check(q, k, nullptr, qkv_strides, dtype, B, H, L, D, 128, 64, topk, nullptr, lut, 4, q8, qs, k8, ks, nullptr,
                      nullptr, v_range, ws + w.prep, w.prep_bytes, false, &lay);
@@ -983,18 +1081,18 @@ extern "C" int sage_module_fwd(const void* q, const void* k, const void* v, cons
     return prepare_entry(q, k, nullptr, qkv_strides, dtype, B, H, L, D, 128, 64, topk, nullptr, lut, 4, q8, qs, k8, ks, nullptr,
                          nullptr, v_range, ws + w.prep, w.prep_bytes, stream, false);
   };
+  RowLayout lq;
+  if ((rc = make_layout(qkv_strides, B, H, L, D, 2, &lq))) return rc;
   const auto attention = [&]() -> int {
-    int r = sage_sparse_attn_fwd(q8, qs, k8, ks, v8, vs, lut, 4, o_s, dtype, B, H, L, D, 128, 64, topk, qk_scale, stream);
-    if (r) return r;
-    return qkv_strides ? sla_linear_out_fwd_strided(q, qkv_strides, bias, o_s, out, out_strides, dtype, fmap, B, H, L, D,
-                                                    ws + w.linear, w.linear_bytes, stream)
-                       : sla_linear_out_fwd(q, bias, o_s, out, dtype, fmap, B, H, L, D, ws + w.linear, w.linear_bytes, stream);
+    const LinWs lw = lin_ws(B * H, L, D);
+    const char* states = ws + w.linear;
+    const SageLinear lin{(const uint16_t*)q, (const uint16_t*)(states + lw.kvwt), (const uint16_t*)(states + lw.z), bias, lq, lout, fmap};
+    return sage_attention_run(q8, qs, k8, ks, v8, vs, lut, 0, out, dtype, B * H, L, D, topk, qk_scale, &lin, st);
   };
   if (!side || side == st || !side_stream_pays(B, H, L, D, topk)) {
-    if ((rc = make_layout(qkv_strides, B, H, L, D, 2, &lay))) return rc;
     SLA_REQUIRE(w.linear_bytes >= linear_fwd_workspace_bytes(B * H, L, D), SLA_ERR_WORKSPACE, "workspace too small");
 #define SAGE_SMALL_CASE(TAG, DD)                                                                                              \
-  launch_small_preparation<TAG, DD>(q, k, v, lay, dtype, weight, fmap, B * H, L, topk, lut, q8, qs, k8, ks, v8, vs, v_range, \
+  launch_small_preparation<TAG, DD>(q, k, v, lq, dtype, weight, fmap, B * H, L, topk, lut, q8, qs, k8, ks, v8, vs, v_range, \
                                     ws + w.prep, ws + w.linear, st)
     if (dtype == SLA_BF16) {
       if (D == 128) SAGE_SMALL_CASE(bf16_tag, 128);
