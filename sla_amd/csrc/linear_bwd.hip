@@ -13,233 +13,33 @@
 //   finish : those sums added up -> dS (16 bit, both orientations), dz, per-head dW, db
 //   heads  : the heads' dW and db added up
 //   keys   : k and v once: dk, dv
-// The complement-mode branch forms dW and db with the states / reduce kernels below, from row-wise temporaries.
+// The complement-mode branch forms dW and db from row-wise temporaries, with the state kernel and the reduction below.
 #include "bwd_steps.h"
 #include "linear_bwd_stream.h"
 
 namespace sla {
 
-// ---- states -------------------------------------------------------------------------------
-// grid (nsplit, BH).  dS^T partial [d2][d1] per (bh, split); dW^T partial [d][e] per (bh, split).
-template <typename Tag, int D>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void linear_bwd_states_kernel(
-    const uint16_t* __restrict__ q, const uint16_t* __restrict__ dn, const uint16_t* __restrict__ gout,
-    const uint16_t* __restrict__ y, const float* __restrict__ dden, const RowLayout lin, const RowLayout ldo,
-    float* __restrict__ ds_part, float* __restrict__ dw_part, float* __restrict__ dz_part, float* __restrict__ db_part, int L,
-    int rows_per_split, int fmap) {
-  using E = Elem<Tag>;
-  constexpr int TR = 64;
-  constexpr int STR = D + 16;
-  constexpr int CPR = D / 8;
-  constexpr int RPP = 256 / CPR;
-  constexpr int NP = TR / RPP;
-  constexpr int DT = D / 32;
-  constexpr int WPT = (DT * DT) / 4;
-
-  __shared__ __attribute__((aligned(16))) uint16_t sA[TR * STR];
-  __shared__ __attribute__((aligned(16))) uint16_t sDN[TR * STR];
-  __shared__ __attribute__((aligned(16))) uint16_t sG[TR * STR];
-  __shared__ __attribute__((aligned(16))) uint16_t sY[TR * STR];
-  // the cross-thread sums of dz / db at the very end reuse the first two tiles (two workgroups per
-  // compute unit need the LDS footprint below 80 KB)
-  static_assert(2 * TR * STR * 2 >= 2 * RPP * D * 4, "reduction scratch does not fit the tiles it reuses");
-  float (*sRed)[RPP][D] = reinterpret_cast<float (*)[RPP][D]>(sA);
-
-  const int split = blockIdx.x, bh = blockIdx.y, nsplit = gridDim.x;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int g = lane >> 5;
-  const int row_begin = split * rows_per_split;
-  const int row_end = min(L, row_begin + rows_per_split);
-  const size_t head_off = (size_t)bh * L * D;
-  const int lrow = tid / CPR, lcol = (tid % CPR) * 8;
-
-  f32x16_t sacc[WPT], wacc[WPT];
-#pragma unroll
-  for (int t = 0; t < WPT; ++t)
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      sacc[t][i] = 0.f;
-      wacc[t][i] = 0.f;
-    }
-  float zacc[8], bacc[8];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    zacc[e] = 0.f;
-    bacc[e] = 0.f;
-  }
-  const int tr_row = (lane & 15) >> 2;
-  const int tr_col = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
-
-  // (no register prefetch of the next tile: the second workgroup on the compute unit covers the latency,
-  //  and the registers it would take are what lets that second workgroup fit)
-  i16x8_t rq[NP], rdn[NP], rg[NP], ry[NP];
-  float rdd[NP];
-  auto fetch = [&](int r0) {
-#pragma unroll
-    for (int p = 0; p < NP; ++p) {
-      const int grow = r0 + lrow + p * RPP;
-      rq[p] = i16x8_t{0, 0, 0, 0, 0, 0, 0, 0};
-      rdn[p] = rq[p];
-      rg[p] = rq[p];
-      ry[p] = rq[p];
-      rdd[p] = 0.f;
-      if (grow < row_end) {
-        const size_t off = head_off + (size_t)grow * D + lcol;          // dn, y: contiguous temporaries
-        rq[p] = *reinterpret_cast<const i16x8_t*>(q + lin.head(bh) + (size_t)grow * (size_t)lin.sl + lcol);
-        rdn[p] = *reinterpret_cast<const i16x8_t*>(dn + off);
-        rg[p] = *reinterpret_cast<const i16x8_t*>(gout + ldo.head(bh) + (size_t)grow * (size_t)ldo.sl + lcol);
-        ry[p] = *reinterpret_cast<const i16x8_t*>(y + off);
-        rdd[p] = dden[(size_t)bh * L + grow];
-      }
-    }
-  };
-  for (int r0 = row_begin; r0 < row_end; r0 += TR) {
-    fetch(r0);
-    __syncthreads();
-#pragma unroll
-    for (int p = 0; p < NP; ++p) {
-      const int row = lrow + p * RPP;
-      const int grow = r0 + row;
-      const bool ok = grow < row_end;
-      const i16x8_t xq = rq[p], xdn = rdn[p], xg = rg[p], xy = ry[p];
-      const float dd = rdd[p];
-      float f[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) f[e] = E::to_float((uint16_t)xq[e]);
-      if (fmap == SLA_FMAP_SOFTMAX) {
-        float mx = f[0];
-#pragma unroll
-        for (int e = 1; e < 8; ++e) mx = fmaxf(mx, f[e]);
-#pragma unroll
-        for (int s = 1; s < CPR; s <<= 1) mx = fmaxf(mx, __shfl_xor(mx, s));
-        float sum = 0.f;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          f[e] = __expf(f[e] - mx);
-          sum += f[e];
-        }
-#pragma unroll
-        for (int s = 1; s < CPR; s <<= 1) sum += __shfl_xor(sum, s);
-        const float inv = 1.0f / sum;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) f[e] = round16<Tag>(f[e] * inv);
-      } else if (fmap == SLA_FMAP_RELU) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) f[e] = fmap_pointwise<Tag>(SLA_FMAP_RELU, f[e]);
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) f[e] = fmap_pointwise<Tag>(SLA_FMAP_ELU, f[e]);
-      }
-      i16x8_t fa;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        if (!ok) f[e] = 0.f;
-        zacc[e] += dd * f[e];
-        bacc[e] += E::to_float((uint16_t)xg[e]);
-        fa[e] = (short)E::from_float(f[e]);
-      }
-      *reinterpret_cast<i16x8_t*>(&sA[row * STR + lcol]) = fa;
-      *reinterpret_cast<i16x8_t*>(&sDN[row * STR + lcol]) = xdn;
-      *reinterpret_cast<i16x8_t*>(&sG[row * STR + lcol]) = xg;
-      *reinterpret_cast<i16x8_t*>(&sY[row * STR + lcol]) = xy;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int c = 0; c < TR / 16; ++c) {
-      const int l0 = 16 * c + 8 * g + tr_row;
-#pragma unroll
-      for (int t = 0; t < WPT; ++t) {
-        const int tile = wave * WPT + t;
-        const int mt = tile / DT, nt = tile % DT;
-        const uint16_t* pa = &sA[l0 * STR + 32 * mt + tr_col];
-        const uint16_t* pb = &sDN[l0 * STR + 32 * nt + tr_col];
-        sacc[t] = E::mfma32(concat4(lds_read_tr16(pa), lds_read_tr16(pa + 4 * STR)),
-                            concat4(lds_read_tr16(pb), lds_read_tr16(pb + 4 * STR)), sacc[t]);
-        const uint16_t* pg = &sG[l0 * STR + 32 * mt + tr_col];
-        const uint16_t* py = &sY[l0 * STR + 32 * nt + tr_col];
-        wacc[t] = E::mfma32(concat4(lds_read_tr16(pg), lds_read_tr16(pg + 4 * STR)),
-                            concat4(lds_read_tr16(py), lds_read_tr16(py + 4 * STR)), wacc[t]);
-      }
-    }
-  }
-  // accumulator: rows = first operand's index (d1 / e), column = second operand's index (d2 / d);
-  // stored with the column as the slow axis: part[col][row]
-  const size_t pidx = (size_t)bh * nsplit + split;
-  float* so = ds_part + pidx * D * D;
-  float* wo = dw_part + pidx * D * D;
-#pragma unroll
-  for (int t = 0; t < WPT; ++t) {
-    const int tile = wave * WPT + t;
-    const int mt = tile / DT, nt = tile % DT;
-    const int col = 32 * nt + (lane & 31);
-#pragma unroll
-    for (int i4 = 0; i4 < 4; ++i4) {
-      const f32x4_t a = {sacc[t][4 * i4], sacc[t][4 * i4 + 1], sacc[t][4 * i4 + 2], sacc[t][4 * i4 + 3]};
-      const f32x4_t b = {wacc[t][4 * i4], wacc[t][4 * i4 + 1], wacc[t][4 * i4 + 2], wacc[t][4 * i4 + 3]};
-      *reinterpret_cast<f32x4_t*>(so + (size_t)col * D + 32 * mt + 8 * i4 + 4 * g) = a;
-      *reinterpret_cast<f32x4_t*>(wo + (size_t)col * D + 32 * mt + 8 * i4 + 4 * g) = b;
-    }
-  }
-  __syncthreads();
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    sRed[0][lrow][lcol + e] = zacc[e];
-    sRed[1][lrow][lcol + e] = bacc[e];
-  }
-  __syncthreads();
-  if (tid < D) {
-    float s0 = 0.f, s1 = 0.f;
-#pragma unroll
-    for (int rr = 0; rr < RPP; ++rr) {
-      s0 += sRed[0][rr][tid];
-      s1 += sRed[1][rr][tid];
-    }
-    dz_part[pidx * D + tid] = s0;
-    db_part[pidx * D + tid] = s1;
-  }
-}
-
-// ---- reduce -------------------------------------------------------------------------------
-// Stage 1, grid (cdiv(D*D,256), BH): per head, add the split partials in ascending order:
-//   dS (16 bit, both orientations), dz, and this head's dW^T / db (fp32).
-// Stage 2 (head_sums_body): add the per-head dW^T / db in ascending head order.
-template <typename Tag>
-__global__ __launch_bounds__(256) void linear_bwd_reduce_kernel(const float* __restrict__ ds_part,
-                                                                const float* __restrict__ dw_part,
-                                                                const float* __restrict__ dz_part,
-                                                                const float* __restrict__ db_part, uint16_t* __restrict__ ds,
-                                                                uint16_t* __restrict__ dst, float* __restrict__ dz,
+// ---- weight gradients apart ------------------------------------------------------------------
+// grid (cdiv(D*D,256), BH): a head's dW^T, db from its slices' partial sums, in ascending order.
+__global__ __launch_bounds__(256) void linear_bwd_reduce_kernel(const float* __restrict__ dw_part, const float* __restrict__ db_part,
                                                                 float* __restrict__ dw_head, float* __restrict__ db_head,
                                                                 int nsplit, int D) {
-  using E = Elem<Tag>;
   const int DD = D * D;
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   const int bh = blockIdx.y;
   if (i < DD) {
-    const float* p = ds_part + (size_t)bh * nsplit * DD + i;
-    const float* pw = dw_part + (size_t)bh * nsplit * DD + i;
-    float s = 0.f, sw = 0.f;
-#pragma unroll 8
-    for (int sp = 0; sp < nsplit; ++sp) {
-      s += p[(size_t)sp * DD];
-      sw += pw[(size_t)sp * DD];
-    }
-    const int d2 = i / D, d1 = i % D;   // partial layout [d2][d1]
-    const uint16_t h = E::from_float(s);
-    dst[(size_t)bh * DD + i] = h;                 // dS^T [d2][d1]
-    ds[(size_t)bh * DD + d1 * D + d2] = h;        // dS   [d1][d2]
-    dw_head[(size_t)bh * DD + i] = sw;            // dW^T [d][e] of this head
+    const float* p = dw_part + (size_t)bh * nsplit * DD + i;
+    float s = 0.f;
+#pragma unroll 16
+    for (int sp = 0; sp < nsplit; ++sp) s += p[(size_t)sp * DD];
+    dw_head[(size_t)bh * DD + i] = s;
   }
   if (i < D) {
-    const float* p = dz_part + (size_t)bh * nsplit * D + i;
-    const float* pb = db_part + (size_t)bh * nsplit * D + i;
-    float s = 0.f, sb = 0.f;
-    for (int sp = 0; sp < nsplit; ++sp) {
-      s += p[(size_t)sp * D];
-      sb += pb[(size_t)sp * D];
-    }
-    dz[(size_t)bh * D + i] = s;
-    db_head[(size_t)bh * D + i] = sb;
+    const float* p = db_part + (size_t)bh * nsplit * D + i;
+    float s = 0.f;
+#pragma unroll 16
+    for (int sp = 0; sp < nsplit; ++sp) s += p[(size_t)sp * D];
+    db_head[(size_t)bh * D + i] = s;
   }
 }
 
@@ -324,25 +124,23 @@ static int linear_bwd_impl(const void* q, const void* k, const void* v, const fl
   return check_launch("linear_bwd");
 }
 
-// dW and db alone, from the row-wise temporaries a rows kernel has left (used by the backward of the complement-mode
-// linear branch, whose state gradients are per query block and formed elsewhere): the states kernel, its reduction and
-// the sum over the heads.  `ws` is a region of weight_grads_workspace_bytes() bytes.
+// dW and db alone, from d(out) and the row-wise y a rows kernel has left (used by the backward of the complement-mode linear
+// branch, whose state gradients are per query block and formed elsewhere): dW^T = y^T d(out) and db = sum d(out) are the state
+// kernel's sums with d(out) and y in the place of k and v.  `ws` is a region of weight_grads_workspace_bytes() bytes.
+// Bound by memory.  12 heads x 16380 x 128: 34 us and their reduction 9, where a kernel that formed the states' gradients
+// beside them, which this branch has per query block already, took 59 and its reduction 22.
 struct WeightGradWs {
   LinSplit st;
-  size_t ds_part, dw_part, dz_part, db_part, ds, dst, dz, dw_head, db_head, total;
+  size_t dw_part, db_part, dw_head, db_head, total;
 };
 static WeightGradWs weight_grad_ws(int BH, int L, int D) {
   WeightGradWs w;
-  w.st = lin_split(BH, L, 512);
+  const int min_rows = L >= 4096 ? 256 : cdiv(L, 16);             // (as in lin_ws)
+  w.st = lin_split(BH, L, 512, D == 64 ? StateTile<64, false>::TR : StateTile<128, false>::TR, min_rows);
   const int64_t np = (int64_t)BH * w.st.nsplit;
   size_t off = 0;
-  w.ds_part = off; off += align_up(np * D * D * 4, 256);
   w.dw_part = off; off += align_up(np * D * D * 4, 256);
-  w.dz_part = off; off += align_up(np * D * 4, 256);
   w.db_part = off; off += align_up(np * D * 4, 256);
-  w.ds = off;      off += align_up((int64_t)BH * D * D * 2, 256);
-  w.dst = off;     off += align_up((int64_t)BH * D * D * 2, 256);
-  w.dz = off;      off += align_up((int64_t)BH * D * 4, 256);
   w.dw_head = off; off += align_up((int64_t)BH * D * D * 4, 256);
   w.db_head = off; off += align_up((int64_t)BH * D * 4, 256);
   w.total = off;
@@ -351,28 +149,25 @@ static WeightGradWs weight_grad_ws(int BH, int L, int D) {
 int64_t weight_grads_workspace_bytes(int BH, int L, int D) { return (int64_t)weight_grad_ws(BH, L, D).total; }
 
 template <typename Tag, int D>
-static void weight_grads_impl(const void* q, const void* dn, const void* gout, const void* y, const float* dden, int BH, int L,
-                              int fmap, char* ws, float* d_weight, float* d_bias, hipStream_t st) {
+static void weight_grads_impl(const void* gout, const void* y, int BH, int L, char* ws, float* d_weight, float* d_bias,
+                              hipStream_t st) {
   const WeightGradWs w = weight_grad_ws(BH, L, D);
-  const RowLayout lay = contiguous_layout(BH, L, D);
-  hipLaunchKernelGGL((linear_bwd_states_kernel<Tag, D>), dim3(w.st.nsplit, BH), dim3(256), 0, st, (const uint16_t*)q,
-                     (const uint16_t*)dn, (const uint16_t*)gout, (const uint16_t*)y, dden, lay, lay, (float*)(ws + w.ds_part),
-                     (float*)(ws + w.dw_part), (float*)(ws + w.dz_part), (float*)(ws + w.db_part), L, w.st.rows_per_split, fmap);
-  hipLaunchKernelGGL((linear_bwd_reduce_kernel<Tag>), dim3(cdiv(D * D, 256), BH), dim3(256), 0, st,
-                     (const float*)(ws + w.ds_part), (const float*)(ws + w.dw_part), (const float*)(ws + w.dz_part),
-                     (const float*)(ws + w.db_part), (uint16_t*)(ws + w.ds), (uint16_t*)(ws + w.dst), (float*)(ws + w.dz),
-                     (float*)(ws + w.dw_head), (float*)(ws + w.db_head), w.st.nsplit, D);
-  launch_head_sums(HeadSums{(const float*)(ws + w.dw_head), (const float*)(ws + w.db_head), d_weight, d_bias, BH, D, D * D / 256},
-                   st);
+  float *const dw_head = (float*)(ws + w.dw_head), *const db_head = (float*)(ws + w.db_head);
+  hipLaunchKernelGGL((linear_state_partial_kernel<Tag, D, false, false, false, true>), dim3(w.st.nsplit, BH),
+                     dim3(StateTile<D, false>::NTH), 0, st, (const uint16_t*)gout, (const uint16_t*)y, contiguous_layout(BH, L, D),
+                     (void*)(ws + w.dw_part), (float*)(ws + w.db_part), L, w.st.rows_per_split, 0);
+  hipLaunchKernelGGL(linear_bwd_reduce_kernel, dim3(cdiv(D * D, 256), BH), dim3(256), 0, st, (const float*)(ws + w.dw_part),
+                     (const float*)(ws + w.db_part), dw_head, db_head, w.st.nsplit, D);
+  launch_head_sums(HeadSums{dw_head, db_head, d_weight, d_bias, BH, D, D * D / 256}, st);
 }
-void launch_weight_grads(int dtype, int D, const void* q, const void* dn, const void* gout, const void* y, const float* dden,
-                         int BH, int L, int fmap, char* ws, float* d_weight, float* d_bias, hipStream_t st) {
+void launch_weight_grads(int dtype, int D, const void* gout, const void* y, int BH, int L, char* ws, float* d_weight, float* d_bias,
+                         hipStream_t st) {
   if (dtype == SLA_BF16) {
-    if (D == 128) weight_grads_impl<bf16_tag, 128>(q, dn, gout, y, dden, BH, L, fmap, ws, d_weight, d_bias, st);
-    else weight_grads_impl<bf16_tag, 64>(q, dn, gout, y, dden, BH, L, fmap, ws, d_weight, d_bias, st);
+    if (D == 128) weight_grads_impl<bf16_tag, 128>(gout, y, BH, L, ws, d_weight, d_bias, st);
+    else weight_grads_impl<bf16_tag, 64>(gout, y, BH, L, ws, d_weight, d_bias, st);
   } else {
-    if (D == 128) weight_grads_impl<f16_tag, 128>(q, dn, gout, y, dden, BH, L, fmap, ws, d_weight, d_bias, st);
-    else weight_grads_impl<f16_tag, 64>(q, dn, gout, y, dden, BH, L, fmap, ws, d_weight, d_bias, st);
+    if (D == 128) weight_grads_impl<f16_tag, 128>(gout, y, BH, L, ws, d_weight, d_bias, st);
+    else weight_grads_impl<f16_tag, 64>(gout, y, BH, L, ws, d_weight, d_bias, st);
   }
 }
 

@@ -24,8 +24,8 @@ namespace sla {
 
 int validate_attn_shape(int dtype, int B, int H, int L, int D, int BLKQ, int BLKK, int topk, int lut_elem_bytes);
 int64_t weight_grads_workspace_bytes(int BH, int L, int D);
-void launch_weight_grads(int dtype, int D, const void* q, const void* dn, const void* gout, const void* y, const float* dden,
-                         int BH, int L, int fmap, char* ws, float* d_weight, float* d_bias, hipStream_t st);
+void launch_weight_grads(int dtype, int D, const void* gout, const void* y, int BH, int L, char* ws, float* d_weight, float* d_bias,
+                         hipStream_t st);
 
 // Weights of the states: one bit per row and block state, 1 where the state takes part; zero from the table's end on.
 // all[head][row] says that the row leaves every block out.  A lane of the matrix instruction holds one row and eight of sixteen
@@ -946,7 +946,7 @@ static int complement_bwd_impl(const void* q, const void* k, const void* v, cons
   hipLaunchKernelGGL((linear_state_partial_kernel<Tag, D, true, true>), dim3(Mblk, BH), dim3(256), 0, st, (const uint16_t*)q,
                      (const uint16_t*)dn, lay, (void*)dhblk, dzblk, L, BLKQ, fmap, (const float*)dden);
   // dW, db
-  launch_weight_grads(dtype, D, q, dn, d_out, y, dden, BH, L, fmap, ws + w.wg, d_weight, d_bias, st);
+  launch_weight_grads(dtype, D, d_out, y, BH, L, ws + w.wg, d_weight, d_bias, st);
   // dk, dv
   uint32_t* const wk = (uint32_t*)(ws + w.fwd.w);
   int* const all = (int*)(ws + w.fwd.all);

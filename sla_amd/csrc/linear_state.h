@@ -17,6 +17,7 @@ namespace sla {
 // instead of sum_rows phi(k) (used by the complement backward, where "k" is q and "v" a row gradient).
 // VMAX: the largest |v| of every column over the slice goes to vmax_part[bh][split][D] (what the FP8 quantiser of v
 // needs of v before it can start: v is streamed here anyway).
+// IDENT: phi is the identity (the projection's gradients: d(out)^T y, with the sum of d(out) as z).
 template <int D, bool OUT16>
 struct StateTile {
   static constexpr int NTH = OUT16 ? 256 : 512;                    // threads
@@ -26,7 +27,7 @@ struct StateTile {
   static constexpr int STR = D + 16;                               // LDS row stride: transposed reads of 4 rows hit disjoint banks
   static constexpr int LDS = 2 * TR * STR * 2;                     // bytes; the final sums reuse it
 };
-template <typename Tag, int D, bool OUT16, bool ZW, bool VMAX>
+template <typename Tag, int D, bool OUT16, bool ZW, bool VMAX, bool IDENT = false>
 static __device__ __forceinline__ void state_partial_body(const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
                                                           const RowLayout lay, void* __restrict__ kv_part_,
                                                           float* __restrict__ z_part, int L, int rows_per_split, int fmap,
@@ -106,7 +107,8 @@ static __device__ __forceinline__ void state_partial_body(const uint16_t* __rest
       float f[8];
 #pragma unroll
       for (int e = 0; e < 8; ++e) f[e] = E::to_float((uint16_t)kk[e]);
-      if (fmap == SLA_FMAP_SOFTMAX) {
+      if constexpr (IDENT) {
+      } else if (fmap == SLA_FMAP_SOFTMAX) {
         // the CPR lanes that share this row are adjacent: reduce max and sum across them
         float mx = f[0];
 #pragma unroll
@@ -224,14 +226,14 @@ static __device__ __forceinline__ void state_partial_body(const uint16_t* __rest
   }
 }
 
-template <typename Tag, int D, bool OUT16 = false, bool ZW = false, bool VMAX = false>
+template <typename Tag, int D, bool OUT16 = false, bool ZW = false, bool VMAX = false, bool IDENT = false>
 __global__ __launch_bounds__((StateTile<D, OUT16>::NTH)) __attribute__((amdgpu_waves_per_eu(OUT16 ? 3 : 4, OUT16 ? 3 : 4))) void linear_state_partial_kernel(
     const uint16_t* __restrict__ k, const uint16_t* __restrict__ v, const RowLayout lay, void* __restrict__ kv_part,
     float* __restrict__ z_part, int L, int rows_per_split, int fmap, const float* __restrict__ zweight = nullptr,
     float* __restrict__ vmax_part = nullptr) {
   __shared__ __attribute__((aligned(16))) char smem[StateTile<D, OUT16>::LDS];
-  state_partial_body<Tag, D, OUT16, ZW, VMAX>(k, v, lay, kv_part, z_part, L, rows_per_split, fmap, zweight, vmax_part, blockIdx.x,
-                                              blockIdx.y, gridDim.x, smem);
+  state_partial_body<Tag, D, OUT16, ZW, VMAX, IDENT>(k, v, lay, kv_part, z_part, L, rows_per_split, fmap, zweight, vmax_part,
+                                                     blockIdx.x, blockIdx.y, gridDim.x, smem);
 }
 
 // Position of column d2 inside a row whose columns are re-ordered to the accumulator slot order of the
