@@ -204,9 +204,10 @@ int sla_sparse_attn_linear_fwd_strided(const void* q, const void* k, const void*
 
 /* Backward of the whole module in one call: the kernels of sla_sparse_attn_bwd(_strided) followed by those of
  * sla_linear_bwd(_strided) with SLA_BWD_ACCUMULATE (the linear branch adds into dq, dk, dv), results equal to those two
- * calls bit for bit (the linear branch's kernels come first, and the attention kernels add).  The only flag is SLA_BWD_STATES_READY.  qkv_strides / do_strides: both NULL for contiguous
- * (B, H, L, D) tensors, else as in the strided calls.  o_s is the attention output the forward saved.  The two workspaces
- * are those of the two calls (SLA_WS_SPARSE_BWD, SLA_WS_LINEAR_BWD).
+ * calls bit for bit (the linear branch's kernels come first, and the attention kernels add).  The only flag is
+ * SLA_BWD_STATES_READY.  qkv_strides / do_strides: both NULL for contiguous (B, H, L, D) tensors, else as in the strided
+ * calls.  o_s is the attention output the forward saved.  The two workspaces are those of the two calls
+ * (SLA_WS_SPARSE_BWD, SLA_WS_LINEAR_BWD).
  * Everything runs on `stream`: the short kernels share the launches of longer ones.  side_stream is accepted for callers that
  * hand one over and not used.
  * Replaces autograd through SparseLinearAttention.forward, sparse_linear_attention/core.py:88-100 with

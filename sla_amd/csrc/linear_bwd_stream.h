@@ -627,7 +627,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void l
       for (int j = 0; j < 8; ++j)
         o = __builtin_amdgcn_mfma_f32_16x16x4f32(E::to_float((uint16_t)sf[j]), sm[l * EP + KQ * h + 8 * c + j], o, 0, 0, 0);
     }
-    // rows d2 = 16 tile + 4 h + i, column e: the layout linear_bwd_reduce_heads_kernel adds up
+    // rows d2 = 16 tile + 4 h + i, column e: the layout head_sums_body adds up
 #pragma unroll
     for (int i = 0; i < 4; ++i) dw_head[(size_t)bh * DD + (size_t)(16 * tile + 4 * h + i) * D + i0 + l] = o[i];
   }
