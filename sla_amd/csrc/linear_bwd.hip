@@ -126,7 +126,8 @@ static int linear_bwd_impl(const void* q, const void* k, const void* v, const fl
 
 // dW and db alone, from d(out) and the row-wise y a rows kernel has left (used by the backward of the complement-mode linear
 // branch, whose state gradients are per query block and formed elsewhere): dW^T = y^T d(out) and db = sum d(out) are the state
-// kernel's sums with d(out) and y in the place of k and v.  `ws` is a region of weight_grads_workspace_bytes() bytes.
+// kernel's sums with d(out) and y in the place of k and v.  Returns the sum over the heads for a later launch to take along.
+// `ws` is a region of weight_grads_workspace_bytes() bytes.
 // Bound by memory.  12 heads x 16380 x 128: 34 us and their reduction 9, where a kernel that formed the states' gradients
 // beside them, which this branch has per query block already, took 59 and its reduction 22.
 struct WeightGradWs {
@@ -149,8 +150,8 @@ static WeightGradWs weight_grad_ws(int BH, int L, int D) {
 int64_t weight_grads_workspace_bytes(int BH, int L, int D) { return (int64_t)weight_grad_ws(BH, L, D).total; }
 
 template <typename Tag, int D>
-static void weight_grads_impl(const void* gout, const void* y, int BH, int L, char* ws, float* d_weight, float* d_bias,
-                              hipStream_t st) {
+static HeadSums weight_grads_impl(const void* gout, const void* y, int BH, int L, char* ws, float* d_weight, float* d_bias,
+                                  hipStream_t st) {
   const WeightGradWs w = weight_grad_ws(BH, L, D);
   float *const dw_head = (float*)(ws + w.dw_head), *const db_head = (float*)(ws + w.db_head);
   hipLaunchKernelGGL((linear_state_partial_kernel<Tag, D, false, false, false, true>), dim3(w.st.nsplit, BH),
@@ -158,17 +159,16 @@ static void weight_grads_impl(const void* gout, const void* y, int BH, int L, ch
                      (void*)(ws + w.dw_part), (float*)(ws + w.db_part), L, w.st.rows_per_split, 0);
   hipLaunchKernelGGL(linear_bwd_reduce_kernel, dim3(cdiv(D * D, 256), BH), dim3(256), 0, st, (const float*)(ws + w.dw_part),
                      (const float*)(ws + w.db_part), dw_head, db_head, w.st.nsplit, D);
-  launch_head_sums(HeadSums{dw_head, db_head, d_weight, d_bias, BH, D, D * D / 256}, st);
+  return HeadSums{dw_head, db_head, d_weight, d_bias, BH, D, D * D / 256};
 }
-void launch_weight_grads(int dtype, int D, const void* gout, const void* y, int BH, int L, char* ws, float* d_weight, float* d_bias,
-                         hipStream_t st) {
+HeadSums launch_weight_grads(int dtype, int D, const void* gout, const void* y, int BH, int L, char* ws, float* d_weight,
+                             float* d_bias, hipStream_t st) {
   if (dtype == SLA_BF16) {
-    if (D == 128) weight_grads_impl<bf16_tag, 128>(gout, y, BH, L, ws, d_weight, d_bias, st);
-    else weight_grads_impl<bf16_tag, 64>(gout, y, BH, L, ws, d_weight, d_bias, st);
-  } else {
-    if (D == 128) weight_grads_impl<f16_tag, 128>(gout, y, BH, L, ws, d_weight, d_bias, st);
-    else weight_grads_impl<f16_tag, 64>(gout, y, BH, L, ws, d_weight, d_bias, st);
+    if (D == 128) return weight_grads_impl<bf16_tag, 128>(gout, y, BH, L, ws, d_weight, d_bias, st);
+    return weight_grads_impl<bf16_tag, 64>(gout, y, BH, L, ws, d_weight, d_bias, st);
   }
+  if (D == 128) return weight_grads_impl<f16_tag, 128>(gout, y, BH, L, ws, d_weight, d_bias, st);
+  return weight_grads_impl<f16_tag, 64>(gout, y, BH, L, ws, d_weight, d_bias, st);
 }
 
 int linear_bwd_steps(const void* q, const void* k, const void* v, const int64_t* qkv_strides, const float* weight,

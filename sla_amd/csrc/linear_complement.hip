@@ -18,14 +18,15 @@
 // At 12 heads of 16380 rows, head dim 128, 12 of 256 blocks selected, with the states formed inside the kernels of the rows (a
 // workgroup per query or key block, the whole state in 64 fp32 registers per thread, two waves per SIMD): out 236 us,
 // rows 171 us, kv 171 us.  With the states in a kernel of their own: out 77 us, rows 110 us, kv 112 us.
+#include "bwd_lists.h"
 #include "linear_state.h"
 
 namespace sla {
 
 int validate_attn_shape(int dtype, int B, int H, int L, int D, int BLKQ, int BLKK, int topk, int lut_elem_bytes);
 int64_t weight_grads_workspace_bytes(int BH, int L, int D);
-void launch_weight_grads(int dtype, int D, const void* gout, const void* y, int BH, int L, char* ws, float* d_weight, float* d_bias,
-                         hipStream_t st);
+HeadSums launch_weight_grads(int dtype, int D, const void* gout, const void* y, int BH, int L, char* ws, float* d_weight,
+                             float* d_bias, hipStream_t st);
 
 // Weights of the states: one bit per row and block state, 1 where the state takes part; zero from the table's end on.
 // all[head][row] says that the row leaves every block out.  A lane of the matrix instruction holds one row and eight of sixteen
@@ -69,14 +70,23 @@ __global__ __launch_bounds__(64) void complement_row_weights_kernel(const void* 
   if (tid == 0) all[at] = topk >= nblk;
 }
 
-// Columns of the map (key blocks): the query blocks that did not select it.  grid (cdiv(Nblk, 64), heads), a lane per key block,
-// a word per wave and pass.
+// Columns of the map (key blocks): the query blocks that did not select it.  A workgroup per strip of 64 key blocks and head, a
+// lane per key block, a word per wave and pass.  In the workgroups from `strips` x heads on the sum of the heads' weight gradients,
+// a wave each, which needs nothing of it: both are bound by latency, 5 us each in launches of their own (forward and backward of 12
+// heads x 16380 x 128 1059 us, in one 1057).
 __global__ __launch_bounds__(512) void complement_column_weights_kernel(const int8_t* __restrict__ map, uint32_t* __restrict__ w,
-                                                                        int* __restrict__ all, int Mblk, int Nblk) {
+                                                                        int* __restrict__ all, int Mblk, int Nblk, int strips,
+                                                                        int first_sum, const HeadSums heads) {
   __shared__ uint32_t any[64];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n = blockIdx.x * 64 + lane;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if ((int)blockIdx.x >= first_sum) {
+    const int job = ((int)blockIdx.x - first_sum) * 8 + wave;
+    if (job < heads.wgs) head_sums_body(heads, job);
+    return;
+  }
+  const int head = blockIdx.x / strips, n = (blockIdx.x - head * strips) * 64 + lane;
   const int steps = (Mblk + WEIGHT_STEP - 1) / WEIGHT_STEP;
-  const size_t bh = blockIdx.y;
+  const size_t bh = head;
   if (wave == 0) any[lane] = 0;
   __syncthreads();
   if (n < Nblk) {
@@ -945,12 +955,14 @@ static int complement_bwd_impl(const void* q, const void* k, const void* v, cons
   // per query block dH_i^T = (a_i^T dn_i)^T and dz_i = sum dden a (the state kernel with q, dn in the place of k, v)
   hipLaunchKernelGGL((linear_state_partial_kernel<Tag, D, true, true>), dim3(Mblk, BH), dim3(256), 0, st, (const uint16_t*)q,
                      (const uint16_t*)dn, lay, (void*)dhblk, dzblk, L, BLKQ, fmap, (const float*)dden);
-  // dW, db
-  launch_weight_grads(dtype, D, d_out, y, BH, L, ws + w.wg, d_weight, d_bias, st);
-  // dk, dv
+  // dW, db of every head
+  const HeadSums heads = launch_weight_grads(dtype, D, d_out, y, BH, L, ws + w.wg, d_weight, d_bias, st);
+  // their sum; dk, dv
   uint32_t* const wk = (uint32_t*)(ws + w.fwd.w);
   int* const all = (int*)(ws + w.fwd.all);
-  hipLaunchKernelGGL(complement_column_weights_kernel, dim3(cdiv(N, 64), BH), dim3(512), 0, st, sparse_map, wk, all, Mblk, N);
+  const int strips = cdiv(N, 64);
+  hipLaunchKernelGGL(complement_column_weights_kernel, dim3(strips * BH + cdiv(heads.wgs, 8)), dim3(512), 0, st, sparse_map, wk, all,
+                     Mblk, N, strips, strips * BH, heads);
   launch_states<Tag, D>(dhblk, dzblk, wk, all, gst, gzst, BH, N, Mblk, st);
   const int total_k = BH * N;
   hipLaunchKernelGGL((complement_bwd_kv_kernel<Tag, D>), dim3(xcd_grid(total_k)), dim3(256), 0, st, (const uint16_t*)k,
