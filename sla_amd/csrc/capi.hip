@@ -32,16 +32,16 @@ int side_events_for_current_device(SideEvents** out) {
   SLA_REQUIRE(hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < 64, SLA_ERR_LAUNCH, "no current device");
   SideEvents& e = per_device[dev];
   if (!e.fork) {
-    // all four or none: the set is published only when every event exists
-    hipEvent_t made[4] = {nullptr, nullptr, nullptr, nullptr};
-    for (int i = 0; i < 4; ++i) {
+    // both or none: the set is published only when every event exists
+    hipEvent_t made[2] = {nullptr, nullptr};
+    for (int i = 0; i < 2; ++i) {
       if (hipEventCreateWithFlags(&made[i], hipEventDisableTiming) != hipSuccess) {
         for (int j = 0; j < i; ++j) (void)hipEventDestroy(made[j]);
         set_error("hipEventCreate failed");
         return SLA_ERR_LAUNCH;
       }
     }
-    e = SideEvents{made[0], made[1], made[2], made[3]};
+    e = SideEvents{made[0], made[1]};
   }
   *out = &e;
   return SLA_OK;

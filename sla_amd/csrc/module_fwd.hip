@@ -207,8 +207,8 @@ extern "C" int sla_module_fwd(const void* q, const void* k, const void* v, const
   rc = linear_state_run(kc, vc, lin, weight, dtype, fmap, BH, L, D, (char*)states, parts, side);
   const int rc_mask = mask_given ? (int)SLA_OK
                                  : block_map_run(q, k, lmap, in_dtype, m, BH, L, D, BLKQ, BLKK, topk, sparse_map, lut, lut64, !casts, st);
-  SLA_HIP_OK(hipEventRecord(ev->first, side));
-  SLA_HIP_OK(hipStreamWaitEvent(st, ev->first, 0));
+  SLA_HIP_OK(hipEventRecord(ev->join, side));
+  SLA_HIP_OK(hipStreamWaitEvent(st, ev->join, 0));
   if (rc) return rc;
   if (rc_mask) return rc_mask;
   return attention();

@@ -1113,8 +1113,8 @@ extern "C" int sage_module_fwd(const void* q, const void* k, const void* v, cons
   // (once the second stream waits on `stream`, no path leaves without `stream` waiting for it in turn)
   rc = state(side);
   const int rc_prep = prepare();
-  SLA_HIP_OK(hipEventRecord(ev->first, side));
-  SLA_HIP_OK(hipStreamWaitEvent(st, ev->first, 0));
+  SLA_HIP_OK(hipEventRecord(ev->join, side));
+  SLA_HIP_OK(hipStreamWaitEvent(st, ev->join, 0));
   if (rc) return rc;
   if (rc_prep) return rc_prep;
   return attention();

@@ -9,7 +9,7 @@ namespace sla {
 // One set per device, made on first use and kept.  A call records and waits on them while it holds the lock: calls from
 // several host threads take turns enqueueing.
 struct SideEvents {
-  hipEvent_t fork = nullptr, first = nullptr, second = nullptr, third = nullptr;
+  hipEvent_t fork = nullptr, join = nullptr;
 };
 std::mutex& side_events_mutex();
 int side_events_for_current_device(SideEvents** out);      // (with the lock held)
