@@ -14,8 +14,12 @@
 //              (16x16x32 products, the row spread over 4 lanes), leaves the weighted rows and dq in LDS; then the workgroup
 //              adds the tile's product to M (both operands read transposed from LDS), dz and db on the vector ALU, and
 //              writes the dq rows whole.
-//   The factor 1/den goes, with one rounding to 16 bit, to a at head dim 128 and to G at head dim 64: there a stays the 16-bit
-//   value it is, and in half precision G / den keeps its bits on long sequences, where a / den falls below the format's normal range.
+//   The factor 1/den goes, with one rounding to 16 bit, to a at head dim 128 and to G at head dim 64, where a stays the 16-bit
+//   value it is.  In half precision G / den leaves the format's range: a row whose phi(q) is zero (relu map, padding) has
+//   den = 1e-5, and 0 times an infinite G / den is no number; small gradients over long sequences lose their bits (3 % of d_weight
+//   for G of 1e-4 over 6001 rows).  There G takes a factor between 1/2 and 1 only and a the power of two that is
+//   left: exact, and in range, since a_d / den <= 1 / z_d.  Both are relative to the power of two below the mean of z,
+//   which the partial sums lose again: the sums' bits are those of G / den wherever that is in range.
 //   finish   : fixed-order sums of the slices' partials -> M^T (fp32), dz, db per head, and from them
 //              dS = M W (16 bit, both orientations) and this head's dW = M^T S (fp32)
 #pragma once
@@ -44,6 +48,8 @@ constexpr int LBS_TR = 128;   // rows per step of the stream kernel
 // Bound by the vector ALU in the row phase (30 instructions per element) with one workgroup per compute unit in step between
 // barriers: 12 heads x 32760 x 128, elu map: 137 us with the floats of a row carried along (the compiler then spills what was
 // fetched ahead, waiting for it) and each product waiting for its fragment, now 112.
+// (At head dim 64 the compiler keeps 3 to 8 of a lane's registers in scratch, 11 with the softmax map in bf16 when accumulating.
+// Half precision's two factors: forward and backward of 16 heads x 6001 x 64 188.5 -> 189.1 us, runs of one side differ by 0.3 %.)
 template <typename Tag, int D, int FMAP, bool ACC>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 128 ? 2 : 4, D == 128 ? 2 : 4))) void linear_bwd_stream_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ gout, const uint16_t* __restrict__ kvw,
@@ -59,8 +65,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 128 ? 
   constexpr int NF = CPR / 4;                    // passes of a wave over its own 16 rows
   constexpr int NT = D / 16, NC = D / 32;        // 16-column tiles of a row, 32-column fragments
   constexpr bool WEIGHT_G = D == 64;             // 1 / den goes to G, not to a
+  constexpr bool SPLIT = WEIGHT_G && __is_same(Tag, f16_tag);      // its power of two to a
   constexpr int PSTR = D * 2 + 16;               // row pitch of sP: 16 rows x 16 bytes of a row-wise read cover every bank
-  __shared__ __attribute__((aligned(16))) char smem[3 * TILE + D * PSTR + D * 4 + D * 2 + TR * 4];
+  __shared__ __attribute__((aligned(16))) char smem[3 * TILE + D * PSTR + D * 4 + D * 2 + TR * 4 + (SPLIT ? 16 : 0)];
   char* const sQ = smem;                         // raw q rows, then a (/ den) of the same rows
   char* const sG = smem + TILE;                  // G rows (then G / den)
   char* const sO = smem + 2 * TILE;              // dq rows of this step (16 bit)
@@ -68,6 +75,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 128 ? 
   float* const sZ = reinterpret_cast<float*>(smem + 3 * TILE + D * PSTR);   // z[d1]
   uint16_t* const sZ16 = reinterpret_cast<uint16_t*>(sZ + D);               // the same, as stored
   float* const sDD = reinterpret_cast<float*>(sZ16 + D);                    // weight in dz of the row that sQ then holds
+  float* const sUnit = sDD + TR;                 // SPLIT: the power of two below the mean of z
   float (*sRed)[8][D] = reinterpret_cast<float (*)[8][D]>(smem);            // final sums over the waves (over the tiles)
 
   const int split = blockIdx.x, bh = blockIdx.y, nsplit = gridDim.x;
@@ -109,6 +117,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 128 ? 
       const uint16_t zz = z[(size_t)bh * D + tid];
       sZ[tid] = E::to_float(zz);
       sZ16[tid] = zz;
+      if constexpr (SPLIT) {                     // (the D threads are one wave)
+        float sum = E::to_float(zz);
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) sum += __shfl_xor(sum, o);
+        if (tid == 0) *sUnit = __uint_as_float(__float_as_uint(fminf(fmaxf(sum / D, 0x1p-14f), 0x1p15f)) & 0x7f800000u);
+      }
     }
     // (the first step's barrier stands before the first read of either)
   }
@@ -246,12 +260,28 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 128 ? 
       const float inv_den = 1.0f / (dsum[0] + 1e-5f);
       s = sum_quarters(s);
       const float dden = -s * inv_den * inv_den;
-      if (h == 0) sDD[prow] = WEIGHT_G ? dden : -s * inv_den;     // the weight of what sQ holds (a, or a/den) in dz
+      // SPLIT: unit / den = weight_g * p1 * p2 with powers of two that half precision holds, weight_g in [1/2, 1).  (A row whose
+      // den is below unit / 2^30 counts with that weight.)
+      float weight_g = inv_den, p1 = 1.f, p2 = 1.f, inv_p = 1.f;
+      if constexpr (SPLIT) {
+        const auto inverse = [](float p) __attribute__((always_inline)) { return __uint_as_float(0x7f000000u - __float_as_uint(p)); };
+        const float x = *sUnit * inv_den;
+        const float p = __uint_as_float((__float_as_uint(x) & 0x7f800000u) + 0x00800000u);
+        p1 = fminf(fmaxf(p, 0x1p-14f), 0x1p15f);
+        p2 = fminf(fmaxf(p * inverse(p1), 0x1p-14f), 0x1p15f);
+        inv_p = inverse(p1) * inverse(p2);
+        weight_g = p > 0x1p30f ? 1.f : x * inv_p;
+      }
+      // the weight of what sQ holds (a, a p1 p2 or a/den) in dz
+      if (h == 0) sDD[prow] = SPLIT ? dden * inv_p : WEIGHT_G ? dden : -s * inv_den;
       f32x4_t zz[NT];
+      const auto fetch_z = [&]() __attribute__((always_inline)) {
 #pragma unroll
-      for (int T = 0; T < NT; ++T) zz[T] = *reinterpret_cast<const f32x4_t*>(sZ + 16 * T + 4 * h);
-      __builtin_amdgcn_sched_barrier(0);
-      // a or a/den takes the place of the raw row, G/den that of G (this lane's own places)
+        for (int T = 0; T < NT; ++T) zz[T] = *reinterpret_cast<const f32x4_t*>(sZ + 16 * T + 4 * h);
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      if (!SPLIT) fetch_z();
+      // a (with its power of two) or a/den takes the place of the raw row, G/den (its other factor) that of G (this lane's own places)
 #pragma unroll
       for (int T = 0; T < NT; ++T) {
         i32x2_t w = apk[T];
@@ -259,6 +289,19 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 128 ? 
 #pragma unroll
           for (int j2 = 0; j2 < 2; ++j2)
             w[j2] = (int)E::pack2(unpack_quarter<Tag>(apk[T], 2 * j2) * inv_den, unpack_quarter<Tag>(apk[T], 2 * j2 + 1) * inv_den);
+        if constexpr (SPLIT) {
+          // (finite where a is: only a component in which no key has weight passes the format's largest number, and what it adds
+          //  to the sums meets zeros.  a is not negative, so the patterns are in the values' order.)
+          typedef unsigned short u16x2_t __attribute__((ext_vector_type(2)));
+          const f16x2_t h1 = {(_Float16)p1, (_Float16)p1}, h2 = {(_Float16)p2, (_Float16)p2};
+#pragma unroll
+          for (int j2 = 0; j2 < 2; ++j2) {
+            const int a2 = apk[T][j2];
+            const u16x2_t most = __builtin_elementwise_max(__builtin_bit_cast(u16x2_t, a2), u16x2_t{0x7bff, 0x7bff});
+            const f16x2_t y = __builtin_bit_cast(f16x2_t, a2) * h1 * h2;
+            w[j2] = __builtin_bit_cast(int, __builtin_elementwise_min(__builtin_bit_cast(u16x2_t, y), most));
+          }
+        }
         *reinterpret_cast<i32x2_t*>(sQ + acc_off(T)) = w;
       }
       if (WEIGHT_G)
@@ -268,9 +311,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 128 ? 
           i32x4_t w;
 #pragma unroll
           for (int j = 0; j < 4; ++j)
-            w[j] = (int)E::pack2(E::to_float((uint16_t)gr[2 * j]) * inv_den, E::to_float((uint16_t)gr[2 * j + 1]) * inv_den);
+            w[j] = (int)E::pack2(E::to_float((uint16_t)gr[2 * j]) * weight_g, E::to_float((uint16_t)gr[2 * j + 1]) * weight_g);
           *reinterpret_cast<i32x4_t*>(sG + g_off(c)) = w;
         }
+      if (SPLIT) fetch_z();
       // da = t / den + dden z (in place), then dq = phi'(q) da
 #pragma unroll
       for (int T = 0; T < NT; ++T)
@@ -320,6 +364,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 128 ? 
   flush_dq(row_begin + (row_end - 1 - row_begin) / TR * TR);
 
   // M^T partial [e][d1] (accumulator rows = d1, columns = e), fp32
+  const float unscale = SPLIT ? 1.f / *sUnit : 1.f;
   const size_t pidx = (size_t)bh * nsplit + split;
   float* mo = m_part + pidx * D * D;
 #pragma unroll
@@ -327,7 +372,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 128 ? 
     const int col = MW * (nt0 + t2) + (lane & (MW - 1));
 #pragma unroll
     for (int i4 = 0; i4 < MR / 4; ++i4) {
-      const f32x4_t v4 = {macc[t2][4 * i4], macc[t2][4 * i4 + 1], macc[t2][4 * i4 + 2], macc[t2][4 * i4 + 3]};
+      f32x4_t v4 = {macc[t2][4 * i4], macc[t2][4 * i4 + 1], macc[t2][4 * i4 + 2], macc[t2][4 * i4 + 3]};
+      if (SPLIT) v4 *= unscale;
       *reinterpret_cast<f32x4_t*>(mo + (size_t)col * D + MW * mt + 8 * i4 + 4 * (D == 128 ? g2 : h)) = v4;
     }
   }
