@@ -452,6 +452,10 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
   if (slot >= 0) {
     // One segment of a long list: fp32 partial [dk | dv][64][D].  The workgroup that finishes a key block's last segment adds
     // all of them up, in segment order: its count is raised only when a workgroup's whole partial is visible to the others.
+    // (One thread releases, behind the barrier, for both waves, and only the last one of a key block acquires: a release writes
+    // an XCD's modified lines back.  With both fences in every thread of every segment, and the sums four values of a thread
+    // at a time, this kernel took 437 us at 2 heads x 75600 x 64 and 718 at 2 x 75600 x 128, now 372 and 658; with the sums in a
+    // launch of their own 356 + 14 and 612 + 24, and 4 to 5 us more where no list is cut.)
     float* pk = part + (size_t)slot * (2 * 64 * D) + (size_t)(w * 32 + r) * D;
     float* pv = pk + 64 * D;
 #pragma unroll
@@ -464,21 +468,38 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
         *reinterpret_cast<f32x4_t*>(pv + d0) =
             f32x4_t{dvacc[dt][4 * i4 + 0], dvacc[dt][4 * i4 + 1], dvacc[dt][4 * i4 + 2], dvacc[dt][4 * i4 + 3]};
       }
-    __threadfence();
     __syncthreads();
     const int ns = nseg[(size_t)bh * Nblk + nb];
-    if (tid == 0) entries[0] = atomicAdd(&done[(size_t)bh * Nblk + nb], 1);
+    if (tid == 0) {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+      entries[0] = atomicAdd(&done[(size_t)bh * Nblk + nb], 1);
+      if (entries[0] == ns - 1) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    }
     __syncthreads();
     if (entries[0] != ns - 1) return;
-    __threadfence();
     const float* p0 = part + (size_t)(slot - sg) * (2 * 64 * D);
-    for (int idx = tid * 4; idx < 2 * 64 * D; idx += 128 * 4) {
-      f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-      for (int x = 0; x < ns; ++x) acc += *reinterpret_cast<const f32x4_t*>(p0 + (size_t)x * (2 * 64 * D) + idx);
-      const int which = idx / (64 * D), rem = idx - which * (64 * D);
-      const int row = nb * 64 + rem / D, col = rem % D;
-      if (row < L) store_4<E>((which ? dv : dk) + head_off + (size_t)row * pitch + col, acc[0], acc[1], acc[2], acc[3], add);
+    // (all of a thread's loads of a segment's dK or dV in flight at once)
+    constexpr int NV = 64 * D / 4 / 128;
+#pragma unroll
+    for (int which = 0; which < 2; ++which) {
+      f32x4_t acc[NV];
+#pragma unroll
+      for (int i = 0; i < NV; ++i) acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      const float* p = p0 + which * (64 * D) + tid * 4;
+      for (int x = 0; x < ns; ++x, p += 2 * 64 * D) {
+        f32x4_t b[NV];
+#pragma unroll
+        for (int i = 0; i < NV; ++i) b[i] = *reinterpret_cast<const f32x4_t*>(p + i * 512);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < NV; ++i) acc[i] += b[i];
+      }
+#pragma unroll
+      for (int i = 0; i < NV; ++i) {
+        const int idx = tid * 4 + i * 512, row = nb * 64 + idx / D;
+        if (row < L)
+          store_4<E>((which ? dv : dk) + head_off + (size_t)row * pitch + idx % D, acc[i][0], acc[i][1], acc[i][2], acc[i][3], add);
+      }
     }
     return;
   }
