@@ -452,8 +452,8 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
   if (slot >= 0) {
     // One segment of a long list: fp32 partial [dk | dv][64][D].  The workgroup that finishes a key block's last segment adds
     // all of them up, in segment order: its count is raised only when a workgroup's whole partial is visible to the others.
-    // (One thread releases, behind the barrier, for both waves, and only the last one of a key block acquires: a release writes
-    // an XCD's modified lines back.  With both fences in every thread of every segment, and the sums four values of a thread
+    // (One thread releases, behind the barrier, for both waves, and only the last workgroup of a key block acquires: a release
+    // writes an XCD's modified lines back.  With both fences in every thread of every segment, and the sums four values of a thread
     // at a time, this kernel took 437 us at 2 heads x 75600 x 64 and 718 at 2 x 75600 x 128, now 372 and 658; with the sums in a
     // launch of their own 356 + 14 and 612 + 24, and 4 to 5 us more where no list is cut.)
     float* pk = part + (size_t)slot * (2 * 64 * D) + (size_t)(w * 32 + r) * D;
@@ -468,15 +468,16 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
         *reinterpret_cast<f32x4_t*>(pv + d0) =
             f32x4_t{dvacc[dt][4 * i4 + 0], dvacc[dt][4 * i4 + 1], dvacc[dt][4 * i4 + 2], dvacc[dt][4 * i4 + 3]};
       }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // (the barrier alone does not wait for a wave's stores)
     __syncthreads();
     const int ns = nseg[(size_t)bh * Nblk + nb];
     if (tid == 0) {
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
       entries[0] = atomicAdd(&done[(size_t)bh * Nblk + nb], 1);
-      if (entries[0] == ns - 1) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     }
     __syncthreads();
     if (entries[0] != ns - 1) return;
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     const float* p0 = part + (size_t)(slot - sg) * (2 * 64 * D);
     // (all of a thread's loads of a segment's dK or dV in flight at once)
     constexpr int NV = 64 * D / 4 / 128;
