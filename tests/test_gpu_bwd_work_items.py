@@ -39,6 +39,34 @@ def test_gradients_over_all_pairs(dev, H, N, T):
             assert bool((err <= 4 * 2.0 ** -9 * r.flatten(1).norm(dim=1).clamp_min(1e-3) + 1e-3).all()), (name, h0, err.max().item())
 
 
+@pytest.mark.parametrize("N", [15, 16, 17, 33, 63, 65, 79, 81, 127])
+def test_lists_of_maps_of_any_width(dev, N):
+    """Key-block counts around the 16 bytes and the 64 columns the lists are read in, and maps that start at any byte."""
+    from sla_amd.sparse_attn import sparse_attn_bwd, sparse_attn_fwd
+    H, D, L, T = 2, 64, 64 * N - 9, 5
+    g = torch.Generator(device=dev).manual_seed(N)
+    q, k, v, do = (torch.randn(1, H, L, D, device=dev, generator=g).bfloat16() for _ in range(4))
+    lut = torch.rand(1, H, N, N, device=dev, generator=g).argsort(-1)[..., :T].sort(-1).values.contiguous()
+    smap = torch.zeros(1, H, N, N, dtype=torch.int8, device=dev).scatter_(3, lut, 1)
+    lut = lut.int()
+    scale = D ** -0.5
+    o, lse = sparse_attn_fwd(q, k, v, lut, T, 64, 64, scale)
+    got = sparse_attn_bwd(q, k, v, o, do, lse, smap, lut, T, 64, 64, scale)
+    mask = smap[0].bool().repeat_interleave(64, 1).repeat_interleave(64, 2)[:, :L, :L]
+    qf, kf, vf = (t[0].float().requires_grad_(True) for t in (q, k, v))
+    s = (torch.bmm(qf, kf.transpose(1, 2).contiguous()) * scale).masked_fill(~mask, float("-inf"))
+    ref = torch.autograd.grad(torch.bmm(torch.softmax(s, -1), vf), (qf, kf, vf), do[0].float())
+    for name, a, r in zip("qkv", got, ref):
+        # (as above)
+        err = (a[0].float() - r).flatten(1).norm(dim=1)
+        assert bool((err <= 4 * 2.0 ** -9 * r.flatten(1).norm(dim=1).clamp_min(1e-3) + 1e-3).all()), (name, err.max().item())
+    for first in (1, 6, 15):
+        moved = torch.ones(smap.numel() + 16, dtype=torch.int8, device=dev)[first:first + smap.numel()].view_as(smap)
+        moved.copy_(smap)
+        for a, r in zip(sparse_attn_bwd(q, k, v, o, do, lse, moved, lut, T, 64, 64, scale), got):
+            assert torch.equal(a, r), first
+
+
 @pytest.mark.parametrize("H,L", [(2, 8320), (1, 4161)])
 def test_added_to_what_the_gradients_hold(dev, H, L):
     """A whole backward over lists in segments equals the attention's gradients plus the linear branch's, bit for bit."""
