@@ -885,7 +885,14 @@ extern "C" int sage_sparse_attn_fwd(const int8_t* q_int8, const float* q_scale, 
 //   q quantised (with its block means), chunk sums of k | slices' partial states (with the maxima of |v|), column mean of k |
 //   states finished, k quantised (with its block means), v quantised | scores and selection
 // Eleven launches of 2 to 12 us were what a call on 16 heads x 5003 x 64 consisted of besides its attention: 54 us in eight, now 36 in three.
+// On one stream from ONE_STREAM_STEPS_BYTES per tensor on the separate calls, whose passes are shaped for memory alone: they load 16
+// bytes per lane, and v's scales are formed once, not by every workgroup of v.  Captured forward, us, this form / separate calls: 2 heads x
+// 75600 x 64 (18 MiB) 245 / 252, 12 x 6500 x 128 (19 MiB) 137 / 147, 8 x 16000 x 128 (31 MiB) 233 / 224, 40 x 6500 x 64 (32 MiB) 172 /
+// 172, 12 x 12000 x 128 and 24 x 12000 x 64 (35 MiB) 212 / 219 and 210 / 220, 2 x 75600 x 128 (37 MiB) 383 / 362, 12 x 16000 x 128 (47 MiB)
+// 291 / 280, 40 x 10000 x 64 (49 MiB) 269 / 254, 32 x 16000 x 64 (62 MiB) 383 / 381, 40 x 32760 x 128 (320 MiB) 2467 / 2262.
 namespace sla {
+
+constexpr int64_t ONE_STREAM_STEPS_BYTES = 36ll << 20;
 
 template <typename Tag>
 struct IoOf;
@@ -1090,6 +1097,11 @@ extern "C" int sage_module_fwd(const void* q, const void* k, const void* v, cons
     return sage_attention_run(q8, qs, k8, ks, v8, vs, lut, 0, out, dtype, B * H, L, D, topk, qk_scale, &lin, st);
   };
   if (!side || side == st || !side_stream_pays(B, H, L, D, topk)) {
+    if ((int64_t)B * H * L * D * 2 >= ONE_STREAM_STEPS_BYTES) {
+      if ((rc = state(st))) return rc;
+      if ((rc = prepare())) return rc;
+      return attention();
+    }
     SLA_REQUIRE(w.linear_bytes >= linear_fwd_workspace_bytes(B * H, L, D), SLA_ERR_WORKSPACE, "workspace too small");
 #define SAGE_SMALL_CASE(TAG, DD)                                                                                              \
   launch_small_preparation<TAG, DD>(q, k, v, lq, dtype, weight, fmap, B * H, L, topk, lut, q8, qs, k8, ks, v8, vs, v_range, \

@@ -58,3 +58,29 @@ def test_quantised_forward_equals_the_steps(dev, H, L, D, fmap, half):
         ws, v8, vs = linear_state_quant_v_fwd(k, v, mod.proj_l.weight, fmap)
         o_s = sage_attn_fwd(q8, qs, k8, ks, v8, vs, lut, T, dtype)
         assert torch.equal(mod(q, k, v), linear_out_fwd(q, mod.proj_l.bias, o_s, ws, fmap))
+
+
+@pytest.mark.parametrize("H,L,D,fmap,half", [(12, 12287, 128, "elu", False), (12, 12288, 128, "softmax", False), (24, 12289, 64, "relu", True)])
+def test_quantised_forward_on_one_stream_equals_the_steps(dev, H, L, D, fmap, half):
+    """On either side of the size (36 MiB per tensor) from which the preparation on one stream, here a capturing one, is the separate
+    calls' again; replayed several times with eager work between."""
+    from sla_amd import SageSparseLinearAttention
+    dtype = torch.float16 if half else torch.bfloat16
+    g = torch.Generator(device=dev).manual_seed(L + D)
+    q, k, v = (torch.randn(1, H, L, D, device=dev, generator=g).to(dtype) for _ in range(3))
+    mod = SageSparseLinearAttention(D, 0.05, fmap, use_bf16=not half).to(dev)
+    with torch.no_grad():
+        for p, t in zip((mod.proj_l.weight, mod.proj_l.bias), make_proj(D)):
+            p.copy_(t)
+        ref = mod(q, k, v)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = mod(q, k, v)
+        for _ in range(3):
+            out.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, ref)
+            assert torch.equal(mod(q, k, v), ref)
+            torch.cuda.synchronize()
