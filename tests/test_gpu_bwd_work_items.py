@@ -88,3 +88,48 @@ def test_added_to_what_the_gradients_hold(dev, H, L):
         got = module_bwd(q, k, v, o, do, lse, smap, lut, T, 64, 64, D ** -0.5, w, b, "elu")
         for a, r in zip(got, ref):
             assert torch.equal(a, r)
+
+
+@pytest.mark.parametrize("D,BLKQ", [(64, 64), (128, 64), (64, 128)])
+def test_rows_too_far_apart_for_the_stream_kernels(dev, D, BLKQ):
+    """Heads that span 2 GiB (one buffer of very long rows) go through the general dQ and dK/dV kernels and the sums behind them:
+    against dense attention, and a whole backward against the attention's gradients plus the linear branch's, bit for bit.  Every
+    row selects key block 0, so that with 64-row blocks its list is cut."""
+    from sla_amd.inputs import make_proj
+    from sla_amd.linear import linear_bwd
+    from sla_amd.module import module_bwd
+    from sla_amd.sparse_attn import sparse_attn_bwd, sparse_attn_fwd
+    H, L, T = 2, 4161, 2
+    M, N, R = -(-L // BLKQ), -(-L // 64), (2 ** 30 // L + 8) // 8 * 8
+    assert 2 * L * R >= 2 ** 31
+
+    def views(buf):
+        return [buf.as_strided((1, H, L, D), (L * R, D, R, 1), i * H * D) for i in range(3)]
+
+    g = torch.Generator(device=dev).manual_seed(D + BLKQ)
+    q, k, v, do = (torch.randn(1, H, L, D, device=dev, generator=g).bfloat16() for _ in range(4))
+    w, b = (t.to(dev) for t in make_proj(D))
+    lut = torch.stack([torch.zeros(M, dtype=torch.long), 1 + torch.arange(M) % (N - 1)], 1).to(dev).expand(1, H, M, T).contiguous()
+    smap = torch.zeros(1, H, M, N, dtype=torch.int8, device=dev).scatter_(3, lut, 1)
+    lut = lut.int()
+    scale = D ** -0.5
+    o, lse = sparse_attn_fwd(q, k, v, lut, T, BLKQ, 64, scale)
+    wide = views(torch.empty(L * R, dtype=torch.bfloat16, device=dev))
+    for x, t in zip(wide, (q, k, v)):
+        x.copy_(t)
+    grads = views(torch.full((L * R,), float("nan"), dtype=torch.bfloat16, device=dev))
+    sparse_attn_bwd(*wide, o, do, lse, smap, lut, T, BLKQ, 64, scale, grads=grads)
+    mask = smap[0].bool().repeat_interleave(BLKQ, 1).repeat_interleave(64, 2)[:, :L, :L]
+    qf, kf, vf = (t[0].float().requires_grad_(True) for t in (q, k, v))
+    s = (torch.bmm(qf, kf.transpose(1, 2).contiguous()) * scale).masked_fill(~mask, float("-inf"))
+    ref = torch.autograd.grad(torch.bmm(torch.softmax(s, -1), vf), (qf, kf, vf), do[0].float())
+    for name, a, r in zip("qkv", grads, ref):
+        # (as above)
+        err = (a[0].float() - r).flatten(1).norm(dim=1)
+        assert bool((err <= 4 * 2.0 ** -9 * r.flatten(1).norm(dim=1).clamp_min(1e-3) + 1e-3).all()), (name, err.max().item())
+    ref = [t.contiguous() for t in linear_bwd(*wide, w, b, do, "elu", accumulate_into=grads)]
+    for t in grads:
+        t.fill_(float("nan"))
+    got = module_bwd(*wide, o, do, lse, smap, lut, T, BLKQ, 64, scale, w, b, "elu", grads=grads)
+    for a, r in zip(got, ref):
+        assert torch.equal(a, r)
