@@ -124,8 +124,8 @@ def test_training_step_in_a_hip_graph(dev):
 @pytest.mark.parametrize("with_states", [False, True])
 @pytest.mark.parametrize("dtype,L,D,BLKQ", [(torch.bfloat16, 2100, 128, 64), (torch.float16, 1000, 64, 128)])
 def test_one_call_backward_equals_the_two_calls(dev, layout, with_states, dtype, L, D, BLKQ):
-    """sla_module_bwd, on one stream and with the short kernels on a second one, against sla_sparse_attn_bwd followed
-    by the accumulating sla_linear_bwd: the same bits.  Ran twice with the side stream (the events are reused)."""
+    """sla_module_bwd against sla_sparse_attn_bwd followed by the accumulating sla_linear_bwd: the same bits, call after call; a side
+    stream that is handed over receives no work (it is idle while the main stream still holds the call back)."""
     from sla_amd import get_block_map
     from sla_amd.linear import linear_bwd, linear_state_fwd, saved_states
     from sla_amd.module import module_bwd
@@ -158,8 +158,12 @@ def test_one_call_backward_equals_the_two_calls(dev, layout, with_states, dtype,
     side = torch.cuda.Stream(device=dev)
     for side_stream in (None, side, side):
         _, grads = new_grads()
+        torch.cuda.synchronize()
+        torch.cuda._sleep(10_000_000)
         out = module_bwd(q, k, v, o_s, d_out, lse, sparse_map, lut, topk, BLKQ, 64, D ** -0.5, w, b, fmap, states=states,
                          grads=grads, side_stream=side_stream)
+        busy, idle = not torch.cuda.current_stream(dev).query(), side.query()
         torch.cuda.synchronize()
+        assert busy and idle
         for name, a, r in zip(("dq", "dk", "dv", "dW", "db"), out, (*ref, dw_ref, db_ref)):
             assert torch.equal(a, r), (name, side_stream is not None)
