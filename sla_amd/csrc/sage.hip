@@ -1102,7 +1102,6 @@ extern "C" int sage_module_fwd(const void* q, const void* k, const void* v, cons
       if ((rc = prepare())) return rc;
       return attention();
     }
-    SLA_REQUIRE(w.linear_bytes >= linear_fwd_workspace_bytes(B * H, L, D), SLA_ERR_WORKSPACE, "workspace too small");
 #define SAGE_SMALL_CASE(TAG, DD)                                                                                              \
   launch_small_preparation<TAG, DD>(q, k, v, lq, dtype, weight, fmap, B * H, L, topk, lut, q8, qs, k8, ks, v8, vs, v_range, \
                                     ws + w.prep, ws + w.linear, st)
