@@ -106,11 +106,15 @@ static int linear_bwd_impl(const void* q, const void* k, const void* v, const fl
     SLA_LB_FMAPS(SLA_LBS_LAUNCH)
 #undef SLA_LBS_LAUNCH
   }
+  const bool presum = w.sp.nsplit >= PRESUM_MIN_SLICES;
+  if ((steps & LB_REDUCE) && presum)
+    hipLaunchKernelGGL((linear_state_presum_kernel<D>), dim3(D * D / 256 + 2, BH), dim3(512), 0, st, m_part, (float*)(ws + w.dz_part),
+                       (float*)(ws + w.db_part), w.sp.nsplit);
   if (steps & LB_REDUCE)
     hipLaunchKernelGGL((linear_bwd_finish_kernel<Tag, D>), dim3(xcd_grid(lists.wgs) + xcd_grid((int64_t)BH * (D / 8))), dim3(512),
                        0, st, (const float*)m_part, (const float*)(ws + w.dz_part), (const float*)(ws + w.db_part), weight, kvt,
                        (uint16_t*)(ws + w.ds), (uint16_t*)(ws + w.dst), (float*)(ws + w.dz), (float*)(ws + w.dw_head),
-                       (float*)(ws + w.db_head), w.sp.nsplit, BH * (D / 8), xcd_grid(lists.wgs), lists);
+                       (float*)(ws + w.db_head), w.sp.nsplit, presum ? 1 : w.sp.nsplit, BH * (D / 8), xcd_grid(lists.wgs), lists);
   if (steps & LB_HEADS) launch_head_sums(hs, st);
   if (steps & LB_KEYS) {
 #define SLA_LBK_LAUNCH(FM, ACC)                                                                                          \

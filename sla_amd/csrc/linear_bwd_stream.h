@@ -581,14 +581,18 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 128 ? 
 // Either way it holds all its products need of M after one hand-over through LDS; the partials are read twice, from the
 // caches.  The slices are summed in two halves side by side, whose sums are then added, eight slices' loads in flight.
 // Against a kernel for the sums and one for the products (on the vector ALU, M through memory in both orientations): 9.3
-// against 12.8 + 10.5 us (B2 H4 L4096).  The first `first_wg` workgroups, a multiple of eight, build the lists of the map for
+// against 12.8 + 10.5 us (B2 H4 L4096).  With many slices of few heads linear_state_presum_kernel has added them up before (the same
+// bits): 1 head x 75600 x 128 (197 slices) 45.9 us without it, 6.1 + 21.4 with it, the latter the lists' time; 2 heads x 20000 x 128 (79)
+// 21.7 and 4.8 + 8.6.  Forward and backward: 1 x 75600 x 128 930 -> 916 us, 4 x 40000 x 64 556 -> 546, 2 x 20000 x 128 382 -> 372, 1 x 8000
+// x 128 (63) 227 -> 217, 12 x 20000 x 64 (42) 461 -> 457.  The first `first_wg` workgroups, a multiple of eight, build the lists of the map for
 // the attention backward: both are short and bound by latency.
 template <typename Tag, int D>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void linear_bwd_finish_kernel(
     const float* __restrict__ m_part, const float* __restrict__ dz_part, const float* __restrict__ db_part,
     const float* __restrict__ weight, const uint16_t* __restrict__ kvt, uint16_t* __restrict__ ds, uint16_t* __restrict__ dst,
-    float* __restrict__ dz, float* __restrict__ dw_head, float* __restrict__ db_head, int nsplit, int total, int first_wg,
-    const ColLists lists) {
+    float* __restrict__ dz, float* __restrict__ dw_head, float* __restrict__ db_head, int nsplit, int nsum, int total,
+    int first_wg, const ColLists lists) {
+  // (nsum: the slices to add up, all nsplit of a head or the first one alone, which then holds the sums)
   using E = Elem<Tag>;
   constexpr int DD = D * D;
   constexpr int NR = D / 64;               // f32x4 sums per thread
@@ -608,7 +612,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void l
   const int bh = logical / (D / 8), rest = logical % (D / 8), kind = rest / (D / 16), i0 = 16 * (rest % (D / 16));
   const int tid = threadIdx.x & 255, half = threadIdx.x >> 8, lane = tid & 63, wave = threadIdx.x >> 6;
   const int l = lane & 15, h = lane >> 4;
-  const int n0 = (nsplit + 1) >> 1;
+  const int n0 = (nsum + 1) >> 1;
   const float* mp = m_part + (size_t)bh * nsplit * DD;
   const int er = kind == 0 ? tid >> 2 : tid >> 4, dc = kind == 0 ? 4 * (tid & 3) : 4 * (tid & 15);
   mp += kind == 0 ? (size_t)er * D + i0 + dc : (size_t)(i0 + er) * D + dc;
@@ -616,7 +620,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void l
   f32x4_t acc[NR];
 #pragma unroll
   for (int i = 0; i < NR; ++i) acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  sum_slices<NR>(mp + (half ? (size_t)n0 * DD : 0), half ? nsplit - n0 : n0, DD, vec, acc);
+  sum_slices<NR>(mp + (half ? (size_t)n0 * DD : 0), half ? nsum - n0 : n0, DD, vec, acc);
   if (half)
 #pragma unroll
     for (int i = 0; i < NR; ++i) *reinterpret_cast<f32x4_t*>(s_half + (i * 256 + tid) * 4) = acc[i];
@@ -624,7 +628,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void l
     const float* q = (tid < 16 ? dz_part : db_part) + (size_t)bh * nsplit * D + i0 + (tid & 15);
     float sum = 0.f;
 #pragma unroll 8
-    for (int sp = 0; sp < nsplit; ++sp) sum += q[(size_t)sp * D];
+    for (int sp = 0; sp < nsum; ++sp) sum += q[(size_t)sp * D];
     (tid < 16 ? dz : db_head)[(size_t)bh * D + i0 + (tid & 15)] = sum;
   }
   __syncthreads();

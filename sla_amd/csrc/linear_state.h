@@ -305,13 +305,14 @@ static __device__ __forceinline__ void sum_slices(const float* __restrict__ p, i
 
 // The same sums in a launch of their own, left in the place of every head's first slice, with the same bits.  The kernel
 // below has D / 16 workgroups per head: few heads with many slices leave it reading on a few compute units.  Here a workgroup
-// of 512 threads takes 256 elements, its halves one half of the slices each, 32 loads in flight; the last one of a head takes z.
+// of 512 threads takes 256 elements, its halves one half of the slices each, 32 loads in flight; the last one of a head takes z,
+// another one behind it (the backward's sums have one) a second vector.
 // Bound by latency.  State build in us without this launch and with it: 1 head x 75600 x 128 (295 slices) 88.6 / 35.8, 2 heads
 // x 75600 x 128 (256) 78.4 / 41.4, 4 heads x 32760 x 128 (128) 53.9 / 37.9, 8 heads x 16384 x 64 (64) 23.2 / 19.9, 12 heads x
 // 24576 x 128 (42) 62.3 / 58.9, 16 heads x 16384 x 128 (32) 53.0 / 53.6, 2 heads x 4096 x 64 (16) 14.2 / 15.7.
 template <int D>
 __global__ __launch_bounds__(512) void linear_state_presum_kernel(float* __restrict__ kv_part, float* __restrict__ z_part,
-                                                                  int nsplit) {
+                                                                  float* __restrict__ z2_part, int nsplit) {
   constexpr int DD = D * D, BATCH = 32;
   __shared__ float s_half[256];
   const int bh = blockIdx.y, tid = threadIdx.x & 255, half = threadIdx.x >> 8;
@@ -328,8 +329,8 @@ __global__ __launch_bounds__(512) void linear_state_presum_kernel(float* __restr
     }
     return acc;
   };
-  if (blockIdx.x == DD / 256) {
-    float* p = z_part + (size_t)bh * nsplit * D + threadIdx.x;
+  if (blockIdx.x >= DD / 256) {
+    float* p = (blockIdx.x == DD / 256 ? z_part : z2_part) + (size_t)bh * nsplit * D + threadIdx.x;
     if (threadIdx.x < D) *p = sum(p, nsplit, D);
     return;
   }
@@ -491,7 +492,7 @@ template <int D>
 static inline void launch_state_presum(int BH, char* parts, const LinWs& w, hipStream_t st) {
   if (w.nsplit >= PRESUM_MIN_SLICES)
     hipLaunchKernelGGL((linear_state_presum_kernel<D>), dim3(D * D / 256 + 1, BH), dim3(512), 0, st,
-                       (float*)(parts + (w.kv_part - w.states_end)), (float*)(parts + (w.z_part - w.states_end)), w.nsplit);
+                       (float*)(parts + (w.kv_part - w.states_end)), (float*)(parts + (w.z_part - w.states_end)), nullptr, w.nsplit);
 }
 template <typename Tag, int D>
 static inline void launch_state_finish(const float* weight, int BH, char* ws, char* parts, const LinWs& w, hipStream_t st) {

@@ -123,3 +123,20 @@ def test_weight_gradients_of_small_and_large_gradients(dev, dtype, fmap, L, scal
         # (as above)
         bound = 8 * u * (ref[i].norm() + mag[i].norm())
         assert (got[i].double() - ref[i]).norm() <= bound, (i, ((got[i].double() - ref[i]).norm() / bound).item())
+
+
+@pytest.mark.parametrize("L", [4992, 4993, 9990])
+@pytest.mark.parametrize("D,dtype", [(64, torch.float16), (128, torch.bfloat16)])
+def test_sums_over_many_slices(dev, D, dtype, L):
+    """39, 40 and 79 slices of 128 rows: from 40 on a launch of its own adds the slices' sums up."""
+    from sla_amd.linear import linear_bwd
+    B, H = 1, 2
+    gen = torch.Generator(device=dev).manual_seed(L)
+    q, k, v, do = (torch.randn(B, H, L, D, device=dev, generator=gen).to(dtype) for _ in range(4))
+    w, b = (t.to(dev) for t in make_proj(D))
+    got = linear_bwd(q, k, v, w, b, do, "softmax")
+    ref, mag = _float64(q, k, v, w, do, "softmax")
+    u = 2.0 ** (-9 if dtype == torch.bfloat16 else -12)
+    for i, (g, r, m) in enumerate(zip(got, ref, mag)):
+        # (as above; the sums over the rows are in 32 bits)
+        assert (g.double() - r).norm() <= 8 * u * (r.norm() + m.norm()), i
