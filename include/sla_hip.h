@@ -202,9 +202,9 @@ int sla_sparse_attn_linear_fwd_strided(const void* q, const void* k, const void*
                                        const int64_t* out_strides, float* lse, int dtype, int fmap, int B, int H, int L,
                                        int D, int BLKQ, int BLKK, int topk, float qk_scale, void* stream);
 
-/* Backward of the whole module in one call: the kernels of sla_sparse_attn_bwd(_strided) followed by those of
- * sla_linear_bwd(_strided) with SLA_BWD_ACCUMULATE (the linear branch adds into dq, dk, dv), results equal to those two
- * calls bit for bit (the linear branch's kernels come first, and the attention kernels add).  The only flag is
+/* Backward of the whole module in one call: the kernels of sla_linear_bwd(_strided), which write dq, dk, dv, then those of
+ * sla_sparse_attn_bwd(_strided), which add to them.  Results equal sla_sparse_attn_bwd followed by sla_linear_bwd with
+ * SLA_BWD_ACCUMULATE bit for bit (a sum of the same two 16-bit values).  The only flag is
  * SLA_BWD_STATES_READY.  qkv_strides / do_strides: both NULL for contiguous (B, H, L, D) tensors, else as in the strided
  * calls.  o_s is the attention output the forward saved.  The two workspaces are those of the two calls
  * (SLA_WS_SPARSE_BWD, SLA_WS_LINEAR_BWD).

@@ -7,7 +7,8 @@
 //   H_i = sum_j h_j - sum_{j in S_i} h_j,   z_i likewise              per query block i
 //   o_l = phi(Q_i) H_i / (1e-5 + phi(Q_i) . z_i);  out = residual + o_l W^T + b
 // Rounding: phi, h_j, H_i, z_i, o_l are rounded to the 16-bit dtype where the global path rounds its
-// counterparts; all sums of states are fp32 in a fixed order (ascending j, then the look-up row in order).
+// counterparts; a state is one fp32 accumulation over the blocks that take part, in ascending order (H_i is formed as the sum over
+// the j outside S_i, nothing is subtracted).
 //
 // Kernels:
 //   block states : linear_state_partial_kernel with one 64-row slice per workgroup, 16-bit h_j^T, fp32 z_j

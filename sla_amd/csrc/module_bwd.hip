@@ -8,7 +8,10 @@
 // The linear branch comes first and writes dq, dk, dv; the attention kernels, which have arithmetic to do meanwhile, read and
 // add.  (The other way round the memory-bound kernels read them: 125 + 108 us for the two at B1 H12 L32760 D128, now 112 + 83.)
 // Five launches where there were ten: B2 H4 L4096 D128 forward and backward 215 -> 195 us; the longest calls run against the
-// power limit in the attention kernels, whatever the others take (40 heads x 75600: 26.0 ms either way).
+// power limit in the attention kernels, whatever the others take (40 heads x 75600: 26.0 ms either way).  More than five: from 40 slices
+// of the sequence per head on their sums are added up first; where the general dQ kernel runs (fewer than 320 query blocks of 64
+// rows, or 512 of 128), delta and the short jobs have a launch each, and the sums behind the general dK/dV kernel another; states
+// that the caller does not have are built before everything else.
 // The results equal the two separate calls, the linear one accumulating into the other's gradients, bit for bit.
 #include "bwd_steps.h"
 

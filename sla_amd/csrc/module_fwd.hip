@@ -6,7 +6,8 @@
 //     block means of q, chunk sums of k [fp32 inputs: and the 16-bit copies] | slices' partial states, column mean of k |
 //     states finished, block means of k | scores and selection | attention
 // (five launches; in eight of their own, and seven with 16-bit inputs, everything before the attention took 34 us for 2 heads x
-// 1024 x 64 in fp32, 57 for 8 x 4096 x 128: now 25 and 43.)
+// 1024 x 64 in fp32, 57 for 8 x 4096 x 128: now 25 and 43.  A sixth adds up the slices' states from 40 slices per head on; scores and
+// selection are two where a row's scores go through memory.)
 // From 64 MiB per tensor on the state build (k, v only) runs on the caller's second stream beside the mask builder instead.
 #include "block_pool.h"
 #include "fwd_steps.h"

@@ -533,7 +533,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 3
 
 // ---- host ---------------------------------------------------------------------------------
 // list[bh][n][0..count[bh][n]) = the query blocks that selected key block n, ascending; capacity Mblk per list
-// (also used by the backward of the complement-mode linear branch)
 static void launch_col_lists(const int8_t* sparse_map, int* list, int* count, int BH, int Mblk, int Nblk, hipStream_t st) {
   const ColLists job = col_lists_job(sparse_map, list, count, BH, Mblk, Nblk);
   hipLaunchKernelGGL(bwd_col_lists_kernel, dim3(job.wgs), dim3(64 * COL_NW), 0, st, job);
