@@ -10,6 +10,7 @@
 // Kernels (linear_bwd_stream.h, linear_state.h):
 //   state build (shared with the forward) : S and z again from k, v
 //   stream : q and G once: dq, and per slice of the sequence the partial sums M^T, dz, db
+//   presum : many slices of few heads added up first
 //   finish : those sums added up -> dS (16 bit, both orientations), dz, per-head dW, db
 //   heads  : the heads' dW and db added up
 //   keys   : k and v once: dk, dv
@@ -106,6 +107,7 @@ static int linear_bwd_impl(const void* q, const void* k, const void* v, const fl
     SLA_LB_FMAPS(SLA_LBS_LAUNCH)
 #undef SLA_LBS_LAUNCH
   }
+  // (the line of the forward's states; both sides measured at linear_bwd_finish_kernel)
   const bool presum = w.sp.nsplit >= PRESUM_MIN_SLICES;
   if ((steps & LB_REDUCE) && presum)
     hipLaunchKernelGGL((linear_state_presum_kernel<D>), dim3(D * D / 256 + 2, BH), dim3(512), 0, st, m_part, (float*)(ws + w.dz_part),
