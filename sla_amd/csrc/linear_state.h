@@ -474,11 +474,7 @@ static inline LinWs lin_ws(int BH, int L, int D) {
   const int min_rows = L >= 4096 ? 256 : cdiv(L, 16);
   const int slots = (int64_t)BH * L * D <= (64ll << 20) ? 256 : 512;
   const int tr = D == 64 ? StateTile<64, false>::TR : StateTile<128, false>::TR;
-  LinSplit sp = lin_split(BH, L, slots, tr, min_rows);
-  // (slices of three tiles become slices of two while a quarter more workgroups are enough: 16 heads x 5003 x 64, quantised, 78.2 ->
-  //  74.9 us)
-  if (sp.rows_per_split == 3 * tr && 2 * tr >= min_rows && BH * cdiv(L, 2 * tr) <= slots + slots / 4)
-    sp = LinSplit{cdiv(L, 2 * tr), 2 * tr};
+  const LinSplit sp = lin_split(BH, L, slots, tr, min_rows);
   w.nsplit = sp.nsplit;
   w.rows_per_split = sp.rows_per_split;
   size_t off = 0;
