@@ -464,15 +464,18 @@ struct LinWs {
 
 static inline LinWs lin_ws(int BH, int L, int D) {
   LinWs w;
-  // One workgroup per compute unit: more, shorter slices only add partial states to write and to add up again by few workgroups
-  // (two per unit / one, module forward: 12 heads x 9360 x 128 133.8 / 128.1 us, 12 x 5400 x 128 91.4 / 87.1, 24 x 6000 x 128
-  // 112.6 / 110.6, 32 x 7813 x 64 112.5 / 110.8, 12 x 32760 x 128 464.8 / 461.8; three workgroups to two units 128.1, 87.1, 110.6
-  // -> 132, 91, 112).  Two above 64 Mi elements, where the sums are a small part: 40 heads x 32760 x 128, quantised 2141 / 2153 us.
+  // One workgroup per compute unit (256 slots): more, shorter slices only add partial states to write and to add up again by few
+  // workgroups (module forward, two per unit / one: 12 heads x 14000 x 128 225.6 / 222.6 us, 24 x 2500 x 128 66.5 / 60.4, 32 x 1500 x
+  // 128 60.3 / 57.3, 36 x 2500 x 128 90.4 / 86.5, 48 x 2500 x 64 60.3 / 58.9, 80 x 1500 x 128 100.5 / 97.6).  Two (512 slots)
+  // - where the whole slices of all heads leave more than three of sixteen units without one (one per unit / two: 129 heads x 2000 x 128
+  //   230 / 186, 130 x 6000 x 64 329 / 296, 96 x 2500 x 64 94.0 / 91.1, 100 x 2500 x 128 183.0 / 179.3; with 210 of 256 or more, 72 x 2500
+  //   x 128 139.9 / 139.7, 112 x 2500 x 128 195 / 204, 128 x 2500 x 128 219 / 236);
+  // - above 64 Mi elements, where the sums are a small part: 40 heads x 32760 x 128, quantised 2153 / 2141.
   // Short sequences: at most sixteen slices, or slices of 256
   // rows; more only lengthen the chain that adds them up (state build of 8 heads x 4096 rows x 128: 64 slices 34.6 us, 16
   // slices 23.8; 4 heads x 7813 x 64: 123 slices 23.5, 31 slices 15.3; with 1024 rows 16 slices of 64 rows 14.7, 4 of 256 19.4).
   const int min_rows = L >= 4096 ? 256 : cdiv(L, 16);
-  const int slots = (int64_t)BH * L * D <= (64ll << 20) ? 256 : 512;
+  const int slots = (int64_t)BH * L * D <= (64ll << 20) && BH * (256 / BH) >= 208 ? 256 : 512;
   const int tr = D == 64 ? StateTile<64, false>::TR : StateTile<128, false>::TR;
   const LinSplit sp = lin_split(BH, L, slots, tr, min_rows);
   w.nsplit = sp.nsplit;

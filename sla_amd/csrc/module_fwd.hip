@@ -42,22 +42,25 @@ __global__ __launch_bounds__(256) void prefix_pool_kernel(const typename IO::raw
                               blockIdx.y, blockIdx.z, cast, n);
 }
 
-// The slices' partial states and, in the first `first_wg` workgroups, the column mean of k; one head's slices are adjacent.
+// The slices' partial states and, in the workgroups from `state_wgs` on, the column mean of k; one head's slices are adjacent.  (The
+// means' workgroups, D / 16 short ones per head, ahead of the slices: from 320 of them on a slice per compute unit no longer
+// starts everywhere at once.  Forward, ahead / behind: 48 heads x 4096 x 128 158 / 149 us, 72 x 2500 x 128 153 / 140, 100 x 2500 x 64 101.4
+// / 96.1; up to 288 of them equal.)
 template <typename Tag, int D, typename IO>
 __global__ __launch_bounds__((StateTile<D, false>::NTH)) __attribute__((amdgpu_waves_per_eu(4, 4))) void prefix_state_kernel(
     const uint16_t* __restrict__ k, const uint16_t* __restrict__ v, const RowLayout lay, float* __restrict__ kv_part,
-    float* __restrict__ z_part, int L, int rows_per_split, int nsplit, int fmap, const MapParts m, int first_wg) {
+    float* __restrict__ z_part, int L, int rows_per_split, int nsplit, int fmap, const MapParts m, int state_wgs) {
   static_assert(COLMEAN_MAX_GROUPS * COLMEAN_SLAB * 4 <= StateTile<D, false>::LDS, "the column mean's sums fit the tiles");
   __shared__ __attribute__((aligned(16))) char smem[StateTile<D, false>::LDS];
-  const int wg = blockIdx.x;
-  if (wg < first_wg) {
+  const int wg = blockIdx.x, mean = wg - state_wgs;
+  if (mean >= 0) {
     colmean_body<IO, StateTile<D, false>::NTH>(m.chunk_sums, (typename IO::raw*)m.colmean, m.nchunk, (m.nchunk + KMEAN_GROUP - 1) / KMEAN_GROUP, D, L,
-                     wg % (D / COLMEAN_SLAB), wg / (D / COLMEAN_SLAB), reinterpret_cast<float*>(smem));
+                     mean % (D / COLMEAN_SLAB), mean / (D / COLMEAN_SLAB), reinterpret_cast<float*>(smem));
     return;
   }
-  const int bh = (wg - first_wg) / nsplit;
+  const int bh = wg / nsplit;
   state_partial_body<Tag, D, false, false, false>(k, v, lay, kv_part, z_part, L, rows_per_split, fmap, nullptr, nullptr,
-                                                  wg - first_wg - bh * nsplit, bh, nsplit, smem);
+                                                  wg - bh * nsplit, bh, nsplit, smem);
 }
 
 // The states finished and, in the workgroups from `first_pool` on (`per_head` for each head), the block means of k.
@@ -95,10 +98,10 @@ static void launch_prefix_rest(const void* k, const RowLayout& lin, const void* 
                                int in_dtype, const float* weight, int fmap, int BH, int L, char* states, char* parts, hipStream_t st) {
   typedef typename IO::raw raw;
   const LinWs w = lin_ws(BH, L, D);
-  const int first_wg = BH * (D / COLMEAN_SLAB);
-  hipLaunchKernelGGL((prefix_state_kernel<Tag, D, IO>), dim3(first_wg + BH * w.nsplit), dim3(StateTile<D, false>::NTH), 0, st, (const uint16_t*)kc,
+  const int state_wgs = BH * w.nsplit;
+  hipLaunchKernelGGL((prefix_state_kernel<Tag, D, IO>), dim3(state_wgs + BH * (D / COLMEAN_SLAB)), dim3(StateTile<D, false>::NTH), 0, st, (const uint16_t*)kc,
                      (const uint16_t*)vc, lay, (float*)(parts + (w.kv_part - w.states_end)),
-                     (float*)(parts + (w.z_part - w.states_end)), L, w.rows_per_split, w.nsplit, fmap, m, first_wg);
+                     (float*)(parts + (w.z_part - w.states_end)), L, w.rows_per_split, w.nsplit, fmap, m, state_wgs);
   launch_state_presum<D>(BH, parts, w, st);
   const StateFinish job = state_finish_job<D>(weight, BH, states, parts, w);
 #define SLA_FINISH_CASE(W)                                                                                                   \

@@ -924,19 +924,19 @@ template <typename Tag, int D>
 __global__ __launch_bounds__((StateTile<D, false>::NTH)) __attribute__((amdgpu_waves_per_eu(4, 4))) void sage_state_kernel(
     const uint16_t* __restrict__ k, const uint16_t* __restrict__ v, const RowLayout lay, float* __restrict__ kv_part,
     float* __restrict__ z_part, float* __restrict__ vmax_part, int L, int rows_per_split, int nsplit, int fmap,
-    const float* __restrict__ chunk_sums, uint16_t* __restrict__ colmean, int nchunk, int first_wg) {
+    const float* __restrict__ chunk_sums, uint16_t* __restrict__ colmean, int nchunk, int state_wgs) {
   static_assert(COLMEAN_MAX_GROUPS * COLMEAN_SLAB * 4 <= StateTile<D, false>::LDS, "the column mean's sums fit the tiles");
   __shared__ __attribute__((aligned(16))) char smem[StateTile<D, false>::LDS];
-  const int wg = blockIdx.x;
-  if (wg < first_wg) {
+  const int wg = blockIdx.x, mean = wg - state_wgs;          // (the means' workgroups behind the slices', as in the module's forward)
+  if (mean >= 0) {
     colmean_body<typename IoOf<Tag>::type, StateTile<D, false>::NTH>(chunk_sums, colmean, nchunk, (nchunk + KMEAN_GROUP - 1) / KMEAN_GROUP,
-                                                                     D, L, wg % (D / COLMEAN_SLAB), wg / (D / COLMEAN_SLAB),
+                                                                     D, L, mean % (D / COLMEAN_SLAB), mean / (D / COLMEAN_SLAB),
                                                                      reinterpret_cast<float*>(smem));
     return;
   }
-  const int bh = (wg - first_wg) / nsplit;
+  const int bh = wg / nsplit;
   state_partial_body<Tag, D, false, false, true>(k, v, lay, kv_part, z_part, L, rows_per_split, fmap, nullptr, vmax_part,
-                                                 wg - first_wg - bh * nsplit, bh, nsplit, smem);
+                                                 wg - bh * nsplit, bh, nsplit, smem);
 }
 
 // first `finish_wgs` workgroups: the states; then two key blocks per workgroup; then 512 * 8 values of v per workgroup, whose
@@ -1017,11 +1017,11 @@ static void launch_small_preparation(const void* q, const void* k, const void* v
   const int per_head = cdiv(N, 256 / (D / 2));               // (chunks of KMEAN_CHUNK = 64 rows)
   hipLaunchKernelGGL((sage_first_kernel<Tag, D>), dim3(BH * M + BH * per_head), dim3(256), 0, st, (const uint16_t*)q,
                      (const uint16_t*)k, lay, q8, qs, pq, M, tiled, chunk_sums, N, L, BH * M, per_head);
-  const int first_wg = BH * (D / COLMEAN_SLAB);
-  hipLaunchKernelGGL((sage_state_kernel<Tag, D>), dim3(first_wg + BH * lw.nsplit), dim3(StateTile<D, false>::NTH), 0, st,
+  const int state_wgs = BH * lw.nsplit;
+  hipLaunchKernelGGL((sage_state_kernel<Tag, D>), dim3(state_wgs + BH * (D / COLMEAN_SLAB)), dim3(StateTile<D, false>::NTH), 0, st,
                      (const uint16_t*)k, (const uint16_t*)v, lay, (float*)(linear + lw.kv_part), (float*)(linear + lw.z_part),
                      (float*)(linear + lw.vmax_part), L, lw.rows_per_split, lw.nsplit, fmap, (const float*)chunk_sums, colmean, N,
-                     first_wg);
+                     state_wgs);
   launch_state_presum<D>(BH, linear + lw.states_end, lw, st);
   const StateFinish job = state_finish_job<D>(weight, BH, linear, linear + lw.states_end, lw);
   const int finish_wgs = xcd_grid(job.total), quant_wgs = BH * cdiv(N, 2), v_wgs = cdiv(L, 512 / (D / 8));

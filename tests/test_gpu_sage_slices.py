@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("H,L,D", [(2, 64, 128), (3, 129, 64), (1, 960, 128), (2, 1024, 128), (1, 4352, 64), (1, 7900, 64), (3, 8192, 128),
-                                   (1, 8200, 128)])                       # 1, 2, 15, 16, 17, 31, 32 and 33 slices
+                                   (1, 8200, 128), (129, 1300, 64)])      # 1, 2, 15, 16, 17, 31, 32, 33 and 3 slices
 def test_module_equals_the_steps(dev, H, L, D):
     g = torch.Generator(device=dev).manual_seed(L + D)
     q, k, v = (torch.randn(1, H, L, D, device=dev, generator=g).bfloat16() for _ in range(3))

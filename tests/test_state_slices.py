@@ -25,3 +25,13 @@ def test_neighbouring_lengths_follow_one_rule(BH, D):
     for L in [*range(4100, 9000, 113), 5003, 6001]:
         n = slices(BH, L, D)
         assert n * BH <= 256 and n == tiles(L, D, min(256 // BH, -(-L // 256))), (BH, L, D, n)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_many_heads_leave_no_compute_units_idle(D):
+    """Long enough sequences come to a workgroup for most of the 256 compute units, and to two rounds of them at most."""
+    for BH in range(1, 513):
+        L = (64 << 20) // (BH * D)             # (the largest below the line of two per unit)
+        if L >= 16 * 128:
+            assert 208 <= BH * slices(BH, L, D) <= 512, BH
+        assert 208 <= BH * slices(BH, 4 * (64 << 20) // (BH * D), D), BH
