@@ -243,20 +243,16 @@ static __device__ __forceinline__ void park_acc_tile(uint16_t* stage, const floa
   wave_lds_fence();
 }
 
-// Accumulator-order tile -> global rows.  An addend is added after the value has been rounded to
-// 16 bit, as a separate 16-bit tensor addition would: `addend` is a tile fetched earlier; with
-// ADD_DEST the addend is what the destination rows hold (read here, while the tile sits in LDS).
-template <typename E, int D, bool ADD_DEST = false>
+// Accumulator-order tile -> global rows.  `addend`, a tile fetched earlier (or null), is added after the value has been
+// rounded to 16 bit, as a separate 16-bit tensor addition would.
+template <typename E, int D>
 static __device__ __forceinline__ void store_acc_tile(uint16_t* stage, const float (&val)[D / 32][16], uint16_t* gtile,
                                                        const TileRows<D>* addend, int rows_valid, int lane,
                                                        size_t pitch = D) {
-  TileRows<D> old;
-  if (ADD_DEST) old.fetch(gtile, rows_valid, lane, pitch);
   park_acc_tile<E, D>(stage, val, lane);
   TileRows<D> t;
   t.unpark(stage, lane);
-  if (ADD_DEST) t.template add<E>(old);
-  else if (addend) t.template add<E>(*addend);
+  if (addend) t.template add<E>(*addend);
   t.store(gtile, rows_valid, lane, pitch);
   wave_lds_fence();   // the staging area may be rewritten right after
 }

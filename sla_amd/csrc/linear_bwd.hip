@@ -108,7 +108,7 @@ static int linear_bwd_impl(const void* q, const void* k, const void* v, const fl
     SLA_LB_FMAPS(SLA_LBS_LAUNCH)
 #undef SLA_LBS_LAUNCH
   }
-  // (the line of the forward's states; both sides measured at linear_bwd_finish_kernel)
+  // (the line of the forward's states)
   const bool presum = w.sp.nsplit >= PRESUM_MIN_SLICES;
   if ((steps & LB_REDUCE) && presum)
     hipLaunchKernelGGL((linear_state_presum_kernel<D>), dim3(D * D / 256 + 2, BH), dim3(512), 0, st, m_part, (float*)(ws + w.dz_part),

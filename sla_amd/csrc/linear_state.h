@@ -252,14 +252,6 @@ __global__ __launch_bounds__((StateTile<D, OUT16>::NTH)) __attribute__((amdgpu_w
                                                      blockIdx.x, blockIdx.y, gridDim.x, smem);
 }
 
-// Position of column d2 inside a row whose columns are re-ordered to the accumulator slot order of the
-// 32x32 MFMA: slot j of 16-column chunk c, lane group gg  <->  d2 = 16c + 8*(j/4) + 4gg + j%4.
-static __device__ __host__ __forceinline__ int slot_order_pos(int d2) {
-  const int c = d2 >> 4, w16 = d2 & 15;
-  const int gg = (w16 >> 2) & 1, j = ((w16 >> 3) << 2) | (w16 & 3);
-  return 16 * c + 8 * gg + j;
-}
-
 // 16-bit copy of the projection weight as the A operand of dY^T = W^T G^T, in the order in which a wave reads it: 32 rows d x 16
 // columns e after one another, a lane's eight columns together.  One thread per element.
 template <typename Tag>
@@ -323,9 +315,12 @@ static __device__ __forceinline__ void sum_slices(const float* __restrict__ p, i
 // below has D / 16 workgroups per head: few heads with many slices leave it reading on a few compute units.  Here a workgroup
 // of 512 threads takes 256 elements, its halves one half of the slices each, 32 loads in flight; the last one of a head takes z,
 // another one behind it (the backward's sums have one) a second vector.
-// Bound by latency.  State build in us without this launch and with it: 1 head x 75600 x 128 (295 slices) 88.6 / 35.8, 2 heads
-// x 75600 x 128 (256) 78.4 / 41.4, 4 heads x 32760 x 128 (128) 53.9 / 37.9, 8 heads x 16384 x 64 (64) 23.2 / 19.9, 12 heads x
-// 24576 x 128 (42) 62.3 / 58.9, 16 heads x 16384 x 128 (32) 53.0 / 53.6, 2 heads x 4096 x 64 (16) 14.2 / 15.7.
+// Bound by latency.  State build in us without this launch and with it: 1 head x 75600 x 128 (256 slices) 72.0 / 29.6, 2 heads x
+// 75600 x 128 (128) 54.8 / 35.6, 4 heads x 32760 x 128 (64) 39.6 / 32.7, 8 heads x 16384 x 64 (32) 18.7 / 17.8, 12 heads x 24576 x
+// 128 (21) 52.3 / 51.6, 16 heads x 16384 x 128 (16) 45.7 / 48.4.  Among the other launches of a forward the line lies between 36 and
+// 50 slices; whole forward without / with: 128 columns 6 heads x 14000 (37) 106.8 / 101.7, 8 x 14000 (32) 120.8 / 121.8, 8 x 20000
+// (32) 136.1 / 137.3; 64 columns 5 x 17000 (45) 70.2 / 72.1, 3 x 12000 (47) 49.6 / 51.2, 4 x 14000 (55) 53.8 / 52.3; quantised 6 x
+// 10000 x 128 (40) 85.5 / 89.3, 6 x 12000 x 128 (38) 117.3 / 113.5, 5 x 25000 x 64 (49) 112.4 / 109.4.
 template <int D>
 __global__ __launch_bounds__(512) void linear_state_presum_kernel(float* __restrict__ kv_part, float* __restrict__ z_part,
                                                                   float* __restrict__ z2_part, int nsplit) {
@@ -501,7 +496,7 @@ __global__ __launch_bounds__(512) void linear_state_finish_kernel(const StateFin
   if (logical >= 0) state_finish_body<Tag, D>(job, logical, smem);
 }
 
-constexpr int PRESUM_MIN_SLICES = 40;       // (measured at linear_state_presum_kernel)
+constexpr int PRESUM_MIN_SLICES = 40;       // (both sides measured at linear_state_presum_kernel; the backward's at linear_bwd_finish_kernel)
 
 // What is left to do behind the partial states (and, with many slices, behind the launch that adds them up first).  ws: where
 // the states go; parts: where the slices' partial sums lie, the offsets of `w` past states_end.
