@@ -8,8 +8,9 @@ namespace sla {
 // tiles of 32 blocks per head; other dtypes and head dims take rows, and so does a workspace with no room for the tiles.
 static inline int score_takes_tiled(int dtype, int D) { return dtype != SLA_F32 && (D == 64 || D == 128); }
 
-// Rows of at most this many key blocks are scored and selected from in one launch (block_map.hip), the scores never in memory.
-constexpr int SELECT_FUSED_N = 128;        // rows of at most so many key blocks need no memory for scores
+// Rows of at most this many key blocks are always scored and selected from in one launch (block_map.hip) and need no memory for
+// scores.  (Longer ones up to 256 are where their workgroups are few; their workspace has room for scores all the same.)
+constexpr int SELECT_FUSED_N = 128;
 static inline bool scores_in_memory(int N, int D) { return N > SELECT_FUSED_N || (D != 64 && D != 128); }
 
 // Operand order: tiles of 32 blocks; per tile and 16 columns a fragment of 64 lanes x 8 elements, lane (r, h) = (block % 32,

@@ -347,12 +347,14 @@ static __device__ __forceinline__ void emit_row(const uint32_t (&keys)[EPL], uin
 
 // The T-th largest of W keys per lane, for R rows at once, built bit by bit from the top (a bit stays when at least T keys are
 // at or above the value it gives; counts through the wave's ballots).  The rows' chains hide each other's latency.
-// Missing keys are 0.
-template <int R, int W, int LOW_BIT>
+// Missing keys are 0.  FOUR: four bits at a time.  (Rows of one or two keys per lane: left alone, the compiler lays out all the bits
+// and keeps 23 to 103 scalar registers elsewhere; mask builder of 8 heads x 4096 x 128 in fp32 25.7 -> 24.5 us, of 32 x 7813 x 64 25.8 ->
+// 24.9.  With four keys it does not, and is faster for it: 8 heads x 16000 x 64 19.9 us, 20.3 four bits at a time.)
+template <int R, int W, int LOW_BIT, bool FOUR = false>
 static __device__ __forceinline__ void kth_largest(const uint32_t (&kx)[R][W], int T, uint32_t (&thr)[R]) {
 #pragma unroll
   for (int x = 0; x < R; ++x) thr[x] = 0;
-  for (int b = 31; b >= LOW_BIT; --b) {
+  const auto bit = [&](int b) __attribute__((always_inline)) {
     int cnt[R];
 #pragma unroll
     for (int x = 0; x < R; ++x) {
@@ -363,6 +365,12 @@ static __device__ __forceinline__ void kth_largest(const uint32_t (&kx)[R][W], i
 #pragma unroll
     for (int x = 0; x < R; ++x)
       if (cnt[x] >= T) thr[x] |= 1u << b;
+  };
+  if constexpr (FOUR) {
+#pragma unroll 4
+    for (int b = 31; b >= LOW_BIT; --b) bit(b);
+  } else {
+    for (int b = 31; b >= LOW_BIT; --b) bit(b);
   }
 }
 template <int W>
@@ -413,7 +421,7 @@ static __device__ __forceinline__ void select_rows(const uint32_t (&kx)[R][EPL],
       }
     }
   }
-  if (!short_list) kth_largest<R, EPL, LOW_BIT>(kx, T, thr);
+  if (!short_list) kth_largest<R, EPL, LOW_BIT, EPL <= 2>(kx, T, thr);
 #pragma unroll
   for (int x = 0; x < R; ++x) {
     if (x >= rows) break;
@@ -599,14 +607,13 @@ __global__ __launch_bounds__(256) void topk_kernel(const typename IO::raw* __res
 // One workgroup of eight waves per 16 query blocks of a head: the waves form the 16 x N scores (16-bit inputs: a tile of 16 x
 // 16 each on the matrix cores; fp32 inputs: every product and sum rounded on the vector ALU as in score_kernel), keep them in LDS,
 // rounded, and then select for two rows each.  The scores never go to memory and a launch is saved: mask builder of 2
-// heads x 1024 x 64 in fp32 25.3 -> 19.6 us, of 32 x 7813 x 64 38.1 -> 35.0.  With longer rows the two kernels, spread over more
-// workgroups, are as fast or faster (12 heads x 9360 x 128, 128-row query blocks: 36.5 us against 39.0; 2 x 75600: 62 against 77).
+// heads x 1024 x 64 in fp32 25.3 -> 19.6 us, of 32 x 7813 x 64 38.1 -> 35.0.
 // Bound by latency: a chain of dependent products, then one of threshold bits.  v_mfma_f32_16x16x4_f32 adds its four products
 // one after the other, each with a single rounding, k ascending: the same bits as the 32 x 32 x 2 chain in a quarter of the cycles
 // per tile.
 // Rows of 129 to 256 key blocks go this way, too, where the workgroups fit the compute units side by side (16-bit inputs; forward, two
 // launches / one: 12 heads x 9360 x 128 141.9 / 139.4 us, 8 x 16000 x 64 79.6 / 77.9; 315 workgroups 344.0 / 345.3; fp32 120.7 /
-// 121.8).
+// 121.8).  They are a variant of their own (MAX_N): its short lists take 14 KB of LDS that the shorter rows do not need.
 constexpr int SELECT_ONE_N = 256;
 static bool select_in_one(int N, int D, int BH, int M, int elem_bytes) {
   return !scores_in_memory(N, D) ||
@@ -637,18 +644,19 @@ struct ScoreFrags16 {                            // 16 blocks, a lane's columns 
     return IO::ld((typename IO::raw)((uint32_t)w[c][t] >> (16 * (TILED ? q >> 1 : q & 1))));
   }
 };
-template <typename IO, int D, bool TILED>
+template <typename IO, int D, bool TILED, int MAX_N>
 __global__ __launch_bounds__(512) void select_kernel(const typename IO::raw* __restrict__ pq, const typename IO::raw* __restrict__ pk,
                                                      int8_t* __restrict__ sparse_map, void* __restrict__ lut, int lut64, int M,
                                                      int N, int T) {
   typedef typename IO::raw raw;
-  constexpr int EB = sizeof(raw), EPL = SELECT_ONE_N / 64;
+  constexpr int EB = sizeof(raw), EPL = MAX_N / 64;
+  static_assert(MAX_N == SELECT_FUSED_N || (MAX_N == SELECT_ONE_N && EB == 2), "two variants, the one of longer rows for 16-bit inputs");
   constexpr int OS = 64 * EPL + 4 / EB;     // scores between rows
   constexpr int RS = D * 4 + 16;            // bytes between rows of an fp32 q tile
   constexpr int LIST = 2 * SELECT_CAND + 16 * EPL;      // words of a wave's short list
   __shared__ __attribute__((aligned(16))) uint8_t sq[EB == 4 ? 16 * RS : 16];
   __shared__ __attribute__((aligned(16))) raw ss[16 * OS];
-  __shared__ uint32_t lists[8 * LIST];
+  __shared__ uint32_t lists[EPL > 2 ? 8 * LIST : 1];
   const int bh = blockIdx.y, m0 = blockIdx.x * 16;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   if constexpr (EB == 2) {
@@ -716,16 +724,16 @@ __global__ __launch_bounds__(512) void select_kernel(const typename IO::raw* __r
   const auto key = [&](int x, int i) {
     return i < N ? order_key<IO::KEY_LOW_BIT>(IO::ld(ss[(2 * wave + x) * OS + i])) : 0u;
   };
-  if (N <= 64) {
-    const uint32_t kx[2][1] = {{key(0, lane)}, {key(1, lane)}};
-    select_rows<1, IO::KEY_LOW_BIT, 2>(kx, nullptr, sparse_map, lut, lut64, row0, rows, N, T, lane);
-  } else if (N > 128) {
+  if constexpr (EPL > 2) {
     uint32_t kx[2][EPL];
 #pragma unroll
     for (int x = 0; x < 2; ++x)
 #pragma unroll
       for (int e = 0; e < EPL; ++e) kx[x][e] = key(x, 64 * e + lane);
     select_rows<EPL, IO::KEY_LOW_BIT, 2>(kx, lists + wave * LIST, sparse_map, lut, lut64, row0, rows, N, T, lane);
+  } else if (N <= 64) {
+    const uint32_t kx[2][1] = {{key(0, lane)}, {key(1, lane)}};
+    select_rows<1, IO::KEY_LOW_BIT, 2>(kx, nullptr, sparse_map, lut, lut64, row0, rows, N, T, lane);
   } else {
     const uint32_t kx[2][2] = {{key(0, lane), key(0, 64 + lane)}, {key(1, lane), key(1, 64 + lane)}};
     select_rows<2, IO::KEY_LOW_BIT, 2>(kx, nullptr, sparse_map, lut, lut64, row0, rows, N, T, lane);
@@ -753,15 +761,19 @@ static void launch_select(const typename IO::raw* pq, const typename IO::raw* pk
                           int8_t* sparse_map, void* lut, int lut64, int BH, int M, int N, int D, int T, hipStream_t st) {
   if (select_in_one(N, D, BH, M, (int)sizeof(typename IO::raw))) {
     const dim3 grid(cdiv(M, 16), BH);
-#define SLA_SELECT_CASE(DD, TILED)                                                                                             \
-  if (D == DD && (tiled != 0) == TILED)                                                                                        \
-    hipLaunchKernelGGL((select_kernel<IO, DD, TILED>), grid, dim3(512), 0, st, pq, pk, sparse_map, lut, lut64, M, N, T);
+#define SLA_SELECT_CASE(DD, TILED, MAX_N)                                                                                      \
+  if (D == DD && (tiled != 0) == TILED && (N > SELECT_FUSED_N) == (MAX_N > SELECT_FUSED_N))                                      \
+    hipLaunchKernelGGL((select_kernel<IO, DD, TILED, MAX_N>), grid, dim3(512), 0, st, pq, pk, sparse_map, lut, lut64, M, N, T);
     if constexpr (sizeof(typename IO::raw) == 2) {
-      SLA_SELECT_CASE(128, true)
-      SLA_SELECT_CASE(64, true)
+      SLA_SELECT_CASE(128, true, SELECT_FUSED_N)
+      SLA_SELECT_CASE(64, true, SELECT_FUSED_N)
+      SLA_SELECT_CASE(128, true, SELECT_ONE_N)
+      SLA_SELECT_CASE(64, true, SELECT_ONE_N)
+      SLA_SELECT_CASE(128, false, SELECT_ONE_N)
+      SLA_SELECT_CASE(64, false, SELECT_ONE_N)
     }
-    SLA_SELECT_CASE(128, false)
-    SLA_SELECT_CASE(64, false)
+    SLA_SELECT_CASE(128, false, SELECT_FUSED_N)
+    SLA_SELECT_CASE(64, false, SELECT_FUSED_N)
 #undef SLA_SELECT_CASE
     return;
   }
