@@ -95,6 +95,9 @@ static __device__ __forceinline__ void col_lists_body(const ColLists& j, int wg,
 // segment is one work item.  item = {bh, key block, segment, slot}: slot < 0 for a key block with a single segment
 // (the workgroup writes dK / dV itself), otherwise the index of the fp32 partial this segment writes; the partials
 // of a key block occupy consecutive slots and are added in segment order.
+// A map whose rows hold more ones than the topk the workspace was sized for: the tables have room for every key block's first
+// segment and `room` further ones, in the order of the key blocks; what exceeds that is left out, and the lists end there.  (Each
+// of the room's segments belongs to at most two slots, of which there are two for each.)
 // One wave per 512 (head, key block) pairs: it counts the items of all pairs before its own (no other wave is waited for),
 // then numbers its own, 64 adjacent pairs at a time.  (One workgroup for all pairs, with eight adjacent ones per thread and
 // therefore scattered stores, took 38 us for 32 heads x 512.)
@@ -104,27 +107,27 @@ struct Segments {
   int *nseg, *slot0, *done;                                            // done: segments finished so far, cleared here
   i32x4_t* items;
   int* totals;
-  int nblocks, Nblk, seg, max_items, max_slots, wgs;                   // nblocks = heads x key blocks; wgs 0: nothing to do
+  int nblocks, Nblk, seg, room, wgs;                                   // nblocks = heads x key blocks; wgs 0: nothing to do
 };
 static __device__ __forceinline__ void segments_body(const Segments& s, int wg) {
   const int lane = threadIdx.x & 63;
   const int first = wg * SEG_PAIRS;
-  const auto nsegs = [&](int c) { return c <= s.seg ? 1 : (c + s.seg - 1) / s.seg; };
-  int item0 = 0, slot = 0;
+  const auto further = [&](int c) { return c <= s.seg ? 0 : (c + s.seg - 1) / s.seg - 1; };      // segments behind the first
+  int extra0 = 0, slot = 0;
   for (int i = lane; i < first; i += SEG_PAIRS) {
     int c[SEG_PAIRS / 64];
 #pragma unroll
     for (int x = 0; x < SEG_PAIRS / 64; ++x) c[x] = s.count[i + 64 * x];
 #pragma unroll
     for (int x = 0; x < SEG_PAIRS / 64; ++x) {
-      const int n = nsegs(c[x]);
-      item0 += n;
-      slot += n > 1 ? n : 0;
+      const int n = further(c[x]);
+      extra0 += n;
+      slot += n > 0 ? n + 1 : 0;
     }
   }
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
-    item0 += __shfl_xor(item0, o);
+    extra0 += __shfl_xor(extra0, o);
     slot += __shfl_xor(slot, o);
   }
   int c[SEG_PAIRS / 64];
@@ -136,7 +139,7 @@ static __device__ __forceinline__ void segments_body(const Segments& s, int wg) 
 #pragma unroll
   for (int x = 0; x < SEG_PAIRS / 64; ++x) {
     const int i = first + 64 * x + lane;
-    const int n = i < s.nblocks ? nsegs(c[x]) : 0, m = n > 1 ? n : 0;
+    const int n = further(c[x]), m = n > 0 ? n + 1 : 0;
     int a = n, b = m;                          // inclusive scans
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
@@ -147,24 +150,18 @@ static __device__ __forceinline__ void segments_body(const Segments& s, int wg) 
       }
     }
     if (i < s.nblocks) {
-      const int fi = item0 + a - n, fs = slot + b - m;
-      s.nseg[i] = n;
+      const int e0 = min(extra0 + a - n, s.room), kept = 1 + min(extra0 + a, s.room) - e0;
+      const int fi = i + e0, fs = slot + b - m;
+      s.nseg[i] = kept;
       s.slot0[i] = fs;
       s.done[i] = 0;
       const int bh = i / s.Nblk, nb = i - bh * s.Nblk;
-      // (a map whose rows hold more ones than the topk the workspace was sized for cannot overrun the tables: its
-      //  surplus items are dropped)
-      for (int sg = 0; sg < n; ++sg)
-        if (fi + sg < s.max_items)
-          s.items[fi + sg] = i32x4_t{bh, nb, sg, fs + m > s.max_slots ? -2 : n > 1 ? fs + sg : -1};
+      for (int sg = 0; sg < kept; ++sg) s.items[fi + sg] = i32x4_t{bh, nb, sg, kept > 1 ? fs + sg : -1};
     }
-    item0 += __shfl(a, 63);
+    extra0 += __shfl(a, 63);
     slot += __shfl(b, 63);
   }
-  if (first + SEG_PAIRS >= s.nblocks && lane == 0) {
-    s.totals[0] = min(item0, s.max_items);
-    s.totals[1] = min(slot, s.max_slots);
-  }
+  if (first + SEG_PAIRS >= s.nblocks && lane == 0) s.totals[0] = s.nblocks + min(extra0, s.room);
 }
 
 // ---- the heads' weight gradients added up, in ascending head order ----------------------------

@@ -90,11 +90,11 @@ template <typename Tag, int D>
 __global__ __launch_bounds__(256) void bwd_dkdv_reduce_kernel(const int* __restrict__ nseg, const int* __restrict__ slot0,
                                                               const float* __restrict__ part, uint16_t* __restrict__ dk,
                                                               uint16_t* __restrict__ dv, const RowLayout lin, int L, int Nblk,
-                                                              int max_slots, int add) {
+                                                              int add) {
   using E = Elem<Tag>;
   const int nb = blockIdx.x, bh = blockIdx.y;
   const int ns = nseg[(size_t)bh * Nblk + nb];
-  if (ns <= 1 || slot0[(size_t)bh * Nblk + nb] + ns > max_slots) return;
+  if (ns <= 1) return;
   const float* p0 = part + (size_t)slot0[(size_t)bh * Nblk + nb] * (2 * 64 * D);
   for (int idx = threadIdx.x * 4; idx < 2 * 64 * D; idx += 256 * 4) {
     f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
@@ -332,7 +332,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 3
   if (logical >= total) return;
   const i32x4_t item = items[logical];
   const int bh = item[0], nb = item[1], sg = item[2], slot = item[3];
-  if (slot < -1) return;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int kh = wave & 1, dh = wave >> 1;
   const int g = lane >> 5, r = lane & 31;
@@ -619,7 +618,7 @@ static int bwd_impl(const void* q, const void* k, const void* v, const void* o, 
   i32x4_t* items = (i32x4_t*)(ws + w.items);
   int* totals = (int*)(ws + w.totals);
   float* part = (float*)(ws + w.part);
-  const Segments segs = {count, nseg, slot0, done, items, totals, BH * Nblk, Nblk, w.seg, (int)w.max_items, (int)w.max_slots,
+  const Segments segs = {count, nseg, slot0, done, items, totals, BH * Nblk, Nblk, w.seg, (int)(w.max_items - BH * Nblk),
                          cdiv(BH * Nblk, SEG_PAIRS)};
   const int jobs = segs.wgs + heads.wgs;
   const int total_q = BH * Mblk;
@@ -680,7 +679,7 @@ static int bwd_impl(const void* q, const void* k, const void* v, const void* o, 
   }
   if ((steps & SB_DKDV) && !stream_dkdv)
     hipLaunchKernelGGL((bwd_dkdv_reduce_kernel<Tag, D>), dim3(Nblk, BH), dim3(256), 0, st, nseg, slot0, part, (uint16_t*)dk,
-                       (uint16_t*)dv, lin, L, Nblk, (int)w.max_slots, add);
+                       (uint16_t*)dv, lin, L, Nblk, add);
   return check_launch("sparse_attn_bwd");
 }
 

@@ -133,3 +133,35 @@ def test_rows_too_far_apart_for_the_stream_kernels(dev, D, BLKQ):
     got = module_bwd(*wide, o, do, lse, smap, lut, T, BLKQ, 64, scale, w, b, "elu", grads=grads)
     for a, r in zip(got, ref):
         assert torch.equal(a, r)
+
+
+@pytest.mark.parametrize("H,D,T,whole", [(1, 128, 1, True), (2, 64, 1, True), (33, 64, 1, True), (2, 128, 3, False), (1, 64, 0, False)])
+def test_map_with_more_ones_than_topk(dev, H, D, T, whole):
+    """A map that contradicts topk (the C entry points accept it): every key block's gradients are written, from the first 64 of its
+    query blocks and as many further segments as there is room for, H M T / 64 in the order of the key blocks; nothing else is
+    touched.  The whole module's backward, with the linear branch formed in dK/dV (two sizes) and beside it (33 heads), and the attention's."""
+    from sla_amd.inputs import make_proj
+    from sla_amd.module import module_bwd
+    from sla_amd.sparse_attn import sparse_attn_bwd
+    M, L = 128, 128 * 64 - 3
+    g = torch.Generator(device=dev).manual_seed(D + T)
+    q, k, v, o, do = (torch.randn(1, H, L, D, device=dev, generator=g).bfloat16() for _ in range(5))
+    lse = 6 + torch.rand(1, H, L, device=dev, generator=g)
+    w, b = (t.to(dev) for t in make_proj(D))
+    lut = torch.arange(M, device=dev, dtype=torch.int32).expand(1, H, M, M).contiguous()
+
+    def run(smap):
+        table = lut[..., :T].contiguous()
+        grads = tuple(torch.full((1, H, L, D), float("nan"), dtype=torch.bfloat16, device=dev) for _ in range(3))
+        if whole:
+            return module_bwd(q, k, v, o, do, lse, smap, table, T, 64, 64, D ** -0.5, w, b, "elu", grads=grads)[1:3]
+        return sparse_attn_bwd(q, k, v, o, do, lse, smap, table, T, 64, 64, D ** -0.5)[1:3]
+
+    ones = torch.ones(1, H, M, M, dtype=torch.int8, device=dev)
+    got = run(ones)
+    kept = torch.ones(H * M, dtype=torch.long, device=dev)
+    kept[:H * M * T // 64] = 2                                # (each list of 128 has one segment beyond its first)
+    rows = torch.arange(M, device=dev)[:, None]
+    ref = run((rows < 64 * kept.view(1, H, 1, M)).to(torch.int8))         # (fills the room and no more)
+    for name, a, r in zip(("dk", "dv"), got, ref):
+        assert torch.isfinite(a).all() and torch.equal(a, r), name
