@@ -400,6 +400,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 128 ? 
 //   dv^T = dS^T c^T and dc^T = dS v^T as 16x16x32 products (a key's row spread over 4 lanes, B operands read row-wise
 //   from the wave's tiles); dk, dv go back over the tiles and leave as whole rows, added to what dk, dv held (asked
 //   for at the start of the tile) when accumulating.
+// The arithmetic is that of KeyTiles (linear_keys.h), which the attention's dK/dV kernel uses in launches with few key blocks: the same
+// products, sums and roundings in the same order, to be kept so.
 template <typename Tag, int D, int FMAP, bool ACC>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 128 ? 2 : 4, D == 128 ? 2 : 4))) void linear_bwd_keys_kernel(
     const uint16_t* __restrict__ k, const uint16_t* __restrict__ v, const uint16_t* __restrict__ ds,

@@ -137,10 +137,11 @@ __global__ __launch_bounds__(512) void complement_column_weights_kernel(const in
 //
 // A matrix product of the weights (nrows x nblk) with the block states (nblk x D*D) on the matrix cores, whose products are
 // exact (weights 0 and 2, the sum halved at the end), accumulated in fp32.  Bound by memory up to some 400 blocks (every block
-// state is read once and every state written once: 2 x 32 KB per row at D = 128), by the matrix cores above.  A workgroup of
-// four waves takes 128 rows x 256 values (RW = 1) or 256 x 128 (RW = 2), a wave 128 x 64 as eight 32 x 32 accumulators (parts of 32 rows that the head does
-// not have are left out): eight products for every four transposed LDS reads.  Tiles of 64 blocks go through registers, two tiles ahead, into one of two LDS buffers.  Even and odd values of a
-// row are parked apart, so that a lane's two column tiles hold neighbouring values and 32 lanes store whole 128-byte lines.
+// state is read once per workgroup's rows and every state written once: 2 x 32 KB per row at D = 128), by the matrix cores above.
+// A workgroup of four waves takes 128 rows x 256 values (RW = 1) or 256 x 128 (RW = 2), a wave 128 x 64 as eight 32 x 32 accumulators
+// (parts of 32 rows that the head does not have are left out): eight products for every four transposed LDS reads.  Tiles of 64 blocks
+// go through registers, two tiles ahead, into one of two LDS buffers.  Even and odd values of a row are parked apart, so that a lane's
+// two column tiles hold neighbouring values and 32 lanes store whole 128-byte lines.
 // z: workgroups of their own (the first ones of a head), 128 RW rows x 32 values, fp32 matrix products.
 // Against `total - sum of the listed states` on the vector ALU, the union of eight rows' lists at a time, and its totals in two
 // launches: 12 heads x 16380 x 128, 12 of 256 blocks selected 70 us where that took 101 + 23 + 8; forward and backward of 12 heads
@@ -412,7 +413,8 @@ static __device__ __forceinline__ i32x4_t pack_half(const float (&x)[16], int c2
 // the last wave is done with the state; W comes in operand order from memory.  Four workgroups of 64 rows fit a compute unit (two
 // before, with half of each one's waves idle in the products): at 12 heads x 16380 x 128 out 79 -> 56 us, rows 110 -> 97, kv 113 -> 75;
 // the whole backward, adding to existing gradients, 386 -> 357 us there, with 128-row blocks 328 -> 301, at 24 heads x 10000 x 64
-// 200 -> 159 and 187 -> 150.
+// 200 -> 159 and 187 -> 150.  No spills in bf16; in half precision at head dim 128, whose feature map and conversions hold more at a
+// time, the compiler keeps 13 registers of the rows' kernel and 17 of the keys' in scratch memory.
 
 // 1-D grid over (head, query block), XCD-aware order, one wave per 32 query rows.  wo: W in operand order.
 template <typename Tag, int D, int BLKQ>

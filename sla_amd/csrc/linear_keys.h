@@ -1,6 +1,9 @@
 // Linear branch's backward, key side, for a wave's tiles of 16 keys: dv = c dS, dc = v dS^T + dz, dk = phi'(k) dc with
-// c = phi(k) (core.py:90-99 of the reference through autograd).  Shared by the kernel that walks k and v for it
-// (linear_bwd_stream.h) and by the attention's dK/dV kernel, which has a key block's gradients at hand when it ends.
+// c = phi(k) (core.py:90-99 of the reference through autograd).  KeyTiles is what the attention's dK/dV kernel, which has a key
+// block's gradients at hand when it ends, does for its rows.  The kernel that walks k and v for it (linear_bwd_keys_kernel in
+// linear_bwd_stream.h: a tile per step, the matrices in LDS) takes only the swizzle from here and forms the same sums by steps of
+// its own: which of the two runs follows from the size of the call and must not show in the bits, so a change to the arithmetic
+// of one is a change to both.
 #pragma once
 #include "linear_common.h"
 
