@@ -29,3 +29,19 @@ def test_values_of_the_16_bit_output(dev, H, L, D, BLKQ, half):
         out = mod(q, k, v)
     assert out.dtype == torch.float32 and out.is_contiguous() and torch.equal(out, ref.float())
     assert torch.equal(mod(q, k, v).detach(), out)                                   # through autograd
+
+
+@pytest.mark.parametrize("H,L,D,BLKQ", [(2, 161, 128, 128), (24, 833, 64, 64)])
+def test_16_bit_output_of_fp32_inputs(dev, monkeypatch, H, L, D, BLKQ):
+    """The C entry point's other form (in_dtype fp32, output in the compute dtype), which the module does not ask for."""
+    from sla_amd import _lib
+    g = torch.Generator().manual_seed(L)
+    q, k, v = (torch.randn(1, H, L, D, generator=g).to(dev) for _ in range(3))
+    mod = SparseLinearAttention(D, 0.5, "elu", BLKQ, 64).to(dev)
+    with torch.no_grad():
+        for p, t in zip((mod.proj_l.weight, mod.proj_l.bias), make_proj(D)):
+            p.copy_(t)
+        out = mod(q, k, v)
+        monkeypatch.setattr(_lib, "SLA_F32_BOTH", _lib.SLA_F32)      # (fills the first half of the fp32 tensor)
+        half = mod(q, k, v).view(-1).view(torch.bfloat16)[:out.numel()].view_as(out)
+    assert torch.equal(half.float(), out)
