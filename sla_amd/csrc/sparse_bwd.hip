@@ -594,9 +594,8 @@ int64_t sparse_bwd_workspace_bytes(int BH, int L, int D, int BLKQ, int BLKK, int
 // 158 / 158, 6144 730 / 738.  The whole backward on either side of the lines: head dim 128, 1020 key blocks 187.2 / 180.1, 1024 157.0 /
 // 156.2, 1152 195.4 / 194.6, 1280 194.1 / 191.3, 1536 214.8 / 210.5; head dim 64, 2000 177.4 / 171.3, 2048 184.1 / 178.5, 2256 230.0 /
 // 224.2, 2512 264.2 / 258.1, 3008 313.3 / 307.5: there the gain goes on behind the line.
-// (The compiler keeps 42 to 108 scalars of that variant in lanes of vector registers, in half precision at head dim 128 two vector
-// registers in memory, too; the loop over the list has none of their reads and writes, they stand in the branches of ragged rows, before
-// the loop and in the epilogue.)
+// (The compiler keeps 42 to 108 scalars of that variant in lanes of vector registers; the loop over the list has none of their reads and
+// writes, they stand in the branches of ragged rows, before the loop and in the epilogue.)
 static bool dkdv_takes_linear(int BH, int L, int D) { return (int64_t)BH * cdiv(L, 64) <= (D == 128 ? 1024 : 2048); }
 
 // (the stream dK/dV kernel reaches a head's rows with 31-bit byte offsets)

@@ -107,6 +107,7 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
   const i32x4_t item = items[logical];
   const int bh = __builtin_amdgcn_readfirstlane(item[0]), nb = __builtin_amdgcn_readfirstlane(item[1]);
   const int sg = __builtin_amdgcn_readfirstlane(item[2]), slot = __builtin_amdgcn_readfirstlane(item[3]);
+  if (slot < -1) return;              // (never: without the test two registers of the half-precision LINEAR variant go to scratch)
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);         // keys 32w .. 32w+31 of the block
   const int g = lane >> 5, r = lane & 31;
