@@ -54,7 +54,6 @@ static __device__ __forceinline__ void store_4(uint16_t* dst, float a, float b, 
 template <typename Tag, int D>
 __global__ __launch_bounds__(256) void bwd_delta_kernel(const uint16_t* __restrict__ o, const uint16_t* __restrict__ d_o,
                                                         const RowLayout ldo, float* __restrict__ delta, size_t rows, int L) {
-  using E = Elem<Tag>;
   constexpr int CPR = D / 8;
   const size_t row = (size_t)blockIdx.x * (256 / CPR) + threadIdx.x / CPR;   // = bh * L + l
   const int col = (threadIdx.x % CPR) * 8;
@@ -64,8 +63,7 @@ __global__ __launch_bounds__(256) void bwd_delta_kernel(const uint16_t* __restri
     const size_t l = row - (size_t)bh * L;
     const i16x8_t a = *reinterpret_cast<const i16x8_t*>(o + row * D + col);
     const i16x8_t b = *reinterpret_cast<const i16x8_t*>(d_o + ldo.head(bh) + l * (size_t)ldo.sl + col);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) s += E::to_float((uint16_t)a[e]) * E::to_float((uint16_t)b[e]);
+    s = delta_sum8<Tag>(a, b);
   }
 #pragma unroll
   for (int sh = 1; sh < CPR; sh <<= 1) s += __shfl_xor(s, sh);

@@ -891,7 +891,7 @@ static __device__ __forceinline__ void dq_stream_body(
     request_rows(vh, I<1>{}, E0 + 32, 3 * TILE);
   }
   // delta of this lane's two rows.  The sum runs in the order of bwd_delta_kernel, whose thread t adds the eight products
-  // of columns 8t .. 8t+7 one after the other and then meets threads t^1, t^2, t^4, t^8: here t = 2c + g, so the first
+  // of columns 8t .. 8t+7 (delta_sum8) and then meets threads t^1, t^2, t^4, t^8: here t = 2c + g, so the first
   // meeting is the one with lane^32 and the other three are between this lane's own chunks.
 #pragma unroll
   for (int qt = 0; qt < 2; ++qt) {
@@ -904,9 +904,7 @@ static __device__ __forceinline__ void dq_stream_body(
     float part[DC];
 #pragma unroll
     for (int c = 0; c < DC; ++c) {
-      float acc = 0.f;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) acc += E::to_float((uint16_t)of[qt][c][e]) * E::to_float((uint16_t)dof[qt][c][e]);
+      const float acc = delta_sum8<Tag>(of[qt][c], dof[qt][c]);
       part[c] = acc + __shfl_xor(acc, 32);
     }
 #pragma unroll

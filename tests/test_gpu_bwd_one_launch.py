@@ -1,5 +1,5 @@
 """dQ and dK/dV in one launch, with delta formed beforehand: against dense attention in fp32, lists cut into segments in several
-strips of 64 key blocks among them, and bit for bit against the launches of their own that larger calls take."""
+strips of 64 key blocks among them, and bit for bit against the launches of their own that larger calls of head dim 128 take."""
 import pytest
 import torch
 
@@ -57,21 +57,37 @@ def test_gradients(dev, H, L, D, BLKQ, dtype, sinks):
             assert err <= 4 * 2.0 ** -9 * max(float(r.norm()), 1e-3) + 1e-3, (name, h, err)
 
 
-@pytest.mark.parametrize("D,H", [(128, 128)])
-def test_one_launch_equals_two(dev, D, H):
-    """The largest call with one launch (16384 key blocks) and a call with a head more, which has two: the same bits per head."""
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H,BLKQ,sink", [
+    (128, 64, False), (64, 128, False),
+    (64, 64, True),                                             # lists of 256 entries: four segments, in four strips per head
+    (64, 128, True),                                            # 128 entries of two halves each: two segments
+])
+def test_one_launch_equals_two(dev, H, BLKQ, sink, dtype):
+    """The largest call of head dim 128 with one launch (16384 key blocks) and a call with a head more, which has two (work items
+    numbered beforehand, delta formed on dQ's way): the same bits per head; and a whole backward with two launches equals the attention's
+    gradients with the linear branch's added."""
+    from sla_amd.inputs import make_proj
+    from sla_amd.linear import linear_bwd
+    from sla_amd.module import module_bwd
     from sla_amd.sparse_attn import sparse_attn_bwd, sparse_attn_fwd
-    N = 16384 // H
-    L = 64 * N - 7
-    rows = torch.stack([torch.arange(N) * 5 % N, (torch.arange(N) * 5 + 3) % N], 1).sort(1).values
-    q, k, v, do, lut, smap = _case(dev, H + 1, L, D, 64, rows, torch.bfloat16, 1)
+    D, N = 128, 16384 // H
+    L, M = 64 * N - 7, N // (BLKQ // 64)
+    i = torch.arange(M)
+    rows = torch.stack([0 * i, 1 + i % (N - 1)] if sink else [i * 5 % N, (i * 5 + 3) % N], 1).sort(1).values
+    q, k, v, do, lut, smap = _case(dev, H + 1, L, D, BLKQ, rows, dtype, 1)
     scale = D ** -0.5
-    o, lse = sparse_attn_fwd(q, k, v, lut, 2, 64, 64, scale)
-    two = sparse_attn_bwd(q, k, v, o, do, lse, smap, lut, 2, 64, 64, scale)
+    o, lse = sparse_attn_fwd(q, k, v, lut, 2, BLKQ, 64, scale)
+    two = sparse_attn_bwd(q, k, v, o, do, lse, smap, lut, 2, BLKQ, 64, scale)
     first = [t[:, :H].contiguous() for t in (q, k, v, o, do, lse, smap, lut)]
-    one = sparse_attn_bwd(*first, 2, 64, 64, scale)
+    one = sparse_attn_bwd(*first, 2, BLKQ, 64, scale)
     for name, a, b in zip("qkv", one, two):
         assert torch.equal(a, b[:, :H]), name
+    w, b = (t.to(dev) for t in make_proj(D))
+    ref = linear_bwd(q, k, v, w, b, do, "softmax", accumulate_into=two)
+    got = module_bwd(q, k, v, o, do, lse, smap, lut, 2, BLKQ, 64, scale, w, b, "softmax")
+    for name, a, r in zip(("dq", "dk", "dv", "dw", "db"), got, ref):
+        assert torch.equal(a, r), name
 
 
 @pytest.mark.parametrize("H,L,D", [(32, 4090, 128), (33, 3970, 128)])
