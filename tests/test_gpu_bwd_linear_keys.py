@@ -1,5 +1,5 @@
-"""dK/dV launches that form the linear branch's dk, dv, too (up to 1024 key blocks of head dim 128, 2048 of 64), and the first ones
-that do not: a whole backward equals the attention's gradients with the linear branch's added, bit for bit."""
+"""Backward launches that form the linear branch's dk, dv, too (up to 2048 key blocks), and the first ones that do not: a whole
+backward equals the attention's gradients with the linear branch's added, bit for bit."""
 import pytest
 import torch
 
@@ -12,9 +12,11 @@ pytestmark = pytest.mark.gpu
     (5, 801, 128, 128, torch.float16, "softmax"),          # 128-row query blocks, the last without a second half
     (7, 831, 64, 64, torch.bfloat16, "relu"),
     (16, 4096, 128, 64, torch.bfloat16, "relu"),           # 1024 key blocks
-    (16, 4097, 128, 64, torch.bfloat16, "elu"),            # 1040
+    (16, 4097, 128, 64, torch.bfloat16, "elu"),            # 1040: two rounds of workgroups and a little more
     (32, 4090, 64, 128, torch.float16, "softmax"),         # 2048
     (33, 3970, 64, 64, torch.bfloat16, "elu"),             # 2079
+    (32, 4090, 128, 128, torch.float16, "softmax"),        # 2048
+    (33, 3970, 128, 128, torch.bfloat16, "relu"),          # 2079
     (1, 6400, 64, 64, torch.bfloat16, "softmax"),          # one list in segments
 ])
 def test_one_launch_equals_two(H, L, D, BLKQ, dtype, fmap):

@@ -1,6 +1,7 @@
-"""Work items of the dK/dV kernel: counts of (head, key block) pairs around the 512 one wave numbers, and key blocks that every
-query block selects, whose lists are cut into segments that the last workgroup to finish adds up; alone and added to what the
-gradients hold."""
+"""Work items of dK/dV: counts of (head, key block) pairs around 512, and key blocks that every query block selects, whose lists are
+cut into segments that the last workgroup to finish adds up; alone and added to what the gradients hold.  Calls of these sizes find
+their items in the launch that dQ shares (from the sums over strips of 64 key blocks); those of rows too far apart have them numbered
+beforehand, 512 pairs to a wave, as have the larger calls of test_gpu_bwd_one_launch and the longer rows of test_gpu_bwd_long_rows."""
 import pytest
 import torch
 
