@@ -21,7 +21,10 @@ def _views(kind, B, H, L, D, dtype, dev, seed):
 @pytest.mark.parametrize("kind", ["blhd", "packed"])
 @pytest.mark.parametrize("B,H,L,D,BLKQ,fmap,dtype,ratio", [(2, 3, 700, 128, 64, "elu", torch.bfloat16, 0.3),
                                                            (1, 2, 333, 64, 128, "softmax", torch.float16, 0.3),
-                                                           (1, 1, 50, 128, 64, "relu", torch.bfloat16, 1.0)])
+                                                           (1, 1, 50, 128, 64, "relu", torch.bfloat16, 1.0),
+                                                           # large inputs (from 40 MiB a tensor), whose chunk sums come with the states
+                                                           (2, 12, 8001, 128, 64, "elu", torch.bfloat16, 0.1),
+                                                           (2, 41, 4501, 64, 128, "softmax", torch.float16, 0.1)])
 def test_module_reads_views_in_place(dev, kind, B, H, L, D, BLKQ, fmap, dtype, ratio):
     q, k, v = _views(kind, B, H, L, D, dtype, dev, L)
     assert not q.is_contiguous() or B * H == 1
@@ -77,7 +80,9 @@ def test_block_inference_equals_block_with_copies(dev):
 
 
 @pytest.mark.parametrize("B,H,L,D,BLKQ,fmap,dtype", [(2, 2, 700, 128, 64, "elu", torch.bfloat16),
-                                                     (1, 3, 333, 64, 128, "softmax", torch.float16)])
+                                                     (1, 3, 333, 64, 128, "softmax", torch.float16),
+                                                     (2, 12, 8001, 128, 128, "relu", torch.bfloat16),       # (as above)
+                                                     (2, 41, 4501, 64, 64, "softmax", torch.float16)])
 def test_packed_training_equals_the_contiguous_route(dev, B, H, L, D, BLKQ, fmap, dtype):
     """forward_packed: output and all gradients (the packed one included) bit for bit what the module gives on
     contiguous (B, H, L, D) copies."""
@@ -110,7 +115,10 @@ def test_packed_training_equals_the_contiguous_route(dev, B, H, L, D, BLKQ, fmap
 
 
 @pytest.mark.parametrize("kind", ["blhd", "packed"])
-@pytest.mark.parametrize("B,H,L,D,fmap,dtype", [(2, 3, 700, 128, "elu", torch.bfloat16), (1, 2, 333, 64, "softmax", torch.float16)])
+@pytest.mark.parametrize("B,H,L,D,fmap,dtype", [(2, 3, 700, 128, "elu", torch.bfloat16), (1, 2, 333, 64, "softmax", torch.float16),
+                                                # large inputs (from 12.5 MiB a tensor), and more than 512 key blocks
+                                                (2, 13, 4001, 128, "relu", torch.bfloat16), (2, 41, 2501, 64, "softmax", torch.float16),
+                                                (2, 2, 64 * 513 + 1, 64, "elu", torch.bfloat16)])
 def test_quantised_module_reads_views_in_place(dev, kind, B, H, L, D, fmap, dtype):
     """SageSLA on (B, L, H, D) activations / packed projections viewed as (B, H, L, D): bit for bit what the contiguous
     copies give (quantisers, state build and output kernel all read the views), output in the views' memory order."""
