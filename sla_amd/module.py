@@ -56,11 +56,6 @@ def module_bwd(q, k, v, o_s, d_out, lse, sparse_map, lut, topk, BLKQ, BLKK, qk_s
     return dq, dk, dv, dw, db
 
 
-def _side_stream(dev):
-    """Second stream for the library's entry points that accept one: none, their work is all on the calling stream."""
-    return None
-
-
 @functools.lru_cache(maxsize=1024)
 def _plan(in_dt, dt, B, H, L, D, BLKQ, BLKK, T, keep):
     """Sizes of one forward: ``(workspace bytes, bytes to keep, offsets)``.  What a backward needs of the forward lies in one
@@ -114,7 +109,7 @@ def _module_fwd(q, k, v, weight, bias, topk_ratio, BLKQ, BLKK, fmap, dtype, keep
         base + off["cast"] if in_dt == _lib.SLA_F32 else None,
         weight.data_ptr(), bias.data_ptr(), out.data_ptr(), s_out, base + off["o_s"] if keep else None, base + off["lse"],
         base + off["map"] if keep else None, base + off["lut"], 4, base + off["states"], dt, _lib.FMAP[fmap], B, H, L, D, BLKQ,
-        BLKK, T, D ** -0.5, ws.data_ptr(), ws_bytes, _lib.stream_ptr(dev), _side_stream(dev))
+        BLKK, T, D ** -0.5, ws.data_ptr(), ws_bytes, _lib.stream_ptr(dev), None)
     _lib.check(rc)
     return out, saved, T
 
@@ -136,7 +131,7 @@ def _module_bwd_saved(saved, off, q_ptr, k_ptr, v_ptr, s_qkv, d_out, s_do, weigh
         q_ptr, k_ptr, v_ptr, s_qkv, base + off["o_s"], d_out.data_ptr(), s_do, base + off["lse"], base + off["map"],
         base + off["lut"], 4, weight.data_ptr(), bias.data_ptr(), base + off["states"], *grads, dw.data_ptr(),
         db.data_ptr(), dt, _lib.FMAP[fmap], B, H, L, D, BLKQ, BLKK, T, D ** -0.5, w0, n_s, w0 + n_s, n_l,
-        _lib.stream_ptr(dev), _side_stream(dev))
+        _lib.stream_ptr(dev), None)
     _lib.check(rc)
     return dw, db
 

@@ -12,7 +12,7 @@ import torch.nn as nn
 from . import _lib
 from .block_map import get_block_map, topk_count
 from .linear import linear_out_fwd
-from .module import FEATURE_MAPS, _side_stream, _StateBuild
+from .module import FEATURE_MAPS, _StateBuild
 
 SAGE_BLKQ, SAGE_BLKK = 128, 64
 # Range of the e4m3 values v is quantised to.  The reference's call passes 2.25 (SageSLA/core.py:129), which keeps the
@@ -135,7 +135,7 @@ def _sage_module_fwd(q, k, v, weight, bias, topk_ratio, fmap):
         s_in, s_out = _lib.strides_arg(q), _lib.strides_arg(out)
     rc = _lib.load().sage_module_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), s_in, weight.data_ptr(), bias.data_ptr(),
                                      out.data_ptr(), s_out, dt, _lib.FMAP[fmap], B, H, L, D, T, D ** -0.5, V_RANGE_E4M3,
-                                     ws.data_ptr(), n, _lib.stream_ptr(dev), _side_stream(dev))
+                                     ws.data_ptr(), n, _lib.stream_ptr(dev), None)
     _lib.check(rc)
     return out
 

@@ -32,8 +32,6 @@ def library(monkeypatch):
     lib = _Library()
     monkeypatch.setattr(_lib, "load", lambda: lib)
     monkeypatch.setattr(_lib, "stream_ptr", lambda dev: 0)
-    for mod in ("sla_amd.module", "sla_amd.sage"):
-        monkeypatch.setattr(mod + "._side_stream", lambda dev: None)
     _lib.workspace_bytes.cache_clear()
     module._plan.cache_clear()
     yield lib
