@@ -165,8 +165,8 @@ static inline bool narrow_pools(int dtype, int BH, int L, int D) {
 
 // Column mean of K, levels 2 and 3 of the summation order: one workgroup of NT threads per (head, slab of COLMEAN_SLAB
 // columns), thread (gi, c) = (tid / COLMEAN_SLAB, tid % COLMEAN_SLAB) forms group sums gi, gi + NT / COLMEAN_SLAB, ...
-// of its column; the first COLMEAN_SLAB threads then add the groups in ascending order.  (Small workgroups: the
-// launch has to find room beside the memory-bound kernels that run on other streams at the same time.)
+// of its column; the first COLMEAN_SLAB threads then add the groups in ascending order.  (256 threads where it is a launch of its
+// own or shares one with v's scales, 512 beside the slices' partial states.)
 constexpr int COLMEAN_SLAB = 16;
 constexpr int COLMEAN_MAX_GROUPS = 256;
 template <typename IO, int NT>

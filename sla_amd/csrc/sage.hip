@@ -173,9 +173,8 @@ __global__ __launch_bounds__(256) void v_amax_partial_kernel(const uint16_t* __r
   }
 }
 
-// grid (D / 16, BH), 256 threads: thread (cg, c) = (tid / 16, tid % 16) takes the maximum of column 16 blockIdx.x + c
-// over chunks cg, cg + 16, ...; the 16 partial maxima per column meet in LDS.  (Small workgroups: the launch has to
-// find room beside the memory-bound kernels of the other stream.)
+// D / 16 workgroups of 256 threads per head: thread (cg, c) = (tid / 16, tid % 16) takes the maximum of column 16 bx + c
+// over chunks cg, cg + 16, ...; the 16 partial maxima per column meet in LDS.
 static __device__ __forceinline__ void v_scale_body(const float* __restrict__ part, float* __restrict__ v_scale, int nchunk, int D,
                                                     float v_range, int bx, int bh, float* sm) {
   const int tid = threadIdx.x;

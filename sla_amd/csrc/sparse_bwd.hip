@@ -6,8 +6,10 @@
 //   P = exp2(S*c - lse) on the selected blocks, dP = dO V^T, dS = P * (dP - delta)
 //   dQ = scale * dS K ; dK = scale * dS^T Q ; dV = P^T dO
 //
-// Four kernels.
-//   delta      : one pass over o and do (the streaming dQ kernel forms it itself).
+// Steps, here and in sparse_bwd_stream.h, which takes every call whose rows lie within 31-bit byte offsets of a head (dQ: and select at
+// most 2048 key blocks each); the kernels of this file take the rest.
+//   delta      : one pass over o and do (beside the lists; a stream dQ launch of its own forms it on its way, and the general dQ
+//                kernel has a launch before it).
 //   col_lists  : the reference scans the dense int8 map column in the dK/dV kernel (about
 //                1/density wasted iterations); here the map is turned once into per-key-block
 //                lists of the query blocks that selected it.
@@ -18,7 +20,8 @@
 //   dkdv       : per key block over its list; S = Q K^T and dP = dO V^T with K^T/V^T resident
 //                in registers as B operands; P and dS leave the accumulators in B-operand layout
 //                for dV^T += dO^T P and dK^T += Q^T dS (Q^T, dO^T via transposing LDS reads).
-//                Four waves: two key halves x two halves of the head dimension.
+//                Four waves here: two key halves x two halves of the head dimension; lists cut into
+//                segments are summed by a launch of their own (the stream kernel's last segment does it).
 #include "bwd_lists.h"
 #include "bwd_steps.h"
 

@@ -1018,7 +1018,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
 
 // The 64 query rows `logical` by two waves of 32 rows each, for a launch whose waves share a SIMD in twos (head dim 64): half the
 // registers of a wave with all 64 (364, which dK/dV's waves cannot share a SIMD with), K and V in rings of four generations of 32 keys that both waves request and read, one barrier
-// per generation, delta read.  Products, arithmetic and roundings are those of dq_stream_body, so the same bits.
+// per generation, delta read.  Order of the products, arithmetic and roundings follow dq_stream_body's scheme, which has head dim 128.
 // smem: DQ_PAIR_LDS bytes, entries: DQ_STREAM_MAX_T numbers of LDS.
 template <int D>
 constexpr int DQ_PAIR_LDS = 8 * BwdTile<D>::BYTES;      // four generations: 32 rows of K and of V

@@ -19,7 +19,7 @@ pytestmark = pytest.mark.gpu
     (1, 2, 4097, 64, 64, torch.float16, "softmax", True), (3, 7, 1023, 128, 64, torch.float32, "elu", False),
     (1, 16, 4160, 64, 64, torch.bfloat16, "elu", False), (1, 8, 8191, 128, 64, torch.bfloat16, "relu", False),
     (2, 40, 321, 64, 64, torch.float32, "softmax", True), (1, 1, 10500, 64, 64, torch.float32, "elu", False),
-    (1, 40, 6601, 128, 128, torch.bfloat16, "elu", False), (1, 40, 6601, 128, 64, torch.float32, "softmax", True)])   # (two streams)
+    (1, 40, 6601, 128, 128, torch.bfloat16, "elu", False), (1, 40, 6601, 128, 64, torch.float32, "softmax", True)])   # (from 64 MiB on)
 def test_forward_equals_the_steps(dev, B, H, L, D, BLKQ, in_dtype, fmap, half):
     dtype = torch.float16 if half else torch.bfloat16
     g = torch.Generator().manual_seed(L + D)

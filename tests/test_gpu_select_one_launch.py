@@ -1,5 +1,5 @@
 """Scores and selection in one launch: key-block counts around its tiles of 16 and 32 blocks and the lengths at which its rows take
-one, two or four keys per lane or leave it (257 blocks, 272 workgroups), against the CPU oracle, bit for bit."""
+one, two or four keys per lane, more (257 blocks of 16-bit inputs) or leave it (129 of fp32), against the CPU oracle, bit for bit."""
 import pytest
 import torch
 
