@@ -594,11 +594,11 @@ int64_t sparse_bwd_workspace_bytes(int BH, int L, int D, int BLKQ, int BLKK, int
 
 // Whether dK/dV forms the linear branch's dk, dv as well, in the place of a launch that walks k and v for them.  It costs each of
 // its workgroups 5 to 6 us, bound by issue (the feature map, two products of 32 rows with D x D, 64 KB of matrices); what it saves is the
-// launch and a pass over dk and dv.  The kernels' times together in us, apart and in one, dQ in the same launch at head dim 128 (512
-// workgroups are resident): 1088 key blocks 153 / 143, 1284 138 / 141, 1512 122 / 119, 1524 194 / 189, 1764 232 / 236, 1896 168 / 167,
-// 2000 399 / 397: the launch and its share of the host's time are what is left of it there, and 6144 key blocks lost 8.  Head dim 64 (1024
-// are resident), the whole backward: 2000 177.4 / 171.3, 2048 184.1 / 178.5, 2256 230.0 / 224.2, 2512 264.2 / 258.1, 3008 313.3 / 307.5: there
-// the gain goes on behind the line.
+// launch and a pass over dk and dv.  Whole backward in us, apart and in one, in turn on one card (runs of one side within 2 %), 64-row
+// blocks, 10 % of the key blocks selected: head dim 128, 1088 key blocks 136.3 / 129.5, 1284 176.0 / 169.3, 1504 268.8 / 264.6, 1512 167.6 /
+// 161.9, 1760 294.0 / 292.5, 1896 208.8 / 205.3, 2000 272.0 / 267.8; head dim 64, 1504 104.1 / 98.3, 2000 148.0 / 144.1.  128-row blocks and
+// normal q and k gain as much, but for single ones that are equal.  The gain goes on behind the line, which no measurement asked for so far:
+// head dim 128, 2512 382.8 / 375.2, 3760 453.9 / 443.2, 6000 817 / 806; head dim 64, 2512 204.0 / 195.7, 6000 659 / 635, 12288 2370 / 2327.
 // (The compiler keeps 42 to 175 scalars of that variant in lanes of vector registers; the loop over the list has none of their reads and
 // writes, they stand in the branches of ragged rows, before the loop and in the epilogue.)
 static bool dkdv_takes_linear(int BH, int L) { return (int64_t)BH * cdiv(L, 64) <= 2048; }
@@ -612,13 +612,18 @@ static bool dkdv_streams(const RowLayout& lin, const RowLayout& ldo, int L) {
 static bool dq_streams(const RowLayout& lin, const RowLayout& ldo, int L, int topk) {
   return dkdv_streams(lin, ldo, L) && topk <= DQ_STREAM_MAX_T && L <= 64 * 65535;
 }
-// Whether dQ and dK/dV then share one launch, for which delta is formed beforehand.  Kernels of a forward and backward in us, before
-// and so: 2 x 1024 x 128, 4 key blocks per row 95 / 77 (general dQ kernel, delta and short jobs in launches of their own), 4 x 9000, 14 per
-// row, 128-row blocks 250 / 200, 8 x 4096, 12 per row 179 / 162, 16 x 6001 x 64, 9 per row 187 / 167; whole passes: 12 x 9360, 14 per row,
-// 128-row blocks 451 / 429, 12 x 16380 without the linear branch 392 / 371, 12 x 32760, 25 per row 1862 / 1842, 32 x 32760, 25 per row,
-// 128-row blocks 4123 / 4103; head dim 64: 12 x 32760, 25 per row 984 / 936, 40 x 60000, 47 per row 9115 / 9004.  At head dim 128 the gain
-// ends there: 40 x 75600 (47280 key blocks) 26.9 / 27.4 ms, where dQ in a launch of its own forms delta on its way and a pass over d(out)
-// and the output more is what one launch costs.
+// Whether dQ and dK/dV then share one launch, for which delta is formed beforehand.  What it gains is the end of the key blocks' part,
+// filled by query blocks, and launches; what it costs are a pass over d(out) and the output for delta, and two kernels that share the
+// L2s.  Head dim 64, whole passes before and so: 12 x 32760, 25 per row 984 / 936, 40 x 60000, 47 per row 9115 / 9004.  Head dim 128,
+// forward and backward in us, two launches and one, in turn on one card (runs of one side within 1 %), 64-row blocks, smooth q and k (neighbours
+// select alike, lists differ in length), in the order of their key blocks: 12 x 9000 408 / 378, 24 x 6000 443 / 405, 12 x 16380 622 / 592,
+// 40 x 6000 677 / 649, 16 x 20000 1085 / 1060, 12 x 32760 1804 / 1779, 24 x 20000 1612 / 1600, 16 x 32760 2378 / 2365, 60 x 10000 2036 / 2035, 24 x
+// 32760 3569 / 3568, 12 x 75600 7931 / 7860, 32 x 32760 (16384) 4681 / 4687; behind the line 60 x 20000 3986 / 3989, 40 x 32760 5860 / 5874, 24 x
+// 60000 10073 / 10063, 160 x 10000 5535 / 5580, 40 x 60000 16952 / 16842, 256 x 10000 8392 / 8467, 40 x 75600 26124 / 26346.  So up to some
+// 14000 key blocks one launch is ahead or equal, from there on the two are within a percent, long sequences ahead in one, short ones in
+// two; where between them the line lies makes no difference that the runs show.  128-row blocks stand up to 1 % more
+// in favour of one.  With normal q and k, whose lists are all equally long, 64-row blocks lose from 6144 key blocks on, most at 12 x 32760 with 51
+// per row (3185 / 3234), 25 per row 1915 / 1922; no size says which inputs a call has.
 static bool both_in_one(const RowLayout& lin, const RowLayout& ldo, int BH, int L, int D, int topk) {
   return dq_streams(lin, ldo, L, topk) && (D == 64 || (int64_t)BH * cdiv(L, 64) <= 16384);
 }
