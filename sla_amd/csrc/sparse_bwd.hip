@@ -597,7 +597,7 @@ int64_t sparse_bwd_workspace_bytes(int BH, int L, int D, int BLKQ, int BLKK, int
 // launch and a pass over dk and dv.  Whole backward in us, apart and in one, in turn on one card (runs of one side within 2 %), 64-row
 // blocks, 10 % of the key blocks selected: head dim 128, 1088 key blocks 136.3 / 129.5, 1284 176.0 / 169.3, 1504 268.8 / 264.6, 1512 167.6 /
 // 161.9, 1760 294.0 / 292.5, 1896 208.8 / 205.3, 2000 272.0 / 267.8; head dim 64, 1504 104.1 / 98.3, 2000 148.0 / 144.1.  128-row blocks and
-// normal q and k gain as much, but for single ones that are equal.  The gain goes on behind the line, which no measurement asked for so far:
+// normal q and k gain as much, but for single ones that are equal.  The gain goes on behind the line:
 // head dim 128, 2512 382.8 / 375.2, 3760 453.9 / 443.2, 6000 817 / 806; head dim 64, 2512 204.0 / 195.7, 6000 659 / 635, 12288 2370 / 2327.
 // (The compiler keeps 42 to 175 scalars of that variant in lanes of vector registers; the loop over the list has none of their reads and
 // writes, they stand in the branches of ragged rows, before the loop and in the epilogue.)
@@ -622,8 +622,8 @@ static bool dq_streams(const RowLayout& lin, const RowLayout& ldo, int L, int to
 // 60000 10073 / 10063, 160 x 10000 5535 / 5580, 40 x 60000 16952 / 16842, 256 x 10000 8392 / 8467, 40 x 75600 26124 / 26346.  So up to some
 // 14000 key blocks one launch is ahead or equal, from there on the two are within a percent, long sequences ahead in one, short ones in
 // two; where between them the line lies makes no difference that the runs show.  128-row blocks stand up to 1 % more
-// in favour of one.  With normal q and k, whose lists are all equally long, 64-row blocks lose from 6144 key blocks on, most at 12 x 32760 with 51
-// per row (3185 / 3234), 25 per row 1915 / 1922; no size says which inputs a call has.
+// in favour of one.  With normal q and k, whose lists are all equally long, one launch stands between 0.9 % ahead and 1.5 % behind from
+// 6144 key blocks of 64-row calls on (12 x 32760 with 51 per row 3185 / 3234, with 25 1915 / 1922); no size says which inputs a call has.
 static bool both_in_one(const RowLayout& lin, const RowLayout& ldo, int BH, int L, int D, int topk) {
   return dq_streams(lin, ldo, L, topk) && (D == 64 || (int64_t)BH * cdiv(L, 64) <= 16384);
 }
